@@ -15,10 +15,12 @@
 //    pass is histogram -> scan -> stable scatter; the scatter ranks equal digits
 //    inside a wave with 8 ballots (no LDS atomics, order preserved) and across
 //    waves with a small LDS table.  What moves is one 64-bit word per edge, key
-//    above and original position below, so a pass is 8 bytes in and 8 bytes out per
-//    edge and the permutation falls out of the last pass.  indptr then comes from
-//    one search per column in the sorted keys, confined to the keys of the
-//    workgroup's 1024 columns (in LDS when they are few).
+//    above and original position below, and the value in 32 bits, so a pass is 12
+//    bytes in and 12 bytes out per edge and the permutation falls out of the last
+//    pass.  indptr then comes from the places where the sorted keys change, or, with
+//    fewer edges than columns, from one search per column confined to the keys of
+//    the workgroup's 256 columns.
+//  * distinct ids of an edge list: a byte per possible id, marked with plain stores.
 #include "gs_common.hpp"
 
 namespace gs {
@@ -194,8 +196,7 @@ compress_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
   }
 }
 
-// Sorted keys as the kernels below read them: an id array, or the sort's own words
-// (key above the low idx_bits bits).
+// Sorted keys as the kernels below read them.
 template <typename KeyT>
 struct PlainKeys {
   const KeyT* key;
@@ -203,11 +204,13 @@ struct PlainKeys {
     return static_cast<int64_t>(key[i]);
   }
 };
-struct WordKeys {
-  const unsigned long long* word;
-  int idx_bits;
+// (keys beyond 32 bits: the sort keeps no copy of them)
+template <typename KeyT>
+struct PermutedKeys {
+  const KeyT* key;
+  const int64_t* perm;
   __device__ __forceinline__ int64_t operator()(int64_t i) const {
-    return static_cast<int64_t>(word[i] >> idx_bits);
+    return static_cast<int64_t>(key[perm[i]]);
   }
 };
 
@@ -287,6 +290,84 @@ indptr_from_sorted_kernel(Keys key, int64_t E, int64_t num_keys, int64_t* __rest
   }
 }
 
+// The same offsets from the places where the keys change, for more edges than columns: item i
+// of [0, E] (key E is the number of columns) writes offset i for the columns after key i - 1
+// up to key i.  Every key is read once, coalesced, where the searches above cost a workgroup
+// five dependent trips before it starts: 14 M keys, 2.45 M columns 75 -> 22 us.  Gaps longer
+// than kGapAlone columns are set aside and filled by whole waves, so that a run of absent
+// ids does not become one lane's loop; with fewer edges than columns (a slice's rows among
+// all rows) nearly every item would be such a gap and the searches are the better split.
+constexpr int kFillItems = 16;
+constexpr int kFillTile = kThreads * kFillItems;
+constexpr int kGapAlone = 16;
+constexpr int kGapWide = 2048;  // columns from which a gap is filled by the whole workgroup
+
+template <typename KeyT>
+__global__ void __launch_bounds__(kThreads)
+indptr_fill_kernel(const KeyT* __restrict__ key, int64_t E, int64_t num_keys,
+                   int64_t* __restrict__ indptr) {
+  __shared__ unsigned short s_gap[kFillTile];
+  __shared__ int s_gaps;
+  if (threadIdx.x == 0) s_gaps = 0;
+  __syncthreads();
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * kFillTile;
+  // (keys outside [0, num_keys) count as the nearest end: every store stays inside indptr)
+  auto bounded = [&](KeyT k) {
+    const int64_t v = static_cast<int64_t>(k);
+    return v < 0 ? int64_t(-1) : (v > num_keys ? num_keys : v);
+  };
+  KeyT hi[kFillItems], lo[kFillItems];
+#pragma unroll
+  for (int k = 0; k < kFillItems; ++k) {
+    const int64_t i = base + k * kThreads + threadIdx.x;
+    hi[k] = key[i < E ? i : E - 1];
+  }
+#pragma unroll
+  for (int k = 0; k < kFillItems; ++k) {
+    const int64_t i = base + k * kThreads + threadIdx.x;
+    lo[k] = key[i < 1 ? 0 : (i <= E ? i - 1 : E - 1)];
+  }
+#pragma unroll
+  for (int k = 0; k < kFillItems; ++k) {
+    const int at = k * kThreads + threadIdx.x;
+    const int64_t i = base + at;
+    if (i > E) continue;
+    const int64_t first = i == 0 ? 0 : bounded(lo[k]) + 1;
+    const int64_t last = i == E ? num_keys : bounded(hi[k]);
+    if (last - first < kGapAlone) {
+      for (int64_t c = first; c <= last; ++c) indptr[c] = i;
+    } else {
+      s_gap[atomicAdd(&s_gaps, 1)] = static_cast<unsigned short>(at);
+    }
+  }
+  __syncthreads();
+  const int n = s_gaps;
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+  for (int g = 0; g < n; ++g) {
+    const int64_t i = base + s_gap[g];
+    const int64_t first = i == 0 ? 0 : bounded(key[i - 1]) + 1;
+    const int64_t last = i == E ? num_keys : bounded(key[i]);
+    if (last - first >= kGapWide) {
+      for (int64_t c = first + threadIdx.x; c <= last; c += kThreads) indptr[c] = i;
+    } else if ((g & (kThreads / kWave - 1)) == wave) {
+      for (int64_t c = first + lane; c <= last; c += kWave) indptr[c] = i;
+    }
+  }
+}
+
+template <typename KeyT>
+void launch_indptr(const KeyT* key, int64_t E, int64_t num_keys, int64_t* indptr, hipStream_t st) {
+  if (E > 0 && num_keys <= E) {
+    hipLaunchKernelGGL((indptr_fill_kernel<KeyT>), dim3(blocks_for(E + 1, kFillTile)),
+                       dim3(kThreads), 0, st, key, E, num_keys, indptr);
+    return;
+  }
+  PlainKeys<KeyT> keys{key};
+  hipLaunchKernelGGL((indptr_from_sorted_kernel<PlainKeys<KeyT>>),
+                     dim3(blocks_for(num_keys + 1, kPtrCols)), dim3(kThreads), 0, st, keys, E,
+                     num_keys, indptr);
+}
+
 // ------------------------------------------------------------ radix sort ----
 // The sort moves ONE 64-bit word per edge: key above, position of the edge below
 // (idx_bits = bits of the edge count).  Sorting the words is the stable sort of the keys,
@@ -294,7 +375,6 @@ indptr_from_sorted_kernel(Keys key, int64_t E, int64_t num_keys, int64_t* __rest
 // edge instead of a widened key and a permutation entry each way.
 constexpr int kRadixBits = 8;
 constexpr int kRadix = 1 << kRadixBits;
-constexpr int kWaves = kThreads / kWave;
 
 __device__ __forceinline__ int digit_of(unsigned long long word, int shift) {
   return static_cast<int>((word >> shift) & (kRadix - 1));
@@ -315,30 +395,53 @@ struct StoredWords {
   __device__ __forceinline__ unsigned long long operator()(int64_t i) const { return word[i]; }
 };
 
-// A tile of the sort: 256 threads, 16 items each with 4-byte values, 8 with 8-byte values (the
-// tile's words and values pass through LDS on their way out).
-template <typename IdT>
+// A tile of the sort.  Its items leave digit by digit, so a run is a 256th of the tile on
+// average: the larger tile writes runs of 256 bytes where the smaller one writes 128, which
+// is what the scatter waits for once there are enough tiles to fill the chip; with few
+// tiles the smaller one spreads them over more compute units.
+template <int THREADS, int PER_THREAD>
 struct SortTile {
-  static constexpr int kPerThread = sizeof(IdT) == 4 ? 16 : 8;
-  static constexpr int kSize = kThreads * kPerThread;
-  static constexpr int kRounds = kSize / kWaves / kWave;  // rounds of 64 consecutive items per wave
+  static constexpr int kThreadsPerTile = THREADS;
+  static constexpr int kPerThread = PER_THREAD;
+  static constexpr int kSize = THREADS * PER_THREAD;
+  static constexpr int kWaves = THREADS / kWave;
 };
+using SmallTile = SortTile<256, 16>;
+using LargeTile = SortTile<512, 16>;
+constexpr int64_t kLargeTileItems = int64_t(1) << 22;  // 512 large tiles: two for every compute unit
 
-// counts[d * num_blocks + b] = items of tile b with digit d
-template <typename Src, int TILE>
-__global__ void __launch_bounds__(kThreads)
-radix_hist_kernel(Src src, int64_t E, int shift, int64_t num_blocks, int64_t* __restrict__ counts) {
-  __shared__ int s_hist[kRadix];
-  s_hist[threadIdx.x] = 0;
+// counts[d * num_blocks + b] = items of tile b with digit d.  Four copies of the histogram, lane
+// by lane in turn: on a skewed graph half a wave holds one digit, and additions to one LDS word
+// queue up.
+constexpr int kHistCopies = 4;
+
+template <typename T, typename Src>
+__global__ void __launch_bounds__(T::kThreadsPerTile)
+radix_hist_kernel(Src src, int64_t E, int shift, int64_t num_blocks, int64_t* __restrict__ counts,
+                  int* __restrict__ clear) {
+  __shared__ int s_hist[kHistCopies][kRadix + 1];
+  for (int j = threadIdx.x; j < kHistCopies * (kRadix + 1); j += T::kThreadsPerTile)
+    (&s_hist[0][0])[j] = 0;
+  if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;
   __syncthreads();
-  const int64_t base = static_cast<int64_t>(blockIdx.x) * TILE;
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * T::kSize;
+  unsigned long long word[T::kPerThread];
 #pragma unroll
-  for (int k = 0; k < TILE / kThreads; ++k) {
-    const int64_t i = base + k * kThreads + threadIdx.x;
-    if (i < E) atomicAdd(&s_hist[digit_of(src(i), shift)], 1);
+  for (int k = 0; k < T::kPerThread; ++k) {
+    const int64_t i = base + k * T::kThreadsPerTile + threadIdx.x;
+    word[k] = src(i < E ? i : E - 1);
   }
+#pragma unroll
+  for (int k = 0; k < T::kPerThread; ++k)
+    if (base + k * T::kThreadsPerTile + threadIdx.x < E)
+      atomicAdd(&s_hist[threadIdx.x & (kHistCopies - 1)][digit_of(word[k], shift)], 1);
   __syncthreads();
-  counts[static_cast<int64_t>(threadIdx.x) * num_blocks + blockIdx.x] = s_hist[threadIdx.x];
+  if (threadIdx.x < kRadix) {
+    int n = 0;
+#pragma unroll
+    for (int c = 0; c < kHistCopies; ++c) n += s_hist[c][threadIdx.x];
+    counts[static_cast<int64_t>(threadIdx.x) * num_blocks + blockIdx.x] = n;
+  }
 }
 
 struct LoadI64 {
@@ -352,11 +455,12 @@ template <typename IdT>
 struct SortOutputs {
   IdT* value;
   int64_t* perm;
-  IdT* key;
+  uint32_t* key;
   int idx_bits;
+  int* wide;  // raised when a 64-bit value does not fit 32 bits (null: 32-bit values)
 };
 
-// One pass of the sort over one tile, stable.  A wave owns a quarter of the tile, in index
+// One pass of the sort over one tile, stable.  A wave owns its share of the tile, in index
 // order, and visits it 64 consecutive items at a time: the rank of an item among the equal
 // digits of its round comes from 8 ballots, the count of the wave's earlier rounds from a
 // small LDS table only that wave touches (no workgroup barrier per round).  One barrier
@@ -366,137 +470,186 @@ struct SortOutputs {
 // scatter straight from registers wrote 8 bytes here and 8 bytes there.
 // The value rides along with its word from the first pass on (read in input order then), so
 // no pass gathers it by position; the LAST pass writes values, permutation and keys instead
-// of words.
+// of words.  64-bit values travel in their low 32 bits: ids of any graph that fits the card do,
+// and a value that does not raises `wide`, on which widen_values_kernel fetches all of them
+// again through the permutation.  That and the larger tile took 14 M edges with 64-bit ids
+// and 22-bit keys from 215 us a pass (histogram, scan, scatter) to 150 (the first, which reads the ids as they come) and 119.
 // SELF: `offsets` holds the tiles' raw counts and every workgroup adds up for itself where its
 // runs start (a sort of few tiles: two launches less per pass than scanning the counts first).
 constexpr int64_t kSelfScanTiles = 64;
 
-template <typename IdT, typename Src, bool LAST, bool SELF>
-__global__ void __launch_bounds__(kThreads)
-radix_pass_kernel(Src src, const IdT* __restrict__ val_in, int64_t E, int shift,
+template <typename T, typename IdT, typename ValT, typename Src, bool LAST, bool SELF>
+__global__ void __launch_bounds__(T::kThreadsPerTile, 4)  // (16 waves a CU is what LDS allows)
+radix_pass_kernel(Src src, const ValT* __restrict__ val_in, int64_t E, int shift,
                   int64_t num_blocks, const int64_t* __restrict__ offsets,
-                  unsigned long long* __restrict__ out, IdT* __restrict__ val_out,
+                  unsigned long long* __restrict__ out, uint32_t* __restrict__ val_out,
                   SortOutputs<IdT> last) {
-  using T = SortTile<IdT>;
+  constexpr int kThreadsHere = T::kThreadsPerTile, kItemsHere = T::kPerThread;
   __shared__ unsigned long long s_word[T::kSize];
-  __shared__ int64_t s_base[kRadix];     // where the tile's run of a digit starts in memory
-  __shared__ int s_cnt[kWaves][kRadix];  // per wave: count, then count of the earlier waves
-  __shared__ int s_start[kRadix];        // where the run of a digit starts in the tile
-  __shared__ int s_scan[kWaves];
+  __shared__ int64_t s_base[kRadix];        // memory position of a digit's run minus its place in the tile
+  __shared__ int s_cnt[T::kWaves][kRadix];  // per wave: count, then count of the earlier waves
+  __shared__ int s_start[kRadix];           // where the run of a digit starts in the tile
+  __shared__ int s_scan[kRadix / kWave];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
+  const int digit = threadIdx.x;  // of the first 256 threads
+  int64_t run_at = 0;
   if (SELF) {
-    // digit threadIdx.x: its items in all tiles, and in the tiles before this one
-    __shared__ int64_t s_digits[kWaves];
-    const int64_t* row = offsets + static_cast<int64_t>(threadIdx.x) * num_blocks;
-    int64_t all = 0, before = 0;
-    for (int64_t b = 0; b < num_blocks; ++b) {
-      const int64_t c = row[b];
-      all += c;
-      before += b < static_cast<int64_t>(blockIdx.x) ? c : 0;
-    }
-    int64_t incl = all;
+    // this digit's items in all tiles, and in the tiles before this one
+    __shared__ int64_t s_digits[kRadix / kWave];
+    int64_t all = 0, before = 0, incl = 0;
+    if (digit < kRadix) {
+      const int64_t* row = offsets + static_cast<int64_t>(digit) * num_blocks;
+      for (int64_t b = 0; b < num_blocks; ++b) {
+        const int64_t c = row[b];
+        all += c;
+        before += b < static_cast<int64_t>(blockIdx.x) ? c : 0;
+      }
+      incl = all;
 #pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-      const int64_t y = __shfl_up(incl, d, kWave);
-      if (lane >= d) incl += y;
+      for (int d = 1; d < kWave; d <<= 1) {
+        const int64_t y = __shfl_up(incl, d, kWave);
+        if (lane >= d) incl += y;
+      }
+      if (lane == kWave - 1) s_digits[wave] = incl;
     }
-    if (lane == kWave - 1) s_digits[wave] = incl;
     __syncthreads();
-    int64_t lower = incl - all;  // items of the smaller digits
-    for (int w = 0; w < wave; ++w) lower += s_digits[w];
-    s_base[threadIdx.x] = lower + before;
-  } else {
-    s_base[threadIdx.x] = offsets[static_cast<int64_t>(threadIdx.x) * num_blocks + blockIdx.x];
+    if (digit < kRadix) {
+      int64_t lower = incl - all;  // items of the smaller digits
+      for (int w = 0; w < wave; ++w) lower += s_digits[w];
+      run_at = lower + before;
+    }
+  } else if (digit < kRadix) {
+    run_at = offsets[static_cast<int64_t>(digit) * num_blocks + blockIdx.x];
   }
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) s_cnt[w][threadIdx.x] = 0;
+  for (int j = threadIdx.x; j < T::kWaves * kRadix; j += kThreadsHere) (&s_cnt[0][0])[j] = 0;
   const int64_t base = static_cast<int64_t>(blockIdx.x) * T::kSize;
-  const int64_t wave_base = base + static_cast<int64_t>(wave) * (T::kSize / kWaves);
-  unsigned long long word[T::kRounds];
-  IdT val[T::kRounds];
+  const int64_t wave_base = base + static_cast<int64_t>(wave) * (T::kSize / T::kWaves);
+  // (indices clamped instead of reads left out: all of a thread's reads go out together)
+  unsigned long long word[kItemsHere];
+  ValT raw[kItemsHere];
 #pragma unroll
-  for (int r = 0; r < T::kRounds; ++r) {
+  for (int r = 0; r < kItemsHere; ++r) {
     const int64_t i = wave_base + r * kWave + lane;
-    word[r] = i < E ? src(i) : ~0ull;
-    val[r] = i < E ? val_in[i] : IdT(0);
+    word[r] = src(i < E ? i : E - 1);
+  }
+  // (what lies behind the last edge takes the last digit; it comes last in index order, so its
+  // places are those behind the tile's live items and none of them is written out)
+#pragma unroll
+  for (int r = 0; r < kItemsHere; ++r)
+    if (wave_base + r * kWave + lane >= E) word[r] = ~0ull;
+#pragma unroll
+  for (int r = 0; r < kItemsHere; ++r) {
+    const int64_t i = wave_base + r * kWave + lane;
+    raw[r] = val_in[i < E ? i : E - 1];
   }
   __syncthreads();  // the tables are zero
-  int place[T::kRounds];
+  int place[kItemsHere];
 #pragma unroll
-  for (int r = 0; r < T::kRounds; ++r) {
-    const bool live = wave_base + r * kWave + lane < E;
+  for (int r = 0; r < kItemsHere; ++r) {
     const int d = digit_of(word[r], shift);
-    unsigned long long peers = __ballot(live);
+    // lanes with this digit: per bit, the lanes whose bit equals this lane's (two instructions a
+    // half-word, and-not-xor in one; sixty-four selects and masks a round bounded the pass before)
+    uint32_t lo = ~0u, hi = ~0u;
 #pragma unroll
     for (int b = 0; b < kRadixBits; ++b) {
-      const bool bit = (d >> b) & 1;
-      const unsigned long long bal = __ballot(live && bit);
-      peers &= bit ? bal : ~bal;
+      const int mine = static_cast<int>(static_cast<uint32_t>(d) << (31 - b)) >> 31;
+      const unsigned long long bal = __ballot(mine);
+      lo = __builtin_amdgcn_bitop3_b32(lo, static_cast<uint32_t>(bal), mine, 0x90);
+      hi = __builtin_amdgcn_bitop3_b32(hi, static_cast<uint32_t>(bal >> 32), mine, 0x90);
     }
-    const int rank = __popcll(peers & ((1ull << lane) - 1ull));
+    const int rank = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0));
     const int before = s_cnt[wave][d];  // the wave's earlier rounds (LDS operations of a wave keep their order)
     place[r] = before + rank;
-    if (live && rank == 0) s_cnt[wave][d] = before + __popcll(peers);
+    if (rank == 0) s_cnt[wave][d] = before + __popc(lo) + __popc(hi);
+  }
+  uint32_t val[kItemsHere];
+  bool wide = false;
+#pragma unroll
+  for (int r = 0; r < kItemsHere; ++r) {
+    val[r] = static_cast<uint32_t>(raw[r]);
+    if (sizeof(ValT) == 8) wide |= static_cast<uint64_t>(raw[r]) != val[r];
+  }
+  if (sizeof(ValT) == 8 && wide) *last.wide = 1;
+  __syncthreads();
+  // digit by digit: counts of the waves -> counts of the earlier waves, total -> start
+  int total = 0, incl = 0;
+  if (digit < kRadix) {
+#pragma unroll
+    for (int w = 0; w < T::kWaves; ++w) {
+      const int c = s_cnt[w][digit];
+      s_cnt[w][digit] = total;
+      total += c;
+    }
+    incl = total;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int y = __shfl_up(incl, d, kWave);
+      if (lane >= d) incl += y;
+    }
+    if (lane == kWave - 1) s_scan[wave] = incl;
   }
   __syncthreads();
-  // digit threadIdx.x: counts of the waves -> counts of the earlier waves, total -> start
-  int total = 0;
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    const int c = s_cnt[w][threadIdx.x];
-    s_cnt[w][threadIdx.x] = total;
-    total += c;
+  if (digit < kRadix) {
+    int start = incl - total;
+    for (int w = 0; w < wave; ++w) start += s_scan[w];
+    s_start[digit] = start;
+    s_base[digit] = run_at - start;
   }
-  int incl = total;
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const int y = __shfl_up(incl, d, kWave);
-    if (lane >= d) incl += y;
-  }
-  if (lane == kWave - 1) s_scan[wave] = incl;
-  __syncthreads();
-  int start = incl - total;
-  for (int w = 0; w < wave; ++w) start += s_scan[w];
-  s_start[threadIdx.x] = start;
   __syncthreads();
   // (words first, then the values through the same LDS: half the footprint of staging both
   // at once, and twice the workgroups per compute unit)
 #pragma unroll
-  for (int r = 0; r < T::kRounds; ++r) {
+  for (int r = 0; r < kItemsHere; ++r) {
     const int d = digit_of(word[r], shift);
     place[r] += s_start[d] + s_cnt[wave][d];
-    if (wave_base + r * kWave + lane < E) s_word[place[r]] = word[r];
+    s_word[place[r]] = word[r];
   }
   __syncthreads();
   const int n = static_cast<int>(E - base < T::kSize ? E - base : T::kSize);
-  int64_t dst[T::kPerThread];
+  int out_digit[kItemsHere];
 #pragma unroll
-  for (int k = 0; k < T::kPerThread; ++k) {
-    const int j = k * kThreads + threadIdx.x;
-    dst[k] = -1;
+  for (int k = 0; k < kItemsHere; ++k) {
+    const int j = k * kThreadsHere + threadIdx.x;
+    out_digit[k] = 0;
     if (j < n) {
       const unsigned long long w = s_word[j];
-      const int d = digit_of(w, shift);
-      dst[k] = s_base[d] + (j - s_start[d]);
+      out_digit[k] = digit_of(w, shift);
+      const int64_t dst = s_base[out_digit[k]] + j;
       if (LAST) {
-        last.perm[dst[k]] = static_cast<int64_t>(w & ((1ull << last.idx_bits) - 1ull));
-        if (last.key) last.key[dst[k]] = static_cast<IdT>(w >> last.idx_bits);
+        last.perm[dst] = static_cast<int64_t>(w & ((1ull << last.idx_bits) - 1ull));
+        if (last.key) last.key[dst] = static_cast<uint32_t>(w >> last.idx_bits);
       } else {
-        out[dst[k]] = w;
+        out[dst] = w;
       }
     }
   }
   __syncthreads();
-  IdT* s_val = reinterpret_cast<IdT*>(s_word);
+  uint32_t* s_val = reinterpret_cast<uint32_t*>(s_word);
 #pragma unroll
-  for (int r = 0; r < T::kRounds; ++r)
-    if (wave_base + r * kWave + lane < E) s_val[place[r]] = val[r];
+  for (int r = 0; r < kItemsHere; ++r) s_val[place[r]] = val[r];
   __syncthreads();
-  IdT* to = LAST ? last.value : val_out;
 #pragma unroll
-  for (int k = 0; k < T::kPerThread; ++k)
-    if (dst[k] >= 0) to[dst[k]] = s_val[k * kThreads + threadIdx.x];
+  for (int k = 0; k < kItemsHere; ++k) {
+    const int j = k * kThreadsHere + threadIdx.x;
+    if (j < n) {
+      const int64_t dst = s_base[out_digit[k]] + j;
+      if (LAST)
+        last.value[dst] = static_cast<IdT>(s_val[j]);
+      else
+        val_out[dst] = s_val[j];
+    }
+  }
+}
+
+// Behind the sort of 64-bit values: fetches them all again when one did not fit 32 bits.
+__global__ void __launch_bounds__(kThreads)
+widen_values_kernel(const int64_t* __restrict__ value, const int64_t* __restrict__ perm, int64_t E,
+                    const int* __restrict__ wide, int64_t* __restrict__ out) {
+  if (*wide == 0) return;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < E; i += stride)
+    out[i] = value[perm[i]];
 }
 
 int bits_for(int64_t n) {  // smallest b with 2^b >= n
@@ -540,30 +693,88 @@ indptr_split_kernel(const int64_t* __restrict__ indptr, const int64_t* __restric
   out[q] = indptr[begin + (q - begin - lo)] - indptr[begin];
 }
 
-template <typename IdT, typename Src>
-void launch_pass(Src src, bool last, bool self, dim3 grid, hipStream_t st, const IdT* vin, int64_t E,
-                 int shift, int64_t blocks, const int64_t* where, unsigned long long* wout,
-                 IdT* vout, const SortOutputs<IdT>& outs) {
+template <typename T, typename IdT, typename ValT, typename Src>
+void launch_pass(Src src, bool last, bool self, hipStream_t st, const ValT* vin, int64_t E, int shift,
+                 int64_t blocks, const int64_t* where, unsigned long long* wout, uint32_t* vout,
+                 const SortOutputs<IdT>& outs) {
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, st, src, vin, E, shift, blocks, where, wout,
-                       vout, outs);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(T::kThreadsPerTile), 0, st,
+                       src, vin, E, shift, blocks, where, wout, vout, outs);
   };
-  if (last && self) go(radix_pass_kernel<IdT, Src, true, true>);
-  else if (last) go(radix_pass_kernel<IdT, Src, true, false>);
-  else if (self) go(radix_pass_kernel<IdT, Src, false, true>);
-  else go(radix_pass_kernel<IdT, Src, false, false>);
+  if (last && self) go(radix_pass_kernel<T, IdT, ValT, Src, true, true>);
+  else if (last) go(radix_pass_kernel<T, IdT, ValT, Src, true, false>);
+  else if (self) go(radix_pass_kernel<T, IdT, ValT, Src, false, true>);
+  else go(radix_pass_kernel<T, IdT, ValT, Src, false, false>);
+}
+
+// the sort's scratch memory
+struct SortSpace {
+  unsigned long long* word[2];
+  uint32_t* value[2];
+  int64_t *counts, *offsets, *tiles;
+  uint32_t* keys;
+  int* wide;
+};
+// (tables sized for the smaller tile, which has the larger ones)
+inline size_t sort_space_bytes(int64_t E) {
+  const int64_t table = kRadix * static_cast<int64_t>(blocks_for(E, SmallTile::kSize));
+  const size_t n = static_cast<size_t>(E > 0 ? E : 1);
+  return 2 * padded(n * 8) + 3 * padded(n * 4) + padded(static_cast<size_t>(table) * 8) +
+         padded(static_cast<size_t>(table + 1) * 8) + scan_workspace_bytes(table) + 256;
+}
+inline bool carve_sort(Carver& ws, int64_t E, SortSpace* s) {
+  const int64_t table = kRadix * static_cast<int64_t>(blocks_for(E, SmallTile::kSize));
+  const size_t n = static_cast<size_t>(E > 0 ? E : 1);
+  for (auto& w : s->word) w = ws.take<unsigned long long>(n);
+  for (auto& v : s->value) v = ws.take<uint32_t>(n);
+  s->keys = ws.take<uint32_t>(n);
+  s->counts = ws.take<int64_t>(static_cast<size_t>(table));
+  s->offsets = ws.take<int64_t>(static_cast<size_t>(table + 1));
+  s->tiles = ws.take<int64_t>(static_cast<size_t>(scan_num_tiles(table) + 1));
+  s->wide = ws.take<int>(1);
+  return ws.ok;
+}
+
+template <typename T, typename IdT>
+int sort_passes(const IdT* key, const IdT* value, int64_t E, int passes, int idx_bits,
+                const SortSpace& s, const SortOutputs<IdT>& outs, hipStream_t st) {
+  const int64_t blocks = blocks_for(E, T::kSize);
+  const int64_t table = kRadix * blocks;
+  const dim3 grid(static_cast<unsigned>(blocks));
+  const bool self = blocks <= kSelfScanTiles;
+  const int64_t* where = self ? s.counts : s.offsets;
+  for (int p = 0; p < passes; ++p) {
+    const int shift = idx_bits + p * kRadixBits;
+    const bool last = p == passes - 1;
+    const FreshWords<IdT> fresh{key, idx_bits};
+    const StoredWords stored{s.word[(p + 1) & 1]};
+    if (p == 0)
+      hipLaunchKernelGGL((radix_hist_kernel<T, FreshWords<IdT>>), grid, dim3(T::kThreadsPerTile), 0,
+                         st, fresh, E, shift, blocks, s.counts, outs.wide);
+    else
+      hipLaunchKernelGGL((radix_hist_kernel<T, StoredWords>), grid, dim3(T::kThreadsPerTile), 0, st,
+                         stored, E, shift, blocks, s.counts, static_cast<int*>(nullptr));
+    if (!self) {
+      LoadI64 f{s.counts};
+      GS_RETURN_IF_ERROR(exclusive_scan(f, table, s.offsets, s.tiles, st));
+    }
+    if (p == 0)
+      launch_pass<T>(fresh, last, self, st, value, E, shift, blocks, where, s.word[0], s.value[0],
+                     outs);
+    else
+      launch_pass<T>(stored, last, self, st, static_cast<const uint32_t*>(s.value[(p + 1) & 1]), E,
+                     shift, blocks, where, s.word[p & 1], s.value[p & 1], outs);
+  }
+  return check_launch("coo2csc");
 }
 
 template <typename IdT>
 int coo2csc_impl(const IdT* key, const IdT* value, int64_t E, int64_t num_keys, int sorted,
                  int64_t* indptr, IdT* out_value, int64_t* perm, void* workspace,
                  size_t workspace_bytes, hipStream_t st) {
-  const dim3 ptr_grid(blocks_for(num_keys + 1, kPtrCols));
   if (E == 0 && !indptr) return GS_OK;
   if (sorted || E == 0) {
-    PlainKeys<IdT> keys{key};
-    hipLaunchKernelGGL((indptr_from_sorted_kernel<PlainKeys<IdT>>), ptr_grid, dim3(kThreads), 0, st,
-                       keys, E, num_keys, indptr);
+    launch_indptr(key, E, num_keys, indptr, st);
     return check_launch("coo2csc");
   }
   const int idx_bits = bits_for(E);
@@ -574,62 +785,174 @@ int coo2csc_impl(const IdT* key, const IdT* value, int64_t E, int64_t num_keys, 
                    static_cast<long long>(E), static_cast<long long>(num_keys));
     return GS_ERR_UNSUPPORTED;
   }
-  using T = SortTile<IdT>;
-  const int64_t blocks = blocks_for(E, T::kSize);
-  const int64_t table = kRadix * blocks;
   Carver ws(workspace, workspace_bytes);
-  unsigned long long* wbuf[2] = {ws.take<unsigned long long>(E), ws.take<unsigned long long>(E)};
-  IdT* vbuf[2] = {ws.take<IdT>(E), ws.take<IdT>(E)};
-  int64_t* counts = ws.take<int64_t>(table);
-  int64_t* offsets = ws.take<int64_t>(table + 1);
-  int64_t* tiles = ws.take<int64_t>(scan_num_tiles(table) + 1);
-  if (!ws.ok) {
+  SortSpace s;
+  if (!carve_sort(ws, E, &s)) {
     set_error_text("gs_coo2csc: workspace needs %zu bytes, 256-byte aligned",
                    gs_coo2csc_workspace_bytes(E, num_keys));
     return GS_ERR_WORKSPACE;
   }
-  // the sorted keys (for the offsets) land where the last pass would have put its words
-  IdT* sorted_keys = indptr ? reinterpret_cast<IdT*>(wbuf[(passes - 1) & 1]) : nullptr;
-  const SortOutputs<IdT> outs{out_value, perm, sorted_keys, idx_bits};
-  const dim3 grid(static_cast<unsigned>(blocks));
-  const unsigned long long* win = nullptr;  // null: the first pass reads the caller's keys
-  const IdT* vin = value;
-  for (int p = 0; p < passes; ++p) {
-    unsigned long long* wout = wbuf[p & 1];
-    IdT* vout = vbuf[p & 1];
-    const int shift = idx_bits + p * kRadixBits;
-    const bool last = p == passes - 1;
-    if (p == 0) {
-      FreshWords<IdT> src{key, idx_bits};
-      hipLaunchKernelGGL((radix_hist_kernel<FreshWords<IdT>, T::kSize>), grid, dim3(kThreads), 0, st,
-                         src, E, shift, blocks, counts);
-    } else {
-      StoredWords src{win};
-      hipLaunchKernelGGL((radix_hist_kernel<StoredWords, T::kSize>), grid, dim3(kThreads), 0, st, src,
-                         E, shift, blocks, counts);
-    }
-    const bool self = blocks <= kSelfScanTiles;
-    if (!self) {
-      LoadI64 f{counts};
-      GS_RETURN_IF_ERROR(exclusive_scan(f, table, offsets, tiles, st));
-    }
-    const int64_t* where = self ? counts : offsets;
-    if (p == 0) {
-      FreshWords<IdT> src{key, idx_bits};
-      launch_pass<IdT>(src, last, self, grid, st, vin, E, shift, blocks, where, wout, vout, outs);
-    } else {
-      StoredWords src{win};
-      launch_pass<IdT>(src, last, self, grid, st, vin, E, shift, blocks, where, wout, vout, outs);
-    }
-    win = wout;
-    vin = vout;
-  }
-  if (indptr) {  // (null: the caller wants the sorted order only)
-    PlainKeys<IdT> keys{sorted_keys};
-    hipLaunchKernelGGL((indptr_from_sorted_kernel<PlainKeys<IdT>>), ptr_grid, dim3(kThreads), 0, st,
-                       keys, E, num_keys, indptr);
-  }
+  const bool may_be_wide = sizeof(IdT) == 8;
+  const bool short_keys = passes * kRadixBits <= 32;
+  const SortOutputs<IdT> outs{out_value, perm, indptr && short_keys ? s.keys : nullptr, idx_bits,
+                              may_be_wide ? s.wide : nullptr};
+  if (E >= kLargeTileItems)
+    GS_RETURN_IF_ERROR((sort_passes<LargeTile, IdT>(key, value, E, passes, idx_bits, s, outs, st)));
+  else
+    GS_RETURN_IF_ERROR((sort_passes<SmallTile, IdT>(key, value, E, passes, idx_bits, s, outs, st)));
+  if (may_be_wide)
+    hipLaunchKernelGGL(widen_values_kernel, dim3(E < (int64_t(1) << 20) ? 64 : 1024), dim3(kThreads),
+                       0, st, reinterpret_cast<const int64_t*>(value), perm, E, s.wide,
+                       reinterpret_cast<int64_t*>(out_value));
+  if (indptr && short_keys)  // (null: the caller wants the sorted order only)
+    launch_indptr(static_cast<const uint32_t*>(s.keys), E, num_keys, indptr, st);
+  else if (indptr)
+    hipLaunchKernelGGL((indptr_from_sorted_kernel<PermutedKeys<IdT>>),
+                       dim3(blocks_for(num_keys + 1, kPtrCols)), dim3(kThreads), 0, st,
+                       PermutedKeys<IdT>{key, perm}, E, num_keys, indptr);
   return check_launch("coo2csc");
+}
+
+// -------------------------------------------------- distinct ids of an edge list ----
+// The larger number of different ids that the two ends of an edge list hold (the node count of
+// Graph::LoadCOO, reference src/graph.cc:25-35, which sorts both ends for it): a byte per
+// possible id, set by a plain store of every edge that finds it clear, then the bytes are
+// counted.  Ids run from zero in practice, so `range` bytes -- about one per edge -- hold
+// them; an id outside is reported and the caller counts another way.  The first end is
+// counted while the second is only looked through for its largest id: when the first holds
+// every id up to the largest of both, the second cannot hold more and its own count is left
+// out (any list with self loops).  What bounds the marking is one request to the L2 per edge.
+// 14 M edges, 64-bit ids: 0.22 ms where the two sorts took 1.79.
+constexpr int kMarkItems = 16;
+constexpr int kMarkTile = kThreads * kMarkItems;
+constexpr int kCountBlocks = 128;
+
+struct DistinctSpace {
+  unsigned char* map;  // range bytes for the first end, then for the second
+  int64_t* largest;    // per workgroup of the first marking launch; -1: an id outside the range
+  int64_t* partial;    // per workgroup of the counting launches
+  int64_t* first;      // {distinct ids of the first end, 1 when the second has to be counted}
+};
+
+__global__ void __launch_bounds__(kThreads) clear_marks_kernel(uint4* map, int64_t n) {
+  const int64_t i0 = static_cast<int64_t>(blockIdx.x) * (kThreads * 4) + threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (i0 + k * kThreads < n) map[i0 + k * kThreads] = make_uint4(0, 0, 0, 0);
+}
+
+// FIRST: workgroups with blockIdx.y 0 mark the ids of `a`, those with 1 look through `b`, all
+// leave their largest id.  Otherwise: the ids of `b`, when they have to be counted.
+template <typename IdT, bool FIRST>
+__global__ void __launch_bounds__(kThreads)
+mark_ids_kernel(const IdT* __restrict__ a, const IdT* __restrict__ b, int64_t E, int64_t range,
+                DistinctSpace s) {
+  __shared__ int64_t s_largest[kThreads / kWave];
+  if (!FIRST && !s.first[1]) return;
+  const bool marks = !FIRST || blockIdx.y == 0;
+  const IdT* __restrict__ ids = FIRST && marks ? a : b;
+  unsigned char* map = s.map + (FIRST ? 0 : range);
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * kMarkTile + threadIdx.x;
+  IdT id[kMarkItems];
+#pragma unroll
+  for (int k = 0; k < kMarkItems; ++k) {
+    const int64_t i = base + k * kThreads;
+    id[k] = ids[i < E ? i : E - 1];
+  }
+  // (an id below zero is a huge one here, and both are outside)
+  uint64_t largest = 0;
+#pragma unroll
+  for (int k = 0; k < kMarkItems; ++k) {
+    const uint64_t v = static_cast<uint64_t>(static_cast<int64_t>(id[k]));
+    largest = v > largest ? v : largest;
+  }
+  const uint64_t bound = static_cast<uint64_t>(range);
+  if (marks) {
+    uint32_t at[kMarkItems];
+    unsigned char seen[kMarkItems];
+#pragma unroll
+    for (int k = 0; k < kMarkItems; ++k) {
+      const uint64_t v = static_cast<uint64_t>(static_cast<int64_t>(id[k]));
+      at[k] = v < bound ? static_cast<uint32_t>(v) : ~0u;
+      seen[k] = map[v < bound ? v : 0];
+    }
+#pragma unroll
+    for (int k = 0; k < kMarkItems; ++k)
+      if (at[k] != ~0u && !seen[k]) map[at[k]] = 1;
+  }
+  if (!FIRST) return;
+  int64_t top = largest < bound ? static_cast<int64_t>(largest) : INT64_MAX;
+#pragma unroll
+  for (int d = kWave / 2; d > 0; d >>= 1) {
+    const int64_t o = __shfl_xor(top, d, kWave);
+    top = o > top ? o : top;
+  }
+  if ((threadIdx.x & (kWave - 1)) == 0) s_largest[threadIdx.x / kWave] = top;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kThreads / kWave; ++w) top = s_largest[w] > top ? s_largest[w] : top;
+    s.largest[static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x] = top;
+  }
+}
+
+// marked bytes of one end (every byte is 0 or 1)
+template <bool FIRST>
+__global__ void __launch_bounds__(kThreads) count_marks_kernel(DistinctSpace s, int64_t range) {
+  __shared__ int64_t lds[kThreads / kWave + 1];
+  if (!FIRST && !s.first[1]) return;
+  const uint4* map = reinterpret_cast<const uint4*>(s.map + (FIRST ? 0 : range));
+  int64_t n = 0;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < range / 16;
+       i += static_cast<int64_t>(kCountBlocks) * kThreads) {
+    const uint4 v = map[i];
+    n += __popc(v.x) + __popc(v.y) + __popc(v.z) + __popc(v.w);
+  }
+  int64_t total;
+  block_exclusive_scan<kThreads>(n, &total, lds);
+  if (threadIdx.x == 0) s.partial[blockIdx.x] = total;
+}
+
+// after the first end: is the second to be counted?  (one workgroup)
+constexpr int kDecideThreads = 1024;
+__global__ void __launch_bounds__(kDecideThreads)
+decide_second_kernel(DistinctSpace s, int64_t num_largest) {
+  __shared__ int64_t lds[kDecideThreads / kWave + 1];
+  __shared__ int64_t s_top[kDecideThreads / kWave];
+  int64_t top = 0;
+  for (int64_t i = threadIdx.x; i < num_largest; i += kDecideThreads)
+    top = s.largest[i] > top ? s.largest[i] : top;
+#pragma unroll
+  for (int d = kWave / 2; d > 0; d >>= 1) {
+    const int64_t o = __shfl_xor(top, d, kWave);
+    top = o > top ? o : top;
+  }
+  if ((threadIdx.x & (kWave - 1)) == 0) s_top[threadIdx.x / kWave] = top;
+  int64_t total;
+  block_exclusive_scan<kDecideThreads>(threadIdx.x < kCountBlocks ? s.partial[threadIdx.x] : 0,
+                                       &total, lds);
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kDecideThreads / kWave; ++w) top = s_top[w] > top ? s_top[w] : top;
+    const bool outside = top == INT64_MAX;
+    s.first[0] = outside ? -1 : total;
+    s.first[1] = !outside && total <= top;  // (total = top + 1: every id up to the largest is there)
+  }
+}
+
+__global__ void __launch_bounds__(kThreads)
+post_distinct_kernel(DistinctSpace s, gs_mailbox* box, int64_t ticket) {
+  __shared__ int64_t lds[kThreads / kWave + 1];
+  int64_t second = 0;
+  const bool counted = s.first[1] != 0;
+  block_exclusive_scan<kThreads>(counted && threadIdx.x < kCountBlocks ? s.partial[threadIdx.x] : 0,
+                                 &second, lds);
+  // (-1, an id outside the range, leaves the second end uncounted)
+  if (threadIdx.x == 0) post_mailbox(box, counted && second > s.first[0] ? second : s.first[0], ticket);
+}
+
+// bytes per end of the list, a multiple of 16; ids of a graph with up to a million nodes always fit
+inline int64_t mark_range(int64_t E) {
+  const int64_t n = E > (int64_t(1) << 20) ? E : (int64_t(1) << 20);
+  return (n + 4095) / 4096 * 4096;
 }
 
 // ---------------------------------------------------- binned scatter-add ----
@@ -648,7 +971,7 @@ constexpr int64_t kBinPartItems = 16384;  // edges a workgroup takes before a ru
 constexpr int kBinMaxShift = 15;         // 2^15 sums = 128 KB of LDS
 
 __global__ void __launch_bounds__(kBinThreads)
-bin_sum_kernel(const unsigned long long* __restrict__ words, const int32_t* __restrict__ vals,
+bin_sum_kernel(const unsigned long long* __restrict__ words, const uint32_t* __restrict__ vals,
                const int64_t* __restrict__ offsets, int64_t num_blocks, int num_bins, int idx_bits,
                int bin_shift, int powk, int64_t num_targets, float* __restrict__ out) {
   extern __shared__ float s_sum[];
@@ -692,7 +1015,7 @@ bin_sum_kernel(const unsigned long long* __restrict__ words, const int32_t* __re
   constexpr int kBatch = 8;
   for (int64_t i0 = begin + threadIdx.x; i0 < end; i0 += kBinThreads * kBatch) {
     unsigned long long w[kBatch];
-    int v[kBatch];
+    uint32_t v[kBatch];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       const int64_t i = i0 + u * kBinThreads;
@@ -708,7 +1031,7 @@ bin_sum_kernel(const unsigned long long* __restrict__ words, const int32_t* __re
       const int64_t t = static_cast<int64_t>(w[u] >> idx_bits) - first;
       // (a target beyond num_targets has no sum to go to: left out, as out has no room for it)
       if (i0 + u * kBinThreads < end && t >= 0 && t < width)
-        atomicAdd(&s_sum[t], powk_f(__int_as_float(v[u]), powk));
+        atomicAdd(&s_sum[t], powk_f(__uint_as_float(v[u]), powk));
     }
   }
   __syncthreads();
@@ -746,12 +1069,12 @@ inline bool bin_sum_applies(int id_bytes, const int64_t* e_ids, int64_t E, int64
 
 int bin_sum_impl(const int32_t* target, const float* data, int64_t E, int powk, int64_t num_targets,
                  float* out, void* workspace, size_t workspace_bytes, hipStream_t st) {
-  using T = SortTile<int32_t>;
+  using T = SmallTile;
   const int64_t blocks = blocks_for(E, T::kSize);
   const int64_t table = kRadix * blocks;
   Carver ws(workspace, workspace_bytes);
   unsigned long long* words = ws.take<unsigned long long>(E);
-  int32_t* vals = ws.take<int32_t>(E);
+  uint32_t* vals = ws.take<uint32_t>(E);
   int64_t* counts = ws.take<int64_t>(table);
   int64_t* offsets = ws.take<int64_t>(table + 1);
   int64_t* tiles = ws.take<int64_t>(scan_num_tiles(table) + 1);
@@ -766,13 +1089,13 @@ int bin_sum_impl(const int32_t* target, const float* data, int64_t E, int powk, 
   const int shift = idx_bits + bin_shift;
   const dim3 grid(static_cast<unsigned>(blocks));
   FreshWords<int32_t> src{target, idx_bits};
-  hipLaunchKernelGGL((radix_hist_kernel<FreshWords<int32_t>, T::kSize>), grid, dim3(kThreads), 0, st,
-                     src, E, shift, blocks, counts);
+  hipLaunchKernelGGL((radix_hist_kernel<T, FreshWords<int32_t>>), grid, dim3(T::kThreadsPerTile), 0,
+                     st, src, E, shift, blocks, counts, static_cast<int*>(nullptr));
   LoadI64 f{counts};
   GS_RETURN_IF_ERROR(exclusive_scan(f, table, offsets, tiles, st));
-  const SortOutputs<int32_t> none{nullptr, nullptr, nullptr, idx_bits};
-  launch_pass<int32_t>(src, false, false, grid, st, reinterpret_cast<const int32_t*>(data), E, shift,
-                       blocks, offsets, words, vals, none);
+  const SortOutputs<int32_t> none{nullptr, nullptr, nullptr, idx_bits, nullptr};
+  launch_pass<T>(src, false, false, st, reinterpret_cast<const uint32_t*>(data), E, shift, blocks,
+                 offsets, words, vals, none);
   const int bins = static_cast<int>(((num_targets - 1) >> bin_shift) + 1);
   // (per call: the attribute belongs to the device the call runs on)
   const hipError_t lds_allowed = hipFuncSetAttribute(
@@ -863,14 +1186,53 @@ int gs_csc_compress(const int64_t* indptr, int64_t num_cols, int id_bytes, void*
 size_t gs_coo2csc_workspace_bytes(int64_t E, int64_t num_keys) {
   (void)num_keys;
   if (E < 0) E = 0;
-  // sized for the smaller tile (8-byte ids), which has the larger table
-  const int64_t blocks = blocks_for(E, SortTile<int64_t>::kSize);
-  const int64_t table = kRadix * blocks;
-  const size_t n = static_cast<size_t>(E > 0 ? E : 1);
-  return 2 * padded(n * 8) +  // the sort's words, ping-pong
-         2 * padded(n * 8) +  // the values riding along, ping-pong
-         padded(static_cast<size_t>(table) * 8) + padded(static_cast<size_t>(table + 1) * 8) +
-         scan_workspace_bytes(table);
+  return sort_space_bytes(E);
+}
+
+size_t gs_distinct_ends_workspace_bytes(int64_t E) {
+  if (E < 0) E = 0;
+  return padded(2 * static_cast<size_t>(mark_range(E))) +
+         padded(2 * static_cast<size_t>(blocks_for(E, kMarkTile)) * 8) + padded(kCountBlocks * 8) + 256;
+}
+
+int gs_distinct_ends(const void* a, const void* b, int id_bytes, int64_t E, void* workspace,
+                     size_t workspace_bytes, gs_mailbox* mailbox, int64_t ticket, void* stream) {
+  GS_REQUIRE(E > 0 && E < (int64_t(1) << 32) - 8192 && a && b && mailbox,
+             "gs_distinct_ends: bad argument");
+  GS_REQUIRE(valid_id_bytes(id_bytes), "gs_distinct_ends: id_bytes must be 4 or 8, got %d", id_bytes);
+  const int64_t range = mark_range(E);
+  const int blocks = blocks_for(E, kMarkTile);
+  Carver ws(workspace, workspace_bytes);
+  DistinctSpace s;
+  s.map = ws.take<unsigned char>(static_cast<size_t>(2 * range));
+  s.largest = ws.take<int64_t>(2 * static_cast<size_t>(blocks));
+  s.partial = ws.take<int64_t>(kCountBlocks);
+  s.first = ws.take<int64_t>(2);
+  if (!ws.ok) {
+    set_error_text("gs_distinct_ends: workspace needs %zu bytes, 256-byte aligned",
+                   gs_distinct_ends_workspace_bytes(E));
+    return GS_ERR_WORKSPACE;
+  }
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int64_t vecs = 2 * range / 16;
+  hipLaunchKernelGGL(clear_marks_kernel, dim3(blocks_for(vecs, kThreads * 4)), dim3(kThreads), 0, st,
+                     reinterpret_cast<uint4*>(s.map), vecs);
+  auto both = [&](auto first, auto second, auto* pa, auto* pb) {
+    hipLaunchKernelGGL(first, dim3(blocks, 2), dim3(kThreads), 0, st, pa, pb, E, range, s);
+    hipLaunchKernelGGL(count_marks_kernel<true>, dim3(kCountBlocks), dim3(kThreads), 0, st, s, range);
+    hipLaunchKernelGGL(decide_second_kernel, dim3(1), dim3(kDecideThreads), 0, st, s,
+                       static_cast<int64_t>(2) * blocks);
+    hipLaunchKernelGGL(second, dim3(blocks), dim3(kThreads), 0, st, pa, pb, E, range, s);
+    hipLaunchKernelGGL(count_marks_kernel<false>, dim3(kCountBlocks), dim3(kThreads), 0, st, s, range);
+  };
+  if (id_bytes == 8)
+    both(mark_ids_kernel<int64_t, true>, mark_ids_kernel<int64_t, false>,
+         static_cast<const int64_t*>(a), static_cast<const int64_t*>(b));
+  else
+    both(mark_ids_kernel<int32_t, true>, mark_ids_kernel<int32_t, false>,
+         static_cast<const int32_t*>(a), static_cast<const int32_t*>(b));
+  hipLaunchKernelGGL(post_distinct_kernel, dim3(1), dim3(kThreads), 0, st, s, mailbox, ticket);
+  return check_launch("distinct_ends");
 }
 
 int gs_coo2csc(const void* key, const void* value, int id_bytes, int64_t E, int64_t num_keys,
@@ -914,7 +1276,7 @@ int gs_indptr_split_cuts(const int64_t* indptr, const int64_t* offsets, int64_t 
 size_t gs_coo_sum_workspace_bytes(int64_t E, int64_t num_targets) {
   if (E < 0) E = 0;
   if (!bin_sum_applies(4, nullptr, E, num_targets)) return 256;
-  const int64_t blocks = blocks_for(E, SortTile<int32_t>::kSize);
+  const int64_t blocks = blocks_for(E, SmallTile::kSize);
   const int64_t table = kRadix * blocks;
   return padded(static_cast<size_t>(E) * 8) + padded(static_cast<size_t>(E) * 4) +
          padded(static_cast<size_t>(table) * 8) + padded(static_cast<size_t>(table + 1) * 8) +

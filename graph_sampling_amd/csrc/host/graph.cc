@@ -36,9 +36,10 @@ void Graph::LoadCSR(torch::Tensor indptr, torch::Tensor indices) {
 // node count = the larger number of distinct endpoints (reference src/graph.cc:25-35)
 void Graph::LoadCOO(torch::Tensor row, torch::Tensor col) {
   coo_ = std::make_shared<COO>(COO{row, col, torch::nullopt, false, false});
-  const int64_t nr = std::get<0>(torch::_unique(row)).numel();
-  const int64_t nc = std::get<0>(torch::_unique(col)).numel();
-  num_cols_ = num_rows_ = std::max(nr, nc);
+  int64_t nodes = hip::DistinctEnds(row, col);
+  if (nodes < 0)
+    nodes = std::max(std::get<0>(torch::_unique(row)).numel(), std::get<0>(torch::_unique(col)).numel());
+  num_cols_ = num_rows_ = nodes;
   num_edges_ = row.numel();
 }
 

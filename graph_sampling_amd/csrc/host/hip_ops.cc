@@ -1344,6 +1344,22 @@ std::tuple<torch::Tensor, torch::Tensor, torch::optional<torch::Tensor>> Coo2Csc
   return {indptr, out_value, perm};
 }
 
+int64_t DistinctEnds(const torch::Tensor& a, const torch::Tensor& b) {
+  const int idb = a.scalar_type() == torch::kInt64 ? 8 : a.scalar_type() == torch::kInt32 ? 4 : 0;
+  const int64_t E = a.numel();
+  if (!idb || E == 0 || E >= (int64_t(1) << 31) || b.scalar_type() != a.scalar_type() || b.numel() != E || !a.is_cuda() ||
+      a.device() != b.device() || !a.is_contiguous() || !b.is_contiguous())
+    return -1;
+  auto ws = Scratch(gs_distinct_ends_workspace_bytes(E), a);
+  void* st = Stream(a);
+  HostBoxes& boxes = Boxes(a.get_device());
+  const int64_t ticket = boxes.next++;
+  Check(gs_distinct_ends(a.data_ptr(), b.data_ptr(), idb, E, ws.data_ptr(), ws.numel(),
+                         boxes.slot(ticket), ticket, st),
+        "gs_distinct_ends");
+  return WaitBox(boxes.slot(ticket), ticket, st, "gs_distinct_ends");
+}
+
 std::tuple<torch::Tensor, torch::Tensor> SortValuesByKey(const torch::Tensor& key,
                                                          const torch::Tensor& value,
                                                          int64_t num_keys) {

@@ -275,6 +275,10 @@ torch::Tensor Csc2CooCols(const torch::Tensor& indptr, int64_t nnz, const torch:
 std::tuple<torch::Tensor, torch::Tensor, torch::optional<torch::Tensor>> Coo2Csc(
     const torch::Tensor& key, const torch::Tensor& value, int64_t num_keys, bool sorted);
 
+// the larger number of distinct ids among the two ends of an edge list; negative when the
+// library's count does not apply (no device tensors, no edges, an id far beyond their number)
+int64_t DistinctEnds(const torch::Tensor& a, const torch::Tensor& b);
+
 // {`value` in the stable order of `key` (keys below num_keys), the permutation}: the
 // library's radix sort alone, no offsets built
 std::tuple<torch::Tensor, torch::Tensor> SortValuesByKey(const torch::Tensor& key,

@@ -776,6 +776,15 @@ int gs_coo_block_values(const void* kept_key, const void* kept_pos, int64_t kept
 int gs_csc2coo(const int64_t* indptr, int64_t num_cols, int64_t nnz, void* col, int id_bytes,
                void* stream);
 
+/* How many distinct ids each of the two ends a[0..E), b[0..E) of an edge list holds, the larger
+ * of the two posted to the mailbox (what Graph::LoadCOO takes for the node count,
+ * src/graph.cc:25-35).  Ids from 0 up to about the number of edges (a million at the least)
+ * are counted; when one lies outside, -1 is posted and the caller counts another way.
+ * workspace: gs_distinct_ends_workspace_bytes(E) bytes, 256-byte aligned. */
+size_t gs_distinct_ends_workspace_bytes(int64_t E);
+int gs_distinct_ends(const void* a, const void* b, int id_bytes, int64_t E, void* workspace,
+                     size_t workspace_bytes, gs_mailbox* mailbox, int64_t ticket, void* stream);
+
 /* Doubly-compressed CSC (only the columns that own an edge are stored; ids[c] names stored
  * column c).  gs_dcsc2coo: col[e] = ids[column owning e], replaces impl::DCSC2COOCUDA
  * (src/cuda/format_transform.cu:48).  gs_csc_compress: CSC -> DCSC, the second half of

@@ -1,0 +1,63 @@
+"""Edge lists: the node count of a loaded COO, the sort's large tiles, offsets over gaps of ids."""
+import numpy as np
+import pytest
+import torch
+
+import graph_sampling_amd as gs
+from graph_sampling_amd import capi
+from util import to_dev
+
+pytestmark = pytest.mark.gpu
+ID_DTYPES = [torch.int32, torch.int64]
+
+
+@pytest.mark.parametrize("idt", ID_DTYPES)
+@pytest.mark.parametrize("E", [1, 4095, 4096, 4097, 70000])
+@pytest.mark.parametrize("how", ["complete", "second_larger", "first_larger", "huge", "negative"])
+def test_node_count_of_an_edge_list(dev, E, how, idt):
+    rng = np.random.default_rng(E)
+    row, col = rng.integers(0, max(1, E // 3), E), rng.integers(0, max(1, E // 3), E)
+    if how == "complete":          # the first end holds every id: the second is not counted
+        row = np.arange(E) % (E // 3 + 1)
+    elif how == "second_larger":   # gaps in both, the second end with more ids
+        row, col = (row // 7) * 7, (col // 2) * 2
+    elif how == "first_larger":
+        row, col = (row // 2) * 2, (col // 7) * 7
+    elif how == "huge":            # an id far beyond the number of edges: counted another way
+        col[E // 2] = (1 << 31) - 1
+    else:
+        row[E // 2] = -1
+    g = gs.Graph(False)
+    g._CAPI_LoadCOO(to_dev(row, dev, idt), to_dev(col, dev, idt))
+    assert g._CAPI_GetNumRows() == max(np.unique(row).size, np.unique(col).size)
+
+
+@pytest.mark.parametrize("idt", ID_DTYPES)
+@pytest.mark.parametrize("extra", [0, 1, 8191])
+@pytest.mark.parametrize("num_keys", [200, 60_000, 3_000_000])
+def test_sort_with_large_tiles(dev, num_keys, extra, idt):
+    E = (1 << 22) + extra
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(num_keys + extra)
+    key = (torch.rand(E, generator=gen, device=dev) ** 3 * num_keys).to(idt)
+    value = torch.randint(0, 1 << 31, (E,), generator=gen, device=dev).to(idt)
+    if idt == torch.int64 and extra == 1:
+        value[E // 2] = 1 << 40    # one value beyond 32 bits
+    ip, val, perm = capi.coo2csc(key, value, num_keys, False)
+    want = torch.sort(key, stable=True)
+    assert torch.equal(perm, want.indices) and torch.equal(val, value[want.indices])
+    ends = torch.cumsum(torch.bincount(key.long(), minlength=num_keys), 0)
+    assert int(ip[0]) == 0 and torch.equal(ip[1:], ends)
+
+
+@pytest.mark.parametrize("idt", ID_DTYPES)
+@pytest.mark.parametrize("keys", [[0], [9999], [0, 17, 18, 9000], [5000, 5016, 5032, 7200, 9998]])
+def test_offsets_over_gaps(dev, keys, idt):
+    """Sorted keys, more edges than columns, gaps on both sides of the lengths one lane, a wave
+    and a workgroup fill, at the front, in between and at the end."""
+    num_keys, E = 10_000, 12_289
+    rng = np.random.default_rng(len(keys))
+    key = np.sort(rng.choice(np.array(keys), E))
+    ip, _, _ = capi.coo2csc(to_dev(key, dev, idt), to_dev(key, dev, idt), num_keys, True)
+    want = np.concatenate([[0], np.cumsum(np.bincount(key, minlength=num_keys))])
+    assert np.array_equal(ip.cpu().numpy(), want)
