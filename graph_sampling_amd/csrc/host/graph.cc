@@ -766,7 +766,19 @@ c10::intrusive_ptr<Graph> Graph::FusedBidirSlicing(torch::Tensor column_seeds,
   CreateSparseFormat(_CSC);
   auto ret = Child(Pick(col_ids_, column_seeds), Pick(row_ids_, row_seeds), column_seeds.numel(),
                    row_seeds.numel());
-  std::shared_ptr<CSC> sliced;
+  auto sliced = std::make_shared<CSC>();
+  if (!data_.has_value() || hip::EdgeData::Fits(data_.value(), csc_->e_ids)) {
+    // the edges' data, if there are any, come along in the slice's own passes
+    const hip::EdgeData edge{data_.value_or(torch::Tensor()), csc_->e_ids};
+    torch::Tensor data;
+    std::tie(sliced->indptr, sliced->indices) =
+        hip::InducedSlicing(csc_->indptr, csc_->indices, column_seeds, row_seeds, num_rows_,
+                            data_.has_value() ? &edge : nullptr, &data);
+    ret->SetCSC(sliced);
+    ret->SetNumEdges(sliced->indices.numel());
+    if (data_.has_value()) ret->SetData(data);
+    return ret;
+  }
   torch::Tensor select_index, parent_index;
   std::tie(sliced, select_index) =
       FusedCSCColRowSlicing(csc_, column_seeds, row_seeds, &parent_index);

@@ -1231,32 +1231,30 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> RowSlicingCoo(
   return {out_key, out_other, select_index};
 }
 
-std::tuple<torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor> ColRowSlicing(
-    const torch::Tensor& indptr, const torch::Tensor& indices, const torch::Tensor& column_ids,
-    const torch::Tensor& row_ids, const torch::optional<torch::Tensor>& col_ptr,
-    const torch::optional<torch::Tensor>& row_ptr, int64_t encoding_size) {
-  NeedI64(indptr, "indptr");
-  const int idb = IdBytes(indices, "indices");
-  TORCH_CHECK(IdBytes(column_ids, "column ids") == idb && IdBytes(row_ids, "row ids") == idb,
-              "column ids, row ids and indices differ in dtype");
-  const int64_t S = column_ids.numel(), nr = row_ids.numel(), ncols = indptr.numel() - 1;
-  const bool batched = col_ptr.has_value();
-  TORCH_CHECK(batched == row_ptr.has_value(), "column and row batch offsets come together");
-  int64_t B = 0;
-  if (batched) {
-    B = col_ptr.value().numel() - 1;
-    TORCH_CHECK(row_ptr.value().numel() == B + 1, "column and row batch offsets differ in length");
-    TORCH_CHECK(encoding_size > 0, "a batched slice needs a positive encoding size");
-  }
-  void* st = Stream(indptr);
+namespace {
+
+// offsets of the column slice and its number of edges (the host waits for it)
+std::tuple<torch::Tensor, int64_t> SliceOffsets(const torch::Tensor& indptr,
+                                                const torch::Tensor& column_ids, int idb) {
+  const int64_t S = column_ids.numel();
   auto sub_indptr = torch::empty({S + 1}, I64(indptr));
-  {
-    auto ws = Scratch(gs_slice_workspace_bytes(S), indptr);
-    Check(gs_slice_count(indptr.data_ptr<int64_t>(), ncols, column_ids.data_ptr(), idb, S,
-                         sub_indptr.data_ptr<int64_t>(), ws.data_ptr(), ws.numel(), st),
-          "gs_slice_count");
-  }
-  const int64_t D = ReadTotal(sub_indptr, S, Stream(sub_indptr), "total");
+  auto ws = Scratch(gs_slice_workspace_bytes(S), indptr);
+  void* st = Stream(indptr);
+  Check(gs_slice_count(indptr.data_ptr<int64_t>(), indptr.numel() - 1, column_ids.data_ptr(), idb, S,
+                       sub_indptr.data_ptr<int64_t>(), ws.data_ptr(), ws.numel(), st),
+        "gs_slice_count");
+  return {sub_indptr, ReadTotal(sub_indptr, S, st, "total")};
+}
+
+// the general column + row slice behind those offsets; index arrays nobody asks for stay undefined
+std::tuple<torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor> ColRowSliceOf(
+    const torch::Tensor& indptr, const torch::Tensor& indices, const torch::Tensor& column_ids,
+    const torch::Tensor& row_ids, const torch::Tensor& sub_indptr, int64_t D,
+    const torch::optional<torch::Tensor>& col_ptr, const torch::optional<torch::Tensor>& row_ptr,
+    int64_t B, int64_t encoding_size, bool with_select, bool with_parent) {
+  const int idb = IdBytes(indices, "indices");
+  const int64_t S = column_ids.numel(), nr = row_ids.numel(), ncols = indptr.numel() - 1;
+  void* st = Stream(indptr);
   auto out_indptr = torch::empty({S + 1}, I64(indptr));
   auto ws = Scratch(gs_col_row_slice_workspace_bytes(nr, D), indptr);
   Check(gs_col_row_slice_mark(indptr.data_ptr<int64_t>(), ncols, indices.data_ptr(), idb,
@@ -1267,13 +1265,90 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor> ColRowSli
         "gs_col_row_slice_mark");
   const int64_t kept = ReadTotal(out_indptr, S, Stream(out_indptr), "total");
   auto out_indices = torch::empty({kept}, indices.options());
-  auto select_index = torch::empty({kept}, I64(indptr));
-  auto parent_index = torch::empty({kept}, I64(indptr));
+  torch::Tensor select_index, parent_index;
+  if (with_select) select_index = torch::empty({kept}, I64(indptr));
+  if (with_parent) parent_index = torch::empty({kept}, I64(indptr));
   if (kept > 0)
-    Check(gs_col_row_slice_compact(D, idb, out_indices.data_ptr(), select_index.data_ptr<int64_t>(),
-                                   parent_index.data_ptr<int64_t>(), ws.data_ptr(), ws.numel(), st),
+    Check(gs_col_row_slice_compact(D, idb, out_indices.data_ptr(),
+                                   with_select ? select_index.data_ptr<int64_t>() : nullptr,
+                                   with_parent ? parent_index.data_ptr<int64_t>() : nullptr,
+                                   ws.data_ptr(), ws.numel(), st),
           "gs_col_row_slice_compact");
   return {out_indptr, out_indices, select_index, parent_index};
+}
+
+}  // namespace
+
+std::tuple<torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor> ColRowSlicing(
+    const torch::Tensor& indptr, const torch::Tensor& indices, const torch::Tensor& column_ids,
+    const torch::Tensor& row_ids, const torch::optional<torch::Tensor>& col_ptr,
+    const torch::optional<torch::Tensor>& row_ptr, int64_t encoding_size) {
+  NeedI64(indptr, "indptr");
+  const int idb = IdBytes(indices, "indices");
+  TORCH_CHECK(IdBytes(column_ids, "column ids") == idb && IdBytes(row_ids, "row ids") == idb,
+              "column ids, row ids and indices differ in dtype");
+  const bool batched = col_ptr.has_value();
+  TORCH_CHECK(batched == row_ptr.has_value(), "column and row batch offsets come together");
+  int64_t B = 0;
+  if (batched) {
+    B = col_ptr.value().numel() - 1;
+    TORCH_CHECK(row_ptr.value().numel() == B + 1, "column and row batch offsets differ in length");
+    TORCH_CHECK(encoding_size > 0, "a batched slice needs a positive encoding size");
+  }
+  torch::Tensor sub_indptr;
+  int64_t D;
+  std::tie(sub_indptr, D) = SliceOffsets(indptr, column_ids, idb);
+  return ColRowSliceOf(indptr, indices, column_ids, row_ids, sub_indptr, D, col_ptr, row_ptr, B,
+                       encoding_size, true, true);
+}
+
+std::tuple<torch::Tensor, torch::Tensor> InducedSlicing(const torch::Tensor& indptr,
+                                                        const torch::Tensor& indices,
+                                                        const torch::Tensor& column_ids,
+                                                        const torch::Tensor& row_ids,
+                                                        int64_t num_rows, const EdgeData* edge,
+                                                        torch::Tensor* data_out) {
+  NeedI64(indptr, "indptr");
+  const int idb = IdBytes(indices, "indices");
+  TORCH_CHECK(IdBytes(column_ids, "column ids") == idb && IdBytes(row_ids, "row ids") == idb,
+              "column ids, row ids and indices differ in dtype");
+  if (edge) TORCH_CHECK(EdgeData::Fits(edge->data, edge->e_ids), "edge data the slice cannot read");
+  const int64_t S = column_ids.numel(), nr = row_ids.numel(), nnz = indices.numel();
+  torch::Tensor sub_indptr;
+  int64_t D;
+  std::tie(sub_indptr, D) = SliceOffsets(indptr, column_ids, idb);
+  if (!gs_induced_slice_applies(nr, S, D, nnz)) {
+    auto r = ColRowSliceOf(indptr, indices, column_ids, row_ids, sub_indptr, D, torch::nullopt,
+                           torch::nullopt, 0, 0, false, edge != nullptr);
+    if (edge) {
+      const torch::Tensor& at = std::get<3>(r);
+      *data_out = edge->data.index({edge->e_ids.has_value() ? edge->e_ids.value().index({at}) : at});
+    }
+    return {std::get<0>(r), std::get<1>(r)};
+  }
+  void* st = Stream(indptr);
+  auto out_indptr = torch::empty({S + 1}, I64(indptr));
+  auto ws = Scratch(gs_induced_slice_workspace_bytes(D, edge != nullptr), indptr);
+  int64_t kept = -1;
+  for (int64_t bound : {num_rows, int64_t(0)}) {  // (again without a bound when an id reaches it)
+    Check(gs_induced_slice_mark(indptr.data_ptr<int64_t>(), indptr.numel() - 1, indices.data_ptr(),
+                                nnz, bound, idb, column_ids.data_ptr(), S,
+                                sub_indptr.data_ptr<int64_t>(), D, row_ids.data_ptr(), nr,
+                                edge ? edge->data.data_ptr<float>() : nullptr,
+                                edge ? OptI64(edge->e_ids, "e_ids") : nullptr,
+                                out_indptr.data_ptr<int64_t>(), ws.data_ptr(), ws.numel(), st),
+          "gs_induced_slice_mark");
+    kept = ReadTotal(out_indptr, S, st, "total");
+    if (kept >= 0) break;
+  }
+  auto out_indices = torch::empty({kept}, indices.options());
+  if (edge) *data_out = torch::empty({kept}, edge->data.options());
+  if (kept > 0)
+    Check(gs_induced_slice_compact(D, idb, out_indices.data_ptr(),
+                                   edge ? data_out->data_ptr<float>() : nullptr, ws.data_ptr(),
+                                   ws.numel(), st),
+          "gs_induced_slice_compact");
+  return {out_indptr, out_indices};
 }
 
 SliceResult DcscColSlicing(const torch::Tensor& indptr, const torch::Tensor& indices,

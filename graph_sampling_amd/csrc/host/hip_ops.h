@@ -258,6 +258,15 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor> ColRowSli
     const torch::Tensor& row_ids, const torch::optional<torch::Tensor>& col_ptr = torch::nullopt,
     const torch::optional<torch::Tensor>& row_ptr = torch::nullopt, int64_t encoding_size = 0);
 
+// The same without batches for a caller that wants the kept edges and, with `edge`, their data in
+// *data_out: {out_indptr, out_indices}.  num_rows: row ids are expected below it.
+std::tuple<torch::Tensor, torch::Tensor> InducedSlicing(const torch::Tensor& indptr,
+                                                        const torch::Tensor& indices,
+                                                        const torch::Tensor& column_ids,
+                                                        const torch::Tensor& row_ids,
+                                                        int64_t num_rows, const EdgeData* edge,
+                                                        torch::Tensor* data_out);
+
 // ---- doubly-compressed formats (only the non-empty columns are stored; ids name them)
 // column slice of a DCSC: a requested column that is not stored is an empty column
 SliceResult DcscColSlicing(const torch::Tensor& indptr, const torch::Tensor& indices,

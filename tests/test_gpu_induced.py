@@ -1,0 +1,72 @@
+"""Induced subgraphs of a node set that fits a compute unit's LDS, against the oracle: set sizes
+around the limits, duplicate nodes, tiles with one column and with thousands, edge data."""
+import numpy as np
+import pytest
+import torch
+
+import graph_sampling_amd as gs
+from oracle import oracle as O
+from util import to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def _graph(n, hubs, hub_degree, small, seed, wide=False):
+    """n columns: `hubs` of them hub_degree edges long, the others 0 .. small edges."""
+    rng = np.random.default_rng(seed)
+    degree = rng.integers(0, small + 1, n)
+    degree[rng.permutation(n)[:hubs]] = hub_degree
+    indptr = np.concatenate([[0], np.cumsum(degree)]).astype(np.int64)
+    indices = rng.integers(0, n, indptr[-1]).astype(np.int64)
+    if wide:  # ids that agree in their low 32 bits
+        indices[::3] += 1 << 40
+    return indptr, indices, rng
+
+
+@pytest.mark.parametrize("idt", [torch.int32, torch.int64])
+@pytest.mark.parametrize("n_ids", [1, 300, 8192, 8193, 16383, 16384])
+@pytest.mark.parametrize("weights", [False, True])
+def test_set_sizes(dev, n_ids, weights, idt):
+    indptr, indices, rng = _graph(30_000, 40, 90_001, 60, n_ids)
+    wide = idt == torch.int64 and n_ids == 300
+    if wide:
+        indptr, indices, rng = _graph(30_000, 40, 90_001, 60, n_ids, wide=True)
+    cols = rng.integers(0, 30_000, 20_000).astype(np.int64)
+    rows = rng.integers(0, 30_000, n_ids).astype(np.int64)      # (some ids twice)
+    if wide:
+        rows[::2] += 1 << 40
+    g = gs.Graph(False)
+    g._CAPI_LoadCSC(to_dev(indptr, dev), to_dev(indices, dev, idt))
+    if weights:
+        w = rng.random(indices.size).astype(np.float32)
+        g._CAPI_SetData(to_dev(w, dev))
+    sub = g._CAPI_FusionSlicing(to_dev(cols, dev, idt), to_dev(rows, dev, idt))
+    ptr, idx, _ = sub._CAPI_GetCSC()
+    want = O.col_row_slice(indptr, indices, cols, rows)
+    assert idx.dtype == idt
+    assert np.array_equal(ptr.cpu().numpy(), want[0])
+    assert np.array_equal(idx.cpu().numpy(), want[1])
+    if weights:
+        assert np.array_equal(sub._CAPI_GetData("default").cpu().numpy(), w[want[3]])
+
+
+@pytest.mark.parametrize("hubs,hub_degree,small,n", [(1, 1_100_000, 0, 5000),      # empty columns between
+                                                     (130, 8192, 0, 60_000),      # thousands of them a tile
+                                                     (3, 400_000, 20, 4000),
+                                                     (64, 16_385, 0, 64),
+                                                     (8, 200_000, 9, 500_000),    # larger bitmaps:
+                                                     (40, 90_000, 1, 2_000_000)])  # one a unit, none
+def test_columns_per_tile(dev, hubs, hub_degree, small, n):
+    indptr, indices, rng = _graph(n, hubs, hub_degree, small, n)
+    hub = np.flatnonzero(np.diff(indptr) == hub_degree)
+    cols = np.concatenate([hub, rng.permutation(n)])[:100_000].astype(np.int64)
+    rows = rng.permutation(n)[: min(n // 2, 9000)].astype(np.int64)
+    at = cols.size // 3
+    cols[at] = n + 7                                             # no such column: empty
+    g = gs.Graph(False)
+    g._CAPI_LoadCSC(to_dev(indptr, dev), to_dev(indices, dev))
+    ptr, idx, _ = g._CAPI_FusionSlicing(to_dev(cols, dev), to_dev(rows, dev))._CAPI_GetCSC()
+    cols = np.delete(cols, at)
+    want = O.col_row_slice(indptr, indices, cols, rows)
+    assert np.array_equal(np.delete(ptr.cpu().numpy(), at), want[0])
+    assert np.array_equal(idx.cpu().numpy(), want[1])
