@@ -5,25 +5,28 @@
 // (src/cuda/fusion/edge_map_reduce.cu:10).
 //
 // The reference gives every segment to one thread (graph_ops.cu:16-39), which
-// stalls a whole wave on a power-law hub.  Two decompositions are used here:
-//  * by segment, for segments of at most 16 edges: one lane per segment, summed
-//    in edge order (bit-identical to a sequential sum).  The typical
-//    layer-wise-sampler call has millions of mostly empty segments
-//    (graph.cc:657: one per graph row): one coalesced pass over the offsets and
-//    one over the output.  The same pass enters every longer segment in the list
-//    of the 1024-edge chunk its first edge falls in, and as the "incoming"
-//    segment of every later chunk it reaches into.
-//  * by edge, for the longer ones: a wave owns one chunk of 1024 consecutive
-//    edges.  Its lanes pick up the chunk's segments (at most 61 can start in it,
-//    plus the incoming one), mark where each starts and stops in an LDS array of
-//    one int per edge, and a running "latest mark" over the edges then tells
-//    every edge its owner without any search; a segmented scan folds 64 edges
-//    per step, coalesced.  A segment that lies inside the chunk is written at
-//    once; the pieces of a segment that crosses chunk borders go to a carry
-//    array and are added up, in chunk order, by the chunk that holds its first
-//    edge.  A 300 000-edge hub is 290 chunks of work for 290 waves, millions of
-//    empty segments cost the by-edge pass nothing, and the order of the additions
-//    is fixed by the layout alone, so results repeat from run to run.
+// stalls a whole wave on a power-law hub.  Here the edges are cut into tiles of 4096,
+// one workgroup each.  The tile's data go to LDS in one coalesced sweep and are not read
+// again: segments of at most 16 edges are added up there by a lane each, in edge order
+// (bit-identical to a sequential sum), up to 128 edges by 16 lanes, longer ones by a
+// wave; a normalise divides in place and stores the tile.  A segment that crosses a tile
+// border leaves a piece in either tile (one of at most 16 edges belongs to the tile it
+// starts in, whole); the pieces are added up in tile order, and the edges of crossing
+// segments, about a third of them on a power-law graph, are all that a normalise reads a
+// second time.  A 300 000-edge hub is 75 workgroups' work, and the order of the additions
+// is fixed by the edges' layout alone, so results repeat from run to run.
+//
+// A workgroup learns its segments from the offsets, 64 at a time in each wave, from the one
+// that holds its first edge on; with few edges per segment (a slice's rows among all rows:
+// millions of empty segments) from one int per edge that a pass over the offsets has left at
+// every segment's first edge.
+//
+// 124 M edges in 2.45 M columns (half of them of at most 16 edges, 19 % of the edges in columns
+// longer than a tile): sum 144 us (3.5 TB/s; the bytes bound it), normalise 308 us (3.2 TB/s
+// over the bytes it needs, 4.3 with the second reading; each tile's chain of LDS steps hides
+// behind five tiles a CU).  A lane per short column, a scan per 1024-edge chunk for the others
+// and a divide pass over all edges, each reading its edges for itself, took 214 and 380.
+// Tiles of 8192 edges: 156 and 324.
 #include <limits>
 #include "gs_common.hpp"
 
@@ -33,591 +36,630 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWave;
 constexpr int64_t kLaneMaxLen = 16;
-constexpr int64_t kChunk = 1024;   // edges per wave in the by-edge pass
-constexpr int kChunkList = 64;     // list slots per chunk: 1024 / 17 + 1 = 61 segments can start in one
-constexpr int kIncomingLane = kWave - 1;
 
-// Per-chunk bookkeeping of the by-edge pass, all in the caller's workspace.
-struct Chunks {
-  unsigned int* any_long;  // does any segment exceed kLaneMaxLen?
-  unsigned int* count;     // [chunks] long segments starting in the chunk
-  int* list;               // [chunks][kChunkList] their ids
-  int* incoming;           // [chunks] long segment that starts earlier and reaches into the chunk, or -1
-  int* outgoing;           // [chunks] long segment that starts here and goes on after the chunk, or -1
-  float* carry;            // [chunks][2]: piece of the incoming segment, piece of the outgoing one
-};
-
-__global__ void __launch_bounds__(kThreads) clear_chunks_kernel(Chunks ck, int64_t chunks) {
-  const int64_t c = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  if (c == 0) *ck.any_long = 0u;
-  if (c < chunks) {
-    ck.count[c] = 0u;
-    ck.incoming[c] = -1;
-  }
+// Value of the lane `CTRL` names, a data-parallel-primitive move inside the vector ALU with no
+// trip through the LDS crossbar (0x121 .. 0x12f: the row of 16 turned by 1 .. 15 lanes).
+template <int CTRL>
+__device__ __forceinline__ float lane_move(float v) {
+  const int bits = __builtin_bit_cast(int, v);
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, bits, CTRL, 0xf, 0xf, false));
 }
 
-// four floats side by side at any 4-byte boundary
-struct __attribute__((packed, aligned(4))) Four {
-  float a, b, c, d;
+constexpr int kLaneEdges = 4;        // of one 16-byte read
+constexpr int kTileItems = 16;
+constexpr int kTile = kThreads * kTileItems;
+constexpr int kGroup = 16;              // lanes that add up a segment of 17 .. kGroupMaxLen edges
+constexpr int kGroupMaxLen = 128;
+
+struct Tiles {
+  int* head;      // [tiles + 1] segment of the tile's first edge; behind the last: of the last edge
+  int* outgoing;  // [tiles] long segment that starts here and goes on after the tile, or -1
+  float* carry;   // [tiles][2] piece of the incoming long segment, piece of the outgoing one
+  int* inner;     // [tiles] normalise: first | end << 16 of the edges that are done
+  int* mark;      // [edges] kMarks: the segment that starts at the edge, or -1
 };
 
-// ---- by segment: the short ones.  NORMALIZE writes out[d] = data[d] / sum instead.  EMAP:
-// with an edge map (a compile-time switch: the two ways of reading hold different things in
-// registers, and one kernel for both would run both at the occupancy of the larger).
-template <bool NORMALIZE, bool EMAP, typename IdT>
+// How a workgroup learns its segments.
+enum Walk {
+  kSearch,  // it searches the offsets for the tile's first and last, and leaves the first in head[]
+  kHeads,   // head[] is there (tile_heads_kernel)
+  kMarks    // head[] and mark[] are
+};
+
+__global__ void __launch_bounds__(kThreads) clear_marks_kernel(int* mark, int64_t n) {
+  const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kTile + threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < kTileItems; ++k)
+    if (i0 + k * kThreads < n) mark[i0 + k * kThreads] = -1;
+}
+
+// head[] of every tile that begins inside a segment; mark[]; a sum's empty segments
+template <bool SUM, bool MARK, typename IdT>
 __global__ void __launch_bounds__(kThreads)
-short_segments_kernel(const int64_t* __restrict__ indptr, const int64_t* __restrict__ emap,
-                      const IdT* __restrict__ nmap, const float* __restrict__ data,
-                      int64_t num_seg, int64_t nnz, int powk, float* __restrict__ out, Chunks ck) {
+tile_heads_kernel(const int64_t* __restrict__ indptr, const IdT* __restrict__ nmap, int64_t num_seg,
+                  float* __restrict__ out, Tiles tl) {
   const int64_t s = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  int64_t begin = 0, end = 0;
+  int64_t t0 = 0, t1 = -1;
   if (s < num_seg) {
-    begin = indptr[s];
-    end = indptr[s + 1];
+    const int64_t begin = indptr[s], end = indptr[s + 1];
+    if (end > begin) {
+      t0 = (begin + kTile - 1) / kTile;
+      t1 = (end - 1) / kTile;
+      if (end == indptr[num_seg]) tl.head[t1 + 1] = static_cast<int>(s);
+      if (MARK) tl.mark[begin] = static_cast<int>(s);
+    } else if (SUM) {
+      out[nmap ? static_cast<int64_t>(nmap[s]) : s] = 0.0f;
+    }
   }
-  const int64_t len = end - begin;
+  const bool wide = t1 - t0 >= kWave;
+  if (!wide)
+    for (int64_t t = t0; t <= t1; ++t) tl.head[t] = static_cast<int>(s);
+  unsigned long long todo = __ballot(wide);
   const int lane = threadIdx.x & (kWave - 1);
-  const bool is_long = len > kLaneMaxLen;
-  // the long segments of a wave enter their chunks' lists, one atomic per chunk touched
-  unsigned long long todo = __ballot(is_long);
-  if (todo && lane == 0) *ck.any_long = 1u;
-  const int64_t c0 = begin / kChunk;
   while (todo) {
-    const int64_t c = __shfl(c0, __ffsll(static_cast<long long>(todo)) - 1, kWave);
-    const unsigned long long same = __ballot(is_long && c0 == c);
-    const int leader = __ffsll(static_cast<long long>(same)) - 1;
-    unsigned int base = 0;
-    if (lane == leader) base = atomicAdd(ck.count + c, static_cast<unsigned int>(__popcll(same)));
-    base = __shfl(base, leader, kWave);
-    if (is_long && c0 == c)
-      ck.list[c * kChunkList + base + __popcll(same & ((1ull << lane) - 1ull))] = static_cast<int>(s);
-    todo &= ~same;
-  }
-  if (s >= num_seg) return;
-  if (is_long) {
-    const int64_t c1 = (end - 1) / kChunk;
-    for (int64_t c = c0 + 1; c <= c1; ++c) ck.incoming[c] = static_cast<int>(s);
-    return;
-  }
-  // at most kLaneMaxLen edges: a fixed number of predicated reads, all in flight together,
-  // added up in edge order.  Without an edge map the lane's edges lie side by side and are
-  // read four at a time (a lane's reads are scattered from its neighbours' either way: every
-  // read instruction is a line access per lane, and this makes four of sixteen).
-  float v[kLaneMaxLen];
-  int64_t at[kLaneMaxLen];
-  if (!EMAP) {
-#pragma unroll
-    for (int j = 0; j < kLaneMaxLen / 4; ++j) {
-      const int64_t p = begin + 4 * j;
-      Four q{0.0f, 0.0f, 0.0f, 0.0f};
-      if (p + 3 < nnz && p < end) {
-        q = *reinterpret_cast<const Four*>(data + p);
-      } else {
-        if (p < end) q.a = data[p];
-        if (p + 1 < end) q.b = data[p + 1];
-        if (p + 2 < end) q.c = data[p + 2];
-      }
-      v[4 * j] = q.a, v[4 * j + 1] = q.b, v[4 * j + 2] = q.c, v[4 * j + 3] = q.d;
-#pragma unroll
-      for (int u = 0; u < 4; ++u) at[4 * j + u] = p + u < end ? p + u : -1;
-    }
-  } else {
-    // (predicated pair by pair: most segments here are far shorter than sixteen, and sweeps
-    // of sixteen clamped reads cost more than the waits they save -- 52 against 36 us over
-    // the 2.45 M mostly empty rows of a sliced graph)
-#pragma unroll
-    for (int k = 0; k < kLaneMaxLen; ++k) {
-      at[k] = begin + k < end ? emap[begin + k] : -1;
-      v[k] = at[k] >= 0 ? data[at[k]] : 0.0f;
-    }
-  }
-  float acc = 0.0f;
-#pragma unroll
-  for (int k = 0; k < kLaneMaxLen; ++k)
-    if (at[k] >= 0) acc += powk_f(v[k], powk);
-  if (NORMALIZE) {
-#pragma unroll
-    for (int k = 0; k < kLaneMaxLen; ++k)
-      if (at[k] >= 0) out[at[k]] = v[k] / acc;
-  } else {
-    out[nmap ? static_cast<int64_t>(nmap[s]) : s] = acc;
+    const int src = __ffsll(static_cast<long long>(todo)) - 1;
+    todo &= todo - 1;
+    const int64_t w0 = __shfl(t0, src, kWave), w1 = __shfl(t1, src, kWave);
+    const int64_t ws = __shfl(s, src, kWave);
+    for (int64_t t = w0 + lane; t <= w1; t += kWave) tl.head[t] = static_cast<int>(ws);
   }
 }
 
-// ---- by edge: the long ones.
-// What a lane knows of the chunk's long segments: lane l < count holds the l-th of the list,
-// the last lane the incoming one.
-struct Owned {
-  int g;           // segment, -1 = none
-  int64_t b, e;    // its edge range
+// sum over the 16 lanes of a row, in every lane
+__device__ __forceinline__ float row_sum(float x) {
+  x += lane_move<0x128>(x);
+  x += lane_move<0x124>(x);
+  x += lane_move<0x122>(x);
+  return x + lane_move<0x121>(x);
+}
+
+using F4 = float __attribute__((ext_vector_type(4)));
+
+// Source: where a tile's data come from.
+enum Source {
+  kPlain,   // data[edge], 16-byte aligned
+  kLoose,   // data[edge]
+  kMapped   // data[emap[edge]]
 };
 
-__device__ __forceinline__ Owned load_owned(const int64_t* __restrict__ indptr, const Chunks& ck,
-                                            int64_t c, int lane) {
-  Owned o;
-  o.g = -1;
-  o.b = o.e = 0;
-  const int n = static_cast<int>(ck.count[c]);
-  if (lane < n) o.g = ck.list[c * kChunkList + lane];
-  if (lane == kIncomingLane) o.g = ck.incoming[c];
-  if (o.g >= 0) {
-    o.b = indptr[o.g];
-    o.e = indptr[o.g + 1];
-  }
-  return o;
-}
-
-// mark[p] = lane + 2 where the lane's segment starts (or the chunk does, for the incoming
-// one), 1 where a segment stops and no other starts, 0 elsewhere
-__device__ __forceinline__ void write_marks(int* mark, const Owned& o, int64_t begin, int64_t end,
-                                            int lane, bool skip = false) {
-  for (int i = lane; i < kChunk; i += kWave) mark[i] = 0;
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  if (o.g >= 0 && !skip) {
-    atomicMax(&mark[(o.b > begin ? o.b : begin) - begin], lane + 2);
-    if (o.e < end) atomicMax(&mark[o.e - begin], 1);
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
-// A step is 256 edges, four consecutive ones per lane (one 16-byte read of the marks, one of
-// the data).  A long segment has at least 17 edges, so inside a lane's four at most one long
-// run ends (at the lane's first mark) and at most one begins (at its last mark); what lies
-// between belongs to short segments.  Lanes therefore exchange one value each: the cross-lane
-// work per edge is a quarter of a lane-per-edge scan's.
-constexpr int kLaneEdges = 4;
-constexpr int kStep = kWave * kLaneEdges;
-
-struct LaneMarks {
-  int first_k, last_k;  // first and last marked edge among the lane's four, -1 = none
-  int last_packed;      // (position + 1) << 8 | mark of the last one, 0 = none
-};
-
-__device__ __forceinline__ LaneMarks scan_lane_marks(const int (&m)[kLaneEdges], int at0) {
-  LaneMarks lm;
-  lm.first_k = lm.last_k = -1;
-  lm.last_packed = 0;
-#pragma unroll
-  for (int k = 0; k < kLaneEdges; ++k) {
-    if (m[k]) {
-      if (lm.first_k < 0) lm.first_k = k;
-      lm.last_k = k;
-      lm.last_packed = (at0 + k + 1) << 8 | m[k];
-    }
-  }
-  return lm;
-}
-
-// Value of the lane `CTRL` names (a data-parallel-primitive move inside the vector ALU, no
-// trip through the LDS crossbar); lanes without a source, or outside ROWS, get `fill`.
-// 0x111/0x112/0x114/0x118: the lane 1/2/4/8 below in the same row of 16; 0x142: lane 15 of
-// the row below (rows 1 and 3 with ROWS = 0xa); 0x143: lane 31 (rows 2 and 3 with 0xc).
-template <int CTRL, int ROWS>
-__device__ __forceinline__ int lane_move(int fill, int v) {
-  return __builtin_amdgcn_update_dpp(fill, v, CTRL, ROWS, 0xf, false);
-}
-
-// latest mark at or before the end of each lane (inclusive) given the lanes' own last marks;
-// positions grow with the lane, so a maximum is "the latest".  Marks are >= 0.
-__device__ __forceinline__ int latest_inclusive(int last_packed, int carried, int) {
-  int p = last_packed;
-  int y;
-  y = lane_move<0x111, 0xf>(0, p); p = y > p ? y : p;
-  y = lane_move<0x112, 0xf>(0, p); p = y > p ? y : p;
-  y = lane_move<0x114, 0xf>(0, p); p = y > p ? y : p;
-  y = lane_move<0x118, 0xf>(0, p); p = y > p ? y : p;
-  y = lane_move<0x142, 0xa>(0, p); p = y > p ? y : p;
-  y = lane_move<0x143, 0xc>(0, p); p = y > p ? y : p;
-  return p > carried ? p : carried;
-}
-
-// inclusive sums of x over the lanes below that share the lane's key; keys do not decrease
-// with the lane and are >= 0
-__device__ __forceinline__ float keyed_inclusive_sum(float x, int key) {
-#define GS_KEYED_STEP(CTRL, ROWS)                                                       \
-  {                                                                                     \
-    const int ky = lane_move<CTRL, ROWS>(-1, key);                                      \
-    const float y = __builtin_bit_cast(float, lane_move<CTRL, ROWS>(0, __builtin_bit_cast(int, x))); \
-    if (ky == key) x += y;                                                              \
-  }
-  GS_KEYED_STEP(0x111, 0xf)
-  GS_KEYED_STEP(0x112, 0xf)
-  GS_KEYED_STEP(0x114, 0xf)
-  GS_KEYED_STEP(0x118, 0xf)
-  GS_KEYED_STEP(0x142, 0xa)
-  GS_KEYED_STEP(0x143, 0xc)
-#undef GS_KEYED_STEP
-  return x;
-}
-
-__device__ __forceinline__ int owner_of_mark(int packed) { return (packed & 0xFF) - 2; }
-
-// sums is indexed by segment (nmap applied when given)
-template <typename IdT>
-__global__ void __launch_bounds__(kThreads)
-long_segments_kernel(const int64_t* __restrict__ indptr, const int64_t* __restrict__ emap,
+// One tile.  Once the data are in LDS (the first barrier) the waves go their own ways: each takes
+// a quarter of the segments that start in the tile (with marks: those that start in its quarter
+// of the edges), the first one the incoming segment as well, 64 at a time -- the short ones a
+// lane each, what is longer from a list in LDS of the wave's own, four at a time or one by one.
+// With lists and flags shared by the workgroup and a barrier after every step a tile took 12 us
+// where it takes 7, which is what held the chip back; with the segments dealt out by
+// quarters of the edges, one tile of 16 k segments kept a wave busy for 80 us at the end.
+template <bool NORMALIZE, Source SOURCE, Walk WALK, typename IdT>
+__global__ void __launch_bounds__(kThreads, WALK == kMarks || SOURCE == kMapped ? 4 : 8)
+segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restrict__ emap,
                      const IdT* __restrict__ nmap, const float* __restrict__ data,
-                     int64_t num_seg, int64_t nnz, int powk, float* __restrict__ sums, Chunks ck) {
-  __shared__ __attribute__((aligned(16))) int s_mark[kWaves][kChunk];
-  if (*ck.any_long == 0u) return;
-  if (indptr[num_seg] < nnz) nnz = indptr[num_seg];  // the caller's count is an upper bound
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t c = static_cast<int64_t>(blockIdx.x) * kWaves + threadIdx.x / kWave;
-  const int64_t begin = c * kChunk;
-  if (begin >= nnz) return;
-  const int64_t end = begin + kChunk < nnz ? begin + kChunk : nnz;
-  int* mark = s_mark[threadIdx.x / kWave];
-  const Owned own = load_owned(indptr, ck, c, lane);
-  // no long segment touches the chunk (a chunk of a thousand one-edge rows): nothing to do
-  if (__ballot(own.g >= 0) == 0ull) {
-    if (lane == 0) ck.outgoing[c] = -1;
-    return;
+                     int64_t num_seg, int64_t nnz, int powk, float* __restrict__ out, Tiles tl) {
+  constexpr bool EMAP = SOURCE == kMapped;
+  __shared__ __attribute__((aligned(16))) float s_v[kTile];
+  __shared__ uint32_t s_list[kWaves][kWave];
+  __shared__ int64_t s_head[2];
+  __shared__ int s_first, s_end, s_out;  // edges in front of `first`, from `end` on: of crossing segments
+  // (the last tile first: where columns are numbered with the busy ones in front, the tiles of
+  // thousands of columns, which take several times as long, come last, and the chip would wait for
+  // the last of them: 144 -> 128 us)
+  const int64_t t = gridDim.x - 1 - blockIdx.x, p0 = t * kTile;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  // (what the chain of dependent reads starts with goes out first)
+  int64_t head = 0, tail = 0;  // segments of the tile's first edge and of the one behind its last
+  if (WALK != kSearch) {
+    head = tl.head[t];
+    if (WALK == kHeads) tail = tl.head[t + 1];
   }
-  // The whole chunk lies inside the incoming segment (most chunks of a hub column do): one
-  // sum, no marks, no scans.
-  if (__shfl(own.g >= 0 ? own.e : int64_t(0), kIncomingLane, kWave) >= end) {
+  const int64_t all = indptr[num_seg];
+  const bool vec = SOURCE == kPlain && p0 + kTile <= nnz;
+  F4 q[kTileItems / kLaneEdges];
+  if (vec) {
+#pragma unroll
+    for (int k = 0; k < kTileItems / kLaneEdges; ++k)
+      q[k] = *reinterpret_cast<const F4*>(data + p0 + (k * kThreads + tid) * kLaneEdges);
+  }
+  if (all < nnz) nnz = all;  // the caller's count is an upper bound
+  if (p0 >= nnz) return;
+  const int n = static_cast<int>(nnz - p0 < kTile ? nnz - p0 : kTile);
+  const int64_t p1 = p0 + n;
+
+  int64_t where[EMAP ? kTileItems : 1];
+  float x[kTileItems];
+  if constexpr (SOURCE != kPlain) {
+    if constexpr (EMAP) {
+#pragma unroll
+      for (int k = 0; k < kTileItems; ++k) {
+        const int i = k * kThreads + tid;
+        where[k] = emap[p0 + (i < n ? i : n - 1)];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kTileItems; ++k) {
+      const int i = k * kThreads + tid;
+      x[k] = data[EMAP ? where[EMAP ? k : 0] : p0 + (i < n ? i : n - 1)];
+    }
+  }
+  if (WALK == kSearch) {
+    if (wave < 2) {
+      const int64_t r = wave_upper_bound(indptr, num_seg + 1, wave == 0 ? p0 : p1 - 1) - 1;
+      if (lane == 0) s_head[wave] = r;
+      if (tid == 0) tl.head[t] = static_cast<int>(r);
+    }
+    __syncthreads();
+    head = s_head[0];
+    tail = s_head[1];
+  }
+  // this wave's segments, and the offsets of the next 256 of them, four sets of 64 (the ends of a
+  // set are the next one's beginnings; of the last, an entry of its own)
+  const int64_t share = (tail - head + kWaves) / kWaves;
+  const int64_t seg0 = head + wave * share;
+  const int64_t seg1 = seg0 + share < tail + 1 ? seg0 + share : tail + 1;
+  constexpr int kSets = 4;
+  int64_t starts[kSets + 1];
+  auto offsets = [&](int64_t first) {
+#pragma unroll
+    for (int u = 0; u <= kSets; ++u) {
+      const int64_t r = first + u * kWave + (u < kSets ? lane : 0);
+      starts[u] = indptr[r < seg1 ? r : seg1];
+    }
+  };
+  if (WALK != kMarks && seg0 < seg1) offsets(seg0);
+  if (tid == 0) {
+    s_first = 0;
+    s_end = n;
+    s_out = -1;
+  }
+  // x^powk of a thread's edges, one loop for all of them (the products are powk_f's)
+  if (vec) {
+    F4 p[kTileItems / kLaneEdges];
+#pragma unroll
+    for (int k = 0; k < kTileItems / kLaneEdges; ++k) p[k] = q[k];
+    if (!NORMALIZE)
+      for (int i = 1; i < powk; ++i) {
+#pragma unroll
+        for (int k = 0; k < kTileItems / kLaneEdges; ++k) p[k] *= q[k];
+      }
+#pragma unroll
+    for (int k = 0; k < kTileItems / kLaneEdges; ++k)
+      *reinterpret_cast<F4*>(s_v + (k * kThreads + tid) * kLaneEdges) = p[k];
+  } else if constexpr (SOURCE == kPlain) {  // (the last tile)
+    for (int i = tid; i < n; i += kThreads) s_v[i] = NORMALIZE ? data[p0 + i] : powk_f(data[p0 + i], powk);
+  } else {
+    float p[kTileItems];
+#pragma unroll
+    for (int k = 0; k < kTileItems; ++k) p[k] = x[k];
+    if (!NORMALIZE)
+      for (int i = 1; i < powk; ++i) {
+#pragma unroll
+        for (int k = 0; k < kTileItems; ++k) p[k] *= x[k];
+      }
+#pragma unroll
+    for (int k = 0; k < kTileItems; ++k) s_v[k * kThreads + tid] = p[k];
+  }
+  __syncthreads();
+
+  auto put = [&](int64_t seg, float total) {
+    out[nmap ? static_cast<int64_t>(nmap[seg]) : seg] = total;
+  };
+  // A segment of at most 16 edges, one lane; what of it lies in the next tile included, which
+  // leaves it alone.
+  auto short_one = [&](int64_t seg, int64_t begin, int64_t end) {
+    const int at = static_cast<int>(begin - p0);
+    const int stop = static_cast<int>((end < p1 ? end : p1) - p0);
     float acc = 0.0f;
-    if (!emap && end - begin == kChunk && (reinterpret_cast<uintptr_t>(data) & 15u) == 0) {
+    for (int j = at; j < stop; j += 4) {  // (four reads, then four additions in edge order)
+      float v[4];
 #pragma unroll
-      for (int t = 0; t < kChunk / kStep; ++t) {
-        const float4 v = *reinterpret_cast<const float4*>(data + begin + t * kStep + lane * kLaneEdges);
-        acc += (powk_f(v.x, powk) + powk_f(v.y, powk)) + (powk_f(v.z, powk) + powk_f(v.w, powk));
-      }
-    } else if (end - begin == kChunk) {
-      // the same additions in the same order through an edge map (or from unaligned data), so
-      // that a sum does not depend on which of its layouts a graph holds
+      for (int u = 0; u < 4; ++u) v[u] = s_v[j + u < kTile ? j + u : kTile - 1];
 #pragma unroll
-      for (int t = 0; t < kChunk / kStep; ++t) {
-        const int64_t e = begin + t * kStep + lane * kLaneEdges;
-        float v[kLaneEdges];
-#pragma unroll
-        for (int k = 0; k < kLaneEdges; ++k) v[k] = powk_f(data[emap ? emap[e + k] : e + k], powk);
-        acc += (v[0] + v[1]) + (v[2] + v[3]);
+      for (int u = 0; u < 4; ++u)
+        if (j + u < stop) acc += v[u];
+    }
+    for (int64_t e = p1; e < end; ++e) {
+      const float v = data[EMAP ? emap[e] : e];
+      acc += NORMALIZE ? v : powk_f(v, powk);
+    }
+    if (NORMALIZE) {
+      for (int j = at; j < stop; ++j) s_v[j] = s_v[j] / acc;
+      for (int64_t e = p1; e < end; ++e) {
+        const int64_t d = EMAP ? emap[e] : e;
+        out[d] = data[d] / acc;
       }
     } else {
-      for (int64_t e = begin + lane; e < end; e += kWave)
-        acc += powk_f(data[emap ? emap[e] : e], powk);
+      put(seg, acc);
     }
+  };
+  // Up to 64 segments, one a lane (seg < 0: none): the lane's starts in the wave's share, or is the
+  // incoming one.
+  // Without marks, lane l's is segment base + l.
+  auto round = [&](int64_t base, int64_t seg, int64_t begin, int64_t end) {
+    const bool here = seg >= 0;
+    const bool incoming = here && begin < p0;
+    const bool is_long = here && end - begin > kLaneMaxLen;
+    const int at = static_cast<int>((incoming ? p0 : begin) - p0);
+    const int stop = static_cast<int>((end < p1 ? end : p1) - p0);
+    const int len = stop - at;
+    if (incoming) s_first = stop;
+    const bool outgoing = is_long && !incoming && end > p1;
+    if (outgoing) {
+      s_end = at;
+      s_out = static_cast<int>(seg);
+    }
+    if (here && !is_long && !incoming) short_one(seg, begin, end);
+    // where a long segment's sum goes: 0 its own place, 1 the incoming piece's, 2 the outgoing one's
+    const int kind = incoming ? 1 : (outgoing ? 2 : 0);
+    auto finish = [&](int k, int64_t s, float total) {
+      if (k == 1) tl.carry[2 * t] = total;
+      else if (k == 2) tl.carry[2 * t + 1] = total;
+      else if (!NORMALIZE) put(s, total);
+    };
+    const bool few = is_long && len <= kGroupMaxLen;
+    const unsigned long long list = __ballot(few);
+    if (list) {
+      const int count = __popcll(list);
+      // {first edge: 12 bits, edges less one: 7, lane: 6, kind: 2}
+      if (few)
+        s_list[wave][__popcll(list & ((1ull << lane) - 1ull))] =
+            static_cast<uint32_t>(at) | static_cast<uint32_t>(len - 1) << 12 |
+            static_cast<uint32_t>(lane) << 19 | static_cast<uint32_t>(kind) << 25;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      for (int i0 = 0; i0 < count; i0 += kWave / kGroup) {
+        const int i = i0 + lane / kGroup, j0 = lane & (kGroup - 1);
+        const bool live = i < count;
+        const uint32_t w = s_list[wave][live ? i : 0];
+        const int left = live ? static_cast<int>((w >> 12) & 0x7F) + 1 - j0 : 0;
+        const int from = left > 0 ? static_cast<int>(w & 0xFFF) + j0 : 0;
+        constexpr int kEach = kGroupMaxLen / kGroup;
+        float v[kEach];
 #pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) acc += __shfl_xor(acc, d, kWave);
-    if (lane == 0) {
-      ck.carry[2 * c] = acc;
-      ck.outgoing[c] = -1;
+        for (int u = 0; u < kEach; ++u) v[u] = s_v[from + (u * kGroup < left ? u * kGroup : 0)];
+        float acc = 0.0f;
+#pragma unroll
+        for (int u = 0; u < kEach; ++u)
+          if (u * kGroup < left) acc += v[u];
+        const float total = row_sum(acc);
+        const int src = static_cast<int>((w >> 19) & 63), k = static_cast<int>(w >> 25);
+        const int64_t s = WALK == kMarks ? __shfl(seg, src, kWave) : base + src;
+        if (live && j0 == 0) finish(k, s, total);
+        if (NORMALIZE && k == 0) {
+#pragma unroll
+          for (int u = 0; u < kEach; ++u)
+            if (u * kGroup < left) s_v[from + u * kGroup] = v[u] / total;
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    for (unsigned long long todo = __ballot(is_long && !few); todo; todo &= todo - 1) {
+      const int src = __ffsll(static_cast<long long>(todo)) - 1;
+      const int from = __builtin_amdgcn_readlane(at, src), size = __builtin_amdgcn_readlane(len, src);
+      const int k = __builtin_amdgcn_readlane(kind, src);
+      constexpr int kEach = 8;
+      float total = 0.0f;
+      for (int j = lane; j < size; j += kEach * kWave) {
+        float v[kEach];
+#pragma unroll
+        for (int u = 0; u < kEach; ++u) v[u] = s_v[from + (j + u * kWave < size ? j + u * kWave : j)];
+#pragma unroll
+        for (int u = 1; u < kEach; ++u)
+          if (j + u * kWave >= size) v[u] = 0.0f;
+        total += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+      }
+      total = row_sum(total);
+      total = (__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, total), 0)) +
+               __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, total), 16))) +
+              (__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, total), 32)) +
+               __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, total), 48)));
+      if (lane == src) finish(k, seg, total);
+      if (NORMALIZE && k == 0)
+        for (int j = lane; j < size; j += kWave) s_v[from + j] = s_v[from + j] / total;
+    }
+  };
+
+  constexpr int kQuarter = kTile / kWaves;
+  const int64_t q0 = p0 + wave * kQuarter;
+  if (WALK == kMarks ? q0 < p1 : seg0 < seg1) {
+    if (WALK == kMarks) {
+      int seg[kQuarter / kWave];
+      int64_t end[kQuarter / kWave];
+#pragma unroll
+      for (int k = 0; k < kQuarter / kWave; ++k) {
+        const int64_t p = q0 + k * kWave + lane;
+        seg[k] = p < p1 ? tl.mark[p] : -1;
+      }
+      int64_t begin_in = 0;
+      bool incoming = false;
+      if (wave == 0) {  // the tile's incoming segment, when no segment starts at its first edge
+        begin_in = indptr[head];
+        incoming = lane == 0 && begin_in < p0;
+        if (incoming) seg[0] = static_cast<int>(head);
+      }
+#pragma unroll
+      for (int k = 0; k < kQuarter / kWave; ++k) end[k] = indptr[seg[k] >= 0 ? seg[k] + 1 : 0];
+#pragma unroll 1
+      for (int k = 0; k < kQuarter / kWave; ++k) {
+        int s = seg[0];
+        int64_t e = end[0];
+#pragma unroll
+        for (int u = 1; u < kQuarter / kWave; ++u)
+          if (u == k) s = seg[u], e = end[u];
+        if (__ballot(s >= 0) == 0ull) continue;
+        round(0, s, k == 0 && incoming ? begin_in : q0 + k * kWave + lane, e);
+      }
+    } else {
+      for (int64_t r0 = seg0;;) {
+        bool any = false;
+#pragma unroll 1
+        for (int u = 0; u < kSets && r0 + u * kWave < seg1; ++u) {
+          int64_t begin = starts[0], next = starts[1];
+#pragma unroll
+          for (int v = 1; v < kSets; ++v)
+            if (u == v) begin = starts[v], next = starts[v + 1];
+          int64_t end = __shfl_down(begin, 1, kWave);
+          next = __shfl(next, 0, kWave);
+          if (lane == kWave - 1) end = next;
+          // (the segment behind the tile's last edge may start there)
+          const int64_t r = r0 + u * kWave + lane;
+          const bool mine = end > begin && begin < p1;
+          if (__ballot(mine)) {
+            any = true;
+            round(r - lane, mine ? r : -1, begin, end);
+          }
+        }
+        const int64_t behind = __shfl(starts[kSets], 0, kWave);
+        r0 += kSets * kWave;
+        if (r0 >= seg1) break;
+        // after nothing but empty segments: on to the one that holds the next edge
+        if (!any) {
+          r0 = wave_upper_bound(indptr, num_seg + 1, behind) - 1;
+          if (r0 >= seg1) break;
+        }
+        offsets(r0);
+      }
+    }
+  }
+  __syncthreads();
+  if (tid == 0) tl.outgoing[t] = s_out;
+  if constexpr (NORMALIZE) {
+    const int first = s_first, stop = s_end > first ? s_end : first;
+    if (tid == 0) tl.inner[t] = first | stop << 16;
+    if constexpr (EMAP) {
+#pragma unroll
+      for (int k = 0; k < kTileItems; ++k) {
+        const int i = k * kThreads + tid;
+        if (i >= first && i < stop) out[where[k]] = s_v[i];
+      }
+    } else if (vec && n == kTile && (reinterpret_cast<uintptr_t>(out) & 15u) == 0) {
+#pragma unroll
+      for (int k = 0; k < kTileItems / kLaneEdges; ++k) {
+        const int i = (k * kThreads + tid) * kLaneEdges;
+        const float4 v = *reinterpret_cast<const float4*>(s_v + i);
+        if (i >= first && i + 3 < stop) {
+          *reinterpret_cast<float4*>(out + p0 + i) = v;
+        } else {
+          if (i >= first && i < stop) out[p0 + i] = v.x;
+          if (i + 1 >= first && i + 1 < stop) out[p0 + i + 1] = v.y;
+          if (i + 2 >= first && i + 2 < stop) out[p0 + i + 2] = v.z;
+          if (i + 3 >= first && i + 3 < stop) out[p0 + i + 3] = v.w;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < kTileItems; ++k) {
+        const int i = k * kThreads + tid;
+        if (i >= first && i < stop) out[p0 + i] = s_v[i];
+      }
+    }
+  }
+}
+
+// The edges of segments that cross tile borders: what lies in front of a tile's inner edges
+// belongs to the incoming segment, what lies behind to the outgoing one.  Each workgroup adds
+// up the pieces of its two segments for itself.
+template <bool EMAP>
+__global__ void __launch_bounds__(kThreads)
+crossing_divide_kernel(const int64_t* __restrict__ indptr, const int64_t* __restrict__ emap,
+                       const float* __restrict__ data, int64_t num_seg, int64_t nnz,
+                       float* __restrict__ out, Tiles tl) {
+  __shared__ float s_total[2];
+  const int64_t t = blockIdx.x, p0 = t * kTile;
+  const int64_t all = indptr[num_seg];
+  const int inner = tl.inner[t], g_in = tl.head[t], g_out = tl.outgoing[t];
+  if (all < nnz) nnz = all;
+  if (p0 >= nnz) return;
+  const int n = static_cast<int>(nnz - p0 < kTile ? nnz - p0 : kTile);
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  int first = inner & 0xFFFF;
+  const int stop = inner >> 16;
+  if (first > 0 && indptr[g_in + 1] - indptr[g_in] <= kLaneMaxLen) first = 0;  // (done where it starts)
+  if (first == 0 && stop == n) return;
+  const bool vec = !EMAP && n == kTile &&
+                   ((reinterpret_cast<uintptr_t>(data) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
+  float4 v[kTileItems / 4];
+  if (vec) {
+#pragma unroll
+    for (int k = 0; k < kTileItems / 4; ++k) {
+      const int i = k * (4 * kThreads) + 4 * tid;
+      v[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (i < first || i + 3 >= stop) v[k] = *reinterpret_cast<const float4*>(data + p0 + i);
+    }
+  }
+  if (wave < 2) {
+    const int g = wave == 0 ? (first > 0 ? g_in : -1) : g_out;
+    if (g >= 0) {
+      const int64_t from = indptr[g] / kTile, to = (indptr[g + 1] - 1) / kTile;
+      float part = 0.0f;
+      for (int64_t k = from + 1 + lane; k <= to; k += kWave) part += tl.carry[2 * k];
+#pragma unroll
+      for (int d = kWave / 2; d > 0; d >>= 1) part += __shfl_xor(part, d, kWave);
+      if (lane == 0) s_total[wave] = tl.carry[2 * from + 1] + part;
+    }
+  }
+  __syncthreads();
+  const float before = s_total[0], behind = s_total[1];
+  if (vec) {
+#pragma unroll
+    for (int k = 0; k < kTileItems / 4; ++k) {
+      const int i = k * (4 * kThreads) + 4 * tid;
+      if (i + 3 < first || i >= stop) {
+        const float d = i >= stop ? behind : before;
+        *reinterpret_cast<float4*>(out + p0 + i) =
+            make_float4(v[k].x / d, v[k].y / d, v[k].z / d, v[k].w / d);
+      } else if (i < first || i + 3 >= stop) {
+        const float w[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (i + u < first) out[p0 + i + u] = w[u] / before;
+          else if (i + u >= stop) out[p0 + i + u] = w[u] / behind;
+        }
+      }
     }
     return;
   }
-  // An incoming segment of which fewer than four edges are left would start and stop inside
-  // the first lane, the one case of a run that does not reach beyond a lane: it gets no marks
-  // and lane 0 adds it up by itself.
-  const int64_t in_left = __shfl(own.g >= 0 ? own.e - begin : int64_t(0), kIncomingLane, kWave);
-  const int tiny = in_left < kLaneEdges ? static_cast<int>(in_left) : 0;
-  // a full chunk of plain data: all four steps' reads are issued before the marks are made,
-  // so that the scans below do not wait for memory step by step
-  const bool ahead = !emap && end - begin == kChunk && (reinterpret_cast<uintptr_t>(data) & 15u) == 0;
-  float4 early[kChunk / kStep];
-  if (ahead) {
-#pragma unroll
-    for (int t = 0; t < kChunk / kStep; ++t)
-      early[t] = *reinterpret_cast<const float4*>(data + begin + t * kStep + lane * kLaneEdges);
-  }
-  write_marks(mark, own, begin, end, lane, tiny > 0 && lane == kIncomingLane);
-  int carried = 0;       // latest mark at the end of the step before
-  bool open = false;     // that mark's segment is a long one: its run goes on
-  float acc_open = 0.0f;
-#pragma unroll
-  for (int t = 0; t < kChunk / kStep; ++t) {
-    const int64_t base = begin + t * kStep;
-    if (base >= end) break;
-    const int at0 = static_cast<int>(base - begin) + lane * kLaneEdges;
-    const int64_t e0 = base + lane * kLaneEdges;
-    int m[kLaneEdges];
-    float v[kLaneEdges];
-    {
-      const int4 mm = *reinterpret_cast<const int4*>(mark + at0);
-      m[0] = mm.x; m[1] = mm.y; m[2] = mm.z; m[3] = mm.w;
+  for (int i = tid; i < n; i += kThreads)
+    if (i < first || i >= stop) {
+      const int64_t d = EMAP ? emap[p0 + i] : p0 + i;
+      out[d] = data[d] / (i < first ? before : behind);
     }
-    if (ahead) {
-      v[0] = powk_f(early[t].x, powk);
-      v[1] = powk_f(early[t].y, powk);
-      v[2] = powk_f(early[t].z, powk);
-      v[3] = powk_f(early[t].w, powk);
-    } else {
-#pragma unroll
-      for (int k = 0; k < kLaneEdges; ++k) {
-        const int64_t e = e0 + k;
-        if (e >= end) m[k] = 0;
-        v[k] = e < end ? powk_f(data[emap ? emap[e] : e], powk) : 0.0f;
-      }
-    }
-    if (tiny > 0 && base == begin && lane == 0) {
-      float piece = 0.0f;
-#pragma unroll
-      for (int k = 0; k < kLaneEdges - 1; ++k)
-        if (k < tiny) piece += v[k];
-      ck.carry[2 * c] = piece;
-    }
-    const LaneMarks lm = scan_lane_marks(m, at0);
-    const bool has_mark = lm.first_k >= 0;
-    float pre = 0.0f, post = 0.0f;  // edges before the first mark; from the last mark on
-#pragma unroll
-    for (int k = 0; k < kLaneEdges; ++k) {
-      if (!has_mark || k < lm.first_k) pre += v[k];
-      if (has_mark && k >= lm.last_k) post += v[k];
-    }
-    const int incl = latest_inclusive(lm.last_packed, carried, lane);
-    // the mark in force where the lane begins: the lane below's (0x138: the whole wave
-    // moved up by one lane), the step before's for lane 0
-    const int in_packed = lane_move<0x138, 0xf>(carried, incl);
-    const int in_owner = owner_of_mark(in_packed);
-    // one value per lane: the start of a run where the lane holds a mark, else its four edges
-    float x = has_mark ? (owner_of_mark(incl) >= 0 ? post : 0.0f) : (in_owner >= 0 ? pre : 0.0f);
-    x = keyed_inclusive_sum(x, incl);
-    // the incoming run's sum over the lanes before
-    const float x_prev = __builtin_bit_cast(float, lane_move<0x138, 0xf>(0, __builtin_bit_cast(int, x)));
-    const int src = in_owner >= 0 ? in_owner : 0;
-    const int64_t in_b = __shfl(own.b, src, kWave);
-    const int in_g = __shfl(own.g, src, kWave);
-    if (has_mark && in_owner >= 0) {  // the incoming long run stops at this lane's first mark
-      float total = x_prev + pre;
-      if (open && in_packed == carried) total += acc_open;
-      if (in_b >= begin)
-        sums[nmap ? static_cast<int64_t>(nmap[in_g]) : in_g] = total;
-      else
-        ck.carry[2 * c] = total;
-    }
-    const int last = __builtin_amdgcn_readlane(incl, kWave - 1);
-    const float x_last =
-        __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), kWave - 1));
-    const bool goes_on = owner_of_mark(last) >= 0;
-    acc_open = goes_on ? x_last + (open && last == carried ? acc_open : 0.0f) : 0.0f;
-    open = goes_on;
-    carried = last;
-  }
-  // the run in force at the end of the chunk
-  int out_g = -1;
-  if (open) {
-    const int owner = owner_of_mark(carried);
-    const int64_t ob = __shfl(own.b, owner, kWave);
-    const int64_t oe = __shfl(own.e, owner, kWave);
-    const int og = __shfl(own.g, owner, kWave);
-    if (lane == 0) {
-      if (oe == end) {
-        if (ob >= begin)
-          sums[nmap ? static_cast<int64_t>(nmap[og]) : og] = acc_open;
-        else
-          ck.carry[2 * c] = acc_open;
-      } else {
-        ck.carry[ob >= begin ? 2 * c + 1 : 2 * c] = acc_open;
-      }
-    }
-    if (oe != end && ob >= begin) out_g = og;
-  }
-  if (lane == 0) ck.outgoing[c] = out_g;
 }
 
 constexpr int64_t kCarryAlone = 16;  // pieces a single lane adds up by itself
 
-// One lane per chunk: a chunk that holds the head of a long segment going on after it adds
-// up the pieces, in chunk order.  A segment that goes on over more than 16 chunks (a hub
-// column: hundreds) is added up by the whole wave instead of one lane walking the pieces.
+// One lane per tile: a tile that holds the head of a long segment going on after it adds
+// up the pieces, in tile order.  A segment that goes on over more than 16 tiles (a hub
+// column) is added up by the whole wave instead of one lane walking the pieces.
 template <typename IdT>
 __global__ void __launch_bounds__(kThreads)
 carry_kernel(const int64_t* __restrict__ indptr, const IdT* __restrict__ nmap, int64_t num_seg,
-             int64_t nnz, float* __restrict__ sums, Chunks ck) {
-  if (*ck.any_long == 0u) return;
+             int64_t nnz, float* __restrict__ sums, Tiles tl) {
   if (indptr[num_seg] < nnz) nnz = indptr[num_seg];
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t c = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
   int g = -1;
-  int64_t last = 0;  // last chunk the segment reaches
-  if (c * kChunk < nnz) {
-    g = ck.outgoing[c];
-    if (g >= 0) last = (indptr[g + 1] - 1) / kChunk;
+  int64_t last = 0;  // last tile the segment reaches
+  if (t * kTile < nnz) {
+    g = tl.outgoing[t];
+    if (g >= 0) last = (indptr[g + 1] - 1) / kTile;
   }
-  const bool wide = g >= 0 && last - c > kCarryAlone;
+  const bool wide = g >= 0 && last - t > kCarryAlone;
   if (g >= 0 && !wide) {
-    float total = ck.carry[2 * c + 1];
-    for (int64_t k = c + 1; k <= last; ++k) total += ck.carry[2 * k];
+    float total = tl.carry[2 * t + 1];
+    for (int64_t k = t + 1; k <= last; ++k) total += tl.carry[2 * k];
     sums[nmap ? static_cast<int64_t>(nmap[g]) : g] = total;
   }
   unsigned long long todo = __ballot(wide);
   while (todo) {
     const int l = __ffsll(static_cast<long long>(todo)) - 1;
     todo &= todo - 1;
-    const int64_t from = __shfl(c, l, kWave) + 1;
+    const int64_t from = __shfl(t, l, kWave) + 1;
     const int64_t to = __shfl(last, l, kWave);
     float part = 0.0f;
-    for (int64_t k = from + lane; k <= to; k += kWave) part += ck.carry[2 * k];
+    for (int64_t k = from + lane; k <= to; k += kWave) part += tl.carry[2 * k];
 #pragma unroll
     for (int d = kWave / 2; d > 0; d >>= 1) part += __shfl_xor(part, d, kWave);
-    if (lane == l) sums[nmap ? static_cast<int64_t>(nmap[g]) : g] = ck.carry[2 * c + 1] + part;
+    if (lane == l) sums[nmap ? static_cast<int64_t>(nmap[g]) : g] = tl.carry[2 * t + 1] + part;
   }
 }
 
-// The steps of a chunk in the divide pass.  AHEAD: a full chunk of plain, aligned data, whose
-// four reads were issued before the marks were made; that variant contains no read at all, so
-// its stores follow one another without waiting (in one body with the other variant every
-// step waited for the store of the step before: a read that may happen makes the compiler
-// wait for all that is in flight).
-template <bool AHEAD>
-__device__ __forceinline__ void divide_steps(const int* mark, const Owned& own, float own_sum,
-                                             const float4 (&early)[kChunk / kStep],
-                                             const int64_t* __restrict__ emap,
-                                             const float* __restrict__ data, int64_t begin,
-                                             int64_t end, int lane, float* __restrict__ out) {
-  int carried = 0;
-#pragma unroll
-  for (int t = 0; t < kChunk / kStep; ++t) {
-    const int64_t base = begin + t * kStep;
-    if (!AHEAD && base >= end) break;
-    const int at0 = static_cast<int>(base - begin) + lane * kLaneEdges;
-    const int64_t e0 = base + lane * kLaneEdges;
-    int m[kLaneEdges];
-    {
-      const int4 mm = *reinterpret_cast<const int4*>(mark + at0);
-      m[0] = mm.x; m[1] = mm.y; m[2] = mm.z; m[3] = mm.w;
-    }
-    if (!AHEAD) {
-#pragma unroll
-      for (int k = 0; k < kLaneEdges; ++k)
-        if (e0 + k >= end) m[k] = 0;
-    }
-    const LaneMarks lm = scan_lane_marks(m, at0);
-    const int incl = latest_inclusive(lm.last_packed, carried, lane);
-    int cur = lane_move<0x138, 0xf>(carried, incl);
-    carried = __builtin_amdgcn_readlane(incl, kWave - 1);
-    const float have[kLaneEdges] = {early[t].x, early[t].y, early[t].z, early[t].w};
-    float res[kLaneEdges];
-    bool mine[kLaneEdges];
-#pragma unroll
-    for (int k = 0; k < kLaneEdges; ++k) {
-      if (m[k]) cur = (at0 + k + 1) << 8 | m[k];
-      const int owner = owner_of_mark(cur);
-      const float total = __shfl(own_sum, owner >= 0 ? owner : 0, kWave);
-      const int64_t e = e0 + k;
-      mine[k] = (AHEAD || e < end) && owner >= 0;
-      res[k] = 0.0f;
-      if (AHEAD) res[k] = have[k] / total;
-      else if (mine[k]) res[k] = data[emap ? emap[e] : e] / total;
-    }
-    if (AHEAD && mine[0] && mine[1] && mine[2] && mine[3]) {
-      *reinterpret_cast<float4*>(out + e0) = make_float4(res[0], res[1], res[2], res[3]);
-    } else {
-#pragma unroll
-      for (int k = 0; k < kLaneEdges; ++k)
-        if (mine[k]) out[!AHEAD && emap ? emap[e0 + k] : e0 + k] = res[k];
-    }
-  }
+inline Source source_of(const int64_t* emap, const float* data) {
+  if (emap) return kMapped;
+  return (reinterpret_cast<uintptr_t>(data) & 15u) == 0 ? kPlain : kLoose;
 }
 
-// out[d] = data[d] / sums[segment of e] for the edges of long segments
-__global__ void __launch_bounds__(kThreads)
-long_divide_kernel(const int64_t* __restrict__ indptr, const int64_t* __restrict__ emap,
-                   const float* __restrict__ data, int64_t num_seg, int64_t nnz,
-                   const float* __restrict__ sums, float* __restrict__ out, Chunks ck) {
-  __shared__ __attribute__((aligned(16))) int s_mark[kWaves][kChunk];
-  if (*ck.any_long == 0u) return;
-  if (indptr[num_seg] < nnz) nnz = indptr[num_seg];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t c = static_cast<int64_t>(blockIdx.x) * kWaves + threadIdx.x / kWave;
-  const int64_t begin = c * kChunk;
-  if (begin >= nnz) return;
-  const int64_t end = begin + kChunk < nnz ? begin + kChunk : nnz;
-  int* mark = s_mark[threadIdx.x / kWave];
-  const Owned own = load_owned(indptr, ck, c, lane);
-  if (__ballot(own.g >= 0) == 0ull) return;  // no long segment touches the chunk
-  const float own_sum = own.g >= 0 ? sums[own.g] : 0.0f;
-  // a full chunk of plain data: all four steps' reads are issued together
-  const bool ahead = !emap && end - begin == kChunk &&
-                     ((reinterpret_cast<uintptr_t>(data) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
-  float4 early[kChunk / kStep];
-#pragma unroll
-  for (int t = 0; t < kChunk / kStep; ++t) early[t] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  // the whole chunk lies inside the incoming segment: one divisor, no marks
-  if (__shfl(own.g >= 0 ? own.e : int64_t(0), kIncomingLane, kWave) >= end) {
-    const float total = __shfl(own_sum, kIncomingLane, kWave);
-    if (ahead) {
-#pragma unroll
-      for (int t = 0; t < kChunk / kStep; ++t)
-        early[t] = *reinterpret_cast<const float4*>(data + begin + t * kStep + lane * kLaneEdges);
-#pragma unroll
-      for (int t = 0; t < kChunk / kStep; ++t)
-        *reinterpret_cast<float4*>(out + begin + t * kStep + lane * kLaneEdges) =
-            make_float4(early[t].x / total, early[t].y / total, early[t].z / total,
-                        early[t].w / total);
-      return;
-    }
-    for (int64_t e = begin + lane; e < end; e += kWave) {
-      const int64_t d = emap ? emap[e] : e;
-      out[d] = data[d] / total;
-    }
-    return;
-  }
-  if (ahead) {
-#pragma unroll
-    for (int t = 0; t < kChunk / kStep; ++t)
-      early[t] = *reinterpret_cast<const float4*>(data + begin + t * kStep + lane * kLaneEdges);
-  }
-  write_marks(mark, own, begin, end, lane);
-  if (ahead)
-    divide_steps<true>(mark, own, own_sum, early, emap, data, begin, end, lane, out);
-  else
-    divide_steps<false>(mark, own, own_sum, early, emap, data, begin, end, lane, out);
-}
+inline int64_t num_tiles(int64_t nnz) { return nnz <= 0 ? 1 : (nnz + kTile - 1) / kTile; }
 
-inline int64_t num_chunks(int64_t nnz) { return nnz <= 0 ? 1 : (nnz + kChunk - 1) / kChunk; }
+// The marks cost 12 bytes per edge; walking the offsets costs a workgroup a round of 256 per
+// 256 segments of its tile, and from eight rounds a tile on that is the longer way.
+inline bool use_marks(int64_t num_seg, int64_t nnz) { return 2 * num_seg > nnz; }
+constexpr int64_t kSearchTiles = 512;  // up to here a normalise's workgroups look for their first segment
 
-struct SegmentScratch {
-  Chunks ck;
-  float* sums;  // normalize only
-  bool ok;
-};
-
-SegmentScratch carve_segment(void* workspace, size_t bytes, int64_t nnz, int64_t num_seg,
-                             bool with_sums) {
+bool carve_tiles(void* workspace, size_t bytes, int64_t num_seg, int64_t nnz, Tiles* tl) {
   Carver ws(workspace, bytes);
-  const int64_t chunks = num_chunks(nnz);
-  SegmentScratch s;
-  s.ck.any_long = ws.take<unsigned int>(64);
-  s.ck.count = ws.take<unsigned int>(chunks);
-  s.ck.list = ws.take<int>(chunks * kChunkList);
-  s.ck.incoming = ws.take<int>(chunks);
-  s.ck.outgoing = ws.take<int>(chunks);
-  s.ck.carry = ws.take<float>(2 * chunks);
-  s.sums = with_sums ? ws.take<float>(num_seg > 0 ? num_seg : 1) : nullptr;
-  s.ok = ws.ok;
-  return s;
+  const size_t tiles = static_cast<size_t>(num_tiles(nnz));
+  tl->head = ws.take<int>(tiles + 1);
+  tl->outgoing = ws.take<int>(tiles);
+  tl->carry = ws.take<float>(2 * tiles);
+  tl->inner = ws.take<int>(tiles);
+  tl->mark = use_marks(num_seg, nnz) ? ws.take<int>(static_cast<size_t>(nnz > 0 ? nnz : 1)) : nullptr;
+  return ws.ok;
 }
 
 size_t segment_workspace_bytes(int64_t num_seg, int64_t nnz) {
-  const size_t chunks = static_cast<size_t>(num_chunks(nnz));
-  return padded(256) + 3 * padded(chunks * 4) + padded(chunks * kChunkList * 4) +
-         padded(chunks * 8) + padded(static_cast<size_t>(num_seg > 0 ? num_seg : 1) * 4);
+  const size_t tiles = static_cast<size_t>(num_tiles(nnz));
+  return padded((tiles + 1) * 4) + 2 * padded(tiles * 4) + padded(tiles * 8) +
+         (use_marks(num_seg, nnz) ? padded(static_cast<size_t>(nnz > 0 ? nnz : 1) * 4) : 0);
+}
+
+// what the tiles' workgroups find in head[] and mark[]
+template <bool SUM, typename IdT>
+void launch_heads(const int64_t* indptr, const IdT* nmap, int64_t num_seg, int64_t nnz, float* out,
+                  const Tiles& tl, hipStream_t st) {
+  const dim3 grid(blocks_for(num_seg, kThreads));
+  if (!tl.mark) {
+    hipLaunchKernelGGL((tile_heads_kernel<SUM, false, IdT>), grid, dim3(kThreads), 0, st, indptr,
+                       nmap, num_seg, out, tl);
+    return;
+  }
+  hipLaunchKernelGGL(clear_marks_kernel, dim3(blocks_for(nnz, kTile)), dim3(kThreads), 0, st, tl.mark,
+                     nnz);
+  hipLaunchKernelGGL((tile_heads_kernel<SUM, true, IdT>), grid, dim3(kThreads), 0, st, indptr, nmap,
+                     num_seg, out, tl);
 }
 
 template <typename IdT>
 int segment_sum_impl(const int64_t* indptr, const int64_t* emap, const void* nmap,
                      const float* data, int64_t num_seg, int64_t nnz, int powk, float* out,
-                     const SegmentScratch& s, hipStream_t st) {
+                     const Tiles& tl, hipStream_t st) {
   const IdT* nm = static_cast<const IdT*>(nmap);
-  const int64_t chunks = num_chunks(nnz);
-  hipLaunchKernelGGL(clear_chunks_kernel, dim3(blocks_for(chunks, kThreads)), dim3(kThreads), 0, st,
-                     s.ck, chunks);
-  if (emap)
-    hipLaunchKernelGGL((short_segments_kernel<false, true, IdT>), dim3(blocks_for(num_seg, kThreads)),
-                       dim3(kThreads), 0, st, indptr, emap, nm, data, num_seg, nnz, powk, out, s.ck);
-  else
-    hipLaunchKernelGGL((short_segments_kernel<false, false, IdT>), dim3(blocks_for(num_seg, kThreads)),
-                       dim3(kThreads), 0, st, indptr, emap, nm, data, num_seg, nnz, powk, out, s.ck);
-  if (nnz > kLaneMaxLen) {
-    hipLaunchKernelGGL(long_segments_kernel<IdT>, dim3(blocks_for(chunks, kWaves)), dim3(kThreads),
-                       0, st, indptr, emap, nm, data, num_seg, nnz, powk, out, s.ck);
-    hipLaunchKernelGGL(carry_kernel<IdT>, dim3(blocks_for(chunks, kThreads)), dim3(kThreads), 0, st,
-                       indptr, nm, num_seg, nnz, out, s.ck);
-  }
+  const int64_t tiles = num_tiles(nnz);
+  launch_heads<true>(indptr, nm, num_seg, nnz, out, tl, st);
+  auto pick = [&](auto walk) {
+    constexpr Walk W = decltype(walk)::value;
+    switch (source_of(emap, data)) {
+      case kMapped: return segment_tiles_kernel<false, kMapped, W, IdT>;
+      case kLoose: return segment_tiles_kernel<false, kLoose, W, IdT>;
+      default: return segment_tiles_kernel<false, kPlain, W, IdT>;
+    }
+  };
+  auto* kernel = tl.mark ? pick(std::integral_constant<Walk, kMarks>{})
+                         : pick(std::integral_constant<Walk, kHeads>{});
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(kThreads), 0, st, indptr, emap,
+                     nm, data, num_seg, nnz, powk, out, tl);
+  if (tiles > 1)
+    hipLaunchKernelGGL((carry_kernel<IdT>), dim3(blocks_for(tiles, kThreads)), dim3(kThreads), 0, st,
+                       indptr, nm, num_seg, nnz, out, tl);
   return check_launch("segment_sum");
+}
+
+template <Source SOURCE>
+void launch_normalize(Walk walk, const int64_t* indptr, const int64_t* emap, const float* data,
+                      int64_t num_seg, int64_t nnz, float* out, const Tiles& tl, hipStream_t st) {
+  const int64_t* no_map = nullptr;
+  const int64_t tiles = num_tiles(nnz);
+  auto* kernel = walk == kSearch   ? segment_tiles_kernel<true, SOURCE, kSearch, int64_t>
+                 : walk == kHeads ? segment_tiles_kernel<true, SOURCE, kHeads, int64_t>
+                                  : segment_tiles_kernel<true, SOURCE, kMarks, int64_t>;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(kThreads), 0, st, indptr, emap,
+                     no_map, data, num_seg, nnz, 1, out, tl);
+  if (tiles > 1)
+    hipLaunchKernelGGL((crossing_divide_kernel<SOURCE == kMapped>),
+                       dim3(static_cast<unsigned>(tiles)), dim3(kThreads), 0, st, indptr, emap, data,
+                       num_seg, nnz, out, tl);
+}
+
+int segment_normalize_impl(const int64_t* indptr, const int64_t* emap, const float* data,
+                           int64_t num_seg, int64_t nnz, float* out, const Tiles& tl,
+                           hipStream_t st) {
+  // (few tiles: a launch costs more than the search)
+  const Walk walk = tl.mark ? kMarks : (num_tiles(nnz) > kSearchTiles ? kHeads : kSearch);
+  if (walk != kSearch)
+    launch_heads<false>(indptr, static_cast<const int64_t*>(nullptr), num_seg, nnz, out, tl, st);
+  const Source source = source_of(emap, data);
+  auto* launch = source == kMapped  ? launch_normalize<kMapped>
+                 : source == kLoose ? launch_normalize<kLoose>
+                                    : launch_normalize<kPlain>;
+  launch(walk, indptr, emap, data, num_seg, nnz, out, tl, st);
+  return check_launch("segment_normalize");
 }
 
 // Sums by an arbitrary key (COO targets).  The reference adds every edge to its target with a
@@ -728,18 +770,15 @@ int gs_segment_sum(const int64_t* indptr, const int64_t* e_ids, const void* n_id
              id_bytes);
   GS_REQUIRE(num_segments < (int64_t(1) << 31), "gs_segment_sum: more than 2^31 segments");
   if (num_segments == 0) return GS_OK;
-  SegmentScratch s = carve_segment(workspace, workspace_bytes, nnz, num_segments, false);
-  if (!s.ok) {
+  Tiles tl;
+  if (!carve_tiles(workspace, workspace_bytes, num_segments, nnz, &tl)) {
     set_error_text("gs_segment_sum: workspace needs %zu bytes, 256-byte aligned",
                    gs_segment_workspace_bytes(num_segments, nnz));
     return GS_ERR_WORKSPACE;
   }
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  return n_ids && id_bytes == 4
-             ? segment_sum_impl<int32_t>(indptr, e_ids, n_ids, data, num_segments, nnz,
-                                         static_cast<int>(powk), out, s, st)
-             : segment_sum_impl<int64_t>(indptr, e_ids, n_ids, data, num_segments, nnz,
-                                         static_cast<int>(powk), out, s, st);
+  auto* impl = n_ids && id_bytes == 4 ? segment_sum_impl<int32_t> : segment_sum_impl<int64_t>;
+  return impl(indptr, e_ids, n_ids, data, num_segments, nnz, static_cast<int>(powk), out, tl,
+              static_cast<hipStream_t>(stream));
 }
 
 int gs_coo_sum(const void* target, int id_bytes, const int64_t* e_ids, const float* data, int64_t E,
@@ -781,35 +820,14 @@ int gs_segment_normalize(const int64_t* indptr, const int64_t* e_ids, const floa
   GS_REQUIRE(num_segments == 0 || nnz == 0 || (indptr && data && out),
              "gs_segment_normalize: null pointer");
   if (num_segments == 0 || nnz == 0) return GS_OK;
-  SegmentScratch s = carve_segment(workspace, workspace_bytes, nnz, num_segments, true);
-  if (!s.ok) {
+  Tiles tl;
+  if (!carve_tiles(workspace, workspace_bytes, num_segments, nnz, &tl)) {
     set_error_text("gs_segment_normalize: workspace needs %zu bytes, 256-byte aligned",
                    gs_segment_workspace_bytes(num_segments, nnz));
     return GS_ERR_WORKSPACE;
   }
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const int64_t* no_map = nullptr;
-  const int64_t chunks = num_chunks(nnz);
-  hipLaunchKernelGGL(clear_chunks_kernel, dim3(blocks_for(chunks, kThreads)), dim3(kThreads), 0, st,
-                     s.ck, chunks);
-  if (e_ids)
-    hipLaunchKernelGGL((short_segments_kernel<true, true, int64_t>),
-                       dim3(blocks_for(num_segments, kThreads)), dim3(kThreads), 0, st, indptr,
-                       e_ids, no_map, data, num_segments, nnz, 1, out, s.ck);
-  else
-    hipLaunchKernelGGL((short_segments_kernel<true, false, int64_t>),
-                       dim3(blocks_for(num_segments, kThreads)), dim3(kThreads), 0, st, indptr,
-                       e_ids, no_map, data, num_segments, nnz, 1, out, s.ck);
-  if (nnz > kLaneMaxLen) {
-    hipLaunchKernelGGL(long_segments_kernel<int64_t>, dim3(blocks_for(chunks, kWaves)),
-                       dim3(kThreads), 0, st, indptr, e_ids, no_map, data, num_segments, nnz, 1,
-                       s.sums, s.ck);
-    hipLaunchKernelGGL(carry_kernel<int64_t>, dim3(blocks_for(chunks, kThreads)), dim3(kThreads), 0,
-                       st, indptr, no_map, num_segments, nnz, s.sums, s.ck);
-    hipLaunchKernelGGL(long_divide_kernel, dim3(blocks_for(chunks, kWaves)), dim3(kThreads), 0, st,
-                       indptr, e_ids, data, num_segments, nnz, s.sums, out, s.ck);
-  }
-  return check_launch("segment_normalize");
+  return segment_normalize_impl(indptr, e_ids, data, num_segments, nnz, out, tl,
+                                static_cast<hipStream_t>(stream));
 }
 
 int gs_e_div_u_sum(const void* row, const void* col, int id_bytes, const float* data,
