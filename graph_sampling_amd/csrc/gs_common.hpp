@@ -269,6 +269,14 @@ __device__ __forceinline__ void block_row_range(const int64_t* __restrict__ ptr,
   __syncthreads();
 }
 
+// Value of the lane `CTRL` names, a data-parallel-primitive move inside the vector ALU with no
+// trip through the LDS crossbar (0x121 .. 0x12f: the row of 16 turned by 1 .. 15 lanes).
+template <int CTRL>
+__device__ __forceinline__ float lane_move(float v) {
+  const int bits = __builtin_bit_cast(int, v);
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, bits, CTRL, 0xf, 0xf, false));
+}
+
 // ------------------------------------------------------------ block scan ----
 // Exclusive scan of one int64 per thread over a block of kThreads threads
 // (multiple of 64).  Returns the exclusive prefix; *total gets the block sum.

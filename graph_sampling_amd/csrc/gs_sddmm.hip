@@ -5,10 +5,10 @@
 //
 // None of this is a dense contraction: every edge gathers two feature rows at
 // random, so the kernels are HBM/latency bound and use no MFMA.
-//  * dot without broadcast (the layer-wise samplers' u_dot_v): a group of
-//    16 lanes per edge reads both rows as float4 (one 256 B row of a 64-wide
-//    feature = one fully coalesced request), multiplies, and reduces with a
-//    4-step butterfly; 4 edges per wave.
+//  * dot without broadcast (the layer-wise samplers' u_dot_v): a group of 2 to
+//    16 lanes per edge and head reads both rows as float4 (one 256 B row of a
+//    64-wide feature = one fully coalesced request), multiplies, and adds up
+//    across the lanes.
 //  * everything else: the reference's 2-D edge x feature decomposition
 //    (sddmm.cu:197-209) with the operator and targets as template parameters.
 //  * CSC flavour: the owning column of an edge comes from a binary search over
@@ -326,36 +326,107 @@ void launch_scalar_flat(const SddmmArgs<IdT>& a, hipStream_t st) {
   hipLaunchKernelGGL((sddmm_scalar_flat_kernel<OP, IdT>), dim3(grid), dim3(kThreads), 0, st, a);
 }
 
-// dot, no broadcast, out_len == 1, R % 4 == 0 and 16-byte aligned rows.
-constexpr int kDotGroup = 16;
-constexpr int kDotEdges = 4;  // edges per 16-lane group
-template <typename IdT>
-__global__ void __launch_bounds__(kThreads) sddmm_dot_rows_kernel(SddmmArgs<IdT> a) {
+// dot without broadcast: `heads` sums of R products per edge over the edge's two rows of
+// heads * R floats each, one group of G lanes per (edge, head), VEC floats a lane and read.
+//
+// A workgroup takes up to 256 consecutive edges.  It first looks up where both rows of every edge
+// are, an edge per thread, and leaves that in LDS; the groups then go over the (edge, head) pairs,
+// consecutive groups on consecutive pairs, four pairs at a time with all their rows' reads in
+// flight together.  (With the ends looked up by each group for itself, in front of each edge's
+// rows, a group had two dependent reads to wait for per edge and one edge's rows in flight.)
+//
+// The rows' bytes bound it, most of them read at random: 8 M edges of 2.45 M nodes, 64 floats
+// on either end, 441 -> 313 us, of which 1.35 GB at the rate of a copy are 282; five waves a
+// SIMD or eight, two pairs at a time or four, 16-byte reads take the same.  (Eight pairs: 573, the
+// registers spill.)  The several heads and the widths that are no multiple of four had been left
+// to the general kernel, a lane per sum: 2.8 M edges of 8 x 8 491 -> 94 us, 5 M edges of
+// 50 1494 -> 171 us.
+constexpr int kDotTile = 256;
+constexpr int kDotPairs = 4;
+
+// sum over groups of G consecutive lanes, in every lane of the group
+template <int G>
+__device__ __forceinline__ float group_sum(float x) {
+  if (G >= 2) x += lane_move<0xB1>(x);    // the other lane of a pair
+  if (G >= 4) x += lane_move<0x4E>(x);    // the other pair of a quad
+  if (G >= 8) x += lane_move<0x141>(x);   // eight lanes mirrored
+  if (G >= 16) x += lane_move<0x140>(x);  // sixteen lanes mirrored
+  return x;
+}
+
+template <int VEC, int G, typename IdT>
+__global__ void __launch_bounds__(kThreads, 4)
+sddmm_dot_kernel(SddmmArgs<IdT> a, int tile) {
+  using V = float __attribute__((ext_vector_type(VEC)));
   __shared__ int64_t s_range[2];
   __shared__ int64_t s_ptr[kStageCols];
-  const int lane = threadIdx.x % kDotGroup;
-  constexpr int kGroups = kThreads / kDotGroup;
-  const int64_t e0 = static_cast<int64_t>(blockIdx.x) * (kGroups * kDotEdges);
-  block_column_range(a, e0, e0 + kGroups * kDotEdges - 1, s_range, s_ptr);
-  for (int j = 0; j < kDotEdges; ++j) {
-    const int64_t e = e0 + j * kGroups + threadIdx.x / kDotGroup;
-    if (e >= a.E) return;
+  __shared__ int64_t s_l[kDotTile], s_r[kDotTile], s_o[kDotTile];
+  const int64_t e0 = static_cast<int64_t>(blockIdx.x) * tile;
+  const int n = static_cast<int>(a.E - e0 < tile ? a.E - e0 : tile);
+  const int tid = threadIdx.x, lane = tid % G, group = tid / G;
+  constexpr int kGroups = kThreads / G;
+  const bool need_src = a.lhs_target == 0 || a.rhs_target == 0;
+  const bool need_dst = a.lhs_target == 2 || a.rhs_target == 2;
+  if (need_dst) block_column_range(a, e0, e0 + n - 1, s_range, s_ptr);
+  if (tid < n) {
     int64_t src, dst, eid;
-    edge_endpoints(a, e, s_range, s_ptr, true, true, &src, &dst, &eid);
-    const float4* l =
-        reinterpret_cast<const float4*>(a.lhs + select3(a.lhs_target, src, eid, dst) * a.lhs_len);
-    const float4* r =
-        reinterpret_cast<const float4*>(a.rhs + select3(a.rhs_target, src, eid, dst) * a.rhs_len);
-    float acc = 0.0f;
-    for (int64_t i = lane; i < a.R / 4; i += kDotGroup) {
-      const float4 x = l[i];
-      const float4 y = r[i];
-      acc += x.x * y.x + x.y * y.y + x.z * y.z + x.w * y.w;
+    edge_endpoints(a, e0 + tid, s_range, s_ptr, need_src, need_dst, &src, &dst, &eid);
+    s_l[tid] = select3(a.lhs_target, src, eid, dst) * a.lhs_len;
+    s_r[tid] = select3(a.rhs_target, src, eid, dst) * a.rhs_len;
+    s_o[tid] = eid * a.out_len;
+  }
+  __syncthreads();
+  // pair `at` of the tile is (edge, head); kGroups pairs further on it is (edge + de, head + dh)
+  const int heads = static_cast<int>(a.out_len), R = static_cast<int>(a.R);
+  const int de = kGroups / heads, dh = kGroups % heads;
+  int edge = group / heads, head = group % heads;
+  while (edge < n) {
+    const float *l[kDotPairs], *r[kDotPairs];
+    float* o[kDotPairs];
+#pragma unroll
+    for (int j = 0; j < kDotPairs; ++j) {
+      const int e = edge < n ? edge : n - 1;  // (past the end: a pair of the last edge, not stored)
+      l[j] = a.lhs + s_l[e] + static_cast<int64_t>(head) * R;
+      r[j] = a.rhs + s_r[e] + static_cast<int64_t>(head) * R;
+      o[j] = edge < n && lane == 0 ? a.out + s_o[e] + head : nullptr;
+      edge += de;
+      head += dh;
+      if (head >= heads) {
+        head -= heads;
+        ++edge;
+      }
+    }
+    float acc[kDotPairs] = {};
+    for (int i = lane * VEC; i < R; i += G * VEC) {
+      V x[kDotPairs], y[kDotPairs];
+#pragma unroll
+      for (int j = 0; j < kDotPairs; ++j) {
+        x[j] = *reinterpret_cast<const V*>(l[j] + i);
+        y[j] = *reinterpret_cast<const V*>(r[j] + i);
+      }
+#pragma unroll
+      for (int j = 0; j < kDotPairs; ++j)
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) acc[j] += x[j][k] * y[j][k];
     }
 #pragma unroll
-    for (int d = kDotGroup / 2; d > 0; d >>= 1) acc += __shfl_xor(acc, d, kDotGroup);
-    if (lane == 0) a.out[eid] = acc;
+    for (int j = 0; j < kDotPairs; ++j) {
+      const float sum = group_sum<G>(acc[j]);
+      if (o[j]) *o[j] = sum;
+    }
   }
+}
+
+template <int VEC, typename IdT>
+void launch_dot(const SddmmArgs<IdT>& a, hipStream_t st) {
+  // small tiles while there are fewer than eight of the large ones for each of 256 CUs
+  const int tile = a.E >= kDotTile * 2048 ? kDotTile : kDotTile / 4;
+  const dim3 grid(static_cast<unsigned>((a.E + tile - 1) / tile)), block(kThreads);
+  const int64_t reads = (a.R + VEC - 1) / VEC;  // of one row's head
+  if (reads > 8) hipLaunchKernelGGL((sddmm_dot_kernel<VEC, 16, IdT>), grid, block, 0, st, a, tile);
+  else if (reads > 4) hipLaunchKernelGGL((sddmm_dot_kernel<VEC, 8, IdT>), grid, block, 0, st, a, tile);
+  else if (reads > 2) hipLaunchKernelGGL((sddmm_dot_kernel<VEC, 4, IdT>), grid, block, 0, st, a, tile);
+  else hipLaunchKernelGGL((sddmm_dot_kernel<VEC, 2, IdT>), grid, block, 0, st, a, tile);
 }
 
 template <int OP, typename IdT>
@@ -371,15 +442,14 @@ void launch_generic(const SddmmArgs<IdT>& a, hipStream_t st) {
 template <typename IdT>
 int sddmm_dispatch(int op, const SddmmArgs<IdT>& a, hipStream_t st) {
   if (a.E == 0 || a.out_len == 0) return GS_OK;
-  const bool aligned = (reinterpret_cast<uintptr_t>(a.lhs) % 16 == 0) &&
-                       (reinterpret_cast<uintptr_t>(a.rhs) % 16 == 0) && a.lhs_len % 4 == 0 &&
-                       a.rhs_len % 4 == 0;
-  if (op == GS_OP_DOT && !a.lhs_off && !a.rhs_off && a.out_len == 1 && a.R % 4 == 0 && a.R >= 16 &&
-      aligned) {
-    const int64_t per_block = static_cast<int64_t>(kThreads / kDotGroup) * kDotEdges;
-    const unsigned grid = static_cast<unsigned>((a.E + per_block - 1) / per_block);
+  // A read takes as many floats as both rows' starts and R are multiples of.
+  if (op == GS_OP_DOT && !a.lhs_off && !a.rhs_off && a.R >= 2 && a.R < (int64_t(1) << 30) &&
+      a.out_len < (int64_t(1) << 30) && a.lhs_len == a.out_len * a.R && a.rhs_len == a.lhs_len) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(a.lhs) | reinterpret_cast<uintptr_t>(a.rhs);
     ProfileScope prof("sddmm_dot", st);
-    hipLaunchKernelGGL(sddmm_dot_rows_kernel<IdT>, dim3(grid), dim3(kThreads), 0, st, a);
+    if (a.R % 4 == 0 && at % 16 == 0) launch_dot<4>(a, st);
+    else if (a.R % 2 == 0 && at % 8 == 0) launch_dot<2>(a, st);
+    else launch_dot<1>(a, st);
     return check_launch("sddmm_dot");
   }
   const bool to_dst = a.lhs_target == 2 || a.rhs_target == 2;

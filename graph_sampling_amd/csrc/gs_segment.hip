@@ -37,14 +37,6 @@ constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWave;
 constexpr int64_t kLaneMaxLen = 16;
 
-// Value of the lane `CTRL` names, a data-parallel-primitive move inside the vector ALU with no
-// trip through the LDS crossbar (0x121 .. 0x12f: the row of 16 turned by 1 .. 15 lanes).
-template <int CTRL>
-__device__ __forceinline__ float lane_move(float v) {
-  const int bits = __builtin_bit_cast(int, v);
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, bits, CTRL, 0xf, 0xf, false));
-}
-
 constexpr int kLaneEdges = 4;        // of one 16-byte read
 constexpr int kTileItems = 16;
 constexpr int kTile = kThreads * kTileItems;

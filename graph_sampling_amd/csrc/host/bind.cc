@@ -89,6 +89,7 @@ TORCH_LIBRARY(gs_classes, m) {
       GS_DEF2("_CAPI_CSCMetadata", "_CAPI_csc_metadata", &Graph::CSCMetaData)
       GS_DEF2("_CAPI_RandomWalk", "_CAPI_random_walk", &Graph::RandomWalk)
       GS_DEF2("_CAPI_SDDMM", "_CAPI_sddmm", &Graph::SDDMM)
+      GS_DEF2("_CAPI_SDDMMOut", "_CAPI_sddmm_out", &Graph::SDDMMOut)
       GS_DEF2("_CAPI_GetCSC", "_CAPI_get_csc", &Graph::GetCSCTensor)
       GS_DEF2("_CAPI_GetCSR", "_CAPI_get_csr", &Graph::GetCSRTensor)
       GS_DEF2("_CAPI_GetBatchCSC", "GetBatchCSC", &Graph::GetBatchCSC)

@@ -997,6 +997,21 @@ void Graph::SDDMM(const std::string& op, torch::Tensor lhs, torch::Tensor rhs, t
   }
 }
 
+torch::Tensor Graph::SDDMMOut(const std::string& op, torch::Tensor lhs, torch::Tensor rhs,
+                              std::vector<int64_t> shape, int64_t lhs_target, int64_t rhs_target,
+                              int64_t on_format) {
+  Settle();
+  shape.insert(shape.begin(), num_edges_);
+  if (num_edges_ == 0) return torch::zeros(shape, lhs.options());
+  CreateSparseFormat(on_format);
+  const auto& fmt = on_format == _COO ? coo_->e_ids : IsCsrLike(on_format) ? csr_->e_ids : csc_->e_ids;
+  // edge i is row i of the result, so every row is written; where the edges go by ids of theirs,
+  // a row that no edge names is zero
+  torch::Tensor out = fmt.has_value() ? torch::zeros(shape, lhs.options()) : torch::empty(shape, lhs.options());
+  SDDMM(op, lhs, rhs, out, lhs_target, rhs_target, on_format);
+  return out;
+}
+
 // ---------------------------------------------------------------- node queries
 torch::Tensor Graph::AllValidNode() {
   Range range("gs::AllValidNode");

@@ -245,6 +245,10 @@ class Graph : public torch::CustomClassHolder {
   std::tuple<c10::intrusive_ptr<Graph>, torch::Tensor> EDivUSum(torch::Tensor divisor);
   void SDDMM(const std::string& op, torch::Tensor lhs, torch::Tensor rhs, torch::Tensor out,
              int64_t lhs_target, int64_t rhs_target, int64_t on_format);
+  // the same into a tensor of its own, [edges] + feature shape
+  torch::Tensor SDDMMOut(const std::string& op, torch::Tensor lhs, torch::Tensor rhs,
+                         std::vector<int64_t> shape, int64_t lhs_target, int64_t rhs_target,
+                         int64_t on_format);
 
   // ---- node queries; a "valid" node is a requested column or a non-isolated row
   torch::Tensor AllValidNode();

@@ -3,8 +3,6 @@
 import sys
 from itertools import product
 
-import torch
-
 from .format import _COO
 
 __all__ = ['gsddmm']
@@ -57,13 +55,9 @@ def gsddmm(g, op, lhs_data, rhs_data, lhs_target='u', rhs_target='v', on_format=
         lhs = lhs.unsqueeze(-1)
     if rhs.dim() == 1:
         rhs = rhs.unsqueeze(-1)
-    gidx = g._graph
-    num_edges = gidx._CAPI_GetNumEdges()
-    out = torch.zeros((num_edges,) + infer_broadcast_shape(op, lhs.shape[1:], rhs.shape[1:]),
-                      dtype=lhs.dtype, device=lhs.device)
-    if num_edges > 0:
-        gidx._CAPI_SDDMM(op, lhs.contiguous(), rhs.contiguous(), out, _TARGET[lhs_target],
-                         _TARGET[rhs_target], on_format)
+    out = g._graph._CAPI_SDDMMOut(op, lhs.contiguous(), rhs.contiguous(),
+                                  infer_broadcast_shape(op, lhs.shape[1:], rhs.shape[1:]),
+                                  _TARGET[lhs_target], _TARGET[rhs_target], on_format)
     return out.squeeze(-1) if squeeze else out
 
 
