@@ -56,7 +56,6 @@ constexpr int kCounterCap = 2 * (1 << kMaxClassesLog2) + (kPartTile >> (kBucketI
                             2 * static_cast<int>(kStagedBatches) + 2;
 constexpr int kSlots = 4096;           // LDS table of a bucket (8-byte slots)
 constexpr int kFlagTile = kThreads * 64;  // positions of a workgroup in the rank pass
-constexpr int kXcds = 8;
 constexpr int kTrip = 8;  // records of a thread that are asked for together (a whole average bucket)
 
 struct Plan {

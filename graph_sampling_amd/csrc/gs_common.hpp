@@ -12,6 +12,7 @@
 namespace gs {
 
 constexpr int kWave = 64;  // CDNA wavefront width
+constexpr int kXcds = 8;   // compute dies of the card: workgroup w runs on die w % 8
 
 // ---------------------------------------------------------------- status ----
 void set_error_text(const char* fmt, ...);
