@@ -366,10 +366,12 @@ class RelabelTable:
                "gs_relabel_table_init")
 
 
-def relabel_sampled(seed_keys, sub_indptr, sub_indices, table, mailbox=None, offsets_copy=None):
+def relabel_sampled(seed_keys, sub_indptr, sub_indices, table, mailbox=None, offsets_copy=None,
+                    num_ids=0):
     """gs_relabel_sampled behind a sampler whose total is still on the device (sub_indptr[S]).
     Returns (frontier buffer, num_unique (device), relabelled sampled ids at capacity[, ticket]);
-    `offsets_copy` (int64[S + 1]) receives a copy of sub_indptr."""
+    `offsets_copy` (int64[S + 1]) receives a copy of sub_indptr.  num_ids: how many different ids
+    there are, 0 when that is not known."""
     idb = _ids(seed_keys, "seed_keys")
     _ids(sub_indices, "sampled ids", like=seed_keys)
     dev = seed_keys.device
@@ -382,22 +384,13 @@ def relabel_sampled(seed_keys, sub_indptr, sub_indices, table, mailbox=None, off
     state, epoch = fused_state(lib().gs_relabel_sampled_state_bytes(_i64(M)), dev)
     ticket = mailbox.ticket() if mailbox is not None else 0
     box = mailbox.ptr() if mailbox is not None else ctypes.c_void_p(0)
-    if table.narrow:
-        _check(lib().gs_relabel_sampled_narrow(
-            _ptr(seed_keys), _i64(S), _ptr(sub_indices), _i64(cap),
-            ctypes.c_void_p(sub_indptr.data_ptr() + 8 * S), _ptr(table.buf),
-            ctypes.c_size_t(table.buf.numel()), _ptr(frontier), _ptr(out_ids), _ptr(num_unique),
-            _ptr(offsets_copy), _ptr(ws), ctypes.c_size_t(ws.numel()), _ptr(state),
-            ctypes.c_size_t(state.numel()), ctypes.c_uint32(epoch), box, _i64(ticket),
-            _stream(dev)), "gs_relabel_sampled_narrow")
-    else:
-        _check(lib().gs_relabel_sampled(
-            _ptr(seed_keys), _i64(S), _ptr(sub_indices), _i64(cap),
-            ctypes.c_void_p(sub_indptr.data_ptr() + 8 * S), idb, _ptr(table.buf),
-            ctypes.c_size_t(table.buf.numel()), _ptr(frontier), _ptr(out_ids), _ptr(num_unique),
-            _ptr(offsets_copy), _ptr(ws), ctypes.c_size_t(ws.numel()), _ptr(state),
-            ctypes.c_size_t(state.numel()), ctypes.c_uint32(epoch), box, _i64(ticket),
-            _stream(dev)), "gs_relabel_sampled")
+    _check(lib().gs_relabel_sampled_among(
+        _ptr(seed_keys), _i64(S), _ptr(sub_indices), _i64(cap),
+        ctypes.c_void_p(sub_indptr.data_ptr() + 8 * S), idb | (NARROW_IDS if table.narrow else 0),
+        _i64(num_ids), _ptr(table.buf), ctypes.c_size_t(table.buf.numel()), _ptr(frontier),
+        _ptr(out_ids), _ptr(num_unique), _ptr(offsets_copy), _ptr(ws),
+        ctypes.c_size_t(ws.numel()), _ptr(state), ctypes.c_size_t(state.numel()),
+        ctypes.c_uint32(epoch), box, _i64(ticket), _stream(dev)), "gs_relabel_sampled")
     if mailbox is not None:
         return frontier, num_unique, out_ids, ticket
     return frontier, num_unique, out_ids

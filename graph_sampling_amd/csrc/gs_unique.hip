@@ -78,7 +78,7 @@ __global__ void __launch_bounds__(kThreads) table_init_kernel(T t, int64_t cap, 
 // (unique_reindex.cu:92-99)
 // too_wide: set to 2 when T keeps 32 bits of a key and a key does not fit them (64-bit ids
 // on the one-word slots); the compaction then reports -2 instead of a count
-template <typename IdT, typename T, bool PEEK>
+template <typename IdT, typename T>
 __global__ void __launch_bounds__(kThreads)
 table_insert_kernel(Spans<IdT> x, int64_t M_bound, T t, uint32_t* __restrict__ pos,
                     unsigned int* __restrict__ too_wide) {
@@ -96,7 +96,7 @@ table_insert_kernel(Spans<IdT> x, int64_t M_bound, T t, uint32_t* __restrict__ p
     pos[i] = 0u;
     return;
   }
-  const uint32_t slot = t.template insert<PEEK>(static_cast<long long>(key), static_cast<uint32_t>(i));
+  const uint32_t slot = t.insert(static_cast<long long>(key), static_cast<uint32_t>(i));
   GS_STAMP(2);  // the slot is known
   pos[i] = slot;
   GS_STAMP(3);
@@ -112,7 +112,7 @@ table_insert_kernel(Spans<IdT> x, int64_t M_bound, T t, uint32_t* __restrict__ p
 constexpr int kGroupSlots = 1024;
 constexpr int kGroupProbes = 4;
 
-template <typename IdT, typename T>
+template <typename IdT, typename T, bool PEEK>
 __global__ void __launch_bounds__(kThreads)
 table_insert_grouped_kernel(Spans<IdT> x, int64_t M_bound, T t, uint32_t* __restrict__ pos,
                             unsigned int* __restrict__ too_wide) {
@@ -153,7 +153,7 @@ table_insert_grouped_kernel(Spans<IdT> x, int64_t M_bound, T t, uint32_t* __rest
   const bool leads = live && (slot < 0 || s_min[slot] == static_cast<unsigned int>(i));
   uint32_t p = 0u;
   if (leads) {
-    p = t.template insert<true>(static_cast<long long>(key), static_cast<uint32_t>(i));
+    p = t.template insert<PEEK>(static_cast<long long>(key), static_cast<uint32_t>(i));
     if (slot >= 0) s_pos[slot] = p;
   }
   __syncthreads();
@@ -415,7 +415,7 @@ int unique_relabel_impl(const gs_span* mapping, int n_mapping, const gs_span* qu
   if (M > 0) {
     ProfileScope prof("table_insert", stream);
     constexpr bool kNarrow = sizeof(IdT) == 8 && std::is_same<T, PackedTable>::value;
-    hipLaunchKernelGGL((table_insert_grouped_kernel<IdT, T>), dim3(blocks_for(M, kThreads)),
+    hipLaunchKernelGGL((table_insert_grouped_kernel<IdT, T, true>), dim3(blocks_for(M, kThreads)),
                        dim3(kThreads), 0, stream, x, M, t, pos,
                        kNarrow ? lb.error : static_cast<unsigned int*>(nullptr));
   }
@@ -436,7 +436,7 @@ int unique_relabel_impl(const gs_span* mapping, int n_mapping, const gs_span* qu
 
 template <typename IdT, typename T>
 int relabel_sampled_impl(const void* seed_keys, int64_t S, const void* sampled, int64_t capacity,
-                         const int64_t* sampled_len, void* table, size_t table_bytes,
+                         const int64_t* sampled_len, int64_t num_ids, void* table, size_t table_bytes,
                          void* frontier, void* out_ids, int64_t* num_unique,
                          int64_t* offsets_copy, void* workspace,
                          size_t workspace_bytes, void* state, size_t state_bytes, uint32_t epoch,
@@ -475,11 +475,15 @@ int relabel_sampled_impl(const void* seed_keys, int64_t S, const void* sampled, 
   x.fixed = S;
   if (M > 0) {
     ProfileScope prof("table_insert", stream);
-    // no peek here: sampled neighbours are mostly new keys, and the extra read costs the
-    // GraphSAGE step 7 % (0.152 ms against 0.142)
+    // No peek at the slot: sampled neighbours are mostly new keys, and the extra read costs the
+    // GraphSAGE step 7 % (0.152 ms against 0.142).  Nor a meeting in LDS first, 2-5 % of a
+    // minibatch on graphs of millions of nodes, unless the items are so many against the ids
+    // there are that hubs come up by the hundred: 5000 seeds, fanouts 25 and 15 on 233 k
+    // nodes, 1.07 M items in all: 134 -> 115 us a minibatch.
     constexpr bool kNarrow = sizeof(IdT) == 8 && std::is_same<T, PackedTable>::value;
-    hipLaunchKernelGGL((table_insert_kernel<IdT, T, false>), dim3(blocks_for(M, kThreads)),
-                       dim3(kThreads), 0, stream, x, M, t, pos,
+    const auto insert = num_ids > 0 && 2 * M >= num_ids ? table_insert_grouped_kernel<IdT, T, false>
+                                                        : table_insert_kernel<IdT, T>;
+    hipLaunchKernelGGL(insert, dim3(blocks_for(M, kThreads)), dim3(kThreads), 0, stream, x, M, t, pos,
                        kNarrow ? lb.error : static_cast<unsigned int*>(nullptr));
   }
   {
@@ -1438,19 +1442,20 @@ size_t gs_relabel_sampled_state_bytes(int64_t num_items) {
   return lookback_state_bytes(compact_num_tiles(num_items));
 }
 
-int gs_relabel_sampled(const void* seed_keys, int64_t S, const void* sampled, int64_t capacity,
-                       const int64_t* sampled_len, int id_bytes, void* table, size_t table_bytes,
-                       void* frontier, void* out_ids, int64_t* num_unique,
-                       int64_t* offsets_copy, void* workspace,
-                       size_t workspace_bytes, void* state, size_t state_bytes, uint32_t epoch,
-                       gs_mailbox* mailbox, int64_t mailbox_ticket, void* stream) {
+int gs_relabel_sampled_among(const void* seed_keys, int64_t S, const void* sampled,
+                             int64_t capacity, const int64_t* sampled_len, int id_bytes,
+                             int64_t num_ids, void* table, size_t table_bytes, void* frontier,
+                             void* out_ids, int64_t* num_unique, int64_t* offsets_copy,
+                             void* workspace, size_t workspace_bytes, void* state,
+                             size_t state_bytes, uint32_t epoch, gs_mailbox* mailbox,
+                             int64_t mailbox_ticket, void* stream) {
   GS_REQUIRE(S >= 0 && capacity >= 0 && sampled_len && table && num_unique && state,
              "gs_relabel_sampled: null pointer or negative size");
   GS_REQUIRE((S == 0 || seed_keys) && (capacity == 0 || (sampled && out_ids)) &&
                  (S + capacity == 0 || frontier),
              "gs_relabel_sampled: null buffer");
-  GS_REQUIRE(valid_id_bytes(id_bytes), "gs_relabel_sampled: id_bytes must be 4 or 8, got %d",
-             id_bytes);
+  GS_REQUIRE(valid_id_bytes(id_bytes) || id_bytes == (8 | GS_NARROW_IDS),
+             "gs_relabel_sampled: id_bytes must be 4 or 8, got %d", id_bytes);
   GS_REQUIRE(epoch >= 1 && epoch <= kLbMaxEpoch, "gs_relabel_sampled: epoch must be in 1..%u",
              kLbMaxEpoch);
   if (S + capacity >= (int64_t(1) << 31)) {
@@ -1458,16 +1463,26 @@ int gs_relabel_sampled(const void* seed_keys, int64_t S, const void* sampled, in
                    static_cast<long long>(S + capacity));
     return GS_ERR_UNSUPPORTED;
   }
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  return id_bytes == 8
-             ? relabel_sampled_impl<int64_t, WideTable>(
-                   seed_keys, S, sampled, capacity, sampled_len, table, table_bytes, frontier,
-                   out_ids, num_unique, offsets_copy, workspace, workspace_bytes, state,
-                   state_bytes, epoch, mailbox, mailbox_ticket, st)
-             : relabel_sampled_impl<int32_t, PackedTable>(
-                   seed_keys, S, sampled, capacity, sampled_len, table, table_bytes, frontier,
-                   out_ids, num_unique, offsets_copy, workspace, workspace_bytes, state,
-                   state_bytes, epoch, mailbox, mailbox_ticket, st);
+  const auto impl = id_bytes == 4   ? relabel_sampled_impl<int32_t, PackedTable>
+                    : id_bytes == 8 ? relabel_sampled_impl<int64_t, WideTable>
+                                    : relabel_sampled_impl<int64_t, PackedTable>;
+  return impl(seed_keys, S, sampled, capacity, sampled_len, num_ids, table, table_bytes, frontier,
+              out_ids, num_unique, offsets_copy, workspace, workspace_bytes, state, state_bytes,
+              epoch, mailbox, mailbox_ticket, static_cast<hipStream_t>(stream));
+}
+
+int gs_relabel_sampled(const void* seed_keys, int64_t S, const void* sampled, int64_t capacity,
+                       const int64_t* sampled_len, int id_bytes, void* table, size_t table_bytes,
+                       void* frontier, void* out_ids, int64_t* num_unique,
+                       int64_t* offsets_copy, void* workspace,
+                       size_t workspace_bytes, void* state, size_t state_bytes, uint32_t epoch,
+                       gs_mailbox* mailbox, int64_t mailbox_ticket, void* stream) {
+  GS_REQUIRE(valid_id_bytes(id_bytes), "gs_relabel_sampled: id_bytes must be 4 or 8, got %d",
+             id_bytes);
+  return gs_relabel_sampled_among(seed_keys, S, sampled, capacity, sampled_len, id_bytes, 0, table,
+                                  table_bytes, frontier, out_ids, num_unique, offsets_copy,
+                                  workspace, workspace_bytes, state, state_bytes, epoch, mailbox,
+                                  mailbox_ticket, stream);
 }
 
 int gs_relabel_sampled_narrow(const void* seed_keys, int64_t S, const void* sampled,
@@ -1477,22 +1492,10 @@ int gs_relabel_sampled_narrow(const void* seed_keys, int64_t S, const void* samp
                               size_t workspace_bytes, void* state, size_t state_bytes,
                               uint32_t epoch, gs_mailbox* mailbox, int64_t mailbox_ticket,
                               void* stream) {
-  GS_REQUIRE(S >= 0 && capacity >= 0 && sampled_len && table && num_unique && state,
-             "gs_relabel_sampled_narrow: null pointer or negative size");
-  GS_REQUIRE((S == 0 || seed_keys) && (capacity == 0 || (sampled && out_ids)) &&
-                 (S + capacity == 0 || frontier),
-             "gs_relabel_sampled_narrow: null buffer");
-  GS_REQUIRE(epoch >= 1 && epoch <= kLbMaxEpoch,
-             "gs_relabel_sampled_narrow: epoch must be in 1..%u", kLbMaxEpoch);
-  if (S + capacity >= (int64_t(1) << 31)) {
-    set_error_text("gs_relabel_sampled_narrow: %lld items exceed the supported 2^31",
-                   static_cast<long long>(S + capacity));
-    return GS_ERR_UNSUPPORTED;
-  }
-  return relabel_sampled_impl<int64_t, PackedTable>(
-      seed_keys, S, sampled, capacity, sampled_len, table, table_bytes, frontier, out_ids,
-      num_unique, offsets_copy, workspace, workspace_bytes, state, state_bytes, epoch, mailbox,
-      mailbox_ticket, static_cast<hipStream_t>(stream));
+  return gs_relabel_sampled_among(seed_keys, S, sampled, capacity, sampled_len, 8 | GS_NARROW_IDS,
+                                  0, table, table_bytes, frontier, out_ids, num_unique,
+                                  offsets_copy, workspace, workspace_bytes, state, state_bytes,
+                                  epoch, mailbox, mailbox_ticket, stream);
 }
 
 }  // extern "C"

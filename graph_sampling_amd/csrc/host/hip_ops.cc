@@ -471,6 +471,7 @@ std::shared_ptr<PendingSample> ColSamplingDeferred(const torch::Tensor& indptr,
   TORCH_CHECK(fanout >= 0, "fanout must be non-negative");
   auto p = std::make_shared<PendingSample>();
   p->S = fused ? column_ids.numel() : indptr.numel() - 1;
+  p->num_ids = fused ? indptr.numel() - 1 : 0;
   const int64_t cap = p->S * fanout;
   {
     Pieces at;
@@ -685,24 +686,15 @@ std::tuple<torch::Tensor, torch::Tensor, int64_t, torch::Tensor> RelabelDeferred
   for (int attempt = 0; attempt < 2 && U == kTooWide; ++attempt) {
     const int64_t ticket = boxes.next++;
     table.clean = false;  // until both totals have come back
-    if (idb == 8 && table.narrow) {
-      Check(gs_relabel_sampled_narrow(col_ids.data_ptr(), S, p.indices.data_ptr(), cap,
-                                      p.sub_indptr.data_ptr<int64_t>() + p.S, table.buf.data_ptr(),
-                                      table.buf.numel(), frontier.data_ptr(), renamed.data_ptr(),
-                                      num.data_ptr<int64_t>(), offsets_copy.data_ptr<int64_t>(),
-                                      ws.data_ptr(), ws.numel(), state.buf.data_ptr(),
-                                      state.buf.numel(), state.epoch, boxes.slot(ticket), ticket,
-                                      p.stream),
-            "gs_relabel_sampled_narrow");
-    } else {
-      Check(gs_relabel_sampled(col_ids.data_ptr(), S, p.indices.data_ptr(), cap,
-                               p.sub_indptr.data_ptr<int64_t>() + p.S, idb, table.buf.data_ptr(),
-                               table.buf.numel(), frontier.data_ptr(), renamed.data_ptr(),
-                               num.data_ptr<int64_t>(), offsets_copy.data_ptr<int64_t>(),
-                               ws.data_ptr(), ws.numel(), state.buf.data_ptr(), state.buf.numel(),
-                               state.epoch, boxes.slot(ticket), ticket, p.stream),
-            "gs_relabel_sampled");
-    }
+    const int table_ids = idb == 8 && table.narrow ? (8 | GS_NARROW_IDS) : idb;
+    Check(gs_relabel_sampled_among(col_ids.data_ptr(), S, p.indices.data_ptr(), cap,
+                                   p.sub_indptr.data_ptr<int64_t>() + p.S, table_ids, p.num_ids,
+                                   table.buf.data_ptr(), table.buf.numel(), frontier.data_ptr(),
+                                   renamed.data_ptr(), num.data_ptr<int64_t>(),
+                                   offsets_copy.data_ptr<int64_t>(), ws.data_ptr(), ws.numel(),
+                                   state.buf.data_ptr(), state.buf.numel(), state.epoch,
+                                   boxes.slot(ticket), ticket, p.stream),
+          "gs_relabel_sampled");
     if (nnz < 0) nnz = p.Wait();
     U = WaitBox(boxes.slot(ticket), ticket, p.stream, "gs_relabel_sampled");
     if (U == kLost) U = num.item<int64_t>();

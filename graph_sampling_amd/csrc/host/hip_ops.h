@@ -78,6 +78,7 @@ struct PendingSample {
   torch::Tensor coo_col;       // capacity; undefined when not requested
   torch::Tensor data;          // capacity; the samples' edge data, undefined without any
   int64_t S = 0;
+  int64_t num_ids = 0;         // columns of the graph sampled from
   int64_t ticket = 0;
   void* stream = nullptr;
   int device = 0;

@@ -453,6 +453,17 @@ int gs_relabel_sampled_narrow(const void* seed_keys, int64_t S, const void* samp
                               uint32_t epoch, gs_mailbox* mailbox, int64_t mailbox_ticket,
                               void* stream);
 
+/* Both of the above (id_bytes: 4, 8, or 8 | GS_NARROW_IDS), told how many different ids there
+ * are (the nodes of the graph; 0: not known).  Results are the same whatever num_ids says: from
+ * half as many items on, ids that a workgroup holds several times go to the table once. */
+int gs_relabel_sampled_among(const void* seed_keys, int64_t S, const void* sampled,
+                             int64_t capacity, const int64_t* sampled_len, int id_bytes,
+                             int64_t num_ids, void* table, size_t table_bytes, void* frontier,
+                             void* out_ids, int64_t* num_unique, int64_t* offsets_copy,
+                             void* workspace, size_t workspace_bytes, void* state,
+                             size_t state_bytes, uint32_t epoch, gs_mailbox* mailbox,
+                             int64_t mailbox_ticket, void* stream);
+
 /* ------------------------------------------------------------------------- */
 /* One GraphSAGE layer -- column slice + uniform sample, then relabel -- as TWO  */
 /* launches that need no host read, so that a caller can queue all layers of a  */

@@ -287,3 +287,25 @@ def test_64_bit_ids_on_one_word_slots(dev):
     assert int(num.item()) == -2
     frontier, num, _ = capi.unique_relabel([to_dev(big, dev)], [], narrow=False)
     assert np.array_equal(frontier[:int(num.item())].cpu().numpy(), O.relabel([big], [])[0])
+
+
+@pytest.mark.parametrize("idt,narrow", [(torch.int32, False), (torch.int64, False),
+                                        (torch.int64, True)])
+@pytest.mark.parametrize("S,cap,held", [(1, 0, 0), (1, 255, 255), (100, 157, 156), (33, 70000, 69999)])
+@pytest.mark.parametrize("spread", ["one", "few", "new"])
+def test_relabel_behind_a_sampler_by_repeats(dev, idt, narrow, S, cap, held, spread):
+    """Ids that repeat inside a workgroup meet in LDS when there are at least half as many items
+    as ids; on both sides of that line the frontier and the ranks are the oracle's, the table
+    is empty again and the next call finds it so.  (held: the true length, on the device)"""
+    rng = np.random.default_rng(cap + len(spread))
+    hi = {"one": 1, "few": 40, "new": 1 << 20}[spread]
+    seeds, rows = rng.permutation(1 << 20)[:S], rng.integers(0, hi, cap)
+    sub_indptr = np.full(S + 1, held, dtype=np.int64)
+    table = capi.RelabelTable(S + cap, idt, dev, narrow=narrow)
+    want, w_out = O.relabel([seeds, rows[:held]], [rows[:held]])
+    for num_ids in (2 * (S + cap), 2 * (S + cap) + 1, 0):
+        frontier, num, out = capi.relabel_sampled(to_dev(seeds, dev, idt), to_dev(sub_indptr, dev),
+                                                  to_dev(rows, dev, idt), table, num_ids=num_ids)
+        assert int(num) == want.size
+        assert np.array_equal(frontier[:want.size].cpu().numpy().astype(np.int64), want)
+        assert np.array_equal(out[:held].cpu().numpy().astype(np.int64), w_out[0])
