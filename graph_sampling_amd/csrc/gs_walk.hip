@@ -8,9 +8,12 @@
 // also the coalesced layout for one lane per walker: at every step the 64 lanes
 // of a wave store 64 consecutive ids.  The walker keeps its current node in a
 // register (the reference re-reads it from the trace, random_walk.cu:32).  A
-// step is two dependent random reads (the indptr pair, then one neighbour), so
-// the kernel is bound by HBM/TLB latency and lives on occupancy: 256 threads
-// per workgroup, no LDS, ~24 VGPRs.  One Philox block feeds four steps.
+// step is two dependent random reads (the indptr pair, then one neighbour).  With
+// enough walkers the kernel is bound by lines fetched behind the L2s: random reads
+// that miss run at about 55 G/s on this machine, in the memory-side cache or not (hits
+// at 260 G/s), and a million walkers on a graph of 4 M nodes and 200 M edges miss
+// 69 M times in 47 M steps.  With few it is latency: 256 threads per workgroup, no
+// LDS, ~24 VGPRs, as many waves as there are.  One Philox block feeds four steps.
 #include "gs_common.hpp"
 
 namespace gs {
@@ -18,17 +21,35 @@ namespace {
 
 constexpr int kThreads = 256;
 
+// Neighbour arrays from this size on are read as streams (the line is the first to leave the
+// L2): hardly one of their lines is met again, and the offsets, which are, stay longer.
+// Arrays that the L2s and the memory-side cache hold in good part lose by it.  1 M walkers,
+// 80 steps, 800 MB: 1456 -> 1426 us; metapath over three of 400 MB: 126 -> 120; but 20 k
+// walkers over 32 MB: 41 -> 68.
+constexpr int64_t kStreamBytes = int64_t(256) << 20;
+
 // A node outside [0, num_nodes) has no neighbours (the walker dies there), so a
 // stray seed can never turn into a wild read.
 template <typename IdT>
 __device__ __forceinline__ int64_t step_from(const int64_t* __restrict__ indptr,
                                              const IdT* __restrict__ indices, int64_t num_nodes,
-                                             int64_t curr, uint32_t x) {
+                                             int64_t curr, uint32_t x, bool stream) {
   if (static_cast<uint64_t>(curr) >= static_cast<uint64_t>(num_nodes)) return -1;
   const int64_t start = indptr[curr];
   const int64_t deg = indptr[curr + 1] - start;
   if (deg <= 0) return -1;
-  return static_cast<int64_t>(indices[start + static_cast<int64_t>(x % static_cast<uint32_t>(deg))]);
+  const IdT* at = indices + start + static_cast<int64_t>(x % static_cast<uint32_t>(deg));
+  IdT next;
+  if (stream) {
+    // (held apart from the other by two empty statements, or the compiler makes one plain load
+    // of the two)
+    asm volatile("" : "+v"(at));
+    next = __builtin_nontemporal_load(at);
+    asm volatile("" : "+v"(next));
+  } else {
+    next = *at;
+  }
+  return static_cast<int64_t>(next);
 }
 
 template <typename IdT>
@@ -40,6 +61,7 @@ random_walk_kernel(const int64_t* __restrict__ indptr, const IdT* __restrict__ i
   if (w >= n) return;
   int64_t curr = static_cast<int64_t>(seeds[w]);
   trace[w] = static_cast<IdT>(curr);
+  const bool stream = indptr[num_nodes] >= kStreamBytes / static_cast<int64_t>(sizeof(IdT));
   U4 x;
   for (int64_t t = 0; t < length; ++t) {
     if (!replay && (t & 3) == 0)
@@ -47,7 +69,7 @@ random_walk_kernel(const int64_t* __restrict__ indptr, const IdT* __restrict__ i
     int64_t pick = -1;
     if (curr >= 0) {
       const uint32_t xv = replay ? replay[t * n + w] : x.v[t & 3];
-      pick = step_from(indptr, indices, num_nodes, curr, xv);
+      pick = step_from(indptr, indices, num_nodes, curr, xv, stream);
     }
     trace[(t + 1) * n + w] = static_cast<IdT>(pick);
     curr = pick;
@@ -67,14 +89,22 @@ metapath_walk_kernel(const int64_t* const* __restrict__ all_indptr,
   int64_t curr = static_cast<int64_t>(seeds[w]);
   trace[w] = static_cast<IdT>(curr);
   U4 x;
+  unsigned long long streams = 0ull;  // bit t: the relation of step t (mod 64) is read as a stream
   for (int64_t t = 0; t < length; ++t) {
+    if ((t & (kWave - 1)) == 0) {  // a lane per step of the next 64
+      const int64_t step = t + (threadIdx.x & (kWave - 1));
+      const int64_t rel = metapath[step < length ? step : length - 1];
+      streams = __ballot(all_indptr[rel][all_num_nodes[rel]] >=
+                         kStreamBytes / static_cast<int64_t>(sizeof(IdT)));
+    }
     if (!replay && (t & 3) == 0)
       x = draw_block(seed, kTagWalk, static_cast<uint64_t>(w), static_cast<uint64_t>(t >> 2));
     int64_t pick = -1;
     if (curr >= 0) {
       const int64_t rel = metapath[t];  // uniform over the wave: scalar loads
       const uint32_t xv = replay ? replay[t * n + w] : x.v[t & 3];
-      pick = step_from(all_indptr[rel], all_indices[rel], all_num_nodes[rel], curr, xv);
+      pick = step_from(all_indptr[rel], all_indices[rel], all_num_nodes[rel], curr, xv,
+                       (streams >> (t & (kWave - 1))) & 1ull);
     }
     trace[(t + 1) * n + w] = static_cast<IdT>(pick);
     curr = pick;

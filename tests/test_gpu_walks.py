@@ -122,3 +122,28 @@ def test_walk_out_of_range_seeds_die(dev):
     assert np.array_equal(got.cpu().numpy(), want)
     tr = want.reshape(5, 6)
     assert (tr[1:, [1, 2, 4, 5]] == -1).all()
+
+
+@pytest.mark.parametrize("idt", [torch.int32, torch.int64])
+@pytest.mark.parametrize("less", [0, 1])
+def test_walks_over_neighbour_arrays_read_as_streams(dev, idt, less):
+    """Neighbour arrays of 256 MB and of one edge less (read as streams and not), alone and as one
+    relation beside a small one, over more than 64 steps; each node has 64 neighbours, the
+    last fewer."""
+    E = (1 << 28) // (4 if idt == torch.int32 else 8) - less
+    N = (E + 63) // 64
+    rng = np.random.default_rng(less)
+    indptr = np.minimum(np.arange(N + 1, dtype=np.int64) * 64, E)
+    indices = rng.integers(0, N, E).astype(np.int32 if idt == torch.int32 else np.int64)
+    small_ptr = np.arange(N + 1, dtype=np.int64)
+    small_ix = rng.permutation(N)
+    seeds = rng.integers(0, N, 300)
+    big = indices.astype(np.int64)
+    keep = _tables([indptr, small_ptr], [indices, small_ix], dev, idt)
+    got = capi.random_walk(keep[0][0], keep[1][0], to_dev(seeds, dev, idt), 9, seed=5)
+    assert np.array_equal(got.cpu().numpy().astype(np.int64), O.random_walk(indptr, big, seeds, 9, seed=5))
+    path = np.array([0, 0, 1] * 22 + [0], dtype=np.int64)
+    got = capi.metapath_walk(keep[2], keep[3], keep[4], idt, to_dev(path, dev), to_dev(seeds, dev, idt),
+                             seed=6)
+    want = O.metapath_walk([indptr, small_ptr], [big, small_ix], path, seeds, seed=6)
+    assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
