@@ -919,16 +919,16 @@ def _sb_sample(b, S, E, U):
 
 # launch sites of the super-batch flow and the least bytes of each one's third-layer launch
 # (M = S + E items; the binned relabel: count reads the ids, scatter reads them and writes an
-# 8-byte record each, flag reads and rewrites the records and marks first occurrences, rank
-# reads a byte and writes 16 bytes per 64 items, rename reads the records and a 16-byte entry
-# each and writes the renamed ids and the frontier)
+# 8-byte record each, first reads the records and writes a 4-byte position each, rank reads
+# those and writes 16 bytes per 64 items, rename reads the positions, a 16-byte entry each and
+# the ids of the frontier and writes the renamed ids and the frontier)
 SUPER_SITES = {
     "sample_fused": _sb_sample,
     "bins_count": lambda b, S, E, U: (S + E) * b,
     "bins_scatter": lambda b, S, E, U: (S + E) * (b + 8),
-    "bins_flag": lambda b, S, E, U: (S + E) * 16 + U,
-    "bins_rank": lambda b, S, E, U: (S + E) * (1 + 0.25),
-    "bins_rename": lambda b, S, E, U: (S + E) * (8 + 16) + E * b + U * b,
+    "bins_first": lambda b, S, E, U: (S + E) * 12,
+    "bins_rank": lambda b, S, E, U: (S + E) * (4 + 0.25),
+    "bins_rename": lambda b, S, E, U: (S + E) * (4 + 16) + E * b + U * 2 * b,
     "batch_init": lambda b, S, E, U: 4 * (S + E) * 8,            # 8-byte slots, 4 per item
     "batch_insert": lambda b, S, E, U: (S + E) * (b + 16 + 4 + 8),  # id, slot RMW, slot index, offsets
     "batch_compact": lambda b, S, E, U: (S + E) * 20 + U * b,

@@ -11,25 +11,30 @@
 // about 26 G/s on this machine whatever else happens.  Here the only atomics on memory are one
 // counter addition per (4096-item tile, class):
 //
-//   plan      every batch is cut into P_b = 2^k classes of about 1-2 k items by the top bits
-//             of its ids' hash; a class of a batch is a "bucket", numbered batch by batch
+//   plan      every batch is cut into P_b classes of about 2 k items by its ids' hash times
+//             P_b; a class of a batch is a "bucket", numbered batch by batch
 //   count     a workgroup counts its tile's items per bucket in LDS, adds the counts to memory
 //   scan      bucket offsets
 //   scatter   the same tile walk; every item's record (id << 32 | position) goes to its bucket.
 //             The order inside a bucket is whatever the atomics make it: nothing below depends
 //             on it, first occurrences are decided by the positions the records carry
-//   flag      one workgroup per bucket: LDS table id -> smallest position; that position is
-//             the id's first occurrence in the batch, and gets a byte in a flag array; every
-//             record is rewritten to carry the first position of its id instead of the id
-//   rank      chained scan over the flag bytes: per 64 positions a mask and the number of
-//             first occurrences before them
-//   rename    a plain pass over the records: the rank of a record's first position from mask
-//             + count, the frontier written by rank, the ids renamed in place
+//   first     one workgroup per bucket: LDS table id -> smallest position; that position is
+//             the id's first occurrence in the batch, and is stored at the record's position
+//   rank      chained scan over the positions that are their own first: per 64 positions a
+//             mask and the number of first occurrences before them
+//   rename    a pass in the order of the positions: the rank of an item's first position from
+//             mask + count; first occurrences write the frontier, ids their new name
+//
+// A record is read once and never written again; of the three places an item touches at
+// random (its first position's store, the rank it looks up, and before these passes were in
+// the order of the positions its new name and its place in the frontier) two are left, and a
+// first occurrence looks up nothing.  17 M items in 64 batches: first 111 -> 112 us (with
+// half as many, twice as large buckets: 132 before that), rank 15 -> 25, rename 143 -> 88.
 //
 // Buckets are handed to workgroups so that consecutive buckets -- one batch's -- run on the
 // same XCD one after the other (workgroup w runs on XCD w % 8): the positions a batch's
-// buckets store to (flags, renamed ids, frontier) are a megabyte or two that stays in that
-// XCD's L2 until its lines are full.
+// buckets store to are a megabyte or two that stays in that XCD's L2 until its lines are
+// full.
 //
 // The ids may come from a sampler that is still running when the relabel is queued, and whose
 // total is then read from the offsets on the device.  A sampler that failed leaves a negative
@@ -50,17 +55,27 @@ constexpr int kBucketItemsLog2 = 11;   // classes are sized for <= 2048 items on
 constexpr int kMaxClassesLog2 = 12;    // at most 4096 classes per batch
 constexpr int kPartItems = 16;         // items of a thread in the count / scatter passes
 constexpr int kPartTile = kThreads * kPartItems;
-// LDS counters of a tile: the buckets of the batches it touches (two batches of 4096 classes
-// at the most, and those wholly inside it, which have a class per 1024 items and two on top)
-constexpr int kCounterCap = 2 * (1 << kMaxClassesLog2) + (kPartTile >> (kBucketItemsLog2 - 1)) +
-                            2 * static_cast<int>(kStagedBatches) + 2;
+// LDS counters of a tile: the buckets of the batches it touches (two batches with all the
+// classes there may be, and those wholly inside it: a class per 2048 items and one on top)
+constexpr int counter_cap(int classes_log2) {
+  return 2 * (1 << classes_log2) + (kPartTile >> (kBucketItemsLog2 - 1)) +
+         2 * static_cast<int>(kStagedBatches) + 2;
+}
+constexpr int kCounterCap = counter_cap(kMaxClassesLog2);
+// Batches of up to 2^20 items on average have up to 512 classes, and counters for two of twice
+// that take 12 KB of LDS instead of 36: twice the workgroups on a compute unit (17 M items in
+// 64 batches: count 53 -> 47 us, scatter 104 -> 100; 43 and 93 with buckets of 2048 items
+// instead of the 1037 that a power of two of classes gave).  A batch that is larger all the
+// same counts what lies beyond them in memory.
+constexpr int kFewCounters = counter_cap(10);
+constexpr int64_t kFewCountersItems = int64_t(1) << 20;
 constexpr int kSlots = 4096;           // LDS table of a bucket (8-byte slots)
-constexpr int kFlagTile = kThreads * 64;  // positions of a workgroup in the rank pass
-constexpr int kTrip = 8;  // records of a thread that are asked for together (a whole average bucket)
+constexpr int kRankTile = kThreads * 64;  // positions of a workgroup in the rank pass
+constexpr int kTrip = 10;  // records of a thread that are asked for together (a whole bucket nearly always)
 
 struct Plan {
   uint32_t* bucket_base;  // [B + 1]: first bucket of every batch; [B] = number of buckets
-  uint32_t* classes_log2; // [B]
+  uint32_t* classes;      // [B]
 };
 
 struct Bins {
@@ -70,13 +85,13 @@ struct Bins {
   int64_t* bucket_ptr;    // [buckets bound + 1]: first record of every bucket
   uint32_t* bucket_batch; // [buckets bound]: the batch of every bucket that holds records
   unsigned long long* records;  // [M]: id << 32 | position
-  unsigned char* flags;   // [tiles * kFlagTile]: 1 at first occurrences
-  uint4* ranks;           // per 64 positions: {flags as bits (x, y), first occurrences before them (z), 0}
+  uint32_t* first;        // [M]: position of the first occurrence of the item's id in its batch
+  uint4* ranks;           // per 64 positions: {first occurrences as bits (x, y), how many before them (z), 0}
   unsigned int* error;    // the look-back state's error word: 2 = id too wide, 3 = a table filled up
 };
 
-inline int64_t buckets_bound(int64_t M, int64_t B) { return (M >> (kBucketItemsLog2 - 1)) + 2 * B + 8; }
-inline int64_t flag_tiles(int64_t M) { return M / kFlagTile + 1; }
+inline int64_t buckets_bound(int64_t M, int64_t B) { return (M >> kBucketItemsLog2) + B + 8; }
+inline int64_t rank_tiles(int64_t M) { return M / kRankTile + 1; }
 
 // slot of an id in a bucket's table: other hash bits than the ones that chose the bucket
 __device__ __forceinline__ uint32_t slot_of(uint32_t key) {
@@ -85,9 +100,8 @@ __device__ __forceinline__ uint32_t slot_of(uint32_t key) {
 static_assert(kSlots == 1 << 12, "slot_of yields 12 bits");
 
 __global__ void __launch_bounds__(kThreads)
-bins_init_kernel(Bins s, int64_t flag_words16, int64_t buckets, LookbackState lb, int64_t tiles) {
+bins_init_kernel(Bins s, int64_t buckets, LookbackState lb, int64_t tiles) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  if (i < flag_words16) reinterpret_cast<uint4*>(s.flags)[i] = make_uint4(0u, 0u, 0u, 0u);
   if (i < buckets) {
     s.count[i] = 0u;
     s.fill[i] = 0u;
@@ -102,13 +116,12 @@ __global__ void __launch_bounds__(512) bins_plan_kernel(BatchItems<IdT> x, Plan 
   __shared__ int64_t s_scan[512 / kWave + 1];
   const int64_t b = threadIdx.x;
   int64_t classes = 0;
-  uint32_t lg = 0;
   if (b < x.B) {
     const int64_t m = x.ids_ptr[x.B] < 0 ? 0 : x.start(b + 1) - x.start(b);
-    const int64_t want = (m + (int64_t(1) << kBucketItemsLog2) - 1) >> kBucketItemsLog2;
-    while ((int64_t(1) << lg) < want && lg < kMaxClassesLog2) ++lg;
-    classes = int64_t(1) << lg;
-    p.classes_log2[b] = lg;
+    classes = (m + (int64_t(1) << kBucketItemsLog2) - 1) >> kBucketItemsLog2;
+    if (classes < 1) classes = 1;
+    if (classes > (int64_t(1) << kMaxClassesLog2)) classes = int64_t(1) << kMaxClassesLog2;
+    p.classes[b] = static_cast<uint32_t>(classes);
   }
   int64_t total;
   const int64_t before = block_exclusive_scan<512>(classes, &total, s_scan);
@@ -117,7 +130,7 @@ __global__ void __launch_bounds__(512) bins_plan_kernel(BatchItems<IdT> x, Plan 
 }
 
 // What the count and the scatter pass share: the tile's items, their batches and buckets.
-template <typename IdT>
+template <typename IdT, int CAP>
 struct TileWalk {
   int64_t lo, hi;          // batches of the tile's first and last item
   uint32_t first_bucket;   // bucket_base[lo]
@@ -126,7 +139,7 @@ struct TileWalk {
   // true one.  False: the tile lies beyond the items (the whole workgroup leaves).
   __device__ __forceinline__ bool open(BatchItems<IdT>& x, const Plan& p, int64_t& M,
                                        int64_t* s_seeds_ptr, int64_t* s_ids_ptr,
-                                       uint32_t* s_base, uint32_t* s_lg, int64_t* s_range,
+                                       uint32_t* s_base, uint32_t* s_classes, int64_t* s_range,
                                        uint32_t* s_cnt) {
     x.stage_offsets(s_seeds_ptr, s_ids_ptr);
     const int64_t held = x.seeds_ptr[x.B] + x.ids_ptr[x.B];
@@ -135,14 +148,14 @@ struct TileWalk {
     if (static_cast<int64_t>(blockIdx.x) * kPartTile >= M) return false;
     for (int64_t b = threadIdx.x; b <= x.B; b += kThreads) {
       s_base[b] = p.bucket_base[b];
-      s_lg[b] = b < x.B ? p.classes_log2[b] : 0u;
+      s_classes[b] = b < x.B ? p.classes[b] : 1u;
     }
     const int64_t first = static_cast<int64_t>(blockIdx.x) * kPartTile;
     const int64_t last = first + kPartTile - 1 < M ? first + kPartTile - 1 : M - 1;
     x.block_range(first, last, s_range, &lo, &hi);  // (ends with a barrier: s_base is there)
     first_bucket = s_base[lo];
     const uint32_t all = s_base[hi + 1] - first_bucket;
-    span = all < static_cast<uint32_t>(kCounterCap) ? all : static_cast<uint32_t>(kCounterCap);
+    span = all < static_cast<uint32_t>(CAP) ? all : static_cast<uint32_t>(CAP);
     for (uint32_t c = threadIdx.x; c < span; c += kThreads) s_cnt[c] = 0u;
     __syncthreads();
     return true;
@@ -150,13 +163,14 @@ struct TileWalk {
 };
 
 // LDS of the two partition passes
+template <int CAP>
 struct PartShared {
   int64_t seeds_ptr[kStagedBatches + 1];
   int64_t ids_ptr[kStagedBatches + 1];
   uint32_t base[kStagedBatches + 1];
-  uint32_t lg[kStagedBatches + 1];
+  uint32_t classes[kStagedBatches + 1];
   int64_t range[2];
-  uint32_t cnt[kCounterCap];
+  uint32_t cnt[CAP];
 };
 
 // count (SCATTER false): items per bucket.  scatter: the same walk, then the tile's share of
@@ -164,12 +178,12 @@ struct PartShared {
 // of several rounds of 4096 items -- fewer additions to memory, longer runs of records side
 // by side -- were slower: 64 / 143 us against 55 / 105 us over 17 M items; workgroups that
 // stay and loop are the slower shape on this machine.)
-template <typename IdT, bool SCATTER>
+template <typename IdT, bool SCATTER, int CAP>
 __global__ void __launch_bounds__(kThreads)
 bins_partition_kernel(BatchItems<IdT> x, int64_t M, Bins s) {
-  __shared__ PartShared sh;
-  TileWalk<IdT> w;
-  if (!w.open(x, s.plan, M, sh.seeds_ptr, sh.ids_ptr, sh.base, sh.lg, sh.range, sh.cnt)) return;
+  __shared__ PartShared<CAP> sh;
+  TileWalk<IdT, CAP> w;
+  if (!w.open(x, s.plan, M, sh.seeds_ptr, sh.ids_ptr, sh.base, sh.classes, sh.range, sh.cnt)) return;
   const int64_t tile_first = static_cast<int64_t>(blockIdx.x) * kPartTile;
   // where every item is: all reads of the thread's items stand together, none behind a
   // condition of its own (the last item again past the end)
@@ -191,8 +205,7 @@ bins_partition_kernel(BatchItems<IdT> x, int64_t M, Bins s) {
 #pragma unroll
   for (int k = 0; k < kPartItems; ++k) {
     const int64_t i = tile_first + k * kThreads + threadIdx.x;
-    const uint32_t lg = sh.lg[batch[k]];
-    const uint32_t cls = lg ? hash32(static_cast<uint32_t>(key[k])) >> (32 - lg) : 0u;
+    const uint32_t cls = __umulhi(hash32(static_cast<uint32_t>(key[k])), sh.classes[batch[k]]);
     bucket[k] = sh.base[batch[k]] + cls;
     rank[k] = 0u;
     if (i < M) {
@@ -255,11 +268,12 @@ __device__ __forceinline__ int64_t bucket_of_workgroup(int64_t num_buckets) {
 
 // Enters the bucket's records into the LDS table: slot = id << 32 | smallest position.
 // Raises the error word when the table is full.  The first trip's records are asked for
-// before the table is cleared, so that the clearing hides under the trip.
+// before the table is cleared, so that the clearing hides under the trip; `rec` holds the
+// last trip's when the table is complete.
 __device__ __forceinline__ void table_fill(unsigned long long* __restrict__ tab,
                                            const unsigned long long* __restrict__ records,
-                                           int64_t begin, int64_t end, unsigned int* error) {
-  unsigned long long rec[kTrip];
+                                           int64_t begin, int64_t end, unsigned int* error,
+                                           unsigned long long (&rec)[kTrip]) {
 #pragma unroll
   for (int u = 0; u < kTrip; ++u) {
     const int64_t r = begin + u * kThreads + threadIdx.x;
@@ -300,57 +314,46 @@ __device__ __forceinline__ void table_fill(unsigned long long* __restrict__ tab,
   __syncthreads();
 }
 
-// One workgroup per bucket.  After the table is complete every record is rewritten in place
-// for the last pass, which then needs no table: a first occurrence keeps its id and gets the
-// top bit of its position set (and its byte in the flag array); any other record trades its
-// id for the position of the id's first occurrence.
-constexpr unsigned long long kFirstBit = 0x80000000ull;
-
-__global__ void __launch_bounds__(kThreads) bins_flag_kernel(Bins s, int64_t B) {
+// One workgroup per bucket: every record's position gets the smallest position of its id.
+// (A bucket of one trip, as most are, still holds its records in registers by then.)
+__global__ void __launch_bounds__(kThreads) bins_first_kernel(Bins s, int64_t B) {
   __shared__ unsigned long long tab[kSlots];
   const int64_t k = bucket_of_workgroup(s.plan.bucket_base[B]);
   if (k < 0) return;
   const int64_t begin = s.bucket_ptr[k], end = s.bucket_ptr[k + 1];
   if (begin == end) return;
-  table_fill(tab, s.records, begin, end, s.error);
-  for (int64_t r0 = begin; r0 < end; r0 += kTrip * kThreads) {
-    unsigned long long rec[kTrip];
+  unsigned long long rec[kTrip];
+  table_fill(tab, s.records, begin, end, s.error, rec);
+  const int64_t trips = (end - begin + kTrip * kThreads - 1) / (kTrip * kThreads);
+  for (int64_t t = trips - 1; t >= 0; --t) {  // (from the last trip backwards)
+    const int64_t r0 = begin + t * (kTrip * kThreads);
 #pragma unroll
     for (int u = 0; u < kTrip; ++u) {
-      const int64_t r = r0 + u * kThreads + threadIdx.x;
-      rec[u] = s.records[r < end ? r : end - 1];
-    }
-    unsigned long long out[kTrip];
-#pragma unroll
-    for (int u = 0; u < kTrip; ++u) {
-      out[u] = 0ull;
-      // (a lane past the end holds a copy of the last record, which its owner may already have
-      // rewritten: it must not look that up)
       if (r0 + u * kThreads + threadIdx.x < end) {
         const uint32_t key = static_cast<uint32_t>(rec[u] >> 32);
         uint32_t p = slot_of(key);
         int probes = 0;
         unsigned long long w = tab[p];
+        // (a table that was too small may lack the id: what is stored then is read by nobody)
         while (static_cast<uint32_t>(w >> 32) != key && ++probes < kSlots) {
           p = (p + 1) & (kSlots - 1);
           w = tab[p];
         }
-        out[u] = w == rec[u] ? rec[u] | kFirstBit
-                             : (w << 32) | static_cast<unsigned long long>(static_cast<uint32_t>(rec[u]));
+        s.first[static_cast<uint32_t>(rec[u])] = static_cast<uint32_t>(w);
       }
     }
+    if (t > 0) {
 #pragma unroll
-    for (int u = 0; u < kTrip; ++u) {
-      const int64_t r = r0 + u * kThreads + threadIdx.x;
-      if (r < end) {
-        s.records[r] = out[u];
-        if (out[u] & kFirstBit) s.flags[static_cast<uint32_t>(rec[u])] = 1;
-      }
+      for (int u = 0; u < kTrip; ++u) rec[u] = s.records[r0 - (kTrip - u) * kThreads + threadIdx.x];
     }
   }
 }
 
-// 64 flag bytes of a thread -> one mask word; scan of the counts over all tiles
+// Positions that are their own first, 64 to a mask word; scan of the counts over all tiles.
+// A wave takes 64 times 64 consecutive positions, one read and one ballot each, and lane l
+// keeps the mask of the l-th.
+constexpr int kRankTrip = 16;
+
 __global__ void __launch_bounds__(kThreads)
 bins_rank_kernel(Bins s, int64_t M, int64_t B, const int64_t* __restrict__ seeds_ptr,
                  const int64_t* __restrict__ ids_ptr, int64_t* __restrict__ num_unique,
@@ -361,20 +364,28 @@ bins_rank_kernel(Bins s, int64_t M, int64_t B, const int64_t* __restrict__ seeds
   __shared__ unsigned long long s_mask[kThreads];
   __shared__ uint32_t s_before[kThreads];
   const unsigned int tile = blockIdx.x;
-  const int64_t word = static_cast<int64_t>(tile) * kThreads + threadIdx.x;
-  const uint4* __restrict__ f = reinterpret_cast<const uint4*>(s.flags) + word * 4;
-  uint4 q[4];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) q[u] = f[u];
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int64_t tile_first = static_cast<int64_t>(tile) * kRankTile;
+  {  // (M may be a bound: the offsets hold the true count; nothing was stored beyond it)
+    const int64_t held = ids_ptr[B] < 0 ? 0 : seeds_ptr[B] + ids_ptr[B];
+    if (held < M) M = held;
+  }
   unsigned long long m = 0ull;
+  const int64_t wave_first = tile_first + wave * (kWave * kWave);
+  if (wave_first < M) {  // (the same for a whole wave)
+    for (int w0 = 0; w0 < kWave; w0 += kRankTrip) {
+      uint32_t f[kRankTrip];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const uint32_t x[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
+      for (int u = 0; u < kRankTrip; ++u) {
+        const int64_t p = wave_first + (w0 + u) * kWave + lane;
+        f[u] = s.first[p < M ? p : M - 1];
+      }
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      // four flag bytes (0 or 1 each) -> four bits, byte j at bit j
-      const unsigned long long nib = ((x[v] & 0x01010101u) * 0x01020408u) >> 24 & 0xFu;
-      m |= nib << (16 * u + 4 * v);
+      for (int u = 0; u < kRankTrip; ++u) {
+        const int64_t p = wave_first + (w0 + u) * kWave + lane;
+        const unsigned long long own = __ballot(p < M && f[u] == static_cast<uint32_t>(p));
+        if (lane == w0 + u) m = own;
+      }
     }
   }
   const int64_t mine = __popcll(m);
@@ -387,15 +398,15 @@ bins_rank_kernel(Bins s, int64_t M, int64_t B, const int64_t* __restrict__ seeds
   }
   __syncthreads();
   const uint32_t before = static_cast<uint32_t>(s_prefix + local);
-  s.ranks[word] = make_uint4(static_cast<uint32_t>(m), static_cast<uint32_t>(m >> 32), before, 0u);
+  s.ranks[static_cast<int64_t>(tile) * kThreads + threadIdx.x] =
+      make_uint4(static_cast<uint32_t>(m), static_cast<uint32_t>(m >> 32), before, 0u);
   // frontier offsets: the rank at every batch's first position, by the thread that owns it
   s_mask[threadIdx.x] = m;
   s_before[threadIdx.x] = before;
   __syncthreads();
-  const int64_t tile_first = static_cast<int64_t>(tile) * kFlagTile;
   for (int64_t b = threadIdx.x; b < B; b += kThreads) {
     const int64_t p = seeds_ptr[b] + ids_ptr[b] - tile_first;
-    if (p >= 0 && p < kFlagTile)
+    if (p >= 0 && p < kRankTile)
       unique_ptr[b] = s_before[p >> 6] + __popcll(s_mask[p >> 6] & ((1ull << (p & 63)) - 1ull));
   }
   if (tile == gridDim.x - 1 && threadIdx.x == 0) {
@@ -409,11 +420,11 @@ bins_rank_kernel(Bins s, int64_t M, int64_t B, const int64_t* __restrict__ seeds
   }
 }
 
-// The last pass, over the records as they lie (bucket by bucket, which is batch by batch): a
-// record knows the position of its id's first occurrence, whose rank is the count before its
-// 64 positions plus the bits below it; first occurrences write the frontier, records of ids
-// (not seeds) the renamed id.  Chunks of records go to workgroups like the buckets did, one
-// batch after the other on one XCD.
+// The last pass, in the order of the positions: the rank of an item's first position is the
+// count before its 64 positions plus the bits below it.  First occurrences write the frontier
+// (neighbours side by side), ids -- not seeds -- their rank in their batch.  Tiles of
+// consecutive positions go to one XCD one after the other: the ranks a batch looks up are a
+// few dozen kilobytes.
 constexpr int kRenameItems = 8;
 constexpr int kRenameTile = kThreads * kRenameItems;
 
@@ -428,6 +439,8 @@ __global__ void __launch_bounds__(kThreads)
 bins_rename_kernel(BatchItems<IdT> x, int64_t M, Bins s, IdT* __restrict__ unique,
                    IdT* __restrict__ out_ids, const int64_t* __restrict__ unique_ptr) {
   __shared__ RenameShared sh;
+  // a table was too small: a stored position may be none
+  if (__hip_atomic_load(s.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
   {  // (M may be a bound: the offsets hold the true count)
     const int64_t held = x.seeds_ptr[x.B] + x.ids_ptr[x.B];
     if (held < M) M = held;
@@ -437,40 +450,32 @@ bins_rename_kernel(BatchItems<IdT> x, int64_t M, Bins s, IdT* __restrict__ uniqu
   const int64_t per = (chunks + kXcds - 1) / kXcds;
   const int64_t chunk = static_cast<int64_t>(blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
   if (blockIdx.x / kXcds >= per || chunk >= chunks) return;
-  const int64_t first = chunk * kRenameTile;
-  unsigned long long rec[kRenameItems];
+  const int64_t tile_first = chunk * kRenameTile;
+  const int64_t last = tile_first + kRenameTile - 1 < M ? tile_first + kRenameTile - 1 : M - 1;
+  uint32_t at[kRenameItems];
 #pragma unroll
   for (int u = 0; u < kRenameItems; ++u) {
-    const int64_t r = first + u * kThreads + threadIdx.x;
-    rec[u] = s.records[r < M ? r : M - 1];
+    const int64_t i = tile_first + u * kThreads + threadIdx.x;
+    at[u] = s.first[i < M ? i : M - 1];
   }
   x.stage_offsets(sh.seeds_ptr, sh.ids_ptr);
   // the entries of the first occurrences' positions: one 16-byte read each, all in flight
   uint4 e[kRenameItems];
-  uint32_t pos[kRenameItems], at[kRenameItems];
+#pragma unroll
+  for (int u = 0; u < kRenameItems; ++u) e[u] = s.ranks[at[u] >> 6];
+  int64_t lo, hi;
+  x.block_range(tile_first, last, sh.range, &lo, &hi);
+  // (reading the ids and the batches' ranks of all eight up front was slower: 94 against 88 us)
 #pragma unroll
   for (int u = 0; u < kRenameItems; ++u) {
-    pos[u] = static_cast<uint32_t>(rec[u]) & ~static_cast<uint32_t>(kFirstBit);
-    at[u] = (rec[u] & kFirstBit) ? pos[u] : static_cast<uint32_t>(rec[u] >> 32);
-    e[u] = s.ranks[at[u] >> 6];
-  }
-  // records of a chunk belong to the batches of its first and last record and those between
-  if (threadIdx.x < 2) {
-    const int64_t r = threadIdx.x == 0 ? first : (first + kRenameTile - 1 < M ? first + kRenameTile - 1 : M - 1);
-    const uint32_t p = static_cast<uint32_t>(s.records[r]) & ~static_cast<uint32_t>(kFirstBit);
-    sh.range[threadIdx.x] = x.batch_of(p, 0, x.B - 1);
-  }
-  __syncthreads();
-  const int64_t lo = sh.range[0], hi = sh.range[1];
-#pragma unroll
-  for (int u = 0; u < kRenameItems; ++u) {
-    if (first + u * kThreads + threadIdx.x < M) {
+    const int64_t i = tile_first + u * kThreads + threadIdx.x;
+    if (i < M) {
       const unsigned long long m = static_cast<unsigned long long>(e[u].y) << 32 | e[u].x;
       const uint32_t rank = e[u].z + __popcll(m & ((1ull << (at[u] & 63u)) - 1ull));
-      if (rec[u] & kFirstBit) unique[rank] = static_cast<IdT>(static_cast<uint32_t>(rec[u] >> 32));
-      const int64_t b = x.batch_of(pos[u], lo, hi);
-      const int64_t off = static_cast<int64_t>(pos[u]) - x.start(b);
+      const int64_t b = x.batch_of(i, lo, hi);
+      const int64_t off = i - x.start(b);
       const int64_t n_seeds = x.seeds_ptr[b + 1] - x.seeds_ptr[b];
+      if (at[u] == static_cast<uint32_t>(i)) unique[rank] = *x.where_in(b, i);
       if (off >= n_seeds)
         out_ids[x.ids_ptr[b] + off - n_seeds] =
             static_cast<IdT>(rank - static_cast<uint32_t>(unique_ptr[b]));
@@ -486,18 +491,18 @@ int binned_impl(const void* seeds, const int64_t* seeds_ptr, const void* ids,
                 hipStream_t stream) {
   const int64_t M = num_seeds + num_ids;
   const int64_t nb = buckets_bound(M, B);
-  const int64_t tiles = flag_tiles(M);
+  const int64_t tiles = rank_tiles(M);
   Carver ws(workspace, workspace_bytes);
   Bins s;
   s.plan.bucket_base = ws.take<uint32_t>(B + 1);
-  s.plan.classes_log2 = ws.take<uint32_t>(B);
+  s.plan.classes = ws.take<uint32_t>(B);
   s.count = ws.take<uint32_t>(nb);
   s.fill = ws.take<uint32_t>(nb);
   s.bucket_ptr = ws.take<int64_t>(nb + 1);
   s.bucket_batch = ws.take<uint32_t>(nb);
   int64_t* scan_ws = ws.take<int64_t>(scan_num_tiles(nb) + 1);
   s.records = ws.take<unsigned long long>(M);
-  s.flags = ws.take<unsigned char>(tiles * kFlagTile);
+  s.first = ws.take<uint32_t>(M);
   s.ranks = ws.take<uint4>(tiles * kThreads);
   LookbackState lb = carve_lookback(ws, tiles, 1u);
   s.error = lb.error;
@@ -508,33 +513,34 @@ int binned_impl(const void* seeds, const int64_t* seeds_ptr, const void* ids,
   }
   BatchItems<IdT> x{static_cast<const IdT*>(seeds), seeds_ptr, static_cast<const IdT*>(ids), ids_ptr,
                     B};
-  const int64_t flag_words16 = tiles * kFlagTile / 16;
-  int64_t n_init = flag_words16 > nb ? flag_words16 : nb;
-  if (tiles > n_init) n_init = tiles;
+  const int64_t n_init = tiles > nb ? tiles : nb;
   {
     ProfileScope prof("bins_init", stream);
     hipLaunchKernelGGL(bins_init_kernel, dim3(blocks_for(n_init, kThreads)), dim3(kThreads), 0,
-                       stream, s, flag_words16, nb, lb, tiles);
+                       stream, s, nb, lb, tiles);
     hipLaunchKernelGGL(bins_plan_kernel<IdT>, dim3(1), dim3(512), 0, stream, x, s.plan);
   }
+  const bool few = M / B <= kFewCountersItems;
   const unsigned part_grid = static_cast<unsigned>(blocks_for(M, kPartTile));
   {
     ProfileScope prof("bins_count", stream);
-    hipLaunchKernelGGL((bins_partition_kernel<IdT, false>), dim3(part_grid), dim3(kThreads), 0,
+    hipLaunchKernelGGL((few ? bins_partition_kernel<IdT, false, kFewCounters>
+                            : bins_partition_kernel<IdT, false, kCounterCap>), dim3(part_grid), dim3(kThreads), 0,
                        stream, x, M, s);
   }
   GS_RETURN_IF_ERROR(exclusive_scan(CountOf{s.count}, nb, s.bucket_ptr, scan_ws, stream));
   {
     ProfileScope prof("bins_scatter", stream);
-    hipLaunchKernelGGL((bins_partition_kernel<IdT, true>), dim3(part_grid), dim3(kThreads), 0,
+    hipLaunchKernelGGL((few ? bins_partition_kernel<IdT, true, kFewCounters>
+                            : bins_partition_kernel<IdT, true, kCounterCap>), dim3(part_grid), dim3(kThreads), 0,
                        stream, x, M, s);
   }
   // a workgroup per bucket (the bound: the number of buckets is on the device), rounded up so
   // that every XCD's share is whole
   const unsigned bucket_grid = static_cast<unsigned>((nb + kXcds - 1) / kXcds * kXcds);
   {
-    ProfileScope prof("bins_flag", stream);
-    hipLaunchKernelGGL(bins_flag_kernel, dim3(bucket_grid), dim3(kThreads), 0, stream, s, B);
+    ProfileScope prof("bins_first", stream);
+    hipLaunchKernelGGL(bins_first_kernel, dim3(bucket_grid), dim3(kThreads), 0, stream, s, B);
   }
   {
     ProfileScope prof("bins_rank", stream);
@@ -556,10 +562,10 @@ size_t binned_relabel_workspace_bytes(int64_t M, int64_t B) {
   if (M < 0) M = 0;
   if (B < 0) B = 0;
   const int64_t nb = buckets_bound(M, B);
-  const int64_t tiles = flag_tiles(M);
+  const int64_t tiles = rank_tiles(M);
   return padded((B + 1) * 4) + padded((B > 0 ? B : 1) * 4) + 3 * padded(nb * 4) +
          padded((nb + 1) * 8) + scan_workspace_bytes(nb) + padded((M > 0 ? M : 1) * 8) +
-         padded(tiles * kFlagTile) + padded(tiles * kThreads * 16) + lookback_state_bytes(tiles);
+         padded((M > 0 ? M : 1) * 4) + padded(tiles * kThreads * 16) + lookback_state_bytes(tiles);
 }
 
 bool binned_relabel_applies(int64_t M, int64_t B) {

@@ -209,6 +209,18 @@ def test_batch_csr_relabel_through_bins_at_size(dev, idt, narrow, shape):
                          np.array(ip, dtype=np.int64), narrow, None)
 
 
+def test_batch_csr_relabel_one_batch_beyond_the_counters(dev):
+    """Batches small on average and one with more classes than a tile's LDS counters; around it
+    batches on both sides of one class."""
+    rng = np.random.default_rng(9)
+    sizes = [(3, 2045), (0, 2049), (10, 9_000_000), (1, 0)] + [(2, 90)] * 12
+    sp = np.concatenate([[0], np.cumsum([a for a, _ in sizes])]).astype(np.int64)
+    ip = np.concatenate([[0], np.cumsum([n for _, n in sizes])]).astype(np.int64)
+    seeds = rng.integers(0, 1 << 22, sp[-1]).astype(np.int64)
+    ids = rng.integers(0, 1 << 22, ip[-1]).astype(np.int64)
+    _check_batch_relabel(dev, torch.int32, seeds, sp, ids, ip, False, None)
+
+
 def test_batch_csr_relabel_bins_report_what_they_cannot_take(dev):
     """An id beyond 32 bits among 64-bit ids promised to be narrow: -2, as on the hash regions.  A
     class with more distinct ids than its LDS table holds: -4 from the C ABI, and the host
