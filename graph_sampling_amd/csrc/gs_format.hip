@@ -20,7 +20,8 @@
 //    pass.  indptr then comes from the places where the sorted keys change, or, with
 //    fewer edges than columns, from one search per column confined to the keys of
 //    the workgroup's 256 columns.
-//  * distinct ids of an edge list: a byte per possible id, marked with plain stores.
+//  * distinct ids of an edge list: a bit per possible id in LDS, slice by slice, or, for short
+//    lists and large ids, a byte per possible id marked with plain stores.
 #include "gs_common.hpp"
 
 namespace gs {
@@ -826,8 +827,9 @@ int coo2csc_impl(const IdT* key, const IdT* value, int64_t E, int64_t num_keys, 
 // them; an id outside is reported and the caller counts another way.  The first end is
 // counted while the second is only looked through for its largest id: when the first holds
 // every id up to the largest of both, the second cannot hold more and its own count is left
-// out (any list with self loops).  What bounds the marking is one request to the L2 per edge.
-// 14 M edges, 64-bit ids: 0.22 ms where the two sorts took 1.79.
+// out (any list with self loops).  What bounds the marking is one request to the L2 per edge
+// and the lines that every die fetches again after another's stores: 180 us of 220 for 14 M
+// edges with 64-bit ids, so lists from 4 M edges on go by bits in LDS (below).
 constexpr int kMarkItems = 16;
 constexpr int kMarkTile = kThreads * kMarkItems;
 constexpr int kCountBlocks = 128;
@@ -836,6 +838,7 @@ struct DistinctSpace {
   unsigned char* map;  // range bytes for the first end, then for the second
   int64_t* largest;    // per workgroup of the first marking launch; -1: an id outside the range
   int64_t* partial;    // per workgroup of the counting launches
+  int64_t num_partial;
   int64_t* first;      // {distinct ids of the first end, 1 when the second has to be counted}
 };
 
@@ -917,10 +920,18 @@ __global__ void __launch_bounds__(kThreads) count_marks_kernel(DistinctSpace s, 
   if (threadIdx.x == 0) s.partial[blockIdx.x] = total;
 }
 
-// after the first end: is the second to be counted?  (one workgroup)
+// this thread's share of the counting launch's sums
+__device__ __forceinline__ int64_t sum_partial(const DistinctSpace& s, int threads) {
+  int64_t n = 0;
+  for (int64_t i = threadIdx.x; i < s.num_partial; i += threads) n += s.partial[i];
+  return n;
+}
+
+// after the first end: is the second to be counted?  (one workgroup; ids from `limit` on are
+// outside)
 constexpr int kDecideThreads = 1024;
 __global__ void __launch_bounds__(kDecideThreads)
-decide_second_kernel(DistinctSpace s, int64_t num_largest) {
+decide_second_kernel(DistinctSpace s, int64_t num_largest, int64_t limit) {
   __shared__ int64_t lds[kDecideThreads / kWave + 1];
   __shared__ int64_t s_top[kDecideThreads / kWave];
   int64_t top = 0;
@@ -933,25 +944,188 @@ decide_second_kernel(DistinctSpace s, int64_t num_largest) {
   }
   if ((threadIdx.x & (kWave - 1)) == 0) s_top[threadIdx.x / kWave] = top;
   int64_t total;
-  block_exclusive_scan<kDecideThreads>(threadIdx.x < kCountBlocks ? s.partial[threadIdx.x] : 0,
-                                       &total, lds);
+  block_exclusive_scan<kDecideThreads>(sum_partial(s, kDecideThreads), &total, lds);
   if (threadIdx.x == 0) {
     for (int w = 1; w < kDecideThreads / kWave; ++w) top = s_top[w] > top ? s_top[w] : top;
-    const bool outside = top == INT64_MAX;
-    s.first[0] = outside ? -1 : total;
+    const bool outside = top >= limit;
+    s.first[0] = !outside ? total : limit == INT64_MAX ? -1 : -2;
     s.first[1] = !outside && total <= top;  // (total = top + 1: every id up to the largest is there)
   }
 }
 
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kDecideThreads)
 post_distinct_kernel(DistinctSpace s, gs_mailbox* box, int64_t ticket) {
-  __shared__ int64_t lds[kThreads / kWave + 1];
+  __shared__ int64_t lds[kDecideThreads / kWave + 1];
   int64_t second = 0;
   const bool counted = s.first[1] != 0;
-  block_exclusive_scan<kThreads>(counted && threadIdx.x < kCountBlocks ? s.partial[threadIdx.x] : 0,
-                                 &second, lds);
-  // (-1, an id outside the range, leaves the second end uncounted)
+  block_exclusive_scan<kDecideThreads>(counted ? sum_partial(s, kDecideThreads) : 0, &second, lds);
+  // (-1 and -2, an id outside the range, leave the second end uncounted)
   if (threadIdx.x == 0) post_mailbox(box, counted && second > s.first[0] ? second : s.first[0], ticket);
+}
+
+// The same for long lists, by bits in LDS: every compute unit keeps a bitmap of 1.28 M ids and
+// marks its share of the edges there, the bitmaps go to memory and are or-ed and counted.
+// The first launch takes ids of the first slice and finds the largest id of both ends (its
+// workgroups read each end once); when that lies beyond, the second shares out the other
+// slices, reading the end once per slice: a stream against a request per edge.  Ids beyond
+// eight slices are reported and the caller asks for the bytes.  14 M edges over 2.45 M
+// nodes, 64-bit ids: 220 -> 145 us (617 -> 551 with the sort behind it; looking a bit up
+// before setting it, or asking for the next reads ahead, changed nothing).  The bitmaps are
+// 80 MB whatever the list, so lists
+// below 4 M edges stay with the bytes.
+constexpr int kBitWords = 39936;  // 156 KB of a compute unit's 160
+constexpr int64_t kSliceIds = int64_t(kBitWords) * 32;
+constexpr int kMaxSlices = 8;
+constexpr int kBitBlocks = 256;   // one for every compute unit
+constexpr int kBitThreads = 1024;
+constexpr int kBitTrip = 8;
+constexpr int64_t kBitMarkEdges = int64_t(1) << 22;
+constexpr int kOrRows = 16, kOrVecs = kThreads / kOrRows;  // of the counting launch
+constexpr int kOrBlocks = kBitWords / 4 / kOrVecs;
+static_assert(kBitWords % (4 * kOrVecs) == 0, "whole workgroups per slice");
+
+// largest id of both ends; every thread gets it
+template <int THREADS>
+__device__ __forceinline__ int64_t largest_of_list(const DistinctSpace& s) {
+  __shared__ int64_t s_top[THREADS / kWave];
+  int64_t top = 0;
+  for (int i = threadIdx.x; i < kBitBlocks; i += THREADS) top = s.largest[i] > top ? s.largest[i] : top;
+#pragma unroll
+  for (int d = kWave / 2; d > 0; d >>= 1) {
+    const int64_t o = __shfl_xor(top, d, kWave);
+    top = o > top ? o : top;
+  }
+  if ((threadIdx.x & (kWave - 1)) == 0) s_top[threadIdx.x / kWave] = top;
+  __syncthreads();
+  for (int w = 0; w < THREADS / kWave; ++w) top = s_top[w] > top ? s_top[w] : top;
+  return top;
+}
+
+// REST: the slices behind the first.  look: the other end, looked through for its largest id
+// (null when the largest is known).
+template <typename IdT, bool REST>
+__global__ void __launch_bounds__(kBitThreads)
+mark_bits_kernel(const IdT* __restrict__ ids, const IdT* __restrict__ look, int64_t E, DistinctSpace s,
+                 bool second) {
+  __shared__ __attribute__((aligned(16))) uint32_t s_bits[kBitWords];
+  __shared__ int64_t s_wave[kBitThreads / kWave];
+  if (second && !s.first[1]) return;
+  int64_t slice = 0, part = blockIdx.x, parts = kBitBlocks;
+  if (REST) {
+    const int64_t rest = largest_of_list<kBitThreads>(s) / kSliceIds;  // slices behind the first
+    if (rest < 1 || rest >= kMaxSlices) return;
+    parts = kBitBlocks / rest;
+    slice = 1 + blockIdx.x % rest;
+    part = blockIdx.x / rest;
+    if (part >= parts) return;
+  }
+  for (int j = threadIdx.x; j < kBitWords / 4; j += kBitThreads)
+    reinterpret_cast<uint4*>(s_bits)[j] = make_uint4(0, 0, 0, 0);
+  __syncthreads();
+  const int64_t lo = E * part / parts, hi = E * (part + 1) / parts;
+  const uint64_t first_id = static_cast<uint64_t>(slice * kSliceIds);
+  uint64_t largest = 0;  // (an id below zero is a huge one here)
+  for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += kBitTrip * kBitThreads) {
+    IdT id[kBitTrip];
+#pragma unroll
+    for (int u = 0; u < kBitTrip; ++u) {
+      const int64_t i = i0 + u * kBitThreads;
+      id[u] = ids[i < hi ? i : hi - 1];
+    }
+#pragma unroll
+    for (int u = 0; u < kBitTrip; ++u) {
+      const uint64_t v = static_cast<uint64_t>(static_cast<int64_t>(id[u]));
+      largest = v > largest ? v : largest;
+      const uint64_t in = v - first_id;
+      if (in < static_cast<uint64_t>(kSliceIds)) {
+        const uint32_t at = static_cast<uint32_t>(in);
+        atomicOr(&s_bits[at >> 5], 1u << (at & 31u));
+      }
+    }
+  }
+  if (!REST && look) {
+    for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += kBitTrip * kBitThreads) {
+      IdT id[kBitTrip];
+#pragma unroll
+      for (int u = 0; u < kBitTrip; ++u) {
+        const int64_t i = i0 + u * kBitThreads;
+        id[u] = look[i < hi ? i : hi - 1];
+      }
+#pragma unroll
+      for (int u = 0; u < kBitTrip; ++u) {
+        const uint64_t v = static_cast<uint64_t>(static_cast<int64_t>(id[u]));
+        largest = v > largest ? v : largest;
+      }
+    }
+    int64_t top = largest >> 62 ? INT64_MAX : static_cast<int64_t>(largest);
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) {
+      const int64_t o = __shfl_xor(top, d, kWave);
+      top = o > top ? o : top;
+    }
+    if ((threadIdx.x & (kWave - 1)) == 0) s_wave[threadIdx.x / kWave] = top;
+  }
+  __syncthreads();
+  if (!REST && look && threadIdx.x == 0) {
+    int64_t top = 0;
+    for (int w = 0; w < kBitThreads / kWave; ++w) top = s_wave[w] > top ? s_wave[w] : top;
+    s.largest[blockIdx.x] = top;
+  }
+  uint4* out = reinterpret_cast<uint4*>(s.map) +
+               static_cast<int64_t>((REST ? kBitBlocks : 0) + blockIdx.x) * (kBitWords / 4);
+  for (int j = threadIdx.x; j < kBitWords / 4; j += kBitThreads)
+    out[j] = reinterpret_cast<const uint4*>(s_bits)[j];
+}
+
+// Ids in any bitmap of slice blockIdx.y: sixteen threads share the bitmaps of a word.
+__global__ void __launch_bounds__(kThreads) count_bits_kernel(DistinctSpace s, bool second) {
+  __shared__ uint4 s_or[kOrRows][kOrVecs];
+  __shared__ int64_t s_scan[kThreads / kWave + 1];
+  if (second && !s.first[1]) return;
+  const int64_t rest = largest_of_list<kThreads>(s) / kSliceIds;
+  const int64_t slice = blockIdx.y;
+  int64_t n = 0;
+  if (slice <= rest && rest < kMaxSlices) {  // (the same for the whole workgroup)
+    const int64_t step = slice ? rest : 1;
+    const int64_t rows = kBitBlocks / step, row0 = slice ? kBitBlocks + slice - 1 : 0;
+    const int g = threadIdx.x / kOrVecs, v = threadIdx.x % kOrVecs;
+    const uint4* map = reinterpret_cast<const uint4*>(s.map) + static_cast<int64_t>(blockIdx.x) * kOrVecs + v;
+    uint4 all = make_uint4(0, 0, 0, 0);
+#pragma unroll 8
+    for (int64_t r = g; r < rows; r += kOrRows) {
+      const uint4 x = map[(row0 + r * step) * (kBitWords / 4)];
+      all.x |= x.x; all.y |= x.y; all.z |= x.z; all.w |= x.w;
+    }
+    s_or[g][v] = all;
+    __syncthreads();
+    if (g == 0) {
+      for (int r = 1; r < kOrRows; ++r) {
+        const uint4 x = s_or[r][v];
+        all.x |= x.x; all.y |= x.y; all.z |= x.z; all.w |= x.w;
+      }
+      n = __popc(all.x) + __popc(all.y) + __popc(all.z) + __popc(all.w);
+    }
+  }
+  int64_t total;
+  block_exclusive_scan<kThreads>(n, &total, s_scan);
+  if (threadIdx.x == 0) s.partial[blockIdx.y * kOrBlocks + blockIdx.x] = total;
+}
+
+template <typename IdT>
+void distinct_by_bits(const IdT* a, const IdT* b, int64_t E, const DistinctSpace& s, hipStream_t st) {
+  for (int end = 0; end < 2; ++end) {
+    const IdT* ids = end ? b : a;
+    const IdT* look = end ? nullptr : b;
+    hipLaunchKernelGGL((mark_bits_kernel<IdT, false>), dim3(kBitBlocks), dim3(kBitThreads), 0, st, ids,
+                       look, E, s, end == 1);
+    hipLaunchKernelGGL((mark_bits_kernel<IdT, true>), dim3(kBitBlocks), dim3(kBitThreads), 0, st, ids,
+                       look, E, s, end == 1);
+    hipLaunchKernelGGL(count_bits_kernel, dim3(kOrBlocks, kMaxSlices), dim3(kThreads), 0, st, s,
+                       end == 1);
+    if (end == 0)
+      hipLaunchKernelGGL(decide_second_kernel, dim3(1), dim3(kDecideThreads), 0, st, s,
+                         static_cast<int64_t>(kBitBlocks), kMaxSlices * kSliceIds);
+  }
 }
 
 // bytes per end of the list, a multiple of 16; ids of a graph with up to a million nodes always fit
@@ -1196,22 +1370,29 @@ size_t gs_coo2csc_workspace_bytes(int64_t E, int64_t num_keys) {
 
 size_t gs_distinct_ends_workspace_bytes(int64_t E) {
   if (E < 0) E = 0;
-  return padded(2 * static_cast<size_t>(mark_range(E))) +
-         padded(2 * static_cast<size_t>(blocks_for(E, kMarkTile)) * 8) + padded(kCountBlocks * 8) + 256;
+  size_t map = 2 * static_cast<size_t>(mark_range(E));
+  const size_t bits = static_cast<size_t>(2 * kBitBlocks) * kBitWords * 4;
+  if (E >= kBitMarkEdges && bits > map) map = bits;
+  const size_t largest = 2 * static_cast<size_t>(blocks_for(E, kMarkTile)) + kBitBlocks;
+  return padded(map) + padded(largest * 8) + padded(kOrBlocks * kMaxSlices * 8) + 256;
 }
 
 int gs_distinct_ends(const void* a, const void* b, int id_bytes, int64_t E, void* workspace,
                      size_t workspace_bytes, gs_mailbox* mailbox, int64_t ticket, void* stream) {
+  const bool by_bits = !(id_bytes & GS_DISTINCT_BYTES) && E >= kBitMarkEdges;
+  id_bytes &= ~GS_DISTINCT_BYTES;
   GS_REQUIRE(E > 0 && E < (int64_t(1) << 32) - 8192 && a && b && mailbox,
              "gs_distinct_ends: bad argument");
   GS_REQUIRE(valid_id_bytes(id_bytes), "gs_distinct_ends: id_bytes must be 4 or 8, got %d", id_bytes);
   const int64_t range = mark_range(E);
   const int blocks = blocks_for(E, kMarkTile);
+  const size_t bits = static_cast<size_t>(2 * kBitBlocks) * kBitWords * 4;
   Carver ws(workspace, workspace_bytes);
   DistinctSpace s;
-  s.map = ws.take<unsigned char>(static_cast<size_t>(2 * range));
-  s.largest = ws.take<int64_t>(2 * static_cast<size_t>(blocks));
-  s.partial = ws.take<int64_t>(kCountBlocks);
+  s.map = ws.take<unsigned char>(by_bits ? bits : static_cast<size_t>(2 * range));
+  s.largest = ws.take<int64_t>(2 * static_cast<size_t>(blocks) + kBitBlocks);
+  s.num_partial = by_bits ? kOrBlocks * kMaxSlices : kCountBlocks;
+  s.partial = ws.take<int64_t>(static_cast<size_t>(s.num_partial));
   s.first = ws.take<int64_t>(2);
   if (!ws.ok) {
     set_error_text("gs_distinct_ends: workspace needs %zu bytes, 256-byte aligned",
@@ -1219,24 +1400,31 @@ int gs_distinct_ends(const void* a, const void* b, int id_bytes, int64_t E, void
     return GS_ERR_WORKSPACE;
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int64_t vecs = 2 * range / 16;
-  hipLaunchKernelGGL(clear_marks_kernel, dim3(blocks_for(vecs, kThreads * 4)), dim3(kThreads), 0, st,
-                     reinterpret_cast<uint4*>(s.map), vecs);
-  auto both = [&](auto first, auto second, auto* pa, auto* pb) {
-    hipLaunchKernelGGL(first, dim3(blocks, 2), dim3(kThreads), 0, st, pa, pb, E, range, s);
-    hipLaunchKernelGGL(count_marks_kernel<true>, dim3(kCountBlocks), dim3(kThreads), 0, st, s, range);
-    hipLaunchKernelGGL(decide_second_kernel, dim3(1), dim3(kDecideThreads), 0, st, s,
-                       static_cast<int64_t>(2) * blocks);
-    hipLaunchKernelGGL(second, dim3(blocks), dim3(kThreads), 0, st, pa, pb, E, range, s);
-    hipLaunchKernelGGL(count_marks_kernel<false>, dim3(kCountBlocks), dim3(kThreads), 0, st, s, range);
-  };
-  if (id_bytes == 8)
-    both(mark_ids_kernel<int64_t, true>, mark_ids_kernel<int64_t, false>,
-         static_cast<const int64_t*>(a), static_cast<const int64_t*>(b));
-  else
-    both(mark_ids_kernel<int32_t, true>, mark_ids_kernel<int32_t, false>,
-         static_cast<const int32_t*>(a), static_cast<const int32_t*>(b));
-  hipLaunchKernelGGL(post_distinct_kernel, dim3(1), dim3(kThreads), 0, st, s, mailbox, ticket);
+  if (by_bits) {
+    if (id_bytes == 8)
+      distinct_by_bits(static_cast<const int64_t*>(a), static_cast<const int64_t*>(b), E, s, st);
+    else
+      distinct_by_bits(static_cast<const int32_t*>(a), static_cast<const int32_t*>(b), E, s, st);
+  } else {
+    const int64_t vecs = 2 * range / 16;
+    hipLaunchKernelGGL(clear_marks_kernel, dim3(blocks_for(vecs, kThreads * 4)), dim3(kThreads), 0, st,
+                       reinterpret_cast<uint4*>(s.map), vecs);
+    auto both = [&](auto first, auto second, auto* pa, auto* pb) {
+      hipLaunchKernelGGL(first, dim3(blocks, 2), dim3(kThreads), 0, st, pa, pb, E, range, s);
+      hipLaunchKernelGGL(count_marks_kernel<true>, dim3(kCountBlocks), dim3(kThreads), 0, st, s, range);
+      hipLaunchKernelGGL(decide_second_kernel, dim3(1), dim3(kDecideThreads), 0, st, s,
+                         static_cast<int64_t>(2) * blocks, static_cast<int64_t>(INT64_MAX));
+      hipLaunchKernelGGL(second, dim3(blocks), dim3(kThreads), 0, st, pa, pb, E, range, s);
+      hipLaunchKernelGGL(count_marks_kernel<false>, dim3(kCountBlocks), dim3(kThreads), 0, st, s, range);
+    };
+    if (id_bytes == 8)
+      both(mark_ids_kernel<int64_t, true>, mark_ids_kernel<int64_t, false>,
+           static_cast<const int64_t*>(a), static_cast<const int64_t*>(b));
+    else
+      both(mark_ids_kernel<int32_t, true>, mark_ids_kernel<int32_t, false>,
+           static_cast<const int32_t*>(a), static_cast<const int32_t*>(b));
+  }
+  hipLaunchKernelGGL(post_distinct_kernel, dim3(1), dim3(kDecideThreads), 0, st, s, mailbox, ticket);
   return check_launch("distinct_ends");
 }
 

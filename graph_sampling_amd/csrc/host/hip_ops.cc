@@ -1420,11 +1420,16 @@ int64_t DistinctEnds(const torch::Tensor& a, const torch::Tensor& b) {
   auto ws = Scratch(gs_distinct_ends_workspace_bytes(E), a);
   void* st = Stream(a);
   HostBoxes& boxes = Boxes(a.get_device());
-  const int64_t ticket = boxes.next++;
-  Check(gs_distinct_ends(a.data_ptr(), b.data_ptr(), idb, E, ws.data_ptr(), ws.numel(),
-                         boxes.slot(ticket), ticket, st),
-        "gs_distinct_ends");
-  return WaitBox(boxes.slot(ticket), ticket, st, "gs_distinct_ends");
+  int64_t nodes = -2;  // (-2: ids too large for the bits in LDS, counted again by bytes)
+  for (const int how : {0, GS_DISTINCT_BYTES}) {
+    const int64_t ticket = boxes.next++;
+    Check(gs_distinct_ends(a.data_ptr(), b.data_ptr(), idb | how, E, ws.data_ptr(), ws.numel(),
+                           boxes.slot(ticket), ticket, st),
+          "gs_distinct_ends");
+    nodes = WaitBox(boxes.slot(ticket), ticket, st, "gs_distinct_ends");
+    if (nodes != -2) break;
+  }
+  return nodes;
 }
 
 std::tuple<torch::Tensor, torch::Tensor> SortValuesByKey(const torch::Tensor& key,

@@ -806,8 +806,11 @@ int gs_csc2coo(const int64_t* indptr, int64_t num_cols, int64_t nnz, void* col, 
 /* How many distinct ids each of the two ends a[0..E), b[0..E) of an edge list holds, the larger
  * of the two posted to the mailbox (what Graph::LoadCOO takes for the node count,
  * src/graph.cc:25-35).  Ids from 0 up to about the number of edges (a million at the least)
- * are counted; when one lies outside, -1 is posted and the caller counts another way.
+ * are counted; when one lies outside, -1 is posted and the caller counts another way.  Lists of
+ * 2^22 edges and more are counted by bits in LDS, which takes ids up to ten million; -2 is posted
+ * when one is larger, and GS_DISTINCT_BYTES or-ed into id_bytes counts by bytes in memory.
  * workspace: gs_distinct_ends_workspace_bytes(E) bytes, 256-byte aligned. */
+#define GS_DISTINCT_BYTES 0x800
 size_t gs_distinct_ends_workspace_bytes(int64_t E);
 int gs_distinct_ends(const void* a, const void* b, int id_bytes, int64_t E, void* workspace,
                      size_t workspace_bytes, gs_mailbox* mailbox, int64_t ticket, void* stream);

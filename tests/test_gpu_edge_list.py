@@ -32,6 +32,44 @@ def test_node_count_of_an_edge_list(dev, E, how, idt):
     assert g._CAPI_GetNumRows() == max(np.unique(row).size, np.unique(col).size)
 
 
+SLICE = 39936 * 32  # ids of one LDS bitmap
+
+
+@pytest.mark.parametrize("idt", ID_DTYPES)
+@pytest.mark.parametrize("largest", [40, SLICE - 1, SLICE, 2 * SLICE, 5 * SLICE + 7, 8 * SLICE - 1,
+                                     8 * SLICE])
+@pytest.mark.parametrize("how", ["complete", "second_larger", "first_larger"])
+def test_node_count_of_a_long_list(dev, largest, how, idt):
+    """Lists counted by bits in LDS, the largest id on both sides of a slice's and of the last
+    slice's end (beyond it: by bytes), in the first end or in the second only."""
+    E = (1 << 22) + 3
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(largest % 1_000_003)
+    row, col = (torch.randint(0, largest + 1, (E,), generator=gen, device=dev) for _ in range(2))
+    if how == "complete" and largest < E:
+        row = torch.arange(E, device=dev) % (largest + 1)
+    elif how == "second_larger":
+        row = row // 3
+        col[E - 1] = largest
+    else:
+        col = col // 3
+        row[E // 2] = largest
+    g = gs.Graph(False)
+    g._CAPI_LoadCOO(row.to(idt), col.to(idt))
+    assert g._CAPI_GetNumRows() == max(torch.unique(row).numel(), torch.unique(col).numel())
+
+
+@pytest.mark.parametrize("idt", ID_DTYPES)
+@pytest.mark.parametrize("stray", [-1, (1 << 31) - 1])
+def test_node_count_of_a_long_list_with_a_stray_id(dev, stray, idt):
+    E = 1 << 22
+    row, col = torch.arange(E, device=dev) % 1000, torch.arange(E, device=dev) % 77
+    col[E - 2] = stray
+    g = gs.Graph(False)
+    g._CAPI_LoadCOO(row.to(idt), col.to(idt))
+    assert g._CAPI_GetNumRows() == 1000
+
+
 @pytest.mark.parametrize("idt", ID_DTYPES)
 @pytest.mark.parametrize("extra", [0, 1, 8191])
 @pytest.mark.parametrize("num_keys", [200, 60_000, 3_000_000])
