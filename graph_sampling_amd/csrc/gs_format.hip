@@ -971,8 +971,7 @@ post_distinct_kernel(DistinctSpace s, gs_mailbox* box, int64_t ticket) {
 // eight slices are reported and the caller asks for the bytes.  14 M edges over 2.45 M
 // nodes, 64-bit ids: 220 -> 145 us (617 -> 551 with the sort behind it; looking a bit up
 // before setting it, or asking for the next reads ahead, changed nothing).  The bitmaps are
-// 80 MB whatever the list, so lists
-// below 4 M edges stay with the bytes.
+// 80 MB whatever the list, so lists below 4 M edges stay with the bytes.
 constexpr int kBitWords = 39936;  // 156 KB of a compute unit's 160
 constexpr int64_t kSliceIds = int64_t(kBitWords) * 32;
 constexpr int kMaxSlices = 8;
