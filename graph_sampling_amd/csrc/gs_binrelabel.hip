@@ -28,7 +28,7 @@
 // A record is read once and never written again; of the three places an item touches at
 // random (its first position's store, the rank it looks up, and before these passes were in
 // the order of the positions its new name and its place in the frontier) two are left, and a
-// first occurrence looks up nothing.  17 M items in 64 batches: first 111 -> 112 us (with
+// first occurrence looks up nothing.  17 M items in 64 batches: first 111 -> 104 us (with
 // half as many, twice as large buckets: 132 before that), rank 15 -> 25, rename 143 -> 88.
 //
 // Buckets are handed to workgroups so that consecutive buckets -- one batch's -- run on the
@@ -71,7 +71,10 @@ constexpr int kFewCounters = counter_cap(10);
 constexpr int64_t kFewCountersItems = int64_t(1) << 20;
 constexpr int kSlots = 4096;           // LDS table of a bucket (8-byte slots)
 constexpr int kRankTile = kThreads * 64;  // positions of a workgroup in the rank pass
-constexpr int kTrip = 10;  // records of a thread that are asked for together (a whole bucket nearly always)
+// Threads of a bucket's workgroup: the table lets five of them share a compute unit, 20 waves
+// of 256 threads, 32 of 512 (17 M items: 112 -> 104 us; 4.3 M: 39 -> 30).
+constexpr int kBucketThreads = 512;
+constexpr int kTrip = 5;  // records of a thread that are asked for together (a whole bucket nearly always)
 
 struct Plan {
   uint32_t* bucket_base;  // [B + 1]: first bucket of every batch; [B] = number of buckets
@@ -276,15 +279,15 @@ __device__ __forceinline__ void table_fill(unsigned long long* __restrict__ tab,
                                            unsigned long long (&rec)[kTrip]) {
 #pragma unroll
   for (int u = 0; u < kTrip; ++u) {
-    const int64_t r = begin + u * kThreads + threadIdx.x;
+    const int64_t r = begin + u * kBucketThreads + threadIdx.x;
     rec[u] = records[r < end ? r : end - 1];
   }
-  for (int c = threadIdx.x; c < kSlots; c += kThreads) tab[c] = ~0ull;
+  for (int c = threadIdx.x; c < kSlots; c += kBucketThreads) tab[c] = ~0ull;
   __syncthreads();
-  for (int64_t r0 = begin; r0 < end; r0 += kTrip * kThreads) {
+  for (int64_t r0 = begin; r0 < end; r0 += kTrip * kBucketThreads) {
 #pragma unroll
     for (int u = 0; u < kTrip; ++u) {
-      if (r0 + u * kThreads + threadIdx.x < end) {
+      if (r0 + u * kBucketThreads + threadIdx.x < end) {
         const uint32_t key = static_cast<uint32_t>(rec[u] >> 32);
         uint32_t p = slot_of(key);
         int probes = 0;
@@ -303,10 +306,10 @@ __device__ __forceinline__ void table_fill(unsigned long long* __restrict__ tab,
         }
       }
     }
-    if (r0 + kTrip * kThreads < end) {
+    if (r0 + kTrip * kBucketThreads < end) {
 #pragma unroll
       for (int u = 0; u < kTrip; ++u) {
-        const int64_t r = r0 + (kTrip + u) * kThreads + threadIdx.x;
+        const int64_t r = r0 + (kTrip + u) * kBucketThreads + threadIdx.x;
         rec[u] = records[r < end ? r : end - 1];
       }
     }
@@ -316,7 +319,7 @@ __device__ __forceinline__ void table_fill(unsigned long long* __restrict__ tab,
 
 // One workgroup per bucket: every record's position gets the smallest position of its id.
 // (A bucket of one trip, as most are, still holds its records in registers by then.)
-__global__ void __launch_bounds__(kThreads) bins_first_kernel(Bins s, int64_t B) {
+__global__ void __launch_bounds__(kBucketThreads) bins_first_kernel(Bins s, int64_t B) {
   __shared__ unsigned long long tab[kSlots];
   const int64_t k = bucket_of_workgroup(s.plan.bucket_base[B]);
   if (k < 0) return;
@@ -324,12 +327,12 @@ __global__ void __launch_bounds__(kThreads) bins_first_kernel(Bins s, int64_t B)
   if (begin == end) return;
   unsigned long long rec[kTrip];
   table_fill(tab, s.records, begin, end, s.error, rec);
-  const int64_t trips = (end - begin + kTrip * kThreads - 1) / (kTrip * kThreads);
+  const int64_t trips = (end - begin + kTrip * kBucketThreads - 1) / (kTrip * kBucketThreads);
   for (int64_t t = trips - 1; t >= 0; --t) {  // (from the last trip backwards)
-    const int64_t r0 = begin + t * (kTrip * kThreads);
+    const int64_t r0 = begin + t * (kTrip * kBucketThreads);
 #pragma unroll
     for (int u = 0; u < kTrip; ++u) {
-      if (r0 + u * kThreads + threadIdx.x < end) {
+      if (r0 + u * kBucketThreads + threadIdx.x < end) {
         const uint32_t key = static_cast<uint32_t>(rec[u] >> 32);
         uint32_t p = slot_of(key);
         int probes = 0;
@@ -344,7 +347,7 @@ __global__ void __launch_bounds__(kThreads) bins_first_kernel(Bins s, int64_t B)
     }
     if (t > 0) {
 #pragma unroll
-      for (int u = 0; u < kTrip; ++u) rec[u] = s.records[r0 - (kTrip - u) * kThreads + threadIdx.x];
+      for (int u = 0; u < kTrip; ++u) rec[u] = s.records[r0 - (kTrip - u) * kBucketThreads + threadIdx.x];
     }
   }
 }
@@ -540,7 +543,7 @@ int binned_impl(const void* seeds, const int64_t* seeds_ptr, const void* ids,
   const unsigned bucket_grid = static_cast<unsigned>((nb + kXcds - 1) / kXcds * kXcds);
   {
     ProfileScope prof("bins_first", stream);
-    hipLaunchKernelGGL(bins_first_kernel, dim3(bucket_grid), dim3(kThreads), 0, stream, s, B);
+    hipLaunchKernelGGL(bins_first_kernel, dim3(bucket_grid), dim3(kBucketThreads), 0, stream, s, B);
   }
   {
     ProfileScope prof("bins_rank", stream);
