@@ -16,6 +16,9 @@
 // second time.  A 300 000-edge hub is 75 workgroups' work, and the order of the additions
 // is fixed by the edges' layout alone, so results repeat from run to run.
 //
+// Tiles, marks and pieces count from the first offset, so a range of a larger matrix's columns,
+// offsets and data as they stand there, costs what its own edges cost.
+//
 // A workgroup learns its segments from the offsets, 64 at a time in each wave, from the one
 // that holds its first edge on; with few edges per segment (a slice's rows among all rows:
 // millions of empty segments) from one int per edge that a pass over the offsets has left at
@@ -51,6 +54,23 @@ struct Tiles {
   int* mark;      // [edges] kMarks: the segment that starts at the edge, or -1
 };
 
+// The edges of the offsets.  The caller's count is an upper bound; there is workspace for that many.
+struct Edges {
+  int64_t first, end;
+  __device__ __forceinline__ Edges(const int64_t* __restrict__ indptr, int64_t num_seg, int64_t nnz)
+      : first(indptr[0]), end(indptr[num_seg]) {
+    if (end - first > nnz) end = first + nnz;
+  }
+  // Edges of the tile that begins at p0 < end.  (The empty statement holds the number apart from
+  // comparisons of it with a whole tile: where the compiler folds such a one into the minimum's, it
+  // loses the instruction that hands the result to the selection, and every tile counts as whole.)
+  __device__ __forceinline__ int in_tile(int64_t p0) const {
+    int n = static_cast<int>(end - p0 < kTile ? end - p0 : kTile);
+    asm volatile("" : "+s"(n));
+    return n;
+  }
+};
+
 // How a workgroup learns its segments.
 enum Walk {
   kSearch,  // it searches the offsets for the tile's first and last, and leaves the first in head[]
@@ -69,16 +89,20 @@ __global__ void __launch_bounds__(kThreads) clear_marks_kernel(int* mark, int64_
 template <bool SUM, bool MARK, typename IdT>
 __global__ void __launch_bounds__(kThreads)
 tile_heads_kernel(const int64_t* __restrict__ indptr, const IdT* __restrict__ nmap, int64_t num_seg,
-                  float* __restrict__ out, Tiles tl) {
+                  int64_t nnz, float* __restrict__ out, Tiles tl) {
   const int64_t s = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  const Edges edges(indptr, num_seg, nnz);
   int64_t t0 = 0, t1 = -1;
   if (s < num_seg) {
     const int64_t begin = indptr[s], end = indptr[s + 1];
     if (end > begin) {
-      t0 = (begin + kTile - 1) / kTile;
-      t1 = (end - 1) / kTile;
-      if (end == indptr[num_seg]) tl.head[t1 + 1] = static_cast<int>(s);
-      if (MARK) tl.mark[begin] = static_cast<int>(s);
+      const int64_t stop = end < edges.end ? end : edges.end;
+      t0 = (begin - edges.first + kTile - 1) / kTile;
+      t1 = (stop - edges.first - 1) / kTile;
+      if (begin < stop) {
+        if (stop == edges.end) tl.head[t1 + 1] = static_cast<int>(s);
+        if (MARK) tl.mark[begin - edges.first] = static_cast<int>(s);
+      }
     } else if (SUM) {
       out[nmap ? static_cast<int64_t>(nmap[s]) : s] = 0.0f;
     }
@@ -95,6 +119,14 @@ tile_heads_kernel(const int64_t* __restrict__ indptr, const IdT* __restrict__ nm
     const int64_t ws = __shfl(s, src, kWave);
     for (int64_t t = w0 + lane; t <= w1; t += kWave) tl.head[t] = static_cast<int>(ws);
   }
+}
+
+// first and last tile of segment g, which has edges
+__device__ __forceinline__ void tiles_of(const int64_t* __restrict__ indptr, int64_t g,
+                                         const Edges& edges, int64_t* from, int64_t* to) {
+  const int64_t end = indptr[g + 1] < edges.end ? indptr[g + 1] : edges.end;
+  *from = (indptr[g] - edges.first) / kTile;
+  *to = (end - edges.first - 1) / kTile;
 }
 
 // sum over the 16 lanes of a row, in every lane
@@ -134,26 +166,36 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
   // (the last tile first: where columns are numbered with the busy ones in front, the tiles of
   // thousands of columns, which take several times as long, come last, and the chip would wait for
   // the last of them: 144 -> 128 us)
-  const int64_t t = gridDim.x - 1 - blockIdx.x, p0 = t * kTile;
+  const int64_t t = gridDim.x - 1 - blockIdx.x;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-  // (what the chain of dependent reads starts with goes out first)
+  // (what the chain of dependent reads starts with goes out first; the data wait for the first and
+  // the last offset, since an array may end where the offsets do: 124 M edges take 126 us in a sum
+  // and 264 in a normalise with that wait, 127 and 262 without)
   int64_t head = 0, tail = 0;  // segments of the tile's first edge and of the one behind its last
   if (WALK != kSearch) {
     head = tl.head[t];
     if (WALK == kHeads) tail = tl.head[t + 1];
   }
-  const int64_t all = indptr[num_seg];
-  const bool vec = SOURCE == kPlain && p0 + kTile <= nnz;
+  const Edges edges(indptr, num_seg, nnz);
+  const int64_t p0 = edges.first + t * kTile;
+  if (p0 >= edges.end) return;
+  const int n = edges.in_tile(p0);
+  const int64_t p1 = p0 + n;
+  const bool vec = SOURCE == kPlain && n == kTile && (reinterpret_cast<uintptr_t>(data + p0) & 15u) == 0;
   F4 q[kTileItems / kLaneEdges];
   if (vec) {
 #pragma unroll
     for (int k = 0; k < kTileItems / kLaneEdges; ++k)
       q[k] = *reinterpret_cast<const F4*>(data + p0 + (k * kThreads + tid) * kLaneEdges);
+  } else if constexpr (SOURCE == kPlain) {  // (the last tile, or a first offset that is no multiple of 4)
+#pragma unroll
+    for (int k = 0; k < kTileItems / kLaneEdges; ++k)
+#pragma unroll
+      for (int u = 0; u < kLaneEdges; ++u) {
+        const int i = (k * kThreads + tid) * kLaneEdges + u;
+        q[k][u] = data[p0 + (i < n ? i : n - 1)];
+      }
   }
-  if (all < nnz) nnz = all;  // the caller's count is an upper bound
-  if (p0 >= nnz) return;
-  const int n = static_cast<int>(nnz - p0 < kTile ? nnz - p0 : kTile);
-  const int64_t p1 = p0 + n;
 
   int64_t where[EMAP ? kTileItems : 1];
   float x[kTileItems];
@@ -202,7 +244,7 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
     s_out = -1;
   }
   // x^powk of a thread's edges, one loop for all of them (the products are powk_f's)
-  if (vec) {
+  if constexpr (SOURCE == kPlain) {
     F4 p[kTileItems / kLaneEdges];
 #pragma unroll
     for (int k = 0; k < kTileItems / kLaneEdges; ++k) p[k] = q[k];
@@ -214,8 +256,6 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
 #pragma unroll
     for (int k = 0; k < kTileItems / kLaneEdges; ++k)
       *reinterpret_cast<F4*>(s_v + (k * kThreads + tid) * kLaneEdges) = p[k];
-  } else if constexpr (SOURCE == kPlain) {  // (the last tile)
-    for (int i = tid; i < n; i += kThreads) s_v[i] = NORMALIZE ? data[p0 + i] : powk_f(data[p0 + i], powk);
   } else {
     float p[kTileItems];
 #pragma unroll
@@ -357,7 +397,7 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
 #pragma unroll
       for (int k = 0; k < kQuarter / kWave; ++k) {
         const int64_t p = q0 + k * kWave + lane;
-        seg[k] = p < p1 ? tl.mark[p] : -1;
+        seg[k] = p < p1 ? tl.mark[p - edges.first] : -1;
       }
       int64_t begin_in = 0;
       bool incoming = false;
@@ -421,7 +461,7 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
         const int i = k * kThreads + tid;
         if (i >= first && i < stop) out[where[k]] = s_v[i];
       }
-    } else if (vec && n == kTile && (reinterpret_cast<uintptr_t>(out) & 15u) == 0) {
+    } else if (vec && (reinterpret_cast<uintptr_t>(out + p0) & 15u) == 0) {
 #pragma unroll
       for (int k = 0; k < kTileItems / kLaneEdges; ++k) {
         const int i = (k * kThreads + tid) * kLaneEdges;
@@ -454,19 +494,19 @@ crossing_divide_kernel(const int64_t* __restrict__ indptr, const int64_t* __rest
                        const float* __restrict__ data, int64_t num_seg, int64_t nnz,
                        float* __restrict__ out, Tiles tl) {
   __shared__ float s_total[2];
-  const int64_t t = blockIdx.x, p0 = t * kTile;
-  const int64_t all = indptr[num_seg];
+  const int64_t t = blockIdx.x;
+  const Edges edges(indptr, num_seg, nnz);
+  const int64_t p0 = edges.first + t * kTile;
   const int inner = tl.inner[t], g_in = tl.head[t], g_out = tl.outgoing[t];
-  if (all < nnz) nnz = all;
-  if (p0 >= nnz) return;
-  const int n = static_cast<int>(nnz - p0 < kTile ? nnz - p0 : kTile);
+  if (p0 >= edges.end) return;
+  const int n = edges.in_tile(p0);
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   int first = inner & 0xFFFF;
   const int stop = inner >> 16;
   if (first > 0 && indptr[g_in + 1] - indptr[g_in] <= kLaneMaxLen) first = 0;  // (done where it starts)
   if (first == 0 && stop == n) return;
   const bool vec = !EMAP && n == kTile &&
-                   ((reinterpret_cast<uintptr_t>(data) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
+                   ((reinterpret_cast<uintptr_t>(data + p0) | reinterpret_cast<uintptr_t>(out + p0)) & 15u) == 0;
   float4 v[kTileItems / 4];
   if (vec) {
 #pragma unroll
@@ -479,7 +519,8 @@ crossing_divide_kernel(const int64_t* __restrict__ indptr, const int64_t* __rest
   if (wave < 2) {
     const int g = wave == 0 ? (first > 0 ? g_in : -1) : g_out;
     if (g >= 0) {
-      const int64_t from = indptr[g] / kTile, to = (indptr[g + 1] - 1) / kTile;
+      int64_t from, to;
+      tiles_of(indptr, g, edges, &from, &to);
       float part = 0.0f;
       for (int64_t k = from + 1 + lane; k <= to; k += kWave) part += tl.carry[2 * k];
 #pragma unroll
@@ -524,14 +565,14 @@ template <typename IdT>
 __global__ void __launch_bounds__(kThreads)
 carry_kernel(const int64_t* __restrict__ indptr, const IdT* __restrict__ nmap, int64_t num_seg,
              int64_t nnz, float* __restrict__ sums, Tiles tl) {
-  if (indptr[num_seg] < nnz) nnz = indptr[num_seg];
+  const Edges edges(indptr, num_seg, nnz);
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t t = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
   int g = -1;
-  int64_t last = 0;  // last tile the segment reaches
-  if (t * kTile < nnz) {
+  int64_t from = 0, last = 0;  // tiles the segment starts in and reaches
+  if (edges.first + t * kTile < edges.end) {
     g = tl.outgoing[t];
-    if (g >= 0) last = (indptr[g + 1] - 1) / kTile;
+    if (g >= 0) tiles_of(indptr, g, edges, &from, &last);
   }
   const bool wide = g >= 0 && last - t > kCarryAlone;
   if (g >= 0 && !wide) {
@@ -543,10 +584,10 @@ carry_kernel(const int64_t* __restrict__ indptr, const IdT* __restrict__ nmap, i
   while (todo) {
     const int l = __ffsll(static_cast<long long>(todo)) - 1;
     todo &= todo - 1;
-    const int64_t from = __shfl(t, l, kWave) + 1;
+    const int64_t next = __shfl(t, l, kWave) + 1;
     const int64_t to = __shfl(last, l, kWave);
     float part = 0.0f;
-    for (int64_t k = from + lane; k <= to; k += kWave) part += tl.carry[2 * k];
+    for (int64_t k = next + lane; k <= to; k += kWave) part += tl.carry[2 * k];
 #pragma unroll
     for (int d = kWave / 2; d > 0; d >>= 1) part += __shfl_xor(part, d, kWave);
     if (lane == l) sums[nmap ? static_cast<int64_t>(nmap[g]) : g] = tl.carry[2 * t + 1] + part;
@@ -589,13 +630,13 @@ void launch_heads(const int64_t* indptr, const IdT* nmap, int64_t num_seg, int64
   const dim3 grid(blocks_for(num_seg, kThreads));
   if (!tl.mark) {
     hipLaunchKernelGGL((tile_heads_kernel<SUM, false, IdT>), grid, dim3(kThreads), 0, st, indptr,
-                       nmap, num_seg, out, tl);
+                       nmap, num_seg, nnz, out, tl);
     return;
   }
   hipLaunchKernelGGL(clear_marks_kernel, dim3(blocks_for(nnz, kTile)), dim3(kThreads), 0, st, tl.mark,
                      nnz);
   hipLaunchKernelGGL((tile_heads_kernel<SUM, true, IdT>), grid, dim3(kThreads), 0, st, indptr, nmap,
-                     num_seg, out, tl);
+                     num_seg, nnz, out, tl);
 }
 
 template <typename IdT>

@@ -618,15 +618,17 @@ int gs_sddmm_csc(int op, const int64_t* indptr, const void* indices, int id_byte
 /* (src/cuda/fusion/edge_map_reduce.cu:10).  Node ids (n_ids, target, row, col) */
 /* are id_bytes wide; e_ids are positions, always int64.                        */
 /* ------------------------------------------------------------------------- */
-/* workspace of gs_segment_sum / gs_segment_normalize; nnz = indptr[num_segments] */
+/* workspace of gs_segment_sum / gs_segment_normalize, with the nnz of the call */
 size_t gs_segment_workspace_bytes(int64_t num_segments, int64_t nnz);
 
 /* out[n_ids ? n_ids[s] : s] = sum over segment s of data[e_ids ? e_ids[e] : e]^powk.
  * Replaces impl::CSCSumCUDA (src/cuda/graph_ops.cu:92).  nnz: number of edges the offsets
- * cover (an upper bound will do).  A segment of at most 16 edges is summed in edge order; a
- * longer one by 1024-edge chunks of the edge array, four edges per lane, pieces across chunk
- * borders added in chunk order: a fixed order that depends on the layout only, but not the
- * sequential one. */
+ * cover, indptr[num_segments] - indptr[0] (an upper bound will do).  The first offset may lie
+ * anywhere (a range of a larger matrix's columns), and nothing outside [indptr[0],
+ * indptr[num_segments]) of data or e_ids is read.  A segment of at most 16 edges is summed in
+ * edge order.  A longer one is added up by 16 lanes (17 to 128 edges) or by a wave inside each
+ * tile of 4096 edges, counted from the first offset, and the tiles' pieces then: a fixed order
+ * that depends on the layout only, but not the sequential one. */
 int gs_segment_sum(const int64_t* indptr, const int64_t* e_ids, const void* n_ids, int id_bytes,
                    const float* data, int64_t num_segments, int64_t nnz, int64_t powk, float* out,
                    void* workspace, size_t workspace_bytes, void* stream);
@@ -648,7 +650,8 @@ int gs_coo_sum_binned(const void* target, int id_bytes, const int64_t* e_ids, co
                       int64_t E, int64_t powk, int64_t num_targets, float* out, void* workspace,
                       size_t workspace_bytes, void* stream);
 
-/* out[d] = data[d] / sum of its segment, d = e_ids ? e_ids[e] : e */
+/* out[d] = data[d] / sum of its segment, d = e_ids ? e_ids[e] : e; edges outside the offsets are
+ * left alone.  nnz as in gs_segment_sum. */
 int gs_segment_normalize(const int64_t* indptr, const int64_t* e_ids, const float* data,
                          int64_t num_segments, int64_t nnz, float* out, void* workspace,
                          size_t workspace_bytes, void* stream);

@@ -1,6 +1,8 @@
 """Segment sums and normalisation by 4096-edge tiles against the oracle: segments around the
 lengths a lane, sixteen lanes and a wave add up, on both sides of tile borders, with and
 without an edge map, with runs of empty segments between."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -69,3 +71,53 @@ def test_sum_and_normalise(dev, kind, total, emap):
     want = np.empty(nnz)
     want[order] = w / total_of[owner]
     np.testing.assert_allclose(out.cpu().numpy(), want, rtol=RTOL)
+
+
+@pytest.mark.parametrize("emap", [False, True])
+@pytest.mark.parametrize("kind,total", [("lane", 200), ("mixed", 150_000), ("border", 2_300_000),
+                                        ("hub", 150_000), ("gaps", 150_000)])  # (gaps: by marks)
+@pytest.mark.parametrize("front", [1, 4096, 10_003])
+@pytest.mark.parametrize("count", ["edges", "array"])
+def test_first_offset_not_zero(dev, count, front, kind, total, emap):
+    """A range of a larger matrix's columns: the offsets start at `front`, the data (and the edge
+    map) go on behind the last one or end there, and the caller's count is the range's own or the
+    array's.  Edges outside are neither summed nor divided."""
+    indptr = _segments(kind, total)
+    edges, nseg = int(indptr[-1]), indptr.size - 1
+    behind = 0 if count == "edges" else 5000
+    held = front + edges + behind
+    rng = np.random.default_rng(edges)
+    data = (rng.random(held) + 0.25).astype(np.float32)
+    order = rng.permutation(held) if emap else np.arange(held)
+    w = data[order[front:front + edges]].astype(np.float64)
+    owner = np.repeat(np.arange(nseg), np.diff(indptr))
+    ptr, d = to_dev(indptr + front, dev), to_dev(data, dev)
+    em = to_dev(order, dev) if emap else None
+    nnz = edges if count == "edges" else held
+    L, st = capi.lib(), capi._stream(dev)
+    ws = capi.workspace(L.gs_segment_workspace_bytes(capi._i64(nseg), capi._i64(nnz)), dev)
+
+    out = torch.full((nseg,), -1.0, device=dev)
+    capi._check(L.gs_segment_sum(capi._ptr(ptr), capi._ptr(em), capi._ptr(None), 8, capi._ptr(d),
+                                 capi._i64(nseg), capi._i64(nnz), capi._i64(2), capi._ptr(out),
+                                 capi._ptr(ws), ctypes.c_size_t(ws.numel()), st), "sum")
+    np.testing.assert_allclose(out.cpu().numpy(), np.bincount(owner, weights=w * w, minlength=nseg),
+                               rtol=RTOL)
+    out = torch.full((held,), -1.0, device=dev)
+    capi._check(L.gs_segment_normalize(capi._ptr(ptr), capi._ptr(em), capi._ptr(d), capi._i64(nseg),
+                                       capi._i64(nnz), capi._ptr(out), capi._ptr(ws),
+                                       ctypes.c_size_t(ws.numel()), st), "normalise")
+    want = np.full(held, -1.0)
+    want[order[front:front + edges]] = w / np.bincount(owner, weights=w, minlength=nseg)[owner]
+    np.testing.assert_allclose(out.cpu().numpy(), want, rtol=RTOL)
+
+
+def test_all_empty_behind_a_first_offset(dev):
+    ptr = torch.full((6,), 4096, dtype=torch.int64, device=dev)
+    data = torch.rand(9000, device=dev)
+    out = torch.full((5,), -1.0, device=dev)
+    capi.segment_sum(ptr, None, None, data, 1, out)
+    assert torch.equal(out, torch.zeros(5, device=dev))
+    out = torch.full((9000,), -1.0, device=dev)
+    capi.segment_normalize(ptr, None, data, out)
+    assert torch.equal(out, torch.full((9000,), -1.0, device=dev))
