@@ -37,11 +37,10 @@ namespace gs {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kWaves = kThreads / kWave;
 constexpr int64_t kLaneMaxLen = 16;
 
 constexpr int kLaneEdges = 4;        // of one 16-byte read
-constexpr int kTileItems = 16;
+constexpr int kTileItems = 16;          // of a thread in the passes before and behind the tiles
 constexpr int kTile = kThreads * kTileItems;
 constexpr int kGroup = 16;              // lanes that add up a segment of 17 .. kGroupMaxLen edges
 constexpr int kGroupMaxLen = 128;
@@ -147,18 +146,22 @@ enum Source {
 };
 
 // One tile.  Once the data are in LDS (the first barrier) the waves go their own ways: each takes
-// a quarter of the segments that start in the tile (with marks: those that start in its quarter
+// an equal share of the segments that start in the tile (with marks: those that start in its share
 // of the edges), the first one the incoming segment as well, 64 at a time -- the short ones a
 // lane each, what is longer from a list in LDS of the wave's own, four at a time or one by one.
 // With lists and flags shared by the workgroup and a barrier after every step a tile took 12 us
 // where it takes 7, which is what held the chip back; with the segments dealt out by
 // quarters of the edges, one tile of 16 k segments kept a wave busy for 80 us at the end.
-template <bool NORMALIZE, Source SOURCE, Walk WALK, typename IdT>
-__global__ void __launch_bounds__(kThreads, WALK == kMarks || SOURCE == kMapped ? 4 : 8)
+// Its 64 segments after 64 are a wave's serial chain, the longest where columns are many and short
+// (a tile of 16 k of them, most empty), so how many waves share a tile goes by what there is
+// to wait for it (tile_threads).
+template <bool NORMALIZE, Source SOURCE, Walk WALK, int THREADS, typename IdT>
+__global__ void __launch_bounds__(THREADS, WALK == kMarks || SOURCE == kMapped ? 4 : 8)
 segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restrict__ emap,
                      const IdT* __restrict__ nmap, const float* __restrict__ data,
                      int64_t num_seg, int64_t nnz, int powk, float* __restrict__ out, Tiles tl) {
   constexpr bool EMAP = SOURCE == kMapped;
+  constexpr int kWaves = THREADS / kWave, kItems = kTile / THREADS;
   __shared__ __attribute__((aligned(16))) float s_v[kTile];
   __shared__ uint32_t s_list[kWaves][kWave];
   __shared__ int64_t s_head[2];
@@ -182,34 +185,34 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
   const int n = edges.in_tile(p0);
   const int64_t p1 = p0 + n;
   const bool vec = SOURCE == kPlain && n == kTile && (reinterpret_cast<uintptr_t>(data + p0) & 15u) == 0;
-  F4 q[kTileItems / kLaneEdges];
+  F4 q[kItems / kLaneEdges];
   if (vec) {
 #pragma unroll
-    for (int k = 0; k < kTileItems / kLaneEdges; ++k)
-      q[k] = *reinterpret_cast<const F4*>(data + p0 + (k * kThreads + tid) * kLaneEdges);
+    for (int k = 0; k < kItems / kLaneEdges; ++k)
+      q[k] = *reinterpret_cast<const F4*>(data + p0 + (k * THREADS + tid) * kLaneEdges);
   } else if constexpr (SOURCE == kPlain) {  // (the last tile, or a first offset that is no multiple of 4)
 #pragma unroll
-    for (int k = 0; k < kTileItems / kLaneEdges; ++k)
+    for (int k = 0; k < kItems / kLaneEdges; ++k)
 #pragma unroll
       for (int u = 0; u < kLaneEdges; ++u) {
-        const int i = (k * kThreads + tid) * kLaneEdges + u;
+        const int i = (k * THREADS + tid) * kLaneEdges + u;
         q[k][u] = data[p0 + (i < n ? i : n - 1)];
       }
   }
 
-  int64_t where[EMAP ? kTileItems : 1];
-  float x[kTileItems];
+  int64_t where[EMAP ? kItems : 1];
+  float x[kItems];
   if constexpr (SOURCE != kPlain) {
     if constexpr (EMAP) {
 #pragma unroll
-      for (int k = 0; k < kTileItems; ++k) {
-        const int i = k * kThreads + tid;
+      for (int k = 0; k < kItems; ++k) {
+        const int i = k * THREADS + tid;
         where[k] = emap[p0 + (i < n ? i : n - 1)];
       }
     }
 #pragma unroll
-    for (int k = 0; k < kTileItems; ++k) {
-      const int i = k * kThreads + tid;
+    for (int k = 0; k < kItems; ++k) {
+      const int i = k * THREADS + tid;
       x[k] = data[EMAP ? where[EMAP ? k : 0] : p0 + (i < n ? i : n - 1)];
     }
   }
@@ -245,28 +248,28 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
   }
   // x^powk of a thread's edges, one loop for all of them (the products are powk_f's)
   if constexpr (SOURCE == kPlain) {
-    F4 p[kTileItems / kLaneEdges];
+    F4 p[kItems / kLaneEdges];
 #pragma unroll
-    for (int k = 0; k < kTileItems / kLaneEdges; ++k) p[k] = q[k];
+    for (int k = 0; k < kItems / kLaneEdges; ++k) p[k] = q[k];
     if (!NORMALIZE)
       for (int i = 1; i < powk; ++i) {
 #pragma unroll
-        for (int k = 0; k < kTileItems / kLaneEdges; ++k) p[k] *= q[k];
+        for (int k = 0; k < kItems / kLaneEdges; ++k) p[k] *= q[k];
       }
 #pragma unroll
-    for (int k = 0; k < kTileItems / kLaneEdges; ++k)
-      *reinterpret_cast<F4*>(s_v + (k * kThreads + tid) * kLaneEdges) = p[k];
+    for (int k = 0; k < kItems / kLaneEdges; ++k)
+      *reinterpret_cast<F4*>(s_v + (k * THREADS + tid) * kLaneEdges) = p[k];
   } else {
-    float p[kTileItems];
+    float p[kItems];
 #pragma unroll
-    for (int k = 0; k < kTileItems; ++k) p[k] = x[k];
+    for (int k = 0; k < kItems; ++k) p[k] = x[k];
     if (!NORMALIZE)
       for (int i = 1; i < powk; ++i) {
 #pragma unroll
-        for (int k = 0; k < kTileItems; ++k) p[k] *= x[k];
+        for (int k = 0; k < kItems; ++k) p[k] *= x[k];
       }
 #pragma unroll
-    for (int k = 0; k < kTileItems; ++k) s_v[k * kThreads + tid] = p[k];
+    for (int k = 0; k < kItems; ++k) s_v[k * THREADS + tid] = p[k];
   }
   __syncthreads();
 
@@ -388,14 +391,14 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
     }
   };
 
-  constexpr int kQuarter = kTile / kWaves;
-  const int64_t q0 = p0 + wave * kQuarter;
+  constexpr int kShare = kTile / kWaves;
+  const int64_t q0 = p0 + wave * kShare;
   if (WALK == kMarks ? q0 < p1 : seg0 < seg1) {
     if (WALK == kMarks) {
-      int seg[kQuarter / kWave];
-      int64_t end[kQuarter / kWave];
+      int seg[kShare / kWave];
+      int64_t end[kShare / kWave];
 #pragma unroll
-      for (int k = 0; k < kQuarter / kWave; ++k) {
+      for (int k = 0; k < kShare / kWave; ++k) {
         const int64_t p = q0 + k * kWave + lane;
         seg[k] = p < p1 ? tl.mark[p - edges.first] : -1;
       }
@@ -407,13 +410,13 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
         if (incoming) seg[0] = static_cast<int>(head);
       }
 #pragma unroll
-      for (int k = 0; k < kQuarter / kWave; ++k) end[k] = indptr[seg[k] >= 0 ? seg[k] + 1 : 0];
+      for (int k = 0; k < kShare / kWave; ++k) end[k] = indptr[seg[k] >= 0 ? seg[k] + 1 : 0];
 #pragma unroll 1
-      for (int k = 0; k < kQuarter / kWave; ++k) {
+      for (int k = 0; k < kShare / kWave; ++k) {
         int s = seg[0];
         int64_t e = end[0];
 #pragma unroll
-        for (int u = 1; u < kQuarter / kWave; ++u)
+        for (int u = 1; u < kShare / kWave; ++u)
           if (u == k) s = seg[u], e = end[u];
         if (__ballot(s >= 0) == 0ull) continue;
         round(0, s, k == 0 && incoming ? begin_in : q0 + k * kWave + lane, e);
@@ -457,14 +460,14 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
     if (tid == 0) tl.inner[t] = first | stop << 16;
     if constexpr (EMAP) {
 #pragma unroll
-      for (int k = 0; k < kTileItems; ++k) {
-        const int i = k * kThreads + tid;
+      for (int k = 0; k < kItems; ++k) {
+        const int i = k * THREADS + tid;
         if (i >= first && i < stop) out[where[k]] = s_v[i];
       }
     } else if (vec && (reinterpret_cast<uintptr_t>(out + p0) & 15u) == 0) {
 #pragma unroll
-      for (int k = 0; k < kTileItems / kLaneEdges; ++k) {
-        const int i = (k * kThreads + tid) * kLaneEdges;
+      for (int k = 0; k < kItems / kLaneEdges; ++k) {
+        const int i = (k * THREADS + tid) * kLaneEdges;
         const float4 v = *reinterpret_cast<const float4*>(s_v + i);
         if (i >= first && i + 3 < stop) {
           *reinterpret_cast<float4*>(out + p0 + i) = v;
@@ -477,8 +480,8 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
       }
     } else {
 #pragma unroll
-      for (int k = 0; k < kTileItems; ++k) {
-        const int i = k * kThreads + tid;
+      for (int k = 0; k < kItems; ++k) {
+        const int i = k * THREADS + tid;
         if (i >= first && i < stop) out[p0 + i] = s_v[i];
       }
     }
@@ -623,6 +626,25 @@ size_t segment_workspace_bytes(int64_t num_seg, int64_t nnz) {
          (use_marks(num_seg, nnz) ? padded(static_cast<size_t>(nnz > 0 ? nnz : 1) * 4) : 0);
 }
 
+// Threads of a tile's workgroup.  A launch of few tiles ends with its longest one, and more waves
+// shorten that; one of many tiles is held up by every wave's share of the common steps.  In us,
+// sum / normalise of R-MAT graphs, by 256, 512 and 1024 threads:
+//   262 k edges, 33 k columns    23 / 40    17 / 25    16 / 21
+//   1.0 M edges, 131 k columns   34 / 54    22 / 33    17 / 25
+//   8 M edges, 1 M columns       60 / 94    38 / 62    32 / 48
+//   8 M edges, 250 k columns     27 / 47    21 / 35    28 / 48
+//   12 M edges, 1.5 M columns    71 / 99    46 / 64    45 / 76
+//   20 M edges, 1.2 M columns    52 / 78    42 / 70    60 / 107
+//   40 M edges, 2.45 M columns   78 / 117   71 / 135  104 / 208
+// 256 alone fell behind a lane per short column and passes of their own for the long ones where
+// columns have few edges (8 M edges, 1 M columns: 43 / 56).
+enum Width { kWidest = 1024, kMiddle = 512, kNarrow = 256 };
+inline Width tile_threads(int64_t num_seg, int64_t nnz) {
+  const int64_t tiles = num_tiles(nnz);
+  if (tiles <= kSearchTiles || (tiles <= 2048 && 16 * num_seg > nnz)) return kWidest;
+  return tiles <= 6144 || use_marks(num_seg, nnz) ? kMiddle : kNarrow;
+}
+
 // what the tiles' workgroups find in head[] and mark[]
 template <bool SUM, typename IdT>
 void launch_heads(const int64_t* indptr, const IdT* nmap, int64_t num_seg, int64_t nnz, float* out,
@@ -646,18 +668,22 @@ int segment_sum_impl(const int64_t* indptr, const int64_t* emap, const void* nma
   const IdT* nm = static_cast<const IdT*>(nmap);
   const int64_t tiles = num_tiles(nnz);
   launch_heads<true>(indptr, nm, num_seg, nnz, out, tl, st);
-  auto pick = [&](auto walk) {
-    constexpr Walk W = decltype(walk)::value;
-    switch (source_of(emap, data)) {
-      case kMapped: return segment_tiles_kernel<false, kMapped, W, IdT>;
-      case kLoose: return segment_tiles_kernel<false, kLoose, W, IdT>;
-      default: return segment_tiles_kernel<false, kPlain, W, IdT>;
-    }
+  const Width width = tile_threads(num_seg, nnz);
+  auto pick = [&](auto source) {
+    constexpr Source S = decltype(source)::value;
+    if (tl.mark)
+      return width == kWidest ? segment_tiles_kernel<false, S, kMarks, kWidest, IdT>
+                              : segment_tiles_kernel<false, S, kMarks, kMiddle, IdT>;
+    return width == kWidest   ? segment_tiles_kernel<false, S, kHeads, kWidest, IdT>
+           : width == kMiddle ? segment_tiles_kernel<false, S, kHeads, kMiddle, IdT>
+                              : segment_tiles_kernel<false, S, kHeads, kNarrow, IdT>;
   };
-  auto* kernel = tl.mark ? pick(std::integral_constant<Walk, kMarks>{})
-                         : pick(std::integral_constant<Walk, kHeads>{});
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(kThreads), 0, st, indptr, emap,
-                     nm, data, num_seg, nnz, powk, out, tl);
+  const Source source = source_of(emap, data);
+  auto* kernel = source == kMapped  ? pick(std::integral_constant<Source, kMapped>{})
+                 : source == kLoose ? pick(std::integral_constant<Source, kLoose>{})
+                                    : pick(std::integral_constant<Source, kPlain>{});
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(width), 0, st, indptr, emap, nm,
+                     data, num_seg, nnz, powk, out, tl);
   if (tiles > 1)
     hipLaunchKernelGGL((carry_kernel<IdT>), dim3(blocks_for(tiles, kThreads)), dim3(kThreads), 0, st,
                        indptr, nm, num_seg, nnz, out, tl);
@@ -669,10 +695,15 @@ void launch_normalize(Walk walk, const int64_t* indptr, const int64_t* emap, con
                       int64_t num_seg, int64_t nnz, float* out, const Tiles& tl, hipStream_t st) {
   const int64_t* no_map = nullptr;
   const int64_t tiles = num_tiles(nnz);
-  auto* kernel = walk == kSearch   ? segment_tiles_kernel<true, SOURCE, kSearch, int64_t>
-                 : walk == kHeads ? segment_tiles_kernel<true, SOURCE, kHeads, int64_t>
-                                  : segment_tiles_kernel<true, SOURCE, kMarks, int64_t>;
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(kThreads), 0, st, indptr, emap,
+  const Width width = tile_threads(num_seg, nnz);
+  auto* kernel = walk == kSearch ? segment_tiles_kernel<true, SOURCE, kSearch, kWidest, int64_t>
+                 : walk == kMarks
+                     ? (width == kWidest ? segment_tiles_kernel<true, SOURCE, kMarks, kWidest, int64_t>
+                                         : segment_tiles_kernel<true, SOURCE, kMarks, kMiddle, int64_t>)
+                 : width == kWidest ? segment_tiles_kernel<true, SOURCE, kHeads, kWidest, int64_t>
+                 : width == kMiddle ? segment_tiles_kernel<true, SOURCE, kHeads, kMiddle, int64_t>
+                                    : segment_tiles_kernel<true, SOURCE, kHeads, kNarrow, int64_t>;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(width), 0, st, indptr, emap,
                      no_map, data, num_seg, nnz, 1, out, tl);
   if (tiles > 1)
     hipLaunchKernelGGL((crossing_divide_kernel<SOURCE == kMapped>),

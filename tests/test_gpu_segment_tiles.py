@@ -24,6 +24,8 @@ LENGTHS = {
     "hub": [70_001, 2, 300_000, 16, 40],
     "gaps": [0] * 700 + [20] * 60 + [0] * 300 + [5000, 16, 16],
     "mixed": [0, 1, 2, 5, 9, 16, 17, 40, 129, 500, 3000],
+    "sparse": [0, 0, 0, 1, 2, 0],
+    "low": [0, 2, 7, 30],
 }
 
 
@@ -45,6 +47,19 @@ def _segments(kind, total):
 @pytest.mark.parametrize("kind", sorted(LENGTHS))
 @pytest.mark.parametrize("total", [1, 4096, 150_000, 2_300_000])
 def test_sum_and_normalise(dev, kind, total, emap):
+    _check(dev, kind, total, emap)
+
+
+@pytest.mark.parametrize("kind,total", [("sparse", 8_500_000),           # marks, the middle width
+                                        ("low", 8_380_000),              # widest and middle on both
+                                        ("low", 8_400_000),              # sides of 2048 tiles
+                                        ("mixed", 25_160_000),           # middle and narrow on both
+                                        ("mixed", 25_200_000)])          # sides of 6144
+def test_widths_of_a_tiles_workgroup(dev, kind, total):
+    _check(dev, kind, total, False)
+
+
+def _check(dev, kind, total, emap):
     indptr = _segments(kind, total)
     nnz, nseg = int(indptr[-1]), indptr.size - 1
     rng = np.random.default_rng(nnz)
