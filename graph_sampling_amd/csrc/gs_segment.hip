@@ -488,15 +488,76 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
   }
 }
 
+// Sum of the pieces of a long segment behind its first tile, by a whole workgroup; in every thread.
+// s_part: a float per wave.
+__device__ __forceinline__ float sum_pieces(const Tiles& tl, int64_t from, int64_t to, float* s_part) {
+  constexpr int kEach = 8;  // reads of a thread in flight
+  float part = 0.0f;
+  for (int64_t k0 = from + 1 + threadIdx.x; k0 <= to; k0 += kEach * kThreads) {
+    float v[kEach];
+#pragma unroll
+    for (int u = 0; u < kEach; ++u) v[u] = tl.carry[2 * (k0 + u * kThreads <= to ? k0 + u * kThreads : to)];
+#pragma unroll
+    for (int u = 0; u < kEach; ++u)
+      if (k0 + u * kThreads <= to) part += v[u];
+  }
+#pragma unroll
+  for (int d = kWave / 2; d > 0; d >>= 1) part += __shfl_xor(part, d, kWave);
+  if ((threadIdx.x & (kWave - 1)) == 0) s_part[threadIdx.x / kWave] = part;
+  __syncthreads();
+  float total = 0.0f;
+#pragma unroll
+  for (int w = 0; w < kThreads / kWave; ++w) total += s_part[w];
+  __syncthreads();
+  return total;
+}
+
+// Normalise, launches of more than kHubLaunch tiles: the sum of a segment of more than kHubTiles of
+// them goes to its outgoing piece's place once, where otherwise each of its tiles adds up all the
+// pieces for itself, a square of reads (one segment of 130 M edges: 691 us with it, of 140 M 342
+// without).  The launch costs a graph without such a segment 7 us, 264 -> 269 for 124 M edges,
+// hence not for fewer tiles.  One segment of so many at most starts in a workgroup's tiles.
+constexpr int64_t kHubTiles = 1024;
+constexpr int64_t kHubLaunch = 32768;
+
+__global__ void __launch_bounds__(kThreads)
+hub_totals_kernel(const int64_t* __restrict__ indptr, int64_t num_seg, int64_t nnz, Tiles tl) {
+  __shared__ int64_t s_from, s_to;
+  __shared__ float s_part[kThreads / kWave];
+  const Edges edges(indptr, num_seg, nnz);
+  if (threadIdx.x == 0) s_to = -1;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kHubTiles / kThreads; ++k) {
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * kHubTiles + k * kThreads + threadIdx.x;
+    const int g = edges.first + t * kTile < edges.end ? tl.outgoing[t] : -1;
+    if (g < 0) continue;
+    int64_t from, to;
+    tiles_of(indptr, g, edges, &from, &to);
+    if (to - from > kHubTiles) {
+      s_from = from;
+      s_to = to;
+    }
+  }
+  __syncthreads();
+  if (s_to < 0) return;
+  const float total = sum_pieces(tl, s_from, s_to, s_part);
+  if (threadIdx.x == 0) tl.carry[2 * s_from + 1] += total;
+}
+
 // The edges of segments that cross tile borders: what lies in front of a tile's inner edges
 // belongs to the incoming segment, what lies behind to the outgoing one.  Each workgroup adds
-// up the pieces of its two segments for itself.
+// up the pieces of its two segments for itself, a wave each or, of segments over more than 64
+// tiles, the whole workgroup (one segment of 32 M edges: 191 -> 85 us, of 100 M 1321 -> 458);
+// `hubs`: the totals of those over more than kHubTiles are there.
 template <bool EMAP>
 __global__ void __launch_bounds__(kThreads)
 crossing_divide_kernel(const int64_t* __restrict__ indptr, const int64_t* __restrict__ emap,
                        const float* __restrict__ data, int64_t num_seg, int64_t nnz,
-                       float* __restrict__ out, Tiles tl) {
+                       float* __restrict__ out, Tiles tl, bool hubs) {
   __shared__ float s_total[2];
+  __shared__ int64_t s_tiles[2][2];
+  __shared__ float s_part[kThreads / kWave];
   const int64_t t = blockIdx.x;
   const Edges edges(indptr, num_seg, nnz);
   const int64_t p0 = edges.first + t * kTile;
@@ -521,17 +582,29 @@ crossing_divide_kernel(const int64_t* __restrict__ indptr, const int64_t* __rest
   }
   if (wave < 2) {
     const int g = wave == 0 ? (first > 0 ? g_in : -1) : g_out;
+    int64_t from = 0, to = 0;
     if (g >= 0) {
-      int64_t from, to;
       tiles_of(indptr, g, edges, &from, &to);
-      float part = 0.0f;
-      for (int64_t k = from + 1 + lane; k <= to; k += kWave) part += tl.carry[2 * k];
+      if (to - from <= kWave) {
+        float part = from + 1 + lane <= to ? tl.carry[2 * (from + 1 + lane)] : 0.0f;
 #pragma unroll
-      for (int d = kWave / 2; d > 0; d >>= 1) part += __shfl_xor(part, d, kWave);
-      if (lane == 0) s_total[wave] = tl.carry[2 * from + 1] + part;
+        for (int d = kWave / 2; d > 0; d >>= 1) part += __shfl_xor(part, d, kWave);
+        if (lane == 0) s_total[wave] = tl.carry[2 * from + 1] + part;
+      }
+    }
+    if (lane == 0) {
+      s_tiles[wave][0] = from;
+      s_tiles[wave][1] = to;
     }
   }
   __syncthreads();
+  for (int r = 0; r < 2; ++r) {
+    const int64_t from = s_tiles[r][0], to = s_tiles[r][1];  // (the same for the whole workgroup)
+    if (to - from <= kWave) continue;
+    const float rest = hubs && to - from > kHubTiles ? 0.0f : sum_pieces(tl, from, to, s_part);
+    if (tid == 0) s_total[r] = tl.carry[2 * from + 1] + rest;
+    __syncthreads();
+  }
   const float before = s_total[0], behind = s_total[1];
   if (vec) {
 #pragma unroll
@@ -705,10 +778,14 @@ void launch_normalize(Walk walk, const int64_t* indptr, const int64_t* emap, con
                                     : segment_tiles_kernel<true, SOURCE, kHeads, kNarrow, int64_t>;
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(width), 0, st, indptr, emap,
                      no_map, data, num_seg, nnz, 1, out, tl);
+  const bool hubs = tiles > kHubLaunch;
+  if (hubs)
+    hipLaunchKernelGGL(hub_totals_kernel, dim3(blocks_for(tiles, kHubTiles)), dim3(kThreads), 0, st,
+                       indptr, num_seg, nnz, tl);
   if (tiles > 1)
     hipLaunchKernelGGL((crossing_divide_kernel<SOURCE == kMapped>),
                        dim3(static_cast<unsigned>(tiles)), dim3(kThreads), 0, st, indptr, emap, data,
-                       num_seg, nnz, out, tl);
+                       num_seg, nnz, out, tl, hubs);
 }
 
 int segment_normalize_impl(const int64_t* indptr, const int64_t* emap, const float* data,

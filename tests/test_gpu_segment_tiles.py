@@ -59,7 +59,25 @@ def test_widths_of_a_tiles_workgroup(dev, kind, total):
     _check(dev, kind, total, False)
 
 
-def _check(dev, kind, total, emap):
+@pytest.mark.parametrize("lens", [[3, 17, 5_000_000, 40, 300_000],            # added up tile by tile
+                                  [3, 17, 130_000_000, 5_300_000, 40, 300_000]])  # totals made first
+def test_segments_of_thousands_of_tiles(dev, lens):
+    ptr = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), device=dev)
+    data = torch.rand(int(ptr[-1]), device=dev) + 0.25
+    parts = torch.split(data.double(), lens)
+    # the pieces of the longest by the lanes of a wave, so many in a row, where RTOL counts 17
+    rtol = RTOL + max(lens) / 4096 / 64 * 2.0 ** -24
+    out = torch.empty(len(lens), device=dev)
+    capi.segment_sum(ptr, None, None, data, 1, out)
+    total = torch.stack([p.sum() for p in parts])
+    torch.testing.assert_close(out.double(), total, rtol=rtol, atol=0)
+    out = torch.empty_like(data)
+    capi.segment_normalize(ptr, None, data, out)
+    for p, t, got in zip(parts, total, torch.split(out, lens)):
+        torch.testing.assert_close(got.double(), p / t, rtol=rtol, atol=0)
+
+
+def _check(dev, kind, total, emap, rtol=RTOL):
     indptr = _segments(kind, total)
     nnz, nseg = int(indptr[-1]), indptr.size - 1
     rng = np.random.default_rng(nnz)
@@ -73,7 +91,7 @@ def _check(dev, kind, total, emap):
     out = torch.full((nseg,), -1.0, device=dev)
     capi.segment_sum(to_dev(indptr, dev), em, None, to_dev(data, dev), 2, out)
     got = out.cpu().numpy()
-    np.testing.assert_allclose(got, want, rtol=RTOL)
+    np.testing.assert_allclose(got, want, rtol=rtol)
     short = np.flatnonzero((lens <= 16) & (lens > 0))[:3000]
     for s in short:  # in edge order: the bits of a sequential sum
         acc = np.float32(0)
@@ -85,7 +103,7 @@ def _check(dev, kind, total, emap):
     total_of = np.bincount(owner, weights=w, minlength=nseg)
     want = np.empty(nnz)
     want[order] = w / total_of[owner]
-    np.testing.assert_allclose(out.cpu().numpy(), want, rtol=RTOL)
+    np.testing.assert_allclose(out.cpu().numpy(), want, rtol=rtol)
 
 
 @pytest.mark.parametrize("emap", [False, True])
