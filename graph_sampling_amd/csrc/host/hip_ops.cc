@@ -1,5 +1,6 @@
 #include "hip_ops.h"
 
+#include <ATen/TensorSubclassLikeUtils.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
@@ -455,6 +456,11 @@ bool EdgeData::Fits(const torch::Tensor& data, const torch::optional<torch::Tens
       return false;
   }
   return true;
+}
+
+bool EdgeData::Followed(const torch::Tensor& data) {
+  return (at::GradMode::is_enabled() && data.requires_grad()) || data._fw_grad(0).defined() ||
+         at::isTensorSubclassLike(data);
 }
 
 // One launch, no host read: the total is posted to a mailbox and collected by Wait().

@@ -66,6 +66,9 @@ struct EdgeData {
   torch::optional<torch::Tensor> e_ids;  // the CSC's edge-id map, when it has one
   // whether the sampler kernels can read it: one contiguous fp32 value per edge on the device
   static bool Fits(const torch::Tensor& data, const torch::optional<torch::Tensor>& e_ids);
+  // whether somebody follows what becomes of it -- a gradient, a forward-mode tangent, a transform
+  // -- whom a kernel that reads it from its address would pass by
+  static bool Followed(const torch::Tensor& data);
 };
 
 // A one-launch sample whose total the host has not read yet.  The buffers have

@@ -70,3 +70,42 @@ def test_columns_per_tile(dev, hubs, hub_degree, small, n):
     want = O.col_row_slice(indptr, indices, cols, rows)
     assert np.array_equal(np.delete(ptr.cpu().numpy(), at), want[0])
     assert np.array_equal(idx.cpu().numpy(), want[1])
+
+
+@pytest.mark.parametrize("coo", [False, True])        # (from an edge list: data by edge id)
+@pytest.mark.parametrize("hub_degree", [20, 90_001])  # the general slice, and the set in LDS
+def test_data_that_is_followed(dev, hub_degree, coo):
+    """Edge data that require a gradient, or carry a forward-mode tangent, keep it in the subgraph,
+    whichever way the slice goes."""
+    n = 3000
+    indptr, indices, rng = _graph(n, 20, hub_degree, 30, 5)
+    indices[:n] = rng.permutation(n)  # every node is there
+    order = np.arange(indices.size)
+    if coo:  # the edges in another order; inside a column they come as in the list
+        shuffle = rng.permutation(indices.size)
+        col, row = np.repeat(np.arange(n), np.diff(indptr))[shuffle], indices[shuffle]
+        order = np.argsort(col, kind="stable")
+        indices = row[order]
+    cols, rows = rng.permutation(n).astype(np.int64), rng.permutation(n)[:900].astype(np.int64)
+    at = torch.from_numpy(order[O.col_row_slice(indptr, indices, cols, rows)[3]]).to(dev)
+    w = torch.rand(indices.size, device=dev)
+
+    def cut(data):
+        g = gs.Graph(False)
+        if coo:
+            g._CAPI_LoadCOO(to_dev(row, dev), to_dev(col, dev))
+        else:
+            g._CAPI_LoadCSC(to_dev(indptr, dev), to_dev(indices, dev))
+        g._CAPI_SetData(data)
+        return g._CAPI_FusionSlicing(to_dev(cols, dev), to_dev(rows, dev))._CAPI_GetData("default")
+
+    r = torch.rand(at.numel(), device=dev)
+    x = w.clone().requires_grad_(True)
+    (cut(x) * r).sum().backward()
+    assert torch.equal(x.grad, torch.zeros_like(w).index_put_((at,), r))
+    with torch.no_grad():
+        assert torch.equal(cut(x), w[at])
+    t = torch.rand_like(w)
+    with torch.autograd.forward_ad.dual_level():
+        got = torch.autograd.forward_ad.unpack_dual(cut(torch.autograd.forward_ad.make_dual(w, t)))
+        assert torch.equal(got.primal, w[at]) and torch.equal(got.tangent, t[at])
