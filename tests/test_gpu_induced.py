@@ -109,3 +109,19 @@ def test_data_that_is_followed(dev, hub_degree, coo):
     with torch.autograd.forward_ad.dual_level():
         got = torch.autograd.forward_ad.unpack_dual(cut(torch.autograd.forward_ad.make_dual(w, t)))
         assert torch.equal(got.primal, w[at]) and torch.equal(got.tangent, t[at])
+
+
+def test_data_of_the_first_edges_only(dev):
+    """Data that end before the edges do serve a subgraph whose kept edges all have theirs."""
+    indptr = np.array([0, 1_200_000, 2_400_000], dtype=np.int64)
+    indices = np.zeros(2_400_000, dtype=np.int64)
+    indices[::3] = 1
+    indices[2_000_000:] = 7  # no node of the subgraph
+    g = gs.Graph(False)
+    g._CAPI_LoadCSC(to_dev(indptr, dev), to_dev(indices, dev))
+    w = torch.rand(2_000_000, device=dev)
+    g._CAPI_SetData(w)
+    ids = torch.tensor([0, 1], device=dev)
+    sub = g._CAPI_FusionSlicing(ids, ids)
+    assert torch.equal(sub._CAPI_GetData("default"), w)
+    assert np.array_equal(sub._CAPI_GetCSC()[1].cpu().numpy(), indices[:2_000_000])
