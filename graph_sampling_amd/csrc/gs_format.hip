@@ -249,11 +249,7 @@ __device__ __forceinline__ int64_t wave_first_not_below(const Keys& key, int64_t
 // searches the whole key array once per column).  A workgroup owns 256 consecutive
 // columns: two wave-wide searches bound the keys that belong to them, and the per-column
 // searches run inside that range -- in LDS when it holds at most 4096 keys, which is every
-// tile but those of hub columns.  A boundary-driven fill (every edge writes the offsets of
-// the columns between it and its predecessor) was tried first and is worse at both ends:
-// with few edges and millions of columns one lane fills a gap of a million offsets by
-// itself, with many edges and few columns it reads every key to find a handful of
-// boundaries.
+// tile but those of hub columns.
 constexpr int kPtrCols = kThreads;
 constexpr int kPtrStage = 4096;
 
@@ -291,13 +287,20 @@ indptr_from_sorted_kernel(Keys key, int64_t E, int64_t num_keys, int64_t* __rest
   }
 }
 
-// The same offsets from the places where the keys change, for more edges than columns: item i
-// of [0, E] (key E is the number of columns) writes offset i for the columns after key i - 1
-// up to key i.  Every key is read once, coalesced, where the searches above cost a workgroup
-// five dependent trips before it starts: 14 M keys, 2.45 M columns 75 -> 22 us.  Gaps longer
-// than kGapAlone columns are set aside and filled by whole waves, so that a run of absent
-// ids does not become one lane's loop; with fewer edges than columns (a slice's rows among
-// all rows) nearly every item would be such a gap and the searches are the better split.
+// The same offsets from the places where the keys change: item i of [0, E] (key E is the number of
+// columns) writes offset i for the columns after key i - 1 up to key i.  Every key is read once,
+// coalesced, where the searches above cost a workgroup five dependent trips before it starts.
+// Gaps longer than kGapAlone columns are set aside and filled by whole waves, so that a run of
+// absent ids does not become one lane's loop; with fewer edges than columns (a slice's rows among
+// all rows) nearly every item would be such a gap and the searches are the better split.  With many
+// edges per column they are too, since the fill reads all keys and they read a few per column.
+// Fill against searches, us, 4-byte keys / 8-byte keys, by edges per column:
+//                  1          5.7         16          50         160         500
+//    1 M keys               5/6 5/6     5/6 5/6     5/6 5/5     5/6 5/5    4/6 5/5
+//   14 M keys  27/37 100/104  19/27 36/39  18/26 26/30  17/26 26/30  16/23 12/14  15/22 7/8
+//  114 M keys 262/343 1000/1029 136/212 289/322 124/206 189/229 123/207 174/207 109/187 101/108 102/188 34/36
+// (even columns; with hubs the searches gain at 50, 17/24 against 15/20 for 14 M): the line lies at
+// 64 edges per column for 4-byte keys, 32 for 8-byte ones.
 constexpr int kFillItems = 16;
 constexpr int kFillTile = kThreads * kFillItems;
 constexpr int kGapAlone = 16;
@@ -358,7 +361,7 @@ indptr_fill_kernel(const KeyT* __restrict__ key, int64_t E, int64_t num_keys,
 
 template <typename KeyT>
 void launch_indptr(const KeyT* key, int64_t E, int64_t num_keys, int64_t* indptr, hipStream_t st) {
-  if (E > 0 && num_keys <= E) {
+  if (E > 0 && num_keys <= E && E * static_cast<int64_t>(sizeof(KeyT)) <= 256 * num_keys) {
     hipLaunchKernelGGL((indptr_fill_kernel<KeyT>), dim3(blocks_for(E + 1, kFillTile)),
                        dim3(kThreads), 0, st, key, E, num_keys, indptr);
     return;

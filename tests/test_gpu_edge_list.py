@@ -99,3 +99,14 @@ def test_offsets_over_gaps(dev, keys, idt):
     ip, _, _ = capi.coo2csc(to_dev(key, dev, idt), to_dev(key, dev, idt), num_keys, True)
     want = np.concatenate([[0], np.cumsum(np.bincount(key, minlength=num_keys))])
     assert np.array_equal(ip.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("idt", ID_DTYPES)
+@pytest.mark.parametrize("E", [999, 1000, 31_999, 32_000, 32_001, 64_000, 64_001, 500_000])
+def test_offsets_by_edges_per_column(dev, E, idt):
+    """Both sides of the lines between the two ways from sorted keys to offsets."""
+    num_keys = 1000
+    key = np.sort((np.random.default_rng(E).random(E) ** 3 * num_keys).astype(np.int64))
+    ip, _, _ = capi.coo2csc(to_dev(key, dev, idt), to_dev(key, dev, idt), num_keys, True)
+    want = np.concatenate([[0], np.cumsum(np.bincount(key, minlength=num_keys))])
+    assert np.array_equal(ip.cpu().numpy(), want)
