@@ -481,6 +481,7 @@ struct SortOutputs {
 // SELF: `offsets` holds the tiles' raw counts and every workgroup adds up for itself where its
 // runs start (a sort of few tiles: two launches less per pass than scanning the counts first).
 constexpr int64_t kSelfScanTiles = 64;
+static_assert(kLargeTileItems / LargeTile::kSize > kSelfScanTiles, "large tiles never scan themselves");
 
 template <typename T, typename IdT, typename ValT, typename Src, bool LAST, bool SELF>
 __global__ void __launch_bounds__(T::kThreadsPerTile, 4)  // (16 waves a CU is what LDS allows)
@@ -710,9 +711,14 @@ void launch_pass(Src src, bool last, bool self, hipStream_t st, const ValT* vin,
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(T::kThreadsPerTile), 0, st,
                        src, vin, E, shift, blocks, where, wout, vout, outs);
   };
-  if (last && self) go(radix_pass_kernel<T, IdT, ValT, Src, true, true>);
-  else if (last) go(radix_pass_kernel<T, IdT, ValT, Src, true, false>);
-  else if (self) go(radix_pass_kernel<T, IdT, ValT, Src, false, true>);
+  if constexpr (std::is_same<T, SmallTile>::value) {  // (a sort by large tiles has 512 at least)
+    if (self) {
+      if (last) go(radix_pass_kernel<T, IdT, ValT, Src, true, true>);
+      else go(radix_pass_kernel<T, IdT, ValT, Src, false, true>);
+      return;
+    }
+  }
+  if (last) go(radix_pass_kernel<T, IdT, ValT, Src, true, false>);
   else go(radix_pass_kernel<T, IdT, ValT, Src, false, false>);
 }
 
