@@ -23,10 +23,14 @@ constexpr int kThreads = 256;
 
 // Neighbour arrays from this size on are read as streams (the line is the first to leave the
 // L2): hardly one of their lines is met again, and the offsets, which are, stay longer.
-// Arrays that the L2s and the memory-side cache hold in good part lose by it.  1 M walkers,
-// 80 steps, 800 MB: 1456 -> 1426 us; metapath over three of 400 MB: 126 -> 120; but 20 k
-// walkers over 32 MB: 41 -> 68.
+// Arrays that the L2s and the memory-side cache hold in good part lose by it.  Metapath over three
+// arrays of 400 MB, 20 steps: 200 k walkers 89 -> 85 us, 1 M walkers 411 -> 383; 1 M walkers, 80
+// steps, 800 MB: 1457 -> 1349 to 1430 from run to run; but 20 k walkers over 32 MB: 41 -> 68.
 constexpr int64_t kStreamBytes = int64_t(256) << 20;
+// A metapath's relations have to be looked up for it in front of the first step, 1.0 to 1.4 us that
+// only long work earns back: 1 M walkers, 4 steps 93 -> 92 us, 200 k walkers, 20 steps 87 -> 85,
+// but 400 k walkers, 8 steps 70 -> 71, 18 k walkers, 8 steps 12.9 -> 13.8.
+constexpr int64_t kStreamSteps = int64_t(1) << 22;
 
 // A node outside [0, num_nodes) has no neighbours (the walker dies there), so a
 // stray seed can never turn into a wild read.
@@ -76,7 +80,8 @@ random_walk_kernel(const int64_t* __restrict__ indptr, const IdT* __restrict__ i
   }
 }
 
-template <typename IdT>
+// LONG_WORK: large neighbour arrays are looked for and read as streams
+template <typename IdT, bool LONG_WORK>
 __global__ void __launch_bounds__(kThreads)
 metapath_walk_kernel(const int64_t* const* __restrict__ all_indptr,
                      const IdT* const* __restrict__ all_indices,
@@ -91,7 +96,7 @@ metapath_walk_kernel(const int64_t* const* __restrict__ all_indptr,
   U4 x;
   unsigned long long streams = 0ull;  // bit t: the relation of step t (mod 64) is read as a stream
   for (int64_t t = 0; t < length; ++t) {
-    if ((t & (kWave - 1)) == 0) {  // a lane per step of the next 64
+    if (LONG_WORK && (t & (kWave - 1)) == 0) {  // a lane per step of the next 64
       const int64_t step = t + (threadIdx.x & (kWave - 1));
       const int64_t rel = metapath[step < length ? step : length - 1];
       streams = __ballot(all_indptr[rel][all_num_nodes[rel]] >=
@@ -104,7 +109,7 @@ metapath_walk_kernel(const int64_t* const* __restrict__ all_indptr,
       const int64_t rel = metapath[t];  // uniform over the wave: scalar loads
       const uint32_t xv = replay ? replay[t * n + w] : x.v[t & 3];
       pick = step_from(all_indptr[rel], all_indices[rel], all_num_nodes[rel], curr, xv,
-                       (streams >> (t & (kWave - 1))) & 1ull);
+                       LONG_WORK && ((streams >> (t & (kWave - 1))) & 1ull));
     }
     trace[(t + 1) * n + w] = static_cast<IdT>(pick);
     curr = pick;
@@ -153,19 +158,18 @@ int gs_metapath_walk(const int64_t* const* all_indptr, const void* const* all_in
   if (n == 0) return GS_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 grid(blocks_for(n, kThreads));
+  const bool long_work = length > 0 && n >= (kStreamSteps + length - 1) / length;
   ProfileScope prof("metapath_walk", st);
+  auto go = [&](auto kernel, auto id) {
+    using IdT = decltype(id);
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, st, all_indptr,
+                       reinterpret_cast<const IdT* const*>(all_indices), all_num_nodes, metapath, length,
+                       static_cast<const IdT*>(seeds), n, seed, replay, static_cast<IdT*>(trace));
+  };
   if (id_bytes == 8)
-    hipLaunchKernelGGL((metapath_walk_kernel<int64_t>), grid, dim3(kThreads), 0, st, all_indptr,
-                       reinterpret_cast<const int64_t* const*>(all_indices), all_num_nodes, metapath,
-                       length,
-                       static_cast<const int64_t*>(seeds), n, seed, replay,
-                       static_cast<int64_t*>(trace));
+    go(long_work ? metapath_walk_kernel<int64_t, true> : metapath_walk_kernel<int64_t, false>, int64_t());
   else
-    hipLaunchKernelGGL((metapath_walk_kernel<int32_t>), grid, dim3(kThreads), 0, st, all_indptr,
-                       reinterpret_cast<const int32_t* const*>(all_indices), all_num_nodes, metapath,
-                       length,
-                       static_cast<const int32_t*>(seeds), n, seed, replay,
-                       static_cast<int32_t*>(trace));
+    go(long_work ? metapath_walk_kernel<int32_t, true> : metapath_walk_kernel<int32_t, false>, int32_t());
   return check_launch("metapath_walk");
 }
 

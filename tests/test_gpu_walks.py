@@ -147,3 +147,21 @@ def test_walks_over_neighbour_arrays_read_as_streams(dev, idt, less):
                              seed=6)
     want = O.metapath_walk([indptr, small_ptr], [big, small_ix], path, seeds, seed=6)
     assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
+
+
+@pytest.mark.parametrize("walkers", [62_601, 62_602])  # 67 steps of each: 2**22 in all, less 37 and more 30
+def test_long_metapath_work_over_streams(dev, walkers):
+    """From 2**22 steps in all, large neighbour arrays of a metapath are read as streams."""
+    E = (1 << 28) // 4
+    N = E // 64
+    rng = np.random.default_rng(walkers)
+    indptr, small_ptr = np.arange(N + 1, dtype=np.int64) * 64, np.arange(N + 1, dtype=np.int64)
+    indices, small_ix = rng.integers(0, N, E).astype(np.int32), rng.permutation(N).astype(np.int32)
+    seeds = rng.integers(0, N, walkers)
+    keep = _tables([indptr, small_ptr], [indices, small_ix], dev, torch.int32)
+    path = np.array([0, 0, 1] * 22 + [0], dtype=np.int64)
+    got = capi.metapath_walk(keep[2], keep[3], keep[4], torch.int32, to_dev(path, dev),
+                             to_dev(seeds, dev, torch.int32), seed=6)
+    want = O.metapath_walk([indptr, small_ptr], [indices.astype(np.int64), small_ix.astype(np.int64)],
+                           path, seeds, seed=6)
+    assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
