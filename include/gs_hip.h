@@ -717,7 +717,7 @@ int gs_col_row_slice_compact(int64_t D, int id_bytes, void* out_indices, int64_t
                              void* stream);
 /* The same slice (no batches) with the kept edges' data and without the positions, for an id set
  * that fits a compute unit's LDS and long columns (gs_induced_slice_applies tells from the
- * sizes; nnz = edges of the parent).  edge_data / edge_ids as for gs_slice_fill_data, NULL:
+ * sizes; nnz = edges of the parent, any number).  edge_data / edge_ids as for gs_slice_fill_data, NULL:
  * none.  num_rows: a bound on the row ids (0: none known); when a row id reaches it,
  * out_indptr[S] is -1 and the call has to be repeated with num_rows 0.  mark, then (total in
  * out_indptr[S]) compact with the same workspace; out_data NULL exactly when edge_data was. */

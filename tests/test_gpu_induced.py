@@ -125,3 +125,29 @@ def test_data_of_the_first_edges_only(dev):
     sub = g._CAPI_FusionSlicing(ids, ids)
     assert torch.equal(sub._CAPI_GetData("default"), w)
     assert np.array_equal(sub._CAPI_GetCSC()[1].cpu().numpy(), indices[:2_000_000])
+
+
+@pytest.mark.parametrize("weights", [False, True])
+def test_more_edges_than_32_bits_count(dev, weights):
+    """Columns at the end of a neighbour array of more than 2**32 edges."""
+    n, degree = 1 << 16, (1 << 16) + 1
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(2)
+    indices = torch.randint(0, n, (n * degree,), generator=gen, device=dev, dtype=torch.int32)
+    g = gs.Graph(False)
+    g._CAPI_LoadCSC(torch.arange(n + 1, device=dev) * degree, indices)
+    if weights:
+        w = torch.empty(n * degree, device=dev)
+        w[-20 * degree:] = torch.rand(20 * degree, device=dev)
+        g._CAPI_SetData(w)
+    cols = torch.arange(n - 20, n, device=dev, dtype=torch.int32)
+    rows = torch.randperm(n, generator=gen, device=dev)[:5000].to(torch.int32)
+    sub = g._CAPI_FusionSlicing(cols, rows)
+    place = torch.full((n,), -1, dtype=torch.int32, device=dev)
+    place[rows.long()] = torch.arange(5000, dtype=torch.int32, device=dev)
+    want = place[indices[-20 * degree:].long()]
+    ptr, idx, _ = sub._CAPI_GetCSC()
+    assert torch.equal(idx, want[want >= 0])
+    assert torch.equal(ptr[1:], torch.cumsum((want >= 0).view(20, degree).sum(1), 0))
+    if weights:
+        assert torch.equal(sub._CAPI_GetData("default"), w[-20 * degree:][want >= 0])
