@@ -151,3 +151,26 @@ def test_more_edges_than_32_bits_count(dev, weights):
     assert torch.equal(ptr[1:], torch.cumsum((want >= 0).view(20, degree).sum(1), 0))
     if weights:
         assert torch.equal(sub._CAPI_GetData("default"), w[-20 * degree:][want >= 0])
+
+
+@pytest.mark.parametrize("hubs,hub_degree,small,n,columns", [(130, 8192, 0, 60_000, 60_000),  # mostly empty
+                                                             (8, 200_000, 9, 500_000, 100_000),
+                                                             (40, 60_000, 20, 700_000, 37_000)])
+@pytest.mark.parametrize("weights", [False, True])
+def test_short_columns(dev, hubs, hub_degree, small, n, columns, weights):
+    """Columns on both sides of 64 edges on average, with data and without (the general slice)."""
+    indptr, indices, rng = _graph(n, hubs, hub_degree, small, n)
+    hub = np.flatnonzero(np.diff(indptr) == hub_degree)
+    cols = np.concatenate([hub, rng.permutation(n)])[:columns].astype(np.int64)
+    rows = rng.permutation(n)[: min(n // 2, 9000)].astype(np.int64)
+    g = gs.Graph(False)
+    g._CAPI_LoadCSC(to_dev(indptr, dev), to_dev(indices, dev))
+    w = rng.random(indices.size).astype(np.float32)
+    if weights:
+        g._CAPI_SetData(to_dev(w, dev))
+    sub = g._CAPI_FusionSlicing(to_dev(cols, dev), to_dev(rows, dev))
+    want = O.col_row_slice(indptr, indices, cols, rows)
+    assert np.array_equal(sub._CAPI_GetCSC()[0].cpu().numpy(), want[0])
+    assert np.array_equal(sub._CAPI_GetCSC()[1].cpu().numpy(), want[1])
+    if weights:
+        assert np.array_equal(sub._CAPI_GetData("default").cpu().numpy(), w[want[3]])
