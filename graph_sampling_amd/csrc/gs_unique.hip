@@ -476,10 +476,16 @@ int relabel_sampled_impl(const void* seed_keys, int64_t S, const void* sampled, 
   if (M > 0) {
     ProfileScope prof("table_insert", stream);
     // No peek at the slot: sampled neighbours are mostly new keys, and the extra read costs the
-    // GraphSAGE step 7 % (0.152 ms against 0.142).  Nor a meeting in LDS first, 2-5 % of a
-    // minibatch on graphs of millions of nodes, unless the items are so many against the ids
-    // there are that hubs come up by the hundred: 5000 seeds, fanouts 25 and 15 on 233 k
-    // nodes, 1.07 M items in all: 134 -> 115 us a minibatch.
+    // GraphSAGE step 7 % (0.152 ms against 0.142).  Nor a meeting in LDS first, unless the items
+    // are so many against the ids there are that hubs come up by the hundred.  The host knows
+    // no more than their bound M, a place for every sample.  One layer, sampling and relabel, without
+    // / with the meeting, us, by M over ids (64-bit ids; 32-bit ones go the same way):
+    //                            0.06       0.25       0.45       0.55       1          2
+    //   131 k nodes, degree 16   34.7/35.6  35.0/35.7  37.0/37.1  37.6/37.0  40.9/38.1  47.7/42.6
+    //   1 M nodes, degree 16     35.7/36.8  41.5/42.0  48.8/48.5  50.6/50.0  63.1/61.6
+    //   233 k nodes, degree 492  35.7/35.8  40.4/37.9  45.8/40.5  48.2/42.1  59.1/49.0  77.0/59.8
+    //   4 M nodes, degree 30     42.2/42.5  58.4/58.4
+    // (5000 seeds, fanouts 25 and 15, 233 k nodes of degree 492: 133 -> 103 a minibatch.)
     constexpr bool kNarrow = sizeof(IdT) == 8 && std::is_same<T, PackedTable>::value;
     const auto insert = num_ids > 0 && 2 * M >= num_ids ? table_insert_grouped_kernel<IdT, T, false>
                                                         : table_insert_kernel<IdT, T>;
