@@ -172,14 +172,17 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
   const int64_t t = gridDim.x - 1 - blockIdx.x;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   // (what the chain of dependent reads starts with goes out first; the data wait for the first and
-  // the last offset, since an array may end where the offsets do: 124 M edges take 126 us in a sum
-  // and 264 in a normalise with that wait, 127 and 262 without)
-  int64_t head = 0, tail = 0;  // segments of the tile's first edge and of the one behind its last
+  // the last offset, since an array may end where the offsets do: sum and normalise of 124 M
+  // edges 391 us with that wait, 389 without)
+  int left_head = 0, left_tail = 0;
   if (WALK != kSearch) {
-    head = tl.head[t];
-    if (WALK == kHeads) tail = tl.head[t + 1];
+    left_head = tl.head[t];
+    if (WALK == kHeads) left_tail = tl.head[t + 1];
   }
   const Edges edges(indptr, num_seg, nnz);
+  // (both are asked for before the workgroup knows whether it has edges)
+  if (WALK != kSearch) asm volatile("" : "+s"(left_head), "+s"(left_tail));
+  int64_t head = left_head, tail = left_tail;  // segments of the tile's first edge and of the one behind its last
   const int64_t p0 = edges.first + t * kTile;
   if (p0 >= edges.end) return;
   const int n = edges.in_tile(p0);
@@ -556,12 +559,14 @@ crossing_divide_kernel(const int64_t* __restrict__ indptr, const int64_t* __rest
                        const float* __restrict__ data, int64_t num_seg, int64_t nnz,
                        float* __restrict__ out, Tiles tl, bool hubs) {
   __shared__ float s_total[2];
+  __shared__ int s_wide[2];  // whether the segment spans more than 64 tiles
   __shared__ int64_t s_tiles[2][2];
   __shared__ float s_part[kThreads / kWave];
   const int64_t t = blockIdx.x;
   const Edges edges(indptr, num_seg, nnz);
   const int64_t p0 = edges.first + t * kTile;
-  const int inner = tl.inner[t], g_in = tl.head[t], g_out = tl.outgoing[t];
+  int inner = tl.inner[t], g_in = tl.head[t], g_out = tl.outgoing[t];
+  asm volatile("" : "+s"(inner), "+s"(g_in), "+s"(g_out));  // (asked for in front of the branch)
   if (p0 >= edges.end) return;
   const int n = edges.in_tile(p0);
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
@@ -593,16 +598,19 @@ crossing_divide_kernel(const int64_t* __restrict__ indptr, const int64_t* __rest
       }
     }
     if (lane == 0) {
+      s_wide[wave] = to - from > kWave;
       s_tiles[wave][0] = from;
       s_tiles[wave][1] = to;
     }
   }
   __syncthreads();
-  for (int r = 0; r < 2; ++r) {
-    const int64_t from = s_tiles[r][0], to = s_tiles[r][1];  // (the same for the whole workgroup)
-    if (to - from <= kWave) continue;
-    const float rest = hubs && to - from > kHubTiles ? 0.0f : sum_pieces(tl, from, to, s_part);
-    if (tid == 0) s_total[r] = tl.carry[2 * from + 1] + rest;
+  if (s_wide[0] | s_wide[1]) {  // (the same for the whole workgroup)
+    for (int r = 0; r < 2; ++r) {
+      if (!s_wide[r]) continue;
+      const int64_t from = s_tiles[r][0], to = s_tiles[r][1];
+      const float rest = hubs && to - from > kHubTiles ? 0.0f : sum_pieces(tl, from, to, s_part);
+      if (tid == 0) s_total[r] = tl.carry[2 * from + 1] + rest;
+    }
     __syncthreads();
   }
   const float before = s_total[0], behind = s_total[1];
