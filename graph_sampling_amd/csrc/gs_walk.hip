@@ -12,7 +12,7 @@
 // enough walkers the kernel is bound by lines fetched behind the L2s: random reads
 // that miss run at about 55 G/s on this machine, in the memory-side cache or not (hits
 // at 260 G/s), and a million walkers on a graph of 4 M nodes and 200 M edges miss
-// 69 M times in 47 M steps.  With few it is latency: 256 threads per workgroup, no
+// 66 M times in 47 M steps.  With few it is latency: 256 threads per workgroup, no
 // LDS, ~24 VGPRs, as many waves as there are.  One Philox block feeds four steps.
 #include "gs_common.hpp"
 
@@ -23,10 +23,18 @@ constexpr int kThreads = 256;
 
 // Neighbour arrays from this size on are read as streams (the line is the first to leave the
 // L2): hardly one of their lines is met again, and the offsets, which are, stay longer.
-// Arrays that the L2s and the memory-side cache hold in good part lose by it.  Metapath over three
-// arrays of 400 MB, 20 steps: 200 k walkers 89 -> 85 us, 1 M walkers 411 -> 383; 1 M walkers, 80
-// steps, 800 MB: 1457 -> 1349 to 1430 from run to run; but 20 k walkers over 32 MB: 41 -> 68.
-constexpr int64_t kStreamBytes = int64_t(256) << 20;
+// Arrays that the L2s and the memory-side cache hold in good part lose by it.  38 steps, three graphs
+// in turn, plain / as a stream, us, by walkers:
+//                               66 k       131 k       400 k       1 M
+//   280 MB (70 M edges, 32-bit)   66/65      86/97     266/281    632/662
+//   400 MB (100 M, 32-bit)        69/67      93/104    289/307    687/724
+//   720 MB (90 M, 64-bit)         73/66      95/98     301/291    710/704
+//   800 MB (200 M, 32-bit)        70/67      98/102    307/301    727/708
+//   1.1 GB (139 M, 64-bit)        72/66      96/96     296/286    693/688
+constexpr int64_t kStreamBytes = int64_t(5) << 27;
+// The same for a relation of a metapath, when the path has two such: three of 400 MB, 20 steps, 200 k
+// walkers 89 -> 85 us, 1 M walkers 411 -> 383.
+constexpr int64_t kStreamRelationBytes = int64_t(256) << 20;
 // A metapath's relations have to be looked up for it in front of the first step, 1.0 to 1.4 us that
 // only long work earns back: 1 M walkers, 4 steps 93 -> 92 us, 200 k walkers, 20 steps 87 -> 85,
 // but 400 k walkers, 8 steps 70 -> 71, 18 k walkers, 8 steps 12.9 -> 13.8.
@@ -99,8 +107,11 @@ metapath_walk_kernel(const int64_t* const* __restrict__ all_indptr,
     if (LONG_WORK && (t & (kWave - 1)) == 0) {  // a lane per step of the next 64
       const int64_t step = t + (threadIdx.x & (kWave - 1));
       const int64_t rel = metapath[step < length ? step : length - 1];
-      streams = __ballot(all_indptr[rel][all_num_nodes[rel]] >=
-                         kStreamBytes / static_cast<int64_t>(sizeof(IdT)));
+      const int64_t bytes = all_indptr[rel][all_num_nodes[rel]] * static_cast<int64_t>(sizeof(IdT));
+      const unsigned long long large = __ballot(bytes >= kStreamRelationBytes);
+      const int64_t one = __shfl(rel, large ? __ffsll(static_cast<long long>(large)) - 1 : 0, kWave);
+      const bool two = __ballot(bytes >= kStreamRelationBytes && rel != one) != 0ull;
+      streams = two ? large : __ballot(bytes >= kStreamBytes);
     }
     if (!replay && (t & 3) == 0)
       x = draw_block(seed, kTagWalk, static_cast<uint64_t>(w), static_cast<uint64_t>(t >> 2));

@@ -127,9 +127,8 @@ def test_walk_out_of_range_seeds_die(dev):
 @pytest.mark.parametrize("idt", [torch.int32, torch.int64])
 @pytest.mark.parametrize("less", [0, 1])
 def test_walks_over_neighbour_arrays_read_as_streams(dev, idt, less):
-    """Neighbour arrays of 256 MB and of one edge less (read as streams and not), alone and as one
-    relation beside a small one, over more than 64 steps; each node has 64 neighbours, the
-    last fewer."""
+    """Neighbour arrays of 256 MB and of one edge less, alone and as one relation beside a small one,
+    over more than 64 steps; each node has 64 neighbours, the last fewer."""
     E = (1 << 28) // (4 if idt == torch.int32 else 8) - less
     N = (E + 63) // 64
     rng = np.random.default_rng(less)
@@ -149,19 +148,37 @@ def test_walks_over_neighbour_arrays_read_as_streams(dev, idt, less):
     assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
 
 
-@pytest.mark.parametrize("walkers", [62_601, 62_602])  # 67 steps of each: 2**22 in all, less 37 and more 30
-def test_long_metapath_work_over_streams(dev, walkers):
-    """From 2**22 steps in all, large neighbour arrays of a metapath are read as streams."""
+@pytest.mark.parametrize("idt", [torch.int32, torch.int64])
+@pytest.mark.parametrize("less", [0, 1])
+def test_walks_over_a_neighbour_array_read_as_a_stream(dev, idt, less):
+    """A neighbour array of 640 MB, from which on it is read as a stream, and of one edge less."""
+    E = (5 << 27) // (4 if idt == torch.int32 else 8) - less
+    N = (E + 63) // 64
+    indptr = np.minimum(np.arange(N + 1, dtype=np.int64) * 64, E)
+    indices = np.random.default_rng(less).integers(0, N, E, dtype=np.int64)
+    seeds = np.random.default_rng(3).integers(0, N, 300)
+    got = capi.random_walk(to_dev(indptr, dev), to_dev(indices, dev, idt), to_dev(seeds, dev, idt), 9,
+                           seed=5)
+    want = O.random_walk(indptr, indices, seeds, 9, seed=5)
+    assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
+
+
+# 67 steps of each: 2**22 in all, less 37 and more 30
+@pytest.mark.parametrize("walkers,relations", [(62_601, 2), (62_602, 2), (62_602, 1)])
+def test_long_metapath_work_over_streams(dev, walkers, relations):
+    """From 2**22 steps in all, the neighbour arrays of a metapath's relations are read as streams
+    when two of them are large."""
     E = (1 << 28) // 4
     N = E // 64
     rng = np.random.default_rng(walkers)
-    indptr, small_ptr = np.arange(N + 1, dtype=np.int64) * 64, np.arange(N + 1, dtype=np.int64)
-    indices, small_ix = rng.integers(0, N, E).astype(np.int32), rng.permutation(N).astype(np.int32)
+    ptr, small_ptr = np.arange(N + 1, dtype=np.int64) * 64, np.arange(N + 1, dtype=np.int64)
+    indices = [rng.integers(0, N, E).astype(np.int32) for _ in range(relations)]
+    small_ix = rng.permutation(N).astype(np.int32)
     seeds = rng.integers(0, N, walkers)
-    keep = _tables([indptr, small_ptr], [indices, small_ix], dev, torch.int32)
-    path = np.array([0, 0, 1] * 22 + [0], dtype=np.int64)
+    ptrs = [ptr] * relations + [small_ptr]
+    keep = _tables(ptrs, indices + [small_ix], dev, torch.int32)
+    path = np.array([0, relations - 1, relations] * 22 + [0], dtype=np.int64)
     got = capi.metapath_walk(keep[2], keep[3], keep[4], torch.int32, to_dev(path, dev),
                              to_dev(seeds, dev, torch.int32), seed=6)
-    want = O.metapath_walk([indptr, small_ptr], [indices.astype(np.int64), small_ix.astype(np.int64)],
-                           path, seeds, seed=6)
+    want = O.metapath_walk(ptrs, [i.astype(np.int64) for i in indices + [small_ix]], path, seeds, seed=6)
     assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
