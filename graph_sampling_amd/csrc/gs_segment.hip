@@ -25,11 +25,12 @@
 // every segment's first edge.
 //
 // 124 M edges in 2.45 M columns (half of them of at most 16 edges, 19 % of the edges in columns
-// longer than a tile): sum 144 us (3.5 TB/s; the bytes bound it), normalise 308 us (3.2 TB/s
-// over the bytes it needs, 4.3 with the second reading; each tile's chain of LDS steps hides
-// behind five tiles a CU).  A lane per short column, a scan per 1024-edge chunk for the others
-// and a divide pass over all edges, each reading its edges for itself, took 214 and 380.
-// Tiles of 8192 edges: 156 and 324.
+// longer than a tile), kernels: sum 137 us (3.8 TB/s; the bytes bound it: tiles 121 of it),
+// normalise 282 us (3.5 TB/s over the bytes it needs, 4.7 with the second reading: tiles 179,
+// the crossing segments 95; each tile's chain of LDS steps hides behind the other tiles of its
+// CU).  A lane per short column, a scan per 1024-edge chunk for the others and a divide pass
+// over all edges, each reading its edges for itself, took 214 and 380.  Tiles of 8192 edges:
+// 156 and 324, against 144 and 308 as the tiles of 4096 were then.
 #include <limits>
 #include "gs_common.hpp"
 

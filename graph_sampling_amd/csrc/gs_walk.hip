@@ -10,8 +10,8 @@
 // register (the reference re-reads it from the trace, random_walk.cu:32).  A
 // step is two dependent random reads (the indptr pair, then one neighbour).  With
 // enough walkers the kernel is bound by lines fetched behind the L2s: random reads
-// that miss run at about 55 G/s on this machine, in the memory-side cache or not (hits
-// at 260 G/s), and a million walkers on a graph of 4 M nodes and 200 M edges miss
+// that miss run at 48-55 G/s on this machine, in the memory-side cache or not (hits
+// at 255 G/s), and a million walkers on a graph of 4 M nodes and 200 M edges miss
 // 66 M times in 47 M steps.  With few it is latency: 256 threads per workgroup, no
 // LDS, ~24 VGPRs, as many waves as there are.  One Philox block feeds four steps.
 #include "gs_common.hpp"
