@@ -770,8 +770,7 @@ c10::intrusive_ptr<Graph> Graph::FusedBidirSlicing(torch::Tensor column_seeds,
   // (that form reads the data of every edge of the columns, dropped ones too: all have to be there)
   if (!data_.has_value() || (hip::EdgeData::Fits(data_.value(), csc_->e_ids) &&
                              !hip::EdgeData::Followed(data_.value()) &&
-                             (csc_->e_ids.has_value() ||
-                              data_.value().numel() >= csc_->indices.numel()))) {
+                             data_.value().numel() >= csc_->indices.numel())) {
     // the edges' data, if there are any, come along in the slice's own passes
     const hip::EdgeData edge{data_.value_or(torch::Tensor()), csc_->e_ids};
     torch::Tensor data;

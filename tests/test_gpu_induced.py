@@ -111,14 +111,19 @@ def test_data_that_is_followed(dev, hub_degree, coo):
         assert torch.equal(got.primal, w[at]) and torch.equal(got.tangent, t[at])
 
 
-def test_data_of_the_first_edges_only(dev):
+@pytest.mark.parametrize("coo", [False, True])
+def test_data_of_the_first_edges_only(dev, coo):
     """Data that end before the edges do serve a subgraph whose kept edges all have theirs."""
     indptr = np.array([0, 1_200_000, 2_400_000], dtype=np.int64)
     indices = np.zeros(2_400_000, dtype=np.int64)
     indices[::3] = 1
     indices[2_000_000:] = 7  # no node of the subgraph
     g = gs.Graph(False)
-    g._CAPI_LoadCSC(to_dev(indptr, dev), to_dev(indices, dev))
+    if coo:  # (with a map from its edges to the data)
+        col = np.repeat(np.arange(8), np.diff(np.append(indptr, [indptr[-1]] * 6)))
+        g._CAPI_LoadCOO(to_dev(indices, dev), to_dev(col, dev))
+    else:
+        g._CAPI_LoadCSC(to_dev(indptr, dev), to_dev(indices, dev))
     w = torch.rand(2_000_000, device=dev)
     g._CAPI_SetData(w)
     ids = torch.tensor([0, 1], device=dev)
