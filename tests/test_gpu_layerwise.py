@@ -95,6 +95,39 @@ def test_pick_rows_and_block_values_against_numpy(dev, idb, E, num_nodes, room):
         assert np.array_equal(out_indptr.cpu().numpy(), want_indptr)
 
 
+@pytest.mark.parametrize("na,nb", [(1024, 0), (1000, 25), (2047, 1), (2000, 49), (4096, 0), (2, 4095)])
+def test_sorted_union_at_the_numbers_of_keys_a_thread(dev, na, nb):
+    for idb, (npt, _) in IDT.items():
+        if na + nb > capi.sorted_union_max(idb):
+            continue
+        rng = np.random.default_rng(na + nb)
+        for top in (3, 1 << 30):  # hardly any value but repeats, hardly any repeats
+            ids = rng.integers(0, top, na + nb).astype(npt)
+            out, count = capi.sorted_union(to_dev(ids[:na], dev), to_dev(ids[na:], dev))
+            assert np.array_equal(out[:int(count.item())].cpu().numpy(), np.unique(ids))
+
+
+@pytest.mark.parametrize("idb,E,num_nodes,room", [
+    (4, 4096, 2, 2), (4, 4097, 1024, 1024), (8, 4095, 1023, 1024), (4, 9000, 8192, 8192),
+    (8, 9000, 4096, 4096), (4, 4096 * 4096 + 5, 3, 3)])
+def test_pick_rows_with_a_full_tree_and_beyond_the_tiles_that_add_up_themselves(dev, idb, E, num_nodes, room):
+    npt, _ = IDT[idb]
+    rng = np.random.default_rng(E)
+    N = 3 * num_nodes
+    row = rng.integers(0, N, E).astype(npt)
+    col = np.zeros(E, npt)
+    nodes = np.sort(rng.permutation(N)[:num_nodes]).astype(npt)
+    row[0], row[-1] = nodes[0], nodes[-1]
+    count = torch.tensor([num_nodes], dtype=torch.int64, device=dev)
+    key, pos, totals = capi.coo_pick_rows(to_dev(row, dev), to_dev(col, dev), to_dev(nodes, dev), count, room)
+    bits = int(np.ceil(np.log2(room)))
+    want_key, want_pos = _np_pick(row, col, nodes, bits)
+    kept = int(totals[1].item())
+    assert kept == want_pos.size
+    assert np.array_equal(key[:kept].cpu().numpy().astype(np.int64), want_key)
+    assert np.array_equal(pos[:kept].cpu().numpy().astype(np.int64), want_pos)
+
+
 def test_block_values_without_edges_has_offsets_of_zero(dev):
     empty = torch.empty(0, dtype=torch.int32, device=dev)
     one = torch.zeros(1, dtype=torch.int32, device=dev)
