@@ -523,9 +523,10 @@ sample_one_keepdim_kernel(const int64_t* __restrict__ indptr, const IdT* __restr
 // ----------------------------------------------------------- host glue -----
 template <typename IdT>
 int slice_count_impl(const int64_t* indptr, int64_t num_cols, const void* cols, int64_t S,
-                     int64_t* sub_indptr, int64_t* tile_ws, hipStream_t stream) {
+                     int64_t* sub_indptr, int64_t* tile_ws, gs_mailbox* box, int64_t ticket,
+                     hipStream_t stream) {
   ColDegree<IdT> f{indptr, static_cast<const IdT*>(cols), num_cols};
-  return exclusive_scan(f, S, sub_indptr, tile_ws, stream);
+  return exclusive_scan(f, S, sub_indptr, tile_ws, stream, box, ticket);
 }
 
 template <typename IdT, bool WITH_COO, bool WITH_DATA>
@@ -571,9 +572,9 @@ int slice_fill_impl(const int64_t* indptr, int64_t num_cols, const void* indices
 template <typename IdT>
 int sample_count_impl(const int64_t* indptr, int64_t num_cols, const void* cols, int64_t S,
                       int64_t k, int replace, int64_t* sub_indptr, int64_t* tile_ws,
-                      hipStream_t stream) {
+                      gs_mailbox* box, int64_t ticket, hipStream_t stream) {
   ColCount<IdT> f{indptr, static_cast<const IdT*>(cols), num_cols, k, replace};
-  return exclusive_scan(f, S, sub_indptr, tile_ws, stream);
+  return exclusive_scan(f, S, sub_indptr, tile_ws, stream, box, ticket);
 }
 
 template <typename IdT, bool WITH_COO>
@@ -1317,9 +1318,9 @@ extern "C" {
 
 size_t gs_slice_workspace_bytes(int64_t num_cols) { return scan_workspace_bytes(num_cols); }
 
-int gs_slice_count(const int64_t* indptr, int64_t num_cols, const void* column_ids, int id_bytes,
-                   int64_t S, int64_t* sub_indptr, void* workspace, size_t workspace_bytes,
-                   void* stream) {
+int gs_slice_count_notify(const int64_t* indptr, int64_t num_cols, const void* column_ids,
+                          int id_bytes, int64_t S, int64_t* sub_indptr, gs_mailbox* mailbox,
+                          int64_t ticket, void* workspace, size_t workspace_bytes, void* stream) {
   GS_REQUIRE(indptr && sub_indptr && S >= 0 && num_cols >= 0,
              "gs_slice_count: null pointer or negative size");
   GS_REQUIRE(S == 0 || column_ids, "gs_slice_count: column_ids is null");
@@ -1333,8 +1334,17 @@ int gs_slice_count(const int64_t* indptr, int64_t num_cols, const void* column_i
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   return id_bytes == 8
-             ? slice_count_impl<int64_t>(indptr, num_cols, column_ids, S, sub_indptr, tiles, st)
-             : slice_count_impl<int32_t>(indptr, num_cols, column_ids, S, sub_indptr, tiles, st);
+             ? slice_count_impl<int64_t>(indptr, num_cols, column_ids, S, sub_indptr, tiles,
+                                         mailbox, ticket, st)
+             : slice_count_impl<int32_t>(indptr, num_cols, column_ids, S, sub_indptr, tiles,
+                                         mailbox, ticket, st);
+}
+
+int gs_slice_count(const int64_t* indptr, int64_t num_cols, const void* column_ids, int id_bytes,
+                   int64_t S, int64_t* sub_indptr, void* workspace, size_t workspace_bytes,
+                   void* stream) {
+  return gs_slice_count_notify(indptr, num_cols, column_ids, id_bytes, S, sub_indptr, nullptr, 0,
+                               workspace, workspace_bytes, stream);
 }
 
 int gs_post_total(const int64_t* value, gs_mailbox* mailbox, int64_t ticket, void* stream) {
@@ -1404,9 +1414,10 @@ size_t gs_sample_workspace_bytes(int64_t S, int64_t fanout) {
   return scan_workspace_bytes(s) + padded(8) + padded(static_cast<size_t>(s + kQueueExtra) * 8);
 }
 
-int gs_sample_count(const int64_t* indptr, int64_t num_cols, const void* column_ids, int id_bytes,
-                    int64_t S, int64_t fanout, int replace, int64_t* sub_indptr, void* workspace,
-                    size_t workspace_bytes, void* stream) {
+int gs_sample_count_notify(const int64_t* indptr, int64_t num_cols, const void* column_ids,
+                           int id_bytes, int64_t S, int64_t fanout, int replace,
+                           int64_t* sub_indptr, gs_mailbox* mailbox, int64_t ticket,
+                           void* workspace, size_t workspace_bytes, void* stream) {
   GS_REQUIRE(indptr && sub_indptr && S >= 0 && fanout >= 0 && num_cols >= 0,
              "gs_sample_count: null pointer or negative size");
   GS_REQUIRE(column_ids || S <= num_cols, "gs_sample_count: S exceeds num_cols without column_ids");
@@ -1421,9 +1432,16 @@ int gs_sample_count(const int64_t* indptr, int64_t num_cols, const void* column_
   hipStream_t st = static_cast<hipStream_t>(stream);
   return id_bytes == 8
              ? sample_count_impl<int64_t>(indptr, num_cols, column_ids, S, fanout, replace,
-                                          sub_indptr, tiles, st)
+                                          sub_indptr, tiles, mailbox, ticket, st)
              : sample_count_impl<int32_t>(indptr, num_cols, column_ids, S, fanout, replace,
-                                          sub_indptr, tiles, st);
+                                          sub_indptr, tiles, mailbox, ticket, st);
+}
+
+int gs_sample_count(const int64_t* indptr, int64_t num_cols, const void* column_ids, int id_bytes,
+                    int64_t S, int64_t fanout, int replace, int64_t* sub_indptr, void* workspace,
+                    size_t workspace_bytes, void* stream) {
+  return gs_sample_count_notify(indptr, num_cols, column_ids, id_bytes, S, fanout, replace,
+                                sub_indptr, nullptr, 0, workspace, workspace_bytes, stream);
 }
 
 int gs_sample_uniform_fill(const int64_t* indptr, int64_t num_cols, const void* indices,

@@ -273,6 +273,34 @@ int64_t ReadTotal(const torch::Tensor& values, int64_t at, void* stream, const c
   const int64_t total = WaitBox(boxes.slot(ticket), ticket, stream, what);
   return total == kLost ? values[at].item<int64_t>() : total;
 }
+
+// A total that the launch which works it out posts by itself: values[at] once the ticket has
+// come, waited for where it is needed.
+struct TotalBox {
+  explicit TotalBox(const torch::Tensor& like) : boxes(Boxes(like.get_device())), ticket(boxes.next++) {}
+  gs_mailbox* slot() const { return boxes.slot(ticket); }
+  int64_t Wait(const torch::Tensor& values, int64_t at, void* stream, const char* what) const {
+    const int64_t total = WaitBox(slot(), ticket, stream, what);
+    return total == kLost ? values[at].item<int64_t>() : total;
+  }
+  HostBoxes& boxes;
+  const int64_t ticket;
+};
+
+// offsets of the column slice, its total on the host
+int64_t SliceCount(const torch::Tensor& indptr, const torch::Tensor& column_ids, int idb,
+                   torch::Tensor& sub_indptr) {
+  const int64_t S = column_ids.numel();
+  sub_indptr = torch::empty({S + 1}, I64(indptr));
+  auto ws = Scratch(gs_slice_workspace_bytes(S), indptr);
+  void* st = Stream(indptr);
+  const TotalBox total(indptr);
+  Check(gs_slice_count_notify(indptr.data_ptr<int64_t>(), indptr.numel() - 1, column_ids.data_ptr(),
+                              idb, S, sub_indptr.data_ptr<int64_t>(), total.slot(), total.ticket,
+                              ws.data_ptr(), ws.numel(), st),
+        "gs_slice_count");
+  return total.Wait(sub_indptr, S, st, "gs_slice_count");
+}
 }  // namespace
 
 Posted PostValueSets(const std::vector<torch::Tensor>& sets, torch::Tensor& pinned) {
@@ -322,13 +350,9 @@ SliceResult ColSlicing(const torch::Tensor& indptr, const torch::Tensor& indices
   const int idb = IdBytes(indices, "indices");
   TORCH_CHECK(IdBytes(column_ids, "column ids") == idb, "column ids and indices differ in dtype");
   const int64_t S = column_ids.numel();
-  auto sub_indptr = torch::empty({S + 1}, I64(indptr));
-  auto ws = Scratch(gs_slice_workspace_bytes(S), indptr);
+  torch::Tensor sub_indptr;
+  const int64_t nnz = SliceCount(indptr, column_ids, idb, sub_indptr);
   void* st = Stream(indptr);
-  Check(gs_slice_count(indptr.data_ptr<int64_t>(), indptr.numel() - 1, column_ids.data_ptr(), idb, S,
-                       sub_indptr.data_ptr<int64_t>(), ws.data_ptr(), ws.numel(), st),
-        "gs_slice_count");
-  const int64_t nnz = ReadTotal(sub_indptr, S, st, "gs_slice_count");
   auto sub_indices = torch::empty({nnz}, indices.options());
   torch::Tensor select_index;
   if (with_select) select_index = torch::empty({nnz}, I64(indptr));
@@ -373,11 +397,14 @@ SliceResult SampleInto(const torch::Tensor& indptr, const torch::Tensor& indices
   auto ws = Scratch(bytes, indptr);
   void* st = Stream(indptr);
   const void* cols = fused ? column_ids.data_ptr() : nullptr;
-  Check(gs_sample_count(indptr.data_ptr<int64_t>(), indptr.numel() - 1, cols, idb, S, fanout, replace ? 1 : 0,
-                        sub_indptr.data_ptr<int64_t>(), ws.data_ptr(), ws.numel(), st),
+  const TotalBox total(indptr);
+  Check(gs_sample_count_notify(indptr.data_ptr<int64_t>(), indptr.numel() - 1, cols, idb, S, fanout,
+                               replace ? 1 : 0, sub_indptr.data_ptr<int64_t>(), total.slot(),
+                               total.ticket, ws.data_ptr(), ws.numel(), st),
         "gs_sample_count");
   fill(cols, idb, S, sub_indptr, sub_indices, select_index, coo_col, ws, st);
-  const int64_t nnz = ReadTotal(sub_indptr, S, Stream(sub_indptr), "total");  // the only host read of the call
+  // the only host read of the call: the total is there before the fill has run
+  const int64_t nnz = total.Wait(sub_indptr, S, st, "gs_sample_count");
   if (with_coo) coo_col = coo_col.narrow(0, 0, nnz);
   return {sub_indptr, coo_col, sub_indices.narrow(0, 0, nnz), select_index.narrow(0, 0, nnz)};
 }
@@ -563,13 +590,7 @@ SliceResult ColSamplingProbs(const torch::Tensor& indptr, const torch::Tensor& i
     int64_t cdf_len = indices.numel();
     if (column_ids.defined()) {
       NeedI64(indptr, "indptr");
-      cdf_ptr = torch::empty({S + 1}, I64(indptr));
-      auto sws = Scratch(gs_slice_workspace_bytes(S), indptr);
-      Check(gs_slice_count(indptr.data_ptr<int64_t>(), indptr.numel() - 1, column_ids.data_ptr(),
-                           IdBytes(column_ids, "column ids"), S, cdf_ptr.data_ptr<int64_t>(),
-                           sws.data_ptr(), sws.numel(), Stream(indptr)),
-            "gs_slice_count");
-      cdf_len = ReadTotal(cdf_ptr, S, Stream(cdf_ptr), "total");
+      cdf_len = SliceCount(indptr, column_ids, IdBytes(column_ids, "column ids"), cdf_ptr);
     }
     auto cdf = torch::empty({cdf_len > 0 ? cdf_len : 1}, probs.options());
     return SampleInto(
@@ -1234,14 +1255,9 @@ namespace {
 // offsets of the column slice and its number of edges (the host waits for it)
 std::tuple<torch::Tensor, int64_t> SliceOffsets(const torch::Tensor& indptr,
                                                 const torch::Tensor& column_ids, int idb) {
-  const int64_t S = column_ids.numel();
-  auto sub_indptr = torch::empty({S + 1}, I64(indptr));
-  auto ws = Scratch(gs_slice_workspace_bytes(S), indptr);
-  void* st = Stream(indptr);
-  Check(gs_slice_count(indptr.data_ptr<int64_t>(), indptr.numel() - 1, column_ids.data_ptr(), idb, S,
-                       sub_indptr.data_ptr<int64_t>(), ws.data_ptr(), ws.numel(), st),
-        "gs_slice_count");
-  return {sub_indptr, ReadTotal(sub_indptr, S, st, "total")};
+  torch::Tensor sub_indptr;
+  const int64_t total = SliceCount(indptr, column_ids, idb, sub_indptr);
+  return {sub_indptr, total};
 }
 
 // the general column + row slice behind those offsets; index arrays nobody asks for stay undefined

@@ -123,6 +123,11 @@ size_t gs_slice_workspace_bytes(int64_t num_cols);
 int gs_slice_count(const int64_t* indptr, int64_t num_cols, const void* column_ids, int id_bytes,
                    int64_t S, int64_t* sub_indptr, void* workspace, size_t workspace_bytes,
                    void* stream);
+/* The same, with the total posted to a mailbox (may be NULL) as soon as it is known (the read
+ * of src/cuda/slicing.cu:147 without a copy or a launch of its own). */
+int gs_slice_count_notify(const int64_t* indptr, int64_t num_cols, const void* column_ids,
+                          int id_bytes, int64_t S, int64_t* sub_indptr, gs_mailbox* mailbox,
+                          int64_t ticket, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Posts *value (a device int64, e.g. sub_indptr + S after gs_slice_count) to a mailbox from a
  * one-thread kernel queued on the stream: the host then spins on the mailbox instead of
@@ -186,6 +191,12 @@ typedef enum gs_sample_algo { GS_SAMPLE_AUTO = 0, GS_SAMPLE_RESERVOIR = 1 } gs_s
 int gs_sample_count(const int64_t* indptr, int64_t num_cols, const void* column_ids, int id_bytes,
                     int64_t S, int64_t fanout, int replace, int64_t* sub_indptr, void* workspace,
                     size_t workspace_bytes, void* stream);
+/* The same, with the total posted to a mailbox (may be NULL) as soon as it is known: the fill is
+ * queued behind it either way, on buffers for S * fanout samples. */
+int gs_sample_count_notify(const int64_t* indptr, int64_t num_cols, const void* column_ids,
+                           int id_bytes, int64_t S, int64_t fanout, int replace,
+                           int64_t* sub_indptr, gs_mailbox* mailbox, int64_t ticket,
+                           void* workspace, size_t workspace_bytes, void* stream);
 
 /* Fill for a sub_indptr made by gs_sample_count on the same stream.  Output
  * buffers need capacity S*fanout (an upper bound known without reading back).
