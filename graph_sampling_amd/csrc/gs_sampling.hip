@@ -25,6 +25,7 @@
 
 #include <mutex>
 
+#include "gs_select.hpp"
 #include "gs_table.hpp"
 
 GS_STAMPS_DEFINE(sampling)
@@ -36,10 +37,6 @@ namespace {
 // A column id outside [0, num_cols) is treated as an empty column everywhere in
 // this file, so that stray ids (e.g. the -1 a dead-end walk step hands back) can
 // never turn into a wild read.
-__device__ __forceinline__ bool valid_col(int64_t c, int64_t num_cols) {
-  return static_cast<uint64_t>(c) < static_cast<uint64_t>(num_cols);
-}
-
 // (Read without a branch: an absent id list is read at a stride of zero from the offsets,
 // an id outside the graph reads entry 0 twice, and the value is then not used.)
 template <typename IdT>
@@ -653,9 +650,6 @@ constexpr int kGroupThreadsLarge = 1024;
 constexpr int64_t kGroupSmallLanes = int64_t(1) << 17;
 constexpr int kGroupMaxLanes = 8;
 
-inline int group_lanes_for(int64_t fanout) {
-  return fanout <= 4 ? 1 : (fanout <= 8 ? 2 : (fanout <= 16 ? 4 : 8));
-}
 // A linked launch is sized for a bound on the columns, of which the live ones are usually
 // a fraction: it keeps the small tiles up to a larger bound (workgroups beyond the count
 // leave at once and take no part in the look-back).
@@ -723,26 +717,6 @@ __device__ __forceinline__ void linked_insert(const PackedTable& t, IdT key, int
   pos[item] = t.template insert<false>(static_cast<long long>(key), static_cast<uint32_t>(item));
 }
 
-// the value lane `owner` of every G-lane group holds (owner is a constant after unrolling)
-template <int G>
-__device__ __forceinline__ uint32_t group_broadcast(uint32_t v, int owner) {
-  if (G == 1) return v;
-  const int x = static_cast<int>(v);
-  if (G == 2) {  // pairs inside a quad: lanes (0,1) read lane owner, lanes (2,3) lane 2 + owner
-    return static_cast<uint32_t>(owner == 0 ? __builtin_amdgcn_update_dpp(0, x, 0xA0, 0xF, 0xF, false)
-                                            : __builtin_amdgcn_update_dpp(0, x, 0xF5, 0xF, 0xF, false));
-  }
-  if (G == 4) {
-    switch (owner) {
-      case 0: return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x, 0x00, 0xF, 0xF, false));
-      case 1: return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x, 0x55, 0xF, 0xF, false));
-      case 2: return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x, 0xAA, 0xF, 0xF, false));
-      default: return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x, 0xFF, 0xF, 0xF, false));
-    }
-  }
-  return static_cast<uint32_t>(__shfl(x, ((threadIdx.x & (kWave - 1)) & ~(G - 1)) | owner, kWave));
-}
-
 template <typename IdT, int G, bool REPLACE, int THREADS, bool LINKED>
 __global__ void __launch_bounds__(THREADS) sample_group_kernel(FusedArgs<IdT> a) {
   constexpr int kRows = THREADS / G;
@@ -788,41 +762,9 @@ __global__ void __launch_bounds__(THREADS) sample_group_kernel(FusedArgs<IdT> a)
 
   // ---- 2. Floyd's selection by the row's lanes: mine[u] = position of output 4*sub+u
   uint32_t mine[4] = {0u, 0u, 0u, 0u};
-  if (!REPLACE && cnt > 0) {
-    if (deg <= a.k) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) mine[u] = static_cast<uint32_t>(4 * sub + u);
-    } else {
-      const uint32_t lowest = static_cast<uint32_t>(deg - a.k);  // step i draws from [0, lowest + i]
-      uint32_t t[4] = {0u, 0u, 0u, 0u};
-      if (4 * sub < k) {
-        U4 blk;
-        if (a.replay) {
-          const uint32_t* rp = a.replay + a.replay_ptr[my_row];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) blk.v[u] = 4 * sub + u < k ? rp[4 * sub + u] : 0u;
-        } else {
-          blk = draw_block(a.seed, kTagUniform, static_cast<uint64_t>(my_row),
-                           static_cast<uint64_t>(sub));
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) t[u] = blk.v[u] % (lowest + static_cast<uint32_t>(4 * sub + u) + 1u);
-      }
-      uint32_t chosen[KMAX];
-#pragma unroll
-      for (int i = 0; i < KMAX; ++i) {
-        if (i < k) {
-          const uint32_t ti = t[i & 3];  // the owner's lane holds the step's draw
-          bool taken = false;
-#pragma unroll
-          for (int m = 0; m < i; ++m) taken |= chosen[m] == ti;
-          const uint32_t c = group_broadcast<G>(taken ? lowest + static_cast<uint32_t>(i) : ti, i >> 2);
-          chosen[i] = c;
-          if (sub == (i >> 2)) mine[i & 3] = c;
-        }
-      }
-    }
-  }
+  if (!REPLACE && cnt > 0)
+    floyd_picks<G>(a.seed, my_row, sub, k, deg, a.replay ? a.replay + a.replay_ptr[my_row] : nullptr,
+                   mine);
   GS_STAMP(3);  // selection done
   if (threadIdx.x < kWave) {
     const int64_t before = lookback_exclusive_prefix(a.lb, tile, tile_total);

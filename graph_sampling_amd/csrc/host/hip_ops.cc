@@ -809,6 +809,76 @@ bool LayerChainApplies(int64_t num_seeds, const std::vector<int64_t>& fanouts, b
   return true;
 }
 
+namespace {
+
+// The minibatch in one launch of one workgroup, for those small enough (gs_minibatch_applies).  With
+// two layers or more it is the quicker one up to the kernel's own limits (whole call in us, layer by
+// layer / this; 131 k nodes, and 2.45 M with 64-bit ids and weights): 32 x [10, 5] 35/22 43/26,
+// 124 x [10, 5] 43/25 48/45, 7 x [15, 10, 5] 47/28 63/53, 256 x [7, 3] 42/25 49/44.  One layer is two
+// launches against one: 256 x [7] 24/19 26/21, 512 x [3] 23/19 26/21, but 255 x [25] 29/30 32/35, 2048 x [3] 27/28 30/37.
+constexpr int64_t kSmallOneLayer = 2048;
+
+std::shared_ptr<PendingLayers> SmallMinibatch(std::shared_ptr<PendingLayers> p,
+                                              const std::vector<int64_t>& S,
+                                              const torch::Tensor& indptr,
+                                              const torch::Tensor& indices,
+                                              const torch::Tensor& seeds,
+                                              const std::vector<int64_t>& fanouts, bool replace,
+                                              const float* edge_data, const int64_t* edge_ids) {
+  const size_t L = fanouts.size();
+  const int idb = IdBytes(indices, "indices");
+  size_t bytes = 0;
+  for (size_t l = 0; l < L; ++l) {
+    PendingLayers::Layer& y = p->layers[l];
+    const size_t cap = static_cast<size_t>(S[l] * fanouts[l]);
+    y.off_offsets = bytes;
+    bytes += Pad256(static_cast<size_t>(S[l] + 1) * 8);
+    y.off_renamed = bytes;
+    bytes += Pad256(cap * idb);
+    y.off_frontier = bytes;
+    bytes += Pad256((static_cast<size_t>(S[l]) + cap) * idb);
+    y.off_data = bytes;
+    if (edge_data) bytes += Pad256(cap * 4);
+  }
+  p->scratch = Scratch(bytes, indptr);
+  char* base = static_cast<char*>(p->scratch.data_ptr());
+  HostBoxes& boxes = Boxes(p->device);
+  p->box_owner = boxes.buf;
+  p->ring = boxes.ring;
+  p->id_type = indices.scalar_type();
+  p->with_data = edge_data != nullptr;
+  std::vector<uint64_t> draws(L);
+  std::vector<int64_t*> offsets(L);
+  std::vector<void*> renamed(L), frontier(L);
+  std::vector<float*> data(L);
+  std::vector<gs_mailbox*> slots(2 * L);
+  std::vector<int64_t> tickets(2 * L);
+  for (size_t l = 0; l < L; ++l) {
+    PendingLayers::Layer& y = p->layers[l];
+    draws[l] = NextSeed();
+    offsets[l] = reinterpret_cast<int64_t*>(base + y.off_offsets);
+    renamed[l] = base + y.off_renamed;
+    frontier[l] = base + y.off_frontier;
+    data[l] = reinterpret_cast<float*>(base + y.off_data);
+    y.ticket_edges = boxes.next++;
+    y.ticket_unique = boxes.next++;
+    tickets[2 * l] = y.ticket_edges;
+    tickets[2 * l + 1] = y.ticket_unique;
+    slots[2 * l] = boxes.slot(y.ticket_edges);
+    slots[2 * l + 1] = boxes.slot(y.ticket_unique);
+  }
+  p->first_seed = draws[0];
+  Check(gs_minibatch_sample(indptr.data_ptr<int64_t>(), indptr.numel() - 1, EdgeArray(indices, indptr),
+                            seeds.data_ptr(), idb, S[0], static_cast<int>(L), fanouts.data(),
+                            replace ? 1 : 0, draws.data(), edge_data, edge_ids, offsets.data(),
+                            renamed.data(), frontier.data(), data.data(), nullptr, slots.data(),
+                            tickets.data(), p->stream),
+        "gs_minibatch_sample");
+  return p;
+}
+
+}  // namespace
+
 std::shared_ptr<PendingLayers> SampleLayersQueued(const torch::Tensor& indptr,
                                                   const torch::Tensor& indices,
                                                   const torch::Tensor& seeds,
@@ -832,6 +902,9 @@ std::shared_ptr<PendingLayers> SampleLayersQueued(const torch::Tensor& indptr,
   std::vector<int64_t> S(L + 1);
   S[0] = seeds.numel();
   for (int64_t l = 0; l < L; ++l) S[l + 1] = S[l] * (1 + fanouts[l]);
+  if (gs_minibatch_applies(S[0], static_cast<int>(L), fanouts.data()) &&
+      (L > 1 || S[1] <= kSmallOneLayer))
+    return SmallMinibatch(std::move(p), S, indptr, indices, seeds, fanouts, replace, edge_data, edge_ids);
   // ONE allocation for the whole minibatch, made before the first launch: per layer the
   // three outputs at their bounds (offsets, renamed ids, frontier) and what no caller sees (the
   // sampled ids before renaming, the items' table slots, the two counts).  The output tensors

@@ -549,6 +549,26 @@ int gs_layer_table_sweep(void* table, size_t table_bytes, const void* workspace,
                          size_t workspace_bytes, int64_t S_bound, const int64_t* S_dev,
                          int64_t capacity, const int64_t* num_edges, void* stream);
 
+/* A whole small minibatch in ONE launch of one workgroup, with the hash table, the frontier and
+ * the sizes in LDS: what num_layers rounds of gs_layer_sample + gs_layer_relabel give (the calls
+ * src/cuda/fusion/slice_sampling.cu:157 and src/cuda/tensor_ops.cu:46 of every layer), the frontier of a
+ * layer being the next one's seeds.  fanouts, layer_seeds (the draws' seed of every layer) and
+ * the arrays of device pointers are HOST arrays of num_layers: sub_indptr[l] (S_l + 1 slots, S_0 =
+ * num_seeds, S_l = the bound S_{l-1} * (1 + fanouts[l-1])), out_ids[l] (S_l * fanouts[l]),
+ * frontier[l] (S_l * (1 + fanouts[l])), data_out[l] (as out_ids, with edge_data; edge_ids may be
+ * NULL).  counts (device int64[2 * num_layers], may be NULL) and mailboxes / tickets (HOST arrays of
+ * 2 * num_layers, may be NULL): edges and frontier length of every layer; the lengths are -2 when
+ * a 64-bit id does not fit 32 bits.  gs_minibatch_applies: up to 8 layers of fanouts up to
+ * GS_FUSED_MAX_FANOUT, 2048 columns in the last layer and 8192 items at their bounds. */
+int gs_minibatch_applies(int64_t num_seeds, int num_layers, const int64_t* fanouts);
+int gs_minibatch_sample(const int64_t* indptr, int64_t num_cols, const void* indices,
+                        const void* seeds, int id_bytes, int64_t num_seeds, int num_layers,
+                        const int64_t* fanouts, int replace, const uint64_t* layer_seeds,
+                        const float* edge_data, const int64_t* edge_ids, int64_t* const* sub_indptr,
+                        void* const* out_ids, void* const* frontier, float* const* data_out,
+                        int64_t* counts, gs_mailbox* const* mailboxes, const int64_t* tickets,
+                        void* stream);
+
 /* B relabels in one pass ("super-batch"): replaces impl::BatchCSRRelabelCUDA
  * (src/cuda/batch_relabel.cu:331).  Batch b owns seeds[seeds_ptr[b]..seeds_ptr[b+1])
  * and ids[ids_ptr[b]..ids_ptr[b+1]) (both *_ptr: device int64[num_batches+1]).
