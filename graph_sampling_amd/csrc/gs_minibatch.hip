@@ -15,14 +15,13 @@
 // numbered from the frontier's length on, so ranks are smaller than every new item's number and
 // one atomic minimum keeps both.  Nothing is entered twice, and a layer needs no pass over the
 // nodes of the earlier ones.
+#include "gs_one.hpp"
 #include "gs_select.hpp"
 #include "gs_table.hpp"
 
 namespace gs {
 namespace {
 
-constexpr int kOneThreads = 1024;
-constexpr int kOneWaves = kOneThreads / kWave;
 constexpr int kOneMaxLayers = 8;
 constexpr int64_t kOneMaxItems = 8192;     // seeds and samples of the last layer, at their bound
 constexpr int kOneMaxSlots = 2 * kOneMaxItems;  // load <= 1/2: 128 KB
@@ -62,47 +61,6 @@ struct OneShared {
   int too_wide;
 };
 
-// A barrier that orders LDS only: the stores to the outputs, which no thread reads back, go on
-// under it (a full barrier waits until memory has acknowledged them).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-template <int CTRL, int ROWS>
-__device__ __forceinline__ int scan_step(int v) {
-  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
-}
-
-// Exclusive prefix of v over the workgroup and its total: one barrier, the wave part in lane
-// moves of the vector ALU.  `which` alternates from call to call (the two halves of s.scan).
-__device__ __forceinline__ int one_scan(int v, int* total, OneShared& s, int which) {
-  int incl = scan_step<0x111, 0xf>(v);  // from 1, 2, 4 and 8 lanes below in a row of 16
-  incl = scan_step<0x112, 0xf>(incl);
-  incl = scan_step<0x114, 0xf>(incl);
-  incl = scan_step<0x118, 0xf>(incl);
-  incl = scan_step<0x142, 0xa>(incl);   // row 0's sum to row 1, row 2's to row 3
-  incl = scan_step<0x143, 0xc>(incl);   // rows 0 and 1's to rows 2 and 3
-  const int wave = threadIdx.x / kWave;
-  if ((threadIdx.x & (kWave - 1)) == kWave - 1) s.scan[which][wave] = incl;
-  lds_barrier();
-  int before = 0, sum = 0;
-#pragma unroll
-  for (int w = 0; w < kOneWaves; ++w) {
-    const int t = s.scan[which][w];
-    before += w < wave ? t : 0;
-    sum += t;
-  }
-  *total = sum;
-  return before + incl - v;
-}
-
-template <typename IdT>
-__device__ __forceinline__ bool fits_slot(IdT id) {
-  return sizeof(IdT) == 4 || (static_cast<unsigned long long>(id) >> 32) == 0ull;
-}
-
 // The table's word of a node is its final one, (id << 32 | rank), for the items that are the
 // first of theirs: those take the next ranks, in the order of the items, and enter the frontier.
 // `flags`: bit u = the lane's item u is the first; key[u], slot[u]: where.
@@ -112,7 +70,7 @@ __device__ __forceinline__ void give_ranks(unsigned int flags, const uint32_t (&
                                            uint32_t* s_cols, int columns, IdT* frontier,
                                            int* unique, OneShared& s, int which) {
   int total;
-  int rank = *unique + one_scan(__popc(flags), &total, s, which);
+  int rank = *unique + one_scan(__popc(flags), &total, s.scan, which);
 #pragma unroll
   for (int u = 0; u < N; ++u) {
     if (flags >> u & 1u) {
@@ -183,7 +141,7 @@ __device__ __forceinline__ void one_layer(const OneArgs& a, int l, int S, int* u
       }
     }
     int total;
-    const int ex = one_scan(sub == 0 ? cnt : 0, &total, s, 0);
+    const int ex = one_scan(sub == 0 ? cnt : 0, &total, s.scan, 0);
     const int out = E + (sub == 0 ? ex : ex - cnt);  // the column's first output
     if (row < S && sub == 0) y.offsets[row] = out;
     uint32_t key[4], item[4], at[4];

@@ -26,6 +26,7 @@
 #include "gs_batch_items.hpp"
 #include <type_traits>
 
+#include "gs_one.hpp"
 #include "gs_table.hpp"
 
 GS_STAMPS_DEFINE(unique)
@@ -350,6 +351,159 @@ size_t workspace_bytes_for(int64_t M) {
          lookback_state_bytes(compact_num_tiles(M));
 }
 
+// ------------------------------------------------------------ one workgroup ----
+// The whole relabel of a short list by one workgroup in one launch: table, ranks and look-ups in
+// LDS.  Init, insert, compact and look-up are four launches of two or three dependent trips to
+// memory each, whatever the length; here the ids are read, and the results written.  Whole call in us, four
+// launches / one, ids of 233 k nodes: 64 items 21/12, 1383 28/14, 6000 32/21, 8192 37/33; beyond, at
+// more than half the table's slots, the chains of a few items hold up their waves (9700 30/39).
+constexpr int64_t kOneItems = 8 * kOneThreads;    // of the mapping: 8 a thread
+constexpr int64_t kOneQueries = 24 * kOneThreads;
+constexpr int kOneSlots = 16384;                  // 128 KB of LDS, load <= 1/2
+
+template <typename IdT, int PER>
+__global__ void __launch_bounds__(kOneThreads)
+unique_one_kernel(Spans<IdT> x, int M, int slots, Query qs, int Q, IdT* __restrict__ frontier,
+                  int64_t* __restrict__ num_unique, gs_mailbox* box, int64_t ticket) {
+  extern __shared__ unsigned long long s_dynamic[];
+  __shared__ int s_counts[PER * kOneWaves];
+  __shared__ int s_total, s_too_wide;
+  PackedTable t;
+  t.slots = s_dynamic;
+  t.mask = static_cast<uint32_t>(slots - 1);
+  t.shift = 64 - (31 - __clz(slots));
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  // item u of a thread is u * 1024 + the thread's number
+  IdT id[PER];
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int i = u * kOneThreads + static_cast<int>(threadIdx.x);
+    id[u] = x.get(i < M ? i : M - 1);
+  }
+  for (int i = threadIdx.x; i < slots; i += kOneThreads) t.slots[i] = ~0ull;
+  if (threadIdx.x == 0) s_too_wide = 0;
+  lds_barrier();
+  uint32_t at[PER];
+  unsigned int live = 0u;
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int i = u * kOneThreads + static_cast<int>(threadIdx.x);
+    at[u] = 0u;
+    if (i < M) {
+      if (fits_slot(id[u])) {
+        at[u] = t.template insert<true>(static_cast<long long>(static_cast<uint32_t>(id[u])),
+                                        static_cast<uint32_t>(i));
+        live |= 1u << u;
+      } else {
+        s_too_wide = 1;
+      }
+    }
+  }
+  lds_barrier();
+  // ranks: the first occurrences before the item, counted by 64 items of a wave
+  unsigned int first = 0u;
+  int ahead[PER];  // in the wave's 64
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const uint32_t i = static_cast<uint32_t>(u * kOneThreads) + threadIdx.x;
+    const bool is_first = (live >> u & 1u) && t.first_index(at[u]) == i;
+    const unsigned long long lanes = __ballot(is_first);
+    ahead[u] = __popcll(lanes & ((1ull << lane) - 1ull));
+    first |= static_cast<unsigned int>(is_first) << u;
+    if (lane == 0) s_counts[u * kOneWaves + wave] = __popcll(lanes);
+  }
+  lds_barrier();
+  if (wave == 0) {  // exclusive scan of the PER * 16 counts
+    constexpr int kEach = (PER * kOneWaves + kWave - 1) / kWave;
+    int c[kEach], mine = 0;
+#pragma unroll
+    for (int j = 0; j < kEach; ++j) {
+      const int e = lane * kEach + j;
+      c[j] = e < PER * kOneWaves ? s_counts[e] : 0;
+      mine += c[j];
+    }
+    const int incl = wave_inclusive_sum(mine);
+    int run = incl - mine;
+#pragma unroll
+    for (int j = 0; j < kEach; ++j) {
+      const int e = lane * kEach + j;
+      if (e < PER * kOneWaves) s_counts[e] = run;
+      run += c[j];
+    }
+    if (lane == kWave - 1) s_total = incl;
+  }
+  lds_barrier();
+  if (threadIdx.x == 0) {
+    const int64_t total = s_too_wide ? int64_t(-2) : int64_t(s_total);
+    *num_unique = total;
+    post_mailbox(box, total, ticket);
+  }
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    if (first >> u & 1u) {
+      const int rank = s_counts[u * kOneWaves + wave] + ahead[u];
+      t.slots[at[u]] = (static_cast<unsigned long long>(static_cast<uint32_t>(id[u])) << 32) |
+                       static_cast<uint32_t>(rank);
+      frontier[rank] = id[u];
+    }
+  }
+  if (Q == 0) return;
+  lds_barrier();
+  constexpr int kBatch = 4;
+  for (int j0 = threadIdx.x; j0 < Q; j0 += kBatch * kOneThreads) {
+    IdT key[kBatch];
+    IdT* to[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const int j = j0 + u * kOneThreads < Q ? j0 + u * kOneThreads : Q - 1;
+      int s = 0;
+      int64_t begin = 0;
+#pragma unroll
+      for (int q = 0; q < GS_MAX_SPANS - 1; ++q) {
+        if (q < qs.n - 1 && j >= qs.end[q]) {
+          s = q + 1;
+          begin = qs.end[q];
+        }
+      }
+      key[u] = static_cast<const IdT*>(qs.in[s])[j - begin];
+      to[u] = static_cast<IdT*>(qs.out[s]) + (j - begin);
+    }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      if (j0 + u * kOneThreads < Q) {
+        const int64_t rank =
+            fits_slot(key[u]) ? t.find(static_cast<long long>(static_cast<uint32_t>(key[u]))) : -1;
+        *to[u] = static_cast<IdT>(rank);
+      }
+    }
+  }
+}
+
+template <typename IdT>
+int unique_one(const Spans<IdT>& x, int64_t M, const Query& qs, int64_t Q, IdT* frontier,
+               int64_t* num_unique, gs_mailbox* box, int64_t ticket, hipStream_t st) {
+  int slots = 1024;
+  while (slots < 2 * M) slots <<= 1;  // (at most kOneSlots)
+  const size_t lds = static_cast<size_t>(slots) * 8;
+  auto* kernel = M <= kOneThreads       ? unique_one_kernel<IdT, 1>
+                 : M <= 2 * kOneThreads ? unique_one_kernel<IdT, 2>
+                 : M <= 4 * kOneThreads ? unique_one_kernel<IdT, 4>
+                                        : unique_one_kernel<IdT, 8>;
+  if (lds > 48 * 1024) {  // (per call: the attribute belongs to the device the call runs on)
+    const hipError_t allowed =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kOneSlots * 8);
+    if (allowed != hipSuccess) {
+      set_error_text("gs_unique_relabel: %s", hipGetErrorString(allowed));
+      return GS_ERR_LAUNCH;
+    }
+  }
+  ProfileScope prof("unique_one", st);
+  hipLaunchKernelGGL(kernel, dim3(1), dim3(kOneThreads), lds, st, x, static_cast<int>(M), slots, qs,
+                     static_cast<int>(Q), frontier, num_unique, box, ticket);
+  return check_launch("unique_relabel");
+}
+
 template <typename IdT, typename T>
 int unique_relabel_impl(const gs_span* mapping, int n_mapping, const gs_span* query,
                         void* const* query_out, int n_query, void* frontier, int64_t* num_unique,
@@ -406,6 +560,11 @@ int unique_relabel_impl(const gs_span* mapping, int n_mapping, const gs_span* qu
   }
   qs.n = n_query;
 
+  if constexpr (std::is_same<T, PackedTable>::value) {
+    if (M >= 1 && M <= kOneItems && Q <= kOneQueries && !last_span_len)
+      return unique_one<IdT>(x, M, qs, Q, static_cast<IdT*>(frontier), num_unique, box, box_ticket,
+                             stream);
+  }
   {
     ProfileScope prof("table_init", stream);
     const int64_t n_init = cap > tiles ? cap : tiles;

@@ -321,3 +321,33 @@ def test_relabel_behind_a_sampler_by_repeats(dev, idt, narrow, S, cap, held, spr
         assert int(num) == want.size
         assert np.array_equal(frontier[:want.size].cpu().numpy().astype(np.int64), want)
         assert np.array_equal(out[:held].cpu().numpy().astype(np.int64), w_out[0])
+
+
+@pytest.mark.parametrize("idt", [torch.int64, torch.int32])
+@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193])
+def test_short_lists_by_one_workgroup_and_past_them(dev, idt, n):
+    """Around the numbers of items a thread of the one-workgroup relabel takes, and its limit: all
+    items distinct, hubs, all the same; four spans, two queries with ids that are not there."""
+    rng = np.random.default_rng(n)
+    for ids in (rng.permutation(4 * n)[:n], rng.integers(0, max(2, n // 20), n), np.full(n, 77)):
+        ids = ids.astype(np.int64)
+        cuts = np.sort(rng.integers(0, n + 1, 3))
+        spans = np.split(ids, cuts)
+        queries = [spans[3], rng.integers(0, 5 * n, 3000).astype(np.int64)]
+        want_frontier, want = O.relabel(spans, queries)
+        frontier, num, outs = capi.unique_relabel([to_dev(s, dev, idt) for s in spans],
+                                                  [to_dev(q, dev, idt) for q in queries],
+                                                  narrow=idt == torch.int64)
+        assert int(num.item()) == want_frontier.size
+        assert np.array_equal(frontier[:want_frontier.size].cpu().numpy().astype(np.int64), want_frontier)
+        for got, w in zip(outs, want):
+            assert np.array_equal(got.cpu().numpy().astype(np.int64), w)
+
+
+def test_short_list_with_an_id_beyond_32_bits(dev):
+    ids = torch.tensor([3, 1, 3, (1 << 40) + 1], dtype=torch.int64, device=dev)
+    assert int(capi.unique_relabel([ids], [ids], narrow=True)[1].item()) == -2
+    # as a query it is an id that is not there, whatever its lower half says
+    frontier, num, (out,) = capi.unique_relabel([ids[:3].contiguous()], [ids], narrow=True)
+    assert int(num.item()) == 2 and out.tolist() == [0, 1, 0, -1]
+    assert capi.unique_relabel([ids], [ids])[2][0].tolist() == [0, 1, 0, 2]
