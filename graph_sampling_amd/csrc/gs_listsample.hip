@@ -122,9 +122,10 @@ __device__ __forceinline__ uint32_t class_of(uint32_t okey, int64_t i, int run_s
              : static_cast<uint32_t>(kKeyBins) + (okey >> 21);
 }
 
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kPassThreads)
 select_init_kernel(uint32_t* hist, SelectCounters* st) {
-  for (int i = threadIdx.x; i < kClasses; i += kThreads) hist[i] = 0;
+  static_assert(kClasses == 4 * kPassThreads, "four classes a thread");
+  reinterpret_cast<uint4*>(hist)[threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);
   if (threadIdx.x < kLists) {
     st->above[threadIdx.x] = 0;
     st->ties[threadIdx.x] = 0;
@@ -527,7 +528,7 @@ int list_weighted_impl(const void* data, const float* probs, int64_t n, int64_t 
   const unsigned grid = static_cast<unsigned>(tiles < 256 ? (tiles < 1 ? 1 : tiles) : 256);
   int run_shift = 0;
   while (((n - 1) >> run_shift) >= kKeyBins) ++run_shift;
-  hipLaunchKernelGGL(select_init_kernel, dim3(1), dim3(kThreads), 0, st, s.hist, s.state);
+  hipLaunchKernelGGL(select_init_kernel, dim3(1), dim3(kPassThreads), 0, st, s.hist, s.state);
   hipLaunchKernelGGL(keys_hist_kernel, dim3(grid), dim3(kPassThreads), 0, st, probs, n, run_shift,
                      k, seed, replay, s.okey, s.hist, s.state);
   hipLaunchKernelGGL(partition_kernel, dim3(grid), dim3(kPassThreads), 0, st, s.okey, n, run_shift,

@@ -820,79 +820,115 @@ int segment_normalize_impl(const int64_t* indptr, const int64_t* emap, const flo
 // add per distinct target: a 300 000-edge hub costs 150 global adds instead of 300 000.  The
 // adds are the hardware's fp32 adds, not the compare-and-swap loop a plain atomicAdd(float*)
 // compiles to here.
-constexpr int kAggEdges = 8;                   // edges per thread
-constexpr int kAggTile = kThreads * kAggEdges;
-constexpr int kAggSlots = 2 * kAggTile;        // LDS table: load <= 1/2
+constexpr int kAggEdges = 8;  // edges per thread
 
+// Few edges are spread over more workgroups, two a thread: the launch is then a handful of trips
+// to memory and an LDS table to clear, which a shorter tile has less of (22 k edges 16 -> 6 us).
+// Every target of a tile costs an addition to memory, so that from 2^17 edges on longer tiles win.
+constexpr int kAggFewEdges = 2;
+constexpr int64_t kAggFew = int64_t(1) << 17;
+
+template <int EDGES>
 struct KeyedSums {
-  long long key[kAggSlots];
-  float sum[kAggSlots];
+  static constexpr int kSlots = 2 * kThreads * EDGES;  // load <= 1/2
+  long long key[kSlots];
+  float sum[kSlots];
 };
 
-__device__ __forceinline__ void keyed_clear(KeyedSums& t) {
-  for (int i = threadIdx.x; i < kAggSlots; i += kThreads) {
+template <int EDGES>
+__device__ __forceinline__ void keyed_clear(KeyedSums<EDGES>& t) {
+  for (int i = threadIdx.x; i < t.kSlots; i += kThreads) {
     t.key[i] = -1;
     t.sum[i] = 0.0f;
   }
   __syncthreads();
 }
 
-__device__ __forceinline__ void keyed_add(KeyedSums& t, long long key, float v) {
+template <int EDGES>
+__device__ __forceinline__ void keyed_add(KeyedSums<EDGES>& t, long long key, float v) {
   unsigned int h = static_cast<unsigned int>((static_cast<unsigned long long>(key) *
-                                              0x9E3779B97F4A7C15ull) >> 40) & (kAggSlots - 1);
+                                              0x9E3779B97F4A7C15ull) >> 40) & (t.kSlots - 1);
   while (true) {
     const long long seen = static_cast<long long>(
         atomicCAS(reinterpret_cast<unsigned long long*>(&t.key[h]), ~0ull,
                   static_cast<unsigned long long>(key)));
     if (seen == -1 || seen == key) break;
-    h = (h + 1) & (kAggSlots - 1);
+    h = (h + 1) & (t.kSlots - 1);
   }
   unsafeAtomicAdd(&t.sum[h], v);
 }
 
 // (a key outside [0, bound) is left out)
-__device__ __forceinline__ void keyed_flush(KeyedSums& t, float* __restrict__ out,
+template <int EDGES>
+__device__ __forceinline__ void keyed_flush(KeyedSums<EDGES>& t, float* __restrict__ out,
                                             long long bound = 0x7FFFFFFFFFFFFFFFll) {
   __syncthreads();
-  for (int i = threadIdx.x; i < kAggSlots; i += kThreads)
+  for (int i = threadIdx.x; i < t.kSlots; i += kThreads)
     if (t.key[i] >= 0 && t.key[i] < bound) unsafeAtomicAdd(out + t.key[i], t.sum[i]);
 }
 
 // out[target[e]] += f(data[emap ? emap[e] : e])   (graph_ops.cu:45-64)
-template <typename IdT>
+// (a thread's reads go out together, clamped to the last edge, before its first addition: one
+// edge at a time every addition waits for its own trips to memory)
+template <typename IdT, int EDGES>
 __global__ void __launch_bounds__(kThreads)
 coo_sum_kernel(const IdT* __restrict__ target, const int64_t* __restrict__ emap,
                const float* __restrict__ data, int64_t E, int powk, float* __restrict__ out,
-               int64_t bound) {
-  __shared__ KeyedSums table;
-  keyed_clear(table);
-  const int64_t base = static_cast<int64_t>(blockIdx.x) * kAggTile + threadIdx.x;
+               long long bound) {
+  __shared__ KeyedSums<EDGES> table;
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * (kThreads * EDGES) + threadIdx.x;
+  IdT to[EDGES];
+  int64_t at[EDGES];
+  float v[EDGES];
 #pragma unroll
-  for (int k = 0; k < kAggEdges; ++k) {
+  for (int k = 0; k < EDGES; ++k) {
     const int64_t e = base + static_cast<int64_t>(k) * kThreads;
-    if (e < E)
-      keyed_add(table, static_cast<long long>(target[e]),
-                powk_f(data[emap ? emap[e] : e], powk));
+    at[k] = e < E ? e : E - 1;
+    to[k] = target[at[k]];
+  }
+  if (emap) {
+#pragma unroll
+    for (int k = 0; k < EDGES; ++k) at[k] = emap[at[k]];
+  }
+#pragma unroll
+  for (int k = 0; k < EDGES; ++k) v[k] = data[at[k]];
+  keyed_clear(table);
+#pragma unroll
+  for (int k = 0; k < EDGES; ++k) {
+    if (base + static_cast<int64_t>(k) * kThreads < E)
+      keyed_add(table, static_cast<long long>(to[k]), powk_f(v[k], powk));
   }
   keyed_flush(table, out, bound);
 }
 
 // edge_map_reduce.cu:15-23
-template <typename IdT>
+template <typename IdT, int EDGES>
 __global__ void __launch_bounds__(kThreads)
 e_div_u_sum_kernel(const IdT* __restrict__ row, const IdT* __restrict__ col,
                    const float* __restrict__ data, const float* __restrict__ divisor, int64_t E,
                    float* __restrict__ out_data, float* __restrict__ out_sum) {
-  __shared__ KeyedSums table;
-  keyed_clear(table);
-  const int64_t base = static_cast<int64_t>(blockIdx.x) * kAggTile + threadIdx.x;
+  __shared__ KeyedSums<EDGES> table;
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * (kThreads * EDGES) + threadIdx.x;
+  IdT from[EDGES], to[EDGES];
+  float v[EDGES], d[EDGES];
 #pragma unroll
-  for (int k = 0; k < kAggEdges; ++k) {
+  for (int k = 0; k < EDGES; ++k) {
+    const int64_t e = base + static_cast<int64_t>(k) * kThreads;
+    const int64_t at = e < E ? e : E - 1;
+    from[k] = row[at];
+    to[k] = col[at];
+    v[k] = data[at];
+  }
+#pragma unroll
+  for (int k = 0; k < EDGES; ++k) d[k] = divisor[from[k]];
+  keyed_clear(table);
+#pragma unroll
+  for (int k = 0; k < EDGES; ++k) {
     const int64_t e = base + static_cast<int64_t>(k) * kThreads;
     if (e < E) {
-      const float v = data[e] / divisor[row[e]];
-      out_data[e] = v;
-      keyed_add(table, static_cast<long long>(col[e]), v);
+      v[k] /= d[k];
+      out_data[e] = v[k];
+      keyed_add(table, static_cast<long long>(to[k]), v[k]);
     }
   }
   keyed_flush(table, out_sum);
@@ -946,16 +982,19 @@ int gs::coo_sum_bounded(const void* target, int id_bytes, const int64_t* e_ids, 
   GS_REQUIRE(E == 0 || (target && data && out), "gs_coo_sum: null pointer");
   GS_REQUIRE(valid_id_bytes(id_bytes), "gs_coo_sum: id_bytes must be 4 or 8, got %d", id_bytes);
   if (E == 0) return GS_OK;
-  const dim3 grid(blocks_for(E, kAggTile));
+  const bool few = E < kAggFew;
+  const dim3 grid(blocks_for(E, kThreads * (few ? kAggFewEdges : kAggEdges)));
   hipStream_t st = static_cast<hipStream_t>(stream);
+  auto launch = [&](auto* kernel, const auto* to) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, st, to, e_ids, data, E,
+                       static_cast<int>(powk), out, static_cast<long long>(num_targets));
+  };
   if (id_bytes == 8)
-    hipLaunchKernelGGL(coo_sum_kernel<int64_t>, grid, dim3(kThreads), 0, st,
-                       static_cast<const int64_t*>(target), e_ids, data, E, static_cast<int>(powk),
-                       out, num_targets);
+    launch(few ? coo_sum_kernel<int64_t, kAggFewEdges> : coo_sum_kernel<int64_t, kAggEdges>,
+           static_cast<const int64_t*>(target));
   else
-    hipLaunchKernelGGL(coo_sum_kernel<int32_t>, grid, dim3(kThreads), 0, st,
-                       static_cast<const int32_t*>(target), e_ids, data, E, static_cast<int>(powk),
-                       out, num_targets);
+    launch(few ? coo_sum_kernel<int32_t, kAggFewEdges> : coo_sum_kernel<int32_t, kAggEdges>,
+           static_cast<const int32_t*>(target));
   return check_launch("coo_sum");
 }
 
@@ -988,16 +1027,19 @@ int gs_e_div_u_sum(const void* row, const void* col, int id_bytes, const float* 
              "gs_e_div_u_sum: null pointer");
   GS_REQUIRE(valid_id_bytes(id_bytes), "gs_e_div_u_sum: id_bytes must be 4 or 8, got %d", id_bytes);
   if (E == 0) return GS_OK;
-  const dim3 grid(blocks_for(E, kAggTile));
+  const bool few = E < kAggFew;
+  const dim3 grid(blocks_for(E, kThreads * (few ? kAggFewEdges : kAggEdges)));
   hipStream_t st = static_cast<hipStream_t>(stream);
+  auto launch = [&](auto* kernel, const auto* from, const auto* to) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, st, from, to, data, divisor, E, out_data,
+                       out_sum);
+  };
   if (id_bytes == 8)
-    hipLaunchKernelGGL(e_div_u_sum_kernel<int64_t>, grid, dim3(kThreads), 0, st,
-                       static_cast<const int64_t*>(row), static_cast<const int64_t*>(col), data,
-                       divisor, E, out_data, out_sum);
+    launch(few ? e_div_u_sum_kernel<int64_t, kAggFewEdges> : e_div_u_sum_kernel<int64_t, kAggEdges>,
+           static_cast<const int64_t*>(row), static_cast<const int64_t*>(col));
   else
-    hipLaunchKernelGGL(e_div_u_sum_kernel<int32_t>, grid, dim3(kThreads), 0, st,
-                       static_cast<const int32_t*>(row), static_cast<const int32_t*>(col), data,
-                       divisor, E, out_data, out_sum);
+    launch(few ? e_div_u_sum_kernel<int32_t, kAggFewEdges> : e_div_u_sum_kernel<int32_t, kAggEdges>,
+           static_cast<const int32_t*>(row), static_cast<const int32_t*>(col));
   return check_launch("e_div_u_sum");
 }
 

@@ -271,6 +271,32 @@ def test_coo_sum_binned_leaves_out_targets_beyond_the_output(dev, edges):
     assert bool((buf[targets:] == 7.0).all())
 
 
+@pytest.mark.parametrize("idt", ID_DTYPES)
+@pytest.mark.parametrize("edges", [1, 511, 513, (1 << 17) - 1, 1 << 17, (1 << 17) + 1])
+def test_keyed_sums_at_both_lengths_of_a_tile(dev, idt, edges):
+    """Two edges a thread below 2^17 edges, eight from there on; every edge once, hubs and all."""
+    rng = np.random.default_rng(edges)
+    n = 3000
+    row = (rng.random(edges) ** 3 * n).astype(np.int64)
+    col = (rng.random(edges) ** 3 * n).astype(np.int64)
+    data = rng.random(edges, dtype=np.float32) + 0.25
+    divisor = rng.random(n, dtype=np.float32) + 0.5
+    e_ids = rng.permutation(edges)
+    out = torch.zeros(n, dtype=torch.float32, device=dev)
+    capi.coo_sum(to_dev(row, dev, idt), to_dev(e_ids, dev), to_dev(data, dev), 2, out)
+    # (positive float32 terms in any order: relative error of a few times 2^-24 a level of additions)
+    want = np.bincount(row, weights=data[e_ids].astype(np.float64) ** 2, minlength=n)
+    np.testing.assert_allclose(out.cpu().numpy(), want, rtol=2e-5)
+    od = torch.empty(edges, dtype=torch.float32, device=dev)
+    osum = torch.zeros(n, dtype=torch.float32, device=dev)
+    capi.e_div_u_sum(to_dev(row, dev, idt), to_dev(col, dev, idt), to_dev(data, dev),
+                     to_dev(divisor, dev), od, osum)
+    assert np.array_equal(od.cpu().numpy(), data / divisor[row])
+    np.testing.assert_allclose(osum.cpu().numpy(),
+                               np.bincount(col, weights=(data / divisor[row]).astype(np.float64), minlength=n),
+                               rtol=2e-5)
+
+
 # ------------------------------------------------------------------ SDDMM
 def _sddmm_coo_gpu(dev, op, row, col, e_ids, lhs, rhs, lt, rt, idt=torch.int64):
     ls = lhs.shape if lhs.ndim > 1 else lhs.shape + (1,)
