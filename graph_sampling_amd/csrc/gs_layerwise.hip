@@ -240,10 +240,8 @@ struct LoadCounts {
 template <typename IdT>
 __global__ void __launch_bounds__(256)
 column_offsets_kernel(const IdT* __restrict__ kept_key, int64_t kept, int node_bits,
-                      int64_t num_cols, int64_t* __restrict__ out_indptr,
-                      unsigned int* __restrict__ num_long) {
+                      int64_t num_cols, int64_t* __restrict__ out_indptr) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i == 0) *num_long = 0u;  // (the list of long columns is made by the next launch)
   if (kept == 0) {
     for (int64_t c = i; c <= num_cols; c += static_cast<int64_t>(gridDim.x) * 256) out_indptr[c] = 0;
     return;
@@ -256,118 +254,106 @@ column_offsets_kernel(const IdT* __restrict__ kept_key, int64_t kept, int node_b
     for (int64_t k = c + 1; k <= num_cols; ++k) out_indptr[k] = kept;
 }
 
-// One workgroup per column puts the kept edges of its column in the order of (new row,
-// position) -- the order of a stable sort of all kept edges by key, which for a few tens of
-// thousands of edges is three radix passes of two launches each -- by a counting sort in LDS:
-// a histogram over the 2^node_bits places, its scan, then the edges in their own order, 4096
-// at a time: a wave walks them 64 at a time, a lane finds the lanes that hold the same place
-// with one ballot per key bit and takes the bin's next free places in lane order; then all
-// lanes write row id and value data / divisor[row] to where the edges go.  Work grows with the
-// column's length, not its square: the hubs among a layer's seeds keep tens of thousands of
-// edges (parallel edges included), most columns a few dozen.  FOUR_WAVES (up to 2048 places):
-// each wave walks a quarter of the 4096 and counts per place in 16-bit counters of its own; an
-// edge's place is the bin's start + the counts of the quarters before its own + its rank
-// inside its quarter.
-constexpr int kColumnStage = 4096;
-constexpr int kColumnBatch = 4;
-constexpr int kFourWavesBits = 11;
-constexpr int kRankShift = 13;  // a key has at most 13 bits, a rank inside a quarter 12
-
+// The kept edges of every column in the order of (new row, position) -- the order of a stable
+// sort of all kept edges by key, which for a few tens of thousands of edges is three radix passes
+// of two launches each -- and their values data / divisor[row].  Two kinds of workgroups in one
+// launch, both bound by the dependent trips to memory of one workgroup (position, row, divisor):
+//  * columns of up to kShortColumn kept edges (nearly all) by edge: a thread counts the edges of
+//    its column that come before its own, among keys that the workgroup has staged in LDS (read
+//    from memory one after another they were most of 14 us for 871 edges);
+//  * the longer ones (hub seeds, parallel edges included) a workgroup each, by a counting sort in
+//    LDS, 4096 edges at a time: a wave walks its share 64 edges at a time, a lane finds the lanes
+//    that hold the same place with one ballot per key bit, and counts per place in 16-bit
+//    counters of the wave's own; an edge's place is the bin's start + the counts of the waves before
+//    its own + its rank in its wave.  A column that fits one round of 4096 gets the bins'
+//    starts from those counters, a longer one from a histogram of all of it beforehand.
+// 512 columns, 871 edges: 14 -> 8 us; 1024 columns, 68 k edges, 82 of them long, up to 3004: 29 ->
+// 18 us (from 256 threads a workgroup, the long columns listed by a launch of their own).
 constexpr int kShortColumn = 256;
+constexpr int kOrderThreads = 1024;
+constexpr int kOrderWaves = kOrderThreads / kWave;
+constexpr int kColumnPer = 4;  // edges of a thread in a round
+constexpr int kColumnStage = kOrderThreads * kColumnPer;
+constexpr int kShortStage = kOrderThreads + 2 * (kShortColumn - 1);
 
-// The columns with more than kShortColumn kept edges, listed for the workgroups that order them
-// in LDS (a thread a column).
-__global__ void __launch_bounds__(256)
-long_columns_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
-                    unsigned int* __restrict__ num_long, unsigned int* __restrict__ long_columns) {
-  const int64_t c = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (c < num_cols && indptr[c + 1] - indptr[c] > kShortColumn)
-    long_columns[atomicAdd(num_long, 1u)] = static_cast<unsigned int>(c);
-}
+// waves that count: as many as leave room for two workgroups a compute unit (one with 8192 places)
+inline int order_groups(int node_bits) { return node_bits <= 10 ? 16 : (node_bits == 11 ? 8 : 4); }
 
-// The short columns (up to 256 kept edges: nearly all of them) by edge: a thread takes one kept
-// edge, finds its column's range in the offsets, and counts the column's edges that come before
-// its own by (key, position) -- the keys of a column lie side by side and the threads of a
-// column read the same ones, out of the caches.  (A workgroup per column, long or short, cost
-// 116 us for 82 k edges over 40 k columns: tens of thousands of workgroups with two edges each.)
 template <typename IdT>
-__device__ __forceinline__ void order_short_edge(int64_t i, const IdT* __restrict__ kept_key,
-                                                 const IdT* __restrict__ kept_pos, int node_bits,
-                                                 const int64_t* __restrict__ indptr,
-                                                 const IdT* __restrict__ row,
-                                                 const float* __restrict__ data,
-                                                 const float* __restrict__ divisor,
-                                                 IdT* __restrict__ out_row,
-                                                 float* __restrict__ out_value) {
-  const unsigned long long key = static_cast<unsigned long long>(kept_key[i]);
-  const int64_t e = static_cast<int64_t>(kept_pos[i]);
-  const int64_t column = static_cast<int64_t>(key >> node_bits);
+__device__ __forceinline__ void order_short_edges(int64_t first, int64_t kept,
+                                                  const IdT* __restrict__ kept_key,
+                                                  const IdT* __restrict__ kept_pos, int node_bits,
+                                                  const int64_t* __restrict__ indptr,
+                                                  const IdT* __restrict__ row,
+                                                  const float* __restrict__ data,
+                                                  const float* __restrict__ divisor,
+                                                  IdT* __restrict__ out_row,
+                                                  float* __restrict__ out_value, IdT* s_keys) {
+  // the keys of every column of up to 256 edges that has one among first .. first + 1023
+  const int64_t from = first < kShortColumn - 1 ? 0 : first - (kShortColumn - 1);
+  const int64_t to = first + kOrderThreads + kShortColumn - 1 < kept
+                         ? first + kOrderThreads + kShortColumn - 1 : kept;
+  const int64_t i = first + threadIdx.x;
+  const int64_t mine = i < kept ? i : kept - 1;
+  const IdT key = kept_key[mine];
+  const int64_t e = static_cast<int64_t>(kept_pos[mine]);
+  for (int64_t j = from + threadIdx.x; j < to; j += kOrderThreads) s_keys[j - from] = kept_key[j];
+  const int64_t column = static_cast<int64_t>(key) >> node_bits;
   const int64_t lo = indptr[column], hi = indptr[column + 1];
-  if (hi - lo > kShortColumn) return;  // (a long column: its own workgroup's)
   const IdT r = row[e];
   const float w = data ? data[e] : 1.0f;
   const float d = divisor[r];
-  int64_t before = 0;
-  for (int64_t j = lo; j < hi; ++j) {
-    const unsigned long long y = static_cast<unsigned long long>(kept_key[j]);
-    before += (y < key) || (y == key && j < i);  // (one column: the keys differ in the place only)
+  __syncthreads();
+  if (i >= kept || hi - lo > kShortColumn) return;  // (a long column: its own workgroup's)
+  int before = 0;
+  const int at = static_cast<int>(i - from), end = static_cast<int>(hi - from);
+#pragma unroll 8
+  for (int j = static_cast<int>(lo - from); j < end; ++j) {
+    const IdT y = s_keys[j];
+    before += (y < key) || (y == key && j < at);  // (one column: the keys differ in the place only)
   }
   out_row[lo + before] = r;
   out_value[lo + before] = w / d;
 }
 
-template <typename IdT, bool FOUR_WAVES>
-__global__ void __launch_bounds__(256)
+template <typename IdT, int GROUPS>
+__global__ void __launch_bounds__(kOrderThreads)
 order_columns_kernel(const IdT* __restrict__ kept_key, const IdT* __restrict__ kept_pos,
                      int node_bits, const int64_t* __restrict__ indptr,
                      const IdT* __restrict__ row, const float* __restrict__ data,
                      const float* __restrict__ divisor, IdT* __restrict__ out_row,
-                     float* __restrict__ out_value, const unsigned int* __restrict__ num_long,
-                     const unsigned int* __restrict__ long_columns, unsigned int long_blocks,
-                     int64_t kept) {
+                     float* __restrict__ out_value, unsigned int long_blocks, int64_t kept) {
   extern __shared__ unsigned long long s_raw[];
-  __shared__ int64_t s_scan[256 / kWave + 1];
-  // the launch's first long_blocks workgroups take a listed long column each, the others 256
-  // kept edges of short columns: both kinds run side by side
+  __shared__ int64_t s_scan[kOrderWaves + 1];
   if (blockIdx.x >= long_blocks) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x - long_blocks) * 256 + threadIdx.x;
-    if (i < kept)
-      order_short_edge(i, kept_key, kept_pos, node_bits, indptr, row, data, divisor, out_row,
-                       out_value);
+    order_short_edges(static_cast<int64_t>(blockIdx.x - long_blocks) * kOrderThreads, kept, kept_key,
+                      kept_pos, node_bits, indptr, row, data, divisor, out_row, out_value,
+                      reinterpret_cast<IdT*>(s_raw));
     return;
   }
-  if (blockIdx.x >= *num_long) return;
-  const unsigned int column = long_columns[blockIdx.x];
+  // The launch's first workgroups: number b takes the column of the kept edge b * 257, if it is a
+  // long one and that is the first such edge in it (a column of 257 edges or more has one).
+  const int64_t probe = static_cast<int64_t>(blockIdx.x) * (kShortColumn + 1);
+  const int64_t column = static_cast<int64_t>(kept_key[probe]) >> node_bits;
   const int64_t lo = indptr[column], hi = indptr[column + 1];
   const int64_t len = hi - lo;
+  if (len <= kShortColumn || probe - (kShortColumn + 1) >= lo) return;
   const int places = 1 << node_bits;
   const unsigned int mask = static_cast<unsigned int>(places) - 1u;
   unsigned int* s_bin = reinterpret_cast<unsigned int*>(s_raw);
-  unsigned int* s_key = s_bin + places;
-  for (int j = threadIdx.x; j < places; j += 256) s_bin[j] = 0u;
-  __syncthreads();
-  // (here and below a thread's reads go out four at a time, clamped to the column, before the
-  // first of them is used: one at a time each waits a whole trip to memory)
-  for (int64_t j0 = threadIdx.x; j0 < len; j0 += 256 * kColumnBatch) {
-    unsigned int k[kColumnBatch];
-#pragma unroll
-    for (int u = 0; u < kColumnBatch; ++u) {
-      const int64_t j = j0 + u * 256;
-      k[u] = static_cast<unsigned int>(kept_key[lo + (j < len ? j : len - 1)]) & mask;
-    }
-#pragma unroll
-    for (int u = 0; u < kColumnBatch; ++u)
-      if (j0 + u * 256 < len) atomicAdd(&s_bin[k[u]], 1u);
-  }
-  __syncthreads();
-  {  // exclusive scan of the bins: a thread owns `per` consecutive ones
-    const int per = places > 256 ? places / 256 : 1;
+  unsigned int* s_key = s_bin + (places < 4 ? 4 : places);  // (all three 16-byte aligned)
+  unsigned short* s_count = reinterpret_cast<unsigned short*>(s_key + kColumnStage);
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const bool one_round = len <= kColumnStage;
+  // exclusive scan of the bins: a thread owns `per` consecutive ones
+  const int per = places > kOrderThreads ? places / kOrderThreads : 1;
+  auto scan_bins = [&]() {
     const int first = threadIdx.x * per;
     int64_t mine = 0;
     for (int u = 0; u < per; ++u)
       if (first + u < places) mine += s_bin[first + u];
     int64_t total;
-    int64_t at = block_exclusive_scan<256>(mine, &total, s_scan);
+    int64_t at = block_exclusive_scan<kOrderThreads>(mine, &total, s_scan);
     for (int u = 0; u < per; ++u) {
       if (first + u < places) {
         const unsigned int n = s_bin[first + u];
@@ -375,38 +361,62 @@ order_columns_kernel(const IdT* __restrict__ kept_key, const IdT* __restrict__ k
         at += n;
       }
     }
+    __syncthreads();
+  };
+  if (!one_round) {
+    for (int j = threadIdx.x; j < places; j += kOrderThreads) s_bin[j] = 0u;
+    __syncthreads();
+    for (int64_t j0 = threadIdx.x; j0 < len; j0 += kColumnStage) {
+      unsigned int k[kColumnPer];
+#pragma unroll
+      for (int u = 0; u < kColumnPer; ++u) {
+        const int64_t j = j0 + u * kOrderThreads;
+        k[u] = static_cast<unsigned int>(kept_key[lo + (j < len ? j : len - 1)]) & mask;
+      }
+#pragma unroll
+      for (int u = 0; u < kColumnPer; ++u)
+        if (j0 + u * kOrderThreads < len) atomicAdd(&s_bin[k[u]], 1u);
+    }
+    __syncthreads();
+    scan_bins();
   }
-  __syncthreads();
-  const int lane = threadIdx.x & (kWave - 1);
   // without data every value is one; the read then goes to a word that is always there
   const bool has_data = data != nullptr;
   const float* values = has_data ? data : divisor;
   for (int64_t base = 0; base < len; base += kColumnStage) {
     const int n = static_cast<int>(len - base < kColumnStage ? len - base : kColumnStage);
-    for (int j0 = threadIdx.x; j0 < n; j0 += 256 * kColumnBatch) {
-      unsigned int k[kColumnBatch];
+    // everything a thread's edges need from memory is on its way while they are ranked
+    unsigned int key[kColumnPer];
+    int64_t e[kColumnPer];
+    IdT r[kColumnPer];
+    float w[kColumnPer], d[kColumnPer];
 #pragma unroll
-      for (int u = 0; u < kColumnBatch; ++u) {
-        const int j = j0 + u * 256;
-        k[u] = static_cast<unsigned int>(kept_key[lo + base + (j < n ? j : n - 1)]) & mask;
-      }
+    for (int u = 0; u < kColumnPer; ++u) {
+      const int j = static_cast<int>(threadIdx.x) + u * kOrderThreads;
+      const int64_t at = lo + base + (j < n ? j : n - 1);
+      key[u] = static_cast<unsigned int>(kept_key[at]) & mask;
+      e[u] = static_cast<int64_t>(kept_pos[at]);
+    }
+    for (int j = threadIdx.x; j < GROUPS * places / 8; j += kOrderThreads)
+      reinterpret_cast<uint4*>(s_count)[j] = make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
-      for (int u = 0; u < kColumnBatch; ++u)
-        if (j0 + u * 256 < n) s_key[j0 + u * 256] = k[u];
+    for (int u = 0; u < kColumnPer; ++u) {
+      const int j = static_cast<int>(threadIdx.x) + u * kOrderThreads;
+      if (j < n) s_key[j] = key[u];
     }
-    if (FOUR_WAVES) {
-      unsigned int* zero = s_key + kColumnStage;  // the four waves' counters: 2 * places words
-      for (int j = threadIdx.x; j < 2 * places; j += 256) zero[j] = 0u;
-    }
+#pragma unroll
+    for (int u = 0; u < kColumnPer; ++u) r[u] = row[e[u]];
+#pragma unroll
+    for (int u = 0; u < kColumnPer; ++u) w[u] = values[has_data ? e[u] : 0];
+#pragma unroll
+    for (int u = 0; u < kColumnPer; ++u) d[u] = divisor[r[u]];
     __syncthreads();
-    if (FOUR_WAVES) {
-      unsigned short* s_count = reinterpret_cast<unsigned short*>(s_key + kColumnStage);
-      const int wave = threadIdx.x / kWave;
-      const int quarter = ((n + 4 * kWave - 1) / (4 * kWave)) * kWave;
-      const int q_hi = (wave + 1) * quarter < n ? (wave + 1) * quarter : n;
+    const int share = ((n + GROUPS * kWave - 1) / (GROUPS * kWave)) * kWave;  // edges of a wave
+    if (wave < GROUPS) {
+      const int end = (wave + 1) * share < n ? (wave + 1) * share : n;
       unsigned short* mine = s_count + wave * places;
-      for (int c = wave * quarter; c < q_hi; c += kWave) {
-        const bool valid = c + lane < q_hi;
+      for (int c = wave * share; c < end; c += kWave) {
+        const bool valid = c + lane < end;
         const unsigned int k = valid ? s_key[c + lane] : 0u;
         unsigned long long peers = __ballot(valid);
         for (int b = 0; b < node_bits; ++b) {
@@ -417,98 +427,76 @@ order_columns_kernel(const IdT* __restrict__ kept_key, const IdT* __restrict__ k
         if (valid) {
           const unsigned int ahead = __popcll(peers & ((1ull << lane) - 1ull));
           const unsigned int start = mine[k];
-          s_key[c + lane] = k | ((start + ahead) << kRankShift);
+          s_key[c + lane] = start + ahead;  // the edge's rank in its wave's share
           if (lane == 63 - __clzll(peers))
             mine[k] = static_cast<unsigned short>(start + __popcll(peers));
         }
       }
-      __syncthreads();
-      for (int j = threadIdx.x; j < n; j += 256) {
-        const unsigned int v = s_key[j];
-        const unsigned int k = v & ((1u << kRankShift) - 1u);
-        unsigned int place = s_bin[k] + (v >> kRankShift);
-        const int w = j / quarter;
-        for (int before = 0; before < w; ++before) place += s_count[before * places + k];
-        s_key[j] = place;
-      }
-      __syncthreads();
-      for (int k = threadIdx.x; k < places; k += 256)
-        s_bin[k] += static_cast<unsigned int>(s_count[k]) + s_count[places + k] +
-                    s_count[2 * places + k] + s_count[3 * places + k];
-    } else if (threadIdx.x < kWave) {
-      for (int c = 0; c < n; c += kWave) {
-        const bool valid = c + lane < n;
-        const unsigned int k = valid ? s_key[c + lane] : 0u;
-        unsigned long long peers = __ballot(valid);
-        for (int b = 0; b < node_bits; ++b) {
-          const bool bit = (k >> b) & 1u;
-          const unsigned long long with_bit = __ballot(valid && bit);
-          peers &= bit ? with_bit : ~with_bit;
-        }
-        if (valid) {
-          const int ahead = __popcll(peers & ((1ull << lane) - 1ull));
-          const unsigned int start = s_bin[k];
-          s_key[c + lane] = start + static_cast<unsigned int>(ahead);  // the edge's place
-          if (lane == 63 - __clzll(peers)) s_bin[k] = start + static_cast<unsigned int>(__popcll(peers));
-        }
-      }
     }
     __syncthreads();
-    for (int j0 = threadIdx.x; j0 < n; j0 += 256 * kColumnBatch) {
-      int64_t e[kColumnBatch];
-      IdT r[kColumnBatch];
-      float w[kColumnBatch], d[kColumnBatch];
+    if (one_round) {
+      for (int k = threadIdx.x; k < places; k += kOrderThreads) {
+        unsigned int total = 0u;
 #pragma unroll
-      for (int u = 0; u < kColumnBatch; ++u) {
-        const int j = j0 + u * 256;
-        e[u] = static_cast<int64_t>(kept_pos[lo + base + (j < n ? j : n - 1)]);
+        for (int g = 0; g < GROUPS; ++g) total += s_count[g * places + k];
+        s_bin[k] = total;
       }
+      __syncthreads();
+      scan_bins();
+    }
 #pragma unroll
-      for (int u = 0; u < kColumnBatch; ++u) r[u] = row[e[u]];
-#pragma unroll
-      for (int u = 0; u < kColumnBatch; ++u) {
-        w[u] = values[has_data ? e[u] : 0];
-        d[u] = divisor[r[u]];
+    for (int u = 0; u < kColumnPer; ++u) {
+      const int j = static_cast<int>(threadIdx.x) + u * kOrderThreads;
+      if (j < n) {
+        unsigned int place = s_bin[key[u]] + s_key[j];
+        const int mine = j / share;
+        for (int g = 0; g < mine; ++g) place += s_count[g * places + key[u]];
+        out_row[lo + place] = r[u];
+        out_value[lo + place] = (has_data ? w[u] : 1.0f) / d[u];
       }
+    }
+    if (one_round) return;
+    __syncthreads();
+    for (int k = threadIdx.x; k < places; k += kOrderThreads) {
+      unsigned int total = s_bin[k];
 #pragma unroll
-      for (int u = 0; u < kColumnBatch; ++u) {
-        const int j = j0 + u * 256;
-        if (j < n) {
-          const int64_t dst = lo + s_key[j];
-          out_row[dst] = r[u];
-          out_value[dst] = (has_data ? w[u] : 1.0f) / d[u];
-        }
-      }
+      for (int g = 0; g < GROUPS; ++g) total += s_count[g * places + k];
+      s_bin[k] = total;
     }
     __syncthreads();
   }
 }
 
 template <typename IdT>
-void order_columns_launch(int64_t num_cols, int64_t kept, int node_bits, hipStream_t st,
-                          const void* kept_key, const void* kept_pos, const int64_t* indptr,
-                          const void* row, const float* data, const float* divisor, void* out_row,
-                          float* out_value, unsigned int* num_long, unsigned int* long_columns) {
-  hipLaunchKernelGGL(long_columns_kernel, dim3(static_cast<unsigned>(blocks_for(num_cols, 256))),
-                     dim3(256), 0, st, indptr, num_cols, num_long, long_columns);
-  // at most kept / 257 columns are long
-  const unsigned int long_blocks = static_cast<unsigned int>(kept / (kShortColumn + 1) + 1);
-  const dim3 grid(long_blocks + static_cast<unsigned>(blocks_for(kept, 256)));
+int order_columns_launch(int64_t kept, int node_bits, hipStream_t st,
+                         const void* kept_key, const void* kept_pos, const int64_t* indptr,
+                         const void* row, const float* data, const float* divisor, void* out_row,
+                         float* out_value) {
+  // one workgroup for each multiple of 257 among the kept edges
+  const unsigned int long_blocks = static_cast<unsigned int>((kept - 1) / (kShortColumn + 1) + 1);
+  const dim3 grid(long_blocks + static_cast<unsigned>(blocks_for(kept, kOrderThreads)));
   const size_t places = size_t(1) << node_bits;
-  if (node_bits <= kFourWavesBits)
-    hipLaunchKernelGGL((order_columns_kernel<IdT, true>), grid, dim3(256),
-                       (places + kColumnStage + 2 * places) * sizeof(unsigned int), st,
-                       static_cast<const IdT*>(kept_key), static_cast<const IdT*>(kept_pos), node_bits,
-                       indptr, static_cast<const IdT*>(row), data, divisor,
-                       static_cast<IdT*>(out_row), out_value, num_long, long_columns, long_blocks,
-                       kept);
-  else
-    hipLaunchKernelGGL((order_columns_kernel<IdT, false>), grid, dim3(256),
-                       (places + kColumnStage) * sizeof(unsigned int), st,
-                       static_cast<const IdT*>(kept_key), static_cast<const IdT*>(kept_pos), node_bits,
-                       indptr, static_cast<const IdT*>(row), data, divisor,
-                       static_cast<IdT*>(out_row), out_value, num_long, long_columns, long_blocks,
-                       kept);
+  const int groups = order_groups(node_bits);
+  size_t lds = ((places < 4 ? 4 : places) + kColumnStage) * sizeof(unsigned int) +
+               places * groups * sizeof(unsigned short);
+  if (lds < kShortStage * sizeof(IdT)) lds = kShortStage * sizeof(IdT);
+  auto* kernel = groups == 16  ? order_columns_kernel<IdT, 16>
+                 : groups == 8 ? order_columns_kernel<IdT, 8>
+                               : order_columns_kernel<IdT, 4>;
+  if (lds > 48 * 1024) {  // (per call: the attribute belongs to the device the call runs on)
+    const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                   static_cast<int>(lds));
+    if (allowed != hipSuccess) {
+      set_error_text("gs_coo_block_values: %s", hipGetErrorString(allowed));
+      return GS_ERR_LAUNCH;
+    }
+  }
+  hipLaunchKernelGGL(kernel, grid, dim3(kOrderThreads), lds, st, static_cast<const IdT*>(kept_key),
+                     static_cast<const IdT*>(kept_pos), node_bits, indptr,
+                     static_cast<const IdT*>(row), data, divisor, static_cast<IdT*>(out_row),
+                     out_value, long_blocks, kept);
+  return GS_OK;
 }
 
 inline int bits_of(int64_t n) {  // smallest b with 2^b >= n
@@ -629,11 +617,7 @@ int gs_coo_pick_rows(const void* row, const void* col, int id_bytes, int64_t E, 
                                               totals, mailbox, ticket, workspace, workspace_bytes, st);
 }
 
-size_t gs_coo_block_values_workspace_bytes(int64_t kept) {
-  if (kept < 0) kept = 0;
-  return 256 + ((static_cast<size_t>(kept / (kShortColumn + 1) + 1) * sizeof(unsigned int) + 255u) &
-                ~size_t(255));
-}
+size_t gs_coo_block_values_workspace_bytes(int64_t) { return 0; }
 
 int gs_coo_block_values(const void* kept_key, const void* kept_pos, int64_t kept, int64_t max_nodes,
                         const void* row, int id_bytes, const float* data, const float* divisor,
@@ -647,31 +631,21 @@ int gs_coo_block_values(const void* kept_key, const void* kept_pos, int64_t kept
              static_cast<long long>(max_nodes), static_cast<long long>(gs_sorted_union_max(id_bytes)));
   GS_REQUIRE(out_indptr && (kept == 0 || (kept_key && kept_pos && row && divisor && out_row && out_value)),
              "gs_coo_block_values: null pointer");
-  Carver ws(workspace, workspace_bytes);
-  unsigned int* num_long = ws.take<unsigned int>(1);
-  unsigned int* long_columns = ws.take<unsigned int>(static_cast<size_t>(kept / (kShortColumn + 1) + 1));
-  if (!ws.ok) {
-    set_error_text("gs_coo_block_values: workspace needs %zu bytes, 256-byte aligned",
-                   gs_coo_block_values_workspace_bytes(kept));
-    return GS_ERR_WORKSPACE;
-  }
+  (void)workspace;
+  (void)workspace_bytes;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int node_bits = bits_of(max_nodes);
   const dim3 by_edge(static_cast<unsigned>(blocks_for(kept, 256)));
-  if (id_bytes == 8) {
+  if (id_bytes == 8)
     hipLaunchKernelGGL(column_offsets_kernel<int64_t>, by_edge, dim3(256), 0, st,
-                       static_cast<const int64_t*>(kept_key), kept, node_bits, num_cols, out_indptr,
-                       num_long);
-    if (kept > 0 && num_cols > 0)
-      order_columns_launch<int64_t>(num_cols, kept, node_bits, st, kept_key, kept_pos, out_indptr, row,
-                                    data, divisor, out_row, out_value, num_long, long_columns);
-  } else {
+                       static_cast<const int64_t*>(kept_key), kept, node_bits, num_cols, out_indptr);
+  else
     hipLaunchKernelGGL(column_offsets_kernel<int32_t>, by_edge, dim3(256), 0, st,
-                       static_cast<const int32_t*>(kept_key), kept, node_bits, num_cols, out_indptr,
-                       num_long);
-    if (kept > 0 && num_cols > 0)
-      order_columns_launch<int32_t>(num_cols, kept, node_bits, st, kept_key, kept_pos, out_indptr, row,
-                                    data, divisor, out_row, out_value, num_long, long_columns);
+                       static_cast<const int32_t*>(kept_key), kept, node_bits, num_cols, out_indptr);
+  if (kept > 0 && num_cols > 0) {
+    auto* order = id_bytes == 8 ? order_columns_launch<int64_t> : order_columns_launch<int32_t>;
+    GS_RETURN_IF_ERROR(order(kept, node_bits, st, kept_key, kept_pos, out_indptr, row, data, divisor,
+                             out_row, out_value));
   }
   return check_launch("coo_block_values");
 }

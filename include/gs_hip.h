@@ -821,8 +821,8 @@ int gs_coo_pick_rows(const void* row, const void* col, int id_bytes, int64_t E, 
  * put in the order of their rows (ties: of their positions) -- the order of a stable sort of
  * all kept edges by kept_key, done column by column -- and leave as out_row = their row
  * ids and out_value = data[pos] / divisor[row] (data NULL: ones; divisor is indexed by row id);
- * out_indptr[num_cols + 1] = the offsets of the columns.  Workspace (the list of the columns
- * with more than 256 kept edges): gs_coo_block_values_workspace_bytes(kept). */
+ * out_indptr[num_cols + 1] = the offsets of the columns.  No workspace is
+ * needed (gs_coo_block_values_workspace_bytes: 0); it may be NULL. */
 size_t gs_coo_block_values_workspace_bytes(int64_t kept);
 int gs_coo_block_values(const void* kept_key, const void* kept_pos, int64_t kept, int64_t max_nodes,
                         const void* row, int id_bytes, const float* data, const float* divisor,

@@ -128,6 +128,32 @@ def test_pick_rows_with_a_full_tree_and_beyond_the_tiles_that_add_up_themselves(
     assert np.array_equal(pos[:kept].cpu().numpy().astype(np.int64), want_pos)
 
 
+@pytest.mark.parametrize("idb,room", [(4, 1), (4, 2), (8, 1000), (4, 1024), (4, 2048), (8, 4096), (4, 8192)])
+def test_block_values_of_short_and_long_columns(dev, idb, room):
+    """Columns on both sides of the line between a thread an edge and a workgroup a column (256),
+    of one and of several rounds (4096), next to one another and apart, for every number of waves
+    that count (places up to 1024, 2048, 4096, 8192)."""
+    npt, _ = IDT[idb]
+    rng = np.random.default_rng(room)
+    lens = [256, 257, 0, 0, 258, 513, 514, 1, 255, 4096, 4097, 3, 256, 256, 300, 12000, 771, 0, 2]
+    bits = int(np.ceil(np.log2(room))) if room > 1 else 0
+    col = np.repeat(np.arange(len(lens)), lens)
+    place = (rng.random(col.size) ** 2 * room).astype(np.int64)
+    pos = np.sort(rng.permutation(2 * col.size)[:col.size])  # edges of the slice, some not kept
+    row = rng.integers(0, 3 * room, 2 * col.size)
+    row[pos] = 3 * place + 1  # a node's row id grows with its place
+    key = (col << bits) | place
+    data = (1.0 - rng.random(row.size)).astype(np.float32)
+    divisor = (0.5 + rng.random(3 * room)).astype(np.float32)
+    out_row, out_value, indptr = capi.coo_block_values(
+        to_dev(key.astype(npt), dev), to_dev(pos.astype(npt), dev), room, to_dev(row.astype(npt), dev),
+        to_dev(data, dev), to_dev(divisor, dev), len(lens))
+    p = pos[np.argsort(key, kind="stable")]
+    assert np.array_equal(out_row.cpu().numpy(), row[p])
+    assert np.array_equal(out_value.cpu().numpy(), data[p] / divisor[row[p]])
+    assert np.array_equal(indptr.cpu().numpy(), np.concatenate([[0], np.cumsum(lens)]))
+
+
 def test_block_values_without_edges_has_offsets_of_zero(dev):
     empty = torch.empty(0, dtype=torch.int32, device=dev)
     one = torch.zeros(1, dtype=torch.int32, device=dev)
