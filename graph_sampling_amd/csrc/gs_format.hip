@@ -389,14 +389,17 @@ template <typename IdT>
 struct FreshWords {
   const IdT* key;
   int idx_bits;
-  __device__ __forceinline__ unsigned long long operator()(int64_t i) const {
-    return (static_cast<unsigned long long>(key[i]) << idx_bits) |
-           static_cast<unsigned long long>(i);
+  // word j of the tile that begins at `base`
+  __device__ __forceinline__ unsigned long long operator()(int64_t base, uint32_t j) const {
+    return (static_cast<unsigned long long>((key + base)[j]) << idx_bits) |
+           static_cast<unsigned long long>(base + j);
   }
 };
 struct StoredWords {
   const unsigned long long* word;
-  __device__ __forceinline__ unsigned long long operator()(int64_t i) const { return word[i]; }
+  __device__ __forceinline__ unsigned long long operator()(int64_t base, uint32_t j) const {
+    return (word + base)[j];
+  }
 };
 
 // A tile of the sort.  Its items leave digit by digit, so a run is a 256th of the tile on
@@ -411,7 +414,7 @@ struct SortTile {
   static constexpr int kWaves = THREADS / kWave;
 };
 using SmallTile = SortTile<256, 16>;
-using LargeTile = SortTile<512, 16>;
+using LargeTile = SortTile<1024, 8>;
 constexpr int64_t kLargeTileItems = int64_t(1) << 22;  // 512 large tiles: two for every compute unit
 
 // counts[d * num_blocks + b] = items of tile b with digit d.  Four copies of the histogram, lane
@@ -429,15 +432,16 @@ radix_hist_kernel(Src src, int64_t E, int shift, int64_t num_blocks, int64_t* __
   if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;
   __syncthreads();
   const int64_t base = static_cast<int64_t>(blockIdx.x) * T::kSize;
+  const uint32_t n = E - base < T::kSize ? static_cast<uint32_t>(E - base) : T::kSize;
   unsigned long long word[T::kPerThread];
 #pragma unroll
   for (int k = 0; k < T::kPerThread; ++k) {
-    const int64_t i = base + k * T::kThreadsPerTile + threadIdx.x;
-    word[k] = src(i < E ? i : E - 1);
+    const uint32_t j = k * T::kThreadsPerTile + threadIdx.x;
+    word[k] = src(base, j < n ? j : n - 1);
   }
 #pragma unroll
   for (int k = 0; k < T::kPerThread; ++k)
-    if (base + k * T::kThreadsPerTile + threadIdx.x < E)
+    if (k * T::kThreadsPerTile + threadIdx.x < n)
       atomicAdd(&s_hist[threadIdx.x & (kHistCopies - 1)][digit_of(word[k], shift)], 1);
   __syncthreads();
   if (threadIdx.x < kRadix) {
@@ -448,10 +452,40 @@ radix_hist_kernel(Src src, int64_t E, int shift, int64_t num_blocks, int64_t* __
   }
 }
 
-struct LoadI64 {
-  const int64_t* p;
-  __device__ __forceinline__ int64_t operator()(int64_t i) const { return p[i]; }
-};
+// Where a digit's items of a tile start among that digit's items (offsets, laid out like counts),
+// and how many the digit has (totals): a workgroup a digit, 2048 tiles at a time.  What the digits
+// below it hold, every workgroup of the pass adds up from the 256 totals by itself.  (One scan over
+// the whole table, which that leaves out, is two launches: 1709 tiles 11 -> 5 us a pass.)
+constexpr int kDigitThreads = 1024;
+constexpr int kDigitItems = 2;
+
+__global__ void __launch_bounds__(kDigitThreads)
+digit_offsets_kernel(const int64_t* __restrict__ counts, int64_t num_blocks,
+                     int64_t* __restrict__ offsets, int64_t* __restrict__ totals) {
+  __shared__ int64_t s_scan[kDigitThreads / kWave + 1];
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * num_blocks;
+  int64_t run = 0;
+  for (int64_t t0 = 0; t0 < num_blocks; t0 += kDigitThreads * kDigitItems) {
+    const int64_t t = t0 + threadIdx.x * kDigitItems;
+    int64_t n[kDigitItems], mine = 0;
+#pragma unroll
+    for (int k = 0; k < kDigitItems; ++k) n[k] = counts[row + (t + k < num_blocks ? t + k : 0)];
+#pragma unroll
+    for (int k = 0; k < kDigitItems; ++k) {
+      if (t + k >= num_blocks) n[k] = 0;
+      mine += n[k];
+    }
+    int64_t all;
+    int64_t at = run + block_exclusive_scan<kDigitThreads>(mine, &all, s_scan);
+#pragma unroll
+    for (int k = 0; k < kDigitItems; ++k) {
+      if (t + k < num_blocks) offsets[row + t + k] = at;
+      at += n[k];
+    }
+    run += all;
+  }
+  if (threadIdx.x == 0) totals[blockIdx.x] = run;
+}
 
 // where the last pass of the sort writes: the values in key order, the permutation, and
 // the sorted keys themselves (for the offsets; null when nobody builds any)
@@ -476,25 +510,27 @@ struct SortOutputs {
 // no pass gathers it by position; the LAST pass writes values, permutation and keys instead
 // of words.  64-bit values travel in their low 32 bits: ids of any graph that fits the card do,
 // and a value that does not raises `wide`, on which widen_values_kernel fetches all of them
-// again through the permutation.  That and the larger tile took 14 M edges with 64-bit ids
-// and 22-bit keys from 215 us a pass (histogram, scan, scatter) to 150 (the first, which reads the ids as they come) and 119.
+// again through the permutation.  14 M edges with 64-bit ids and 22-bit keys: 109 us the first pass
+// (histogram, scan, scatter; it reads the ids as they come), 96 and 111 the others.
 // SELF: `offsets` holds the tiles' raw counts and every workgroup adds up for itself where its
-// runs start (a sort of few tiles: two launches less per pass than scanning the counts first).
+// runs start (a sort of few tiles: a launch less per pass than scanning the counts first).
 constexpr int64_t kSelfScanTiles = 64;
 static_assert(kLargeTileItems / LargeTile::kSize > kSelfScanTiles, "large tiles never scan themselves");
 
 template <typename T, typename IdT, typename ValT, typename Src, bool LAST, bool SELF>
-__global__ void __launch_bounds__(T::kThreadsPerTile, 4)  // (16 waves a CU is what LDS allows)
+__global__ void __launch_bounds__(T::kThreadsPerTile, T::kWaves == 16 ? 8 : 4)  // (what LDS allows)
 radix_pass_kernel(Src src, const ValT* __restrict__ val_in, int64_t E, int shift,
                   int64_t num_blocks, const int64_t* __restrict__ offsets,
-                  unsigned long long* __restrict__ out, uint32_t* __restrict__ val_out,
-                  SortOutputs<IdT> last) {
+                  const int64_t* __restrict__ totals, unsigned long long* __restrict__ out,
+                  uint32_t* __restrict__ val_out, SortOutputs<IdT> last) {
   constexpr int kThreadsHere = T::kThreadsPerTile, kItemsHere = T::kPerThread;
   __shared__ unsigned long long s_word[T::kSize];
   __shared__ int64_t s_base[kRadix];        // memory position of a digit's run minus its place in the tile
-  __shared__ int s_cnt[T::kWaves][kRadix];  // per wave: count, then count of the earlier waves
+  __shared__ unsigned short s_cnt[T::kWaves][kRadix];  // per wave: count, then count of the earlier waves
   __shared__ int s_start[kRadix];           // where the run of a digit starts in the tile
   __shared__ int s_scan[kRadix / kWave];
+  __shared__ int64_t s_digits[kRadix / kWave];
+  __shared__ int64_t s_all[kRadix];         // a digit's items in all tiles, and in the tiles before this one
   // Consecutive tiles on one XCD (workgroup w runs on XCD w % 8): the runs of a digit that they
   // write lie side by side, and the line that two of them share is filled in one L2.  Load +
   // CSC of 14 M edges: 645 -> 623 us.
@@ -503,55 +539,41 @@ radix_pass_kernel(Src src, const ValT* __restrict__ val_in, int64_t E, int shift
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const int digit = threadIdx.x;  // of the first 256 threads
-  int64_t run_at = 0;
-  if (SELF) {
-    // this digit's items in all tiles, and in the tiles before this one
-    __shared__ int64_t s_digits[kRadix / kWave];
-    int64_t all = 0, before = 0, incl = 0;
-    if (digit < kRadix) {
-      const int64_t* row = offsets + static_cast<int64_t>(digit) * num_blocks;
+  int64_t all = 0, before_tile = 0;
+  if (digit < kRadix) {
+    const int64_t* row = offsets + static_cast<int64_t>(digit) * num_blocks;
+    if (SELF) {
       for (int64_t b = 0; b < num_blocks; ++b) {
         const int64_t c = row[b];
         all += c;
-        before += b < tile ? c : 0;
+        before_tile += b < tile ? c : 0;
       }
-      incl = all;
-#pragma unroll
-      for (int d = 1; d < kWave; d <<= 1) {
-        const int64_t y = __shfl_up(incl, d, kWave);
-        if (lane >= d) incl += y;
-      }
-      if (lane == kWave - 1) s_digits[wave] = incl;
+    } else {
+      all = totals[digit];
+      before_tile = row[tile];
     }
-    __syncthreads();
-    if (digit < kRadix) {
-      int64_t lower = incl - all;  // items of the smaller digits
-      for (int w = 0; w < wave; ++w) lower += s_digits[w];
-      run_at = lower + before;
-    }
-  } else if (digit < kRadix) {
-    run_at = offsets[static_cast<int64_t>(digit) * num_blocks + tile];
   }
-  for (int j = threadIdx.x; j < T::kWaves * kRadix; j += kThreadsHere) (&s_cnt[0][0])[j] = 0;
+  for (int j = threadIdx.x; j < T::kWaves * kRadix / 2; j += kThreadsHere)
+    reinterpret_cast<uint32_t*>(&s_cnt[0][0])[j] = 0u;
   const int64_t base = tile * T::kSize;
-  const int64_t wave_base = base + static_cast<int64_t>(wave) * (T::kSize / T::kWaves);
-  // (indices clamped instead of reads left out: all of a thread's reads go out together)
+  // (indices clamped instead of reads left out: all of a thread's reads go out together; counted
+  // from the tile's start, in 32 bits, so that they take one register each)
+  const uint32_t n = E - base < T::kSize ? static_cast<uint32_t>(E - base) : T::kSize;
+  const uint32_t mine0 = wave * (T::kSize / T::kWaves) + lane;
   unsigned long long word[kItemsHere];
-  ValT raw[kItemsHere];
 #pragma unroll
   for (int r = 0; r < kItemsHere; ++r) {
-    const int64_t i = wave_base + r * kWave + lane;
-    word[r] = src(i < E ? i : E - 1);
+    const uint32_t j = mine0 + r * kWave;
+    word[r] = src(base, j < n ? j : n - 1);
   }
   // (what lies behind the last edge takes the last digit; it comes last in index order, so its
   // places are those behind the tile's live items and none of them is written out)
 #pragma unroll
   for (int r = 0; r < kItemsHere; ++r)
-    if (wave_base + r * kWave + lane >= E) word[r] = ~0ull;
-#pragma unroll
-  for (int r = 0; r < kItemsHere; ++r) {
-    const int64_t i = wave_base + r * kWave + lane;
-    raw[r] = val_in[i < E ? i : E - 1];
+    if (mine0 + r * kWave >= n) word[r] = ~0ull;
+  if (digit < kRadix) {  // (out of the registers until the items are counted)
+    s_all[digit] = all;
+    s_base[digit] = before_tile;
   }
   __syncthreads();  // the tables are zero
   int place[kItemsHere];
@@ -571,38 +593,57 @@ radix_pass_kernel(Src src, const ValT* __restrict__ val_in, int64_t E, int shift
     const int rank = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0));
     const int before = s_cnt[wave][d];  // the wave's earlier rounds (LDS operations of a wave keep their order)
     place[r] = before + rank;
-    if (rank == 0) s_cnt[wave][d] = before + __popc(lo) + __popc(hi);
+    if (rank == 0) s_cnt[wave][d] = static_cast<unsigned short>(before + __popc(lo) + __popc(hi));
   }
-  uint32_t val[kItemsHere];
-  bool wide = false;
+  // The values are asked for only now and needed behind the words' way out: on their way from the
+  // start, they did not fit the registers beside the words, and every one was waited for and
+  // set aside in memory before the next (14 M edges, 64-bit ids, with tiles of 1024 threads instead
+  // of 512: first pass 102 -> 78 us, the others 72 -> 67 and 84 -> 82).
+  ValT raw[kItemsHere];
+  const ValT* __restrict__ tile_val = val_in + base;
+  uint32_t again0 = mine0;  // (indices and digits made a second time rather than kept)
+  asm volatile("" : "+v"(again0), "+s"(shift));
 #pragma unroll
   for (int r = 0; r < kItemsHere; ++r) {
-    val[r] = static_cast<uint32_t>(raw[r]);
-    if (sizeof(ValT) == 8) wide |= static_cast<uint64_t>(raw[r]) != val[r];
+    const uint32_t j = again0 + r * kWave;
+    raw[r] = tile_val[j < n ? j : n - 1];
   }
-  if (sizeof(ValT) == 8 && wide) *last.wide = 1;
   __syncthreads();
-  // digit by digit: counts of the waves -> counts of the earlier waves, total -> start
+  // digit by digit: counts of the waves -> counts of the earlier waves, total -> start; and where
+  // the digit's items of this tile go, behind the smaller digits' of all tiles
   int total = 0, incl = 0;
+  int64_t run_at = 0;
   if (digit < kRadix) {
+    run_at = s_all[digit];
 #pragma unroll
     for (int w = 0; w < T::kWaves; ++w) {
       const int c = s_cnt[w][digit];
-      s_cnt[w][digit] = total;
+      s_cnt[w][digit] = static_cast<unsigned short>(total);
       total += c;
     }
     incl = total;
 #pragma unroll
     for (int d = 1; d < kWave; d <<= 1) {
       const int y = __shfl_up(incl, d, kWave);
-      if (lane >= d) incl += y;
+      const int64_t z = __shfl_up(run_at, d, kWave);
+      if (lane >= d) {
+        incl += y;
+        run_at += z;
+      }
     }
-    if (lane == kWave - 1) s_scan[wave] = incl;
+    if (lane == kWave - 1) {
+      s_scan[wave] = incl;
+      s_digits[wave] = run_at;
+    }
   }
   __syncthreads();
   if (digit < kRadix) {
     int start = incl - total;
-    for (int w = 0; w < wave; ++w) start += s_scan[w];
+    run_at += s_base[digit] - s_all[digit];
+    for (int w = 0; w < wave; ++w) {
+      start += s_scan[w];
+      run_at += s_digits[w];
+    }
     s_start[digit] = start;
     s_base[digit] = run_at - start;
   }
@@ -616,11 +657,10 @@ radix_pass_kernel(Src src, const ValT* __restrict__ val_in, int64_t E, int shift
     s_word[place[r]] = word[r];
   }
   __syncthreads();
-  const int n = static_cast<int>(E - base < T::kSize ? E - base : T::kSize);
   int out_digit[kItemsHere];
 #pragma unroll
   for (int k = 0; k < kItemsHere; ++k) {
-    const int j = k * kThreadsHere + threadIdx.x;
+    const uint32_t j = k * kThreadsHere + threadIdx.x;
     out_digit[k] = 0;
     if (j < n) {
       const unsigned long long w = s_word[j];
@@ -634,14 +674,19 @@ radix_pass_kernel(Src src, const ValT* __restrict__ val_in, int64_t E, int shift
       }
     }
   }
+  bool wide = false;
+#pragma unroll
+  for (int r = 0; r < kItemsHere; ++r)
+    if (sizeof(ValT) == 8) wide |= static_cast<uint64_t>(raw[r]) != static_cast<uint32_t>(raw[r]);
+  if (sizeof(ValT) == 8 && wide) *last.wide = 1;
   __syncthreads();
   uint32_t* s_val = reinterpret_cast<uint32_t*>(s_word);
 #pragma unroll
-  for (int r = 0; r < kItemsHere; ++r) s_val[place[r]] = val[r];
+  for (int r = 0; r < kItemsHere; ++r) s_val[place[r]] = static_cast<uint32_t>(raw[r]);
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < kItemsHere; ++k) {
-    const int j = k * kThreadsHere + threadIdx.x;
+    const uint32_t j = k * kThreadsHere + threadIdx.x;
     if (j < n) {
       const int64_t dst = s_base[out_digit[k]] + j;
       if (LAST)
@@ -705,11 +750,11 @@ indptr_split_kernel(const int64_t* __restrict__ indptr, const int64_t* __restric
 
 template <typename T, typename IdT, typename ValT, typename Src>
 void launch_pass(Src src, bool last, bool self, hipStream_t st, const ValT* vin, int64_t E, int shift,
-                 int64_t blocks, const int64_t* where, unsigned long long* wout, uint32_t* vout,
-                 const SortOutputs<IdT>& outs) {
+                 int64_t blocks, const int64_t* where, const int64_t* totals,
+                 unsigned long long* wout, uint32_t* vout, const SortOutputs<IdT>& outs) {
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(T::kThreadsPerTile), 0, st,
-                       src, vin, E, shift, blocks, where, wout, vout, outs);
+                       src, vin, E, shift, blocks, where, totals, wout, vout, outs);
   };
   if constexpr (std::is_same<T, SmallTile>::value) {  // (a sort by large tiles has 512 at least)
     if (self) {
@@ -726,7 +771,7 @@ void launch_pass(Src src, bool last, bool self, hipStream_t st, const ValT* vin,
 struct SortSpace {
   unsigned long long* word[2];
   uint32_t* value[2];
-  int64_t *counts, *offsets, *tiles;
+  int64_t *counts, *offsets, *totals;
   uint32_t* keys;
   int* wide;
 };
@@ -734,8 +779,8 @@ struct SortSpace {
 inline size_t sort_space_bytes(int64_t E) {
   const int64_t table = kRadix * static_cast<int64_t>(blocks_for(E, SmallTile::kSize));
   const size_t n = static_cast<size_t>(E > 0 ? E : 1);
-  return 2 * padded(n * 8) + 3 * padded(n * 4) + padded(static_cast<size_t>(table) * 8) +
-         padded(static_cast<size_t>(table + 1) * 8) + scan_workspace_bytes(table) + 256;
+  return 2 * padded(n * 8) + 3 * padded(n * 4) + 2 * padded(static_cast<size_t>(table) * 8) +
+         padded(kRadix * 8) + 256;
 }
 inline bool carve_sort(Carver& ws, int64_t E, SortSpace* s) {
   const int64_t table = kRadix * static_cast<int64_t>(blocks_for(E, SmallTile::kSize));
@@ -744,8 +789,8 @@ inline bool carve_sort(Carver& ws, int64_t E, SortSpace* s) {
   for (auto& v : s->value) v = ws.take<uint32_t>(n);
   s->keys = ws.take<uint32_t>(n);
   s->counts = ws.take<int64_t>(static_cast<size_t>(table));
-  s->offsets = ws.take<int64_t>(static_cast<size_t>(table + 1));
-  s->tiles = ws.take<int64_t>(static_cast<size_t>(scan_num_tiles(table) + 1));
+  s->offsets = ws.take<int64_t>(static_cast<size_t>(table));
+  s->totals = ws.take<int64_t>(kRadix);
   s->wide = ws.take<int>(1);
   return ws.ok;
 }
@@ -754,7 +799,6 @@ template <typename T, typename IdT>
 int sort_passes(const IdT* key, const IdT* value, int64_t E, int passes, int idx_bits,
                 const SortSpace& s, const SortOutputs<IdT>& outs, hipStream_t st) {
   const int64_t blocks = blocks_for(E, T::kSize);
-  const int64_t table = kRadix * blocks;
   const dim3 grid(static_cast<unsigned>(blocks));
   const bool self = blocks <= kSelfScanTiles;
   const int64_t* where = self ? s.counts : s.offsets;
@@ -769,16 +813,15 @@ int sort_passes(const IdT* key, const IdT* value, int64_t E, int passes, int idx
     else
       hipLaunchKernelGGL((radix_hist_kernel<T, StoredWords>), grid, dim3(T::kThreadsPerTile), 0, st,
                          stored, E, shift, blocks, s.counts, static_cast<int*>(nullptr));
-    if (!self) {
-      LoadI64 f{s.counts};
-      GS_RETURN_IF_ERROR(exclusive_scan(f, table, s.offsets, s.tiles, st));
-    }
+    if (!self)
+      hipLaunchKernelGGL(digit_offsets_kernel, dim3(kRadix), dim3(kDigitThreads), 0, st, s.counts,
+                         blocks, s.offsets, s.totals);
     if (p == 0)
-      launch_pass<T>(fresh, last, self, st, value, E, shift, blocks, where, s.word[0], s.value[0],
-                     outs);
+      launch_pass<T>(fresh, last, self, st, value, E, shift, blocks, where, s.totals, s.word[0],
+                     s.value[0], outs);
     else
       launch_pass<T>(stored, last, self, st, static_cast<const uint32_t*>(s.value[(p + 1) & 1]), E,
-                     shift, blocks, where, s.word[p & 1], s.value[p & 1], outs);
+                     shift, blocks, where, s.totals, s.word[p & 1], s.value[p & 1], outs);
   }
   return check_launch("coo2csc");
 }
@@ -1159,8 +1202,8 @@ constexpr int kBinMaxShift = 15;         // 2^15 sums = 128 KB of LDS
 
 __global__ void __launch_bounds__(kBinThreads)
 bin_sum_kernel(const unsigned long long* __restrict__ words, const uint32_t* __restrict__ vals,
-               const int64_t* __restrict__ offsets, int64_t num_blocks, int num_bins, int idx_bits,
-               int bin_shift, int powk, int64_t num_targets, float* __restrict__ out) {
+               const int64_t* __restrict__ totals, int num_bins, int idx_bits, int bin_shift,
+               int powk, int64_t num_targets, float* __restrict__ out) {
   extern __shared__ float s_sum[];
   // Which run, and which share of it, this workgroup takes: the launch has one workgroup per
   // share that can exist (a run of n edges has ceil(n / 16 k) of them, 64 at most), and every
@@ -1169,16 +1212,19 @@ bin_sum_kernel(const unsigned long long* __restrict__ words, const uint32_t* __r
   // to workgroups with nothing to do.)
   __shared__ int64_t s_scan[kBinThreads / kWave + 1];
   __shared__ int s_first[kRadix + 1];
+  __shared__ int64_t s_lo[kRadix + 1];
   {
-    int64_t mine = 0;
-    if (threadIdx.x < num_bins) {
-      const int64_t n = offsets[(threadIdx.x + 1) * num_blocks] - offsets[threadIdx.x * num_blocks];
-      mine = (n + kBinPartItems - 1) / kBinPartItems;
-      if (mine > kBinParts) mine = kBinParts;
-    }
+    int64_t n = 0;
+    if (threadIdx.x < num_bins) n = totals[threadIdx.x];
+    int64_t shares = (n + kBinPartItems - 1) / kBinPartItems;
+    if (shares > kBinParts) shares = kBinParts;
+    // (both sums in one scan: up to 2^14 shares above, fewer than 2^31 edges below)
     int64_t total;
-    const int64_t before = block_exclusive_scan<kBinThreads>(mine, &total, s_scan);
-    if (threadIdx.x <= num_bins) s_first[threadIdx.x] = static_cast<int>(before);
+    const int64_t before = block_exclusive_scan<kBinThreads>(shares << 32 | n, &total, s_scan);
+    if (threadIdx.x <= num_bins) {
+      s_first[threadIdx.x] = static_cast<int>(before >> 32);
+      s_lo[threadIdx.x] = before & 0xFFFFFFFFll;
+    }
     __syncthreads();
   }
   if (static_cast<int>(blockIdx.x) >= s_first[num_bins]) return;
@@ -1186,7 +1232,7 @@ bin_sum_kernel(const unsigned long long* __restrict__ words, const uint32_t* __r
   for (int step = kRadix / 2; step > 0; step >>= 1)
     if (bin + step <= num_bins && s_first[bin + step] <= static_cast<int>(blockIdx.x)) bin += step;
   const int part = static_cast<int>(blockIdx.x) - s_first[bin];
-  const int64_t lo = offsets[bin * num_blocks], hi = offsets[(bin + 1) * num_blocks];
+  const int64_t lo = s_lo[bin], hi = s_lo[bin + 1];
   const int64_t n = hi - lo;
   int64_t parts = (n + kBinPartItems - 1) / kBinPartItems;
   if (parts > kBinParts) parts = kBinParts;
@@ -1263,8 +1309,8 @@ int bin_sum_impl(const int32_t* target, const float* data, int64_t E, int powk, 
   unsigned long long* words = ws.take<unsigned long long>(E);
   uint32_t* vals = ws.take<uint32_t>(E);
   int64_t* counts = ws.take<int64_t>(table);
-  int64_t* offsets = ws.take<int64_t>(table + 1);
-  int64_t* tiles = ws.take<int64_t>(scan_num_tiles(table) + 1);
+  int64_t* offsets = ws.take<int64_t>(table);
+  int64_t* totals = ws.take<int64_t>(kRadix);
   if (!ws.ok) {
     set_error_text("gs_coo_sum_binned: workspace needs %zu bytes, 256-byte aligned",
                    gs_coo_sum_workspace_bytes(E, num_targets));
@@ -1278,11 +1324,11 @@ int bin_sum_impl(const int32_t* target, const float* data, int64_t E, int powk, 
   FreshWords<int32_t> src{target, idx_bits};
   hipLaunchKernelGGL((radix_hist_kernel<T, FreshWords<int32_t>>), grid, dim3(T::kThreadsPerTile), 0,
                      st, src, E, shift, blocks, counts, static_cast<int*>(nullptr));
-  LoadI64 f{counts};
-  GS_RETURN_IF_ERROR(exclusive_scan(f, table, offsets, tiles, st));
+  hipLaunchKernelGGL(digit_offsets_kernel, dim3(kRadix), dim3(kDigitThreads), 0, st, counts, blocks,
+                     offsets, totals);
   const SortOutputs<int32_t> none{nullptr, nullptr, nullptr, idx_bits, nullptr};
   launch_pass<T>(src, false, false, st, reinterpret_cast<const uint32_t*>(data), E, shift, blocks,
-                 offsets, words, vals, none);
+                 offsets, totals, words, vals, none);
   const int bins = static_cast<int>(((num_targets - 1) >> bin_shift) + 1);
   // (per call: the attribute belongs to the device the call runs on)
   const hipError_t lds_allowed = hipFuncSetAttribute(
@@ -1294,8 +1340,8 @@ int bin_sum_impl(const int32_t* target, const float* data, int64_t E, int powk, 
   }
   const int64_t shares = E / kBinPartItems + bins;  // at most: sum of ceil(n / 16 k) over the runs
   hipLaunchKernelGGL(bin_sum_kernel, dim3(static_cast<unsigned>(shares)), dim3(kBinThreads),
-                     sizeof(float) << bin_shift, st, words, vals, offsets, blocks, bins, idx_bits,
-                     bin_shift, powk, num_targets, out);
+                     sizeof(float) << bin_shift, st, words, vals, totals, bins, idx_bits, bin_shift, powk,
+                      num_targets, out);
   return check_launch("coo_sum_binned");
 }
 
@@ -1480,8 +1526,7 @@ size_t gs_coo_sum_workspace_bytes(int64_t E, int64_t num_targets) {
   const int64_t blocks = blocks_for(E, SmallTile::kSize);
   const int64_t table = kRadix * blocks;
   return padded(static_cast<size_t>(E) * 8) + padded(static_cast<size_t>(E) * 4) +
-         padded(static_cast<size_t>(table) * 8) + padded(static_cast<size_t>(table + 1) * 8) +
-         scan_workspace_bytes(table);
+         2 * padded(static_cast<size_t>(table) * 8) + padded(kRadix * 8);
 }
 
 int gs_coo_sum_binned(const void* target, int id_bytes, const int64_t* e_ids, const float* data,
