@@ -892,6 +892,7 @@ struct DistinctSpace {
   int64_t* partial;    // per workgroup of the counting launches
   int64_t num_partial;
   int64_t* first;      // {distinct ids of the first end, 1 when the second has to be counted}
+  int64_t* slices;     // by bits: slices that the first marking launch takes
 };
 
 __global__ void __launch_bounds__(kThreads) clear_marks_kernel(uint4* map, int64_t n) {
@@ -1017,13 +1018,14 @@ post_distinct_kernel(DistinctSpace s, gs_mailbox* box, int64_t ticket) {
 
 // The same for long lists, by bits in LDS: every compute unit keeps a bitmap of 1.28 M ids and
 // marks its share of the edges there, the bitmaps go to memory and are or-ed and counted.
-// The first launch takes ids of the first slice and finds the largest id of both ends (its
-// workgroups read each end once); when that lies beyond, the second shares out the other
-// slices, reading the end once per slice: a stream against a request per edge.  Ids beyond
-// eight slices are reported and the caller asks for the bytes.  14 M edges over 2.45 M
-// nodes, 64-bit ids: 220 -> 145 us (617 -> 551 with the sort behind it; looking a bit up
-// before setting it, or asking for the next reads ahead, changed nothing).  The bitmaps are
-// 80 MB whatever the list, so lists below 4 M edges stay with the bytes.
+// How many such slices the ids take is guessed from 1024 of them (guess_slices_kernel): the first
+// launch deals its workgroups out to that many, so that it reads the end once for each -- the
+// workgroups of a share sit on one die, whose L2 has it for the second -- and finds the largest id
+// of both ends; a second takes the slices behind those, if there are any.  Ids beyond eight
+// slices are reported and the caller asks for the bytes.  14 M edges over 2.45 M nodes, 64-bit
+// ids: 220 us by bytes, 145 with one slice in the first launch and a second launch for the
+// rest, 113 so (the list loaded and sorted: 494 -> 462).  The bitmaps are 80 MB whatever the list, so lists below 4 M edges stay
+// with the bytes.
 constexpr int kBitWords = 39936;  // 156 KB of a compute unit's 160
 constexpr int64_t kSliceIds = int64_t(kBitWords) * 32;
 constexpr int kMaxSlices = 8;
@@ -1052,7 +1054,44 @@ __device__ __forceinline__ int64_t largest_of_list(const DistinctSpace& s) {
   return top;
 }
 
-// REST: the slices behind the first.  look: the other end, looked through for its largest id
+// Slices that the largest of a sample of both ends asks for: one id a thread of either (a compute
+// unit alone fetches a line every 2.5 ns: eight a thread took 40 us).
+constexpr int kGuessThreads = 512;
+template <typename IdT>
+__global__ void __launch_bounds__(kGuessThreads)
+guess_slices_kernel(const IdT* __restrict__ a, const IdT* __restrict__ b, int64_t E, DistinctSpace s) {
+  __shared__ uint64_t s_top[kGuessThreads / kWave];
+  const int64_t step = E / kGuessThreads;  // (lists that are counted by bits are longer)
+  const IdT x = a[threadIdx.x * step], y = b[threadIdx.x * step];
+  const uint64_t u = static_cast<uint64_t>(static_cast<int64_t>(x));
+  const uint64_t v = static_cast<uint64_t>(static_cast<int64_t>(y));
+  uint64_t top = u > v ? u : v;
+#pragma unroll
+  for (int d = kWave / 2; d > 0; d >>= 1) {
+    const uint64_t o = __shfl_xor(top, d, kWave);
+    top = o > top ? o : top;
+  }
+  if ((threadIdx.x & (kWave - 1)) == 0) s_top[threadIdx.x / kWave] = top;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kGuessThreads / kWave; ++w) top = s_top[w] > top ? s_top[w] : top;
+    const uint64_t n = top / static_cast<uint64_t>(kSliceIds) + 1;
+    *s.slices = n <= static_cast<uint64_t>(kMaxSlices) ? static_cast<int64_t>(n) : 1;  // (beyond: reported)
+  }
+}
+
+// Of the first launch, which takes `slices` slices: workgroup w works on die w % 8, takes slice
+// (w / 8) % slices and one of the die's 32 / slices shares of the end.
+struct FirstSlices {
+  int64_t per_die;
+  __device__ __forceinline__ explicit FirstSlices(int64_t slices) : per_die(kBitBlocks / kXcds / slices) {}
+  __device__ __forceinline__ int64_t parts() const { return per_die * kXcds; }
+  __device__ __forceinline__ int64_t workgroup(int64_t slices, int64_t slice, int64_t part) const {
+    return ((part / kXcds) * slices + slice) * kXcds + part % kXcds;
+  }
+};
+
+// REST: the slices behind the first launch's.  look: the other end, looked through for its largest id
 // (null when the largest is known).
 template <typename IdT, bool REST>
 __global__ void __launch_bounds__(kBitThreads)
@@ -1061,19 +1100,28 @@ mark_bits_kernel(const IdT* __restrict__ ids, const IdT* __restrict__ look, int6
   __shared__ __attribute__((aligned(16))) uint32_t s_bits[kBitWords];
   __shared__ int64_t s_wave[kBitThreads / kWave];
   if (second && !s.first[1]) return;
-  int64_t slice = 0, part = blockIdx.x, parts = kBitBlocks;
+  const int64_t slices = *s.slices;
+  int64_t slice, part, parts;
   if (REST) {
-    const int64_t rest = largest_of_list<kBitThreads>(s) / kSliceIds;  // slices behind the first
-    if (rest < 1 || rest >= kMaxSlices) return;
+    const int64_t all = largest_of_list<kBitThreads>(s) / kSliceIds + 1;
+    if (all <= slices || all > kMaxSlices) return;
+    const int64_t rest = all - slices;
     parts = kBitBlocks / rest;
-    slice = 1 + blockIdx.x % rest;
+    slice = slices + blockIdx.x % rest;
     part = blockIdx.x / rest;
     if (part >= parts) return;
+  } else {
+    const FirstSlices f(slices);
+    parts = f.parts();
+    slice = blockIdx.x / kXcds % slices;
+    part = blockIdx.x / kXcds / slices * kXcds + blockIdx.x % kXcds;
   }
   for (int j = threadIdx.x; j < kBitWords / 4; j += kBitThreads)
     reinterpret_cast<uint4*>(s_bits)[j] = make_uint4(0, 0, 0, 0);
   __syncthreads();
-  const int64_t lo = E * part / parts, hi = E * (part + 1) / parts;
+  // (a workgroup that finds no share of its own marks nothing, but looks through the other end)
+  const int64_t lo = part < parts ? E * part / parts : 0;
+  const int64_t hi = part < parts ? E * (part + 1) / parts : 0;
   const uint64_t first_id = static_cast<uint64_t>(slice * kSliceIds);
   uint64_t largest = 0;  // (an id below zero is a huge one here)
   for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += kBitTrip * kBitThreads) {
@@ -1095,12 +1143,13 @@ mark_bits_kernel(const IdT* __restrict__ ids, const IdT* __restrict__ look, int6
     }
   }
   if (!REST && look) {
-    for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += kBitTrip * kBitThreads) {
+    const int64_t from = E * blockIdx.x / kBitBlocks, to = E * (blockIdx.x + 1) / kBitBlocks;
+    for (int64_t i0 = from + threadIdx.x; i0 < to; i0 += kBitTrip * kBitThreads) {
       IdT id[kBitTrip];
 #pragma unroll
       for (int u = 0; u < kBitTrip; ++u) {
         const int64_t i = i0 + u * kBitThreads;
-        id[u] = look[i < hi ? i : hi - 1];
+        id[u] = look[i < to ? i : to - 1];
       }
 #pragma unroll
       for (int u = 0; u < kBitTrip; ++u) {
@@ -1133,18 +1182,22 @@ __global__ void __launch_bounds__(kThreads) count_bits_kernel(DistinctSpace s, b
   __shared__ uint4 s_or[kOrRows][kOrVecs];
   __shared__ int64_t s_scan[kThreads / kWave + 1];
   if (second && !s.first[1]) return;
-  const int64_t rest = largest_of_list<kThreads>(s) / kSliceIds;
+  const int64_t slices = *s.slices, known = largest_of_list<kThreads>(s) / kSliceIds + 1;
   const int64_t slice = blockIdx.y;
   int64_t n = 0;
-  if (slice <= rest && rest < kMaxSlices) {  // (the same for the whole workgroup)
-    const int64_t step = slice ? rest : 1;
-    const int64_t rows = kBitBlocks / step, row0 = slice ? kBitBlocks + slice - 1 : 0;
+  if (slice < known && known <= kMaxSlices) {  // (the same for the whole workgroup)
+    // the slice's bitmaps: of the first launch's workgroups, or of the second's
+    const bool rest = slice >= slices;
+    const FirstSlices f(slices);
+    const int64_t step = known - slices;
+    const int64_t rows = rest ? kBitBlocks / step : f.parts();
     const int g = threadIdx.x / kOrVecs, v = threadIdx.x % kOrVecs;
     const uint4* map = reinterpret_cast<const uint4*>(s.map) + static_cast<int64_t>(blockIdx.x) * kOrVecs + v;
     uint4 all = make_uint4(0, 0, 0, 0);
 #pragma unroll 8
     for (int64_t r = g; r < rows; r += kOrRows) {
-      const uint4 x = map[(row0 + r * step) * (kBitWords / 4)];
+      const int64_t row = rest ? kBitBlocks + slice - slices + r * step : f.workgroup(slices, slice, r);
+      const uint4 x = map[row * (kBitWords / 4)];
       all.x |= x.x; all.y |= x.y; all.z |= x.z; all.w |= x.w;
     }
     s_or[g][v] = all;
@@ -1164,6 +1217,7 @@ __global__ void __launch_bounds__(kThreads) count_bits_kernel(DistinctSpace s, b
 
 template <typename IdT>
 void distinct_by_bits(const IdT* a, const IdT* b, int64_t E, const DistinctSpace& s, hipStream_t st) {
+  hipLaunchKernelGGL((guess_slices_kernel<IdT>), dim3(1), dim3(kGuessThreads), 0, st, a, b, E, s);
   for (int end = 0; end < 2; ++end) {
     const IdT* ids = end ? b : a;
     const IdT* look = end ? nullptr : b;
@@ -1447,7 +1501,8 @@ int gs_distinct_ends(const void* a, const void* b, int id_bytes, int64_t E, void
   s.largest = ws.take<int64_t>(2 * static_cast<size_t>(blocks) + kBitBlocks);
   s.num_partial = by_bits ? kOrBlocks * kMaxSlices : kCountBlocks;
   s.partial = ws.take<int64_t>(static_cast<size_t>(s.num_partial));
-  s.first = ws.take<int64_t>(2);
+  s.first = ws.take<int64_t>(3);
+  s.slices = s.first + 2;
   if (!ws.ok) {
     set_error_text("gs_distinct_ends: workspace needs %zu bytes, 256-byte aligned",
                    gs_distinct_ends_workspace_bytes(E));
