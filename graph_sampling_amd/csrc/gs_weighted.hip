@@ -10,27 +10,41 @@
 // composite (ordered key << 32 | ~position): composites are distinct, so
 // "largest k" is unambiguous and bit-reproducible.
 //
-// Selection is a wave-level top-k over at most 2048 candidates, 32 per lane, held in
-// registers: the k-th largest of the 64 lanes' own maxima is a floor that at least k
-// candidates reach, so everything below it is dropped at once; the few survivors
-// (between k and 32 k, typically about 2 k) are packed into LDS with ballots and each
-// one counts how many survivors beat it -- that count is its place in the output.  No
-// per-lane sorted lists, no k rounds of wave-wide maxima.  Rows up to 2048 edges are
-// one wave each.  Longer rows are cut into 2048-edge chunks that go through a device
-// queue: one wave per chunk writes its local top-k composites, then one wave per
-// long row merges them (per-lane sorted lists in LDS and k rounds of "largest head
-// wins": the candidates of a hub's chunks can be many more than 2048).  That spreads a
-// 10^5-edge hub over hundreds of waves instead of pinning one warp on it.
+// Selection is a top-k over at most 2048 edges held in registers, by a rough key first: the
+// hardware's log2 and reciprocal instead of the exact recipe with its two divisions.  The k-th
+// largest of a wave's 64 lane maxima is a floor that at least k edges reach, so an edge that
+// stays below it by more than both keys can be off is dropped at once; the few survivors
+// (typically about 2 k) are packed into LDS, get their exact keys, and each counts how many
+// survivors beat it -- that count is its place in the output.
+//
+// Rows up to 256 edges are one wave each; longer ones are cut into chunks of 2048 edges, a
+// workgroup each, so that a 10^5-edge hub is spread over fifty workgroups.  What bounds the fill
+// is instructions, not bytes (a Philox block per four edges, the keys, the floors: that is why
+// exact keys are left to the survivors), then the chain of dependent reads of a task (offsets,
+// weights, the picks' ids).  So the chunks are found by a launch of their own that only reads
+// offsets, and rows and chunks then go side by side; the last chunk of a row to finish merges
+// the row's candidates.
 #include "gs_common.hpp"
+#include "gs_one.hpp"
 
 namespace gs {
 namespace {
 
-constexpr int64_t kChunk = 2048;          // edges per wave task
-constexpr int64_t kMaxFanout = 96;        // 64 lanes * 96 * 8 B = 48 KB of LDS per wave
-constexpr int kQueueGrid = 1024;          // workgroups draining a queue
-constexpr int64_t kQueueExtra = 1 << 19;  // chunk-queue capacity = S + kQueueExtra
-constexpr int kQueueParts = 64;           // one lane per part where the parts are added up
+constexpr int kThreads = 256;
+constexpr int kWaves = kThreads / kWave;
+constexpr int64_t kChunk = 2048;          // edges per workgroup task
+constexpr int64_t kSmall = 4 * kWave;     // longest row of one wave: 4 edges a lane
+constexpr int kMaxFanout = 96;
+constexpr int64_t kHubTasks = 1 << 19;    // chunks of rows with several
+constexpr int kPlanRows = 1024;           // rows (threads) of a planning workgroup
+constexpr int kQueueGrid = 2048;          // workgroups that take chunks
+
+// A row of one chunk, or chunk number (index of this entry - base) of a longer one.
+struct Task {
+  int64_t row;  // -1: void
+  int64_t start, deg, out;
+  int64_t base;  // entry of the row's first chunk
+};
 
 template <typename IdT>
 struct WArgs {
@@ -48,16 +62,17 @@ struct WArgs {
   IdT* sub_indices;
   int64_t* select_index;
   IdT* coo_col;
-  // long rows
-  // [1] long rows, [2 + q] chunks reserved in part q of the queue.  The queue is kept in
-  // kQueueParts parts, each with a counter of its own (a workgroup reserves in part
-  // blockIdx % kQueueParts): reservations at ONE counter queue up at its address, 11 ns
-  // apiece, and 2000 rows above 256 edges among 45 k made that the rows kernel's last 20 us.
-  unsigned long long* counters;
-  long long* chunk_queue;        // row << 20 | chunk, -1 = void
-  int64_t chunk_cap;             // slots of one part
-  long long* long_rows;          // 3 entries per long row: row, first queue slot, #chunks
-  unsigned long long* cand;      // chunk_cap * k composites
+  // edge data that follows the samples: data_out[o] = edge_data[q] for the output o taken at
+  // position q; data_out == nullptr: none
+  const float* edge_data;
+  float* data_out;
+  unsigned long long* reserved;  // chunks of rows with several << 32 | rows of one chunk
+  // kHubTasks entries of the former, then S of the latter: those with a merge behind them are
+  // taken first
+  Task* tasks;
+  int64_t* row_base;             // first entry of a row with several chunks
+  unsigned int* done;            // [base]: chunks of the row that have left their candidates
+  unsigned long long* cand;      // kHubTasks * k composites
 };
 
 __device__ __forceinline__ unsigned long long composite(float key, uint32_t pos) {
@@ -67,336 +82,438 @@ __device__ __forceinline__ uint32_t composite_pos(unsigned long long c) {
   return 0xFFFFFFFFu - static_cast<uint32_t>(c);
 }
 
-// insert c into this lane's descending list (at most k entries)
-__device__ __forceinline__ void lane_insert(unsigned long long* list, int lane, int& cnt, int k,
-                                            unsigned long long c) {
-  if (cnt == k && c <= list[(k - 1) * kWave + lane]) return;
-  int j = cnt < k ? cnt : k - 1;
-  while (j > 0 && list[(j - 1) * kWave + lane] < c) {
-    list[j * kWave + lane] = list[(j - 1) * kWave + lane];
-    --j;
-  }
-  list[j * kWave + lane] = c;
-  if (cnt < k) ++cnt;
+// log2(u) / w as the hardware's one-instruction log2 and reciprocal give it.  Over all 2^24
+// values of u the first is within 3.1e-7 of log2_u24, the second within 9.2e-8 (measured, gfx950);
+// with the roundings of the product and of the exact quotient a rough key is within 5.3e-7 of the
+// exact one.  Weights whose keys could leave the normal range take the exact key.
+constexpr float kRoughSlack = 1.9073486e-6f;  // 2^-19: twice that, and some
+__device__ __forceinline__ float rough_key(uint32_t x, float w) {
+  constexpr uint32_t kLow = 27u << 23, kSpan = 200u << 23;  // 2^-100 <= w < 2^100
+  if (__float_as_uint(w) - kLow >= kSpan) return ares_key(x, w);
+  const float u = static_cast<float>((x >> 8) + 1u) * 5.9604644775390625e-08f;
+  return __builtin_amdgcn_logf(u) * __builtin_amdgcn_rcpf(w);
 }
 
-__device__ __forceinline__ unsigned long long wave_max(unsigned long long v) {
+__device__ __forceinline__ float float_from_ordered(uint32_t o) {
+  return __uint_as_float(o & 0x80000000u ? o & 0x7FFFFFFFu : ~o);
+}
+
+// four edges a trip: draws, the weights' bits and rough keys (NaN where there is no edge); or composites,
+// the upper halves in x, the lower ones in w
+template <int TRIPS>
+struct Edges {
+  uint32_t x[4 * TRIPS], w[4 * TRIPS];
+  float rough[4 * TRIPS];
+  __device__ __forceinline__ float most() const {
+    float m = -__builtin_inff();
 #pragma unroll
-  for (int d = kWave / 2; d > 0; d >>= 1) {
-    const unsigned long long o = __shfl_xor(v, d, kWave);
-    v = o > v ? o : v;
+    for (int u = 0; u < 4 * TRIPS; ++u) m = fmaxf(m, rough[u]);
+    return m;
   }
-  return v;
-}
+};
 
-// k rounds of "largest list head wins"; emit(j, composite) is called by every
-// lane with the same arguments (0 = fewer than j+1 candidates existed).
-template <typename Emit>
-__device__ __forceinline__ void wave_drain(const unsigned long long* list, int lane, int cnt, int k,
-                                           Emit emit) {
-  int head = 0;
-  for (int j = 0; j < k; ++j) {
-    const unsigned long long mine = head < cnt ? list[head * kWave + lane] : 0ull;
-    const unsigned long long best = wave_max(mine);
-    if (best != 0ull && mine == best) ++head;
-    emit(j, best);
-  }
-}
-
-template <typename IdT>
-__device__ __forceinline__ unsigned long long edge_composite(const WArgs<IdT>& a, int64_t r,
-                                                             int64_t start, const uint32_t* rp,
-                                                             int64_t i, const U4& x) {
-  const uint32_t xv = rp ? rp[i] : x.v[i & 3];
-  return composite(ares_key(xv, a.probs[start + i]), static_cast<uint32_t>(i));
-}
-
-constexpr int kTrips = kChunk / (4 * kWave);  // a lane holds 4 consecutive edges per trip
-constexpr int64_t kSmall = 4 * kWave;         // rows of one trip: selected where they are found
-
-// composites of edges [lo, hi) of row r (lo a multiple of 2048, hi - lo <= TRIPS * 256):
-// the lane's share, 0 where it has none.  A lane takes 4 consecutive edges (one Philox
-// block) per trip.
+// Edges lo + at .. lo + at + 3 of row r (lo a multiple of 4), those below lo + len: one Philox block.
+// The weights are read without conditions, the last one again past the end, so that all are on
+// their way at once.
 template <int TRIPS, typename IdT>
-__device__ __forceinline__ void load_items(const WArgs<IdT>& a, int64_t r, int64_t start,
-                                           int64_t lo, int64_t hi, int lane,
-                                           unsigned long long (&items)[TRIPS][4]) {
-  const uint32_t* rp = a.replay ? a.replay + a.replay_ptr[r] : nullptr;
-#pragma unroll
-  for (int t = 0; t < TRIPS; ++t) {
-    const int64_t q = (lo >> 2) + lane + t * kWave;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) items[t][j] = 0ull;
-    if (q * 4 < hi) {
-      U4 x;
-      if (!rp) x = draw_block(a.seed, kTagWeighted, static_cast<uint64_t>(r), static_cast<uint64_t>(q));
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int64_t i = q * 4 + j;
-        if (i < hi) items[t][j] = edge_composite(a, r, start, rp, i, x);
-      }
-    }
-  }
-}
-
-__device__ __forceinline__ unsigned long long lane_value(unsigned long long v, int l) {
-  const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(v), l);
-  const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(v >> 32), l);
-  return (static_cast<unsigned long long>(hi) << 32) | lo;
-}
-
-// The k largest of the wave's items, in descending order: emit(place, composite) is called
-// once per winner by the lane that holds it in the end; returns how many there were
-// (fewer than k when the wave holds fewer items).  `list` is the wave's k * 64 LDS words.
-// Every lane of the wave calls this.
-template <int TRIPS, typename Emit>
-__device__ __forceinline__ int wave_topk(const unsigned long long (&items)[TRIPS][4],
-                                         unsigned long long* list, int lane, int k, Emit emit) {
-  unsigned long long mx = 0ull;
-#pragma unroll
-  for (int t = 0; t < TRIPS; ++t)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) mx = items[t][j] > mx ? items[t][j] : mx;
-  // floor: the k-th largest of the lanes' maxima (composites are distinct; lanes without
-  // items hold 0 and never qualify).  At least k items reach it, so the winners do.
-  int greater = 0;
-#pragma unroll 8
-  for (int l = 0; l < kWave; ++l) greater += lane_value(mx, l) > mx ? 1 : 0;
-  const unsigned long long holder = __ballot(mx != 0ull && greater == k - 1);
-  const unsigned long long floor_c = holder ? lane_value(mx, __ffsll(holder) - 1) : 0ull;
-  // survivors, packed into LDS in (trip, item, lane) order
-  const unsigned long long lower = (1ull << lane) - 1ull;
-  int n = 0;
-#pragma unroll
-  for (int t = 0; t < TRIPS; ++t) {
+__device__ __forceinline__ void load_edges(const WArgs<IdT>& a, int64_t r, int64_t start, int64_t lo,
+                                           int len, int at, int trip, Edges<TRIPS>& e) {
+  const int wave_at = __builtin_amdgcn_readfirstlane(at);
+  if (wave_at >= len) {  // the whole wave is past the end
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const bool keep = items[t][j] != 0ull && items[t][j] >= floor_c;
-      const unsigned long long votes = __ballot(keep);
-      if (keep) list[n + __popcll(votes & lower)] = items[t][j];
-      n += __popcll(votes);
-    }
-  }
-  // the wave's own stores must have landed before other lanes read them back
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-  for (int i = lane; i < n; i += kWave) {
-    const unsigned long long mine = list[i];
-    int place = 0;
-    for (int x = 0; x < n; ++x) place += list[x] > mine ? 1 : 0;
-    if (place < k) emit(place, mine);
-  }
-  // the list is free again only when every lane has finished reading it
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-  return n < k ? n : k;
-}
-
-// pick number j of row r is the edge the composite names; called by one lane
-template <typename IdT, bool WITH_COO>
-__device__ __forceinline__ void emit_final(const WArgs<IdT>& a, int64_t r, int64_t start,
-                                           int64_t out_start, int j, unsigned long long c) {
-  const int64_t q = start + composite_pos(c);
-  a.sub_indices[out_start + j] = a.indices[q];
-  a.select_index[out_start + j] = q;
-  if (WITH_COO) a.coo_col[out_start + j] = static_cast<IdT>(r);
-}
-
-// One wave per row.  deg <= k: copy; deg <= 256: select here; longer: queue (rows up to
-// 2048 edges as one chunk that the chunk pass finishes by itself).
-template <typename IdT, bool WITH_COO>
-__global__ void weighted_rows_kernel(WArgs<IdT> a) {
-  extern __shared__ unsigned long long s_lists[];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-  const int waves = blockDim.x / kWave;
-  unsigned long long* list = s_lists + static_cast<size_t>(wave) * a.k * kWave;
-  const int64_t r = static_cast<int64_t>(blockIdx.x) * waves + wave;
-  if (r >= a.S) return;
-  const int64_t c = a.cols ? static_cast<int64_t>(a.cols[r]) : r;
-  // an id outside [0, num_cols) is an empty column
-  if (static_cast<uint64_t>(c) >= static_cast<uint64_t>(a.num_cols)) return;
-  const int64_t start = a.indptr[c];
-  const int64_t deg = a.indptr[c + 1] - start;
-  const int64_t out_start = a.sub_indptr[r];
-  if (deg <= a.k) {
-    for (int64_t j = lane; j < deg; j += kWave) {
-      a.sub_indices[out_start + j] = a.indices[start + j];
-      a.select_index[out_start + j] = start + j;
-      if (WITH_COO) a.coo_col[out_start + j] = static_cast<IdT>(r);
+      e.x[trip * 4 + j] = 0u;
+      e.w[trip * 4 + j] = 0u;
+      e.rough[trip * 4 + j] = __builtin_nanf("");
     }
     return;
   }
-  bool here = deg <= kSmall;
-  if (!here) {
-    const int64_t nchunks = (deg + kChunk - 1) / kChunk;
-    const int64_t part = blockIdx.x & (kQueueParts - 1);
-    const int64_t part0 = part * a.chunk_cap;
-    unsigned long long base = 0;
-    if (lane == 0)
-      base = atomicAdd(&a.counters[2 + part], static_cast<unsigned long long>(nchunks));
-    base = __shfl(base, 0, kWave);
-    if (static_cast<int64_t>(base) + nchunks <= a.chunk_cap) {
-      for (int64_t ch = lane; ch < nchunks; ch += kWave)
-        a.chunk_queue[part0 + base + ch] = static_cast<long long>((r << 20) | ch);
-      if (lane == 0 && nchunks > 1) {
-        const unsigned long long slot = atomicAdd(&a.counters[1], 1ull);
-        a.long_rows[slot * 3 + 0] = r;
-        a.long_rows[slot * 3 + 1] = part0 + static_cast<long long>(base);
-        a.long_rows[slot * 3 + 2] = nchunks;
-      }
+  const float* __restrict__ probs = a.probs + (start + lo);
+  float w[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) w[j] = probs[at + j < len ? at + j : len - 1];
+  U4 x;
+  if (a.replay) {
+    const uint32_t* rp = a.replay + a.replay_ptr[r] + lo;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x.v[j] = rp[at + j < len ? at + j : len - 1];
+  } else {
+    x = draw_block(a.seed, kTagWeighted, static_cast<uint64_t>(r),
+                   static_cast<uint64_t>((lo + at) >> 2));
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    e.x[trip * 4 + j] = x.v[j];
+    e.w[trip * 4 + j] = __float_as_uint(w[j]);
+    e.rough[trip * 4 + j] = at + j < len ? rough_key(x.v[j], w[j]) : __builtin_nanf("");
+  }
+}
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float max_step(float v) {
+  return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v),
+                                                             CTRL, ROWS, 0xf, false)));
+}
+// the wave's largest value, in every lane
+__device__ __forceinline__ float wave_most(float v) {
+  v = max_step<0x111, 0xf>(v);  // row_shr:1
+  v = max_step<0x112, 0xf>(v);
+  v = max_step<0x114, 0xf>(v);
+  v = max_step<0x118, 0xf>(v);
+  v = max_step<0x142, 0xa>(v);  // row_bcast:15
+  v = max_step<0x143, 0xc>(v);  // row_bcast:31
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), kWave - 1));
+}
+
+// A value that at least k lanes reach, -inf when fewer than k hold one above that: the k-th
+// largest of the lanes' (of equal ones, one at a time).  Taking the largest away k times is ten
+// instructions each, comparing every lane with every other 200.
+__device__ __forceinline__ float wave_floor(float mine, int k) {
+  constexpr int kRounds = 16;
+  if (k <= kRounds) {
+    float f = -__builtin_inff();
+    for (int round = 0; round < k; ++round) {
+      f = wave_most(mine);
+      const unsigned long long holders = __ballot(mine == f);
+      if (static_cast<int>(threadIdx.x & (kWave - 1)) == __ffsll(holders) - 1) mine = -__builtin_inff();
+    }
+    return f;
+  }
+  int reach = 0;
+#pragma unroll 16
+  for (int l = 0; l < kWave; ++l)
+    reach += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine), l)) >= mine ? 1 : 0;
+  const unsigned long long holder = __ballot(reach == k);
+  if (holder)
+    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine), __ffsll(holder) - 1));
+  return wave_most(reach >= k ? mine : -__builtin_inff());  // equal maxima, or k above 64
+}
+
+// (keys are not positive)
+__device__ __forceinline__ float floor_with_slack(float f) { return f + f * kRoughSlack; }
+
+// how many of list[0..n) beat `mine`
+__device__ __forceinline__ int beaten_by(const unsigned long long* list, int n,
+                                         unsigned long long mine) {
+  int place = 0;
+#pragma unroll 8
+  for (int x = 0; x < n; ++x) place += list[x] > mine ? 1 : 0;
+  return place;
+}
+
+// survivors of a selection: draw << 32 | weight and the edge's place in its chunk, then the composite
+struct Shared {
+  unsigned long long list[kChunk];  // (a wave that is on its own has a quarter of it)
+  unsigned short pos[kChunk];
+  unsigned long long best[kMaxFanout];
+  float floors[kWaves];
+  int n, last;
+};
+constexpr int kWaveList = kChunk / kWaves;
+
+// packs the edges whose rough key reaches `cut` from list[at] on, in the order (trip, item, lane);
+// item j of trip t is edge first + t * step + j of the chunk
+template <int TRIPS>
+__device__ __forceinline__ void pack(const Edges<TRIPS>& e, float cut, int at, int first, int step,
+                                     unsigned long long* list, unsigned short* pos) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const unsigned long long lower = (1ull << lane) - 1ull;
+#pragma unroll
+  for (int u = 0; u < 4 * TRIPS; ++u) {
+    const bool keep = e.rough[u] >= cut;
+    const unsigned long long votes = __ballot(keep);
+    if (keep) {
+      const int slot = at + __popcll(votes & lower);
+      list[slot] = (static_cast<unsigned long long>(e.x[u]) << 32) | e.w[u];
+      pos[slot] = static_cast<unsigned short>(first + (u >> 2) * step + (u & 3));
+    }
+    at += __popcll(votes);
+  }
+}
+template <int TRIPS>
+__device__ __forceinline__ int count_kept(const Edges<TRIPS>& e, float cut) {
+  int n = 0;
+#pragma unroll
+  for (int u = 0; u < 4 * TRIPS; ++u) n += __popcll(__ballot(e.rough[u] >= cut));
+  return n;
+}
+
+__device__ __forceinline__ unsigned long long exact_composite(unsigned long long packed,
+                                                              uint32_t pos) {
+  return composite(ares_key(static_cast<uint32_t>(packed >> 32),
+                            __uint_as_float(static_cast<uint32_t>(packed))),
+                   pos);
+}
+
+// The k best of the wave's edges [lo, lo + 256) and of the k composites in `best` (null: none) go to
+// emit(place, composite), called once per winner by the lane that holds it in the end.  `list`
+// and `pos` are the wave's own.  Every lane of the wave calls this.
+template <typename Emit>
+__device__ __forceinline__ void wave_topk(const Edges<1>& e, int64_t lo,
+                                          const unsigned long long* best,
+                                          unsigned long long* list, unsigned short* pos, int k,
+                                          Emit emit) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const float cut = floor_with_slack(wave_floor(e.most(), k));
+  int n = count_kept(e, cut);
+  pack(e, cut, 0, 4 * lane, 0, list, pos);
+  // the wave's own stores must have landed before other lanes read them back
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup", "local");
+  for (int i = lane; i < n; i += kWave)
+    list[i] = exact_composite(list[i], static_cast<uint32_t>(lo) + pos[i]);
+  if (best) {
+    for (int i = lane; i < k; i += kWave) list[n + i] = best[i];
+    n += k;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup", "local");
+  for (int i = lane; i < n; i += kWave) {
+    const unsigned long long mine = list[i];
+    const int place = beaten_by(list, n, mine);
+    if (place < k) emit(place, mine);
+  }
+  // the list is free again only when every lane has finished reading it
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup", "local");
+}
+
+// The k best of a workgroup's edges [lo, lo + 2048), or composites; returns how many there were.
+// Every thread calls this; item j of trip t is edge lo + 4 * (t * 256 + the thread's number) + j.
+// Every lane of the first `full` waves holds items: ceil(k / full) in each of them reach the
+// lowest of these waves' floors.
+template <bool COMPOSITES, int TRIPS, typename Emit>
+__device__ __forceinline__ int group_topk(const Edges<TRIPS>& e, int64_t lo, int full,
+                                          Shared& s, int k, Emit emit) {
+  static_assert(4 * TRIPS * kThreads <= kChunk, "the list holds every edge");
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  if (wave < full) {
+    const float mine = wave_floor(e.most(), (k + full - 1) / full);
+    if (lane == 0) s.floors[wave] = mine;
+  }
+  if (threadIdx.x == 0) s.n = 0;
+  lds_barrier();
+  float floor_all = full > 0 ? s.floors[0] : -__builtin_inff();
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w)
+    if (w < full) floor_all = fminf(floor_all, s.floors[w]);
+  const float cut = floor_with_slack(floor_all);
+  const int count = count_kept(e, cut);
+  int at = 0;
+  if (lane == 0 && count > 0) at = atomicAdd(&s.n, count);
+  at = __builtin_amdgcn_readfirstlane(at);
+  if (count > 0) pack(e, cut, at, 4 * static_cast<int>(threadIdx.x), 4 * kThreads, s.list, s.pos);
+  lds_barrier();
+  const int n = s.n;
+  if (!COMPOSITES) {
+    for (int i = threadIdx.x; i < n; i += kThreads)
+      s.list[i] = exact_composite(s.list[i], static_cast<uint32_t>(lo) + s.pos[i]);
+    lds_barrier();
+  }
+  for (int i = threadIdx.x; i < n; i += kThreads) {
+    const unsigned long long one = s.list[i];
+    const int place = beaten_by(s.list, n, one);
+    if (place < k) emit(place, one);
+  }
+  lds_barrier();
+  return n < k ? n : k;
+}
+
+// output o is the edge at position q, of row r
+template <typename IdT, bool WITH_COO>
+__device__ __forceinline__ void emit_edge(const WArgs<IdT>& a, int64_t r, int64_t o, int64_t q) {
+  const IdT id = a.indices[q];
+  if (a.data_out) a.data_out[o] = a.edge_data[q];
+  a.sub_indices[o] = id;
+  a.select_index[o] = q;
+  if (WITH_COO) a.coo_col[o] = static_cast<IdT>(r);
+}
+
+// Lays out the chunks of the rows above 256 edges: an entry each, a row's one after the other.  A
+// workgroup reserves for its 1024 rows at once (a single one does not need the counter, which
+// is then not cleared before either).
+template <typename IdT>
+__global__ void __launch_bounds__(kPlanRows) weighted_plan_kernel(WArgs<IdT> a) {
+  __shared__ int64_t s_scan[kPlanRows / kWave + 1];
+  __shared__ int64_t s_base;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t r = static_cast<int64_t>(blockIdx.x) * kPlanRows + threadIdx.x;
+  int64_t start = 0, deg = 0, out = 0;
+  if (r < a.S) {
+    const int64_t col = a.cols ? static_cast<int64_t>(a.cols[r]) : r;
+    out = a.sub_indptr[r];
+    // an id outside [0, num_cols) is an empty column
+    if (static_cast<uint64_t>(col) < static_cast<uint64_t>(a.num_cols)) {
+      start = a.indptr[col];
+      deg = a.indptr[col + 1] - start;
+    }
+  }
+  const int64_t chunks = deg > kChunk ? (deg + kChunk - 1) / kChunk : 0;
+  const bool single = deg > kSmall && chunks == 0;
+  int64_t total;
+  int64_t at = block_exclusive_scan<kPlanRows>((chunks << 32) | (single ? 1 : 0), &total, s_scan);
+  if (threadIdx.x == 0) {
+    if (gridDim.x == 1) {
+      *a.reserved = static_cast<unsigned long long>(total);
+      s_base = 0;
     } else {
-      // this part of the queue is full: void the reserved tail and select the whole row with
-      // this wave
-      for (int64_t ch = static_cast<int64_t>(base) + lane;
-           ch < a.chunk_cap && ch < static_cast<int64_t>(base) + nchunks; ch += kWave)
-        a.chunk_queue[part0 + ch] = -1;
-      here = true;
+      s_base = static_cast<int64_t>(atomicAdd(a.reserved, static_cast<unsigned long long>(total)));
     }
   }
-  if (here && deg <= kSmall) {
-    unsigned long long items[1][4];
-    load_items<1>(a, r, start, 0, deg, lane, items);
-    wave_topk<1>(items, list, lane, a.k, [&](int j, unsigned long long c) {
-      emit_final<IdT, WITH_COO>(a, r, start, out_start, j, c);
-    });
-  } else if (here) {
-    // a row that found the queue full: this wave streams it whole
-    int cnt = 0;
-    for (int64_t i = lane; i < deg; i += kWave) {
-      U4 x;
-      const uint32_t* rp = a.replay ? a.replay + a.replay_ptr[r] : nullptr;
-      if (!rp) x = draw_block(a.seed, kTagWeighted, static_cast<uint64_t>(r), static_cast<uint64_t>(i >> 2));
-      lane_insert(list, lane, cnt, a.k, edge_composite(a, r, start, rp, i, x));
-    }
-    wave_drain(list, lane, cnt, a.k, [&](int j, unsigned long long best) {
-      if (lane == (j & (kWave - 1)) && best != 0ull)
-        emit_final<IdT, WITH_COO>(a, r, start, out_start, j, best);
-    });
+  __syncthreads();
+  at += s_base;
+  if (single) {
+    const int64_t e = kHubTasks + (at & 0xFFFFFFFF);
+    a.tasks[e] = Task{r, start, deg, out, e};
+  }
+  at >>= 32;
+  // a row whose chunks do not all fit is left to its wave of the fill (its entries are void)
+  const Task t{at + chunks <= kHubTasks ? r : -1, start, deg, out, at};
+  if (chunks > 0) {
+    a.row_base[r] = at;
+    if (at < kHubTasks) a.done[at] = 0u;
+  }
+  // a few entries are written by the row's lane, many by its whole wave
+  constexpr int64_t kFew = 4;
+  if (chunks <= kFew)
+    for (int64_t e = at; e < at + chunks && e < kHubTasks; ++e) a.tasks[e] = t;
+  unsigned long long hubs = __ballot(chunks > kFew);
+  while (hubs) {
+    const int l = __ffsll(hubs) - 1;
+    hubs &= hubs - 1;
+    const Task h{__shfl(t.row, l, kWave), __shfl(t.start, l, kWave), __shfl(t.deg, l, kWave),
+                 __shfl(t.out, l, kWave), __shfl(t.base, l, kWave)};
+    const int64_t n = __shfl(chunks, l, kWave);
+    for (int64_t e = h.base + lane; e < h.base + n && e < kHubTasks; e += kWave) a.tasks[e] = h;
   }
 }
 
-// One wave per queued chunk: local top-k composites -> cand[slot * k + j]; the only chunk
-// of a row is final and goes to the output.
+// a chunk: its k largest go to the output when it is the row's only one, else to cand, and the
+// row's last chunk to get there merges them
 template <typename IdT, bool WITH_COO>
-__global__ void weighted_chunks_kernel(WArgs<IdT> a) {
-  extern __shared__ unsigned long long s_lists[];
+__device__ __forceinline__ void run_task(const WArgs<IdT>& a, const Task& e, int64_t t, Shared& s) {
+  const auto emit_final = [&](int j, unsigned long long c) {
+    emit_edge<IdT, WITH_COO>(a, e.row, e.out + j, e.start + composite_pos(c));
+  };
+  const int64_t lo = (t - e.base) * kChunk;
+  const int len = static_cast<int>(kChunk < e.deg - lo ? kChunk : e.deg - lo);
+  constexpr int kTrips = kChunk / (4 * kThreads);
+  Edges<kTrips> edges;
+#pragma unroll
+  for (int trip = 0; trip < kTrips; ++trip)
+    load_edges(a, e.row, e.start, lo, len, 4 * static_cast<int>(threadIdx.x + trip * kThreads), trip,
+               edges);
+  const int full_here = len >= kWaves * kSmall ? kWaves : len / static_cast<int>(kSmall);
+  if (e.deg <= kChunk) {
+    group_topk<false>(edges, lo, full_here, s, a.k, emit_final);
+    return;
+  }
+  unsigned long long* out = a.cand + static_cast<size_t>(t) * a.k;
+  const int found = group_topk<false>(edges, lo, full_here, s, a.k, [&](int j, unsigned long long c) { lb_store(&out[j], c); });
+  for (int j = found + threadIdx.x; j < a.k; j += kThreads) lb_store(&out[j], 0ull);  // fewer than k edges
+  const int64_t chunks = (e.deg + kChunk - 1) / kChunk;
+  // the candidates are stored and read with device scope and every wave's have completed before
+  // the workgroup counts itself (an L2 released per chunk: 52 us a fill, so 30)
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __syncthreads();
+  if (threadIdx.x == 0)
+    s.last = __hip_atomic_fetch_add(&a.done[e.base], 1u, __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT) == static_cast<unsigned>(chunks - 1);
+  __syncthreads();
+  if (!s.last) return;
+  // 2048 candidates at a time, from the second time on the k best so far in front of the next
+  // ones (k of them: the row's first chunk is full)
+  const int64_t m = chunks * a.k;
+  const unsigned long long* src = a.cand + static_cast<size_t>(e.base) * a.k;
+  int64_t taken = 0;
+  int kept = 0, full = 0;
+  while (true) {
+#pragma unroll
+    for (int u = 0; u < 4 * kTrips; ++u) {
+      const int i = u * kThreads + static_cast<int>(threadIdx.x);
+      const int64_t from = taken + i - kept;
+      const unsigned long long c = i < kept ? s.best[i] : (from < m ? lb_load(&src[from]) : 0ull);
+      edges.x[u] = static_cast<uint32_t>(c >> 32);
+      edges.w[u] = static_cast<uint32_t>(c);
+      edges.rough[u] = c ? float_from_ordered(edges.x[u]) : __builtin_nanf("");
+    }
+    const int64_t here = kept + (m - taken < kChunk - kept ? m - taken : kChunk - kept);
+    full = here >= kThreads ? kWaves : static_cast<int>(here) / kWave;
+    taken += kChunk - kept;
+    kept = a.k;
+    if (taken >= m) break;
+    group_topk<true>(edges, 0, full, s, a.k, [&](int j, unsigned long long c) { s.best[j] = c; });
+  }
+  group_topk<true>(edges, 0, full, s, a.k, emit_final);
+}
+
+// Workgroups below kQueueGrid take chunks, the others four rows each, a wave a row: deg <= k: copy;
+// deg <= 256: select here; longer: the row's chunks are somebody else's.
+// 5000 columns of 233 k with 114.6 M edges, fanout 25 (2.6 M edges looked at): 26 us and 6 for the
+// layout; as rows, chunks and merge one after the other, with exact keys for all, it was 51.
+// A third of that is instructions, the rest the trips of a task: two rounds of workgroups.
+template <typename IdT, bool WITH_COO>
+__global__ void __launch_bounds__(kThreads) weighted_fill_kernel(WArgs<IdT> a) {
+  __shared__ Shared s;
+  const int64_t chunks = static_cast<int64_t>(*a.reserved >> 32);
+  if (blockIdx.x < kQueueGrid) {
+    const int64_t hubs = chunks < kHubTasks ? chunks : kHubTasks;
+    const int64_t n = hubs + static_cast<int64_t>(*a.reserved & 0xFFFFFFFFu);
+    for (int64_t i = blockIdx.x; i < n; i += kQueueGrid) {
+      const int64_t t = i < hubs ? i : kHubTasks + i - hubs;
+      const Task e = a.tasks[t];
+      if (e.row >= 0) run_task<IdT, WITH_COO>(a, e, t, s);
+    }
+    return;
+  }
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
-  const int waves = blockDim.x / kWave;
-  unsigned long long* list = s_lists + static_cast<size_t>(wave) * a.k * kWave;
-  // lane q: entries of part q, and how many lie in the parts before it
-  static_assert(kQueueParts == kWave, "one lane per part of the queue");
-  const unsigned long long reserved = a.counters[2 + lane];
-  const int64_t mine = reserved < static_cast<unsigned long long>(a.chunk_cap)
-                           ? static_cast<int64_t>(reserved)
-                           : a.chunk_cap;
-  int64_t incl = mine;
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const int64_t o = __shfl_up(incl, d, kWave);
-    if (lane >= d) incl += o;
+  const int64_t r = static_cast<int64_t>(blockIdx.x - kQueueGrid) * kWaves + wave;
+  if (r >= a.S) return;
+  const int64_t c = a.cols ? static_cast<int64_t>(a.cols[r]) : r;
+  if (static_cast<uint64_t>(c) >= static_cast<uint64_t>(a.num_cols)) return;
+  const int64_t start = a.indptr[c];
+  const int64_t deg = a.indptr[c + 1] - start;
+  const int64_t out = a.sub_indptr[r];
+  if (deg <= a.k) {
+    for (int64_t j = lane; j < deg; j += kWave)
+      emit_edge<IdT, WITH_COO>(a, r, out + j, start + j);
+    return;
   }
-  const int64_t before = incl - mine;
-  const int64_t n = __shfl(incl, kWave - 1, kWave);
-  for (int64_t v = static_cast<int64_t>(blockIdx.x) * waves + wave; v < n;
-       v += static_cast<int64_t>(gridDim.x) * waves) {
-    int lo_part = 0, hi_part = kQueueParts;  // the last part that starts at or before v
-#pragma unroll
-    for (int step = 0; step < 6; ++step) {
-      const int mid = (lo_part + hi_part) >> 1;
-      if (__shfl(before, mid, kWave) <= v) lo_part = mid; else hi_part = mid;
-    }
-    const int64_t t = static_cast<int64_t>(lo_part) * a.chunk_cap + (v - __shfl(before, lo_part, kWave));
-    const long long e = a.chunk_queue[t];
-    if (e < 0) continue;
-    const int64_t r = e >> 20;
-    const int64_t ch = e & ((1 << 20) - 1);
-    const int64_t c = a.cols ? static_cast<int64_t>(a.cols[r]) : r;
-    const int64_t start = a.indptr[c];
-    const int64_t deg = a.indptr[c + 1] - start;
-    const int64_t lo = ch * kChunk;
-    const int64_t hi = lo + kChunk < deg ? lo + kChunk : deg;
-    unsigned long long items[kTrips][4];
-    load_items<kTrips>(a, r, start, lo, hi, lane, items);
-    if (deg <= kChunk) {
-      const int64_t out_start = a.sub_indptr[r];
-      wave_topk<kTrips>(items, list, lane, a.k, [&](int j, unsigned long long c) {
-        emit_final<IdT, WITH_COO>(a, r, start, out_start, j, c);
-      });
-      continue;
-    }
-    unsigned long long* out = a.cand + static_cast<size_t>(t) * a.k;
-    const int found = wave_topk<kTrips>(items, list, lane, a.k,
-                                        [&](int j, unsigned long long c) { out[j] = c; });
-    for (int j = found + lane; j < a.k; j += kWave) out[j] = 0ull;  // fewer than k edges
+  unsigned long long* list = s.list + wave * kWaveList;
+  unsigned short* pos = s.pos + wave * kWaveList;
+  const auto emit_final = [&](int j, unsigned long long cmp) {
+    emit_edge<IdT, WITH_COO>(a, r, out + j, start + composite_pos(cmp));
+  };
+  Edges<1> edges;
+  if (deg <= kSmall) {
+    load_edges(a, r, start, 0, static_cast<int>(deg), 4 * lane, 0, edges);
+    wave_topk(edges, 0, nullptr, list, pos, a.k, emit_final);
+    return;
   }
+  if (deg <= kChunk || chunks <= kHubTasks ||
+      a.row_base[r] + (deg + kChunk - 1) / kChunk <= kHubTasks)
+    return;
+  // a row that found the queue full: 256 edges at a time, the k best so far beside them
+  static_assert(kSmall + 2 * kMaxFanout <= kWaveList, "the quarter holds both and the best of them");
+  unsigned long long* best = list + kSmall + kMaxFanout;
+  for (int64_t lo = 0; lo < deg; lo += kSmall) {
+    load_edges(a, r, start, lo, static_cast<int>(kSmall < deg - lo ? kSmall : deg - lo), 4 * lane, 0,
+               edges);
+    wave_topk(edges, lo, lo > 0 ? best : nullptr, list, pos, a.k,
+              [&](int j, unsigned long long cmp) { best[j] = cmp; });
+  }
+  for (int j = lane; j < a.k; j += kWave) emit_final(j, best[j]);
 }
 
-// One wave per long row: merge its chunks' candidates.
-template <typename IdT, bool WITH_COO>
-__global__ void weighted_merge_kernel(WArgs<IdT> a) {
-  extern __shared__ unsigned long long s_lists[];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-  const int waves = blockDim.x / kWave;
-  unsigned long long* list = s_lists + static_cast<size_t>(wave) * a.k * kWave;
-  const int64_t n = static_cast<int64_t>(a.counters[1]);
-  for (int64_t t = static_cast<int64_t>(blockIdx.x) * waves + wave; t < n;
-       t += static_cast<int64_t>(gridDim.x) * waves) {
-    const int64_t r = a.long_rows[t * 3 + 0];
-    const int64_t base = a.long_rows[t * 3 + 1];
-    const int64_t m = a.long_rows[t * 3 + 2] * a.k;
-    const int64_t c = a.cols ? static_cast<int64_t>(a.cols[r]) : r;
-    const int64_t start = a.indptr[c];
-    const int64_t out_start = a.sub_indptr[r];
-    const unsigned long long* src = a.cand + static_cast<size_t>(base) * a.k;
-    if (m <= kChunk) {
-      // few enough candidates for the register-resident selection (0 = an empty slot)
-      unsigned long long items[kTrips][4];
-#pragma unroll
-      for (int tr = 0; tr < kTrips; ++tr)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int64_t i = (static_cast<int64_t>(tr) * 4 + j) * kWave + lane;
-          items[tr][j] = i < m ? src[i] : 0ull;
-        }
-      wave_topk<kTrips>(items, list, lane, a.k, [&](int j, unsigned long long cmp) {
-        emit_final<IdT, WITH_COO>(a, r, start, out_start, j, cmp);
-      });
-      continue;
-    }
-    int cnt = 0;
-    for (int64_t i = lane; i < m; i += kWave) {
-      const unsigned long long cmp = src[i];
-      if (cmp != 0ull) lane_insert(list, lane, cnt, a.k, cmp);
-    }
-    wave_drain(list, lane, cnt, a.k, [&](int j, unsigned long long best) {
-      if (lane == (j & (kWave - 1)) && best != 0ull)
-        emit_final<IdT, WITH_COO>(a, r, start, out_start, j, best);
-    });
-  }
-}
-
-static __global__ void zero2_kernel(unsigned long long* p) {
-  for (int i = threadIdx.x; i < 2 + kQueueParts; i += blockDim.x) p[i] = 0;
-}
-
-int waves_per_block(int64_t k) {
-  // 48 KB of LDS per workgroup
-  const int64_t per_wave = k * kWave * 8;
-  int w = static_cast<int>((48 * 1024) / per_wave);
-  return w >= 4 ? 4 : (w >= 2 ? 2 : 1);
-}
+static __global__ void zero_kernel(unsigned long long* p) { *p = 0; }
 
 template <typename IdT, bool WITH_COO>
 int weighted_launch(const WArgs<IdT>& a, hipStream_t st) {
-  const int waves = waves_per_block(a.k);
-  const size_t lds = static_cast<size_t>(waves) * a.k * kWave * 8;
-  const dim3 block(waves * kWave);
-  hipLaunchKernelGGL(zero2_kernel, dim3(1), dim3(64), 0, st, a.counters);
-  hipLaunchKernelGGL((weighted_rows_kernel<IdT, WITH_COO>),
-                     dim3(static_cast<unsigned>((a.S + waves - 1) / waves)), block, lds, st, a);
-  hipLaunchKernelGGL((weighted_chunks_kernel<IdT, WITH_COO>), dim3(kQueueGrid), block, lds, st, a);
-  hipLaunchKernelGGL((weighted_merge_kernel<IdT, WITH_COO>), dim3(kQueueGrid), block, lds, st, a);
+  const unsigned plan = static_cast<unsigned>((a.S + kPlanRows - 1) / kPlanRows);
+  ProfileScope prof("sample_weighted", st);
+  if (plan > 1) hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(1), 0, st, a.reserved);
+  hipLaunchKernelGGL((weighted_plan_kernel<IdT>), dim3(plan), dim3(kPlanRows), 0, st, a);
+  hipLaunchKernelGGL((weighted_fill_kernel<IdT, WITH_COO>),
+                     dim3(static_cast<unsigned>(kQueueGrid + (a.S + kWaves - 1) / kWaves)),
+                     dim3(kThreads), 0, st, a);
   return check_launch("sample_weighted");
 }
 
@@ -404,8 +521,8 @@ template <typename IdT>
 int weighted_impl(const int64_t* indptr, int64_t num_cols, const void* indices, const float* probs,
                   const void* cols, int64_t S, int64_t k, uint64_t seed, const uint32_t* replay,
                   const int64_t* replay_ptr, const int64_t* sub_indptr, void* sub_indices,
-                  int64_t* select_index, void* coo_col, void* workspace, size_t workspace_bytes,
-                  hipStream_t st) {
+                  int64_t* select_index, void* coo_col, const float* edge_data, float* data_out,
+                  void* workspace, size_t workspace_bytes, hipStream_t st) {
   Carver ws(workspace, workspace_bytes);
   WArgs<IdT> a;
   a.indptr = indptr;
@@ -422,11 +539,13 @@ int weighted_impl(const int64_t* indptr, int64_t num_cols, const void* indices, 
   a.sub_indices = static_cast<IdT*>(sub_indices);
   a.select_index = select_index;
   a.coo_col = static_cast<IdT*>(coo_col);
-  a.chunk_cap = (S + kQueueExtra) / kQueueParts;
-  a.counters = ws.take<unsigned long long>(2 + kQueueParts);
-  a.chunk_queue = ws.take<long long>(static_cast<size_t>(a.chunk_cap) * kQueueParts);
-  a.long_rows = ws.take<long long>(static_cast<size_t>(S) * 3);
-  a.cand = ws.take<unsigned long long>(static_cast<size_t>(a.chunk_cap) * kQueueParts * k);
+  a.edge_data = edge_data;
+  a.data_out = data_out;
+  a.reserved = ws.take<unsigned long long>(1);
+  a.tasks = ws.take<Task>(static_cast<size_t>(kHubTasks + S));
+  a.row_base = ws.take<int64_t>(static_cast<size_t>(S));
+  a.done = ws.take<unsigned int>(static_cast<size_t>(kHubTasks));
+  a.cand = ws.take<unsigned long long>(static_cast<size_t>(kHubTasks) * k);
   if (!ws.ok) {
     set_error_text("gs_sample_weighted_fill: workspace needs %zu bytes, 256-byte aligned",
                    gs_sample_weighted_workspace_bytes(S, k));
@@ -704,17 +823,19 @@ extern "C" {
 size_t gs_sample_weighted_workspace_bytes(int64_t S, int64_t fanout) {
   if (S < 0) S = 0;
   if (fanout < 1) fanout = 1;
-  const size_t cap = static_cast<size_t>(S + kQueueExtra);
-  return padded((2 + kQueueParts) * 8) + padded(cap * 8) + padded(static_cast<size_t>(S) * 24) +
-         padded(cap * static_cast<size_t>(fanout) * 8);
+  const size_t hubs = static_cast<size_t>(kHubTasks);
+  return padded(8) + padded((hubs + static_cast<size_t>(S)) * sizeof(Task)) +
+         padded(static_cast<size_t>(S) * 8) + padded(hubs * 4) +
+         padded(hubs * static_cast<size_t>(fanout) * 8);
 }
 
-int gs_sample_weighted_fill(const int64_t* indptr, int64_t num_cols, const void* indices,
-                            const float* probs, const void* column_ids, int id_bytes, int64_t S,
-                            int64_t fanout,
-                            uint64_t seed, const uint32_t* replay, const int64_t* replay_ptr,
-                            const int64_t* sub_indptr, void* sub_indices, int64_t* select_index,
-                            void* coo_col, void* workspace, size_t workspace_bytes, void* stream) {
+int gs_sample_weighted_fill_data(const int64_t* indptr, int64_t num_cols, const void* indices,
+                                 const float* probs, const void* column_ids, int id_bytes,
+                                 int64_t S, int64_t fanout, uint64_t seed, const uint32_t* replay,
+                                 const int64_t* replay_ptr, const int64_t* sub_indptr,
+                                 void* sub_indices, int64_t* select_index, void* coo_col,
+                                 const float* edge_data, float* data_out, void* workspace,
+                                 size_t workspace_bytes, void* stream) {
   GS_REQUIRE(indptr && sub_indptr && S >= 0 && fanout >= 0 && num_cols >= 0,
              "gs_sample_weighted_fill: null pointer or negative size");
   GS_REQUIRE(column_ids || S <= num_cols,
@@ -726,20 +847,31 @@ int gs_sample_weighted_fill(const int64_t* indptr, int64_t num_cols, const void*
   if (S == 0 || fanout == 0) return GS_OK;
   GS_REQUIRE(indices && probs && sub_indices && select_index,
              "gs_sample_weighted_fill: null buffer");
+  GS_REQUIRE((edge_data == nullptr) == (data_out == nullptr),
+             "gs_sample_weighted_fill: edge_data and data_out go together");
   if (fanout > kMaxFanout) {
-    set_error_text("gs_sample_weighted_fill: fanout %lld above the supported %lld "
+    set_error_text("gs_sample_weighted_fill: fanout %lld above the supported %d "
                    "(the reference stops at 32)",
-                   static_cast<long long>(fanout), static_cast<long long>(kMaxFanout));
+                   static_cast<long long>(fanout), kMaxFanout);
     return GS_ERR_UNSUPPORTED;
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  return id_bytes == 8
-             ? weighted_impl<int64_t>(indptr, num_cols, indices, probs, column_ids, S, fanout, seed, replay,
-                                      replay_ptr, sub_indptr, sub_indices, select_index, coo_col,
-                                      workspace, workspace_bytes, st)
-             : weighted_impl<int32_t>(indptr, num_cols, indices, probs, column_ids, S, fanout, seed, replay,
-                                      replay_ptr, sub_indptr, sub_indices, select_index, coo_col,
-                                      workspace, workspace_bytes, st);
+  const auto impl = id_bytes == 8 ? weighted_impl<int64_t> : weighted_impl<int32_t>;
+  return impl(indptr, num_cols, indices, probs, column_ids, S, fanout, seed, replay, replay_ptr,
+              sub_indptr, sub_indices, select_index, coo_col, edge_data, data_out, workspace,
+              workspace_bytes, st);
+}
+
+int gs_sample_weighted_fill(const int64_t* indptr, int64_t num_cols, const void* indices,
+                            const float* probs, const void* column_ids, int id_bytes, int64_t S,
+                            int64_t fanout,
+                            uint64_t seed, const uint32_t* replay, const int64_t* replay_ptr,
+                            const int64_t* sub_indptr, void* sub_indices, int64_t* select_index,
+                            void* coo_col, void* workspace, size_t workspace_bytes, void* stream) {
+  return gs_sample_weighted_fill_data(indptr, num_cols, indices, probs, column_ids, id_bytes, S,
+                                      fanout, seed, replay, replay_ptr, sub_indptr, sub_indices,
+                                      select_index, coo_col, nullptr, nullptr, workspace,
+                                      workspace_bytes, stream);
 }
 
 int gs_sample_weighted_replace(const int64_t* indptr, int64_t num_cols, const void* indices,

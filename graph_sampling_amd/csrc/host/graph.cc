@@ -454,9 +454,17 @@ c10::intrusive_ptr<Graph> Graph::SampleImpl(int64_t axis, const torch::Tensor* e
   const bool with_coo = output_format & _COO;
   std::shared_ptr<CSC> fmt = on_csc ? csc_ : csr_;
   std::shared_ptr<_TMP> tmp;
-  torch::Tensor select_index;
+  torch::Tensor select_index, carried;
+  // the sampler's own launch gathers the edge data where one value belongs to every position and
+  // nobody follows them
+  const bool carry = edge_probs && !replace && data_.has_value() && !fmt->e_ids.has_value() &&
+                     hip::EdgeData::Fits(data_.value(), fmt->e_ids) &&
+                     !hip::EdgeData::Followed(data_.value()) &&
+                     data_.value().numel() >= fmt->indices.numel();
   if (edge_probs)
-    std::tie(tmp, select_index) = CSCColSamplingProbs(fmt, *edge_probs, fanout, replace, with_coo);
+    std::tie(tmp, select_index) =
+        CSCColSamplingProbs(fmt, *edge_probs, fanout, replace, with_coo,
+                            carry ? &data_.value() : nullptr, carry ? &carried : nullptr);
   else
     std::tie(tmp, select_index) = CSCColSampling(fmt, fanout, replace, with_coo);
 
@@ -472,7 +480,10 @@ c10::intrusive_ptr<Graph> Graph::SampleImpl(int64_t axis, const torch::Tensor* e
                                                    torch::nullopt, true, false}));
   }
   ret->SetNumEdges(tmp->coo_in_indices.numel());
-  InheritData(ret.get(), fmt->e_ids, select_index);
+  if (carry)
+    ret->SetData(carried);
+  else
+    InheritData(ret.get(), fmt->e_ids, select_index);
   return ret;
 }
 

@@ -52,12 +52,11 @@ std::pair<std::shared_ptr<_TMP>, torch::Tensor> CSCColSampling(std::shared_ptr<C
   return Wrap(hip::ColSampling(csc->indptr, csc->indices, torch::Tensor(), fanout, replace, with_coo));
 }
 
-std::pair<std::shared_ptr<_TMP>, torch::Tensor> CSCColSamplingProbs(std::shared_ptr<CSC> csc,
-                                                                    torch::Tensor edge_probs,
-                                                                    int64_t fanout, bool replace,
-                                                                    bool with_coo) {
+std::pair<std::shared_ptr<_TMP>, torch::Tensor> CSCColSamplingProbs(
+    std::shared_ptr<CSC> csc, torch::Tensor edge_probs, int64_t fanout, bool replace, bool with_coo,
+    const torch::Tensor* edge_data, torch::Tensor* data_out) {
   return Wrap(hip::ColSamplingProbs(csc->indptr, csc->indices, edge_probs, torch::Tensor(), fanout,
-                                    replace, with_coo));
+                                    replace, with_coo, edge_data, data_out));
 }
 
 std::pair<std::shared_ptr<CSC>, torch::Tensor> FusedCSCColSlicingAndSampling(

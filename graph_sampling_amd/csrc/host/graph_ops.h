@@ -38,10 +38,10 @@ std::pair<std::shared_ptr<_TMP>, torch::Tensor> CSCColSampling(std::shared_ptr<C
                                                                int64_t fanout, bool replace,
                                                                bool with_coo);
 
-std::pair<std::shared_ptr<_TMP>, torch::Tensor> CSCColSamplingProbs(std::shared_ptr<CSC> csc,
-                                                                    torch::Tensor edge_probs,
-                                                                    int64_t fanout, bool replace,
-                                                                    bool with_coo);
+// edge_data, data_out: as for hip::ColSamplingProbs
+std::pair<std::shared_ptr<_TMP>, torch::Tensor> CSCColSamplingProbs(
+    std::shared_ptr<CSC> csc, torch::Tensor edge_probs, int64_t fanout, bool replace, bool with_coo,
+    const torch::Tensor* edge_data = nullptr, torch::Tensor* data_out = nullptr);
 
 std::pair<std::shared_ptr<CSC>, torch::Tensor> FusedCSCColSlicingAndSampling(
     std::shared_ptr<CSC> csc, torch::Tensor node_ids, int64_t fanout, bool replace);

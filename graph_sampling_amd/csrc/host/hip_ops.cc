@@ -580,10 +580,12 @@ SliceResult ColSampling(const torch::Tensor& indptr, const torch::Tensor& indice
 
 SliceResult ColSamplingProbs(const torch::Tensor& indptr, const torch::Tensor& indices,
                              const torch::Tensor& probs, const torch::Tensor& column_ids,
-                             int64_t fanout, bool replace, bool with_coo) {
+                             int64_t fanout, bool replace, bool with_coo,
+                             const torch::Tensor* edge_data, torch::Tensor* data_out) {
   NeedF32(probs, "edge_probs");
   const int64_t S = column_ids.defined() ? column_ids.numel() : indptr.numel() - 1;
   if (replace) {
+    TORCH_CHECK(!edge_data, "edge data ride along only without replacement");
     // inverse-CDF picks; the prefix sums of every column live in a scratch laid out like
     // the edges themselves (the offsets of the input, or of the column slice)
     torch::Tensor cdf_ptr = indptr;
@@ -607,20 +609,25 @@ SliceResult ColSamplingProbs(const torch::Tensor& indptr, const torch::Tensor& i
                 "gs_sample_weighted_replace");
         });
   }
-  return SampleInto(
+  if (edge_data) *data_out = torch::empty({S * fanout}, edge_data->options());
+  SliceResult sampled = SampleInto(
       indptr, indices, column_ids, fanout, false, with_coo,
       gs_sample_weighted_workspace_bytes(S, fanout),
       [&](const void* cols, int idb, int64_t S_, torch::Tensor& sub_indptr,
           torch::Tensor& sub_indices, torch::Tensor& select_index, torch::Tensor& coo_col,
           torch::Tensor& ws, void* st) {
-        Check(gs_sample_weighted_fill(indptr.data_ptr<int64_t>(), indptr.numel() - 1, EdgeArray(indices, indptr),
-                                      static_cast<const float*>(EdgeArray(probs, indptr)), cols, idb, S_, fanout, NextSeed(),
-                                      nullptr, nullptr, sub_indptr.data_ptr<int64_t>(),
-                                      sub_indices.data_ptr(), select_index.data_ptr<int64_t>(),
-                                      with_coo ? coo_col.data_ptr() : nullptr, ws.data_ptr(),
-                                      ws.numel(), st),
+        Check(gs_sample_weighted_fill_data(
+                  indptr.data_ptr<int64_t>(), indptr.numel() - 1, EdgeArray(indices, indptr),
+                  static_cast<const float*>(EdgeArray(probs, indptr)), cols, idb, S_, fanout,
+                  NextSeed(), nullptr, nullptr, sub_indptr.data_ptr<int64_t>(),
+                  sub_indices.data_ptr(), select_index.data_ptr<int64_t>(),
+                  with_coo ? coo_col.data_ptr() : nullptr,
+                  edge_data ? static_cast<const float*>(EdgeArray(*edge_data, indptr)) : nullptr,
+                  edge_data ? data_out->data_ptr<float>() : nullptr, ws.data_ptr(), ws.numel(), st),
               "gs_sample_weighted_fill");
       });
+  if (edge_data) *data_out = data_out->narrow(0, 0, std::get<2>(sampled).numel());
+  return sampled;
 }
 
 std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> SampleOneKeepDim(

@@ -181,9 +181,13 @@ struct SeedState {
 SeedState SaveSeedState();
 void RestoreSeedState(const SeedState& s);
 
+// edge_data (with data_out; without replacement only): one fp32 value per position of `indices`,
+// whose samples' share comes back in *data_out from the same launch
 SliceResult ColSamplingProbs(const torch::Tensor& indptr, const torch::Tensor& indices,
                              const torch::Tensor& probs, const torch::Tensor& column_ids,
-                             int64_t fanout, bool replace, bool with_coo);
+                             int64_t fanout, bool replace, bool with_coo,
+                             const torch::Tensor* edge_data = nullptr,
+                             torch::Tensor* data_out = nullptr);
 std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> SampleOneKeepDim(
     const torch::Tensor& indptr, const torch::Tensor& indices, const torch::Tensor& column_ids);
 

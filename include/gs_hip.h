@@ -337,6 +337,16 @@ int gs_sample_weighted_fill(const int64_t* indptr, int64_t num_cols, const void*
                             const int64_t* sub_indptr, void* sub_indices, int64_t* select_index,
                             void* coo_col, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same with the edge data of the samples: data_out[o] = edge_data[select_index[o]] (one value
+ * per position of `indices`; both NULL, or data_out as long as sub_indices). */
+int gs_sample_weighted_fill_data(const int64_t* indptr, int64_t num_cols, const void* indices,
+                                 const float* probs, const void* column_ids, int id_bytes,
+                                 int64_t S, int64_t fanout, uint64_t seed, const uint32_t* replay,
+                                 const int64_t* replay_ptr, const int64_t* sub_indptr,
+                                 void* sub_indices, int64_t* select_index, void* coo_col,
+                                 const float* edge_data, float* data_out, void* workspace,
+                                 size_t workspace_bytes, void* stream);
+
 /* Weighted neighbour sampling WITH replacement (inverse CDF): replaces
  * _CSRRowWiseSampleReplaceKernel (src/cuda/sampling_probs.cu:112-183).  A column with
  * deg > 0 gets fanout picks.  cdf = inclusive prefix of max(probs, 0) over the column's

@@ -4,7 +4,9 @@ import pytest
 import torch
 
 from oracle import oracle as O
+import graph_sampling_amd as gs
 from graph_sampling_amd import capi
+from graph_sampling_amd.format import _COO, _CSC
 from tests.util import rmat_csc_np, to_dev, u32_draws
 
 pytestmark = pytest.mark.gpu
@@ -93,6 +95,46 @@ def test_weighted_degrees_around_the_selection_paths(dev, k):
         want = O.sample_weighted(indptr, indices, probs, None, k, seed=31)
         for g, w in zip(got, want):
             assert np.array_equal(g, w)
+
+
+@pytest.mark.parametrize("rows", [8191, 8192, 8193, 20000])
+def test_weighted_rows_around_the_planning_workgroup(dev, rows):
+    # 8192 rows are laid out by one workgroup, more by several that reserve side by side; rows of
+    # five chunks and more have their entries written by a whole wave
+    degs = np.random.default_rng(rows).integers(0, 12, rows).astype(np.int64)
+    degs[::97] = 300
+    degs[[0, 1, rows // 2, rows - 2, rows - 1]] = [8192, 8193, 30000, 2049, 257]
+    indptr = np.concatenate([[0], np.cumsum(degs)])
+    rng = np.random.default_rng(3)
+    indices = rng.integers(0, 1 << 20, int(indptr[-1])).astype(np.int64)
+    probs = (1.0 - rng.random(indices.size)).astype(np.float32)
+    got = _weighted_gpu(dev, indptr, indices, probs, None, 10, torch.int32, seed=7)
+    want = O.sample_weighted(indptr, indices, probs, None, 10, seed=7)
+    for g, w in zip(got, want):
+        assert np.array_equal(g, w)
+
+
+@pytest.mark.parametrize("replace", [False, True])
+def test_weighted_samples_carry_their_edge_data(dev, replace):
+    # copied, selected by a wave, by a workgroup and by a merge; data that are not the weights
+    degs = np.array([3, 0, 200, 1500, 9000], dtype=np.int64)
+    indptr = np.concatenate([[0], np.cumsum(degs)])
+    rng = np.random.default_rng(4)
+    indices = rng.integers(0, 5, int(indptr[-1])).astype(np.int64)
+    probs = to_dev((1.0 - rng.random(indices.size)).astype(np.float32), dev)
+    data = rng.random(indices.size, dtype=np.float32)
+    for wide in (False, True):  # (a column more: data the sampler's launch cannot read)
+        graph = gs.Graph(False)
+        graph._CAPI_LoadCSC(to_dev(indptr, dev), to_dev(indices, dev))
+        graph._CAPI_SetData(to_dev(np.stack([data, -data], 1) if wide else data, dev))
+        gs.set_seed(12)
+        sub = graph._CAPI_SamplingWithProbs(0, probs, 7, replace, _CSC, _COO)
+        got = sub._CAPI_GetData("default").cpu().numpy()
+        gs.set_seed(12)
+        sel = (capi.sample_weighted_replace if replace else capi.sample_weighted)(
+            to_dev(indptr, dev), to_dev(indices, dev), probs, None, 7, seed=12)[2]
+        want = data[sel[:got.shape[0]].cpu().numpy()]
+        assert np.array_equal(got, np.stack([want, -want], 1) if wide else want)
 
 
 def test_weighted_special_cases(dev):
