@@ -112,6 +112,14 @@ table_insert_kernel(Spans<IdT> x, int64_t M_bound, T t, uint32_t* __restrict__ p
 // lowest index goes to the table in memory, and hands the slot it found to the others.
 constexpr int kGroupSlots = 1024;
 constexpr int kGroupProbes = 4;
+// From so many items on a slot is read before the compare-and-swap: later workgroups then find
+// most keys there, and a read costs less than an atomic.  Before, all workgroups are under way
+// together, the reads find the table empty and are one more trip.  Insert alone in us, without /
+// with the read, skewed ids among 2^17 | 2^21 and uniform ones among 2^21 (load <= 1/2):
+//    70 k   9.2/12.1   10.7/12.2  11.0/13.1     700 k  44.9/49.3   39.9/42.4  34.4/37.6
+//   200 k  16.7/20.8   16.2/19.4  18.9/22.0       1 M  61.1/51.0   54.6/48.2  47.0/47.8
+//   400 k  29.2/40.8   32.1/32.7  26.8/30.7       2 M   130/55      105/57    86.1/75.1
+constexpr int64_t kPeekItems = int64_t(3) << 18;
 
 template <typename IdT, typename T, bool PEEK>
 __global__ void __launch_bounds__(kThreads)
@@ -574,8 +582,9 @@ int unique_relabel_impl(const gs_span* mapping, int n_mapping, const gs_span* qu
   if (M > 0) {
     ProfileScope prof("table_insert", stream);
     constexpr bool kNarrow = sizeof(IdT) == 8 && std::is_same<T, PackedTable>::value;
-    hipLaunchKernelGGL((table_insert_grouped_kernel<IdT, T, true>), dim3(blocks_for(M, kThreads)),
-                       dim3(kThreads), 0, stream, x, M, t, pos,
+    const auto insert = M >= kPeekItems ? table_insert_grouped_kernel<IdT, T, true>
+                                        : table_insert_grouped_kernel<IdT, T, false>;
+    hipLaunchKernelGGL(insert, dim3(blocks_for(M, kThreads)), dim3(kThreads), 0, stream, x, M, t, pos,
                        kNarrow ? lb.error : static_cast<unsigned int*>(nullptr));
   }
   {
@@ -634,9 +643,10 @@ int relabel_sampled_impl(const void* seed_keys, int64_t S, const void* sampled, 
   x.fixed = S;
   if (M > 0) {
     ProfileScope prof("table_insert", stream);
-    // No peek at the slot: sampled neighbours are mostly new keys, and the extra read costs the
-    // GraphSAGE step 7 % (0.152 ms against 0.142).  Nor a meeting in LDS first, unless the items
-    // are so many against the ids there are that hubs come up by the hundred.  The host knows
+    // No meeting in LDS first, unless the items are so many against the ids there are that hubs
+    // come up by the hundred; the slot is read first only for very many (kPeekItems; whole
+    // minibatches without / with, us: 30000 x [25, 15] on 233 k nodes 234/193, 40000 x [15, 10, 5] on
+    // 4 M nodes 422/367, 60000 x [15] on 4 M nodes 82/70): neighbours are mostly new keys.  The host knows
     // no more than their bound M, a place for every sample.  One layer, sampling and relabel, without
     // / with the meeting, us, by M over ids (64-bit ids; 32-bit ones go the same way):
     //                            0.06       0.25       0.45       0.55       1          2
@@ -646,8 +656,10 @@ int relabel_sampled_impl(const void* seed_keys, int64_t S, const void* sampled, 
     //   4 M nodes, degree 30     42.2/42.5  58.4/58.4
     // (5000 seeds, fanouts 25 and 15, 233 k nodes of degree 492: 133 -> 103 a minibatch.)
     constexpr bool kNarrow = sizeof(IdT) == 8 && std::is_same<T, PackedTable>::value;
-    const auto insert = num_ids > 0 && 2 * M >= num_ids ? table_insert_grouped_kernel<IdT, T, false>
-                                                        : table_insert_kernel<IdT, T>;
+    const auto insert = num_ids > 0 && M >= kPeekItems && 8 * M >= num_ids
+                            ? table_insert_grouped_kernel<IdT, T, true>
+                        : num_ids > 0 && 2 * M >= num_ids ? table_insert_grouped_kernel<IdT, T, false>
+                                                          : table_insert_kernel<IdT, T>;
     hipLaunchKernelGGL(insert, dim3(blocks_for(M, kThreads)), dim3(kThreads), 0, stream, x, M, t, pos,
                        kNarrow ? lb.error : static_cast<unsigned int*>(nullptr));
   }
