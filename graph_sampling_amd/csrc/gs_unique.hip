@@ -1399,7 +1399,7 @@ int gs_batch_csr_relabel(const void* seeds, const int64_t* seeds_ptr, const void
     return GS_ERR_UNSUPPORTED;
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // ids that ride in 32 bits go through the bins from about half a million items on
+  // ids that ride in 32 bits go through the bins from 128 k items on
   const bool can_bin = (id_bytes == 4 || narrow) && num_seeds + num_ids > 0 &&
                        num_batches <= kStagedBatches;
   if (want_bins && !can_bin) {

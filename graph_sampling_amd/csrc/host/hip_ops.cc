@@ -1097,9 +1097,9 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> BatchCsrRelabelQueued(
   const int64_t B = seeds_ptr.numel() - 1;
   const int64_t M = seeds.numel() + ids.numel();
   const int table_ids = TableIds(idb);
-  // (below half a million items the relabel on hash regions, three launches, is the quicker one:
-  // there the caller's wait for the edge count costs less than the bins' eight launches)
-  if ((idb == 8 && !(table_ids & GS_NARROW_IDS)) || B > 511 || M < (int64_t(1) << 19) ||
+  // (fewer items are quicker on hash regions, for which the caller waits for the edge count:
+  // binned_relabel_applies)
+  if ((idb == 8 && !(table_ids & GS_NARROW_IDS)) || B > 511 || M < (int64_t(1) << 17) ||
       M >= (int64_t(1) << 30))
     return {torch::Tensor(), torch::Tensor(), torch::Tensor()};
   auto unique = torch::empty({M}, seeds.options());

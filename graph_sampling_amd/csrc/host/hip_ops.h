@@ -208,7 +208,7 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> BatchCsrRelabel(
 // that it left because that sampler failed, the sampler is waited for, which raises its error
 // and clears its look-back state.  Undefined tensors and *num_unique untouched when the path through
 // bins is not the one to take the call (ids that do not ride in 32 bits, more than 511 batches,
-// fewer than 2^19 items by the buffers' sizes).
+// fewer than 2^17 items by the buffers' sizes).
 std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> BatchCsrRelabelQueued(
     const torch::Tensor& seeds, const torch::Tensor& seeds_ptr, const torch::Tensor& ids,
     const torch::Tensor& ids_ptr, int64_t* num_unique, const PendingSample* producer = nullptr);

@@ -79,7 +79,7 @@ typedef struct gs_mailbox {
 #define GS_NARROW_IDS 0x100
 
 /* Or-ed into id_bytes of gs_batch_csr_relabel: which of its two implementations runs.  By
- * default ids that fit 32 bits (id_bytes 4, or 8 | GS_NARROW_IDS), from about half a million
+ * default ids that fit 32 bits (id_bytes 4, or 8 | GS_NARROW_IDS), from 128 k
  * items on and with at most 511 batches, are relabelled through bins (the items of a batch
  * are brought together by hash class and deduplicated in LDS: no atomic on memory per item);
  * everything else through one hash region per batch.  GS_RELABEL_REGIONS forces the second,
@@ -95,7 +95,7 @@ typedef struct gs_mailbox {
  * record a hipEvent pair on its stream (up to 4096 launches); NULL or ""
  * disables.  Sites: "sample_fused", "sample_floyd", "table_init", "table_insert",
  * "unique_compact", "unique_finish", "layer_sample", "layer_relabel", "layer_sweep",
- * "batch_init", "batch_insert", "batch_compact", "batch_finish", "bins_init", "bins_count",
+ * "batch_init", "batch_insert", "batch_compact", "batch_finish", "bins_init", "bins_plan", "bins_tiles", "bins_count",
  * "bins_scatter", "bins_flag", "bins_rank", "bins_rename", "scan_tile_sums",
  * "scan_apply", "random_walk", "metapath_walk", "sddmm_dot".  gs_profile_collect waits for the recorded
  * events, returns their summed duration and count (and, when per_launch_ms is

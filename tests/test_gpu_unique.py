@@ -209,6 +209,29 @@ def test_batch_csr_relabel_through_bins_at_size(dev, idt, narrow, shape):
                          np.array(ip, dtype=np.int64), narrow, None)
 
 
+@pytest.mark.parametrize("idt,narrow", [(torch.int32, False), (torch.int64, True)])
+@pytest.mark.parametrize("items,spread", [([1, 63, 64, 65], 1 << 20), ([8191, 8192, 8193, 0, 1], 1 << 20),
+                                          ([2048, 2049, 4097, 0, 0, 16385], 40),
+                                          ([64 * 8192, 64 * 8192 + 1], 1 << 20),
+                                          ([70_000, 100_000], 300)])
+def test_batch_csr_relabel_runs_around_their_tiles(dev, idt, narrow, items, spread):
+    """A tile is 8192 items of a batch, a class about 2048, a piece of a run 64 records; a workgroup
+    looks at 64 tiles' runs at a time and keeps 128 pieces: batches on both sides of each (half of
+    the ids drawn from `spread`, so that a class's runs may be a few long ones)."""
+    rng = np.random.default_rng(len(items) + spread)
+    seeds, ids, sp, ip = [], [], [0], [0]
+    for m in items:
+        ns = m // 3
+        seeds.append(rng.permutation(1 << 20)[:ns])
+        ids.append(np.where(rng.random(m - ns) < 0.5, rng.integers(0, spread, m - ns),
+                            rng.integers(0, 1 << 20, m - ns)))
+        sp.append(sp[-1] + ns)
+        ip.append(ip[-1] + m - ns)
+    _check_batch_relabel(dev, idt, np.concatenate(seeds).astype(np.int64), np.array(sp, dtype=np.int64),
+                         np.concatenate(ids).astype(np.int64), np.array(ip, dtype=np.int64), narrow,
+                         "bins")
+
+
 def test_batch_csr_relabel_one_batch_beyond_the_counters(dev):
     """Batches small on average and one with more classes than a tile's LDS counters; around it
     batches on both sides of one class."""
