@@ -709,6 +709,53 @@ bins_rename_kernel(BatchItems<IdT> x, int64_t M, Bins s, IdT* __restrict__ uniqu
   }
 }
 
+// The same where the batches are cut into tiles: four workgroups a tile, whose batch is found once
+// and not for every item.
+template <typename IdT>
+__global__ void __launch_bounds__(kThreads)
+bins_rename_runs_kernel(BatchItems<IdT> x, Bins s, IdT* __restrict__ unique,
+                        IdT* __restrict__ out_ids, const int64_t* __restrict__ unique_ptr) {
+  constexpr int kParts = kTile / kRenameTile;
+  // a table was too small: a stored position may be none
+  if (__hip_atomic_load(s.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+  const int64_t chunks = static_cast<int64_t>(s.plan.tile_base[x.B]) * kParts;
+  const int64_t per = (chunks + kXcds - 1) / kXcds;
+  const int64_t chunk = static_cast<int64_t>(blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
+  if (blockIdx.x / kXcds >= per || chunk >= chunks) return;
+  const uint32_t tile = static_cast<uint32_t>(chunk / kParts);
+  const int64_t b = batch_at(s.plan.tile_base, x.B, tile);
+  const int64_t first_seed = x.seeds_ptr[b], n_seeds = x.seeds_ptr[b + 1] - first_seed;
+  const int64_t first_id = x.ids_ptr[b];
+  const int64_t from = (tile - s.plan.tile_base[b]) * kTile + chunk % kParts * kRenameTile;
+  const int64_t left = n_seeds + x.ids_ptr[b + 1] - first_id - from;
+  if (left <= 0) return;
+  const int n = static_cast<int>(left < kRenameTile ? left : kRenameTile);
+  const uint32_t first_item = static_cast<uint32_t>(first_seed + first_id + from);
+  uint32_t at[kRenameItems];
+#pragma unroll
+  for (int u = 0; u < kRenameItems; ++u) {
+    const int i = u * kThreads + static_cast<int>(threadIdx.x);
+    at[u] = s.first[first_item + (i < n ? i : n - 1)];
+  }
+  const uint32_t frontier = static_cast<uint32_t>(unique_ptr[b]);
+  uint4 e[kRenameItems];
+#pragma unroll
+  for (int u = 0; u < kRenameItems; ++u) e[u] = s.ranks[at[u] >> 6];
+#pragma unroll
+  for (int u = 0; u < kRenameItems; ++u) {
+    const int i = u * kThreads + static_cast<int>(threadIdx.x);
+    if (i < n) {
+      const unsigned long long m = static_cast<unsigned long long>(e[u].y) << 32 | e[u].x;
+      const uint32_t rank = e[u].z + __popcll(m & ((1ull << (at[u] & 63u)) - 1ull));
+      const int64_t off = from + i;
+      const bool is_id = off >= n_seeds;
+      if (at[u] == first_item + i)
+        unique[rank] = *(is_id ? x.ids + first_id + off - n_seeds : x.seeds + first_seed + off);
+      if (is_id) out_ids[first_id + off - n_seeds] = static_cast<IdT>(rank - frontier);
+    }
+  }
+}
+
 template <typename IdT>
 int binned_impl(const void* seeds, const int64_t* seeds_ptr, const void* ids,
                 const int64_t* ids_ptr, int64_t B, int64_t num_seeds, int64_t num_ids,
@@ -798,6 +845,14 @@ int binned_impl(const void* seeds, const int64_t* seeds_ptr, const void* ids,
                        ids_ptr, num_unique, unique_ptr, lb, box, box_ticket);
   }
   ProfileScope prof("bins_rename", stream);
+  if (runs) {
+    const int64_t most = tiles_bound(M, B) * (kTile / kRenameTile);
+    hipLaunchKernelGGL(bins_rename_runs_kernel<IdT>,
+                       dim3(static_cast<unsigned>((most + kXcds - 1) / kXcds * kXcds)), dim3(kThreads),
+                       0, stream, x, s, static_cast<IdT*>(unique), static_cast<IdT*>(out_ids),
+                       static_cast<const int64_t*>(unique_ptr));
+    return check_launch("batch_csr_relabel (binned)");
+  }
   const int64_t chunks = (M + kRenameTile - 1) / kRenameTile;
   hipLaunchKernelGGL(bins_rename_kernel<IdT>,
                      dim3(static_cast<unsigned>((chunks + kXcds - 1) / kXcds * kXcds)), dim3(kThreads),
