@@ -24,8 +24,8 @@
 //   rename    a pass in the order of the positions: the rank of an item's first position from
 //             mask + count; first occurrences write the frontier, ids their new name
 //
-// 17 M items in 64 batches: plan 4 us, tiles 39, first 117, rank 24, rename 86; counted, scanned
-// and scattered it was 43 + 9 + 92 and first 99.  Batches of more than 2^20 items on average have so many
+// 17 M items in 64 batches: plan 4 us, tiles 39, first 117, rank 24, rename 71; counted, scanned
+// and scattered it was 43 + 9 + 92, first 99 and rename 86.  Batches of more than 2^20 items on average have so many
 // classes that a tile's runs are a few records; they are counted, the buckets laid out by a scan
 // and the records scattered to them, with a counter addition per (4096-item tile, class).
 //
