@@ -23,6 +23,7 @@
 //  * distinct ids of an edge list: a bit per possible id in LDS, slice by slice, or, for short
 //    lists and large ids, a byte per possible id marked with plain stores.
 #include "gs_common.hpp"
+#include "gs_one.hpp"
 
 namespace gs {
 namespace {
@@ -1240,162 +1241,293 @@ inline int64_t mark_range(int64_t E) {
 }
 
 // ---------------------------------------------------- binned scatter-add ----
-// out[target[e]] += data[e]^powk without an atomic to memory: one partition pass of the sort
-// above brings the edges of every run of 2^bin_shift targets together (at most 256 runs),
-// and a workgroup then adds a run's edges up in LDS and writes its sums with plain stores.
-// Atomics to memory run at about ten per nanosecond on this part whatever the kernel does
-// around them; edges that mostly hit different targets paid that price one by one.
+// out[target[e]] += data[e]^powk without an atomic to memory: the edges of up to 1024 bins of
+// targets are brought together, and a workgroup adds a bin's edges up in LDS and writes its sums
+// with plain stores.  Atomics to memory run at some twenty-five per nanosecond on this part
+// whatever the kernel does around them; edges that mostly hit different targets paid that price
+// one by one.
+//
+// A bin is as many lines of 32 targets as the others, dealt out by a multiplication of the line
+// number: a run of neighbouring targets as a bin held a third of a skewed graph's edges, which
+// then took dozens of workgroups and their sums atomics to memory after all.
+//
+//   tiles    8192 edges are put in the order of their bins in LDS and written side by side, place in
+//            the bin (2 bytes) and value, with the places where the bins' runs start
+//   totals   edges of every bin
+//   sums     a workgroup per bin (or share of one with many more than the average) reads its runs
+//
+// The sums in LDS are 64-bit ones: 64 additions to 32-bit floats in LDS take 81 ns on a compute
+// unit, to 64-bit floats 8 (to 32-bit integers 2.3).
+//
+// 2 M edges over 2.45 M targets, uniform / skewed like R-MAT's rows: 56 / 58 us with bins of neighbours,
+// made by a pass of the sort above, and 32-bit sums; 32 / 40 now (64-bit ids, one by one: 115 / 276).
 constexpr int kBinThreads = 1024;
-// A run with many edges (the hubs' run of a skewed graph holds a third of them) is shared by
-// several workgroups, which then add their sums to memory with atomics: the additions to one
-// LDS word queue up, and 16 k edges a workgroup measured fastest (2 M edges over 2.45 M
-// targets: 0.32 ms with one workgroup a run, 0.14 at 64 k edges, 0.10 at 16 k or 8 k).
-constexpr int kBinParts = 64;             // workgroups that may share one run of targets
-constexpr int64_t kBinPartItems = 16384;  // edges a workgroup takes before a run is shared
-constexpr int kBinMaxShift = 15;         // 2^15 sums = 128 KB of LDS
+constexpr int kSumTileItems = 8;
+constexpr int kSumTile = kBinThreads * kSumTileItems;
+constexpr int kMaxBins = 1024;
+constexpr int kBinMaxShift = 13;          // 2^13 sums = 64 KB of LDS
+constexpr int kBinMinBits = 8;            // 256 bins at least, where there are as many targets
+// The additions to one LDS word queue up, so a bin of more than twice the average (a hub's) is shared
+// by several workgroups, the average each, which then add their sums to memory with atomics.
+constexpr int kBinParts = 256;           // workgroups that may share one bin
+constexpr int64_t kBinPartItems = 8192;  // edges a share has at least
+constexpr int kBinLineBits = 5;           // 32 targets, 128 bytes
+
+// Target t is sum `place` of bin `place >> bin_shift`: its line number times an odd number.
+struct BinOrder {
+  uint32_t mult, inverse, mask;  // of the line number
+  int line_bits, bin_shift, bins;
+  __device__ __forceinline__ uint32_t place(uint32_t t) const {
+    return ((((t >> line_bits) * mult) & mask) << line_bits) | (t & ((1u << line_bits) - 1u));
+  }
+  __device__ __forceinline__ uint32_t target(uint32_t place) const {
+    return ((((place >> line_bits) * inverse) & mask) << line_bits) |
+           (place & ((1u << line_bits) - 1u));
+  }
+};
+
+inline BinOrder bin_order(int64_t num_targets) {
+  BinOrder o;
+  const int bits = bits_for(num_targets);
+  o.bin_shift = bits > kBinMinBits ? bits - kBinMinBits : 0;
+  if (o.bin_shift > kBinMaxShift) o.bin_shift = kBinMaxShift;
+  o.bins = 1 << (bits - o.bin_shift);
+  o.line_bits = o.bin_shift < kBinLineBits ? o.bin_shift : kBinLineBits;
+  o.mask = static_cast<uint32_t>((int64_t(1) << (bits - o.line_bits)) - 1);
+  o.mult = 0x9E3779B1u;
+  o.inverse = o.mult;  // Newton: right in three more bits each time, from three
+  for (int i = 0; i < 4; ++i) o.inverse *= 2u - o.mult * o.inverse;
+  return o;
+}
+
+struct SumSpace {
+  unsigned short* place;  // [E]: in the bin
+  float* value;           // [E]
+  unsigned short* start;  // [tiles][bins + 1]
+  int64_t* totals;        // [bins]
+};
+
+template <typename IdT>
+__global__ void __launch_bounds__(kBinThreads)
+sum_tiles_kernel(const IdT* __restrict__ target, const float* __restrict__ data, int64_t E,
+                 int64_t num_targets, int powk, BinOrder order, SumSpace s) {
+  static_assert(kBinThreads == kOneThreads && kMaxBins <= kBinThreads, "one_scan is over 1024 threads");
+  __shared__ uint32_t s_cnt[kMaxBins];
+  __shared__ float s_value[kSumTile];
+  __shared__ unsigned short s_place[kSumTile];
+  __shared__ int s_scan[2][kOneWaves];
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * kSumTile;
+  const int n = static_cast<int>(E - base < kSumTile ? E - base : kSumTile);
+  // (no read carries a condition: the last edge again past the end)
+  IdT t[kSumTileItems];
+  float x[kSumTileItems];
+#pragma unroll
+  for (int u = 0; u < kSumTileItems; ++u) {
+    const int i = u * kBinThreads + static_cast<int>(threadIdx.x);
+    t[u] = target[base + (i < n ? i : n - 1)];
+  }
+#pragma unroll
+  for (int u = 0; u < kSumTileItems; ++u) {
+    const int i = u * kBinThreads + static_cast<int>(threadIdx.x);
+    x[u] = data[base + (i < n ? i : n - 1)];
+  }
+  const int bins = order.bins;
+  s_cnt[threadIdx.x] = 0u;
+  lds_barrier();
+  uint32_t bin[kSumTileItems], rank[kSumTileItems], place[kSumTileItems];
+#pragma unroll
+  for (int u = 0; u < kSumTileItems; ++u) {
+    const int i = u * kBinThreads + static_cast<int>(threadIdx.x);
+    // (a target that is none of num_targets has no sum to go to: left out)
+    const bool live = i < n && t[u] >= 0 && static_cast<int64_t>(t[u]) < num_targets;
+    const uint32_t p = order.place(static_cast<uint32_t>(t[u]));
+    bin[u] = live ? p >> order.bin_shift : kMaxBins;
+    place[u] = p & ((1u << order.bin_shift) - 1u);
+    rank[u] = live ? atomicAdd(&s_cnt[bin[u]], 1u) : 0u;
+  }
+  lds_barrier();
+  unsigned short* __restrict__ start = s.start + static_cast<int64_t>(blockIdx.x) * (bins + 1);
+  const int mine = static_cast<int>(s_cnt[threadIdx.x]);
+  int total;
+  const int at = one_scan(mine, &total, s_scan, 0);
+  s_cnt[threadIdx.x] = static_cast<uint32_t>(at);
+  if (static_cast<int>(threadIdx.x) < bins) start[threadIdx.x] = static_cast<unsigned short>(at);
+  if (threadIdx.x == 0) start[bins] = static_cast<unsigned short>(total);
+  lds_barrier();
+#pragma unroll
+  for (int u = 0; u < kSumTileItems; ++u) {
+    if (bin[u] < kMaxBins) {
+      const uint32_t to = s_cnt[bin[u]] + rank[u];
+      s_value[to] = powk_f(x[u], powk);
+      s_place[to] = static_cast<unsigned short>(place[u]);
+    }
+  }
+  lds_barrier();
+#pragma unroll
+  for (int u = 0; u < kSumTileItems; ++u) {
+    const int i = u * kBinThreads + static_cast<int>(threadIdx.x);
+    if (i < total) {
+      s.value[base + i] = s_value[i];
+      s.place[base + i] = s_place[i];
+    }
+  }
+}
+
+__global__ void __launch_bounds__(kThreads) sum_totals_kernel(SumSpace s, int64_t tiles, int bins) {
+  __shared__ int64_t s_scan[kThreads / kWave + 1];
+  const unsigned short* __restrict__ start = s.start + blockIdx.x;
+  int64_t mine = 0;
+  for (int64_t t = threadIdx.x; t < tiles; t += kThreads)
+    mine += start[t * (bins + 1) + 1] - start[t * (bins + 1)];
+  int64_t total;
+  block_exclusive_scan<kThreads>(mine, &total, s_scan);
+  if (threadIdx.x == 0) s.totals[blockIdx.x] = total;
+}
+
+constexpr int kSumTrip = 8;  // pieces of runs, of up to 64 edges, that a wave asks for together
 
 __global__ void __launch_bounds__(kBinThreads)
-bin_sum_kernel(const unsigned long long* __restrict__ words, const uint32_t* __restrict__ vals,
-               const int64_t* __restrict__ totals, int num_bins, int idx_bits, int bin_shift,
-               int powk, int64_t num_targets, float* __restrict__ out) {
-  extern __shared__ float s_sum[];
-  // Which run, and which share of it, this workgroup takes: the launch has one workgroup per
-  // share that can exist (a run of n edges has ceil(n / 16 k) of them, 64 at most), and every
-  // workgroup works the numbering out for itself from the runs' sizes.  (A launch of 64
-  // workgroups per run, most of which left at once, spent 30 of its 48 us handing 64 KB of LDS
-  // to workgroups with nothing to do.)
-  __shared__ int64_t s_scan[kBinThreads / kWave + 1];
-  __shared__ int s_first[kRadix + 1];
-  __shared__ int64_t s_lo[kRadix + 1];
+bin_sum_kernel(SumSpace s, int64_t tiles, int64_t alone, int64_t part_items, BinOrder order,
+               int64_t num_targets, float* __restrict__ out) {
+  extern __shared__ double s_sum[];
+  // Which bin, and which share of it, this workgroup takes: the launch has one workgroup per
+  // share that can exist (a bin of n > alone edges has ceil(n / part_items) of them, 256 at most),
+  // and every workgroup works the numbering out for itself from the bins' sizes.
+  __shared__ int s_scan[2][kOneWaves];
+  __shared__ int s_first[kMaxBins + 1];
+  const int bins = order.bins;
   {
-    int64_t n = 0;
-    if (threadIdx.x < num_bins) n = totals[threadIdx.x];
-    int64_t shares = (n + kBinPartItems - 1) / kBinPartItems;
-    if (shares > kBinParts) shares = kBinParts;
-    // (both sums in one scan: up to 2^14 shares above, fewer than 2^31 edges below)
-    int64_t total;
-    const int64_t before = block_exclusive_scan<kBinThreads>(shares << 32 | n, &total, s_scan);
-    if (threadIdx.x <= num_bins) {
-      s_first[threadIdx.x] = static_cast<int>(before >> 32);
-      s_lo[threadIdx.x] = before & 0xFFFFFFFFll;
+    int shares = 0, total;
+    if (static_cast<int>(threadIdx.x) < bins) {
+      const int64_t n = s.totals[threadIdx.x];
+      const int64_t some = (n + part_items - 1) / part_items;
+      shares = n > alone ? static_cast<int>(some < kBinParts ? some : kBinParts) : (n > 0 ? 1 : 0);
     }
+    s_first[threadIdx.x] = one_scan(shares, &total, s_scan, 0);
+    if (threadIdx.x == 0) s_first[kBinThreads] = total;
     __syncthreads();
   }
-  if (static_cast<int>(blockIdx.x) >= s_first[num_bins]) return;
+  if (static_cast<int>(blockIdx.x) >= s_first[bins]) return;
   int bin = 0;
-  for (int step = kRadix / 2; step > 0; step >>= 1)
-    if (bin + step <= num_bins && s_first[bin + step] <= static_cast<int>(blockIdx.x)) bin += step;
+  for (int step = kMaxBins / 2; step > 0; step >>= 1)
+    if (bin + step <= bins && s_first[bin + step] <= static_cast<int>(blockIdx.x)) bin += step;
   const int part = static_cast<int>(blockIdx.x) - s_first[bin];
-  const int64_t lo = s_lo[bin], hi = s_lo[bin + 1];
-  const int64_t n = hi - lo;
-  int64_t parts = (n + kBinPartItems - 1) / kBinPartItems;
-  if (parts > kBinParts) parts = kBinParts;
-  const int width = 1 << bin_shift;
-  for (int j = threadIdx.x; j < width; j += kBinThreads) s_sum[j] = 0.0f;
+  const int parts = s_first[bin + 1] - s_first[bin];
+  const int64_t tile_lo = tiles * part / parts, tile_hi = tiles * (part + 1) / parts;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int width = 1 << order.bin_shift;
+  for (int j = threadIdx.x; j < width; j += kBinThreads) s_sum[j] = 0.0;
   __syncthreads();
-  const int64_t per = (n + parts - 1) / parts;
-  const int64_t begin = lo + part * per;
-  const int64_t end = begin + per < hi ? begin + per : hi;
-  const int64_t first = static_cast<int64_t>(bin) << bin_shift;
-  // a thread's edges eight at a time, all reads (clamped to the part) before the first
-  // addition: one edge at a time every addition waits for its own trip to memory
-  constexpr int kBatch = 8;
-  for (int64_t i0 = begin + threadIdx.x; i0 < end; i0 += kBinThreads * kBatch) {
-    unsigned long long w[kBatch];
-    uint32_t v[kBatch];
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int64_t i = i0 + u * kBinThreads;
-      w[u] = words[i < end ? i : end - 1];
+  // a wave takes every sixteenth tile, 64 at a time: a lane knows a tile's run
+  for (int64_t t0 = tile_lo + wave; t0 < tile_hi; t0 += kOneWaves * kWave) {
+    const int64_t tile = t0 + static_cast<int64_t>(lane) * kOneWaves;
+    int start = 0, len = 0;
+    if (tile < tile_hi) {
+      start = s.start[tile * (bins + 1) + bin];
+      len = static_cast<int>(s.start[tile * (bins + 1) + bin + 1]) - start;
     }
+    const int ends = wave_inclusive_sum((len + kWave - 1) / kWave);
+    const int pieces = __builtin_amdgcn_readlane(ends, kWave - 1);
+    for (int p0 = 0; p0 < pieces; p0 += kSumTrip) {
+      float v[kSumTrip];
+      unsigned short at[kSumTrip];
+      unsigned int held = 0u;
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int64_t i = i0 + u * kBinThreads;
-      v[u] = vals[i < end ? i : end - 1];
-    }
+      for (int u = 0; u < kSumTrip; ++u) {
+        v[u] = 0.0f;
+        at[u] = 0;
+        if (p0 + u < pieces) {
+          const int j = __popcll(__ballot(ends <= p0 + u));
+          const int run = __builtin_amdgcn_readlane(len, j);
+          const int i = (p0 + u - (__builtin_amdgcn_readlane(ends, j) - (run + kWave - 1) / kWave)) * kWave + lane;
+          if (i < run) {
+            const int64_t from = (t0 + static_cast<int64_t>(j) * kOneWaves) * kSumTile +
+                                 __builtin_amdgcn_readlane(start, j) + i;
+            v[u] = s.value[from];
+            at[u] = s.place[from];
+            held |= 1u << u;
+          }
+        }
+      }
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int64_t t = static_cast<int64_t>(w[u] >> idx_bits) - first;
-      // (a target beyond num_targets has no sum to go to: left out, as out has no room for it)
-      if (i0 + u * kBinThreads < end && t >= 0 && t < width)
-        atomicAdd(&s_sum[t], powk_f(__uint_as_float(v[u]), powk));
+      for (int u = 0; u < kSumTrip; ++u)
+        if (held >> u & 1u) unsafeAtomicAdd(&s_sum[at[u]], static_cast<double>(v[u]));
     }
   }
   __syncthreads();
+  const uint32_t first = static_cast<uint32_t>(bin) << order.bin_shift;
   if (parts > 1) {
     for (int j = threadIdx.x; j < width; j += kBinThreads) {
-      const float x = s_sum[j];
-      if (x != 0.0f && first + j < num_targets) unsafeAtomicAdd(out + first + j, x);
+      const float x = static_cast<float>(s_sum[j]);
+      const uint32_t t = order.target(first + j);
+      if (x != 0.0f && t < num_targets) unsafeAtomicAdd(out + t, x);
     }
     return;
   }
-  // the run is this workgroup's alone: plain read, add, write -- a thread's sums eight at a
+  // the bin is this workgroup's alone: plain read, add, write -- a thread's sums eight at a
   // time, the reads (of a word that is always there where the sum is zero) before the writes
+  constexpr int kBatch = 8;
   for (int j0 = threadIdx.x; j0 < width; j0 += kBinThreads * kBatch) {
     float x[kBatch], was[kBatch];
+    uint32_t t[kBatch];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       const int j = j0 + u * kBinThreads;
-      x[u] = (j < width && first + j < num_targets) ? s_sum[j] : 0.0f;
+      t[u] = order.target(first + j);
+      x[u] = (j < width && t[u] < num_targets) ? static_cast<float>(s_sum[j]) : 0.0f;
     }
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) was[u] = out[x[u] != 0.0f ? first + j0 + u * kBinThreads : first];
+    for (int u = 0; u < kBatch; ++u) was[u] = out[x[u] != 0.0f ? t[u] : 0u];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u)
-      if (x[u] != 0.0f) out[first + j0 + u * kBinThreads] = was[u] + x[u];
+      if (x[u] != 0.0f) out[t[u]] = was[u] + x[u];
   }
 }
 
-// whether the binned path takes the call: 4-byte ids (the value rides along in an id-sized
-// word), plain edge order, few enough targets for 256 runs of at most 2^15, enough edges
-// for five launches to pay
-inline bool bin_sum_applies(int id_bytes, const int64_t* e_ids, int64_t E, int64_t num_targets) {
-  return id_bytes == 4 && !e_ids && E >= (int64_t(1) << 17) && num_targets > 0 &&
-         num_targets <= (int64_t(kRadix) << kBinMaxShift) && E < (int64_t(1) << 31);
+// whether the binned path takes the call: plain edge order, few enough targets for 1024 bins of
+// 2^13, enough edges for three launches to pay
+inline bool bin_sum_applies(const int64_t* e_ids, int64_t E, int64_t num_targets) {
+  return !e_ids && E >= (int64_t(1) << 17) && num_targets > 0 &&
+         num_targets <= (int64_t(kMaxBins) << kBinMaxShift) && E < (int64_t(1) << 31);
 }
 
-int bin_sum_impl(const int32_t* target, const float* data, int64_t E, int powk, int64_t num_targets,
+inline int64_t sum_tiles(int64_t E) { return (E + kSumTile - 1) / kSumTile; }
+
+template <typename IdT>
+int bin_sum_impl(const IdT* target, const float* data, int64_t E, int powk, int64_t num_targets,
                  float* out, void* workspace, size_t workspace_bytes, hipStream_t st) {
-  using T = SmallTile;
-  const int64_t blocks = blocks_for(E, T::kSize);
-  const int64_t table = kRadix * blocks;
+  const int64_t tiles = sum_tiles(E);
   Carver ws(workspace, workspace_bytes);
-  unsigned long long* words = ws.take<unsigned long long>(E);
-  uint32_t* vals = ws.take<uint32_t>(E);
-  int64_t* counts = ws.take<int64_t>(table);
-  int64_t* offsets = ws.take<int64_t>(table);
-  int64_t* totals = ws.take<int64_t>(kRadix);
+  SumSpace s;
+  s.place = ws.take<unsigned short>(E);
+  s.value = ws.take<float>(E);
+  const BinOrder order = bin_order(num_targets);
+  s.start = ws.take<unsigned short>(tiles * (order.bins + 1));
+  s.totals = ws.take<int64_t>(order.bins);
   if (!ws.ok) {
     set_error_text("gs_coo_sum_binned: workspace needs %zu bytes, 256-byte aligned",
                    gs_coo_sum_workspace_bytes(E, num_targets));
     return GS_ERR_WORKSPACE;
   }
-  const int idx_bits = bits_for(E);
-  int bin_shift = bits_for(num_targets) - kRadixBits;
-  if (bin_shift < 0) bin_shift = 0;
-  const int shift = idx_bits + bin_shift;
-  const dim3 grid(static_cast<unsigned>(blocks));
-  FreshWords<int32_t> src{target, idx_bits};
-  hipLaunchKernelGGL((radix_hist_kernel<T, FreshWords<int32_t>>), grid, dim3(T::kThreadsPerTile), 0,
-                     st, src, E, shift, blocks, counts, static_cast<int*>(nullptr));
-  hipLaunchKernelGGL(digit_offsets_kernel, dim3(kRadix), dim3(kDigitThreads), 0, st, counts, blocks,
-                     offsets, totals);
-  const SortOutputs<int32_t> none{nullptr, nullptr, nullptr, idx_bits, nullptr};
-  launch_pass<T>(src, false, false, st, reinterpret_cast<const uint32_t*>(data), E, shift, blocks,
-                 offsets, totals, words, vals, none);
-  const int bins = static_cast<int>(((num_targets - 1) >> bin_shift) + 1);
   // (per call: the attribute belongs to the device the call runs on)
   const hipError_t lds_allowed = hipFuncSetAttribute(
       reinterpret_cast<const void*>(bin_sum_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-      static_cast<int>(sizeof(float) << kBinMaxShift));
+      static_cast<int>(sizeof(double) << kBinMaxShift));
   if (lds_allowed != hipSuccess) {
     set_error_text("gs_coo_sum_binned: %s", hipGetErrorString(lds_allowed));
     return GS_ERR_LAUNCH;
   }
-  const int64_t shares = E / kBinPartItems + bins;  // at most: sum of ceil(n / 16 k) over the runs
+  hipLaunchKernelGGL(sum_tiles_kernel<IdT>, dim3(static_cast<unsigned>(tiles)), dim3(kBinThreads), 0, st,
+                     target, data, E, num_targets, powk, order, s);
+  hipLaunchKernelGGL(sum_totals_kernel, dim3(order.bins), dim3(kThreads), 0, st, s, tiles, order.bins);
+  const int64_t average = E / order.bins;
+  const int64_t part_items = average > kBinPartItems ? average : kBinPartItems;
+  const int64_t alone = 2 * part_items;
+  const int64_t shares = E / part_items + order.bins;  // at most: sum of ceil(n / part_items) over the bins
   hipLaunchKernelGGL(bin_sum_kernel, dim3(static_cast<unsigned>(shares)), dim3(kBinThreads),
-                     sizeof(float) << bin_shift, st, words, vals, totals, bins, idx_bits, bin_shift, powk,
-                      num_targets, out);
+                     sizeof(double) << order.bin_shift, st, s, tiles, alone, part_items, order,
+                     num_targets, out);
   return check_launch("coo_sum_binned");
 }
 
@@ -1577,11 +1709,10 @@ int gs_indptr_split_cuts(const int64_t* indptr, const int64_t* offsets, int64_t 
 
 size_t gs_coo_sum_workspace_bytes(int64_t E, int64_t num_targets) {
   if (E < 0) E = 0;
-  if (!bin_sum_applies(4, nullptr, E, num_targets)) return 256;
-  const int64_t blocks = blocks_for(E, SmallTile::kSize);
-  const int64_t table = kRadix * blocks;
-  return padded(static_cast<size_t>(E) * 8) + padded(static_cast<size_t>(E) * 4) +
-         2 * padded(static_cast<size_t>(table) * 8) + padded(kRadix * 8);
+  if (!bin_sum_applies(nullptr, E, num_targets)) return 256;
+  return padded(static_cast<size_t>(E) * 2) + padded(static_cast<size_t>(E) * 4) +
+         padded(static_cast<size_t>(sum_tiles(E)) * (bin_order(num_targets).bins + 1) * 2) +
+         padded(static_cast<size_t>(bin_order(num_targets).bins) * 8);
 }
 
 int gs_coo_sum_binned(const void* target, int id_bytes, const int64_t* e_ids, const float* data,
@@ -1593,11 +1724,14 @@ int gs_coo_sum_binned(const void* target, int id_bytes, const int64_t* e_ids, co
   GS_REQUIRE(valid_id_bytes(id_bytes), "gs_coo_sum_binned: id_bytes must be 4 or 8, got %d",
              id_bytes);
   if (E == 0) return GS_OK;
-  if (!bin_sum_applies(id_bytes, e_ids, E, num_targets))
+  if (!bin_sum_applies(e_ids, E, num_targets))
     return coo_sum_bounded(target, id_bytes, e_ids, data, E, powk, num_targets, out, stream);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (id_bytes == 8)
+    return bin_sum_impl(static_cast<const int64_t*>(target), data, E, static_cast<int>(powk),
+                        num_targets, out, workspace, workspace_bytes, st);
   return bin_sum_impl(static_cast<const int32_t*>(target), data, E, static_cast<int>(powk),
-                      num_targets, out, workspace, workspace_bytes,
-                      static_cast<hipStream_t>(stream));
+                      num_targets, out, workspace, workspace_bytes, st);
 }
 
 }  // extern "C"

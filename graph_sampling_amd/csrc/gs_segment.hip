@@ -824,22 +824,24 @@ constexpr int kAggEdges = 8;  // edges per thread
 
 // Few edges are spread over more workgroups, two a thread: the launch is then a handful of trips
 // to memory and an LDS table to clear, which a shorter tile has less of (22 k edges 16 -> 6 us).
-// Every target of a tile costs an addition to memory, so that from 2^17 edges on longer tiles win.
+// Every target of a tile costs an addition to memory, so that longer tiles win beyond (60 k edges,
+// whole call, two / eight a thread: uniform targets 10/12 us, skewed like R-MAT's rows 14-20/15-17,
+// a tenth of them on one target 24-27/17).
 constexpr int kAggFewEdges = 2;
-constexpr int64_t kAggFew = int64_t(1) << 17;
+constexpr int64_t kAggFew = int64_t(1) << 15;
 
 template <int EDGES>
 struct KeyedSums {
   static constexpr int kSlots = 2 * kThreads * EDGES;  // load <= 1/2
   long long key[kSlots];
-  float sum[kSlots];
+  double sum[kSlots];  // (64 additions to 32-bit floats in LDS take 81 ns here, to 64-bit ones 8)
 };
 
 template <int EDGES>
 __device__ __forceinline__ void keyed_clear(KeyedSums<EDGES>& t) {
   for (int i = threadIdx.x; i < t.kSlots; i += kThreads) {
     t.key[i] = -1;
-    t.sum[i] = 0.0f;
+    t.sum[i] = 0.0;
   }
   __syncthreads();
 }
@@ -855,7 +857,7 @@ __device__ __forceinline__ void keyed_add(KeyedSums<EDGES>& t, long long key, fl
     if (seen == -1 || seen == key) break;
     h = (h + 1) & (t.kSlots - 1);
   }
-  unsafeAtomicAdd(&t.sum[h], v);
+  unsafeAtomicAdd(&t.sum[h], static_cast<double>(v));
 }
 
 // (a key outside [0, bound) is left out)
@@ -864,7 +866,7 @@ __device__ __forceinline__ void keyed_flush(KeyedSums<EDGES>& t, float* __restri
                                             long long bound = 0x7FFFFFFFFFFFFFFFll) {
   __syncthreads();
   for (int i = threadIdx.x; i < t.kSlots; i += kThreads)
-    if (t.key[i] >= 0 && t.key[i] < bound) unsafeAtomicAdd(out + t.key[i], t.sum[i]);
+    if (t.key[i] >= 0 && t.key[i] < bound) unsafeAtomicAdd(out + t.key[i], static_cast<float>(t.sum[i]));
 }
 
 // out[target[e]] += f(data[emap ? emap[e] : e])   (graph_ops.cu:45-64)

@@ -679,11 +679,10 @@ int gs_coo_sum(const void* target, int id_bytes, const int64_t* e_ids, const flo
                int64_t powk, float* out, void* stream);
 
 /* The same sums for callers that know how many targets there are (out has num_targets
- * entries; a target beyond is left out) and bring a workspace: with 4-byte ids, no e_ids,
- * at least 2^17 edges and at most 2^23 targets the edges are first brought together by runs
- * of targets (one partition pass of the sort behind gs_coo2csc) and then added up in LDS, a
- * run per workgroup, with no atomic to memory -- several times faster than gs_coo_sum when
- * most edges hit different targets.  Any other call is passed on to gs_coo_sum.  The order of
+ * entries; a target beyond is left out) and bring a workspace: with no e_ids, at least 2^17
+ * edges and at most 2^23 targets the edges are first brought together by bins of targets and then
+ * added up in LDS, a bin per workgroup, with no atomic to memory -- several times faster than
+ * gs_coo_sum when most edges hit different targets.  Any other call is passed on to gs_coo_sum.  The order of
  * the additions is not fixed in either (impl::COOSumCUDA, src/cuda/graph_ops.cu:45-64, adds
  * with atomics too). */
 size_t gs_coo_sum_workspace_bytes(int64_t E, int64_t num_targets);
