@@ -808,8 +808,7 @@ int gs_index_search(const void* data, int64_t n, const void* keys, int64_t m, in
 /* ------------------------------------------------------------------------- */
 /* out = the distinct values of a[na] and b[nb] in increasing order (torch.unique of their
  * concatenation, for ids >= 0), *count (device) = how many; out has room for na + nb.
- * 1 <= na + nb <= gs_sorted_union_max(id_bytes) (8192 / 4096 for 4- / 8-byte ids: one
- * workgroup sorts them in LDS). */
+ * 1 <= na + nb <= gs_sorted_union_max(id_bytes) (8192: one workgroup sorts them in LDS). */
 int64_t gs_sorted_union_max(int id_bytes);
 int gs_sorted_union(const void* a, int64_t na, const void* b, int64_t nb, int id_bytes, void* out,
                     int64_t* count, void* stream);

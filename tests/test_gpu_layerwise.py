@@ -107,9 +107,20 @@ def test_sorted_union_at_the_numbers_of_keys_a_thread(dev, na, nb):
             assert np.array_equal(out[:int(count.item())].cpu().numpy(), np.unique(ids))
 
 
+@pytest.mark.parametrize("n", [5, 1024, 1500, 3000, 8192])
+@pytest.mark.parametrize("top", [(1 << 32) - 2, (1 << 32) - 1, 1 << 32, 1 << 40])
+def test_sorted_union_of_64_bit_ids_around_32_bits(dev, n, top):
+    """Ids that all stay below 2^32 - 1 are sorted as 32-bit keys."""
+    rng = np.random.default_rng(n)
+    ids = rng.integers(0, 1 << 31, n)
+    ids[n // 2] = top
+    out, count = capi.sorted_union(to_dev(ids[:n // 3], dev), to_dev(ids[n // 3:], dev))
+    assert np.array_equal(out[:int(count.item())].cpu().numpy(), np.unique(ids))
+
+
 @pytest.mark.parametrize("idb,E,num_nodes,room", [
     (4, 4096, 2, 2), (4, 4097, 1024, 1024), (8, 4095, 1023, 1024), (4, 9000, 8192, 8192),
-    (8, 9000, 4096, 4096), (4, 4096 * 4096 + 5, 3, 3)])
+    (8, 9000, 4096, 4096), (8, 20000, 8191, 8192), (4, 4096 * 4096 + 5, 3, 3)])
 def test_pick_rows_with_a_full_tree_and_beyond_the_tiles_that_add_up_themselves(dev, idb, E, num_nodes, room):
     npt, _ = IDT[idb]
     rng = np.random.default_rng(E)
