@@ -418,14 +418,15 @@ using SmallTile = SortTile<256, 16>;
 using LargeTile = SortTile<1024, 8>;
 constexpr int64_t kLargeTileItems = int64_t(1) << 22;  // 512 large tiles: two for every compute unit
 
-// counts[d * num_blocks + b] = items of tile b with digit d.  Four copies of the histogram, lane
+// counts[b * 256 + d] = items of tile b with digit d (a tile's side by side: digit by digit they were
+// 437 k stores to as many lines for 14 M edges, 24 -> 19 us).  Four copies of the histogram, lane
 // by lane in turn: on a skewed graph half a wave holds one digit, and additions to one LDS word
 // queue up.
 constexpr int kHistCopies = 4;
 
 template <typename T, typename Src>
 __global__ void __launch_bounds__(T::kThreadsPerTile)
-radix_hist_kernel(Src src, int64_t E, int shift, int64_t num_blocks, int64_t* __restrict__ counts,
+radix_hist_kernel(Src src, int64_t E, int shift, int64_t* __restrict__ counts,
                   int* __restrict__ clear) {
   __shared__ int s_hist[kHistCopies][kRadix + 1];
   for (int j = threadIdx.x; j < kHistCopies * (kRadix + 1); j += T::kThreadsPerTile)
@@ -449,11 +450,46 @@ radix_hist_kernel(Src src, int64_t E, int shift, int64_t num_blocks, int64_t* __
     int n = 0;
 #pragma unroll
     for (int c = 0; c < kHistCopies; ++c) n += s_hist[c][threadIdx.x];
-    counts[static_cast<int64_t>(threadIdx.x) * num_blocks + blockIdx.x] = n;
+    counts[static_cast<int64_t>(blockIdx.x) * kRadix + threadIdx.x] = n;
   }
 }
 
-// Where a digit's items of a tile start among that digit's items (offsets, laid out like counts),
+// The same from the digits alone, a byte each (a multiple of eight can be read): eight a read.  14 M
+// edges: 24 us from the words, 14 byte by byte, 13 so (8 with the counts of a tile side by side).
+template <typename T>
+__global__ void __launch_bounds__(T::kThreadsPerTile)
+digit_hist_kernel(const unsigned char* __restrict__ digit, int64_t E, int64_t* __restrict__ counts) {
+  constexpr int kReads = T::kPerThread / 8;
+  __shared__ int s_hist[kHistCopies][kRadix + 1];
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * T::kSize;
+  const uint32_t n = E - base < T::kSize ? static_cast<uint32_t>(E - base) : T::kSize;
+  unsigned long long eight[kReads];
+#pragma unroll
+  for (int k = 0; k < kReads; ++k) {
+    const uint32_t j = (k * T::kThreadsPerTile + threadIdx.x) * 8;
+    eight[k] = *reinterpret_cast<const unsigned long long*>(digit + base + (j < n ? j : 0u));
+  }
+  for (int j = threadIdx.x; j < kHistCopies * (kRadix + 1); j += T::kThreadsPerTile)
+    (&s_hist[0][0])[j] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kReads; ++k) {
+    const uint32_t j = (k * T::kThreadsPerTile + threadIdx.x) * 8;
+#pragma unroll
+    for (int b = 0; b < 8; ++b)
+      if (j + b < n)
+        atomicAdd(&s_hist[threadIdx.x & (kHistCopies - 1)][static_cast<int>(eight[k] >> (8 * b)) & (kRadix - 1)], 1);
+  }
+  __syncthreads();
+  if (threadIdx.x < kRadix) {
+    int all = 0;
+#pragma unroll
+    for (int c = 0; c < kHistCopies; ++c) all += s_hist[c][threadIdx.x];
+    counts[static_cast<int64_t>(blockIdx.x) * kRadix + threadIdx.x] = all;
+  }
+}
+
+// Where a digit's items of a tile start among that digit's items (offsets[d * num_blocks + b]),
 // and how many the digit has (totals): a workgroup a digit, 2048 tiles at a time.  What the digits
 // below it hold, every workgroup of the pass adds up from the 256 totals by itself.  (One scan over
 // the whole table, which that leaves out, is two launches: 1709 tiles 11 -> 5 us a pass.)
@@ -470,7 +506,8 @@ digit_offsets_kernel(const int64_t* __restrict__ counts, int64_t num_blocks,
     const int64_t t = t0 + threadIdx.x * kDigitItems;
     int64_t n[kDigitItems], mine = 0;
 #pragma unroll
-    for (int k = 0; k < kDigitItems; ++k) n[k] = counts[row + (t + k < num_blocks ? t + k : 0)];
+    for (int k = 0; k < kDigitItems; ++k)
+      n[k] = counts[(t + k < num_blocks ? t + k : 0) * kRadix + blockIdx.x];
 #pragma unroll
     for (int k = 0; k < kDigitItems; ++k) {
       if (t + k >= num_blocks) n[k] = 0;
@@ -542,16 +579,15 @@ radix_pass_kernel(Src src, const ValT* __restrict__ val_in, int64_t E, int shift
   const int digit = threadIdx.x;  // of the first 256 threads
   int64_t all = 0, before_tile = 0;
   if (digit < kRadix) {
-    const int64_t* row = offsets + static_cast<int64_t>(digit) * num_blocks;
     if (SELF) {
       for (int64_t b = 0; b < num_blocks; ++b) {
-        const int64_t c = row[b];
+        const int64_t c = offsets[b * kRadix + digit];
         all += c;
         before_tile += b < tile ? c : 0;
       }
     } else {
       all = totals[digit];
-      before_tile = row[tile];
+      before_tile = offsets[static_cast<int64_t>(digit) * num_blocks + tile];
     }
   }
   for (int j = threadIdx.x; j < T::kWaves * kRadix / 2; j += kThreadsHere)
@@ -698,10 +734,230 @@ radix_pass_kernel(Src src, const ValT* __restrict__ val_in, int64_t E, int shift
   }
 }
 
-// Behind the sort of 64-bit values: fetches them all again when one did not fit 32 bits.
+// The same with the value INSIDE the word, which then is all that a pass moves: 16 bits of what is
+// left of the key, then the value, then the position of the edge.  The word of a pass does not
+// hold the digit that the pass sorted by: the next pass knows it from where it finds the word
+// (the digits' totals) and puts it in the place of its own, so that a key of up to three digits
+// needs room for two.  A value that does not fit the bits that are left raises `wide`.  The next
+// pass's digits are written beside the words, for its histogram to read a byte an edge.
+// 14 M edges, 22-bit keys (24 bits each for value and position): the passes 72 + 65 + 82 us with the
+// values beside the words, 67 + 59 + 81 so; the last two histograms 24 -> 8 each.
+constexpr int kRestAt = 48;     // of the key's digits in a word
+constexpr int kPackedPasses = 3;
+
+template <typename T, typename IdT, int PASS, bool LAST>
+__global__ void __launch_bounds__(T::kThreadsPerTile, T::kWaves == 16 ? 8 : 4)  // (what LDS allows)
+packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
+                   const unsigned long long* __restrict__ in, int64_t E, int value_bits,
+                   int64_t num_blocks, const int64_t* __restrict__ offsets,
+                   const int64_t* __restrict__ totals, const int64_t* __restrict__ totals_before,
+                   unsigned long long* __restrict__ out, unsigned char* __restrict__ next_digit,
+                   SortOutputs<IdT> last) {
+  constexpr int kThreadsHere = T::kThreadsPerTile, kItemsHere = T::kPerThread;
+  constexpr bool FIRST = PASS == 0;
+  constexpr int kCountBytes = T::kWaves * kRadix * 2;
+  __shared__ unsigned long long s_word[T::kSize];
+  __shared__ int64_t s_base[kRadix];  // memory position of a digit's run minus its place in the tile
+  __shared__ int64_t s_all[kRadix];
+  // per wave: count, then count of the earlier waves; and when every item has its place, the
+  // digits in the tile's sorted order
+  __shared__ __attribute__((aligned(16))) unsigned char
+      s_shared[kCountBytes > T::kSize ? kCountBytes : T::kSize];
+  __shared__ int s_start[kRadix];     // where the run of a digit starts in the tile
+  __shared__ uint32_t s_bound[kRadix];  // where the items of a digit of the pass before end
+  __shared__ int s_scan[kRadix / kWave];
+  __shared__ uint32_t s_ends[kRadix / kWave];
+  __shared__ int64_t s_digits[kRadix / kWave];
+  unsigned short (*s_cnt)[kRadix] = reinterpret_cast<unsigned short (*)[kRadix]>(s_shared);
+  unsigned char* s_dig = s_shared;
+  // consecutive tiles on one XCD, as above
+  const int64_t share = num_blocks / kXcds, more = num_blocks % kXcds, xcd = blockIdx.x % kXcds;
+  const int64_t tile = xcd * share + (xcd < more ? xcd : more) + blockIdx.x / kXcds;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x / kWave;
+  const int digit = threadIdx.x;  // of the first 256 threads
+  int64_t all = 0, before_tile = 0;
+  uint32_t ends = 0;
+  if (digit < kRadix) {
+    all = totals[digit];
+    before_tile = offsets[static_cast<int64_t>(digit) * num_blocks + tile];
+    if (!FIRST) ends = static_cast<uint32_t>(totals_before[digit]);
+  }
+  for (int j = threadIdx.x; j < kCountBytes / 4; j += kThreadsHere)
+    reinterpret_cast<uint32_t*>(s_shared)[j] = 0u;
+  const int64_t base = tile * T::kSize;
+  const uint32_t n = E - base < T::kSize ? static_cast<uint32_t>(E - base) : T::kSize;
+  const uint32_t mine0 = wave * (T::kSize / T::kWaves) + lane;
+  uint32_t fresh[FIRST ? kItemsHere : 1];
+  unsigned long long word[FIRST ? 1 : kItemsHere];
+#pragma unroll
+  for (int r = 0; r < kItemsHere; ++r) {
+    const uint32_t j = mine0 + r * kWave;
+    if constexpr (FIRST)
+      fresh[r] = static_cast<uint32_t>((key + base)[j < n ? j : n - 1]);
+    else
+      word[r] = (in + base)[j < n ? j : n - 1];
+  }
+  // (what lies behind the last edge takes the last digit, as above)
+#pragma unroll
+  for (int r = 0; r < kItemsHere; ++r) {
+    if (mine0 + r * kWave >= n) {
+      if constexpr (FIRST) fresh[r] = ~0u; else word[r] = ~0ull;
+    }
+  }
+  if (digit < kRadix) {
+    s_all[digit] = all;
+    s_base[digit] = before_tile;
+    if (!FIRST) {
+#pragma unroll
+      for (int d = 1; d < kWave; d <<= 1) {
+        const uint32_t y = __shfl_up(ends, d, kWave);
+        if (lane >= d) ends += y;
+      }
+      s_bound[digit] = ends;
+      if (lane == kWave - 1) s_ends[wave] = ends;
+    }
+  }
+  __syncthreads();  // the tables are zero
+  auto digit_here = [&](int r) {
+    if constexpr (FIRST)
+      return static_cast<int>(fresh[r] & (kRadix - 1));
+    else
+      return static_cast<int>(word[r] >> (kRestAt + kRadixBits * (PASS - 1))) & (kRadix - 1);
+  };
+  int place[kItemsHere];
+#pragma unroll
+  for (int r = 0; r < kItemsHere; ++r) {
+    const int d = digit_here(r);
+    uint32_t lo = ~0u, hi = ~0u;  // lanes with this digit, as above
+#pragma unroll
+    for (int b = 0; b < kRadixBits; ++b) {
+      const int mine = static_cast<int>(static_cast<uint32_t>(d) << (31 - b)) >> 31;
+      const unsigned long long bal = __ballot(mine);
+      lo = __builtin_amdgcn_bitop3_b32(lo, static_cast<uint32_t>(bal), mine, 0x90);
+      hi = __builtin_amdgcn_bitop3_b32(hi, static_cast<uint32_t>(bal >> 32), mine, 0x90);
+    }
+    const int rank = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0));
+    const int before = s_cnt[wave][d];  // the wave's earlier rounds (LDS operations of a wave keep their order)
+    place[r] = before + rank;
+    if (rank == 0) s_cnt[wave][d] = static_cast<unsigned short>(before + __popc(lo) + __popc(hi));
+  }
+  IdT raw[FIRST ? kItemsHere : 1];
+  if constexpr (FIRST) {  // the values, asked for behind the ranking: see above
+    const IdT* __restrict__ tile_val = value + base;
+    uint32_t again0 = mine0;
+    asm volatile("" : "+v"(again0));
+#pragma unroll
+    for (int r = 0; r < kItemsHere; ++r) {
+      const uint32_t j = again0 + r * kWave;
+      raw[r] = tile_val[j < n ? j : n - 1];
+    }
+  }
+  __syncthreads();
+  int total = 0, incl = 0;
+  int64_t run_at = 0;
+  if (digit < kRadix) {
+    run_at = s_all[digit];
+    if (!FIRST)
+      for (int w = 0; w < wave; ++w) ends += s_ends[w];
+#pragma unroll
+    for (int w = 0; w < T::kWaves; ++w) {
+      const int c = s_cnt[w][digit];
+      s_cnt[w][digit] = static_cast<unsigned short>(total);
+      total += c;
+    }
+    incl = total;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int y = __shfl_up(incl, d, kWave);
+      const int64_t z = __shfl_up(run_at, d, kWave);
+      if (lane >= d) {
+        incl += y;
+        run_at += z;
+      }
+    }
+    if (lane == kWave - 1) {
+      s_scan[wave] = incl;
+      s_digits[wave] = run_at;
+    }
+  }
+  __syncthreads();
+  if (digit < kRadix) {
+    int start = incl - total;
+    run_at += s_base[digit] - s_all[digit];
+    for (int w = 0; w < wave; ++w) {
+      start += s_scan[w];
+      run_at += s_digits[w];
+    }
+    s_start[digit] = start;
+    s_base[digit] = run_at - start;
+    if (!FIRST) s_bound[digit] = ends;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kItemsHere; ++r) {
+    const int d = digit_here(r);
+    place[r] += s_start[d] + s_cnt[wave][d];
+  }
+  // the digit of the pass before at the thread's first item; its later ones lie behind
+  int was = 0;
+  if (!FIRST) {
+    const uint32_t at = static_cast<uint32_t>(base) + mine0;
+#pragma unroll
+    for (int step = kRadix / 2; step > 0; step >>= 1)
+      if (s_bound[was + step - 1] <= at) was += step;
+  }
+  __syncthreads();  // (the counts make room for the digits)
+  bool wide = false;
+  uint32_t third0 = mine0;  // (indices made once more rather than kept)
+  asm volatile("" : "+v"(third0));
+#pragma unroll
+  for (int r = 0; r < kItemsHere; ++r) {
+    const uint32_t j = third0 + r * kWave;
+    const int d = digit_here(r);
+    unsigned long long w;
+    if constexpr (FIRST) {
+      const unsigned long long v = static_cast<unsigned long long>(raw[r]);
+      wide |= (v >> value_bits) != 0ull;
+      w = static_cast<unsigned long long>(fresh[r] >> kRadixBits) << kRestAt |
+          (v & ((1ull << value_bits) - 1ull)) << (kRestAt - value_bits) | static_cast<uint32_t>(base + j);
+    } else {
+      const uint32_t at = static_cast<uint32_t>(base) + j;
+      while (was < kRadix - 1 && s_bound[was] <= at) ++was;
+      constexpr int kAt = kRestAt + kRadixBits * (PASS - 1);  // this pass's digit
+      w = (word[r] & ~(static_cast<unsigned long long>(kRadix - 1) << kAt)) |
+          static_cast<unsigned long long>(was) << kAt;
+    }
+    s_word[place[r]] = w;
+    s_dig[place[r]] = static_cast<unsigned char>(d);
+  }
+  if (FIRST && wide) *last.wide = 1;  // (the last edge's value again past the end)
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kItemsHere; ++k) {
+    const uint32_t j = k * kThreadsHere + threadIdx.x;
+    if (j < n) {
+      const unsigned long long w = s_word[j];
+      const uint32_t d = s_dig[j];
+      const int64_t dst = s_base[d] + j;
+      if (LAST) {
+        last.perm[dst] = static_cast<int64_t>(w & ((1ull << (kRestAt - value_bits)) - 1ull));
+        last.value[dst] = static_cast<IdT>((w & ((1ull << kRestAt) - 1ull)) >> (kRestAt - value_bits));
+        if (last.key)
+          last.key[dst] = d << (kRadixBits * PASS) | static_cast<uint32_t>(w >> kRestAt);
+      } else {
+        out[dst] = w;
+        next_digit[dst] = static_cast<unsigned char>(w >> (kRestAt + kRadixBits * PASS));
+      }
+    }
+  }
+}
+
+// Behind the sort: fetches the values all again when one did not fit its bits.
+template <typename IdT>
 __global__ void __launch_bounds__(kThreads)
-widen_values_kernel(const int64_t* __restrict__ value, const int64_t* __restrict__ perm, int64_t E,
-                    const int* __restrict__ wide, int64_t* __restrict__ out) {
+widen_values_kernel(const IdT* __restrict__ value, const int64_t* __restrict__ perm, int64_t E,
+                    const int* __restrict__ wide, IdT* __restrict__ out) {
   if (*wide == 0) return;
   const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < E; i += stride)
@@ -772,7 +1028,7 @@ void launch_pass(Src src, bool last, bool self, hipStream_t st, const ValT* vin,
 struct SortSpace {
   unsigned long long* word[2];
   uint32_t* value[2];
-  int64_t *counts, *offsets, *totals;
+  int64_t *counts, *offsets, *totals, *totals_before;
   uint32_t* keys;
   int* wide;
 };
@@ -781,7 +1037,7 @@ inline size_t sort_space_bytes(int64_t E) {
   const int64_t table = kRadix * static_cast<int64_t>(blocks_for(E, SmallTile::kSize));
   const size_t n = static_cast<size_t>(E > 0 ? E : 1);
   return 2 * padded(n * 8) + 3 * padded(n * 4) + 2 * padded(static_cast<size_t>(table) * 8) +
-         padded(kRadix * 8) + 256;
+         2 * padded(kRadix * 8) + 256;
 }
 inline bool carve_sort(Carver& ws, int64_t E, SortSpace* s) {
   const int64_t table = kRadix * static_cast<int64_t>(blocks_for(E, SmallTile::kSize));
@@ -792,6 +1048,7 @@ inline bool carve_sort(Carver& ws, int64_t E, SortSpace* s) {
   s->counts = ws.take<int64_t>(static_cast<size_t>(table));
   s->offsets = ws.take<int64_t>(static_cast<size_t>(table));
   s->totals = ws.take<int64_t>(kRadix);
+  s->totals_before = ws.take<int64_t>(kRadix);
   s->wide = ws.take<int>(1);
   return ws.ok;
 }
@@ -810,10 +1067,10 @@ int sort_passes(const IdT* key, const IdT* value, int64_t E, int passes, int idx
     const StoredWords stored{s.word[(p + 1) & 1]};
     if (p == 0)
       hipLaunchKernelGGL((radix_hist_kernel<T, FreshWords<IdT>>), grid, dim3(T::kThreadsPerTile), 0,
-                         st, fresh, E, shift, blocks, s.counts, outs.wide);
+                         st, fresh, E, shift, s.counts, outs.wide);
     else
       hipLaunchKernelGGL((radix_hist_kernel<T, StoredWords>), grid, dim3(T::kThreadsPerTile), 0, st,
-                         stored, E, shift, blocks, s.counts, static_cast<int*>(nullptr));
+                         stored, E, shift, s.counts, static_cast<int*>(nullptr));
     if (!self)
       hipLaunchKernelGGL(digit_offsets_kernel, dim3(kRadix), dim3(kDigitThreads), 0, st, s.counts,
                          blocks, s.offsets, s.totals);
@@ -823,6 +1080,43 @@ int sort_passes(const IdT* key, const IdT* value, int64_t E, int passes, int idx
     else
       launch_pass<T>(stored, last, self, st, static_cast<const uint32_t*>(s.value[(p + 1) & 1]), E,
                      shift, blocks, where, s.totals, s.word[p & 1], s.value[p & 1], outs);
+  }
+  return check_launch("coo2csc");
+}
+
+// Bits of a value in the words of a sort; 0: not packed (few tiles, one pass or more than three, or
+// hardly any bits left for the values, which are expected to be ids like the keys).
+inline int packed_value_bits(int64_t E, int64_t num_keys, int passes, int64_t tiles) {
+  const int bits = kRestAt - bits_for(E) < 32 ? kRestAt - bits_for(E) : 32;
+  return passes >= 2 && passes <= kPackedPasses && E < (int64_t(1) << 32) && tiles > kSelfScanTiles &&
+                 bits >= bits_for(num_keys) ? bits : 0;
+}
+
+template <typename T, typename IdT>
+int packed_passes(const IdT* key, const IdT* value, int64_t E, int passes, int value_bits,
+                  const SortSpace& s, const SortOutputs<IdT>& outs, hipStream_t st) {
+  const int64_t blocks = blocks_for(E, T::kSize);
+  const dim3 grid(static_cast<unsigned>(blocks)), threads(T::kThreadsPerTile);
+  const int idx_bits = bits_for(E);
+  unsigned char* digits = reinterpret_cast<unsigned char*>(s.value[0]);  // (the values have no place of their own)
+  for (int p = 0; p < passes; ++p) {
+    const bool last = p == passes - 1;
+    const unsigned long long* in = s.word[(p + 1) & 1];
+    if (p == 0)
+      hipLaunchKernelGGL((radix_hist_kernel<T, FreshWords<IdT>>), grid, threads, 0, st,
+                         FreshWords<IdT>{key, idx_bits}, E, idx_bits, s.counts, outs.wide);
+    else
+      hipLaunchKernelGGL(digit_hist_kernel<T>, grid, threads, 0, st, digits, E, s.counts);
+    int64_t* totals = p & 1 ? s.totals_before : s.totals;
+    const int64_t* totals_before = p & 1 ? s.totals : s.totals_before;
+    hipLaunchKernelGGL(digit_offsets_kernel, dim3(kRadix), dim3(kDigitThreads), 0, st, s.counts, blocks,
+                       s.offsets, totals);
+    const auto kernel = p == 0 ? packed_pass_kernel<T, IdT, 0, false>
+                        : p == 2 ? packed_pass_kernel<T, IdT, 2, true>
+                        : last ? packed_pass_kernel<T, IdT, 1, true>
+                               : packed_pass_kernel<T, IdT, 1, false>;
+    hipLaunchKernelGGL(kernel, grid, threads, 0, st, key, value, in, E, value_bits, blocks, s.offsets,
+                       totals, totals_before, s.word[p & 1], digits, outs);
   }
   return check_launch("coo2csc");
 }
@@ -851,18 +1145,23 @@ int coo2csc_impl(const IdT* key, const IdT* value, int64_t E, int64_t num_keys, 
                    gs_coo2csc_workspace_bytes(E, num_keys));
     return GS_ERR_WORKSPACE;
   }
-  const bool may_be_wide = sizeof(IdT) == 8;
+  const bool large = E >= kLargeTileItems;
+  const int value_bits =
+      packed_value_bits(E, num_keys, passes, blocks_for(E, large ? LargeTile::kSize : SmallTile::kSize));
+  const bool may_be_wide = sizeof(IdT) == 8 || value_bits > 0;
   const bool short_keys = passes * kRadixBits <= 32;
   const SortOutputs<IdT> outs{out_value, perm, indptr && short_keys ? s.keys : nullptr, idx_bits,
                               may_be_wide ? s.wide : nullptr};
-  if (E >= kLargeTileItems)
-    GS_RETURN_IF_ERROR((sort_passes<LargeTile, IdT>(key, value, E, passes, idx_bits, s, outs, st)));
-  else
-    GS_RETURN_IF_ERROR((sort_passes<SmallTile, IdT>(key, value, E, passes, idx_bits, s, outs, st)));
+  if (value_bits > 0) {
+    const auto sort = large ? packed_passes<LargeTile, IdT> : packed_passes<SmallTile, IdT>;
+    GS_RETURN_IF_ERROR(sort(key, value, E, passes, value_bits, s, outs, st));
+  } else {
+    const auto sort = large ? sort_passes<LargeTile, IdT> : sort_passes<SmallTile, IdT>;
+    GS_RETURN_IF_ERROR(sort(key, value, E, passes, idx_bits, s, outs, st));
+  }
   if (may_be_wide)
-    hipLaunchKernelGGL(widen_values_kernel, dim3(E < (int64_t(1) << 20) ? 64 : 1024), dim3(kThreads),
-                       0, st, reinterpret_cast<const int64_t*>(value), perm, E, s.wide,
-                       reinterpret_cast<int64_t*>(out_value));
+    hipLaunchKernelGGL(widen_values_kernel<IdT>, dim3(E < (int64_t(1) << 20) ? 64 : 1024),
+                       dim3(kThreads), 0, st, value, perm, E, s.wide, out_value);
   if (indptr && short_keys)  // (null: the caller wants the sorted order only)
     launch_indptr(static_cast<const uint32_t*>(s.keys), E, num_keys, indptr, st);
   else if (indptr)

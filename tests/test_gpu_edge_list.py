@@ -89,6 +89,26 @@ def test_sort_with_large_tiles(dev, num_keys, extra, idt):
 
 
 @pytest.mark.parametrize("idt", ID_DTYPES)
+@pytest.mark.parametrize("E", [64 * 4096, 64 * 4096 + 1, 70 * 4096 - 1, (1 << 22) - 1, (1 << 22) + 8193])
+@pytest.mark.parametrize("num_keys,skew", [(257, 1), (65536, 3), (65537, 3), (1 << 22, 12), (1 << 24, 1)])
+def test_sort_with_the_values_in_its_words(dev, num_keys, skew, E, idt):
+    """From 65 tiles on a sort of two or three digits carries the values in its 64-bit words, beside
+    sixteen bits of the key and the edge's position: the largest value that fits, and one more."""
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(num_keys + E)
+    key = (torch.rand(E, generator=gen, device=dev, dtype=torch.float64) ** skew * num_keys).to(idt)
+    bits = min(32, 48 - (E - 1).bit_length(), 31 if idt == torch.int32 else 32)
+    value = torch.randint(0, 1 << 20, (E,), generator=gen, device=dev).to(idt)
+    want = torch.sort(key, stable=True)
+    ends = torch.cumsum(torch.bincount(key.long(), minlength=num_keys), 0)
+    for extra in ([0, 1] if bits < 31 else [0]):
+        value[E // 3] = (1 << bits) - 1 + extra
+        ip, val, perm = capi.coo2csc(key, value, num_keys, False)
+        assert torch.equal(perm, want.indices) and torch.equal(val, value[want.indices])
+        assert int(ip[0]) == 0 and torch.equal(ip[1:], ends)
+
+
+@pytest.mark.parametrize("idt", ID_DTYPES)
 @pytest.mark.parametrize("keys", [[0], [9999], [0, 17, 18, 9000], [5000, 5016, 5032, 7200, 9998]])
 def test_offsets_over_gaps(dev, keys, idt):
     """Sorted keys, more edges than columns, gaps on both sides of the lengths one lane, a wave
