@@ -102,6 +102,8 @@ tile_heads_kernel(const int64_t* __restrict__ indptr, const IdT* __restrict__ nm
       if (begin < stop) {
         if (stop == edges.end) tl.head[t1 + 1] = static_cast<int>(s);
         if (MARK) tl.mark[begin - edges.first] = static_cast<int>(s);
+      } else if (SUM) {  // (behind the last edge that counts)
+        out[nmap ? static_cast<int64_t>(nmap[s]) : s] = 0.0f;
       }
     } else if (SUM) {
       out[nmap ? static_cast<int64_t>(nmap[s]) : s] = 0.0f;

