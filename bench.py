@@ -918,7 +918,7 @@ def _sb_sample(b, S, E, U):
 
 
 # launch sites of the super-batch flow and the least bytes of each one's third-layer launch
-# (M = S + E items; the binned relabel: count reads the ids, scatter reads them and writes an
+# (M = S + E items; the binned relabel: tiles, or count and scatter, read the ids and write an
 # 8-byte record each, first reads the records and writes a 4-byte position each, rank reads
 # those and writes 16 bytes per 64 items, rename reads the positions, a 16-byte entry each and
 # the ids of the frontier and writes the renamed ids and the frontier)
@@ -926,6 +926,8 @@ SUPER_SITES = {
     "sample_fused": _sb_sample,
     "bins_count": lambda b, S, E, U: (S + E) * b,
     "bins_scatter": lambda b, S, E, U: (S + E) * (b + 8),
+    "bins_plan": lambda b, S, E, U: 0,
+    "bins_tiles": lambda b, S, E, U: (S + E) * (b + 8),
     "bins_first": lambda b, S, E, U: (S + E) * 12,
     "bins_rank": lambda b, S, E, U: (S + E) * (4 + 0.25),
     "bins_rename": lambda b, S, E, U: (S + E) * (4 + 16) + E * b + U * 2 * b,

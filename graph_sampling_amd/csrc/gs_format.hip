@@ -548,8 +548,9 @@ struct SortOutputs {
 // no pass gathers it by position; the LAST pass writes values, permutation and keys instead
 // of words.  64-bit values travel in their low 32 bits: ids of any graph that fits the card do,
 // and a value that does not raises `wide`, on which widen_values_kernel fetches all of them
-// again through the permutation.  14 M edges with 64-bit ids and 22-bit keys: 109 us the first pass
-// (histogram, scan, scatter; it reads the ids as they come), 96 and 111 the others.
+// again through the permutation.  14 M edges with 64-bit ids and 22-bit keys: 78 us the first pass
+// (it reads the ids as they come), 67 and 82 the others; with the values inside the words
+// (packed_pass_kernel) 67, 59 and 82.
 // SELF: `offsets` holds the tiles' raw counts and every workgroup adds up for itself where its
 // runs start (a sort of few tiles: a launch less per pass than scanning the counts first).
 constexpr int64_t kSelfScanTiles = 64;
