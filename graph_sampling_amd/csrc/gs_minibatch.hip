@@ -83,9 +83,10 @@ __device__ __forceinline__ void give_ranks(unsigned int flags, const uint32_t (&
   *unique += total;
 }
 
-// Layer `l`: columns 0..S-1, whose ids s_from holds, sampled kRows at a time, G lanes a column; *unique = the frontier's length so far.  A round's samples are
-// all entered before any of them is ranked, and a later round's items have larger numbers, so
-// what a round finds to be a first occurrence is one.
+// Layer `l`: columns 0..S-1, whose ids s_from holds, sampled kRows at a time, G lanes a column;
+// *unique = the frontier's length so far.  The samples of one such pass are all entered before any
+// of them is ranked, and a later pass's items have larger numbers than every item and rank before
+// them, so what a pass finds to be a first occurrence is one.
 template <typename IdT, int G, bool REPLACE>
 __device__ __forceinline__ void one_layer(const OneArgs& a, int l, int S, int* unique,
                                           const PackedTable& t, const uint32_t* s_from,
