@@ -409,8 +409,11 @@ __device__ __forceinline__ void run_task(const WArgs<IdT>& a, const Task& e, int
   const int found = group_topk<false>(edges, lo, full_here, s, a.k, [&](int j, unsigned long long c) { lb_store(&out[j], c); });
   for (int j = found + threadIdx.x; j < a.k; j += kThreads) lb_store(&out[j], 0ull);  // fewer than k edges
   const int64_t chunks = (e.deg + kChunk - 1) / kChunk;
-  // the candidates are stored and read with device scope and every wave's have completed before
-  // the workgroup counts itself (an L2 released per chunk: 52 us a fill, so 30)
+  // The candidates are stored and read with device scope, past the caches, so all that the count
+  // needs before it is that they have arrived: every thread waits for its OWN stores (the
+  // vector-memory counter; neither a workgroup-scope release nor the barrier waits for it) and only
+  // then meets the others.  (An L2 released per chunk: 52 us a fill, so 30.)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __syncthreads();
   if (threadIdx.x == 0)
