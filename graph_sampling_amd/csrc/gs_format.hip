@@ -22,6 +22,8 @@
 //    the workgroup's 256 columns.
 //  * distinct ids of an edge list: a bit per possible id in LDS, slice by slice, or, for short
 //    lists and large ids, a byte per possible id marked with plain stores.
+#include <algorithm>
+
 #include "gs_common.hpp"
 #include "gs_one.hpp"
 
@@ -1602,10 +1604,14 @@ constexpr int kSumTile = kBinThreads * kSumTileItems;
 constexpr int kMaxBins = 1024;
 constexpr int kBinMaxShift = 13;          // 2^13 sums = 64 KB of LDS
 constexpr int kBinMinBits = 8;            // 256 bins at least, where there are as many targets
-// The additions to one LDS word queue up, so a bin of more than twice the average (a hub's) is shared
-// by several workgroups, the average each, which then add their sums to memory with atomics.
+// The additions to one LDS word queue up, so a bin of more than 5/4 of the average (a hub's) is
+// shared by several workgroups, which then add their sums to memory with atomics.  Shares by the average
+// alone left a bin of twice as much to one workgroup, and, of three targets, each: 30 M edges,
+// uniform / skewed, 3 targets 12900 / 7630 us, now 279 / 330; 40: 1090 / 1192, now 282 / 294; 256: 277 / 542,
+// now 277 / 455; 30 k: 216 / 274, now 215 / 259.
 constexpr int kBinParts = 256;           // workgroups that may share one bin
-constexpr int64_t kBinPartItems = 8192;  // edges a share has at least
+constexpr int64_t kBinPartItems = 4096;  // edges a share has at least
+constexpr int64_t kBinPartMost = 16384;  // and at most, where 256 shares of the bin allow it
 constexpr int kBinLineBits = 5;           // 32 targets, 128 bytes
 
 // Target t is sum `place` of bin `place >> bin_shift`: its line number times an odd number.
@@ -1820,11 +1826,19 @@ bin_sum_kernel(SumSpace s, int64_t tiles, int64_t alone, int64_t part_items, Bin
   }
 }
 
-// whether the binned path takes the call: plain edge order, few enough targets for 1024 bins of
-// 2^13, enough edges for three launches to pay
+// Whether the binned path takes the call: plain edge order, few enough targets for 1024 bins of
+// 2^13, enough edges for three launches to pay.  Few targets meet in the plain kernel's LDS tables
+// already; among very many, its atomics to memory cost less than clearing and writing all sums.
+// Plain / binned, us, uniform and skewed targets, at the lines and beyond:
+//   E x targets 2^23: 131 k edges, 10 targets  13/34  14/46, 100   28/16  29/33
+//                     524 k        10          38/29  38/47,  40   66/19  66/38
+//                       1 M         3          29/37  30/60,  10   73/28  75/49
+//                     8.4 M         1         100/108 99/108,  3  174/100 176/104
+//   32 targets an edge: 131 k, 8 M targets     16/26  27/28, 2.45 M 16/18 28/22; 262 k, 8 M 21/28 46/31
 inline bool bin_sum_applies(const int64_t* e_ids, int64_t E, int64_t num_targets) {
   return !e_ids && E >= (int64_t(1) << 17) && num_targets > 0 &&
-         num_targets <= (int64_t(kMaxBins) << kBinMaxShift) && E < (int64_t(1) << 31);
+         num_targets <= (int64_t(kMaxBins) << kBinMaxShift) && E < (int64_t(1) << 31) &&
+         E * num_targets > (int64_t(1) << 23) && num_targets <= 32 * E;
 }
 
 inline int64_t sum_tiles(int64_t E) { return (E + kSumTile - 1) / kSumTile; }
@@ -1856,9 +1870,10 @@ int bin_sum_impl(const IdT* target, const float* data, int64_t E, int powk, int6
   hipLaunchKernelGGL(sum_tiles_kernel<IdT>, dim3(static_cast<unsigned>(tiles)), dim3(kBinThreads), 0, st,
                      target, data, E, num_targets, powk, order, s);
   hipLaunchKernelGGL(sum_totals_kernel, dim3(order.bins), dim3(kThreads), 0, st, s, tiles, order.bins);
-  const int64_t average = E / order.bins;
-  const int64_t part_items = average > kBinPartItems ? average : kBinPartItems;
-  const int64_t alone = 2 * part_items;
+  // (few targets make few bins: the average is that of 256 then, so that every bin is shared)
+  const int64_t average = std::max(E / std::max(order.bins, 1 << kBinMinBits), kBinPartItems);
+  const int64_t part_items = std::min(average, kBinPartMost);
+  const int64_t alone = average + average / 4;
   const int64_t shares = E / part_items + order.bins;  // at most: sum of ceil(n / part_items) over the bins
   hipLaunchKernelGGL(bin_sum_kernel, dim3(static_cast<unsigned>(shares)), dim3(kBinThreads),
                      sizeof(double) << order.bin_shift, st, s, tiles, alone, part_items, order,

@@ -680,7 +680,7 @@ int gs_coo_sum(const void* target, int id_bytes, const int64_t* e_ids, const flo
 
 /* The same sums for callers that know how many targets there are (out has num_targets
  * entries; a target beyond is left out) and bring a workspace: with no e_ids, at least 2^17
- * edges and at most 2^23 targets the edges are first brought together by bins of targets and then
+ * edges, at most 2^23 targets and 32 an edge, and more than 2^23 edges times targets, the edges are first brought together by bins of targets and then
  * added up in LDS, a bin per workgroup, with no atomic to memory -- several times faster than
  * gs_coo_sum when most edges hit different targets.  Any other call is passed on to gs_coo_sum.  The order of
  * the additions is not fixed in either (impl::COOSumCUDA, src/cuda/graph_ops.cu:45-64, adds

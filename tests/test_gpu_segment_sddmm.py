@@ -217,11 +217,18 @@ def test_coo_sum_and_e_div_u_sum(dev, idt):
 @pytest.mark.parametrize("targets,edges,skew", [
     (2_450_000, 1 << 20, True),    # a LADIES row sum: many targets, hubs among them
     (2_450_000, 1 << 20, False),
-    (1000, 1 << 18, False),        # fewer targets than runs: every run is one target
-    (1 << 23, 300_000, True),      # the widest runs (2^15 sums in LDS)
-    ((1 << 23) + 1, 300_000, False),  # one target too many for the runs: the plain kernel
+    (1000, 1 << 18, False),        # bins of a few targets
+    (1 << 23, 300_000, True),      # the widest bins (2^13 sums in LDS)
+    ((1 << 23) + 1, 300_000, False),  # one target too many for the bins: the plain kernel
     (70_000, (1 << 17) - 1, False),   # one edge short of the binned path
-    (5, 1 << 19, False),           # one run shared by several workgroups
+    (5, 1 << 19, False),           # so few targets that they meet in the plain kernel's tables
+    (5, 1 << 21, False),           # a bin a target, all of them shared by several workgroups
+    (1, (1 << 23) + 1, False),     # one bin, 256 shares
+    (3, (1 << 23) // 3, False),    # edges times targets at the line ...
+    (3, (1 << 23) // 3 + 1, False),   # ... and beyond
+    (1 << 22, 1 << 17, False),     # 32 targets an edge ...
+    ((1 << 22) + 1, 1 << 17, False),  # ... and beyond: the plain kernel
+    (200, 3 << 20, True),          # bins of one target, some alone, the hubs' shared
 ])
 def test_coo_sum_binned(dev, idt, targets, edges, skew):
     """The sums with a known number of targets: against float64 sums of the same products (the
@@ -269,6 +276,27 @@ def test_coo_sum_binned_leaves_out_targets_beyond_the_output(dev, edges):
     want = np.bincount(t[ok], weights=data[ok].astype(np.float64), minlength=targets)
     np.testing.assert_allclose(out.cpu().numpy(), want, rtol=2e-5)
     assert bool((buf[targets:] == 7.0).all())
+
+
+def test_coo_sum_binned_of_few_targets_is_spread_over_the_chip(dev):
+    """Three targets' bins are shared like a hub's: 4 M edges in at most eight times what they take
+    for 1000 targets (1.5 times; some fifty when a bin was one workgroup's)."""
+    edges = 1 << 22
+    data = torch.rand(edges, device=dev)
+    took = {}
+    for targets in (3, 1000):
+        t = torch.randint(0, targets, (edges,), device=dev, dtype=torch.int32)
+        out = torch.zeros(targets, dtype=torch.float32, device=dev)
+        times = []
+        for _ in range(6):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            capi.coo_sum_binned(t, None, data, 1, out)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        took[targets] = min(times)
+    assert took[3] < 8 * took[1000], took
 
 
 @pytest.mark.parametrize("idt", ID_DTYPES)
