@@ -825,12 +825,22 @@ int segment_normalize_impl(const int64_t* indptr, const int64_t* emap, const flo
 constexpr int kAggEdges = 8;  // edges per thread
 
 // Few edges are spread over more workgroups, two a thread: the launch is then a handful of trips
-// to memory and an LDS table to clear, which a shorter tile has less of (22 k edges 16 -> 6 us).
-// Every target of a tile costs an addition to memory, so that longer tiles win beyond (60 k edges,
-// whole call, two / eight a thread: uniform targets 10/12 us, skewed like R-MAT's rows 14-20/15-17,
-// a tenth of them on one target 24-27/17).
+// to memory and an LDS table to clear, which a shorter tile has less of.  Every target of a tile costs
+// an addition to memory, though, and those to one target queue up, so beyond 8192 edges short tiles
+// are for eight targets an edge and more.  The launch alone in us, two / eight a thread, targets
+// skewed (a sixth to a third of the edges on one) and uniform:
+//            100 targets          20 k               2.45 M
+//    5 k    5.1/5.3  5.1/4.9    4.5/7.2  4.0/8.9    4.3/10.2 5.0/10.1
+//    8 k    6.9/5.3  7.0/4.9    5.9/7.2  4.0/9.0    4.9/10.0 5.0/10.1
+//   22 k   15.0/7.7 15.5/7.4   11.6/8.9  4.6/10.2   8.6/10.1 5.5/11.8
+//   30 k   19.9/9.2 20.7/8.8   15.3/10.2 5.0/9.8   10.5/12.3 6.0/11.2
+// e_div_u_sum adds up by the column of a slice's edges, which come column by column: a tile has few
+// of them (512 columns, 2 k to 30 k edges: 3.1-3.6/6.7-8.1; columns in random order, 1000 skewed
+// ones, 20 k edges: 13/9).
 constexpr int kAggFewEdges = 2;
 constexpr int64_t kAggFew = int64_t(1) << 15;
+constexpr int64_t kAggFewAny = int64_t(1) << 13;
+constexpr int64_t kAggFewTargets = 8;  // an edge
 
 template <int EDGES>
 struct KeyedSums {
@@ -986,7 +996,8 @@ int gs::coo_sum_bounded(const void* target, int id_bytes, const int64_t* e_ids, 
   GS_REQUIRE(E == 0 || (target && data && out), "gs_coo_sum: null pointer");
   GS_REQUIRE(valid_id_bytes(id_bytes), "gs_coo_sum: id_bytes must be 4 or 8, got %d", id_bytes);
   if (E == 0) return GS_OK;
-  const bool few = E < kAggFew;
+  const bool many_targets = num_targets != std::numeric_limits<int64_t>::max() && num_targets >= kAggFewTargets * E;
+  const bool few = E <= kAggFewAny || (E < kAggFew && many_targets);
   const dim3 grid(blocks_for(E, kThreads * (few ? kAggFewEdges : kAggEdges)));
   hipStream_t st = static_cast<hipStream_t>(stream);
   auto launch = [&](auto* kernel, const auto* to) {

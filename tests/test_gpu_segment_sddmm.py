@@ -300,9 +300,11 @@ def test_coo_sum_binned_of_few_targets_is_spread_over_the_chip(dev):
 
 
 @pytest.mark.parametrize("idt", ID_DTYPES)
-@pytest.mark.parametrize("edges", [1, 511, 513, (1 << 17) - 1, 1 << 17, (1 << 17) + 1])
+@pytest.mark.parametrize("edges", [1, 511, 513, 1 << 13, (1 << 13) + 1, (1 << 15) - 1, 1 << 15,
+                                   (1 << 15) + 1, (1 << 17) - 1, 1 << 17, (1 << 17) + 1])
 def test_keyed_sums_at_both_lengths_of_a_tile(dev, idt, edges):
-    """Two edges a thread below 2^17 edges, eight from there on; every edge once, hubs and all."""
+    """Two edges a thread up to 2^13 edges (2^15 where a column adds up, or with eight targets an
+    edge), eight beyond; every edge once, hubs and all."""
     rng = np.random.default_rng(edges)
     n = 3000
     row = (rng.random(edges) ** 3 * n).astype(np.int64)
@@ -323,6 +325,14 @@ def test_keyed_sums_at_both_lengths_of_a_tile(dev, idt, edges):
     np.testing.assert_allclose(osum.cpu().numpy(),
                                np.bincount(col, weights=(data / divisor[row]).astype(np.float64), minlength=n),
                                rtol=2e-5)
+    # sums that know their number of targets: eight an edge, and one short of that
+    for targets in (8 * edges, 8 * edges - 1):
+        to = (rng.random(edges) ** 3 * targets).astype(np.int64)
+        out = torch.zeros(targets, dtype=torch.float32, device=dev)
+        capi.coo_sum_binned(to_dev(to, dev, idt), None, to_dev(data, dev), 2, out)
+        np.testing.assert_allclose(out.cpu().numpy(),
+                                   np.bincount(to, weights=data.astype(np.float64) ** 2, minlength=targets),
+                                   rtol=2e-5)
 
 
 # ------------------------------------------------------------------ SDDMM
