@@ -365,8 +365,12 @@ size_t workspace_bytes_for(int64_t M) {
 // memory each, whatever the length; here the ids are read, and the results written.  Whole call in us, four
 // launches / one, ids of 233 k nodes: 64 items 21/12, 1383 28/14, 6000 32/21, 8192 37/33; beyond, at
 // more than half the table's slots, the chains of a few items hold up their waves (9700 30/39).
+// Look-ups are the same: of skewed ids of 4 M nodes, 4000 items and 4 k, 8 k, 12 k, 16 k, 24 k of them 29/17
+// 29/25 28/25 33/36 28/36, 8192 items 30/26 29/28 29/31 30/37 30/49 (of 1000 nodes, where chains are
+// short, 24/15 to 24/18).  As a COO's columns and rows are renamed, 25 samples a column: 100
+// columns 24/17, 200 24/18, 315 28/32.
 constexpr int64_t kOneItems = 8 * kOneThreads;    // of the mapping: 8 a thread
-constexpr int64_t kOneQueries = 24 * kOneThreads;
+constexpr int64_t kOneQueries = 10 * kOneThreads;
 constexpr int kOneSlots = 16384;                  // 128 KB of LDS, load <= 1/2
 
 template <typename IdT, int PER>

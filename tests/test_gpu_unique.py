@@ -367,6 +367,23 @@ def test_short_lists_by_one_workgroup_and_past_them(dev, idt, n):
             assert np.array_equal(got.cpu().numpy().astype(np.int64), w)
 
 
+@pytest.mark.parametrize("idt", [torch.int64, torch.int32])
+@pytest.mark.parametrize("queries", [1, 4095, 4096, 4097, 10240, 10241, 24577])
+def test_look_ups_of_one_workgroup_and_past_them(dev, idt, queries):
+    """Four look-ups of a thread at a time, up to 10240 by the one-workgroup relabel, from two spans
+    that meet anywhere."""
+    rng = np.random.default_rng(queries)
+    for n in (5, 8192):
+        ids = rng.integers(0, 3 * n, n).astype(np.int64)
+        spans = np.split(rng.integers(0, 4 * n, queries).astype(np.int64), [queries // 3])
+        want_frontier, want = O.relabel([ids], spans)
+        frontier, num, outs = capi.unique_relabel([to_dev(ids, dev, idt)], [to_dev(q, dev, idt) for q in spans],
+                                                  narrow=idt == torch.int64)
+        assert int(num.item()) == want_frontier.size
+        for got, w in zip(outs, want):
+            assert np.array_equal(got.cpu().numpy().astype(np.int64), w)
+
+
 def test_short_list_with_an_id_beyond_32_bits(dev):
     ids = torch.tensor([3, 1, 3, (1 << 40) + 1], dtype=torch.int64, device=dev)
     assert int(capi.unique_relabel([ids], [ids], narrow=True)[1].item()) == -2
