@@ -67,7 +67,15 @@ constexpr int counter_cap(int classes_log2) {
 }
 constexpr int kCounterCap = counter_cap(kMaxClassesLog2);
 // Batches of up to so many items on average go by tiles of runs: at 2^20 items a batch has 512
-// classes and a tile's runs 16 records; 2 M items in one batch, of 8 each, are 139 us by counting.
+// classes and a tile's runs 16 records, at 2^22 of 2048 classes 4.  By counting / by runs, us, ids
+// skewed like R-MAT's rows of 2^14 | 2^17 | 2^21 nodes:
+//    items a batch    one batch                      four
+//    2^19          59/58   53/42   51/37       81/68   79/58   80/55
+//    2^20          87/91   76/72   70/58      158/122 156/122 158/121
+//    2^21         147/163 124/122 117/105     292/296 291/301 300/305
+//    2^22         270/309 225/286 210/280     578/866 585/910 608/964
+// An id that has 4 % of a batch's items fills a bucket that one workgroup reads, and runs
+// are slower to read than records side by side: 2^20 items of 2^12 nodes in one batch 103/123.
 constexpr int64_t kRunsItems = int64_t(1) << 20;
 constexpr int kTileThreads = 1024;     // two such workgroups fill a compute unit's waves
 constexpr int kTileItems = 8;          // items of a thread

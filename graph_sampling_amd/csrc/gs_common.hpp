@@ -329,7 +329,10 @@ constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;
 
 // More items than that and up to kScanFew, a thread takes two instead of eight: what counts at
-// the sizes of a minibatch is how many compute units share the reads (5000 column degrees: 10.4 -> 8.5 us; one workgroup of 1024 threads: 14.4).
+// the sizes of a minibatch is how many compute units share the reads.  Column degrees, eight / two a
+// thread, the launches alone in us: 2049 7.3/5.3, 5000 7.7/5.7, 10000 7.8/5.8, 15872 7.9/5.8, and 20000
+// 8.1/5.7, where scratch for the sums would have to grow; one workgroup of 1024 threads took 14.4 for
+// 5000 where these took 8.5.
 constexpr int kScanFewItems = 2;
 constexpr int64_t kScanFewTile = kScanThreads * kScanFewItems;
 constexpr int64_t kScanFew = 31 * kScanFewTile;  // (their sums fit the 256 bytes that scratch comes in)
