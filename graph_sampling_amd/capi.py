@@ -515,8 +515,9 @@ def sample_one_keepdim(indptr, indices, column_ids, seed=0, replay=None):
 
 
 def sample_weighted(indptr, indices, probs, column_ids, fanout, seed=0, replay=None,
-                    replay_ptr=None, with_coo=False):
-    """gs_sample_count(replace=0) + gs_sample_weighted_fill; same return shape as sample_uniform."""
+                    replay_ptr=None, with_coo=False, queue_chunks=None, ws=None):
+    """gs_sample_count(replace=0) + gs_sample_weighted_fill; same return shape as sample_uniform.
+    queue_chunks: room for so many chunks of long rows (gs_sample_weighted_fill_queue)."""
     _need(indptr, torch.int64, "indptr")
     _need(probs, torch.float32, "probs")
     idb = _ids(indices, "indices")
@@ -533,11 +534,18 @@ def sample_weighted(indptr, indices, probs, column_ids, fanout, seed=0, replay=N
     coo_col = torch.empty(cap, dtype=indices.dtype, device=dev) if with_coo else None
     nbytes = max(lib().gs_sample_workspace_bytes(_i64(S), _i64(fanout)),
                  lib().gs_sample_weighted_workspace_bytes(_i64(S), _i64(fanout)))
-    ws = workspace(nbytes, dev)
+    ws = workspace(nbytes, dev) if ws is None else ws
     st = _stream(dev)
     _check(lib().gs_sample_count(_ptr(indptr), _i64(indptr.numel() - 1), _ptr(column_ids), idb, _i64(S), _i64(fanout), 0,
                                  _ptr(sub_indptr), _ptr(ws), ctypes.c_size_t(ws.numel()), st),
            "gs_sample_count")
+    if queue_chunks is not None:
+        _check(lib().gs_sample_weighted_fill_queue(
+            _ptr(indptr), _i64(indptr.numel() - 1), _ptr(indices), _ptr(probs), _ptr(column_ids), idb,
+            _i64(S), _i64(fanout), _u64(seed), _ptr(replay), _ptr(replay_ptr), _ptr(sub_indptr),
+            _ptr(sub_indices), _ptr(select_index), _ptr(coo_col), None, None, _i64(queue_chunks),
+            _ptr(ws), ctypes.c_size_t(ws.numel()), st), "gs_sample_weighted_fill_queue")
+        return sub_indptr, sub_indices, select_index, coo_col
     _check(lib().gs_sample_weighted_fill(_ptr(indptr), _i64(indptr.numel() - 1), _ptr(indices), _ptr(probs), _ptr(column_ids),
                                          idb, _i64(S), _i64(fanout), _u64(seed), _ptr(replay),
                                          _ptr(replay_ptr), _ptr(sub_indptr), _ptr(sub_indices),

@@ -24,6 +24,8 @@
 // weights, the picks' ids).  So the chunks are found by a launch of their own that only reads
 // offsets, and rows and chunks then go side by side; the last chunk of a row to finish merges
 // the row's candidates.
+#include <limits>
+
 #include "gs_common.hpp"
 #include "gs_one.hpp"
 
@@ -35,7 +37,11 @@ constexpr int kWaves = kThreads / kWave;
 constexpr int64_t kChunk = 2048;          // edges per workgroup task
 constexpr int64_t kSmall = 4 * kWave;     // longest row of one wave: 4 edges a lane
 constexpr int kMaxFanout = 96;
-constexpr int64_t kHubTasks = 1 << 19;    // chunks of rows with several
+// Chunks of rows with several that the queue has room for (their candidates are 8 * fanout bytes
+// each, whether there are any or not).  Rows beyond are a wave's work each, 256 edges at a time, and
+// keep the chip as busy: fanout 10, 300 k rows of 4096 edges (600 k chunks) 4.9 ms, 5.3 with room
+// for all; 70 k of 20000 (700 k chunks) 5.2 and 5.7.
+constexpr int64_t kHubTasks = 1 << 19;
 constexpr int kPlanRows = 1024;           // rows (threads) of a planning workgroup
 constexpr int kQueueGrid = 2048;          // workgroups that take chunks
 
@@ -67,12 +73,13 @@ struct WArgs {
   const float* edge_data;
   float* data_out;
   unsigned long long* reserved;  // chunks of rows with several << 32 | rows of one chunk
-  // kHubTasks entries of the former, then S of the latter: those with a merge behind them are
+  // hub_tasks entries of the former, then S of the latter: those with a merge behind them are
   // taken first
   Task* tasks;
+  int64_t hub_tasks;
   int64_t* row_base;             // first entry of a row with several chunks
   unsigned int* done;            // [base]: chunks of the row that have left their candidates
-  unsigned long long* cand;      // kHubTasks * k composites
+  unsigned long long* cand;      // hub_tasks * k composites
 };
 
 __device__ __forceinline__ unsigned long long composite(float key, uint32_t pos) {
@@ -360,20 +367,20 @@ __global__ void __launch_bounds__(kPlanRows) weighted_plan_kernel(WArgs<IdT> a) 
   __syncthreads();
   at += s_base;
   if (single) {
-    const int64_t e = kHubTasks + (at & 0xFFFFFFFF);
+    const int64_t e = a.hub_tasks + (at & 0xFFFFFFFF);
     a.tasks[e] = Task{r, start, deg, out, e};
   }
   at >>= 32;
   // a row whose chunks do not all fit is left to its wave of the fill (its entries are void)
-  const Task t{at + chunks <= kHubTasks ? r : -1, start, deg, out, at};
+  const Task t{at + chunks <= a.hub_tasks ? r : -1, start, deg, out, at};
   if (chunks > 0) {
     a.row_base[r] = at;
-    if (at < kHubTasks) a.done[at] = 0u;
+    if (at < a.hub_tasks) a.done[at] = 0u;
   }
   // a few entries are written by the row's lane, many by its whole wave
   constexpr int64_t kFew = 4;
   if (chunks <= kFew)
-    for (int64_t e = at; e < at + chunks && e < kHubTasks; ++e) a.tasks[e] = t;
+    for (int64_t e = at; e < at + chunks && e < a.hub_tasks; ++e) a.tasks[e] = t;
   unsigned long long hubs = __ballot(chunks > kFew);
   while (hubs) {
     const int l = __ffsll(hubs) - 1;
@@ -381,7 +388,7 @@ __global__ void __launch_bounds__(kPlanRows) weighted_plan_kernel(WArgs<IdT> a) 
     const Task h{__shfl(t.row, l, kWave), __shfl(t.start, l, kWave), __shfl(t.deg, l, kWave),
                  __shfl(t.out, l, kWave), __shfl(t.base, l, kWave)};
     const int64_t n = __shfl(chunks, l, kWave);
-    for (int64_t e = h.base + lane; e < h.base + n && e < kHubTasks; e += kWave) a.tasks[e] = h;
+    for (int64_t e = h.base + lane; e < h.base + n && e < a.hub_tasks; e += kWave) a.tasks[e] = h;
   }
 }
 
@@ -457,10 +464,10 @@ __global__ void __launch_bounds__(kThreads) weighted_fill_kernel(WArgs<IdT> a) {
   __shared__ Shared s;
   const int64_t chunks = static_cast<int64_t>(*a.reserved >> 32);
   if (blockIdx.x < kQueueGrid) {
-    const int64_t hubs = chunks < kHubTasks ? chunks : kHubTasks;
+    const int64_t hubs = chunks < a.hub_tasks ? chunks : a.hub_tasks;
     const int64_t n = hubs + static_cast<int64_t>(*a.reserved & 0xFFFFFFFFu);
     for (int64_t i = blockIdx.x; i < n; i += kQueueGrid) {
-      const int64_t t = i < hubs ? i : kHubTasks + i - hubs;
+      const int64_t t = i < hubs ? i : a.hub_tasks + i - hubs;
       const Task e = a.tasks[t];
       if (e.row >= 0) run_task<IdT, WITH_COO>(a, e, t, s);
     }
@@ -491,8 +498,8 @@ __global__ void __launch_bounds__(kThreads) weighted_fill_kernel(WArgs<IdT> a) {
     wave_topk(edges, 0, nullptr, list, pos, a.k, emit_final);
     return;
   }
-  if (deg <= kChunk || chunks <= kHubTasks ||
-      a.row_base[r] + (deg + kChunk - 1) / kChunk <= kHubTasks)
+  if (deg <= kChunk || chunks <= a.hub_tasks ||
+      a.row_base[r] + (deg + kChunk - 1) / kChunk <= a.hub_tasks)
     return;
   // a row that found the queue full: 256 edges at a time, the k best so far beside them
   static_assert(kSmall + 2 * kMaxFanout <= kWaveList, "the quarter holds both and the best of them");
@@ -525,7 +532,7 @@ int weighted_impl(const int64_t* indptr, int64_t num_cols, const void* indices, 
                   const void* cols, int64_t S, int64_t k, uint64_t seed, const uint32_t* replay,
                   const int64_t* replay_ptr, const int64_t* sub_indptr, void* sub_indices,
                   int64_t* select_index, void* coo_col, const float* edge_data, float* data_out,
-                  void* workspace, size_t workspace_bytes, hipStream_t st) {
+                  int64_t queue_chunks, void* workspace, size_t workspace_bytes, hipStream_t st) {
   Carver ws(workspace, workspace_bytes);
   WArgs<IdT> a;
   a.indptr = indptr;
@@ -545,10 +552,11 @@ int weighted_impl(const int64_t* indptr, int64_t num_cols, const void* indices, 
   a.edge_data = edge_data;
   a.data_out = data_out;
   a.reserved = ws.take<unsigned long long>(1);
-  a.tasks = ws.take<Task>(static_cast<size_t>(kHubTasks + S));
+  a.hub_tasks = queue_chunks < kHubTasks ? queue_chunks : kHubTasks;
+  a.tasks = ws.take<Task>(static_cast<size_t>(a.hub_tasks + S));
   a.row_base = ws.take<int64_t>(static_cast<size_t>(S));
-  a.done = ws.take<unsigned int>(static_cast<size_t>(kHubTasks));
-  a.cand = ws.take<unsigned long long>(static_cast<size_t>(kHubTasks) * k);
+  a.done = ws.take<unsigned int>(static_cast<size_t>(a.hub_tasks));
+  a.cand = ws.take<unsigned long long>(static_cast<size_t>(a.hub_tasks) * k);
   if (!ws.ok) {
     set_error_text("gs_sample_weighted_fill: workspace needs %zu bytes, 256-byte aligned",
                    gs_sample_weighted_workspace_bytes(S, k));
@@ -832,13 +840,13 @@ size_t gs_sample_weighted_workspace_bytes(int64_t S, int64_t fanout) {
          padded(hubs * static_cast<size_t>(fanout) * 8);
 }
 
-int gs_sample_weighted_fill_data(const int64_t* indptr, int64_t num_cols, const void* indices,
-                                 const float* probs, const void* column_ids, int id_bytes,
-                                 int64_t S, int64_t fanout, uint64_t seed, const uint32_t* replay,
-                                 const int64_t* replay_ptr, const int64_t* sub_indptr,
-                                 void* sub_indices, int64_t* select_index, void* coo_col,
-                                 const float* edge_data, float* data_out, void* workspace,
-                                 size_t workspace_bytes, void* stream) {
+int gs_sample_weighted_fill_queue(const int64_t* indptr, int64_t num_cols, const void* indices,
+                                  const float* probs, const void* column_ids, int id_bytes,
+                                  int64_t S, int64_t fanout, uint64_t seed, const uint32_t* replay,
+                                  const int64_t* replay_ptr, const int64_t* sub_indptr,
+                                  void* sub_indices, int64_t* select_index, void* coo_col,
+                                  const float* edge_data, float* data_out, int64_t queue_chunks,
+                                  void* workspace, size_t workspace_bytes, void* stream) {
   GS_REQUIRE(indptr && sub_indptr && S >= 0 && fanout >= 0 && num_cols >= 0,
              "gs_sample_weighted_fill: null pointer or negative size");
   GS_REQUIRE(column_ids || S <= num_cols,
@@ -852,6 +860,7 @@ int gs_sample_weighted_fill_data(const int64_t* indptr, int64_t num_cols, const 
              "gs_sample_weighted_fill: null buffer");
   GS_REQUIRE((edge_data == nullptr) == (data_out == nullptr),
              "gs_sample_weighted_fill: edge_data and data_out go together");
+  GS_REQUIRE(queue_chunks >= 1, "gs_sample_weighted_fill: a queue without room");
   if (fanout > kMaxFanout) {
     set_error_text("gs_sample_weighted_fill: fanout %lld above the supported %d "
                    "(the reference stops at 32)",
@@ -861,8 +870,22 @@ int gs_sample_weighted_fill_data(const int64_t* indptr, int64_t num_cols, const 
   hipStream_t st = static_cast<hipStream_t>(stream);
   const auto impl = id_bytes == 8 ? weighted_impl<int64_t> : weighted_impl<int32_t>;
   return impl(indptr, num_cols, indices, probs, column_ids, S, fanout, seed, replay, replay_ptr,
-              sub_indptr, sub_indices, select_index, coo_col, edge_data, data_out, workspace,
-              workspace_bytes, st);
+              sub_indptr, sub_indices, select_index, coo_col, edge_data, data_out, queue_chunks,
+              workspace, workspace_bytes, st);
+}
+
+int gs_sample_weighted_fill_data(const int64_t* indptr, int64_t num_cols, const void* indices,
+                                 const float* probs, const void* column_ids, int id_bytes,
+                                 int64_t S, int64_t fanout, uint64_t seed, const uint32_t* replay,
+                                 const int64_t* replay_ptr, const int64_t* sub_indptr,
+                                 void* sub_indices, int64_t* select_index, void* coo_col,
+                                 const float* edge_data, float* data_out, void* workspace,
+                                 size_t workspace_bytes, void* stream) {
+  return gs_sample_weighted_fill_queue(indptr, num_cols, indices, probs, column_ids, id_bytes, S,
+                                       fanout, seed, replay, replay_ptr, sub_indptr, sub_indices,
+                                       select_index, coo_col, edge_data, data_out,
+                                       std::numeric_limits<int64_t>::max(), workspace, workspace_bytes,
+                                       stream);
 }
 
 int gs_sample_weighted_fill(const int64_t* indptr, int64_t num_cols, const void* indices,

@@ -347,6 +347,17 @@ int gs_sample_weighted_fill_data(const int64_t* indptr, int64_t num_cols, const 
                                  const float* edge_data, float* data_out, void* workspace,
                                  size_t workspace_bytes, void* stream);
 
+/* The same with a queue of at most queue_chunks (>= 1) chunks of 2048 edges for the rows that are
+ * longer than one; rows that do not fit are selected by a wave each, with the same result (no
+ * counterpart in the reference; the other entries take the room the workspace has). */
+int gs_sample_weighted_fill_queue(const int64_t* indptr, int64_t num_cols, const void* indices,
+                                  const float* probs, const void* column_ids, int id_bytes,
+                                  int64_t S, int64_t fanout, uint64_t seed, const uint32_t* replay,
+                                  const int64_t* replay_ptr, const int64_t* sub_indptr,
+                                  void* sub_indices, int64_t* select_index, void* coo_col,
+                                  const float* edge_data, float* data_out, int64_t queue_chunks,
+                                  void* workspace, size_t workspace_bytes, void* stream);
+
 /* Weighted neighbour sampling WITH replacement (inverse CDF): replaces
  * _CSRRowWiseSampleReplaceKernel (src/cuda/sampling_probs.cu:112-183).  A column with
  * deg > 0 gets fanout picks.  cdf = inclusive prefix of max(probs, 0) over the column's

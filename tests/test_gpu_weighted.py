@@ -114,6 +114,33 @@ def test_weighted_rows_around_the_planning_workgroup(dev, rows):
         assert np.array_equal(g, w)
 
 
+@pytest.mark.parametrize("k", [1, 16, 17, 64, 96])
+@pytest.mark.parametrize("queue", [1, 2, 3, 51, 52, 55, 1 << 19])
+def test_weighted_rows_that_find_the_queue_full(dev, queue, k):
+    # 49 + 2 + 2 + 2 + 5 chunks: rows that fit, one that lies across the end of the queue (its
+    # entries are void) and rows wholly beyond it, which a wave selects 256 edges at a time; several
+    # planning workgroups, whose reservations come in any order.  Few positive weights in one of them.
+    for rows in (12, 2100):
+        degs = np.full(rows, 3, dtype=np.int64)
+        long = np.linspace(0, rows - 1, 7).astype(np.int64)
+        degs[long] = [100000, 2049, 4096, 300, 2100, 2048, 10000]
+        indptr = np.concatenate([[0], np.cumsum(degs)])
+        rng = np.random.default_rng(queue)
+        indices = rng.integers(0, 1 << 20, int(indptr[-1])).astype(np.int64)
+        probs = (1.0 - rng.random(indices.size)).astype(np.float32)
+        at = int(indptr[long[2]])
+        probs[at:at + 4096] = 0.0
+        probs[at + 3000:at + 3005] = 0.5
+        nbytes = int(capi.lib().gs_sample_weighted_workspace_bytes(capi._i64(rows), capi._i64(k)))
+        ws = torch.full((nbytes,), 0xA5, dtype=torch.uint8, device=dev)
+        sp, si, sel, coo = capi.sample_weighted(to_dev(indptr, dev), to_dev(indices, dev), to_dev(probs, dev),
+                                                None, k, seed=21, with_coo=True, queue_chunks=queue, ws=ws)
+        want = O.sample_weighted(indptr, indices, probs, None, k, seed=21)
+        n = int(sp[-1].item())
+        for g, w in zip((sp, coo[:n], si[:n], sel[:n]), want):
+            assert np.array_equal(g.cpu().numpy(), w)
+
+
 @pytest.mark.parametrize("replace", [False, True])
 def test_weighted_samples_carry_their_edge_data(dev, replace):
     # copied, selected by a wave, by a workgroup and by a merge; data that are not the weights
