@@ -97,10 +97,11 @@ def test_weighted_degrees_around_the_selection_paths(dev, k):
             assert np.array_equal(g, w)
 
 
-@pytest.mark.parametrize("rows", [8191, 8192, 8193, 20000])
+@pytest.mark.parametrize("rows", [1023, 1024, 1025, 8192, 20000])
 def test_weighted_rows_around_the_planning_workgroup(dev, rows):
-    # 8192 rows are laid out by one workgroup, more by several that reserve side by side; rows of
-    # five chunks and more have their entries written by a whole wave
+    # 1024 rows are laid out by one workgroup, which sets the counter of what is reserved, more by
+    # several that add to it side by side; rows of five chunks and more have their entries written
+    # by a whole wave.  The workspace holds no zeros: whoever reads it reads what was left there.
     degs = np.random.default_rng(rows).integers(0, 12, rows).astype(np.int64)
     degs[::97] = 300
     degs[[0, 1, rows // 2, rows - 2, rows - 1]] = [8192, 8193, 30000, 2049, 257]
@@ -108,10 +109,14 @@ def test_weighted_rows_around_the_planning_workgroup(dev, rows):
     rng = np.random.default_rng(3)
     indices = rng.integers(0, 1 << 20, int(indptr[-1])).astype(np.int64)
     probs = (1.0 - rng.random(indices.size)).astype(np.float32)
-    got = _weighted_gpu(dev, indptr, indices, probs, None, 10, torch.int32, seed=7)
+    nbytes = int(capi.lib().gs_sample_weighted_workspace_bytes(capi._i64(rows), capi._i64(10)))
+    ws = torch.full((nbytes,), 0x5A, dtype=torch.uint8, device=dev)
+    sp, si, sel, coo = capi.sample_weighted(to_dev(indptr, dev), to_dev(indices, dev, torch.int32),
+                                            to_dev(probs, dev), None, 10, seed=7, with_coo=True, ws=ws)
     want = O.sample_weighted(indptr, indices, probs, None, 10, seed=7)
-    for g, w in zip(got, want):
-        assert np.array_equal(g, w)
+    n = int(sp[-1].item())
+    for g, w in zip((sp, coo[:n], si[:n], sel[:n]), want):
+        assert np.array_equal(g.cpu().numpy().astype(np.int64), w)
 
 
 @pytest.mark.parametrize("k", [1, 16, 17, 64, 96])
