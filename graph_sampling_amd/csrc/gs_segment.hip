@@ -858,8 +858,11 @@ __device__ __forceinline__ void keyed_clear(KeyedSums<EDGES>& t) {
   __syncthreads();
 }
 
+// (a negative key is no target: it is left out here, as -1 would add to a slot that stays empty for
+// the next key to take)
 template <int EDGES>
 __device__ __forceinline__ void keyed_add(KeyedSums<EDGES>& t, long long key, float v) {
+  if (key < 0) return;
   unsigned int h = static_cast<unsigned int>((static_cast<unsigned long long>(key) *
                                               0x9E3779B97F4A7C15ull) >> 40) & (t.kSlots - 1);
   while (true) {
@@ -872,7 +875,7 @@ __device__ __forceinline__ void keyed_add(KeyedSums<EDGES>& t, long long key, fl
   unsafeAtomicAdd(&t.sum[h], static_cast<double>(v));
 }
 
-// (a key outside [0, bound) is left out)
+// (a key of bound or more is left out)
 template <int EDGES>
 __device__ __forceinline__ void keyed_flush(KeyedSums<EDGES>& t, float* __restrict__ out,
                                             long long bound = 0x7FFFFFFFFFFFFFFFll) {

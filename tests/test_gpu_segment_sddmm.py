@@ -338,6 +338,32 @@ def test_keyed_sums_at_both_lengths_of_a_tile(dev, idt, edges):
                                    rtol=2e-5)
 
 
+@pytest.mark.parametrize("idt", ID_DTYPES)
+@pytest.mark.parametrize("edges,targets", [(600, 1693), (1 << 14, 1693), (1 << 17, 64)])
+def test_sums_by_key_leave_out_minus_one(dev, idt, edges, targets):
+    """The -1 of a step that found no neighbour marks an empty slot of the tables too: what it would
+    add must not wait there for the target whose place that is (1692's, in tables of 1024 slots
+    and of 4096), nor for another that is pushed there."""
+    rng = np.random.default_rng(edges)
+    to = rng.integers(0, targets, size=edges)
+    to[::4] = -1
+    to[1::4] = targets - 1
+    data = rng.random(edges, dtype=np.float32) + 0.25
+    ok = to >= 0
+    want = np.bincount(to[ok], weights=data[ok].astype(np.float64), minlength=targets)
+    for call in (capi.coo_sum, capi.coo_sum_binned):
+        out = torch.zeros(targets, dtype=torch.float32, device=dev)
+        call(to_dev(to, dev, idt), None, to_dev(data, dev), 1, out)
+        # (positive terms in any order, as above)
+        np.testing.assert_allclose(out.cpu().numpy(), want, rtol=2e-5)
+    divisor = torch.ones(1, dtype=torch.float32, device=dev)
+    quotients = torch.empty(edges, dtype=torch.float32, device=dev)
+    out = torch.zeros(targets, dtype=torch.float32, device=dev)
+    capi.e_div_u_sum(torch.zeros(edges, dtype=idt, device=dev), to_dev(to, dev, idt), to_dev(data, dev),
+                     divisor, quotients, out)
+    np.testing.assert_allclose(out.cpu().numpy(), want, rtol=2e-5)
+
+
 # ------------------------------------------------------------------ SDDMM
 def _sddmm_coo_gpu(dev, op, row, col, e_ids, lhs, rhs, lt, rt, idt=torch.int64):
     ls = lhs.shape if lhs.ndim > 1 else lhs.shape + (1,)
