@@ -514,6 +514,15 @@ def sample_one_keepdim(indptr, indices, column_ids, seed=0, replay=None):
     return sub_indptr, sub_indices, select_index
 
 
+def weighted_keys(draws, weights):
+    """(exact, rough) keys of the weighted sampler, gs_weighted_debug_keys (test hook)."""
+    _need(weights, torch.float32, "weights")
+    exact, rough = torch.empty_like(weights), torch.empty_like(weights)
+    _check(lib().gs_weighted_debug_keys(_ptr(draws), _ptr(weights), _i64(weights.numel()), _ptr(exact),
+                                        _ptr(rough), _stream(weights.device)), "gs_weighted_debug_keys")
+    return exact, rough
+
+
 def sample_weighted(indptr, indices, probs, column_ids, fanout, seed=0, replay=None,
                     replay_ptr=None, with_coo=False, queue_chunks=None, ws=None):
     """gs_sample_count(replace=0) + gs_sample_weighted_fill; same return shape as sample_uniform.

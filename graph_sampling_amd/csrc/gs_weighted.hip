@@ -90,7 +90,8 @@ __device__ __forceinline__ uint32_t composite_pos(unsigned long long c) {
 }
 
 // log2(u) / w as the hardware's one-instruction log2 and reciprocal give it.  Over all 2^24
-// values of u the first is within 3.1e-7 of log2_u24, the second within 9.2e-8 (measured, gfx950);
+// values of u the first is within 3.1e-7 of log2_u24, the second within 9.2e-8 (measured, gfx950;
+// test_rough_keys_stay_within_half_the_slack);
 // with the roundings of the product and of the exact quotient a rough key is within 5.3e-7 of the
 // exact one.  Weights whose keys could leave the normal range take the exact key.
 constexpr float kRoughSlack = 1.9073486e-6f;  // 2^-19: twice that, and some
@@ -513,6 +514,15 @@ __global__ void __launch_bounds__(kThreads) weighted_fill_kernel(WArgs<IdT> a) {
   for (int j = lane; j < a.k; j += kWave) emit_final(j, best[j]);
 }
 
+__global__ void __launch_bounds__(kThreads)
+weighted_keys_kernel(const uint32_t* __restrict__ draws, const float* __restrict__ weights, int64_t n,
+                     float* __restrict__ exact, float* __restrict__ rough) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  if (i >= n) return;
+  exact[i] = ares_key(draws[i], weights[i]);
+  rough[i] = rough_key(draws[i], weights[i]);
+}
+
 static __global__ void zero_kernel(unsigned long long* p) { *p = 0; }
 
 template <typename IdT, bool WITH_COO>
@@ -838,6 +848,16 @@ size_t gs_sample_weighted_workspace_bytes(int64_t S, int64_t fanout) {
   return padded(8) + padded((hubs + static_cast<size_t>(S)) * sizeof(Task)) +
          padded(static_cast<size_t>(S) * 8) + padded(hubs * 4) +
          padded(hubs * static_cast<size_t>(fanout) * 8);
+}
+
+int gs_weighted_debug_keys(const uint32_t* draws, const float* weights, int64_t n, float* exact,
+                           float* rough, void* stream) {
+  GS_REQUIRE(n >= 0 && n < (int64_t(1) << 31) && (n == 0 || (draws && weights && exact && rough)),
+             "gs_weighted_debug_keys: null pointer or size");
+  if (n == 0) return GS_OK;
+  hipLaunchKernelGGL(weighted_keys_kernel, dim3(static_cast<unsigned>(blocks_for(n, kThreads))),
+                     dim3(kThreads), 0, static_cast<hipStream_t>(stream), draws, weights, n, exact, rough);
+  return check_launch("weighted_debug_keys");
 }
 
 int gs_sample_weighted_fill_queue(const int64_t* indptr, int64_t num_cols, const void* indices,

@@ -358,6 +358,12 @@ int gs_sample_weighted_fill_queue(const int64_t* indptr, int64_t num_cols, const
                                   const float* edge_data, float* data_out, int64_t queue_chunks,
                                   void* workspace, size_t workspace_bytes, void* stream);
 
+/* The two keys by which the sampler ranks an edge of weight weights[i] and draw draws[i]: the exact
+ * one, and the rough one of the hardware's log2 and reciprocal that most edges are dropped by
+ * (test hook; no counterpart in the reference).  The rough key is within 2^-20 of the exact one. */
+int gs_weighted_debug_keys(const uint32_t* draws, const float* weights, int64_t n, float* exact,
+                           float* rough, void* stream);
+
 /* Weighted neighbour sampling WITH replacement (inverse CDF): replaces
  * _CSRRowWiseSampleReplaceKernel (src/cuda/sampling_probs.cu:112-183).  A column with
  * deg > 0 gets fanout picks.  cdf = inclusive prefix of max(probs, 0) over the column's

@@ -146,6 +146,30 @@ def test_weighted_rows_that_find_the_queue_full(dev, queue, k):
             assert np.array_equal(g.cpu().numpy(), w)
 
 
+@pytest.mark.parametrize("weight", [1.0, 0.7, 3.0, 1.0000001, 0.9999999, 123.456, 2.0 ** -100,
+                                    1.9999999 * 2.0 ** 99])
+def test_rough_keys_stay_within_half_the_slack(dev, weight):
+    """Edges are dropped by rough keys with a slack of 2^-19, which is right as long as a rough key is
+    within half of it of the exact one: over all 2^24 draws."""
+    draws = torch.arange(1 << 24, dtype=torch.int32, device=dev) << 8  # (the key's bits of a draw)
+    weights = torch.full(draws.shape, weight, dtype=torch.float32, device=dev)
+    exact, rough = (k.double() for k in capi.weighted_keys(draws, weights))
+    assert bool(torch.isfinite(exact).all()) and bool((exact <= 0).all())
+    assert bool(((rough - exact).abs() <= exact.abs() * 2.0 ** -20).all())
+    # (and the exact one is log2(u) / w to a few roundings)
+    u = ((draws.long() & 0xFFFFFFFF) // 256 + 1).double() / (1 << 24)
+    want = torch.log2(u) / float(np.float32(weight))
+    assert bool(((exact - want).abs() <= want.abs() * 4e-6 + 1e-37).all())
+
+
+def test_rough_keys_of_other_weights_are_exact(dev):
+    w = [0.0, -0.0, -1.0, float("nan"), float("inf"), 2.0 ** 100, 3e38, 1e-31, 2.0 ** -101, 1e-40, -float("inf")]
+    weights = torch.tensor(w, dtype=torch.float32, device=dev).repeat_interleave(5)
+    draws = torch.tensor([0, 255, 256, 1 << 31, 0xFFFFFFFF], dtype=torch.int64, device=dev).to(torch.int32)
+    exact, rough = capi.weighted_keys(draws.repeat(len(w)), weights)
+    assert torch.equal(exact.view(torch.int32), rough.view(torch.int32))
+
+
 @pytest.mark.parametrize("replace", [False, True])
 def test_weighted_samples_carry_their_edge_data(dev, replace):
     # copied, selected by a wave, by a workgroup and by a merge; data that are not the weights
