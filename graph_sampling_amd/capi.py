@@ -1209,8 +1209,9 @@ def dcsc2coo(indptr, nnz, ids):
     return col
 
 
-def coo2csc(key, value, num_keys, is_sorted):
-    """Returns (indptr, sorted value | value, perm | None)."""
+def coo2csc(key, value, num_keys, is_sorted, num_values=None):
+    """Returns (indptr, sorted value | value, perm | None).  num_values: what the values are below, where
+    they are not like the keys (gs_coo2csc_values)."""
     idb = _ids(key, "key")
     _ids(value, "value", like=key)
     dev = key.device
@@ -1219,7 +1220,10 @@ def coo2csc(key, value, num_keys, is_sorted):
     out_value = None if is_sorted else torch.empty(E, dtype=value.dtype, device=dev)
     perm = None if is_sorted else torch.empty(E, dtype=torch.int64, device=dev)
     ws = workspace(lib().gs_coo2csc_workspace_bytes(_i64(E), _i64(num_keys)), dev)
-    _check(lib().gs_coo2csc(_ptr(key), _ptr(value), idb, _i64(E), _i64(num_keys),
-                            int(bool(is_sorted)), _ptr(indptr), _ptr(out_value), _ptr(perm), _ptr(ws),
-                            ctypes.c_size_t(ws.numel()), _stream(dev)), "gs_coo2csc")
+    call, sizes = lib().gs_coo2csc, (_i64(num_keys),)
+    if num_values is not None:
+        call, sizes = lib().gs_coo2csc_values, (_i64(num_keys), _i64(num_values))
+    _check(call(_ptr(key), _ptr(value), idb, _i64(E), *sizes, int(bool(is_sorted)), _ptr(indptr),
+                _ptr(out_value), _ptr(perm), _ptr(ws), ctypes.c_size_t(ws.numel()), _stream(dev)),
+           "gs_coo2csc")
     return indptr, (value if is_sorted else out_value), perm

@@ -737,18 +737,18 @@ radix_pass_kernel(Src src, const ValT* __restrict__ val_in, int64_t E, int shift
   }
 }
 
-// The same with the value INSIDE the word, which then is all that a pass moves: 16 bits of what is
-// left of the key, then the value, then the position of the edge.  The word of a pass does not
+// The same with the value INSIDE the word, which then is all that a pass moves: what is left of the
+// key, then the value, then the position of the edge.  The word of a pass does not
 // hold the digit that the pass sorted by: the next pass knows it from where it finds the word
-// (the digits' totals) and puts it in the place of its own, so that a key of up to three digits
-// needs room for two.  A value that does not fit the bits that are left raises `wide`.  The next
-// pass's digits are written beside the words, for its histogram to read a byte an edge.
+// (the digits' totals) and puts it in the place of its own, so that a key of three digits
+// needs room for two, and one of two for one.  A value that does not fit the bits that are left raises
+// `wide`.  The next pass's digits are written beside the words, for its histogram to read a byte an edge.
 // 14 M edges, 22-bit keys (24 bits each for value and position): the passes 72 + 65 + 82 us with the
 // values beside the words, 67 + 59 + 81 so; the last two histograms 24 -> 8 each.
-constexpr int kRestAt = 48;     // of the key's digits in a word
 constexpr int kPackedPasses = 3;
+constexpr int rest_at(int passes) { return 64 - kRadixBits * (passes - 1); }  // of the key's digits in a word
 
-template <typename T, typename IdT, int PASS, bool LAST>
+template <typename T, typename IdT, int PASSES, int PASS>
 __global__ void __launch_bounds__(T::kThreadsPerTile, T::kWaves == 16 ? 8 : 4)  // (what LDS allows)
 packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
                    const unsigned long long* __restrict__ in, int64_t E, int value_bits,
@@ -757,7 +757,8 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
                    unsigned long long* __restrict__ out, unsigned char* __restrict__ next_digit,
                    SortOutputs<IdT> last) {
   constexpr int kThreadsHere = T::kThreadsPerTile, kItemsHere = T::kPerThread;
-  constexpr bool FIRST = PASS == 0;
+  constexpr bool FIRST = PASS == 0, LAST = PASS == PASSES - 1;
+  constexpr int kRestAt = rest_at(PASSES);
   constexpr int kCountBytes = T::kWaves * kRadix * 2;
   __shared__ unsigned long long s_word[T::kSize];
   __shared__ int64_t s_base[kRadix];  // memory position of a digit's run minus its place in the tile
@@ -1087,12 +1088,14 @@ int sort_passes(const IdT* key, const IdT* value, int64_t E, int passes, int idx
   return check_launch("coo2csc");
 }
 
-// Bits of a value in the words of a sort; 0: not packed (few tiles, one pass or more than three, or
-// hardly any bits left for the values, which are expected to be ids like the keys).
-inline int packed_value_bits(int64_t E, int64_t num_keys, int passes, int64_t tiles) {
-  const int bits = kRestAt - bits_for(E) < 32 ? kRestAt - bits_for(E) : 32;
-  return passes >= 2 && passes <= kPackedPasses && E < (int64_t(1) << 32) && tiles > kSelfScanTiles &&
-                 bits >= bits_for(num_keys) ? bits : 0;
+// Bits of a value in the words of a sort; 0: not packed (few tiles, one pass or more than three, or too
+// few bits for the values, which are expected below num_values).  A value that does not fit after all costs the
+// sort a gather of all of them by their positions: 14 M edges, 2.45 M keys, ids up to 100 M 526 us
+// where the values beside the words take 350.
+inline int packed_value_bits(int64_t E, int64_t num_values, int passes, int64_t tiles) {
+  if (passes < 2 || passes > kPackedPasses || E >= (int64_t(1) << 32) || tiles <= kSelfScanTiles) return 0;
+  const int left = rest_at(passes) - bits_for(E), bits = left < 32 ? left : 32;
+  return bits >= bits_for(num_values) ? bits : 0;
 }
 
 template <typename T, typename IdT>
@@ -1114,10 +1117,10 @@ int packed_passes(const IdT* key, const IdT* value, int64_t E, int passes, int v
     const int64_t* totals_before = p & 1 ? s.totals : s.totals_before;
     hipLaunchKernelGGL(digit_offsets_kernel, dim3(kRadix), dim3(kDigitThreads), 0, st, s.counts, blocks,
                        s.offsets, totals);
-    const auto kernel = p == 0 ? packed_pass_kernel<T, IdT, 0, false>
-                        : p == 2 ? packed_pass_kernel<T, IdT, 2, true>
-                        : last ? packed_pass_kernel<T, IdT, 1, true>
-                               : packed_pass_kernel<T, IdT, 1, false>;
+    const auto kernel = passes == 2 ? (last ? packed_pass_kernel<T, IdT, 2, 1> : packed_pass_kernel<T, IdT, 2, 0>)
+                        : p == 0 ? packed_pass_kernel<T, IdT, 3, 0>
+                        : last ? packed_pass_kernel<T, IdT, 3, 2>
+                               : packed_pass_kernel<T, IdT, 3, 1>;
     hipLaunchKernelGGL(kernel, grid, threads, 0, st, key, value, in, E, value_bits, blocks, s.offsets,
                        totals, totals_before, s.word[p & 1], digits, outs);
   }
@@ -1125,7 +1128,7 @@ int packed_passes(const IdT* key, const IdT* value, int64_t E, int passes, int v
 }
 
 template <typename IdT>
-int coo2csc_impl(const IdT* key, const IdT* value, int64_t E, int64_t num_keys, int sorted,
+int coo2csc_impl(const IdT* key, const IdT* value, int64_t E, int64_t num_keys, int64_t num_values, int sorted,
                  int64_t* indptr, IdT* out_value, int64_t* perm, void* workspace,
                  size_t workspace_bytes, hipStream_t st) {
   if (E == 0 && !indptr) return GS_OK;
@@ -1150,7 +1153,7 @@ int coo2csc_impl(const IdT* key, const IdT* value, int64_t E, int64_t num_keys, 
   }
   const bool large = E >= kLargeTileItems;
   const int value_bits =
-      packed_value_bits(E, num_keys, passes, blocks_for(E, large ? LargeTile::kSize : SmallTile::kSize));
+      packed_value_bits(E, num_values, passes, blocks_for(E, large ? LargeTile::kSize : SmallTile::kSize));
   const bool may_be_wide = sizeof(IdT) == 8 || value_bits > 0;
   const bool short_keys = passes * kRadixBits <= 32;
   const SortOutputs<IdT> outs{out_value, perm, indptr && short_keys ? s.keys : nullptr, idx_bits,
@@ -2019,10 +2022,10 @@ int gs_distinct_ends(const void* a, const void* b, int id_bytes, int64_t E, void
   return check_launch("distinct_ends");
 }
 
-int gs_coo2csc(const void* key, const void* value, int id_bytes, int64_t E, int64_t num_keys,
-               int sorted, int64_t* indptr, void* out_value, int64_t* perm, void* workspace,
-               size_t workspace_bytes, void* stream) {
-  GS_REQUIRE(E >= 0 && num_keys >= 0, "gs_coo2csc: negative size");
+int gs_coo2csc_values(const void* key, const void* value, int id_bytes, int64_t E, int64_t num_keys,
+                      int64_t num_values, int sorted, int64_t* indptr, void* out_value, int64_t* perm,
+                      void* workspace, size_t workspace_bytes, void* stream) {
+  GS_REQUIRE(E >= 0 && num_keys >= 0 && num_values >= 0, "gs_coo2csc: negative size");
   GS_REQUIRE(indptr || !sorted, "gs_coo2csc: sorted keys and no indptr leave nothing to do");
   GS_REQUIRE(E == 0 || key, "gs_coo2csc: key is null");
   GS_REQUIRE(sorted || E == 0 || (value && out_value && perm),
@@ -2031,13 +2034,20 @@ int gs_coo2csc(const void* key, const void* value, int id_bytes, int64_t E, int6
   hipStream_t st = static_cast<hipStream_t>(stream);
   return id_bytes == 8
              ? coo2csc_impl<int64_t>(static_cast<const int64_t*>(key),
-                                     static_cast<const int64_t*>(value), E, num_keys, sorted,
+                                     static_cast<const int64_t*>(value), E, num_keys, num_values, sorted,
                                      indptr, static_cast<int64_t*>(out_value), perm, workspace,
                                      workspace_bytes, st)
              : coo2csc_impl<int32_t>(static_cast<const int32_t*>(key),
-                                     static_cast<const int32_t*>(value), E, num_keys, sorted,
+                                     static_cast<const int32_t*>(value), E, num_keys, num_values, sorted,
                                      indptr, static_cast<int32_t*>(out_value), perm, workspace,
                                      workspace_bytes, st);
+}
+
+int gs_coo2csc(const void* key, const void* value, int id_bytes, int64_t E, int64_t num_keys,
+               int sorted, int64_t* indptr, void* out_value, int64_t* perm, void* workspace,
+               size_t workspace_bytes, void* stream) {
+  return gs_coo2csc_values(key, value, id_bytes, E, num_keys, num_keys, sorted, indptr, out_value, perm,
+                           workspace, workspace_bytes, stream);
 }
 
 int gs_indptr_split(const int64_t* indptr, const int64_t* offsets, int64_t num_batches,

@@ -99,13 +99,13 @@ torch::optional<torch::Tensor> Graph::GetData(std::string order) {
 void Graph::CSC2CSR() {
   Settle();
   CreateSparseFormat(_COO);
-  SetCSR(GraphCOO2CSC(coo_, num_rows_, false));
+  SetCSR(GraphCOO2CSC(coo_, num_rows_, false, num_cols_));
 }
 
 void Graph::CSR2CSC() {
   Settle();
   CreateSparseFormat(_COO);
-  SetCSC(GraphCOO2CSC(coo_, num_cols_, true));
+  SetCSC(GraphCOO2CSC(coo_, num_cols_, true, num_rows_));
 }
 
 void Graph::CSC2DCSR() {
@@ -113,7 +113,7 @@ void Graph::CSC2DCSR() {
   CreateSparseFormat(_COO);
   std::shared_ptr<CSR> csr;
   torch::Tensor val;
-  std::tie(csr, val) = GraphCOO2DCSC(coo_, num_rows_, false);
+  std::tie(csr, val) = GraphCOO2DCSC(coo_, num_rows_, false, num_cols_);
   val_row_ids_ = val;
   SetCSR(csr);
 }
@@ -123,7 +123,7 @@ void Graph::CSR2DCSC() {
   CreateSparseFormat(_COO);
   std::shared_ptr<CSC> csc;
   torch::Tensor val;
-  std::tie(csc, val) = GraphCOO2DCSC(coo_, num_cols_, true);
+  std::tie(csc, val) = GraphCOO2DCSC(coo_, num_cols_, true, num_rows_);
   val_col_ids_ = val;
   SetCSC(csc);
 }
@@ -160,7 +160,7 @@ void Graph::CreateSparseFormat(int64_t format) {
     if (spare_csc_)
       SetCSC(std::move(spare_csc_));
     else if (coo_)
-      SetCSC(GraphCOO2CSC(coo_, num_cols_, true));
+      SetCSC(GraphCOO2CSC(coo_, num_cols_, true, num_rows_));
     else
       CSR2CSC();
   } else if (format == _CSR) {
@@ -171,7 +171,7 @@ void Graph::CreateSparseFormat(int64_t format) {
     if (spare_csr_)
       SetCSR(std::move(spare_csr_));
     else if (coo_)
-      SetCSR(GraphCOO2CSC(coo_, num_rows_, false));
+      SetCSR(GraphCOO2CSC(coo_, num_rows_, false, num_cols_));
     else
       CSC2CSR();
   } else {
@@ -377,7 +377,7 @@ c10::intrusive_ptr<Graph> Graph::RowSliceOfCoo(const torch::Tensor& n_ids) {
   if (!distinct) return nullptr;
   torch::Tensor indptr, sorted_cols;
   torch::optional<torch::Tensor> perm;
-  std::tie(indptr, sorted_cols, perm) = hip::Coo2Csc(new_row, cols, n_ids.numel(), false);
+  std::tie(indptr, sorted_cols, perm) = hip::Coo2Csc(new_row, cols, n_ids.numel(), false, num_cols_);
   if (perm.has_value()) select_index = select_index.index({perm.value()});
   auto ret = Child(col_ids_, Pick(row_ids_, n_ids), num_cols_, n_ids.numel());
   ret->SetNumEdges(sorted_cols.numel());

@@ -137,13 +137,17 @@ std::shared_ptr<COO> GraphCSC2COO(std::shared_ptr<CSC> csc, bool CSC2COO) {
   return coo;
 }
 
-std::shared_ptr<CSC> GraphCOO2CSC(std::shared_ptr<COO> coo, int64_t num_items, bool COO2CSC) {
+std::shared_ptr<CSC> GraphCOO2CSC(std::shared_ptr<COO> coo, int64_t num_items, bool COO2CSC,
+                                  int64_t num_others) {
+  if (num_others <= 0) num_others = num_items;
   auto csc = std::make_shared<CSC>();
   torch::optional<torch::Tensor> perm;
   if (COO2CSC)
-    std::tie(csc->indptr, csc->indices, perm) = hip::Coo2Csc(coo->col, coo->row, num_items, coo->col_sorted);
+    std::tie(csc->indptr, csc->indices, perm) =
+        hip::Coo2Csc(coo->col, coo->row, num_items, coo->col_sorted, num_others);
   else
-    std::tie(csc->indptr, csc->indices, perm) = hip::Coo2Csc(coo->row, coo->col, num_items, coo->row_sorted);
+    std::tie(csc->indptr, csc->indices, perm) =
+        hip::Coo2Csc(coo->row, coo->col, num_items, coo->row_sorted, num_others);
   // edge ids follow the sort (reference src/graph_ops.cc:46-54)
   if (coo->e_ids.has_value())
     csc->e_ids = perm.has_value() ? coo->e_ids.value().index({perm.value()}) : coo->e_ids.value();
@@ -154,8 +158,9 @@ std::shared_ptr<CSC> GraphCOO2CSC(std::shared_ptr<COO> coo, int64_t num_items, b
 
 // sort by the compressed side, then keep only the offsets of the non-empty columns
 std::pair<std::shared_ptr<CSC>, torch::Tensor> GraphCOO2DCSC(std::shared_ptr<COO> coo,
-                                                             int64_t num_items, bool COO2DCSC) {
-  std::shared_ptr<CSC> full = GraphCOO2CSC(coo, num_items, COO2DCSC);
+                                                             int64_t num_items, bool COO2DCSC,
+                                                             int64_t num_others) {
+  std::shared_ptr<CSC> full = GraphCOO2CSC(coo, num_items, COO2DCSC, num_others);
   torch::Tensor val_ids;
   std::tie(full->indptr, val_ids) = hip::CscCompress(full->indptr, full->indices);
   return {full, val_ids};

@@ -73,11 +73,14 @@ void COOGraphDiv(std::shared_ptr<COO> coo, torch::Tensor data, torch::Tensor div
 
 std::shared_ptr<COO> GraphCSC2COO(std::shared_ptr<CSC> csc, bool CSC2COO);
 
-std::shared_ptr<CSC> GraphCOO2CSC(std::shared_ptr<COO> coo, int64_t num_items, bool COO2CSC);
+// num_items: of the compressed side, num_others: of the other (0: not known, expected to be as many)
+std::shared_ptr<CSC> GraphCOO2CSC(std::shared_ptr<COO> coo, int64_t num_items, bool COO2CSC,
+                                  int64_t num_others = 0);
 
 // doubly-compressed counterparts (reference src/graph_ops.cc:62-104,156-171)
 std::pair<std::shared_ptr<CSC>, torch::Tensor> GraphCOO2DCSC(std::shared_ptr<COO> coo,
-                                                             int64_t num_items, bool COO2DCSC);
+                                                             int64_t num_items, bool COO2DCSC,
+                                                             int64_t num_others = 0);
 std::shared_ptr<COO> GraphDCSC2COO(std::shared_ptr<CSC> csc, torch::Tensor ids, bool DCSC2COO);
 std::pair<std::shared_ptr<_TMP>, torch::Tensor> DCSCColSlicing(std::shared_ptr<CSC> csc,
                                                                torch::Tensor nid_map,

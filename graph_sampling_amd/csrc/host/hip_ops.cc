@@ -1497,7 +1497,7 @@ torch::Tensor Csc2CooCols(const torch::Tensor& indptr, int64_t nnz, const torch:
 }
 
 std::tuple<torch::Tensor, torch::Tensor, torch::optional<torch::Tensor>> Coo2Csc(
-    const torch::Tensor& key, const torch::Tensor& value, int64_t num_keys, bool sorted) {
+    const torch::Tensor& key, const torch::Tensor& value, int64_t num_keys, bool sorted, int64_t num_values) {
   const int idb = IdBytes(key, "coo key");
   TORCH_CHECK(IdBytes(value, "coo value") == idb, "coo key and value differ in dtype");
   const int64_t E = key.numel();
@@ -1511,9 +1511,9 @@ std::tuple<torch::Tensor, torch::Tensor, torch::optional<torch::Tensor>> Coo2Csc
   auto out_value = torch::empty({E}, value.options());
   auto perm = torch::empty({E}, I64(key));
   auto ws = Scratch(gs_coo2csc_workspace_bytes(E, num_keys), key);
-  Check(gs_coo2csc(key.data_ptr(), value.data_ptr(), idb, E, num_keys, 0,
-                   indptr.data_ptr<int64_t>(), out_value.data_ptr(), perm.data_ptr<int64_t>(),
-                   ws.data_ptr(), ws.numel(), Stream(key)),
+  Check(gs_coo2csc_values(key.data_ptr(), value.data_ptr(), idb, E, num_keys, num_values, 0,
+                          indptr.data_ptr<int64_t>(), out_value.data_ptr(), perm.data_ptr<int64_t>(),
+                          ws.data_ptr(), ws.numel(), Stream(key)),
         "gs_coo2csc");
   return {indptr, out_value, perm};
 }

@@ -288,9 +288,10 @@ std::tuple<torch::Tensor, torch::Tensor> CscCompress(const torch::Tensor& indptr
 
 // col[e] = column owning edge e, in the dtype of `ids_like`
 torch::Tensor Csc2CooCols(const torch::Tensor& indptr, int64_t nnz, const torch::Tensor& ids_like);
-// {indptr, values in key order, sort permutation (nullopt when already sorted)}
+// {indptr, values in key order, sort permutation (nullopt when already sorted)}; the values are
+// expected to be below num_values (larger ones only make it slower)
 std::tuple<torch::Tensor, torch::Tensor, torch::optional<torch::Tensor>> Coo2Csc(
-    const torch::Tensor& key, const torch::Tensor& value, int64_t num_keys, bool sorted);
+    const torch::Tensor& key, const torch::Tensor& value, int64_t num_keys, bool sorted, int64_t num_values);
 
 // the larger number of distinct ids among the two ends of an edge list; negative when the
 // library's count does not apply (no device tensors, no edges, an id far beyond their number)

@@ -898,6 +898,13 @@ int gs_coo2csc(const void* key, const void* value, int id_bytes, int64_t E, int6
                int sorted, int64_t* indptr, void* out_value, int64_t* perm, void* workspace,
                size_t workspace_bytes, void* stream);
 
+/* The same for a caller that knows the values to be below num_values (gs_coo2csc expects values like the
+ * keys): the sort chooses by it what it moves.  Values beyond it are sorted as well, only slower (no
+ * counterpart in the reference). */
+int gs_coo2csc_values(const void* key, const void* value, int id_bytes, int64_t E, int64_t num_keys,
+                      int64_t num_values, int sorted, int64_t* indptr, void* out_value, int64_t* perm,
+                      void* workspace, size_t workspace_bytes, void* stream);
+
 /* Offsets of a batched CSC cut into its batches: replaces
  * impl::SplitIndptrByOffsetCUDA / SplitIndptrBySizeCUDA (src/cuda/batch_split.cu:101,96).
  * offsets: device int64[num_batches+1], column ranges of the batches; out (length

@@ -93,7 +93,8 @@ def test_sort_with_large_tiles(dev, num_keys, extra, idt):
 @pytest.mark.parametrize("num_keys,skew", [(257, 1), (65536, 3), (65537, 3), (1 << 22, 12), (1 << 24, 1)])
 def test_sort_with_the_values_in_its_words(dev, num_keys, skew, E, idt):
     """From 65 tiles on a sort of two or three digits carries the values in its 64-bit words, beside
-    sixteen bits of the key and the edge's position: the largest value that fits, and one more."""
+    a digit of the key or two and the edge's position: the largest value that fits beside two, and one
+    more."""
     gen = torch.Generator(device=dev)
     gen.manual_seed(num_keys + E)
     key = (torch.rand(E, generator=gen, device=dev, dtype=torch.float64) ** skew * num_keys).to(idt)
@@ -106,6 +107,26 @@ def test_sort_with_the_values_in_its_words(dev, num_keys, skew, E, idt):
         ip, val, perm = capi.coo2csc(key, value, num_keys, False)
         assert torch.equal(perm, want.indices) and torch.equal(val, value[want.indices])
         assert int(ip[0]) == 0 and torch.equal(ip[1:], ends)
+
+
+@pytest.mark.parametrize("idt", ID_DTYPES)
+@pytest.mark.parametrize("num_keys", [60_000, 65_537])
+def test_sort_of_values_unlike_the_keys(dev, num_keys, idt):
+    """Values below a bound that the caller knows, with two digits of the key (which leave them all 32
+    bits) and three: in the words as long as the bound fits there, else beside them; the same
+    result when the bound is not kept, up to beyond 32 bits."""
+    E = 3_000_000  # (22 bits of a position: 34 and 26 are left)
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(num_keys)
+    key = torch.randint(0, num_keys, (E,), generator=gen, device=dev).to(idt)
+    want = torch.sort(key, stable=True).indices
+    for top in ([1 << 26, (1 << 26) + 1, (1 << 31) - 1] + ([1 << 32, (1 << 32) + 1, 1 << 40] if idt == torch.int64 else [])):
+        value = torch.randint(0, top, (E,), generator=gen, device=dev, dtype=torch.int64)
+        value[E // 2] = top - 1
+        value = value.to(idt)
+        for bound in (top, 0, num_keys):
+            _, val, perm = capi.coo2csc(key, value, num_keys, False, num_values=bound)
+            assert torch.equal(perm, want) and torch.equal(val, value[want])
 
 
 @pytest.mark.parametrize("idt", ID_DTYPES)
