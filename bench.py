@@ -908,7 +908,7 @@ def super_batch_leg(torch, graph, timer, fresh_seeds, b, weighted, workload):
                                   "over its wall time; gpu_busy_frac = the sites' kernel time "
                                   "over the same"},
         "what": "fused sampling over the concatenated seeds + the batches' edge cuts + one relabel "
-                "per minibatch in one pass (through hash classes and LDS tables from 2^19 items "
+                "per minibatch in one pass (through hash classes and LDS tables from 2^17 items "
                 "on) + per-minibatch views, 64 minibatches of 1024 seeds at once"}
     return out
 

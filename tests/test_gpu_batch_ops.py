@@ -394,7 +394,7 @@ def _oracle_super_batch(indptr, indices, seed_sets, fanouts, replace, first_seed
 def test_sample_layers_batched_equals_the_oracle_flow(dev, idt, with_data, sizes, fanouts, replace):
     """_CAPI_SampleLayersBatched (the super-batch flow inside the C++ layer: fused sampling over
     the concatenated seeds, the batches' edge cuts, one relabel per minibatch in one pass -- through
-    the bins from 2^19 items on --, the per-minibatch views) against the oracle doing the same."""
+    the bins from 2^17 items on --, the per-minibatch views) against the oracle doing the same."""
     import graph_sampling_amd as gs
     n = 1 << 15
     indptr, indices = rmat_csc_np(n, 1 << 20, seed=41)
@@ -408,7 +408,7 @@ def test_sample_layers_batched_equals_the_oracle_flow(dev, idt, with_data, sizes
     ops = torch.ops.gs_ops
     # first with every layer's relabel queued behind its sampler (sized by the sampler's capacity,
     # one host wait a layer), then with the wait for the edge count too (exact sizes): the same
-    # minibatches either way, and from 2^19 items on the first way is the one taken
+    # minibatches either way, and from 2^17 items on the first way is the one taken
     for first, no_wait in ((700, True), (710, False)):
         through, repeated = ops._CAPI_BatchedNoWaitCounts()
         ops._CAPI_SetBatchedNoWait(no_wait)
@@ -423,7 +423,7 @@ def test_sample_layers_batched_equals_the_oracle_flow(dev, idt, with_data, sizes
         if not no_wait:
             assert now[0] == through
         elif idt == torch.int32 and len(sizes) == 64:
-            assert now == [through + len(fanouts), repeated]  # 2^19 items and more: all queued
+            assert now == [through + len(fanouts), repeated]  # 2^17 items and more: all queued
         want = _oracle_super_batch(indptr, indices, seed_sets, fanouts, replace, first, data)
         assert len(got) == len(want)
         for b, (g_b, w_b) in enumerate(zip(got, want)):

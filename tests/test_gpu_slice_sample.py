@@ -54,6 +54,28 @@ def test_slice_rmat(dev, idt, with_coo, S):
     _cmp(got, O.slice_columns(indptr, indices, cols, with_coo))
 
 
+@pytest.mark.parametrize("idt", ID_DTYPES)
+@pytest.mark.parametrize("S", [2047, 2048, 2049, 2560, 2561, 15872, 15873])
+def test_offsets_around_the_lengths_of_the_scans_tiles(dev, idt, S):
+    """One tile up to 2048 columns, tiles of 512 up to 15872, of 2048 beyond, for slices and samples;
+    the total that the scan posts to the host is what the sliced graph's arrays are cut to."""
+    import graph_sampling_amd as gs
+    gs.load_library()
+    indptr, indices = rmat_csc_np(1 << 13, 1 << 17, seed=3)
+    cols = np.random.default_rng(S).integers(0, indptr.size - 1, size=S).astype(np.int64)
+    cols[S // 2] = int(np.argmax(np.diff(indptr)))
+    deg = np.diff(indptr)[cols]
+    t_indptr, t_indices, t_cols = to_dev(indptr, dev), to_dev(indices, dev, idt), to_dev(cols, dev, idt)
+    want = np.concatenate([[0], np.cumsum(deg)])
+    assert np.array_equal(capi.slice_count(t_indptr, t_cols).cpu().numpy(), want)
+    picked = capi.sample_uniform(t_indptr, t_indices, t_cols, 5, False, seed=1)[0]
+    assert np.array_equal(picked.cpu().numpy(), np.concatenate([[0], np.cumsum(np.minimum(deg, 5))]))
+    g = gs.Graph(False)
+    g._CAPI_LoadCSC(t_indptr, t_indices)
+    sub = g._CAPI_Slicing(t_cols, 0, gs._CSC, gs._CSC, False)
+    assert sub._CAPI_GetNumEdges() == want[-1]
+
+
 def test_slice_many_empty_columns(dev):
     # more rows than the LDS stage holds inside one 2048-edge tile
     deg = np.zeros(6000, dtype=np.int64)

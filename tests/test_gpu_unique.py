@@ -175,8 +175,8 @@ def test_batch_csr_relabel_through_bins_small(dev, idt, narrow, B, max_seeds, ma
 @pytest.mark.parametrize("idt,narrow", [(torch.int32, False), (torch.int64, True)])
 @pytest.mark.parametrize("shape", ["even", "one_large", "hubs", "single", "all_same"])
 def test_batch_csr_relabel_through_bins_at_size(dev, idt, narrow, shape):
-    """From 2^19 items on the library takes the bins by itself: batches of equal size, one batch
-    that holds nearly everything (thousands of classes) beside tiny and empty ones, ids that
+    """Half a million items and more, which the library takes through bins by itself: batches of equal
+    size, one batch that holds nearly everything (thousands of classes) beside tiny and empty ones, ids that
     repeat tens of thousands of times, one batch only, one id only; the last batches empty."""
     rng = np.random.default_rng(len(shape))
     n_nodes = 1 << 21
@@ -207,6 +207,23 @@ def test_batch_csr_relabel_through_bins_at_size(dev, idt, narrow, shape):
     assert seeds.size + ids.size >= 1 << 19
     _check_batch_relabel(dev, idt, seeds, np.array(sp, dtype=np.int64), ids,
                          np.array(ip, dtype=np.int64), narrow, None)
+
+
+@pytest.mark.parametrize("idt,narrow", [(torch.int32, False), (torch.int64, True)])
+@pytest.mark.parametrize("B,items", [(3, (1 << 17) - 1), (3, 1 << 17), (3, (1 << 17) + 1),
+                                     (1, 1 << 20), (1, (1 << 20) + 1)])
+def test_batch_csr_relabel_at_the_lines_of_its_forms(dev, idt, narrow, B, items):
+    """Hash regions below 2^17 items, bins from there on; by runs up to 2^20 items a batch on average,
+    counted and scattered beyond."""
+    rng = np.random.default_rng(items)
+    ends = np.concatenate([[0], np.sort(rng.integers(0, items + 1, B - 1)), [items]])
+    sizes = np.diff(ends)
+    sp = np.concatenate([[0], np.cumsum(sizes // 5)]).astype(np.int64)
+    ip = np.concatenate([[0], np.cumsum(sizes - sizes // 5)]).astype(np.int64)
+    seeds = rng.integers(0, 1 << 18, sp[-1]).astype(np.int64)
+    ids = (rng.random(ip[-1]) ** 2 * (1 << 18)).astype(np.int64)
+    assert seeds.size + ids.size == items
+    _check_batch_relabel(dev, idt, seeds, sp, ids, ip, narrow, None)
 
 
 @pytest.mark.parametrize("idt,narrow", [(torch.int32, False), (torch.int64, True)])
