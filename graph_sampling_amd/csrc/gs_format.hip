@@ -1607,8 +1607,8 @@ constexpr int kSumTile = kBinThreads * kSumTileItems;
 constexpr int kMaxBins = 1024;
 constexpr int kBinMaxShift = 13;          // 2^13 sums = 64 KB of LDS
 constexpr int kBinMinBits = 8;            // 256 bins at least, where there are as many targets
-// The additions to one LDS word queue up, so a bin of more than 5/4 of the average (a hub's) is
-// shared by several workgroups, which then add their sums to memory with atomics.  Shares by the average
+// The additions to one LDS word queue up, so a bin of more than 5/4 of the average (a hub's) and of
+// two edges a sum is shared by several workgroups, which then add their sums to memory with atomics.  Shares by the average
 // alone left a bin of twice as much to one workgroup, and, of three targets, each: 30 M edges,
 // uniform / skewed, 3 targets 12900 / 7630 us, now 279 / 330; 40: 1090 / 1192, now 282 / 294; 256: 277 / 542,
 // now 277 / 455; 30 k: 216 / 274, now 215 / 259.
@@ -1873,10 +1873,14 @@ int bin_sum_impl(const IdT* target, const float* data, int64_t E, int powk, int6
   hipLaunchKernelGGL(sum_tiles_kernel<IdT>, dim3(static_cast<unsigned>(tiles)), dim3(kBinThreads), 0, st,
                      target, data, E, num_targets, powk, order, s);
   hipLaunchKernelGGL(sum_totals_kernel, dim3(order.bins), dim3(kThreads), 0, st, s, tiles, order.bins);
-  // (few targets make few bins: the average is that of 256 then, so that every bin is shared)
-  const int64_t average = std::max(E / std::max(order.bins, 1 << kBinMinBits), kBinPartItems);
+  // (few targets make few bins: the average is that of 256 then, so that every bin is shared.  A share
+  // clears and writes all sums of its bin, so bins of many sums are shared for many edges only, in
+  // larger shares: 2 M R-MAT edges into 2.45 M sums, call, 52 us by edges alone, 49 so; a tenth of them
+  // on one target 45 and 41)
+  const int64_t width = int64_t(1) << order.bin_shift;
+  const int64_t average = std::max({E / std::max(order.bins, 1 << kBinMinBits), kBinPartItems, width});
   const int64_t part_items = std::min(average, kBinPartMost);
-  const int64_t alone = average + average / 4;
+  const int64_t alone = std::max(average + average / 4, 2 * width);
   const int64_t shares = E / part_items + order.bins;  // at most: sum of ceil(n / part_items) over the bins
   hipLaunchKernelGGL(bin_sum_kernel, dim3(static_cast<unsigned>(shares)), dim3(kBinThreads),
                      sizeof(double) << order.bin_shift, st, s, tiles, alone, part_items, order,
