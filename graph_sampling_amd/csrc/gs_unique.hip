@@ -858,7 +858,8 @@ __global__ void __launch_bounds__(kThreads) rank_linked_kernel(RankArgs<IdT> a) 
     if (threadIdx.x == 0) s_prefix = before;
   }
   GS_STAMP(4);  // look-back done
-  // every wave's distance stores have completed before the tile closes
+  // (the distances' stores may still be under way when the tile closes: every word says by its epoch
+  // whether it is this launch's, and who reads it earlier asks again, back_wait)
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __syncthreads();
   const int64_t tile_excl = s_prefix;
