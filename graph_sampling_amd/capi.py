@@ -38,7 +38,7 @@ def lib():
                      "gs_segment_workspace_bytes", "gs_layer_workspace_bytes",
                      "gs_layer_sample_state_bytes", "gs_layer_relabel_state_bytes",
                      "gs_coo_sum_workspace_bytes", "gs_coo_pick_rows_workspace_bytes",
-                     "gs_coo_block_values_workspace_bytes"):
+                     "gs_coo_block_values_workspace_bytes", "gs_random_walk_workspace_bytes"):
             if hasattr(_lib, name):
                 getattr(_lib, name).restype = ctypes.c_size_t
         _lib.gs_sorted_union_max.restype = ctypes.c_int64
@@ -975,15 +975,23 @@ def coo_block_values(kept_key, kept_pos, max_nodes, row, data, divisor, num_cols
 
 
 # ------------------------------------------------------------------ walks ----
-def random_walk(indptr, indices, seeds, length, seed=0, replay=None):
+def random_walk(indptr, indices, seeds, length, seed=0, replay=None, packed=None):
+    """packed: whether a packed table of the offsets is made first (None: where it pays)."""
     _need(indptr, torch.int64, "indptr")
     idb = _ids(indices, "indices")
     _ids(seeds, "seeds", like=indices)
     dev = indptr.device
     n = seeds.numel()
     trace = torch.empty((int(length) + 1) * n, dtype=indices.dtype, device=dev)
-    _check(lib().gs_random_walk(_ptr(indptr), _i64(indptr.numel() - 1), _ptr(indices), idb, _ptr(seeds), _i64(n), _i64(length),
-                                _u64(seed), _ptr(replay), _ptr(trace), _stream(dev)),
+    nodes = indptr.numel() - 1
+    size = lib().gs_random_walk_workspace_bytes(_i64(nodes), _i64(indices.numel()), _i64(n),
+                                                _i64(length))
+    if packed is not None:
+        size = (nodes // 6 + 1) * 16 + 256 if packed else 0
+    ws = torch.empty(size, dtype=torch.uint8, device=dev)
+    _check(lib().gs_random_walk_workspace(_ptr(indptr), _i64(nodes), _ptr(indices), idb, _ptr(seeds), _i64(n),
+                                          _i64(length), _u64(seed), _ptr(replay), _ptr(trace), _ptr(ws),
+                                          ctypes.c_size_t(size), _stream(dev)),
            "gs_random_walk")
     return trace
 

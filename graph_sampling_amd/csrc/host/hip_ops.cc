@@ -1154,8 +1154,13 @@ torch::Tensor RandomWalk(const torch::Tensor& seeds, int64_t length, const torch
   TORCH_CHECK(length >= 0, "walk_length must be non-negative");
   const int64_t n = seeds.numel();
   auto trace = torch::empty({n * (length + 1)}, seeds.options());
-  Check(gs_random_walk(indptr.data_ptr<int64_t>(), indptr.numel() - 1, indices.data_ptr(), idb, seeds.data_ptr(), n,
-                       length, NextSeed(), nullptr, trace.data_ptr(), Stream(seeds)),
+  const int64_t nodes = indptr.numel() - 1;
+  const size_t bytes = gs_random_walk_workspace_bytes(nodes, indices.numel(), n, length);
+  torch::Tensor ws;
+  if (bytes) ws = Scratch(bytes, indptr);
+  Check(gs_random_walk_workspace(indptr.data_ptr<int64_t>(), nodes, indices.data_ptr(), idb, seeds.data_ptr(),
+                                 n, length, NextSeed(), nullptr, trace.data_ptr(),
+                                 bytes ? ws.data_ptr() : nullptr, bytes, Stream(seeds)),
         "gs_random_walk");
   return trace;
 }

@@ -642,6 +642,15 @@ int gs_random_walk(const int64_t* indptr, int64_t num_nodes, const void* indices
                    const void* seeds, int64_t n, int64_t length, uint64_t seed, const uint32_t* replay,
                    void* trace, void* stream);
 
+/* The same with scratch memory: long walks over graphs whose offsets are larger than the L2s pack
+ * them first, six nodes to 16 bytes.  workspace_bytes 0: the offsets are read as they are, which is
+ * what gs_random_walk_workspace_bytes says where a table does not pay. */
+size_t gs_random_walk_workspace_bytes(int64_t num_nodes, int64_t nnz, int64_t n, int64_t length);
+int gs_random_walk_workspace(const int64_t* indptr, int64_t num_nodes, const void* indices, int id_bytes,
+                             const void* seeds, int64_t n, int64_t length, uint64_t seed,
+                             const uint32_t* replay, void* trace, void* workspace,
+                             size_t workspace_bytes, void* stream);
+
 /* all_indptr / all_indices: device arrays of device pointers, one per relation
  * (src/hetero_graph.cc:33-50); all_num_nodes: device int64 array, the number of
  * columns of each relation; metapath: device int64[length] relation ids. */

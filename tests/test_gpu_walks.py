@@ -182,3 +182,37 @@ def test_long_metapath_work_over_streams(dev, walkers, relations):
                              to_dev(seeds, dev, torch.int32), seed=6)
     want = O.metapath_walk(ptrs, [i.astype(np.int64) for i in indices + [small_ix]], path, seeds, seed=6)
     assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
+
+
+@pytest.mark.parametrize("idt", [torch.int32, torch.int64])
+@pytest.mark.parametrize("nodes,hub", [(1, 3), (5, 65535), (6, 65535), (7, 65536), (601, 65530), (4096, 70000)])
+def test_random_walk_with_packed_offsets(dev, idt, nodes, hub):
+    """Records of six nodes: the last one part empty, ends up to 16 bits behind the start and beyond."""
+    rng = np.random.default_rng(nodes)
+    degree = rng.integers(0, 9, nodes)
+    degree[min(nodes - 1, 3)] = hub
+    indptr = np.concatenate([[0], np.cumsum(degree)]).astype(np.int64)
+    indices = rng.integers(0, nodes, indptr[-1])
+    seeds = np.concatenate([rng.integers(0, nodes, 700), [-1, nodes, nodes + 5]])
+    got = capi.random_walk(to_dev(indptr, dev), to_dev(indices, dev, idt), to_dev(seeds, dev, idt), 13, seed=5,
+                           packed=True)
+    want = O.random_walk(indptr, indices, seeds, 13, seed=5)
+    assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
+
+
+@pytest.mark.parametrize("less", [0, 1])
+def test_random_walk_at_the_line_of_packed_offsets(dev, less):
+    """2^18 walkers over 2^18 nodes for ten steps make a table, over one node less they make none."""
+    nodes, n, length = (1 << 18) - less, 1 << 18, 10
+    size = capi.lib().gs_random_walk_workspace_bytes
+    import ctypes
+    assert (size(*(ctypes.c_int64(v) for v in (nodes, 3 * nodes, n, length))) > 0) == (less == 0)
+    rng = np.random.default_rng(less)
+    degree = rng.integers(1, 6, nodes)
+    indptr = np.concatenate([[0], np.cumsum(degree)]).astype(np.int64)
+    indices = rng.integers(0, nodes, indptr[-1])
+    seeds = rng.integers(0, nodes, n)
+    got = capi.random_walk(to_dev(indptr, dev), to_dev(indices, dev, torch.int32),
+                           to_dev(seeds, dev, torch.int32), length, seed=9)
+    want = O.random_walk(indptr, indices, seeds, length, seed=9)
+    assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
