@@ -30,7 +30,10 @@
 // the crossing segments 95; each tile's chain of LDS steps hides behind the other tiles of its
 // CU).  A lane per short column, a scan per 1024-edge chunk for the others and a divide pass
 // over all edges, each reading its edges for itself, took 214 and 380.  Tiles of 8192 edges:
-// 156 and 324, against 144 and 308 as the tiles of 4096 were then.
+// 156 and 324, against 144 and 308 as the tiles of 4096 were then.  With streamed accesses
+// (kStreamEdges) the sum's tiles took 118 where they took 129, the normalise's 187 / 202 and its crossing
+// segments 90 / 99.  Workgroups that stay for two or four tiles, the next one's data on their way
+// while one is added up: 64 registers are too few for that, and at 96 both calls took 449 us against 357.
 #include <limits>
 #include "gs_common.hpp"
 
@@ -143,10 +146,31 @@ using F4 = float __attribute__((ext_vector_type(4)));
 
 // Source: where a tile's data come from.
 enum Source {
-  kPlain,   // data[edge], 16-byte aligned
-  kLoose,   // data[edge]
-  kMapped   // data[emap[edge]]
+  kPlain,     // data[edge], 16-byte aligned
+  kStreamed,  // the same, of at least kStreamEdges edges
+  kLoose,     // data[edge]
+  kMapped     // data[emap[edge]]
 };
+
+// From here on data and results (8 bytes an edge) are more than the 256 MB that the memory-side
+// cache holds, and reads and writes past it that say so are the faster ones: a bare read of 496 MB 6.5 TB/s
+// against 5.9, sum and normalise of 124 M edges 390 -> 357 us, of 60 M 245 -> 229, of 40 M 150 -> 142.
+// Shorter arrays gain less or nothing (16 M edges 118 -> 114), and what reads a result soon
+// after finds it in the cache no more (normalise, then the sum of its result: 16 M edges 84 -> 85.5,
+// 32 M the same, 60 M 218 -> 212).
+constexpr int64_t kStreamEdges = int64_t(1) << 25;
+
+template <Source SOURCE>
+__device__ __forceinline__ F4 read_four(const float* at) {
+  const F4* p = reinterpret_cast<const F4*>(at);
+  return SOURCE == kStreamed ? __builtin_nontemporal_load(p) : *p;
+}
+template <Source SOURCE>
+__device__ __forceinline__ void write_four(float* at, F4 v) {
+  F4* p = reinterpret_cast<F4*>(at);
+  if (SOURCE == kStreamed) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
 
 // One tile.  Once the data are in LDS (the first barrier) the waves go their own ways: each takes
 // an equal share of the segments that start in the tile (with marks: those that start in its share
@@ -163,7 +187,7 @@ __global__ void __launch_bounds__(THREADS, WALK == kMarks || SOURCE == kMapped ?
 segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restrict__ emap,
                      const IdT* __restrict__ nmap, const float* __restrict__ data,
                      int64_t num_seg, int64_t nnz, int powk, float* __restrict__ out, Tiles tl) {
-  constexpr bool EMAP = SOURCE == kMapped;
+  constexpr bool EMAP = SOURCE == kMapped, PLAIN = SOURCE == kPlain || SOURCE == kStreamed;
   constexpr int kWaves = THREADS / kWave, kItems = kTile / THREADS;
   __shared__ __attribute__((aligned(16))) float s_v[kTile];
   __shared__ uint32_t s_list[kWaves][kWave];
@@ -190,13 +214,13 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
   if (p0 >= edges.end) return;
   const int n = edges.in_tile(p0);
   const int64_t p1 = p0 + n;
-  const bool vec = SOURCE == kPlain && n == kTile && (reinterpret_cast<uintptr_t>(data + p0) & 15u) == 0;
+  const bool vec = PLAIN && n == kTile && (reinterpret_cast<uintptr_t>(data + p0) & 15u) == 0;
   F4 q[kItems / kLaneEdges];
   if (vec) {
 #pragma unroll
     for (int k = 0; k < kItems / kLaneEdges; ++k)
-      q[k] = *reinterpret_cast<const F4*>(data + p0 + (k * THREADS + tid) * kLaneEdges);
-  } else if constexpr (SOURCE == kPlain) {  // (the last tile, or a first offset that is no multiple of 4)
+      q[k] = read_four<SOURCE>(data + p0 + (k * THREADS + tid) * kLaneEdges);
+  } else if constexpr (PLAIN) {  // (the last tile, or a first offset that is no multiple of 4)
 #pragma unroll
     for (int k = 0; k < kItems / kLaneEdges; ++k)
 #pragma unroll
@@ -208,7 +232,7 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
 
   int64_t where[EMAP ? kItems : 1];
   float x[kItems];
-  if constexpr (SOURCE != kPlain) {
+  if constexpr (!PLAIN) {
     if constexpr (EMAP) {
 #pragma unroll
       for (int k = 0; k < kItems; ++k) {
@@ -253,7 +277,7 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
     s_out = -1;
   }
   // x^powk of a thread's edges, one loop for all of them (the products are powk_f's)
-  if constexpr (SOURCE == kPlain) {
+  if constexpr (PLAIN) {
     F4 p[kItems / kLaneEdges];
 #pragma unroll
     for (int k = 0; k < kItems / kLaneEdges; ++k) p[k] = q[k];
@@ -474,9 +498,9 @@ segment_tiles_kernel(const int64_t* __restrict__ indptr, const int64_t* __restri
 #pragma unroll
       for (int k = 0; k < kItems / kLaneEdges; ++k) {
         const int i = (k * THREADS + tid) * kLaneEdges;
-        const float4 v = *reinterpret_cast<const float4*>(s_v + i);
+        const F4 v = *reinterpret_cast<const F4*>(s_v + i);
         if (i >= first && i + 3 < stop) {
-          *reinterpret_cast<float4*>(out + p0 + i) = v;
+          write_four<SOURCE>(out + p0 + i, v);
         } else {
           if (i >= first && i < stop) out[p0 + i] = v.x;
           if (i + 1 >= first && i + 1 < stop) out[p0 + i + 1] = v.y;
@@ -556,11 +580,12 @@ hub_totals_kernel(const int64_t* __restrict__ indptr, int64_t num_seg, int64_t n
 // up the pieces of its two segments for itself, a wave each or, of segments over more than 64
 // tiles, the whole workgroup (one segment of 32 M edges: 191 -> 85 us, of 100 M 1321 -> 458);
 // `hubs`: the totals of those over more than kHubTiles are there.
-template <bool EMAP>
+template <Source SOURCE>
 __global__ void __launch_bounds__(kThreads)
 crossing_divide_kernel(const int64_t* __restrict__ indptr, const int64_t* __restrict__ emap,
                        const float* __restrict__ data, int64_t num_seg, int64_t nnz,
                        float* __restrict__ out, Tiles tl, bool hubs) {
+  constexpr bool EMAP = SOURCE == kMapped;
   __shared__ float s_total[2];
   __shared__ int s_wide[2];  // whether the segment spans more than 64 tiles
   __shared__ int64_t s_tiles[2][2];
@@ -579,13 +604,13 @@ crossing_divide_kernel(const int64_t* __restrict__ indptr, const int64_t* __rest
   if (first == 0 && stop == n) return;
   const bool vec = !EMAP && n == kTile &&
                    ((reinterpret_cast<uintptr_t>(data + p0) | reinterpret_cast<uintptr_t>(out + p0)) & 15u) == 0;
-  float4 v[kTileItems / 4];
+  F4 v[kTileItems / 4];
   if (vec) {
 #pragma unroll
     for (int k = 0; k < kTileItems / 4; ++k) {
       const int i = k * (4 * kThreads) + 4 * tid;
-      v[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      if (i < first || i + 3 >= stop) v[k] = *reinterpret_cast<const float4*>(data + p0 + i);
+      v[k] = 0.0f;
+      if (i < first || i + 3 >= stop) v[k] = read_four<SOURCE>(data + p0 + i);
     }
   }
   if (wave < 2) {
@@ -623,8 +648,7 @@ crossing_divide_kernel(const int64_t* __restrict__ indptr, const int64_t* __rest
       const int i = k * (4 * kThreads) + 4 * tid;
       if (i + 3 < first || i >= stop) {
         const float d = i >= stop ? behind : before;
-        *reinterpret_cast<float4*>(out + p0 + i) =
-            make_float4(v[k].x / d, v[k].y / d, v[k].z / d, v[k].w / d);
+        write_four<SOURCE>(out + p0 + i, F4{v[k].x / d, v[k].y / d, v[k].z / d, v[k].w / d});
       } else if (i < first || i + 3 >= stop) {
         const float w[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
 #pragma unroll
@@ -681,9 +705,10 @@ carry_kernel(const int64_t* __restrict__ indptr, const IdT* __restrict__ nmap, i
   }
 }
 
-inline Source source_of(const int64_t* emap, const float* data) {
+inline Source source_of(const int64_t* emap, const float* data, int64_t nnz) {
   if (emap) return kMapped;
-  return (reinterpret_cast<uintptr_t>(data) & 15u) == 0 ? kPlain : kLoose;
+  if ((reinterpret_cast<uintptr_t>(data) & 15u) != 0) return kLoose;
+  return nnz >= kStreamEdges ? kStreamed : kPlain;
 }
 
 inline int64_t num_tiles(int64_t nnz) { return nnz <= 0 ? 1 : (nnz + kTile - 1) / kTile; }
@@ -753,18 +778,24 @@ int segment_sum_impl(const int64_t* indptr, const int64_t* emap, const void* nma
   const int64_t tiles = num_tiles(nnz);
   launch_heads<true>(indptr, nm, num_seg, nnz, out, tl, st);
   const Width width = tile_threads(num_seg, nnz);
+  // (so many edges that they are streamed are more than 6144 tiles)
+  static_assert(kStreamEdges / kTile > 6144, "tile_threads: marks and kMiddle, or kNarrow");
   auto pick = [&](auto source) {
     constexpr Source S = decltype(source)::value;
-    if (tl.mark)
+    if constexpr (S == kStreamed)
+      return tl.mark ? segment_tiles_kernel<false, S, kMarks, kMiddle, IdT>
+                     : segment_tiles_kernel<false, S, kHeads, kNarrow, IdT>;
+    else if (tl.mark)
       return width == kWidest ? segment_tiles_kernel<false, S, kMarks, kWidest, IdT>
                               : segment_tiles_kernel<false, S, kMarks, kMiddle, IdT>;
     return width == kWidest   ? segment_tiles_kernel<false, S, kHeads, kWidest, IdT>
            : width == kMiddle ? segment_tiles_kernel<false, S, kHeads, kMiddle, IdT>
                               : segment_tiles_kernel<false, S, kHeads, kNarrow, IdT>;
   };
-  const Source source = source_of(emap, data);
+  const Source source = source_of(emap, data, nnz);
   auto* kernel = source == kMapped  ? pick(std::integral_constant<Source, kMapped>{})
                  : source == kLoose ? pick(std::integral_constant<Source, kLoose>{})
+                 : source == kStreamed ? pick(std::integral_constant<Source, kStreamed>{})
                                     : pick(std::integral_constant<Source, kPlain>{});
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(width), 0, st, indptr, emap, nm,
                      data, num_seg, nnz, powk, out, tl);
@@ -780,13 +811,19 @@ void launch_normalize(Walk walk, const int64_t* indptr, const int64_t* emap, con
   const int64_t* no_map = nullptr;
   const int64_t tiles = num_tiles(nnz);
   const Width width = tile_threads(num_seg, nnz);
-  auto* kernel = walk == kSearch ? segment_tiles_kernel<true, SOURCE, kSearch, kWidest, int64_t>
-                 : walk == kMarks
-                     ? (width == kWidest ? segment_tiles_kernel<true, SOURCE, kMarks, kWidest, int64_t>
-                                         : segment_tiles_kernel<true, SOURCE, kMarks, kMiddle, int64_t>)
-                 : width == kWidest ? segment_tiles_kernel<true, SOURCE, kHeads, kWidest, int64_t>
-                 : width == kMiddle ? segment_tiles_kernel<true, SOURCE, kHeads, kMiddle, int64_t>
-                                    : segment_tiles_kernel<true, SOURCE, kHeads, kNarrow, int64_t>;
+  auto* kernel = [&] {
+    if constexpr (SOURCE == kStreamed)
+      return walk == kMarks ? segment_tiles_kernel<true, SOURCE, kMarks, kMiddle, int64_t>
+                            : segment_tiles_kernel<true, SOURCE, kHeads, kNarrow, int64_t>;
+    else
+      return walk == kSearch ? segment_tiles_kernel<true, SOURCE, kSearch, kWidest, int64_t>
+             : walk == kMarks
+                 ? (width == kWidest ? segment_tiles_kernel<true, SOURCE, kMarks, kWidest, int64_t>
+                                     : segment_tiles_kernel<true, SOURCE, kMarks, kMiddle, int64_t>)
+             : width == kWidest ? segment_tiles_kernel<true, SOURCE, kHeads, kWidest, int64_t>
+             : width == kMiddle ? segment_tiles_kernel<true, SOURCE, kHeads, kMiddle, int64_t>
+                                : segment_tiles_kernel<true, SOURCE, kHeads, kNarrow, int64_t>;
+  }();
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(width), 0, st, indptr, emap,
                      no_map, data, num_seg, nnz, 1, out, tl);
   const bool hubs = tiles > kHubLaunch;
@@ -794,7 +831,7 @@ void launch_normalize(Walk walk, const int64_t* indptr, const int64_t* emap, con
     hipLaunchKernelGGL(hub_totals_kernel, dim3(blocks_for(tiles, kHubTiles)), dim3(kThreads), 0, st,
                        indptr, num_seg, nnz, tl);
   if (tiles > 1)
-    hipLaunchKernelGGL((crossing_divide_kernel<SOURCE == kMapped>),
+    hipLaunchKernelGGL((crossing_divide_kernel<SOURCE>),
                        dim3(static_cast<unsigned>(tiles)), dim3(kThreads), 0, st, indptr, emap, data,
                        num_seg, nnz, out, tl, hubs);
 }
@@ -806,10 +843,11 @@ int segment_normalize_impl(const int64_t* indptr, const int64_t* emap, const flo
   const Walk walk = tl.mark ? kMarks : (num_tiles(nnz) > kSearchTiles ? kHeads : kSearch);
   if (walk != kSearch)
     launch_heads<false>(indptr, static_cast<const int64_t*>(nullptr), num_seg, nnz, out, tl, st);
-  const Source source = source_of(emap, data);
+  const Source source = source_of(emap, data, nnz);
   auto* launch = source == kMapped  ? launch_normalize<kMapped>
                  : source == kLoose ? launch_normalize<kLoose>
-                                    : launch_normalize<kPlain>;
+                 : source == kStreamed ? launch_normalize<kStreamed>
+                                       : launch_normalize<kPlain>;
   launch(walk, indptr, emap, data, num_seg, nnz, out, tl, st);
   return check_launch("segment_normalize");
 }

@@ -77,6 +77,30 @@ def test_segments_of_thousands_of_tiles(dev, lens):
         torch.testing.assert_close(got.double(), p / t, rtol=rtol, atol=0)
 
 
+# both sides of the 2**25 edges from which data and results are streamed; offsets that begin
+# at an edge whose place is no multiple of four; more segments than edges (marks)
+@pytest.mark.parametrize("kind", ["mixed", "border", "sparse"])
+@pytest.mark.parametrize("nnz,front", [((1 << 25) - 1, 0), (1 << 25, 0), ((1 << 25) + 4099, 3)])
+def test_streamed_edges(dev, kind, nnz, front):
+    some = torch.from_numpy(np.diff(_segments(kind, 1_500_000))).to(dev)
+    lens = some.repeat(nnz // int(some.sum()) + 1)
+    ends = torch.cumsum(lens, 0).clamp_(max=nnz)
+    ptr = torch.cat([ends.new_zeros(1), ends])
+    data = torch.rand(front + nnz, device=dev) + 0.25
+    owner = torch.repeat_interleave(torch.diff(ptr), output_size=nnz)
+    w = data[front:].double()
+    for power in (1, 2):
+        want = torch.zeros(lens.numel(), dtype=torch.float64, device=dev).index_add_(0, owner, w ** power)
+        out = torch.full((lens.numel(),), -1.0, device=dev)
+        capi.segment_sum(ptr + front, None, None, data, power, out)
+        torch.testing.assert_close(out.double(), want, rtol=RTOL, atol=0)
+        if power == 1:
+            out = torch.full_like(data, -1.0)
+            capi.segment_normalize(ptr + front, None, data, out)
+            torch.testing.assert_close(out[front:].double(), w / want[owner], rtol=RTOL, atol=0)
+            assert (out[:front] == -1).all()
+
+
 def _check(dev, kind, total, emap, rtol=RTOL):
     indptr = _segments(kind, total)
     nnz, nseg = int(indptr[-1]), indptr.size - 1
