@@ -536,6 +536,7 @@ struct SortOutputs {
   uint32_t* key;
   int idx_bits;
   int* wide;  // raised when a 64-bit value does not fit 32 bits (null: 32-bit values)
+  bool stream;  // packed_pass_kernel: results as streams (kStreamResults)
 };
 
 // One pass of the sort over one tile, stable.  A wave owns its share of the tile, in index
@@ -745,7 +746,12 @@ radix_pass_kernel(Src src, const ValT* __restrict__ val_in, int64_t E, int shift
 // `wide`.  The next pass's digits are written beside the words, for its histogram to read a byte an edge.
 // 14 M edges, 22-bit keys (24 bits each for value and position): the passes 72 + 65 + 82 us with the
 // values beside the words, 67 + 59 + 81 so; the last two histograms 24 -> 8 each.
+// What a pass reads, nothing reads again, so it reads past the caches (14 M edges with 64-bit ids, loaded
+// and sorted: 420 -> 415 us; 11 M / 8 M with 32-bit ids 322 -> 301, 290 -> 277).  The words it writes are the next
+// pass's: written past the caches they cost 456.  The last pass's results go past them where they
+// fill more than half of the memory-side cache (14 M: 415 -> 404, 11 M: 301 -> 290; 8 M, 128 MB: 277, 278).
 constexpr int kPackedPasses = 3;
+constexpr int64_t kStreamResults = int64_t(1) << 27;  // bytes
 constexpr int rest_at(int passes) { return 64 - kRadixBits * (passes - 1); }  // of the key's digits in a word
 
 template <typename T, typename IdT, int PASSES, int PASS>
@@ -780,6 +786,8 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const int digit = threadIdx.x;  // of the first 256 threads
+  // (a value that did not fit its bits, met by the first pass: they are all fetched again)
+  const bool refetch = LAST && *last.wide != 0;
   int64_t all = 0, before_tile = 0;
   uint32_t ends = 0;
   if (digit < kRadix) {
@@ -798,9 +806,9 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
   for (int r = 0; r < kItemsHere; ++r) {
     const uint32_t j = mine0 + r * kWave;
     if constexpr (FIRST)
-      fresh[r] = static_cast<uint32_t>((key + base)[j < n ? j : n - 1]);
+      fresh[r] = static_cast<uint32_t>(__builtin_nontemporal_load(key + base + (j < n ? j : n - 1)));
     else
-      word[r] = (in + base)[j < n ? j : n - 1];
+      word[r] = __builtin_nontemporal_load(in + base + (j < n ? j : n - 1));
   }
   // (what lies behind the last edge takes the last digit, as above)
 #pragma unroll
@@ -822,7 +830,7 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
       if (lane == kWave - 1) s_ends[wave] = ends;
     }
   }
-  __syncthreads();  // the tables are zero
+  lds_barrier();  // the tables are zero
   auto digit_here = [&](int r) {
     if constexpr (FIRST)
       return static_cast<int>(fresh[r] & (kRadix - 1));
@@ -854,10 +862,10 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
 #pragma unroll
     for (int r = 0; r < kItemsHere; ++r) {
       const uint32_t j = again0 + r * kWave;
-      raw[r] = tile_val[j < n ? j : n - 1];
+      raw[r] = __builtin_nontemporal_load(tile_val + (j < n ? j : n - 1));
     }
   }
-  __syncthreads();
+  lds_barrier();
   int total = 0, incl = 0;
   int64_t run_at = 0;
   if (digit < kRadix) {
@@ -885,7 +893,7 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
       s_digits[wave] = run_at;
     }
   }
-  __syncthreads();
+  lds_barrier();
   if (digit < kRadix) {
     int start = incl - total;
     run_at += s_base[digit] - s_all[digit];
@@ -897,7 +905,7 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
     s_base[digit] = run_at - start;
     if (!FIRST) s_bound[digit] = ends;
   }
-  __syncthreads();
+  lds_barrier();
 #pragma unroll
   for (int r = 0; r < kItemsHere; ++r) {
     const int d = digit_here(r);
@@ -911,7 +919,7 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
     for (int step = kRadix / 2; step > 0; step >>= 1)
       if (s_bound[was + step - 1] <= at) was += step;
   }
-  __syncthreads();  // (the counts make room for the digits)
+  lds_barrier();  // (the counts make room for the digits)
   bool wide = false;
   uint32_t third0 = mine0;  // (indices made once more rather than kept)
   asm volatile("" : "+v"(third0));
@@ -936,7 +944,7 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
     s_dig[place[r]] = static_cast<unsigned char>(d);
   }
   if (FIRST && wide) *last.wide = 1;  // (the last edge's value again past the end)
-  __syncthreads();
+  lds_barrier();
 #pragma unroll
   for (int k = 0; k < kItemsHere; ++k) {
     const uint32_t j = k * kThreadsHere + threadIdx.x;
@@ -945,8 +953,16 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
       const uint32_t d = s_dig[j];
       const int64_t dst = s_base[d] + j;
       if (LAST) {
-        last.perm[dst] = static_cast<int64_t>(w & ((1ull << (kRestAt - value_bits)) - 1ull));
-        last.value[dst] = static_cast<IdT>((w & ((1ull << kRestAt) - 1ull)) >> (kRestAt - value_bits));
+        const int64_t from = static_cast<int64_t>(w & ((1ull << (kRestAt - value_bits)) - 1ull));
+        IdT v = static_cast<IdT>((w & ((1ull << kRestAt) - 1ull)) >> (kRestAt - value_bits));
+        if (refetch) v = value[from];
+        if (last.stream) {
+          __builtin_nontemporal_store(from, last.perm + dst);
+          __builtin_nontemporal_store(v, last.value + dst);
+        } else {
+          last.perm[dst] = from;
+          last.value[dst] = v;
+        }
         if (last.key)
           last.key[dst] = d << (kRadixBits * PASS) | static_cast<uint32_t>(w >> kRestAt);
       } else {
@@ -957,7 +973,7 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
   }
 }
 
-// Behind the sort: fetches the values all again when one did not fit its bits.
+// Behind a sort with the values beside the words: fetches them all again when one did not fit 32 bits.
 template <typename IdT>
 __global__ void __launch_bounds__(kThreads)
 widen_values_kernel(const IdT* __restrict__ value, const int64_t* __restrict__ perm, int64_t E,
@@ -1157,7 +1173,8 @@ int coo2csc_impl(const IdT* key, const IdT* value, int64_t E, int64_t num_keys, 
   const bool may_be_wide = sizeof(IdT) == 8 || value_bits > 0;
   const bool short_keys = passes * kRadixBits <= 32;
   const SortOutputs<IdT> outs{out_value, perm, indptr && short_keys ? s.keys : nullptr, idx_bits,
-                              may_be_wide ? s.wide : nullptr};
+                              may_be_wide ? s.wide : nullptr,
+                              E * static_cast<int64_t>(sizeof(int64_t) + sizeof(IdT) + sizeof(uint32_t)) >= kStreamResults};
   if (value_bits > 0) {
     const auto sort = large ? packed_passes<LargeTile, IdT> : packed_passes<SmallTile, IdT>;
     GS_RETURN_IF_ERROR(sort(key, value, E, passes, value_bits, s, outs, st));
@@ -1165,7 +1182,7 @@ int coo2csc_impl(const IdT* key, const IdT* value, int64_t E, int64_t num_keys, 
     const auto sort = large ? sort_passes<LargeTile, IdT> : sort_passes<SmallTile, IdT>;
     GS_RETURN_IF_ERROR(sort(key, value, E, passes, idx_bits, s, outs, st));
   }
-  if (may_be_wide)
+  if (may_be_wide && value_bits == 0)  // (words with the value inside: the last pass does it)
     hipLaunchKernelGGL(widen_values_kernel<IdT>, dim3(E < (int64_t(1) << 20) ? 64 : 1024),
                        dim3(kThreads), 0, st, value, perm, E, s.wide, out_value);
   if (indptr && short_keys)  // (null: the caller wants the sorted order only)
@@ -1199,6 +1216,7 @@ struct DistinctSpace {
   int64_t num_partial;
   int64_t* first;      // {distinct ids of the first end, 1 when the second has to be counted}
   int64_t* slices;     // by bits: slices that the first marking launch takes
+  bool bits;
 };
 
 __global__ void __launch_bounds__(kThreads) clear_marks_kernel(uint4* map, int64_t n) {
@@ -1317,8 +1335,9 @@ post_distinct_kernel(DistinctSpace s, gs_mailbox* box, int64_t ticket) {
   int64_t second = 0;
   const bool counted = s.first[1] != 0;
   block_exclusive_scan<kDecideThreads>(counted ? sum_partial(s, kDecideThreads) : 0, &second, lds);
-  // (-1 and -2, an id outside the range, leave the second end uncounted)
-  if (threadIdx.x == 0) post_mailbox(box, counted && second > s.first[0] ? second : s.first[0], ticket);
+  // (-1 and -2, an id outside the range, leave the second end uncounted; by bits, the launch that found
+  // so has posted)
+  if (threadIdx.x == 0 && (counted || !s.bits)) post_mailbox(box, counted && second > s.first[0] ? second : s.first[0], ticket);
 }
 
 // The same for long lists, by bits in LDS: every compute unit keeps a bitmap of 1.28 M ids and
@@ -1420,7 +1439,8 @@ struct FirstSlices {
 };
 
 // A thread's ids of [lo, hi) to `use`, the next trip's on their way meanwhile; `before` runs behind
-// the first trip's loads.  (Ids behind hi are the last one again; 419 -> 417 us, 6 M over 1 M nodes 254 -> 252.)
+// the first trip's loads.  (Ids behind hi are the last one again; 419 -> 417 us, 6 M over 1 M nodes 254 -> 252.
+// As streams: the list loaded and sorted 415 -> 406, 11 M edges, 32-bit ids 301 -> 295.)
 template <typename IdT, typename Before, typename Use>
 __device__ __forceinline__ void each_id(const IdT* __restrict__ ids, int64_t lo, int64_t hi, Before before,
                                         Use use) {
@@ -1430,7 +1450,7 @@ __device__ __forceinline__ void each_id(const IdT* __restrict__ ids, int64_t lo,
 #pragma unroll
     for (int u = 0; u < kBitTrip; ++u) {
       const int64_t at = i + u * kBitThreads;
-      to[u] = ids[at < hi ? at : hi - 1];
+      to[u] = __builtin_nontemporal_load(ids + (at < hi ? at : hi - 1));
     }
   };
   if (i < hi) load(id);
@@ -1449,14 +1469,18 @@ __device__ __forceinline__ void each_id(const IdT* __restrict__ ids, int64_t lo,
 // (null when the largest is known).
 template <typename IdT, bool REST, bool SECOND>
 __global__ void __launch_bounds__(kBitThreads)
-mark_bits_kernel(const IdT* __restrict__ ids, const IdT* __restrict__ look, int64_t E, DistinctSpace s) {
+mark_bits_kernel(const IdT* __restrict__ ids, const IdT* __restrict__ look, int64_t E, DistinctSpace s,
+                 gs_mailbox* box, int64_t ticket) {
   static_assert(!(REST && SECOND), "nothing is left behind the second end's launch");
   __shared__ __attribute__((aligned(16))) uint32_t s_bits[kBitWords];
   __shared__ int64_t s_wave[kBitThreads / kWave];
   int64_t slices;
   if constexpr (SECOND) {
     slices = second_slices(s);
-    if (!slices) return;
+    if (!slices) {  // the count is known: the host has it two launches earlier
+      if (blockIdx.x == 0 && threadIdx.x == 0) post_mailbox(box, s.first[0], ticket);
+      return;
+    }
   } else {
     slices = *s.slices;
   }
@@ -1563,14 +1587,18 @@ __global__ void __launch_bounds__(kThreads) count_bits_kernel(DistinctSpace s) {
 }
 
 template <typename IdT>
-void distinct_by_bits(const IdT* a, const IdT* b, int64_t E, const DistinctSpace& s, hipStream_t st) {
+void distinct_by_bits(const IdT* a, const IdT* b, int64_t E, const DistinctSpace& s, gs_mailbox* box,
+                      int64_t ticket, hipStream_t st) {
   hipLaunchKernelGGL((guess_slices_kernel<IdT>), dim3(1), dim3(kGuessThreads), 0, st, a, b, E, s);
   const IdT* known = nullptr;
   const dim3 marks(kBitBlocks), counts(kOrBlocks, kMaxSlices);
-  hipLaunchKernelGGL((mark_bits_kernel<IdT, false, false>), marks, dim3(kBitThreads), 0, st, a, b, E, s);
-  hipLaunchKernelGGL((mark_bits_kernel<IdT, true, false>), marks, dim3(kBitThreads), 0, st, a, b, E, s);
+  hipLaunchKernelGGL((mark_bits_kernel<IdT, false, false>), marks, dim3(kBitThreads), 0, st, a, b, E, s,
+                     box, ticket);
+  hipLaunchKernelGGL((mark_bits_kernel<IdT, true, false>), marks, dim3(kBitThreads), 0, st, a, b, E, s,
+                     box, ticket);
   hipLaunchKernelGGL(count_bits_kernel<false>, counts, dim3(kThreads), 0, st, s);
-  hipLaunchKernelGGL((mark_bits_kernel<IdT, false, true>), marks, dim3(kBitThreads), 0, st, b, known, E, s);
+  hipLaunchKernelGGL((mark_bits_kernel<IdT, false, true>), marks, dim3(kBitThreads), 0, st, b, known, E, s,
+                     box, ticket);
   hipLaunchKernelGGL(count_bits_kernel<true>, counts, dim3(kThreads), 0, st, s);
 }
 
@@ -1992,6 +2020,7 @@ int gs_distinct_ends(const void* a, const void* b, int id_bytes, int64_t E, void
   s.partial = ws.take<int64_t>(static_cast<size_t>(s.num_partial));
   s.first = ws.take<int64_t>(3);
   s.slices = s.first + 2;
+  s.bits = by_bits;
   if (!ws.ok) {
     set_error_text("gs_distinct_ends: workspace needs %zu bytes, 256-byte aligned",
                    gs_distinct_ends_workspace_bytes(E));
@@ -2000,9 +2029,11 @@ int gs_distinct_ends(const void* a, const void* b, int id_bytes, int64_t E, void
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (by_bits) {
     if (id_bytes == 8)
-      distinct_by_bits(static_cast<const int64_t*>(a), static_cast<const int64_t*>(b), E, s, st);
+      distinct_by_bits(static_cast<const int64_t*>(a), static_cast<const int64_t*>(b), E, s, mailbox,
+                       ticket, st);
     else
-      distinct_by_bits(static_cast<const int32_t*>(a), static_cast<const int32_t*>(b), E, s, st);
+      distinct_by_bits(static_cast<const int32_t*>(a), static_cast<const int32_t*>(b), E, s, mailbox,
+                       ticket, st);
   } else {
     const int64_t vecs = 2 * range / 16;
     hipLaunchKernelGGL(clear_marks_kernel, dim3(blocks_for(vecs, kThreads * 4)), dim3(kThreads), 0, st,
