@@ -15,7 +15,7 @@
 //   * the ids (and data) of the NEXT tile are asked for before this tile's are looked up, since
 //     the few waves beside the set have little else to hide that latency behind;
 //   * kept edges leave one bit each and, packed to the front of the tile's range of a scratch
-//     array, their new row number in 4 bytes and their datum.
+//     array, their new row number in 2 bytes and their datum.
 // A scan of the tile counts and one copy kernel put the pieces together.  (With the tiles shared
 // by the waves of a workgroup, offsets and counts through LDS and two barriers a tile, the marks
 // took 293 us where they take 225.)
@@ -31,7 +31,8 @@
 // What bounds the bitmap form: 785 MB in 225 us in the case below, 3.5 TB/s, with the vector ALUs
 // issuing 45 % of the time; more waves than the set leaves room for would be needed to
 // overlap the two better.  7263 nodes whose columns hold 50.8 M edges, 22.0 M kept, 64-bit ids
-// and weights: 225 us for the marks and 70 us for the copy, where a filter and a table in the
+// and weights: 225 us for the marks and 70 us for the copy (new row numbers in 2 bytes instead of 4 and
+// streamed: 185 + 84), where a filter and a table in the
 // L2s, parent positions carried along and a gather of the data behind took 546 + 226 + 104.
 #include "gs_common.hpp"
 
@@ -54,7 +55,7 @@ struct InducedMarks {
   int32_t* word_rank;        // kept positions of the tile before each 64-position word
   int64_t* tile_counts;
   int64_t* tile_base;        // exclusive scan of tile_counts
-  uint32_t* packed;          // new row numbers of the kept edges, at the front of the tile's range
+  uint16_t* packed;          // new row numbers (places, 14 bits) of the kept edges, at the front of the tile's range
   float* packed_data;        // their data (null: none)
   int* outside;              // set when an id lies beyond the bitmap: the call has to be repeated
   int64_t n;
@@ -270,7 +271,7 @@ __device__ __forceinline__ int row_of(const int64_t* off, int lo, int hi, int64_
 // What a wave's edges bring along: nothing, data[position], or data[e_ids[position]].
 enum Data { kNoData, kByPosition, kByEdgeId };
 
-template <typename IdT, typename Set, int BLOCK, Data DATA>
+template <typename IdT, typename Set, int BLOCK, Data DATA, bool STREAM>
 __global__ void __launch_bounds__(BLOCK, 4)  // (16 waves a compute unit: what the set leaves room for)
 induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
                     const IdT* __restrict__ indices, const IdT* __restrict__ cols, int64_t S,
@@ -356,6 +357,8 @@ induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
     float w[DATA == kByPosition ? kPer : 1];
     int64_t e[DATA == kByEdgeId ? kPer : 1];
   };
+  // (STREAM: beyond the caches' size what a call reads is gone from them before anyone reads it again)
+  auto once = [](const auto* p) { return STREAM ? __builtin_nontemporal_load(p) : *p; };
   auto fetch = [&](int64_t t, Held& h) {
     int64_t at[kPer];
 #pragma unroll
@@ -364,15 +367,15 @@ induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
       at[k] = locate(q < D ? q : D - 1);
     }
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) h.id[k] = indices[at[k]];
+    for (int k = 0; k < kPer; ++k) h.id[k] = once(indices + at[k]);
     // (the data of all: 64 neighbours share their lines with the kept ones among them)
     if constexpr (DATA == kByPosition) {
 #pragma unroll
-      for (int k = 0; k < kPer; ++k) h.w[k] = data[at[k]];
+      for (int k = 0; k < kPer; ++k) h.w[k] = once(data + at[k]);
     }
     if constexpr (DATA == kByEdgeId) {
 #pragma unroll
-      for (int k = 0; k < kPer; ++k) h.e[k] = e_ids[at[k]];
+      for (int k = 0; k < kPer; ++k) h.e[k] = once(e_ids + at[k]);
     }
   };
 
@@ -408,7 +411,7 @@ induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
                                                               static_cast<uint32_t>(kept), 0));
       before += __popcll(kept);
       if (val[k] >= 0) {
-        m.packed[p0 + rank] = static_cast<uint32_t>(val[k]);
+        m.packed[p0 + rank] = static_cast<uint16_t>(val[k]);
         if constexpr (DATA == kByPosition) m.packed_data[p0 + rank] = now.w[k];
         if constexpr (DATA == kByEdgeId) m.packed_data[p0 + rank] = w[k];
       }
@@ -446,7 +449,7 @@ induced_indptr_kernel(const int64_t* __restrict__ sub_indptr, int64_t S, Induced
 // time: eight times 64, all reads before the stores.
 constexpr int kCopyTiles = 4;  // of a workgroup, one for every wave
 
-template <typename IdT>
+template <typename IdT, bool STREAM>
 __global__ void __launch_bounds__(256)
 induced_compact_kernel(InducedMarks m, IdT* __restrict__ out_indices, float* __restrict__ out_data) {
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
@@ -455,7 +458,7 @@ induced_compact_kernel(InducedMarks m, IdT* __restrict__ out_indices, float* __r
   const int64_t base = m.tile_base[t];
   const int count = static_cast<int>(m.tile_base[t + 1] - base);
   if (count == 0) return;
-  uint32_t v[kPer];
+  uint16_t v[kPer];
   float x[kPer];
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
@@ -473,8 +476,13 @@ induced_compact_kernel(InducedMarks m, IdT* __restrict__ out_indices, float* __r
   for (int k = 0; k < kPer; ++k) {
     const int r = k * kWave + lane;
     if (r < count) {
-      out_indices[base + r] = static_cast<IdT>(v[k]);
-      if (out_data) out_data[base + r] = x[k];
+      if (STREAM) {
+        __builtin_nontemporal_store(static_cast<IdT>(v[k]), out_indices + base + r);
+        if (out_data) __builtin_nontemporal_store(x[k], out_data + base + r);
+      } else {
+        out_indices[base + r] = static_cast<IdT>(v[k]);
+        if (out_data) out_data[base + r] = x[k];
+      }
     }
   }
 }
@@ -492,7 +500,7 @@ bool carve_induced(void* workspace, size_t bytes, int64_t D, bool with_data, Ind
   m->tile_base = ws.take<int64_t>(most + 2);
   *scan_tiles = ws.take<int64_t>(static_cast<size_t>(scan_num_tiles(m->tiles) + 1));
   m->outside = ws.take<int>(1);
-  m->packed = ws.take<uint32_t>(static_cast<size_t>(D));
+  m->packed = ws.take<uint16_t>(static_cast<size_t>(D));
   m->packed_data = with_data ? ws.take<float>(static_cast<size_t>(D)) : nullptr;
   return ws.ok;
 }
@@ -510,9 +518,19 @@ struct MarkCall {
   const int64_t* e_ids;
 };
 
+// Whether the ids and data of D positions are more than the 256 MB that the memory-side cache holds.
+// The whole call (walk, unique nodes and subgraph), plain / streamed: 50.8 M positions with 64-bit ids and data (610 MB)
+// 398-412 / 383-394 us (marks 216 / 185, copy 67 / 84: who stores past the cache leaves it to the other);
+// graphs of 100 M edges, 1.5 M nodes and of 50 M, 0.2 M, a few hundred seeds, 32-bit ids 217 / 216, 157 / 159.
+inline bool streams(int64_t D, size_t id_bytes, bool with_data) {
+  return D * static_cast<int64_t>(id_bytes + (with_data ? 4 : 0)) >= int64_t(1) << 28;
+}
+
 template <typename IdT, typename Set, int BLOCK, Data DATA>
 int launch_mark(const MarkCall& c, int per_unit, const InducedMarks& m, hipStream_t st) {
-  auto* kernel = induced_mark_kernel<IdT, Set, BLOCK, DATA>;
+  auto* kernel = streams(c.D, sizeof(IdT), DATA != kNoData)
+                     ? induced_mark_kernel<IdT, Set, BLOCK, DATA, true>
+                     : induced_mark_kernel<IdT, Set, BLOCK, DATA, false>;
   const size_t bytes = Set::lds_bytes(c.bound, c.n_ids);
   // (per call: the attribute belongs to the device the call runs on)
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -582,7 +600,7 @@ size_t gs_induced_slice_workspace_bytes(int64_t D, int with_data) {
   const int64_t tiles = ((D - 1) >> kTileShift) + 1;
   return padded(words * 8) + padded(words * 4) + padded(static_cast<size_t>(tiles + 1) * 8) +
          padded(static_cast<size_t>(tiles + 2) * 8) + scan_workspace_bytes(tiles) + 256 +
-         padded(n * 4) + (with_data ? padded(n * 4) : 0);
+         padded(n * 2) + (with_data ? padded(n * 4) : 0);
 }
 
 int gs_induced_slice_mark(const int64_t* indptr, int64_t num_cols, const void* indices, int64_t nnz,
@@ -629,12 +647,16 @@ int gs_induced_slice_compact(int64_t D, int id_bytes, void* out_indices, float* 
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 grid(blocks_for(m.tiles, kCopyTiles));
+  const bool stream_out = streams(D, static_cast<size_t>(id_bytes), out_data != nullptr);
+  auto go = [&](auto* kernel, auto* indices) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, m, indices, out_data);
+  };
   if (id_bytes == 8)
-    hipLaunchKernelGGL(induced_compact_kernel<int64_t>, grid, dim3(256), 0, st, m,
-                       static_cast<int64_t*>(out_indices), out_data);
+    go(stream_out ? induced_compact_kernel<int64_t, true> : induced_compact_kernel<int64_t, false>,
+       static_cast<int64_t*>(out_indices));
   else
-    hipLaunchKernelGGL(induced_compact_kernel<int32_t>, grid, dim3(256), 0, st, m,
-                       static_cast<int32_t*>(out_indices), out_data);
+    go(stream_out ? induced_compact_kernel<int32_t, true> : induced_compact_kernel<int32_t, false>,
+       static_cast<int32_t*>(out_indices));
   return check_launch("induced_slice_compact");
 }
 

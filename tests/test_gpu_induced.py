@@ -179,3 +179,38 @@ def test_short_columns(dev, hubs, hub_degree, small, n, columns, weights):
     assert np.array_equal(sub._CAPI_GetCSC()[1].cpu().numpy(), want[1])
     if weights:
         assert np.array_equal(sub._CAPI_GetData("default").cpu().numpy(), w[want[3]])
+
+
+# more bytes of ids and data than are read through the caches; both forms of the set
+@pytest.mark.parametrize("idt", [torch.int32, torch.int64])
+@pytest.mark.parametrize("n", [60_000, 2_000_000])
+@pytest.mark.parametrize("data", ["none", "by position", "by edge id"])
+def test_streamed_positions(dev, data, n, idt):
+    S, degree = 20, 3_400_001
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(n)
+    row = torch.randint(0, n, (S * degree,), generator=gen, device=dev, dtype=idt)
+    w = torch.rand(S * degree, generator=gen, device=dev)
+    g = gs.Graph(False)
+    if data == "by edge id":  # the columns from the last to the first
+        col = torch.arange(S - 1, -1, -1, device=dev, dtype=idt).repeat_interleave(degree)
+        g._CAPI_LoadCOO(row, col)
+        row, order = row.view(S, degree).flip(0).reshape(-1), w.view(S, degree).flip(0).reshape(-1)
+    else:
+        ptr = torch.full((n + 1,), S * degree, device=dev)
+        ptr[:S + 1] = torch.arange(S + 1, device=dev) * degree
+        g._CAPI_LoadCSC(ptr, row)
+        order = w
+    if data != "none":
+        g._CAPI_SetData(w)
+    cols = torch.arange(S, device=dev, dtype=idt)
+    rows = torch.randperm(n, generator=gen, device=dev)[:7001].to(idt)
+    sub = g._CAPI_FusionSlicing(cols, rows)
+    place = torch.full((n,), -1, dtype=idt, device=dev)
+    place[rows.long()] = torch.arange(7001, dtype=idt, device=dev)
+    want = place[row.long()]
+    ptr, idx, _ = sub._CAPI_GetCSC()
+    assert torch.equal(idx, want[want >= 0])
+    assert torch.equal(ptr[1:], torch.cumsum((want >= 0).view(S, degree).sum(1), 0))
+    if data != "none":
+        assert torch.equal(sub._CAPI_GetData("default"), order[want >= 0])
