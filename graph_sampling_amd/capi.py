@@ -38,7 +38,8 @@ def lib():
                      "gs_segment_workspace_bytes", "gs_layer_workspace_bytes",
                      "gs_layer_sample_state_bytes", "gs_layer_relabel_state_bytes",
                      "gs_coo_sum_workspace_bytes", "gs_coo_pick_rows_workspace_bytes",
-                     "gs_coo_block_values_workspace_bytes", "gs_random_walk_workspace_bytes"):
+                     "gs_coo_block_values_workspace_bytes", "gs_random_walk_workspace_bytes",
+                     "gs_metapath_walk_workspace_bytes"):
             if hasattr(_lib, name):
                 getattr(_lib, name).restype = ctypes.c_size_t
         _lib.gs_sorted_union_max.restype = ctypes.c_int64
@@ -997,9 +998,11 @@ def random_walk(indptr, indices, seeds, length, seed=0, replay=None, packed=None
 
 
 def metapath_walk(indptr_table, indices_table, num_nodes_table, id_dtype, metapath, seeds, seed=0,
-                  replay=None):
+                  replay=None, num_nodes=0, packed=None):
     """indptr_table / indices_table: device int64 tensors holding device addresses;
-    num_nodes_table: device int64 tensor, columns per relation."""
+    num_nodes_table: device int64 tensor, columns per relation; num_nodes: their sum, for which
+    packed tables of the offsets have room (0: none are made); packed: whether they are (None: where
+    it pays)."""
     _need(num_nodes_table, torch.int64, "num_nodes_table")
     _need(metapath, torch.int64, "metapath")
     idb = _ids(seeds, "seeds")
@@ -1009,9 +1012,15 @@ def metapath_walk(indptr_table, indices_table, num_nodes_table, id_dtype, metapa
     n = seeds.numel()
     L = metapath.numel()
     trace = torch.empty((L + 1) * n, dtype=seeds.dtype, device=dev)
-    _check(lib().gs_metapath_walk(_ptr(indptr_table), _ptr(indices_table), _ptr(num_nodes_table), idb, _ptr(metapath),
-                                  _i64(L), _ptr(seeds), _i64(n), _u64(seed), _ptr(replay),
-                                  _ptr(trace), _stream(dev)), "gs_metapath_walk")
+    relations = num_nodes_table.numel()
+    size = lib().gs_metapath_walk_workspace_bytes(_i64(relations), _i64(num_nodes), _i64(n), _i64(L))
+    if packed is not None:
+        size = (num_nodes // 6 + relations + 1) * 16 + relations * 8 + 512 if packed else 0
+    ws = torch.empty(size, dtype=torch.uint8, device=dev)
+    _check(lib().gs_metapath_walk_workspace(
+        _ptr(indptr_table), _ptr(indices_table), _ptr(num_nodes_table), _i64(relations),
+        _i64(num_nodes), idb, _ptr(metapath), _i64(L), _ptr(seeds), _i64(n), _u64(seed), _ptr(replay),
+        _ptr(trace), _ptr(ws), ctypes.c_size_t(size), _stream(dev)), "gs_metapath_walk")
     return trace
 
 

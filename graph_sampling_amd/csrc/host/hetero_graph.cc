@@ -18,6 +18,7 @@ void HeteroGraph::LoadFromHomo(
   for (size_t i = 0; i < node_types.size(); ++i) node_type_id_[node_types[i]] = static_cast<int64_t>(i);
   std::vector<int64_t> indptr_addr, indices_addr, num_nodes;
   torch::Device device(torch::kCPU);
+  num_nodes_ = 0;
   for (size_t i = 0; i < edge_types.size(); ++i) {
     edge_type_id_[std::get<1>(edge_types[i])] = static_cast<int64_t>(i);
     auto csc = edge_relations[i]->GetCSC();
@@ -30,6 +31,7 @@ void HeteroGraph::LoadFromHomo(
     indptr_addr.push_back(reinterpret_cast<int64_t>(csc->indptr.data_ptr()));
     indices_addr.push_back(reinterpret_cast<int64_t>(csc->indices.data_ptr()));
     num_nodes.push_back(csc->indptr.numel() - 1);
+    num_nodes_ += num_nodes.back();
     device = csc->indptr.device();
   }
   if (!edge_types.empty()) {
@@ -60,7 +62,7 @@ torch::Tensor HeteroGraph::MetapathRandomWalkFused(torch::Tensor seeds,
     cached = metapath_cache_.emplace(metapath, dev).first;
   }
   return hip::MetapathWalk(seeds, cached->second, indptr_table_, indices_table_, num_nodes_table_,
-                           id_bytes_)
+                           num_nodes_, id_bytes_)
       .reshape({seeds.numel(), -1});
 }
 

@@ -38,6 +38,7 @@ class HeteroGraph : public torch::CustomClassHolder {
   std::vector<c10::intrusive_ptr<Graph>> relations_;
   // device tables of the relations' indptr / indices addresses, built once
   torch::Tensor indptr_table_, indices_table_, num_nodes_table_;
+  int64_t num_nodes_ = 0;  // of all relations together
   int id_bytes_ = 8;
   // metapaths already uploaded (the reference re-uploads on every call,
   // src/hetero_graph.cc:66-69)

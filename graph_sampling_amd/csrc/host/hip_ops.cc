@@ -1167,17 +1167,22 @@ torch::Tensor RandomWalk(const torch::Tensor& seeds, int64_t length, const torch
 
 torch::Tensor MetapathWalk(const torch::Tensor& seeds, const torch::Tensor& metapath,
                            const torch::Tensor& indptr_table, const torch::Tensor& indices_table,
-                           const torch::Tensor& num_nodes_table, int id_bytes) {
+                           const torch::Tensor& num_nodes_table, int64_t num_nodes, int id_bytes) {
   NeedI64(num_nodes_table, "relation sizes");
   TORCH_CHECK(IdBytes(seeds, "seeds") == id_bytes, "seeds and relation graphs differ in dtype");
   NeedI64(metapath, "metapath");
   const int64_t n = seeds.numel();
   const int64_t L = metapath.numel();
   auto trace = torch::empty({n * (L + 1)}, seeds.options());
-  Check(gs_metapath_walk(reinterpret_cast<const int64_t* const*>(indptr_table.data_ptr<int64_t>()),
-                         reinterpret_cast<const void* const*>(indices_table.data_ptr<int64_t>()),
-                         num_nodes_table.data_ptr<int64_t>(), id_bytes, metapath.data_ptr<int64_t>(), L, seeds.data_ptr(), n, NextSeed(),
-                         nullptr, trace.data_ptr(), Stream(seeds)),
+  const int64_t relations = num_nodes_table.numel();
+  const size_t bytes = gs_metapath_walk_workspace_bytes(relations, num_nodes, n, L);
+  torch::Tensor ws;
+  if (bytes) ws = Scratch(bytes, seeds);
+  Check(gs_metapath_walk_workspace(reinterpret_cast<const int64_t* const*>(indptr_table.data_ptr<int64_t>()),
+                                   reinterpret_cast<const void* const*>(indices_table.data_ptr<int64_t>()),
+                                   num_nodes_table.data_ptr<int64_t>(), relations, num_nodes, id_bytes,
+                                   metapath.data_ptr<int64_t>(), L, seeds.data_ptr(), n, NextSeed(), nullptr,
+                                   trace.data_ptr(), bytes ? ws.data_ptr() : nullptr, bytes, Stream(seeds)),
         "gs_metapath_walk");
   return trace;
 }

@@ -221,7 +221,7 @@ torch::Tensor RandomWalk(const torch::Tensor& seeds, int64_t length, const torch
                          const torch::Tensor& indices);
 torch::Tensor MetapathWalk(const torch::Tensor& seeds, const torch::Tensor& metapath,
                            const torch::Tensor& indptr_table, const torch::Tensor& indices_table,
-                           const torch::Tensor& num_nodes_table, int id_bytes);
+                           const torch::Tensor& num_nodes_table, int64_t num_nodes, int id_bytes);
 
 struct Bcast {
   int64_t lhs_len, rhs_len, out_len, reduce_size;

@@ -659,6 +659,16 @@ int gs_metapath_walk(const int64_t* const* all_indptr, const void* const* all_in
                      int64_t length, const void* seeds, int64_t n, uint64_t seed,
                      const uint32_t* replay, void* trace, void* stream);
 
+/* The same with scratch memory, as gs_random_walk_workspace (workspace_bytes 0: no table).  num_relations:
+ * how many the arrays hold; num_nodes: their columns together. */
+size_t gs_metapath_walk_workspace_bytes(int64_t num_relations, int64_t num_nodes, int64_t n,
+                                        int64_t length);
+int gs_metapath_walk_workspace(const int64_t* const* all_indptr, const void* const* all_indices,
+                               const int64_t* all_num_nodes, int64_t num_relations, int64_t num_nodes,
+                               int id_bytes, const int64_t* metapath, int64_t length,
+                               const void* seeds, int64_t n, uint64_t seed, const uint32_t* replay,
+                               void* trace, void* workspace, size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------- */
 /* SDDMM: replaces impl::SDDMMCOO / impl::SDDMMCSC (src/cuda/sddmm.cu:280,263). */
 /* out[eid, k] = op(lhs[sel_l, lhs_off[k]], rhs[sel_r, rhs_off[k]]) with         */

@@ -216,3 +216,76 @@ def test_random_walk_at_the_line_of_packed_offsets(dev, less):
                            to_dev(seeds, dev, torch.int32), length, seed=9)
     want = O.random_walk(indptr, indices, seeds, length, seed=9)
     assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
+
+
+@pytest.mark.parametrize("idt", [torch.int32, torch.int64])
+@pytest.mark.parametrize("less_edges,less_walkers", [(0, 0), (1, 0), (0, 1)])
+def test_random_walk_at_the_lines_of_streams(dev, idt, less_edges, less_walkers):
+    """320 MB of neighbours and 120 000 walkers are read as streams, one edge or one walker less are not."""
+    E = (5 << 26) // (4 if idt == torch.int32 else 8) - less_edges
+    N, n = (E + 63) // 64, 120_000 - less_walkers
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(1)
+    indices = torch.randint(0, N, (E,), generator=gen, device=dev, dtype=idt)
+    indptr = np.minimum(np.arange(N + 1, dtype=np.int64) * 64, E)
+    seeds = np.random.default_rng(1).integers(0, N, n)
+    got = capi.random_walk(to_dev(indptr, dev), indices, to_dev(seeds, dev, idt), 6, seed=4, packed=False)
+    want = O.random_walk(indptr, indices.cpu().numpy().astype(np.int64), seeds, 6, seed=4)
+    assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
+
+
+@pytest.mark.parametrize("idt", [torch.int32, torch.int64])
+@pytest.mark.parametrize("path", [[0], [2, 1], [0, 1, 2, 1, 0]])
+@pytest.mark.parametrize("room", ["all", "two", "none"])
+def test_metapath_walk_with_packed_offsets(dev, idt, path, room):
+    """Records of three relations one behind the other, a hub in each; where they have no room the offsets
+    are read.  Relations of different sizes: walkers that leave one die."""
+    rng = np.random.default_rng(len(path))
+    sizes, hubs = [601, 7, 3000], [65536, 65535, 70000]
+    indptrs, indicess = [], []
+    for nodes, hub in zip(sizes, hubs):
+        degree = rng.integers(0, 9, nodes)
+        degree[3] = hub
+        indptrs.append(np.concatenate([[0], np.cumsum(degree)]).astype(np.int64))
+        indicess.append(rng.integers(0, rng.choice([7, 700]), indptrs[-1][-1]))
+    keep = _tables(indptrs, indicess, dev, idt)
+    seeds = np.concatenate([rng.integers(0, 3001, 700), [-1, 3, 3, 3]])
+    num_nodes = {"all": sum(sizes), "two": sizes[0] + sizes[1], "none": 0}[room]
+    got = capi.metapath_walk(keep[2], keep[3], keep[4], idt, to_dev(np.array(path), dev), to_dev(seeds, dev, idt),
+                             seed=8, num_nodes=num_nodes, packed=True)
+    want = O.metapath_walk(indptrs, indicess, np.array(path), seeds, seed=8)
+    assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
+
+
+def test_metapath_walk_replay(dev):
+    rels = [rmat_csc_np(1 << 11, 1 << 14, seed=s) for s in (1, 2)]
+    indptrs, indicess = [r[0] for r in rels], [r[1] for r in rels]
+    keep = _tables(indptrs, indicess, dev, torch.int64)
+    path, n = np.array([0, 1, 1, 0, 1, 0, 0]), 1000
+    seeds = np.random.default_rng(0).integers(0, 1 << 11, size=n).astype(np.int64)
+    replay = u32_draws(n * path.size, 5)
+    got = capi.metapath_walk(keep[2], keep[3], keep[4], torch.int64, to_dev(path, dev), to_dev(seeds, dev),
+                             replay=to_dev(replay, dev))
+    want = O.metapath_walk(indptrs, indicess, path, seeds, replay=replay)
+    assert np.array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("less", [0, 1])
+def test_metapath_walk_at_the_line_of_packed_offsets(dev, less):
+    """Two relations of 2^17 nodes, 2^17 walkers and twenty steps make tables, a walker less makes none."""
+    import ctypes
+    nodes, n, length = 1 << 17, (1 << 17) - less, 20
+    size = capi.lib().gs_metapath_walk_workspace_bytes
+    assert (size(*(ctypes.c_int64(v) for v in (2, 2 * nodes, n, length))) > 0) == (less == 0)
+    rng = np.random.default_rng(less)
+    indptrs, indicess = [], []
+    for _ in range(2):
+        degree = rng.integers(1, 6, nodes)
+        indptrs.append(np.concatenate([[0], np.cumsum(degree)]).astype(np.int64))
+        indicess.append(rng.integers(0, nodes, indptrs[-1][-1]))
+    keep = _tables(indptrs, indicess, dev, torch.int32)
+    path, seeds = np.array([0, 1] * 10), rng.integers(0, nodes, n)
+    got = capi.metapath_walk(keep[2], keep[3], keep[4], torch.int32, to_dev(path, dev),
+                             to_dev(seeds, dev, torch.int32), seed=9, num_nodes=2 * nodes)
+    want = O.metapath_walk(indptrs, indicess, path, seeds, seed=9)
+    assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
