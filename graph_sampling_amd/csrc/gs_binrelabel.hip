@@ -24,7 +24,7 @@
 //   rename    a pass in the order of the positions: the rank of an item's first position from
 //             mask + count; first occurrences write the frontier, ids their new name
 //
-// 17 M items in 64 batches: plan 4 us, tiles 39, first 117, rank 24, rename 71; counted, scanned
+// 17 M items in 64 batches: plan 4 us, tiles 40, first 104, rank 24, rename 66; counted, scanned
 // and scattered it was 43 + 9 + 92, first 99 and rename 86.  Batches of more than 2^20 items on average have so many
 // classes that a tile's runs are a few records; they are counted, the buckets laid out by a scan
 // and the records scattered to them, with a counter addition per (4096-item tile, class).
@@ -67,8 +67,8 @@ constexpr int counter_cap(int classes_log2) {
 }
 constexpr int kCounterCap = counter_cap(kMaxClassesLog2);
 // Batches of up to so many items on average go by tiles of runs: at 2^20 items a batch has 512
-// classes and a tile's runs 16 records, at 2^22 of 2048 classes 4.  By counting / by runs, us, ids
-// skewed like R-MAT's rows of 2^14 | 2^17 | 2^21 nodes:
+// classes and a tile's runs 16 records, at 2^22 of 2048 classes 4.  By counting / by runs (which are
+// read a tenth faster since), us, ids skewed like R-MAT's rows of 2^14 | 2^17 | 2^21 nodes:
 //    items a batch    one batch                      four
 //    2^19          59/58   53/42   51/37       81/68   79/58   80/55
 //    2^20          87/91   76/72   70/58      158/122 156/122 158/121
@@ -446,11 +446,9 @@ __device__ __forceinline__ void table_enter(unsigned long long* __restrict__ tab
 // the first position of the record's id
 // (a table that was too small may lack the id: what is returned then is read by nobody)
 __device__ __forceinline__ uint32_t table_first(const unsigned long long* __restrict__ tab,
-                                                unsigned long long rec) {
-  const uint32_t key = static_cast<uint32_t>(rec >> 32);
+                                                unsigned long long w, uint32_t key) {  // w: its slot
   uint32_t p = slot_of(key);
   int probes = 0;
-  unsigned long long w = tab[p];
   while (static_cast<uint32_t>(w >> 32) != key && ++probes < kSlots) {
     p = (p + 1) & (kSlots - 1);
     w = tab[p];
@@ -493,8 +491,10 @@ __global__ void __launch_bounds__(kBucketThreads) bins_first_kernel(Bins s, int6
     const int64_t r0 = begin + t * (kTrip * kBucketThreads);
 #pragma unroll
     for (int u = 0; u < kTrip; ++u)
-      if (r0 + u * kBucketThreads + threadIdx.x < end)
-        s.first[static_cast<uint32_t>(rec[u])] = table_first(tab, rec[u]);
+      if (r0 + u * kBucketThreads + threadIdx.x < end) {
+        const uint32_t key = static_cast<uint32_t>(rec[u] >> 32);
+        s.first[static_cast<uint32_t>(rec[u])] = table_first(tab, tab[slot_of(key)], key);
+      }
     if (t > 0) {
 #pragma unroll
       for (int u = 0; u < kTrip; ++u) rec[u] = s.records[r0 - (kTrip - u) * kBucketThreads + threadIdx.x];
@@ -507,8 +507,9 @@ __global__ void __launch_bounds__(kBucketThreads) bins_first_kernel(Bins s, int6
 // waves in turn, a piece a read.
 constexpr int kRunTrip = 16;  // pieces of a wave that are asked for together
 constexpr int kBucketWaves = kBucketThreads / kWave;
+constexpr int kLookTrip = 4;   // slots of a wave's lane that are looked up together
 
-__global__ void __launch_bounds__(kBucketThreads) bins_first_runs_kernel(Bins s, int64_t B) {
+__global__ void __launch_bounds__(kBucketThreads, 8) bins_first_runs_kernel(Bins s, int64_t B) {
   __shared__ unsigned long long tab[kSlots];
   const int64_t k = bucket_of_workgroup(s.plan.bucket_base[B]);
   if (k < 0) return;
@@ -517,7 +518,9 @@ __global__ void __launch_bounds__(kBucketThreads) bins_first_runs_kernel(Bins s,
   const uint4 at_bucket = s.plan.bucket[k];
   const int64_t tiles = at_bucket.z, row = at_bucket.y, first_item = at_bucket.w;
   const unsigned short* __restrict__ starts = s.run_start + at_bucket.x;
-  unsigned long long rec[kRunTrip];
+  // The records as they come: put together where they are used (put together here, every read waited for
+  // the one before: 17 M items 121 -> 104 us).
+  uint32_t id[kRunTrip], in_tile[kRunTrip];
   unsigned int held = 0u;  // which of them are records
   int start = 0, len = 0, ends = 0, pieces = 0;
   // the runs of the 64 tiles from t0 on
@@ -530,26 +533,27 @@ __global__ void __launch_bounds__(kBucketThreads) bins_first_runs_kernel(Bins s,
     ends = wave_inclusive_sum((len + kWave - 1) / kWave);
     pieces = __builtin_amdgcn_readlane(ends, kWave - 1);
   };
+  // the first position of the tile that piece p is of
+  const auto tile_of = [&](int64_t t0, int p) {
+    return static_cast<uint32_t>(first_item + (t0 + __popcll(__ballot(ends <= p))) * kTile);
+  };
   // the wave's pieces from number p0 on (in steps of the workgroup's waves)
   const auto read = [&](int64_t t0, int p0) {
     held = 0u;
 #pragma unroll
     for (int u = 0; u < kRunTrip; ++u) {
       const int p = p0 + u * kBucketWaves;
-      rec[u] = 0ull;
-      if (p < pieces) {
-        const int j = __popcll(__ballot(ends <= p));
-        const int run_len = __builtin_amdgcn_readlane(len, j);
-        const int before = __builtin_amdgcn_readlane(ends, j) - (run_len + kWave - 1) / kWave;
-        const int at = (p - before) * kWave + lane;
-        const int64_t tile_first = first_item + (t0 + j) * kTile;
-        if (at < run_len) {
-          const int64_t r = tile_first + __builtin_amdgcn_readlane(start, j) + at;
-          rec[u] = static_cast<unsigned long long>(s.run_id[r]) << 32 |
-                   static_cast<uint32_t>(tile_first + s.run_pos[r]);
-          held |= 1u << u;
-        }
-      }
+      if (p >= pieces) break;
+      const int j = __popcll(__ballot(ends <= p));
+      const int run_len = __builtin_amdgcn_readlane(len, j);
+      const int before = __builtin_amdgcn_readlane(ends, j) - (run_len + kWave - 1) / kWave;
+      const int at = (p - before) * kWave + lane;
+      const int64_t tile_at = first_item + (t0 + j) * kTile;
+      // (past the run's end its last record again)
+      const int64_t r = tile_at + __builtin_amdgcn_readlane(start, j) + (at < run_len ? at : run_len - 1);
+      id[u] = s.run_id[r];
+      in_tile[u] = s.run_pos[r];
+      if (at < run_len) held |= 1u << u;
     }
   };
   open(0);
@@ -562,8 +566,14 @@ __global__ void __launch_bounds__(kBucketThreads) bins_first_runs_kernel(Bins s,
     for (int p0 = wave; p0 < pieces; p0 += kRunTrip * kBucketWaves) {
       if (t0 > 0 || p0 > wave) read(t0, p0);
 #pragma unroll
-      for (int u = 0; u < kRunTrip; ++u)
-        if (held >> u & 1u) table_enter(tab, rec[u], s.error);
+      for (int u = 0; u < kRunTrip; ++u) {
+        if (p0 + u * kBucketWaves >= pieces) break;
+        const uint32_t tile_first = tile_of(t0, p0 + u * kBucketWaves);
+        uint32_t key = id[u];
+        asm volatile("" : "+v"(key));  // (the halves of a record side by side no earlier: 16 registers)
+        if (held >> u & 1u)
+          table_enter(tab, static_cast<unsigned long long>(key) << 32 | (tile_first + in_tile[u]), s.error);
+      }
     }
   }
   __syncthreads();
@@ -572,8 +582,18 @@ __global__ void __launch_bounds__(kBucketThreads) bins_first_runs_kernel(Bins s,
     for (int p0 = wave; p0 < pieces; p0 += kRunTrip * kBucketWaves) {
       if (!once) read(t0, p0);
 #pragma unroll
-      for (int u = 0; u < kRunTrip; ++u)
-        if (held >> u & 1u) s.first[static_cast<uint32_t>(rec[u])] = table_first(tab, rec[u]);
+      for (int u0 = 0; u0 < kRunTrip; u0 += kLookTrip) {
+        if (p0 + u0 * kBucketWaves >= pieces) break;
+        unsigned long long w[kLookTrip];
+#pragma unroll
+        for (int u = 0; u < kLookTrip; ++u) w[u] = tab[held >> (u0 + u) & 1u ? slot_of(id[u0 + u]) : 0u];
+#pragma unroll
+        for (int u = 0; u < kLookTrip; ++u) {
+          const uint32_t tile_first = tile_of(t0, p0 + (u0 + u) * kBucketWaves);
+          if (held >> (u0 + u) & 1u)
+            s.first[tile_first + in_tile[u0 + u]] = table_first(tab, w[u], id[u0 + u]);
+        }
+      }
     }
   }
 }
@@ -660,6 +680,7 @@ bins_rank_kernel(Bins s, int64_t M, int64_t B, const int64_t* __restrict__ seeds
 // consecutive positions go to one XCD one after the other: the ranks a batch looks up are a
 // few dozen kilobytes.
 constexpr int kRenameItems = 8;
+constexpr int kLoadsDone = 0x0F70;  // s_waitcnt vmcnt(0), the other counters as they are
 constexpr int kRenameTile = kThreads * kRenameItems;
 
 struct RenameShared {
@@ -720,7 +741,7 @@ bins_rename_kernel(BatchItems<IdT> x, int64_t M, Bins s, IdT* __restrict__ uniqu
 // The same where the batches are cut into tiles: four workgroups a tile, whose batch is found once
 // and not for every item.
 template <typename IdT>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kThreads, sizeof(IdT) == 8 ? 6 : 8)  // (what fits without spilling)
 bins_rename_runs_kernel(BatchItems<IdT> x, Bins s, IdT* __restrict__ unique,
                         IdT* __restrict__ out_ids, const int64_t* __restrict__ unique_ptr) {
   constexpr int kParts = kTile / kRenameTile;
@@ -749,17 +770,31 @@ bins_rename_runs_kernel(BatchItems<IdT> x, Bins s, IdT* __restrict__ unique,
   uint4 e[kRenameItems];
 #pragma unroll
   for (int u = 0; u < kRenameItems; ++u) e[u] = s.ranks[at[u] >> 6];
+  uint32_t rank[kRenameItems];
+#pragma unroll
+  for (int u = 0; u < kRenameItems; ++u) {
+    const unsigned long long m = static_cast<unsigned long long>(e[u].y) << 32 | e[u].x;
+    rank[u] = e[u].z + __popcll(m & ((1ull << (at[u] & 63u)) - 1ull));
+  }
+  // (the first occurrences' ids all asked for before one is written: 17 M items 68 -> 66 us, 4.5 M 16 -> 13,
+  // 0.9 M 6.9 -> 4.9)
+  IdT key[kRenameItems];
+#pragma unroll
+  for (int u = 0; u < kRenameItems; ++u) {
+    const int i = u * kThreads + static_cast<int>(threadIdx.x);
+    const int64_t off = from + i;
+    if (at[u] == first_item + i)
+      key[u] = *(off >= n_seeds ? x.ids + first_id + off - n_seeds : x.seeds + first_seed + off);
+  }
+  // (said once that all are there, or the stores, which are counted with the loads, wait for one another)
+  __builtin_amdgcn_s_waitcnt(kLoadsDone);
 #pragma unroll
   for (int u = 0; u < kRenameItems; ++u) {
     const int i = u * kThreads + static_cast<int>(threadIdx.x);
     if (i < n) {
-      const unsigned long long m = static_cast<unsigned long long>(e[u].y) << 32 | e[u].x;
-      const uint32_t rank = e[u].z + __popcll(m & ((1ull << (at[u] & 63u)) - 1ull));
       const int64_t off = from + i;
-      const bool is_id = off >= n_seeds;
-      if (at[u] == first_item + i)
-        unique[rank] = *(is_id ? x.ids + first_id + off - n_seeds : x.seeds + first_seed + off);
-      if (is_id) out_ids[first_id + off - n_seeds] = static_cast<IdT>(rank - frontier);
+      if (at[u] == first_item + i) unique[rank[u]] = key[u];
+      if (off >= n_seeds) out_ids[first_id + off - n_seeds] = static_cast<IdT>(rank[u] - frontier);
     }
   }
 }
