@@ -1802,25 +1802,23 @@ bin_sum_kernel(SumSpace s, int64_t tiles, int64_t alone, int64_t part_items, Bin
     const int ends = wave_inclusive_sum((len + kWave - 1) / kWave);
     const int pieces = __builtin_amdgcn_readlane(ends, kWave - 1);
     for (int p0 = 0; p0 < pieces; p0 += kSumTrip) {
+      // (no read under a condition of its own, past the run's end its last edge again: a place that might be
+      // none was cut to its 16 bits at once, and so waited for before the next read was asked for: 1.0 M edges
+      // 26 -> 22 us)
       float v[kSumTrip];
-      unsigned short at[kSumTrip];
+      uint32_t at[kSumTrip];
       unsigned int held = 0u;
 #pragma unroll
       for (int u = 0; u < kSumTrip; ++u) {
-        v[u] = 0.0f;
-        at[u] = 0;
-        if (p0 + u < pieces) {
-          const int j = __popcll(__ballot(ends <= p0 + u));
-          const int run = __builtin_amdgcn_readlane(len, j);
-          const int i = (p0 + u - (__builtin_amdgcn_readlane(ends, j) - (run + kWave - 1) / kWave)) * kWave + lane;
-          if (i < run) {
-            const int64_t from = (t0 + static_cast<int64_t>(j) * kOneWaves) * kSumTile +
-                                 __builtin_amdgcn_readlane(start, j) + i;
-            v[u] = s.value[from];
-            at[u] = s.place[from];
-            held |= 1u << u;
-          }
-        }
+        if (p0 + u >= pieces) break;
+        const int j = __popcll(__ballot(ends <= p0 + u));
+        const int run = __builtin_amdgcn_readlane(len, j);
+        const int i = (p0 + u - (__builtin_amdgcn_readlane(ends, j) - (run + kWave - 1) / kWave)) * kWave + lane;
+        const int64_t from = (t0 + static_cast<int64_t>(j) * kOneWaves) * kSumTile +
+                             __builtin_amdgcn_readlane(start, j) + (i < run ? i : run - 1);
+        v[u] = s.value[from];
+        at[u] = s.place[from];
+        if (i < run) held |= 1u << u;
       }
 #pragma unroll
       for (int u = 0; u < kSumTrip; ++u)
