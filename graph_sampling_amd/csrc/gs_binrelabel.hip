@@ -680,7 +680,6 @@ bins_rank_kernel(Bins s, int64_t M, int64_t B, const int64_t* __restrict__ seeds
 // consecutive positions go to one XCD one after the other: the ranks a batch looks up are a
 // few dozen kilobytes.
 constexpr int kRenameItems = 8;
-constexpr int kLoadsDone = 0x0F70;  // s_waitcnt vmcnt(0), the other counters as they are
 constexpr int kRenameTile = kThreads * kRenameItems;
 
 struct RenameShared {

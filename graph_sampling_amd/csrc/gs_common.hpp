@@ -278,6 +278,11 @@ __device__ __forceinline__ float lane_move(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, bits, CTRL, 0xf, 0xf, false));
 }
 
+// For __builtin_amdgcn_s_waitcnt: vmcnt(0), the other counters as they are.  Loads and stores are counted
+// together; where reads were asked for under conditions the compiler cannot tell how many are under
+// way, and waits for the stores issued since with every use.  Said once that all reads are there, the stores wait for nothing.
+constexpr int kLoadsDone = 0x0F70;
+
 // ------------------------------------------------------------ block scan ----
 // Exclusive scan of one int64 per thread over a block of kThreads threads
 // (multiple of 64).  Returns the exclusive prefix; *total gets the block sum.
