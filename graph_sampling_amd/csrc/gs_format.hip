@@ -415,6 +415,7 @@ struct SortTile {
   static constexpr int kPerThread = PER_THREAD;
   static constexpr int kSize = THREADS * PER_THREAD;
   static constexpr int kWaves = THREADS / kWave;
+  static constexpr bool kStreams = THREADS > 256;  // reads past the caches (packed_pass_kernel)
 };
 using SmallTile = SortTile<256, 16>;
 using LargeTile = SortTile<1024, 8>;
@@ -746,8 +747,11 @@ radix_pass_kernel(Src src, const ValT* __restrict__ val_in, int64_t E, int shift
 // `wide`.  The next pass's digits are written beside the words, for its histogram to read a byte an edge.
 // 14 M edges, 22-bit keys (24 bits each for value and position): the passes 72 + 65 + 82 us with the
 // values beside the words, 67 + 59 + 81 so; the last two histograms 24 -> 8 each.
-// What a pass reads, nothing reads again, so it reads past the caches (14 M edges with 64-bit ids, loaded
-// and sorted: 420 -> 415 us; 11 M / 8 M with 32-bit ids 322 -> 301, 290 -> 277).  The words it writes are the next
+// What a pass of large tiles reads, nothing reads again before it has left the caches, so it reads past them (14 M
+// edges with 64-bit ids, loaded and sorted: 420 -> 415 us; 11 M / 8 M with 32-bit ids 322 -> 301, 290 -> 277).  Up to
+// 4 M edges (small tiles) the lists and the words stay in the L2s, plain / past the caches, lists loaded and sorted again
+// and again: 2.3 M edges, 64-bit ids 136/140 us, 4.0 M 183/189, 32-bit ids 174/178; 6.1 M 223/208, 193/191.
+// The words it writes are the next
 // pass's: written past the caches they cost 456.  The last pass's results go past them where they
 // fill more than half of the memory-side cache (14 M: 415 -> 404, 11 M: 301 -> 290; 8 M, 128 MB: 277, 278).
 constexpr int kPackedPasses = 3;
@@ -788,6 +792,7 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
   const int digit = threadIdx.x;  // of the first 256 threads
   // (a value that did not fit its bits, met by the first pass: they are all fetched again)
   const bool refetch = LAST && *last.wide != 0;
+  auto once = [](const auto* p) { return T::kStreams ? __builtin_nontemporal_load(p) : *p; };
   int64_t all = 0, before_tile = 0;
   uint32_t ends = 0;
   if (digit < kRadix) {
@@ -806,9 +811,9 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
   for (int r = 0; r < kItemsHere; ++r) {
     const uint32_t j = mine0 + r * kWave;
     if constexpr (FIRST)
-      fresh[r] = static_cast<uint32_t>(__builtin_nontemporal_load(key + base + (j < n ? j : n - 1)));
+      fresh[r] = static_cast<uint32_t>(once(key + base + (j < n ? j : n - 1)));
     else
-      word[r] = __builtin_nontemporal_load(in + base + (j < n ? j : n - 1));
+      word[r] = once(in + base + (j < n ? j : n - 1));
   }
   // (what lies behind the last edge takes the last digit, as above)
 #pragma unroll
@@ -862,7 +867,7 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
 #pragma unroll
     for (int r = 0; r < kItemsHere; ++r) {
       const uint32_t j = again0 + r * kWave;
-      raw[r] = __builtin_nontemporal_load(tile_val + (j < n ? j : n - 1));
+      raw[r] = once(tile_val + (j < n ? j : n - 1));
     }
   }
   lds_barrier();
