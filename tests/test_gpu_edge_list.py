@@ -110,6 +110,28 @@ def test_sort_with_the_values_in_its_words(dev, num_keys, skew, E, idt):
 
 
 @pytest.mark.parametrize("idt", ID_DTYPES)
+@pytest.mark.parametrize("less", [0, 1])
+@pytest.mark.parametrize("num_keys", [60_000, 3_000_000])
+def test_sort_with_long_results(dev, num_keys, less, idt):
+    """Results of 128 MB and of an edge less, by two digits and by three: the last pass writes the longer ones past
+    the caches, and fetches values again where one does not fit its bits."""
+    edge = 8 + 4 + (4 if idt == torch.int32 else 8)  # position, key and value
+    E = -(-(1 << 27) // edge) - less
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(num_keys)
+    key = (torch.rand(E, generator=gen, device=dev, dtype=torch.float64) ** 3 * num_keys).to(idt)
+    value = torch.randint(0, num_keys, (E,), generator=gen, device=dev).to(idt)
+    want = torch.sort(key, stable=True).indices
+    ends = torch.cumsum(torch.bincount(key.long(), minlength=num_keys), 0)
+    # (two digits leave 32 bits for a value of 23-bit positions, three leave 25, or 24 beside 24-bit positions)
+    for wide in [0, (1 << 31) - 1] + ([1 << 40] if idt == torch.int64 else []):
+        value[E // 3] = wide
+        ip, val, perm = capi.coo2csc(key, value, num_keys, False)
+        assert torch.equal(perm, want) and torch.equal(val, value[want])
+        assert int(ip[0]) == 0 and torch.equal(ip[1:], ends)
+
+
+@pytest.mark.parametrize("idt", ID_DTYPES)
 @pytest.mark.parametrize("num_keys", [60_000, 65_537])
 def test_sort_of_values_unlike_the_keys(dev, num_keys, idt):
     """Values below a bound that the caller knows, with two digits of the key (which leave them all 32
