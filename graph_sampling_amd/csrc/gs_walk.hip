@@ -22,22 +22,46 @@ namespace {
 
 constexpr int kThreads = 256;
 
-// Neighbour arrays from this size on are read as streams (the line is the first to leave the
-// L2) by walkers enough: hardly one of their lines is met again, and the offsets, which are, stay
-// longer.  Arrays that the L2s and the memory-side cache hold in good part lose by it, and so
-// do few walkers, and all with a packed table of the offsets (below), which stays without it: 1 M walkers, 80 steps,
-// 4 M nodes of 50 edges 1237 us plain, 1455 as a stream.  Without a table, 38 steps, plain / as a stream, us, by walkers:
-//                               66 k       131 k       400 k       1 M
-//   280 MB (70 M edges, 32-bit)   42/55        77/73      249/245     569/577
-//   400 MB (100 M, 32-bit)        47/57        88/82      281/272     653/644
-//   720 MB (90 M, 64-bit)         53/59        91/84      284/275     669/663
-//   800 MB (200 M, 32-bit)        53/60        93/87      295/284     685/670
-//   1.1 GB (139 M, 64-bit)        49/56        88/82      281/270     650/650
+// Neighbour arrays from this size on, of so many nodes, are read as streams (the line is the first to
+// leave the L2) by walkers enough: hardly one of their lines is met again, and the offsets, which are, stay
+// longer.  Arrays that the L2s and the memory-side cache hold in good part lose by it, and so do few
+// walkers, and graphs of few nodes, however long their lists: the offsets need no room there, and the hubs' lists are
+// met again.  With a packed table of the offsets (below) arrays are read plainly.  R-MAT graphs, 32-bit ids, plain / as a
+// stream, us, by walkers x steps:
+//                                 131 k x 10   131 k x 30   300 k x 8   300 k x 30   1 M x 4   1 M x 80
+//   0.13 M nodes x 492 (258 MB)     27.5/32.2    78/93        49/64       178/233      80/105   1467/2039
+//   0.13 M x 700 (367 MB)           28.6/32.1    80/94        51/64       183/237      82/106   1482/2084
+//   0.23 M x 492 (459 MB)           29.1/32.0    81/94        52/64       184/235      87/106   1501/2058
+//   0.5 M x 360 (720 MB)            30.2/30.7    81/92        55/62       187/228      93/104   1563/1995
+//   1 M x 100 (419 MB)              28.0/28.0    76/82        51/55       174/194      90/92    1387/1650
+//   1 M x 250 (1.0 GB)              30.7/29.4    82/90        56/59       192/217      98/101   1630/1901
+//   2.1 M x 25 (210 MB)             23.2/23.9                 42/43       134/139      77/75    1005/1087
+//   2.1 M x 50 (419 MB)             26.9/25.7                 49/49       162/169      88/84    1306/1374
+//   2.1 M x 100 (839 MB)            29.8/27.7                 54/53       184/191      97/92    1514/1627
+//   4.2 M x 25 (419 MB)             24.8/24.0                 45/43       142/138      83/78    1048/1062
+//   4.2 M x 50 (839 MB)             28.5/27.3                 52/48       170/165      93/86    1321/1344
+//   8.4 M x 16 (537 MB)             23.3/22.5                 42/40                    78/74     888/858
+//   16.8 M x 16 (1.1 GB)            24.6/23.4                 46/43                    82/77    1021/856
+// (most of the long walks of the last column have a table).  66 k walkers, 30 steps: 2.4 M nodes of 35 edges
+// 46.6/48.8, 1 M nodes of 80 48.2/50.9.  64-bit ids: 0.23 M nodes x 492 (917 MB), 300 k x 30 204/241, 4 M x 25 (839 MB)
+// 154/142.
 constexpr int64_t kStreamBytes = int64_t(5) << 26;
-constexpr int64_t kStreamWalkers = 120'000;  // (the line lies between 66 and 131 k; 131 k is on the winning side)
-// The same for a relation of a metapath, when the path has two such: three of 400 MB, 20 steps, 200 k
-// walkers 84 -> 83 us, 30 steps, 1 M walkers 516 -> 496.
+constexpr int64_t kStreamNodes = int64_t(1) << 21;
+constexpr int64_t kStreamWalkers = 120'000;
+// The same for a relation of a metapath, when the path has two such (of half as many nodes: they share the L2s),
+// by any number of walkers.  Three relations, 32-bit ids, plain / as streams, us:
+//                                  50 k x 64   100 k x 40   131 k x 30   400 k x 8   1 M x 4   1 M x 10
+//   0.3 M nodes x 250 (300 MB)       85/94        99/110                    79/88
+//   1 M x 80 (335 MB)                80/80        86/93        82/82        72/74      94/92
+//   1 M x 160 (671 MB)               86/84        98/99        88/88        79/79     103/98
+//   2.1 M x 50 (419 MB)              80/78        82/81        79/74        71/70      91/87     205/195
+//   4.2 M x 25 (419 MB)              77/75        68/67        70/65        67/65      89/85     191/176
+// and a path over one relation alone, which takes the line above:
+//   1 M x 80 (335 MB)                69/80        75/92                     68/75
+//   2.1 M x 50 (419 MB)              71/77        73/80        70/73        68/69      88/85
+//   4.2 M x 25 (419 MB)              70/74        63/67        63/60        63/61      84/78     175/166
 constexpr int64_t kStreamRelationBytes = int64_t(256) << 20;
+constexpr int64_t kStreamRelationNodes = int64_t(1) << 20;
 // A metapath's relations have to be looked up for it in front of the first step, which only long work earns
 // back: three of 400 MB, 64-bit / 32-bit ids, 131 k walkers, 30 steps 71 -> 66 / 72 -> 66 us, 1 M walkers, 4 steps
 // 87 -> 85 / 87 -> 83, but 200 k walkers, 10 steps 42.6 -> 44.5 / 42 -> 43, 18 k walkers, 30 steps 28 -> 34 / 31 -> 37.
@@ -201,7 +225,7 @@ random_walk_kernel(const int64_t* __restrict__ indptr, const uint4* __restrict__
   const int64_t w = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
   if (w >= n) return;
   int64_t curr = static_cast<int64_t>(seeds[w]);
-  const bool stream = !PACKED && n >= kStreamWalkers &&
+  const bool stream = !PACKED && n >= kStreamWalkers && num_nodes >= kStreamNodes &&
                       indptr[num_nodes] >= kStreamBytes / static_cast<int64_t>(sizeof(IdT));
   U4 x;
   for (int64_t t = 0; t < length; ++t) {
@@ -291,11 +315,13 @@ metapath_walk_kernel(const int64_t* const* __restrict__ all_indptr,
     if (LONG_WORK && (t & (kWave - 1)) == 0) {  // a lane per step of the next 64
       const int64_t step = t + (threadIdx.x & (kWave - 1));
       const int64_t rel = metapath[step < length ? step : length - 1];
-      const int64_t bytes = all_indptr[rel][all_num_nodes[rel]] * static_cast<int64_t>(sizeof(IdT));
-      const unsigned long long large = __ballot(bytes >= kStreamRelationBytes);
+      const int64_t nodes = all_num_nodes[rel];
+      const int64_t bytes = all_indptr[rel][nodes] * static_cast<int64_t>(sizeof(IdT));
+      const bool one_of_two = bytes >= kStreamRelationBytes && nodes >= kStreamRelationNodes;
+      const unsigned long long large = __ballot(one_of_two);
       const int64_t one = __shfl(rel, large ? __ffsll(static_cast<long long>(large)) - 1 : 0, kWave);
-      const bool two = __ballot(bytes >= kStreamRelationBytes && rel != one) != 0ull;
-      streams = two ? large : __ballot(bytes >= kStreamBytes);
+      const bool two = __ballot(one_of_two && rel != one) != 0ull;
+      streams = two ? large : __ballot(n >= kStreamWalkers && bytes >= kStreamBytes && nodes >= kStreamNodes);
     }
     const bool alive = static_cast<uint64_t>(curr) < static_cast<uint64_t>(here.num_nodes);
     Offsets<PACKED> off;

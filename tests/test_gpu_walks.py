@@ -126,9 +126,9 @@ def test_walk_out_of_range_seeds_die(dev):
 
 @pytest.mark.parametrize("idt", [torch.int32, torch.int64])
 @pytest.mark.parametrize("less", [0, 1])
-def test_walks_over_neighbour_arrays_read_as_streams(dev, idt, less):
+def test_few_walkers_over_large_neighbour_arrays(dev, idt, less):
     """Neighbour arrays of 256 MB and of one edge less, alone and as one relation beside a small one,
-    over more than 64 steps; each node has 64 neighbours, the last fewer."""
+    over more than 64 steps; each node has 64 neighbours, the last fewer.  (Too few walkers for streams.)"""
     E = (1 << 28) // (4 if idt == torch.int32 else 8) - less
     N = (E + 63) // 64
     rng = np.random.default_rng(less)
@@ -148,30 +148,42 @@ def test_walks_over_neighbour_arrays_read_as_streams(dev, idt, less):
     assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
 
 
+def _even_offsets(nodes, edges):
+    return np.arange(nodes + 1, dtype=np.int64) * edges // nodes
+
+
 @pytest.mark.parametrize("idt", [torch.int32, torch.int64])
-@pytest.mark.parametrize("less", [0, 1])
-def test_walks_over_a_neighbour_array_read_as_a_stream(dev, idt, less):
-    """A neighbour array of 640 MB, from which on it is read as a stream, and of one edge less."""
-    E = (5 << 27) // (4 if idt == torch.int32 else 8) - less
-    N = (E + 63) // 64
-    indptr = np.minimum(np.arange(N + 1, dtype=np.int64) * 64, E)
-    indices = np.random.default_rng(less).integers(0, N, E, dtype=np.int64)
-    seeds = np.random.default_rng(3).integers(0, N, 300)
-    got = capi.random_walk(to_dev(indptr, dev), to_dev(indices, dev, idt), to_dev(seeds, dev, idt), 9,
-                           seed=5)
-    want = O.random_walk(indptr, indices, seeds, 9, seed=5)
+@pytest.mark.parametrize("less_edges,less_walkers,less_nodes", [(0, 0, 0), (1, 0, 0), (0, 1, 0), (0, 0, 1)])
+def test_long_metapath_work_over_one_large_relation(dev, idt, less_edges, less_walkers, less_nodes):
+    """A path's only large relation is read as a stream from 320 MB of neighbours, 2^21 nodes and
+    120 000 walkers on; a small relation beside it is not."""
+    E = (5 << 26) // (4 if idt == torch.int32 else 8) - less_edges
+    N, n = (1 << 21) - less_nodes, 120_000 - less_walkers
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(1)
+    indices = torch.randint(0, N, (E,), generator=gen, device=dev, dtype=idt)
+    rng = np.random.default_rng(1)
+    small_ix = rng.permutation(N)
+    indptr, small_ptr = _even_offsets(N, E), np.arange(N + 1, dtype=np.int64)
+    keep = _tables([indptr, small_ptr], [np.zeros(1, np.int64), small_ix], dev, idt)
+    keep[3][0] = indices.data_ptr()
+    seeds, path = rng.integers(0, N, n), np.array([0, 0, 1] * 9, dtype=np.int64)  # 3.24 M steps: long work
+    got = capi.metapath_walk(keep[2], keep[3], keep[4], idt, to_dev(path, dev), to_dev(seeds, dev, idt), seed=6)
+    want = O.metapath_walk([indptr, small_ptr], [indices.cpu().numpy().astype(np.int64), small_ix], path, seeds,
+                           seed=6)
     assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
 
 
-# 67 steps of each: 2**22 in all, less 37 and more 30
-@pytest.mark.parametrize("walkers,relations", [(62_601, 2), (62_602, 2), (62_602, 1)])
-def test_long_metapath_work_over_streams(dev, walkers, relations):
-    """From 2**22 steps in all, the neighbour arrays of a metapath's relations are read as streams
-    when two of them are large."""
-    E = (1 << 28) // 4
-    N = E // 64
+# 67 steps of each: 3 * 2**20 in all, less 11 and more 56
+@pytest.mark.parametrize("walkers,relations,less_edges,less_nodes",
+                         [(46_951, 2, 0, 0), (46_952, 2, 0, 0), (46_952, 1, 0, 0), (46_952, 2, 1, 0),
+                          (46_952, 2, 0, 1)])
+def test_long_metapath_work_over_streams(dev, walkers, relations, less_edges, less_nodes):
+    """From 3 * 2**20 steps in all, the neighbour arrays of a metapath's relations are read as streams
+    when two of them have 256 MB and 2^20 nodes."""
+    E, N = (1 << 28) // 4 - less_edges, (1 << 20) - less_nodes
     rng = np.random.default_rng(walkers)
-    ptr, small_ptr = np.arange(N + 1, dtype=np.int64) * 64, np.arange(N + 1, dtype=np.int64)
+    ptr, small_ptr = _even_offsets(N, E), np.arange(N + 1, dtype=np.int64)
     indices = [rng.integers(0, N, E).astype(np.int32) for _ in range(relations)]
     small_ix = rng.permutation(N).astype(np.int32)
     seeds = rng.integers(0, N, walkers)
@@ -219,15 +231,15 @@ def test_random_walk_at_the_line_of_packed_offsets(dev, less):
 
 
 @pytest.mark.parametrize("idt", [torch.int32, torch.int64])
-@pytest.mark.parametrize("less_edges,less_walkers", [(0, 0), (1, 0), (0, 1)])
-def test_random_walk_at_the_lines_of_streams(dev, idt, less_edges, less_walkers):
-    """320 MB of neighbours and 120 000 walkers are read as streams, one edge or one walker less are not."""
+@pytest.mark.parametrize("less_edges,less_walkers,less_nodes", [(0, 0, 0), (1, 0, 0), (0, 1, 0), (0, 0, 1)])
+def test_random_walk_at_the_lines_of_streams(dev, idt, less_edges, less_walkers, less_nodes):
+    """320 MB of neighbours, 2^21 nodes and 120 000 walkers are read as streams, one of any less is not."""
     E = (5 << 26) // (4 if idt == torch.int32 else 8) - less_edges
-    N, n = (E + 63) // 64, 120_000 - less_walkers
+    N, n = (1 << 21) - less_nodes, 120_000 - less_walkers
     gen = torch.Generator(device=dev)
     gen.manual_seed(1)
     indices = torch.randint(0, N, (E,), generator=gen, device=dev, dtype=idt)
-    indptr = np.minimum(np.arange(N + 1, dtype=np.int64) * 64, E)
+    indptr = _even_offsets(N, E)
     seeds = np.random.default_rng(1).integers(0, N, n)
     got = capi.random_walk(to_dev(indptr, dev), indices, to_dev(seeds, dev, idt), 6, seed=4, packed=False)
     want = O.random_walk(indptr, indices.cpu().numpy().astype(np.int64), seeds, 6, seed=4)
