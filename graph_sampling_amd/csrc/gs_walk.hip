@@ -114,10 +114,48 @@ constexpr int kRecordNodes = 6;
 //     2 M           110/101       52/51       100/93       346/307       80/73       174/156      1140/989
 //     8 M            93/103       50/62        91/99       286/281       76/86       157/162       954/869
 //    16 M            98/120       54/77        96/115      303/308       81/102      167/180       965/904
+// The more nodes, the more walkers a table wants, however many steps they take (table_walkers); 16 edges a node, the
+// steps from where the line lies, and twice as many:
+//                  131 k walkers          300 k                500 k                1 M                  4 M
+//     4.2 M        112/120 (25 edges)    138/134 (x 30)
+//     8.4 M        152/188               176/188, 296/306     198/207, 345/349     209/221, 380/367     279/272, 464/455
+//    16.8 M        256/349               294/307, 452/476     335/346, 551/548     371/367, 646/613     461/434, 806/754
+//    33.6 M                              467/505, 687/774     573/563, 852/831     669/651, 1087/1025   845/782, 1481/1340
+//    67 M                                697/853, 1084/1296   867/908, 1197/1284   1117/1121, 1669/1650 1445/1394, 2594/2418
+// and graphs of more nodes than that want their walks not to end early: 111 M nodes of 8 edges 915/1131 us by 1 M
+// walkers, 1551/1733 by 4 M, of 14 edges 1589/1529, 2419/2200 (kWideNodes, kWideDegree; no larger one was measured).
+// A record with a hub among its nodes costs three reads one behind the other, and in dense graphs of many
+// edges many steps meet one.  As above, by edges a node (kDenseEdges, kDenseDegree):
+//                        131 k x 30   300 k x 30    1 M x 4     1 M x 8     1 M x 80
+//   262 k nodes x 250      76/75        172/167      82/78       160/151     1428/1346
+//   262 k x 492            80/82        183/181      87/82       165/157     1485/1482
+//   262 k x 600            80/86        185/192      87/85       164/164     1542/1584
+//   262 k x 1000           87/96        208/220      90/95       180/189     1798/1869
+//   524 k x 300            80/83        183/182      91/83       170/157     1528/1476
+//   524 k x 492            85/94        202/211      94/92       176/181     1725/1768
+//     1 M x 160            80/81        183/174      95/84       173/155     1460/1396
+//     1 M x 250            82/90        192/199      98/91       178/173     1630/1646
+//     1 M x 320            86/95        204/212      99/95       181/185     1739/1774
+//     1 M x 492            92/102       219/230     102/101      192/200     1898/1944
+//   2.1 M x 200           114/122       209/208                  189/184     1823/1719
+//   2.1 M x 300           118/132       218/224                  196/197     1911/1875
+//   4.2 M x 200           182/198       205/217                  209/218     1797/1788
+constexpr int64_t kMostNodes = int64_t(1) << 27, kWideNodes = int64_t(1) << 26, kWideDegree = 12;
+constexpr int64_t kDenseEdges = int64_t(1) << 27, kDenseDegree = 320;
+
+// a walker for so many nodes, 2^17 at the least; a million are enough for any
+inline int64_t table_walkers(int64_t num_nodes, int64_t nodes_a_walker) {
+  const int64_t n = num_nodes / nodes_a_walker < 1'000'000 ? num_nodes / nodes_a_walker : 1'000'000;
+  return n > (int64_t(1) << 17) ? n : int64_t(1) << 17;
+}
+inline bool steps_pay(int64_t num_nodes, int64_t n, int64_t length) {
+  return length > 0 && n > ((int64_t(1) << 21) + num_nodes * 3 / 2 - 1) / length;
+}
 bool packed_pays(int64_t num_nodes, int64_t nnz, int64_t n, int64_t length) {
-  return num_nodes >= (int64_t(1) << 18) && num_nodes < (int64_t(1) << 32) && nnz < (int64_t(1) << 32) &&
-         n >= (int64_t(1) << 17) && length > 0 &&
-         n >= ((int64_t(1) << 21) + num_nodes * 3 / 2 + length - 1) / length;
+  return num_nodes >= (int64_t(1) << 18) && num_nodes <= kMostNodes && nnz < (int64_t(1) << 32) &&
+         (num_nodes <= kWideNodes || nnz >= kWideDegree * num_nodes) &&
+         (nnz < kDenseEdges || nnz < kDenseDegree * num_nodes) && n >= table_walkers(num_nodes, 16) &&
+         steps_pay(num_nodes, n, length);
 }
 // The same for a metapath; num_nodes: of all relations together, which are packed whether the path takes them or not
 // (few of them: a record's thread goes through them in turn).  Offsets as they are / table, us, three relations:
@@ -129,10 +167,19 @@ bool packed_pays(int64_t num_nodes, int64_t nnz, int64_t n, int64_t length) {
 //   2 M, 20 M                  32/40        55/62        77/84       109/109      68/70     145/139    363/326
 //   2 M, 50 M, 64-bit ids      43/52        83/91       116/119      146/150      85/91     181/183    496/465
 //   4 M, 100 M                 42/63        80/98       110/128      143/157      83/101    179/192    471/466
+// A walker for every 32 nodes, the steps from where the line lies, and twice as many:
+//                            131 k             200 k             300 k             500 k             1 M
+//   2.1 M, 25 M              116/135, 205/233  144/146, 222/219  142/143, 235/226  161/157, 282/262  174/168, 313/292
+//   2.1 M, 52 M              166/183, 277/320  200/192, 351/319  190/188, 343/312  205/194, 377/345  217/200, 408/361
+//   4.2 M, 50 M              205/260, 360/434  222/235, 349/380  231/235, 359/356  274/263, 448/418  294/288, 522/486
+//   4.2 M, 105 M             249/308, 427/535  309/317, 493/506  302/317, 510/517  326/337, 586/561  347/343, 632/606
+//   8.4 M, 67 M              314/405, 543/654  282/352, 459/555  268/317, 432/492  320/358, 449/506  390/426, 606/644
+//   8.4 M, 134 M             372/492, 653/807  381/443, 617/708  398/439, 592/650  475/486, 731/734  533/545, 914/900
+// (from 400 MB a relation on, as streams).  No more nodes were measured.
+constexpr int64_t kMostRelationNodes = int64_t(1) << 25;
 bool packed_relations_pay(int64_t num_relations, int64_t num_nodes, int64_t n, int64_t length) {
   return num_relations > 0 && num_relations <= 16 && num_nodes >= (int64_t(1) << 18) &&
-         num_nodes < (int64_t(1) << 34) && n >= (int64_t(1) << 17) && length > 0 &&
-         n >= ((int64_t(1) << 21) + num_nodes * 3 / 2 + length - 1) / length;
+         num_nodes <= kMostRelationNodes && n >= table_walkers(num_nodes, 32) && steps_pay(num_nodes, n, length);
 }
 size_t tables_bytes(int64_t num_relations, int64_t num_nodes) {
   return padded(static_cast<size_t>(num_relations) * 8) +

@@ -72,3 +72,40 @@ def test_every_entry_point_names_what_it_replaces():
         if not re.search(r"(src/|examples/|tests/|python/)[A-Za-z_/\.]+:\d+|counterpart", above, re.I):
             uncited.append(m.group(2))
     assert not uncited, uncited
+
+
+def test_walks_make_a_table_of_offsets_where_it_pays():
+    """Both sides of every line of the rule: nodes, walkers, walkers for the nodes, steps, edges a node (dense graphs,
+    whose hubs' records cost more than they save, and large graphs whose walks end early)."""
+    from graph_sampling_amd import capi
+
+    def made(nodes, edges, walkers, length):
+        return capi.lib().gs_random_walk_workspace_bytes(*(ctypes.c_int64(v) for v in (nodes, edges, walkers, length))) > 0
+
+    k, M = 1 << 10, 1 << 20
+    for yes, no in [((256 * k, 4 * M, 128 * k, 20), (256 * k - 1, 4 * M, 128 * k, 20)),
+                    ((256 * k, 4 * M, 128 * k, 20), (256 * k, 4 * M, 128 * k - 1, 21)),
+                    ((M, 20 * M, M, 4), (M, 20 * M, M, 3)),  # 2^21 + 1.5 * 2^20 steps
+                    ((4 * M, 100 * M, 256 * k, 40), (4 * M, 100 * M, 256 * k - 1, 40)),  # a walker for 16 nodes
+                    ((8 * M, 80 * M, 512 * k, 30), (8 * M, 80 * M, 300_000, 200)),
+                    ((64 * M, 800 * M, 1_000_000, 120), (64 * M, 800 * M, 999_999, 400)),
+                    ((64 * M, 64 * 8 * M, M, 120), (64 * M + 1, 64 * 8 * M, M, 120)),
+                    ((111_000_000, 1_600_000_000, M, 200), (111_000_000, 900_000_000, M, 200)),
+                    ((128 * M, 128 * 12 * M, M, 200), (128 * M + 1, 128 * 16 * M, M, 200)),
+                    ((256 * k, 128 * M - 1, M, 80), (256 * k, 128 * M, M, 80)),  # 512 edges a node
+                    ((M, 320 * M - 1, M, 80), (M, 320 * M, M, 80)),
+                    ((4 * M, 200 * M, M, 80), (4 * M, 4096 * M, M, 80))]:
+        assert made(*yes) and not made(*no), (yes, no)
+    assert not made(M, 20 * M, M, 0) and not made(0, 0, M, 4) and not made(M, 20 * M, 0, 80)
+
+    def metapath(relations, nodes, walkers, length):
+        return capi.lib().gs_metapath_walk_workspace_bytes(*(ctypes.c_int64(v) for v in (relations, nodes, walkers, length))) > 0
+
+    for yes, no in [((3, 256 * k, 128 * k, 20), (3, 256 * k - 1, 128 * k, 20)),
+                    ((16, M, 200_000, 20), (17, M, 200_000, 20)),
+                    ((3, 4 * M, 128 * k, 80), (3, 4 * M + 32, 128 * k, 80)),  # a walker for 32 nodes
+                    ((3, 32 * M, 1_000_000, 80), (3, 32 * M, 999_999, 80)),
+                    ((3, 32 * M, M, 80), (3, 32 * M + 1, M, 80)),
+                    ((1, M, M, 4), (1, M, M, 3))]:
+        assert metapath(*yes) and not metapath(*no), (yes, no)
+    assert not metapath(0, M, M, 80)
