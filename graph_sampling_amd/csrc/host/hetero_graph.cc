@@ -1,4 +1,7 @@
 #include "hetero_graph.h"
+
+#include <algorithm>
+
 #include "range.h"
 
 #include "hip_ops.h"
@@ -16,9 +19,7 @@ void HeteroGraph::LoadFromHomo(
   relations_ = edge_relations;
   metapath_cache_.clear();
   for (size_t i = 0; i < node_types.size(); ++i) node_type_id_[node_types[i]] = static_cast<int64_t>(i);
-  std::vector<int64_t> indptr_addr, indices_addr, num_nodes;
-  torch::Device device(torch::kCPU);
-  num_nodes_ = 0;
+  tables_.clear();
   for (size_t i = 0; i < edge_types.size(); ++i) {
     edge_type_id_[std::get<1>(edge_types[i])] = static_cast<int64_t>(i);
     auto csc = edge_relations[i]->GetCSC();
@@ -28,16 +29,9 @@ void HeteroGraph::LoadFromHomo(
     const int idb = csc->indices.scalar_type() == torch::kInt32 ? 4 : 8;
     if (i == 0) id_bytes_ = idb;
     TORCH_CHECK(idb == id_bytes_, "relation graphs differ in id dtype");
-    indptr_addr.push_back(reinterpret_cast<int64_t>(csc->indptr.data_ptr()));
-    indices_addr.push_back(reinterpret_cast<int64_t>(csc->indices.data_ptr()));
-    num_nodes.push_back(csc->indptr.numel() - 1);
-    num_nodes_ += num_nodes.back();
-    device = csc->indptr.device();
-  }
-  if (!edge_types.empty()) {
-    indptr_table_ = torch::tensor(indptr_addr, torch::dtype(torch::kInt64)).to(device);
-    indices_table_ = torch::tensor(indices_addr, torch::dtype(torch::kInt64)).to(device);
-    num_nodes_table_ = torch::tensor(num_nodes, torch::dtype(torch::kInt64)).to(device);
+    tables_.push_back({reinterpret_cast<int64_t>(csc->indptr.data_ptr()),
+                       reinterpret_cast<int64_t>(csc->indices.data_ptr()), csc->indptr.numel() - 1});
+    device_ = csc->indptr.device();
   }
 }
 
@@ -52,17 +46,30 @@ torch::Tensor HeteroGraph::MetapathRandomWalkFused(torch::Tensor seeds,
   Range range("gs::MetapathRandomWalk");
   auto cached = metapath_cache_.find(metapath);
   if (cached == metapath_cache_.end()) {
-    std::vector<int64_t> ids;
+    // the relations that the path takes, in the order in which it meets them (their offsets are what a
+    // walk may pack, and another large relation is none of its business)
+    std::vector<int64_t> used, steps;
     for (const auto& name : metapath) {
       auto it = edge_type_id_.find(name);
       TORCH_CHECK(it != edge_type_id_.end(), "unknown edge type ", name, " in metapath");
-      ids.push_back(it->second);
+      auto at = std::find(used.begin(), used.end(), it->second);
+      steps.push_back(at - used.begin());
+      if (at == used.end()) used.push_back(it->second);
     }
-    torch::Tensor dev = torch::tensor(ids, torch::dtype(torch::kInt64)).to(seeds.device());
-    cached = metapath_cache_.emplace(metapath, dev).first;
+    const int64_t length = static_cast<int64_t>(steps.size()), relations = static_cast<int64_t>(used.size());
+    Path path;
+    for (int k = 0; k < 3; ++k)
+      for (int64_t r : used) steps.push_back(tables_[r][k]);
+    for (int64_t r : used) path.num_nodes += tables_[r][2];
+    auto all = torch::tensor(steps, torch::dtype(torch::kInt64)).to(device_);
+    path.steps = all.narrow(0, 0, length);
+    path.indptr = all.narrow(0, length, relations);
+    path.indices = all.narrow(0, length + relations, relations);
+    path.sizes = all.narrow(0, length + 2 * relations, relations);
+    cached = metapath_cache_.emplace(metapath, path).first;
   }
-  return hip::MetapathWalk(seeds, cached->second, indptr_table_, indices_table_, num_nodes_table_,
-                           num_nodes_, id_bytes_)
+  const Path& path = cached->second;
+  return hip::MetapathWalk(seeds, path.steps, path.indptr, path.indices, path.sizes, path.num_nodes, id_bytes_)
       .reshape({seeds.numel(), -1});
 }
 

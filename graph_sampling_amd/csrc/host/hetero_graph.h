@@ -5,6 +5,7 @@
 #include <torch/custom_class.h>
 #include <torch/script.h>
 
+#include <array>
 #include <map>
 #include <string>
 #include <tuple>
@@ -36,13 +37,17 @@ class HeteroGraph : public torch::CustomClassHolder {
  private:
   std::map<std::string, int64_t> node_type_id_, edge_type_id_;
   std::vector<c10::intrusive_ptr<Graph>> relations_;
-  // device tables of the relations' indptr / indices addresses, built once
-  torch::Tensor indptr_table_, indices_table_, num_nodes_table_;
-  int64_t num_nodes_ = 0;  // of all relations together
+  // of every relation: the addresses of its indptr and its indices, and its columns
+  std::vector<std::array<int64_t, 3>> tables_;
+  torch::Device device_ = torch::kCPU;
   int id_bytes_ = 8;
   // metapaths already uploaded (the reference re-uploads on every call,
-  // src/hetero_graph.cc:66-69)
-  std::map<std::vector<std::string>, torch::Tensor> metapath_cache_;
+  // src/hetero_graph.cc:66-69), each with the tables of the relations that it takes
+  struct Path {
+    torch::Tensor steps, indptr, indices, sizes;
+    int64_t num_nodes = 0;  // of its relations together
+  };
+  std::map<std::vector<std::string>, Path> metapath_cache_;
 };
 
 }  // namespace gs

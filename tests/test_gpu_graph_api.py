@@ -619,6 +619,35 @@ def test_random_walk_and_metapath_flow(dev):
             assert (d == -1) if s == -1 else (d == -1 or d in ix[ip[s]:ip[s + 1]])
 
 
+@pytest.mark.parametrize("path", [["small"], ["small", "other"], ["other", "small", "small"], ["large", "other"], []])
+def test_metapath_counts_the_relations_it_takes(dev, path):
+    """A large relation that a path leaves out changes nothing about it: no table of its offsets (2^18 nodes and 2^17
+    walkers of twenty steps would make one) is made for the walk.  The same walks whichever relations lie in between."""
+    rng = np.random.default_rng(4)
+    graphs = {}
+    for name, nodes in (("large", 1 << 18), ("other", 3000), ("small", 1000)):
+        indptr = np.concatenate([[0], np.cumsum(rng.integers(0, 6, nodes))]).astype(np.int64)
+        graphs[name] = indptr, rng.integers(0, 3000, indptr[-1])
+    names = list(graphs)
+    hm = gs.HeteroMatrix()
+    hm.load_from_homo(["n"], [("n", name, "n") for name in names],
+                      [gs.Matrix().load_csc(to_dev(p, dev), to_dev(i, dev)) for p, i in graphs.values()])
+    path = (path * 20)[:20]
+    seeds = rng.integers(0, 1000, 1 << 17)
+    here = to_dev(seeds, dev)
+    for _ in range(2):  # (the second time the path is on the GPU)
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        gs.set_seed(10)
+        tr = hm.metapath_random_walk_fused(here, path)
+        scratch = torch.cuda.max_memory_allocated() - before - tr.numel() * 8
+    want = O.metapath_walk([p for p, _ in graphs.values()], [i for _, i in graphs.values()],
+                           [names.index(name) for name in path], seeds, seed=10)
+    assert np.array_equal(tr.reshape(-1).cpu().numpy(), want)
+    table = (1 << 18) // 6 * 16
+    assert scratch >= table if "large" in path else scratch < table // 8
+
+
 def test_gsddmm_ops(dev):
     m, indptr, indices, _ = _rmat_matrix(dev, 10, 14, 8)
     N, E = 1 << 10, indices.size
