@@ -205,7 +205,8 @@ def main():
         mstarts = rand_ids(1_000_000, 2_000_000)
         run("metapath_walk", "gs_metapath_walk: 1M walkers x 16 steps over three 50M-edge relations; "
             "28 B per live step",
-            lambda: capi.metapath_walk(ptr_tab, idx_tab, n_tab, idt, path, mstarts, seed=4),
+            lambda: capi.metapath_walk(ptr_tab, idx_tab, n_tab, idt, path, mstarts, seed=4,
+                                       num_nodes=sum(r[0].numel() - 1 for r in rels)),
             lambda o: (int((o[1_000_000:] >= 0).sum().item()) * 28,
                        int((o[1_000_000:] >= 0).sum().item()), "steps"))
         del rels

@@ -1001,8 +1001,8 @@ def metapath_walk(indptr_table, indices_table, num_nodes_table, id_dtype, metapa
                   replay=None, num_nodes=0, packed=None):
     """indptr_table / indices_table: device int64 tensors holding device addresses;
     num_nodes_table: device int64 tensor, columns per relation; num_nodes: their sum, for which
-    packed tables of the offsets have room (0: none are made); packed: whether they are (None: where
-    it pays)."""
+    packed tables of the offsets have room (0, as when it is not said: none are made); packed: whether they
+    are (None: where it pays, which takes num_nodes)."""
     _need(num_nodes_table, torch.int64, "num_nodes_table")
     _need(metapath, torch.int64, "metapath")
     idb = _ids(seeds, "seeds")
