@@ -717,7 +717,8 @@ __device__ __forceinline__ void linked_insert(const PackedTable& t, IdT key, int
   pos[item] = t.template insert<false>(static_cast<long long>(key), static_cast<uint32_t>(item));
 }
 
-template <typename IdT, int G, bool REPLACE, int THREADS, bool LINKED>
+// DATA: edge data follow the samples
+template <typename IdT, int G, bool REPLACE, int THREADS, bool LINKED, bool DATA>
 __global__ void __launch_bounds__(THREADS) sample_group_kernel(FusedArgs<IdT> a) {
   constexpr int kRows = THREADS / G;
   constexpr int KMAX = 4 * G;
@@ -775,15 +776,19 @@ __global__ void __launch_bounds__(THREADS) sample_group_kernel(FusedArgs<IdT> a)
   // ---- 3. gather: outputs 4*sub .. 4*sub+3 of the row (round 0)
   const IdT* __restrict__ indices = a.indices;
   const uint32_t* rp_replace = REPLACE && a.replay && cnt > 0 ? a.replay + a.replay_ptr[my_row] : nullptr;
-  // (a lane with picks reads four, its first one again past the row's last, ids and edge data one behind the
+  // (kTogether: a lane with picks reads four, its first one again past the row's last, ids and edge data one behind the
   // other with nothing in between: under a condition each, the first was waited for before the second
   // was asked for, and all the ids before the data: of 1024 seeds' three layers with edge weights the second
-  // takes 11.0 us for 13.2, the third 15.5 for 16.3)
+  // takes 11.0 us for 13.2, the third 15.5 for 16.3.  Not with replacement and no data to read behind the ids, nor for
+  // rows of one lane, in turn / together: 718 seeds, fanout 7, 64-bit ids 9.3/10.1 us, 250 seeds, 15 9.8/10.7, 718 and their
+  // samples, fanout 3 9.3/10.0; a row's picks are on few lines, and those asked for after the first find them.)
+  constexpr bool kTogether = G > 1 && (DATA || !REPLACE);
   int64_t q[4];
   IdT v[4];
   float w[4];
-  const bool picks = 4 * sub < cnt;
-  if (picks) {
+#pragma unroll
+  for (int u = 0; u < 4; ++u) q[u] = -1;
+  if (cnt > 0) {
     if (REPLACE) {
       U4 blk;
       if (rp_replace) {
@@ -796,25 +801,49 @@ __global__ void __launch_bounds__(THREADS) sample_group_kernel(FusedArgs<IdT> a)
 #pragma unroll
       for (int u = 0; u < 4; ++u) mine[u] = blk.v[u] % static_cast<uint32_t>(deg);
     }
-    int64_t from[4];
+    if constexpr (kTogether) {
+      if (4 * sub < cnt) {
+        int64_t from[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const uint32_t other = mine[u], first = mine[0];
-      from[u] = start + (4 * sub + u < cnt ? other : first);
-    }
+        for (int u = 0; u < 4; ++u) {
+          const uint32_t other = mine[u], first = mine[0];
+          from[u] = start + (4 * sub + u < cnt ? other : first);
+          if (4 * sub + u < cnt) q[u] = from[u];
+        }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = indices[from[u]];
-    if (a.data_out) {
-      if (a.edge_ids) {
+        for (int u = 0; u < 4; ++u) v[u] = indices[from[u]];
+        if (DATA) {
+          if (a.edge_ids) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) from[u] = a.edge_ids[from[u]];
+            for (int u = 0; u < 4; ++u) from[u] = a.edge_ids[from[u]];
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u) w[u] = a.edge_data[from[u]];
+        }
       }
+    } else {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) w[u] = a.edge_data[from[u]];
+      for (int u = 0; u < 4; ++u) {
+        if (4 * sub + u < cnt) {
+          q[u] = start + mine[u];
+          v[u] = indices[q[u]];
+        }
+      }
+      if (DATA) {
+        int64_t at_data[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) at_data[u] = q[u];
+        if (a.edge_ids) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (q[u] >= 0) at_data[u] = a.edge_ids[q[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (q[u] >= 0) w[u] = a.edge_data[at_data[u]];
+      }
     }
   }
-#pragma unroll
-  for (int u = 0; u < 4; ++u) q[u] = picks && 4 * sub + u < cnt ? start + mine[u] : -1;
   __syncthreads();
   __builtin_amdgcn_s_waitcnt(kLoadsDone);
   const int64_t out0 = s_prefix;
@@ -836,7 +865,7 @@ __global__ void __launch_bounds__(THREADS) sample_group_kernel(FusedArgs<IdT> a)
       a.sub_indices[o] = v[u];
       if (a.select_index) a.select_index[o] = q[u];
       if (a.coo_col) a.coo_col[o] = static_cast<IdT>(my_row);
-      if (a.data_out) a.data_out[o] = w[u];
+      if (DATA) a.data_out[o] = w[u];
     }
   }
   if (LINKED) {
@@ -942,7 +971,7 @@ __global__ void __launch_bounds__(THREADS) sample_group_kernel(FusedArgs<IdT> a)
           a.sub_indices[o] = got;
           if (a.select_index) a.select_index[o] = p;
           if (a.coo_col) a.coo_col[o] = static_cast<IdT>(my_row);
-          if (a.data_out) a.data_out[o] = a.edge_data[a.edge_ids ? a.edge_ids[p] : p];
+          if (DATA) a.data_out[o] = a.edge_data[a.edge_ids ? a.edge_ids[p] : p];
           if (LINKED) linked_insert<IdT>(a.table, got, S + o, a.pos, a.lb.error);
         }
       }
@@ -955,12 +984,21 @@ __global__ void __launch_bounds__(THREADS) sample_group_kernel(FusedArgs<IdT> a)
 template <typename IdT, int G, bool REPLACE, bool LINKED>
 int sample_group_launch(const FusedArgs<IdT>& a, hipStream_t stream) {
   const unsigned grid = static_cast<unsigned>(group_tiles(a.S, G, LINKED));
+  auto go = [&](auto threads, auto data) {
+    constexpr int kHere = decltype(threads)::value;
+    hipLaunchKernelGGL((sample_group_kernel<IdT, G, REPLACE, kHere, LINKED, decltype(data)::value>), dim3(grid),
+                       dim3(kHere), 0, stream, a);
+  };
+  auto by_data = [&](auto threads) {
+    if (a.data_out)
+      go(threads, std::true_type());
+    else
+      go(threads, std::false_type());
+  };
   if (group_tile_threads(a.S, G, LINKED) == kGroupThreadsLarge)
-    hipLaunchKernelGGL((sample_group_kernel<IdT, G, REPLACE, kGroupThreadsLarge, LINKED>),
-                       dim3(grid), dim3(kGroupThreadsLarge), 0, stream, a);
+    by_data(std::integral_constant<int, kGroupThreadsLarge>());
   else
-    hipLaunchKernelGGL((sample_group_kernel<IdT, G, REPLACE, kGroupThreadsSmall, LINKED>),
-                       dim3(grid), dim3(kGroupThreadsSmall), 0, stream, a);
+    by_data(std::integral_constant<int, kGroupThreadsSmall>());
   return check_launch("sample_fused");
 }
 
