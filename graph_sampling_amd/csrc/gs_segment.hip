@@ -147,7 +147,7 @@ using F4 = float __attribute__((ext_vector_type(4)));
 // Source: where a tile's data come from.
 enum Source {
   kPlain,     // data[edge], 16-byte aligned
-  kStreamed,  // the same, of at least kStreamEdges edges
+  kStreamed,  // the same, of at least kStreamEdges edges (a sum: and kStreamSumBytes)
   kLoose,     // data[edge]
   kMapped     // data[emap[edge]]
 };
@@ -159,6 +159,12 @@ enum Source {
 // after finds it in the cache no more (normalise, then the sum of its result: 16 M edges 84 -> 85.5,
 // 32 M the same, 60 M 218 -> 212).
 constexpr int64_t kStreamEdges = int64_t(1) << 25;
+// A sum leaves its data where they were: from so many bytes of data, offsets and sums on, 4 an edge and 12 a segment.
+// The same array summed again and again / three in turn, plain -> as a stream, us: 34 M edges, 80 k segments 32.3 ->
+// 33.7 / 33.6 -> 33.4, 40 M, 5 M segments (220 MB) 133.6 -> 138.9 / 138.2 -> 138.2, 62.5 M, 1.2 M segments (265 MB)
+// 65.0 -> 70.7 / 65.4 -> 66.9, 64 M, 0.13 M segments (258 MB) 51.1 -> 54.4 / 54.2 -> 53.8; 64 M, 8 M segments (352 MB)
+// 148.5 -> 139.2 / 148.0 -> 139.0, 100 M, 10 M segments 229.5 -> 204.9 / 229.7 -> 204.2.
+constexpr int64_t kStreamSumBytes = int64_t(1) << 28;
 
 template <Source SOURCE>
 __device__ __forceinline__ F4 read_four(const float* at) {
@@ -705,10 +711,10 @@ carry_kernel(const int64_t* __restrict__ indptr, const IdT* __restrict__ nmap, i
   }
 }
 
-inline Source source_of(const int64_t* emap, const float* data, int64_t nnz) {
+inline Source source_of(const int64_t* emap, const float* data, bool streams) {
   if (emap) return kMapped;
   if ((reinterpret_cast<uintptr_t>(data) & 15u) != 0) return kLoose;
-  return nnz >= kStreamEdges ? kStreamed : kPlain;
+  return streams ? kStreamed : kPlain;
 }
 
 inline int64_t num_tiles(int64_t nnz) { return nnz <= 0 ? 1 : (nnz + kTile - 1) / kTile; }
@@ -792,7 +798,8 @@ int segment_sum_impl(const int64_t* indptr, const int64_t* emap, const void* nma
            : width == kMiddle ? segment_tiles_kernel<false, S, kHeads, kMiddle, IdT>
                               : segment_tiles_kernel<false, S, kHeads, kNarrow, IdT>;
   };
-  const Source source = source_of(emap, data, nnz);
+  const Source source =
+      source_of(emap, data, nnz >= kStreamEdges && 4 * nnz + 12 * num_seg >= kStreamSumBytes);
   auto* kernel = source == kMapped  ? pick(std::integral_constant<Source, kMapped>{})
                  : source == kLoose ? pick(std::integral_constant<Source, kLoose>{})
                  : source == kStreamed ? pick(std::integral_constant<Source, kStreamed>{})
@@ -843,7 +850,7 @@ int segment_normalize_impl(const int64_t* indptr, const int64_t* emap, const flo
   const Walk walk = tl.mark ? kMarks : (num_tiles(nnz) > kSearchTiles ? kHeads : kSearch);
   if (walk != kSearch)
     launch_heads<false>(indptr, static_cast<const int64_t*>(nullptr), num_seg, nnz, out, tl, st);
-  const Source source = source_of(emap, data, nnz);
+  const Source source = source_of(emap, data, nnz >= kStreamEdges);
   auto* launch = source == kMapped  ? launch_normalize<kMapped>
                  : source == kLoose ? launch_normalize<kLoose>
                  : source == kStreamed ? launch_normalize<kStreamed>

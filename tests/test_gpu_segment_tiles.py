@@ -101,6 +101,22 @@ def test_streamed_edges(dev, kind, nnz, front):
             assert (out[:front] == -1).all()
 
 
+# 4 bytes an edge and 12 a segment: 2**28 in all, from which on a sum's data are streamed, and an edge less; beyond them
+# the last segments are empty
+@pytest.mark.parametrize("less", [0, 1])
+@pytest.mark.parametrize("nseg", [1000, 5_000_000, (1 << 25) // 3])
+def test_streamed_sums(dev, nseg, less):
+    nnz = (1 << 26) - 3 * nseg - less
+    ptr = (torch.arange(nseg + 1, device=dev) * nnz // (nseg - 7)).clamp_(max=nnz)
+    data = torch.rand(nnz, device=dev) + 0.25
+    owner = torch.repeat_interleave(torch.diff(ptr), output_size=nnz)
+    for power in (1, 2):
+        want = torch.zeros(nseg, dtype=torch.float64, device=dev).index_add_(0, owner, data.double() ** power)
+        out = torch.full((nseg,), -1.0, device=dev)
+        capi.segment_sum(ptr, None, None, data, power, out)
+        torch.testing.assert_close(out.double(), want, rtol=RTOL, atol=0)
+
+
 def _check(dev, kind, total, emap, rtol=RTOL):
     indptr = _segments(kind, total)
     nnz, nseg = int(indptr[-1]), indptr.size - 1
