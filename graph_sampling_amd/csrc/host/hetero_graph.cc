@@ -1,6 +1,7 @@
 #include "hetero_graph.h"
 
 #include <algorithm>
+#include <numeric>
 
 #include "range.h"
 
@@ -33,6 +34,24 @@ void HeteroGraph::LoadFromHomo(
                        reinterpret_cast<int64_t>(csc->indices.data_ptr()), csc->indptr.numel() - 1});
     device_ = csc->indptr.device();
   }
+  std::vector<int64_t> all(tables_.size());
+  std::iota(all.begin(), all.end(), 0);
+  all_ = Path();
+  if (!all.empty()) all_ = Upload({}, all);
+}
+
+HeteroGraph::Path HeteroGraph::Upload(std::vector<int64_t> values, const std::vector<int64_t>& relations) const {
+  const int64_t length = static_cast<int64_t>(values.size()), R = static_cast<int64_t>(relations.size());
+  Path path;
+  for (int k = 0; k < 3; ++k)
+    for (int64_t r : relations) values.push_back(tables_[r][k]);
+  for (int64_t r : relations) path.num_nodes += tables_[r][2];
+  auto all = torch::tensor(values, torch::dtype(torch::kInt64)).to(device_);
+  path.steps = all.narrow(0, 0, length);
+  path.indptr = all.narrow(0, length, R);
+  path.indices = all.narrow(0, length + R, R);
+  path.sizes = all.narrow(0, length + 2 * R, R);
+  return path;
 }
 
 c10::intrusive_ptr<Graph> HeteroGraph::GetHomoGraph(const std::string& edge_type) const {
@@ -56,16 +75,14 @@ torch::Tensor HeteroGraph::MetapathRandomWalkFused(torch::Tensor seeds,
       steps.push_back(at - used.begin());
       if (at == used.end()) used.push_back(it->second);
     }
-    const int64_t length = static_cast<int64_t>(steps.size()), relations = static_cast<int64_t>(used.size());
     Path path;
-    for (int k = 0; k < 3; ++k)
-      for (int64_t r : used) steps.push_back(tables_[r][k]);
-    for (int64_t r : used) path.num_nodes += tables_[r][2];
-    auto all = torch::tensor(steps, torch::dtype(torch::kInt64)).to(device_);
-    path.steps = all.narrow(0, 0, length);
-    path.indptr = all.narrow(0, length, relations);
-    path.indices = all.narrow(0, length + relations, relations);
-    path.sizes = all.narrow(0, length + 2 * relations, relations);
+    if (used.size() == tables_.size()) {  // (all: their tables are there, and only the steps go up)
+      for (int64_t& step : steps) step = used[step];
+      path = all_;
+      path.steps = torch::tensor(steps, torch::dtype(torch::kInt64)).to(device_);
+    } else {
+      path = Upload(std::move(steps), used);
+    }
     cached = metapath_cache_.emplace(metapath, path).first;
   }
   const Path& path = cached->second;

@@ -619,7 +619,8 @@ def test_random_walk_and_metapath_flow(dev):
             assert (d == -1) if s == -1 else (d == -1 or d in ix[ip[s]:ip[s + 1]])
 
 
-@pytest.mark.parametrize("path", [["small"], ["small", "other"], ["other", "small", "small"], ["large", "other"], []])
+@pytest.mark.parametrize("path", [["small"], ["small", "other"], ["other", "small", "small"], ["large", "other"],
+                                  ["other", "large", "small"], []])
 def test_metapath_counts_the_relations_it_takes(dev, path):
     """A large relation that a path leaves out changes nothing about it: no table of its offsets (2^18 nodes and 2^17
     walkers of twenty steps would make one) is made for the walk.  The same walks whichever relations lie in between."""
