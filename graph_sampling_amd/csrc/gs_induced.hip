@@ -18,7 +18,7 @@
 //     array, their new row number in 2 bytes and their datum.
 // A scan of the tile counts and one copy kernel put the pieces together.  (With the tiles shared
 // by the waves of a workgroup, offsets and counts through LDS and two barriers a tile, the marks
-// took 293 us where they take 225.)
+// took 293 us where a wave's own tiles took 225, before they were streamed.)
 //
 // Two forms of the set.  BitmapSet, for graphs whose numbers of nodes fit (about 600 k): a bit
 // per node, the set bits before each 32-bit word, and the place of every set bit's id: three
@@ -28,11 +28,11 @@
 // Its loop over buckets and slots is what bounds it (a kernel of this kind that shared its tiles
 // among the waves took 419 us with it where it took 293 with the bitmap).
 //
-// What bounds the bitmap form: 785 MB in 225 us in the case below, 3.5 TB/s, with the vector ALUs
-// issuing 45 % of the time; more waves than the set leaves room for would be needed to
+// What bounds the bitmap form: the LDS look-ups and the vector ALUs beside 750 MB in 184 us in the case below,
+// 4.1 TB/s (reads that are truly a tile ahead: 183); more waves than the set leaves room for would be needed to
 // overlap the two better.  7263 nodes whose columns hold 50.8 M edges, 22.0 M kept, 64-bit ids
-// and weights: 225 us for the marks and 70 us for the copy (new row numbers in 2 bytes instead of 4 and
-// streamed: 185 + 84), where a filter and a table in the
+// and weights: 184 us for the marks and 71-84 us for the copy (new row numbers in 4 bytes and nothing
+// streamed: 225 + 70), where a filter and a table in the
 // L2s, parent positions carried along and a gather of the data behind took 546 + 226 + 104.
 #include "gs_common.hpp"
 

@@ -25,15 +25,14 @@
 // every segment's first edge.
 //
 // 124 M edges in 2.45 M columns (half of them of at most 16 edges, 19 % of the edges in columns
-// longer than a tile), kernels: sum 137 us (3.8 TB/s; the bytes bound it: tiles 121 of it),
-// normalise 282 us (3.5 TB/s over the bytes it needs, 4.7 with the second reading: tiles 179,
-// the crossing segments 95; each tile's chain of LDS steps hides behind the other tiles of its
-// CU).  A lane per short column, a scan per 1024-edge chunk for the others and a divide pass
-// over all edges, each reading its edges for itself, took 214 and 380.  Tiles of 8192 edges:
-// 156 and 324, against 144 and 308 as the tiles of 4096 were then.  With streamed accesses
-// (kStreamEdges) the sum's tiles took 118 where they took 129, the normalise's 187 / 202 and its crossing
-// segments 90 / 99.  Workgroups that stay for two or four tiles, the next one's data on their way
-// while one is added up: 64 registers are too few for that, and at 96 both calls took 449 us against 357.
+// longer than a tile), as streams (kStreamEdges), kernels of calls one after the other: sum 112 us (4.9 TB/s; the bytes
+// bound it: tiles 100 of it), normalise 247 us (4.1 TB/s over the bytes it needs, 4.8 with the second reading: tiles
+// 160, the crossing segments 80; each tile's chain of LDS steps hides behind the other tiles of its
+// CU); one of each in turn 349-353 (plainly 380-390).  A lane per short column, a scan per 1024-edge chunk for the
+// others and a divide pass over all edges, each reading its edges for itself, took 214 and 380.  Tiles of 8192 edges:
+// 156 and 324, against 144 and 308 as the tiles of 4096 were then, plainly.  Workgroups that stay for two or four
+// tiles, the next one's data on their way while one is added up: 64 registers are too few for that, and at 96 both
+// calls took 449 us against 357.
 #include <limits>
 #include "gs_common.hpp"
 

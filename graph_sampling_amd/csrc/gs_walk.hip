@@ -98,10 +98,10 @@ __device__ __forceinline__ int64_t neighbour(Indices indices, int64_t start, int
 // end as its distance from that start, in 16 bits each and in order.  Where that cannot be said (a
 // hub among the nodes), the first distance is larger than the last and the offsets themselves are
 // read instead.  A step reads a record at once, and what the L2s (4 MB a die) have to hold of the offsets
-// is a third: 1 M walkers, 80 steps, 4 M nodes of 50 edges 1428 -> 1237 us with the making of the table
-// (12).  60 nodes to a line of 128 bytes, start and two ends read apart, were a fifth smaller and no
-// better: 1 M nodes 1132 us against 1166, but 200 k walkers 266 against 263, 4 M nodes of 8 edges 673
-// against 668.
+// is a third: 1 M walkers, 80 steps, 4 M nodes of 50 edges 1321 -> 1148 us with the making of the table
+// (11).  60 nodes to a line of 128 bytes, start and two ends read apart, are a fifth smaller and were no better (both
+// in the kernel as it was with the draws in scratch memory and the store in front of the offsets): 1 M nodes 1132 us
+// against 1166, but 200 k walkers 266 against 263, 4 M nodes of 8 edges 673 against 668.
 constexpr int kRecordNodes = 6;
 
 // Whether a table of the offsets is made in front of a walk: where they outgrow an L2 by far or by a little, the
