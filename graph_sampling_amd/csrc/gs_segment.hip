@@ -25,10 +25,10 @@
 // every segment's first edge.
 //
 // 124 M edges in 2.45 M columns (half of them of at most 16 edges, 19 % of the edges in columns
-// longer than a tile), as streams (kStreamEdges), kernels of calls one after the other: sum 112 us (4.9 TB/s; the bytes
-// bound it: tiles 100 of it), normalise 247 us (4.1 TB/s over the bytes it needs, 4.8 with the second reading: tiles
-// 160, the crossing segments 80; each tile's chain of LDS steps hides behind the other tiles of its
-// CU); one of each in turn 349-353 (plainly 380-390).  A lane per short column, a scan per 1024-edge chunk for the
+// longer than a tile), as streams (kStreamEdges), kernels of one of each in turn: sum 116 us (4.7 TB/s; the bytes
+// bound it: tiles 105 of it), normalise 236 us (4.3 TB/s over the bytes it needs, 5.0 with the second reading: tiles
+// 151, the crossing segments 79; each tile's chain of LDS steps hides behind the other tiles of its
+// CU); the calls 348-353 (plainly 380-390).  A lane per short column, a scan per 1024-edge chunk for the
 // others and a divide pass over all edges, each reading its edges for itself, took 214 and 380.  Tiles of 8192 edges:
 // 156 and 324, against 144 and 308 as the tiles of 4096 were then, plainly.  Workgroups that stay for two or four
 // tiles, the next one's data on their way while one is added up: 64 registers are too few for that, and at 96 both
