@@ -17,7 +17,8 @@
 //    waves with a small LDS table.  What moves is one 64-bit word per edge, key
 //    above and original position below, and the value in 32 bits, so a pass is 12
 //    bytes in and 12 bytes out per edge and the permutation falls out of the last
-//    pass.  indptr then comes from the places where the sorted keys change, or, with
+//    pass.  indptr comes from the tiles of the last pass where the values travel in
+//    the words, else from the places where the sorted keys change, or, with
 //    fewer edges than columns, from one search per column confined to the keys of
 //    the workgroup's 256 columns.
 //  * distinct ids of an edge list: a bit per possible id in LDS, slice by slice, or, for short
@@ -387,14 +388,16 @@ __device__ __forceinline__ int digit_of(unsigned long long word, int shift) {
   return static_cast<int>((word >> shift) & (kRadix - 1));
 }
 
-// words of the first pass, made from the caller's keys on the fly
-template <typename IdT>
+// words of the first pass, made from the caller's keys on the fly (STREAM: read past the caches)
+template <typename IdT, bool STREAM = false>
 struct FreshWords {
   const IdT* key;
   int idx_bits;
   // word j of the tile that begins at `base`
   __device__ __forceinline__ unsigned long long operator()(int64_t base, uint32_t j) const {
-    return (static_cast<unsigned long long>((key + base)[j]) << idx_bits) |
+    const IdT* p = key + base + j;
+    const IdT k = STREAM ? __builtin_nontemporal_load(p) : *p;
+    return (static_cast<unsigned long long>(k) << idx_bits) |
            static_cast<unsigned long long>(base + j);
   }
 };
@@ -425,6 +428,10 @@ constexpr int64_t kLargeTileItems = int64_t(1) << 22;  // 512 large tiles: two f
 // 437 k stores to as many lines for 14 M edges, 24 -> 19 us).  Four copies of the histogram, lane
 // by lane in turn: on a skewed graph half a wave holds one digit, and additions to one LDS word
 // queue up.
+// What bounds it is the list's bytes.  Large tiles read it past the caches: a plain read of a list that the
+// memory-side cache does not hold takes the place of lines there that were written last (the sort's own words) and
+// waits for them to be written back: 112 MB 42 us plain, 20 so.  The first pass, which then found the list there, takes
+// 81 for 62; the list loaded and sorted 379 -> 372.
 constexpr int kHistCopies = 4;
 
 template <typename T, typename Src>
@@ -432,10 +439,6 @@ __global__ void __launch_bounds__(T::kThreadsPerTile)
 radix_hist_kernel(Src src, int64_t E, int shift, int64_t* __restrict__ counts,
                   int* __restrict__ clear) {
   __shared__ int s_hist[kHistCopies][kRadix + 1];
-  for (int j = threadIdx.x; j < kHistCopies * (kRadix + 1); j += T::kThreadsPerTile)
-    (&s_hist[0][0])[j] = 0;
-  if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;
-  __syncthreads();
   const int64_t base = static_cast<int64_t>(blockIdx.x) * T::kSize;
   const uint32_t n = E - base < T::kSize ? static_cast<uint32_t>(E - base) : T::kSize;
   unsigned long long word[T::kPerThread];
@@ -444,10 +447,15 @@ radix_hist_kernel(Src src, int64_t E, int shift, int64_t* __restrict__ counts,
     const uint32_t j = k * T::kThreadsPerTile + threadIdx.x;
     word[k] = src(base, j < n ? j : n - 1);
   }
+  for (int j = threadIdx.x; j < kHistCopies * (kRadix + 1); j += T::kThreadsPerTile)
+    (&s_hist[0][0])[j] = 0;
+  if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;
+  lds_barrier();  // (the words stay on their way)
 #pragma unroll
-  for (int k = 0; k < T::kPerThread; ++k)
-    if (k * T::kThreadsPerTile + threadIdx.x < n)
-      atomicAdd(&s_hist[threadIdx.x & (kHistCopies - 1)][digit_of(word[k], shift)], 1);
+  for (int k = 0; k < T::kPerThread; ++k) {
+    const int d = k * T::kThreadsPerTile + threadIdx.x < n ? digit_of(word[k], shift) : kRadix;
+    atomicAdd(&s_hist[threadIdx.x & (kHistCopies - 1)][d], 1);
+  }
   __syncthreads();
   if (threadIdx.x < kRadix) {
     int n = 0;
@@ -538,6 +546,8 @@ struct SortOutputs {
   int idx_bits;
   int* wide;  // raised when a 64-bit value does not fit 32 bits (null: 32-bit values)
   bool stream;  // packed_pass_kernel: results as streams (kStreamResults)
+  int64_t* indptr;  // packed_pass_kernel: the columns' offsets, from the tiles themselves (null: not here)
+  int64_t num_keys;
 };
 
 // One pass of the sort over one tile, stable.  A wave owns its share of the tile, in index
@@ -754,7 +764,11 @@ radix_pass_kernel(Src src, const ValT* __restrict__ val_in, int64_t E, int shift
 // The words it writes are the next
 // pass's: written past the caches they cost 456.  The last pass's results go past them where they
 // fill more than half of the memory-side cache (14 M: 415 -> 404, 11 M: 301 -> 290; 8 M, 128 MB: 277, 278).
+// The last pass leaves the columns' offsets too where edges are many for the columns (coo2csc_impl): it holds a tile in key order, and
+// the keys that it wrote for a launch behind the sort to read back were 112 of the 1500 MB that a list of 14 M edges
+// moves: that pass 84 -> 85 us, the launch behind it, 19, gone; the list loaded and sorted 392 -> 379.
 constexpr int kPackedPasses = 3;
+constexpr uint32_t kWideTile = 16;  // offsets a thread beyond which a tile has long gaps
 constexpr int64_t kStreamResults = int64_t(1) << 27;  // bytes
 constexpr int rest_at(int passes) { return 64 - kRadixBits * (passes - 1); }  // of the key's digits in a word
 
@@ -782,6 +796,7 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
   __shared__ int s_scan[kRadix / kWave];
   __shared__ uint32_t s_ends[kRadix / kWave];
   __shared__ int64_t s_digits[kRadix / kWave];
+  __shared__ uint32_t s_lows[2];  // LAST: the tile's lower digits, from and to (offsets below)
   unsigned short (*s_cnt)[kRadix] = reinterpret_cast<unsigned short (*)[kRadix]>(s_shared);
   unsigned char* s_dig = s_shared;
   // consecutive tiles on one XCD, as above
@@ -815,6 +830,8 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
     else
       word[r] = once(in + base + (j < n ? j : n - 1));
   }
+  unsigned long long ahead = 0;  // the word in front of the tile
+  if constexpr (LAST) ahead = in[tile > 0 ? base - 1 : 0];
   // (what lies behind the last edge takes the last digit, as above)
 #pragma unroll
   for (int r = 0; r < kItemsHere; ++r) {
@@ -918,11 +935,27 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
   }
   // the digit of the pass before at the thread's first item; its later ones lie behind
   int was = 0;
-  if (!FIRST) {
-    const uint32_t at = static_cast<uint32_t>(base) + mine0;
+  auto digit_before = [&](uint32_t at) {
+    int d = 0;
 #pragma unroll
     for (int step = kRadix / 2; step > 0; step >>= 1)
-      if (s_bound[was + step - 1] <= at) was += step;
+      if (s_bound[d + step - 1] <= at) d += step;
+    return d;
+  };
+  constexpr int kAt = kRestAt + kRadixBits * (PASS - 1);  // this pass's digit (not of the first)
+  auto with_digit_before = [](unsigned long long w, int d) {
+    return (w & ~(static_cast<unsigned long long>(kRadix - 1) << kAt)) |
+           static_cast<unsigned long long>(d) << kAt;
+  };
+  if constexpr (!FIRST) was = digit_before(static_cast<uint32_t>(base) + mine0);
+  if constexpr (LAST) {
+    if (last.indptr && threadIdx.x == 0) {
+      uint32_t from = 0;
+      if (tile > 0)
+        from = static_cast<uint32_t>(with_digit_before(ahead, digit_before(static_cast<uint32_t>(base) - 1)) >>
+                                     kRestAt) + 1;
+      s_lows[0] = from;
+    }
   }
   lds_barrier();  // (the counts make room for the digits)
   bool wide = false;
@@ -941,9 +974,9 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
     } else {
       const uint32_t at = static_cast<uint32_t>(base) + j;
       while (was < kRadix - 1 && s_bound[was] <= at) ++was;
-      constexpr int kAt = kRestAt + kRadixBits * (PASS - 1);  // this pass's digit
-      w = (word[r] & ~(static_cast<unsigned long long>(kRadix - 1) << kAt)) |
-          static_cast<unsigned long long>(was) << kAt;
+      w = with_digit_before(word[r], was);
+      if (LAST && j == n - 1)
+        s_lows[1] = base + n == E ? 1u << (kRadixBits * PASS) : static_cast<uint32_t>(w >> kRestAt) + 1;
     }
     s_word[place[r]] = w;
     s_dig[place[r]] = static_cast<unsigned char>(d);
@@ -975,6 +1008,45 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
         next_digit[dst] = static_cast<unsigned char>(w >> (kRestAt + kRadixBits * PASS));
       }
     }
+  }
+  // The offsets of the columns whose lower digits begin in this tile, whatever their last digit: all
+  // edges with lower digits below come before the tile's or lie in it, so the offset is the place of the
+  // digit's first edge that is not below.  Every column is one tile's, with or without edges.
+  if constexpr (LAST) {
+    if (!last.indptr) return;
+    constexpr int kLowBits = kRadixBits * PASS;
+    const uint32_t from = s_lows[0], lows = s_lows[1] - from;
+    const int64_t most = (last.num_keys >> kLowBits) + 1;  // (offset num_keys among them)
+    const uint32_t digits = most < kRadix ? static_cast<uint32_t>(most) : kRadix;
+    auto leave = [&](uint32_t d, uint32_t low, uint32_t lo, uint32_t hi) {
+      const int64_t c = static_cast<int64_t>(d) << kLowBits | low;
+      if (c > last.num_keys) return;
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (static_cast<uint32_t>(s_word[mid] >> kRestAt) < low) lo = mid + 1; else hi = mid;
+      }
+      last.indptr[c] = s_base[d] + lo;
+    };
+    auto run_end = [&](uint32_t d) -> uint32_t { return d == kRadix - 1 ? n : s_start[d + 1]; };
+    if (lows * digits <= kWideTile * kThreadsHere) {
+      for (uint32_t i = threadIdx.x; i < lows * digits; i += kThreadsHere) {
+        const uint32_t d = i / lows;
+        leave(d, from + i % lows, s_start[d], run_end(d));
+      }
+    } else {  // long gaps: a wave or more a digit, and no search behind the digit's last edge
+      const uint32_t parts = digits < T::kWaves ? T::kWaves / digits : 1u;
+      for (uint32_t u = wave; u < digits * parts; u += T::kWaves) {
+        const uint32_t d = u % digits, hi = run_end(d);
+        const uint32_t lo = s_start[d];
+        const uint32_t top = lo < hi ? static_cast<uint32_t>(s_word[hi - 1] >> kRestAt) + 1 : from;
+        uint32_t low = from + u / digits * kWave + lane;
+        for (; low < top; low += parts * kWave) leave(d, low, lo, hi);
+        const int64_t first = static_cast<int64_t>(d) << kLowBits, end = s_base[d] + hi;
+        const int64_t most_low = last.num_keys - first;
+        for (; low < from + lows && low <= most_low; low += parts * kWave) last.indptr[first + low] = end;
+      }
+    }
+    if (threadIdx.x == 0 && base + n == E && last.num_keys >> kLowBits == kRadix) last.indptr[last.num_keys] = E;
   }
 }
 
@@ -1130,8 +1202,8 @@ int packed_passes(const IdT* key, const IdT* value, int64_t E, int passes, int v
     const bool last = p == passes - 1;
     const unsigned long long* in = s.word[(p + 1) & 1];
     if (p == 0)
-      hipLaunchKernelGGL((radix_hist_kernel<T, FreshWords<IdT>>), grid, threads, 0, st,
-                         FreshWords<IdT>{key, idx_bits}, E, idx_bits, s.counts, outs.wide);
+      hipLaunchKernelGGL((radix_hist_kernel<T, FreshWords<IdT, T::kStreams>>), grid, threads, 0, st,
+                         FreshWords<IdT, T::kStreams>{key, idx_bits}, E, idx_bits, s.counts, outs.wide);
     else
       hipLaunchKernelGGL(digit_hist_kernel<T>, grid, threads, 0, st, digits, E, s.counts);
     int64_t* totals = p & 1 ? s.totals_before : s.totals;
@@ -1177,9 +1249,15 @@ int coo2csc_impl(const IdT* key, const IdT* value, int64_t E, int64_t num_keys, 
       packed_value_bits(E, num_values, passes, blocks_for(E, large ? LargeTile::kSize : SmallTile::kSize));
   const bool may_be_wide = sizeof(IdT) == 8 || value_bits > 0;
   const bool short_keys = passes * kRadixBits <= 32;
-  const SortOutputs<IdT> outs{out_value, perm, indptr && short_keys ? s.keys : nullptr, idx_bits,
+  // (offsets by the last pass's tiles; written keys and a launch of their own / so, us: 14 M edges, 2.45 M columns 301/281,
+  // 20 k 178/165, one of 2.45 M has all 628/557; 5 M, 5 M 151/143; small tiles: 1 M edges, 200 k columns 63/62, 60 k
+  // 46/42, 300 k, 20 k 40/37, but 1 M, 1 M 66/73 and 300 k, 300 k 58/67, a few tiles' searches)
+  const bool by_tiles = indptr && value_bits > 0 && (large ? num_keys : 4 * num_keys) <= E;
+  const bool by_keys = indptr && short_keys && !by_tiles;
+  const SortOutputs<IdT> outs{out_value, perm, by_keys ? s.keys : nullptr, idx_bits,
                               may_be_wide ? s.wide : nullptr,
-                              E * static_cast<int64_t>(sizeof(int64_t) + sizeof(IdT) + sizeof(uint32_t)) >= kStreamResults};
+                              E * static_cast<int64_t>(sizeof(int64_t) + sizeof(IdT) + sizeof(uint32_t)) >= kStreamResults,
+                              by_tiles ? indptr : nullptr, num_keys};
   if (value_bits > 0) {
     const auto sort = large ? packed_passes<LargeTile, IdT> : packed_passes<SmallTile, IdT>;
     GS_RETURN_IF_ERROR(sort(key, value, E, passes, value_bits, s, outs, st));
@@ -1190,9 +1268,9 @@ int coo2csc_impl(const IdT* key, const IdT* value, int64_t E, int64_t num_keys, 
   if (may_be_wide && value_bits == 0)  // (words with the value inside: the last pass does it)
     hipLaunchKernelGGL(widen_values_kernel<IdT>, dim3(E < (int64_t(1) << 20) ? 64 : 1024),
                        dim3(kThreads), 0, st, value, perm, E, s.wide, out_value);
-  if (indptr && short_keys)  // (null: the caller wants the sorted order only)
+  if (by_keys)  // (null: the caller wants the sorted order only)
     launch_indptr(static_cast<const uint32_t*>(s.keys), E, num_keys, indptr, st);
-  else if (indptr)
+  else if (indptr && !by_tiles)
     hipLaunchKernelGGL((indptr_from_sorted_kernel<PermutedKeys<IdT>>),
                        dim3(blocks_for(num_keys + 1, kPtrCols)), dim3(kThreads), 0, st,
                        PermutedKeys<IdT>{key, perm}, E, num_keys, indptr);

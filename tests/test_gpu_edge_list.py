@@ -110,6 +110,25 @@ def test_sort_with_the_values_in_its_words(dev, num_keys, skew, E, idt):
 
 
 @pytest.mark.parametrize("idt", ID_DTYPES)
+@pytest.mark.parametrize("E,num_keys", [(64 * 4096 + 1, 257), (64 * 4096 + 1, 64 * 4096 + 1), (64 * 4096 + 1, 64 * 4096 + 2),
+                                        (1_000_003, 65_536), ((1 << 22) + 5, 65_537), (1 << 24, 1 << 24)])
+@pytest.mark.parametrize("keys", ["first", "last", "ends", "one low digit", "few"])
+def test_offsets_from_the_last_pass(dev, keys, E, num_keys, idt):
+    """Two digits and three, as many columns as edges and one more, and as many as three digits hold; keys
+    that leave long runs of columns without edges in front, in between and behind, which single tiles write."""
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(E)
+    choice = {"first": [0], "last": [num_keys - 1], "ends": [0, num_keys - 1],
+              "one low digit": list(range(5, num_keys, 256)), "few": [1, 3, 255, 256, num_keys // 2 + 1]}[keys]
+    choice = torch.tensor([k for k in choice if k < num_keys], device=dev)
+    key = choice[torch.randint(0, choice.numel(), (E,), generator=gen, device=dev)].to(idt)
+    ip, val, perm = capi.coo2csc(key, key, num_keys, False)
+    assert torch.equal(val, torch.sort(key).values) and torch.equal(key[perm], val)
+    ends = torch.cumsum(torch.bincount(key.long(), minlength=num_keys), 0)
+    assert int(ip[0]) == 0 and torch.equal(ip[1:], ends)
+
+
+@pytest.mark.parametrize("idt", ID_DTYPES)
 @pytest.mark.parametrize("less", [0, 1])
 @pytest.mark.parametrize("num_keys", [60_000, 3_000_000])
 def test_sort_with_long_results(dev, num_keys, less, idt):
