@@ -434,9 +434,9 @@ constexpr int64_t kLargeTileItems = int64_t(1) << 22;  // 512 large tiles: two f
 // 81 for 62; the list loaded and sorted 379 -> 372.
 constexpr int kHistCopies = 4;
 
-template <typename T, typename Src>
+template <typename T, typename Src, typename Count>
 __global__ void __launch_bounds__(T::kThreadsPerTile)
-radix_hist_kernel(Src src, int64_t E, int shift, int64_t* __restrict__ counts,
+radix_hist_kernel(Src src, int64_t E, int shift, Count* __restrict__ counts,
                   int* __restrict__ clear) {
   __shared__ int s_hist[kHistCopies][kRadix + 1];
   const int64_t base = static_cast<int64_t>(blockIdx.x) * T::kSize;
@@ -469,7 +469,7 @@ radix_hist_kernel(Src src, int64_t E, int shift, int64_t* __restrict__ counts,
 // edges: 24 us from the words, 14 byte by byte, 13 so (8 with the counts of a tile side by side).
 template <typename T>
 __global__ void __launch_bounds__(T::kThreadsPerTile)
-digit_hist_kernel(const unsigned char* __restrict__ digit, int64_t E, int64_t* __restrict__ counts) {
+digit_hist_kernel(const unsigned char* __restrict__ digit, int64_t E, uint32_t* __restrict__ counts) {
   constexpr int kReads = T::kPerThread / 8;
   __shared__ int s_hist[kHistCopies][kRadix + 1];
   const int64_t base = static_cast<int64_t>(blockIdx.x) * T::kSize;
@@ -503,22 +503,25 @@ digit_hist_kernel(const unsigned char* __restrict__ digit, int64_t E, int64_t* _
 // Where a digit's items of a tile start among that digit's items (offsets[d * num_blocks + b]),
 // and how many the digit has (totals): a workgroup a digit, 2048 tiles at a time.  What the digits
 // below it hold, every workgroup of the pass adds up from the 256 totals by itself.  (One scan over
-// the whole table, which that leaves out, is two launches: 1709 tiles 11 -> 5 us a pass.)
+// the whole table, which that leaves out, is two launches: 1709 tiles 11 -> 5 us a pass.)  The digits
+// whose counts share lines are one die's.
 constexpr int kDigitThreads = 1024;
 constexpr int kDigitItems = 2;
 
+template <typename Count>
 __global__ void __launch_bounds__(kDigitThreads)
-digit_offsets_kernel(const int64_t* __restrict__ counts, int64_t num_blocks,
-                     int64_t* __restrict__ offsets, int64_t* __restrict__ totals) {
+digit_offsets_kernel(const Count* __restrict__ counts, int64_t num_blocks,
+                     Count* __restrict__ offsets, int64_t* __restrict__ totals) {
   __shared__ int64_t s_scan[kDigitThreads / kWave + 1];
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * num_blocks;
+  const int digit = blockIdx.x % kXcds * (kRadix / kXcds) + blockIdx.x / kXcds;
+  const int64_t row = static_cast<int64_t>(digit) * num_blocks;
   int64_t run = 0;
   for (int64_t t0 = 0; t0 < num_blocks; t0 += kDigitThreads * kDigitItems) {
     const int64_t t = t0 + threadIdx.x * kDigitItems;
     int64_t n[kDigitItems], mine = 0;
 #pragma unroll
     for (int k = 0; k < kDigitItems; ++k)
-      n[k] = counts[(t + k < num_blocks ? t + k : 0) * kRadix + blockIdx.x];
+      n[k] = static_cast<int64_t>(counts[(t + k < num_blocks ? t + k : 0) * kRadix + digit]);
 #pragma unroll
     for (int k = 0; k < kDigitItems; ++k) {
       if (t + k >= num_blocks) n[k] = 0;
@@ -528,12 +531,12 @@ digit_offsets_kernel(const int64_t* __restrict__ counts, int64_t num_blocks,
     int64_t at = run + block_exclusive_scan<kDigitThreads>(mine, &all, s_scan);
 #pragma unroll
     for (int k = 0; k < kDigitItems; ++k) {
-      if (t + k < num_blocks) offsets[row + t + k] = at;
+      if (t + k < num_blocks) offsets[row + t + k] = static_cast<Count>(at);
       at += n[k];
     }
     run += all;
   }
-  if (threadIdx.x == 0) totals[blockIdx.x] = run;
+  if (threadIdx.x == 0) totals[digit] = run;
 }
 
 // where the last pass of the sort writes: the values in key order, the permutation, and
@@ -776,7 +779,7 @@ template <typename T, typename IdT, int PASSES, int PASS>
 __global__ void __launch_bounds__(T::kThreadsPerTile, T::kWaves == 16 ? 8 : 4)  // (what LDS allows)
 packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
                    const unsigned long long* __restrict__ in, int64_t E, int value_bits,
-                   int64_t num_blocks, const int64_t* __restrict__ offsets,
+                   int64_t num_blocks, const uint32_t* __restrict__ offsets,
                    const int64_t* __restrict__ totals, const int64_t* __restrict__ totals_before,
                    unsigned long long* __restrict__ out, unsigned char* __restrict__ next_digit,
                    SortOutputs<IdT> last) {
@@ -1163,13 +1166,13 @@ int sort_passes(const IdT* key, const IdT* value, int64_t E, int passes, int idx
     const FreshWords<IdT> fresh{key, idx_bits};
     const StoredWords stored{s.word[(p + 1) & 1]};
     if (p == 0)
-      hipLaunchKernelGGL((radix_hist_kernel<T, FreshWords<IdT>>), grid, dim3(T::kThreadsPerTile), 0,
+      hipLaunchKernelGGL((radix_hist_kernel<T, FreshWords<IdT>, int64_t>), grid, dim3(T::kThreadsPerTile), 0,
                          st, fresh, E, shift, s.counts, outs.wide);
     else
-      hipLaunchKernelGGL((radix_hist_kernel<T, StoredWords>), grid, dim3(T::kThreadsPerTile), 0, st,
+      hipLaunchKernelGGL((radix_hist_kernel<T, StoredWords, int64_t>), grid, dim3(T::kThreadsPerTile), 0, st,
                          stored, E, shift, s.counts, static_cast<int*>(nullptr));
     if (!self)
-      hipLaunchKernelGGL(digit_offsets_kernel, dim3(kRadix), dim3(kDigitThreads), 0, st, s.counts,
+      hipLaunchKernelGGL(digit_offsets_kernel<int64_t>, dim3(kRadix), dim3(kDigitThreads), 0, st, s.counts,
                          blocks, s.offsets, s.totals);
     if (p == 0)
       launch_pass<T>(fresh, last, self, st, value, E, shift, blocks, where, s.totals, s.word[0],
@@ -1198,23 +1201,25 @@ int packed_passes(const IdT* key, const IdT* value, int64_t E, int passes, int v
   const dim3 grid(static_cast<unsigned>(blocks)), threads(T::kThreadsPerTile);
   const int idx_bits = bits_for(E);
   unsigned char* digits = reinterpret_cast<unsigned char*>(s.value[0]);  // (the values have no place of their own)
+  uint32_t* counts = reinterpret_cast<uint32_t*>(s.counts);    // (fewer than 2^32 edges: half the tables' size)
+  uint32_t* offsets = reinterpret_cast<uint32_t*>(s.offsets);
   for (int p = 0; p < passes; ++p) {
     const bool last = p == passes - 1;
     const unsigned long long* in = s.word[(p + 1) & 1];
     if (p == 0)
-      hipLaunchKernelGGL((radix_hist_kernel<T, FreshWords<IdT, T::kStreams>>), grid, threads, 0, st,
-                         FreshWords<IdT, T::kStreams>{key, idx_bits}, E, idx_bits, s.counts, outs.wide);
+      hipLaunchKernelGGL((radix_hist_kernel<T, FreshWords<IdT, T::kStreams>, uint32_t>), grid, threads, 0, st,
+                         FreshWords<IdT, T::kStreams>{key, idx_bits}, E, idx_bits, counts, outs.wide);
     else
-      hipLaunchKernelGGL(digit_hist_kernel<T>, grid, threads, 0, st, digits, E, s.counts);
+      hipLaunchKernelGGL(digit_hist_kernel<T>, grid, threads, 0, st, digits, E, counts);
     int64_t* totals = p & 1 ? s.totals_before : s.totals;
     const int64_t* totals_before = p & 1 ? s.totals : s.totals_before;
-    hipLaunchKernelGGL(digit_offsets_kernel, dim3(kRadix), dim3(kDigitThreads), 0, st, s.counts, blocks,
-                       s.offsets, totals);
+    hipLaunchKernelGGL(digit_offsets_kernel<uint32_t>, dim3(kRadix), dim3(kDigitThreads), 0, st, counts, blocks,
+                       offsets, totals);
     const auto kernel = passes == 2 ? (last ? packed_pass_kernel<T, IdT, 2, 1> : packed_pass_kernel<T, IdT, 2, 0>)
                         : p == 0 ? packed_pass_kernel<T, IdT, 3, 0>
                         : last ? packed_pass_kernel<T, IdT, 3, 2>
                                : packed_pass_kernel<T, IdT, 3, 1>;
-    hipLaunchKernelGGL(kernel, grid, threads, 0, st, key, value, in, E, value_bits, blocks, s.offsets,
+    hipLaunchKernelGGL(kernel, grid, threads, 0, st, key, value, in, E, value_bits, blocks, offsets,
                        totals, totals_before, s.word[p & 1], digits, outs);
   }
   return check_launch("coo2csc");
