@@ -11,12 +11,14 @@
 // between them: each owns a run of consecutive 512-position tiles of the virtual column slice,
 // all runs of equal length and as many waves as the chip holds at once.  Per tile:
 //   * position -> column from 64 staged offsets of the wave's own, bounded to the columns that 64
-//     positions touch (with long columns: no search at all);
-//   * the ids (and data) of the NEXT tile are asked for before this tile's are looked up, since
-//     the few waves beside the set have little else to hide that latency behind;
+//     positions touch (a tile inside one column: one look at the offsets, one address);
+//   * the ids of the NEXT tile are asked for before this tile's marks leave, since the few waves
+//     beside the set have little else to hide that latency behind;
 //   * kept edges leave one bit each and, packed to the front of the tile's range of a scratch
-//     array, their new row number in 2 bytes and their datum.
-// A scan of the tile counts and one copy kernel put the pieces together.  (With the tiles shared
+//     array, their new row number in 2 bytes; every 64 positions leave where they are in the parent.
+// A scan of the tile counts and one copy kernel put the pieces together; the copy reads the kept
+// edges' data from the parent.  (The marks reading them too and packing them beside the row numbers took
+// 185 us and the copy 85 in the case below, 1142 MB together; 967 MB so, 130 and 114.)  (With the tiles shared
 // by the waves of a workgroup, offsets and counts through LDS and two barriers a tile, the marks
 // took 293 us where a wave's own tiles took 225, before they were streamed.)
 //
@@ -28,11 +30,11 @@
 // Its loop over buckets and slots is what bounds it (a kernel of this kind that shared its tiles
 // among the waves took 419 us with it where it took 293 with the bitmap).
 //
-// What bounds the bitmap form: the LDS look-ups and the vector ALUs beside 750 MB in 184 us in the case below,
-// 4.1 TB/s (reads that are truly a tile ahead: 183); more waves than the set leaves room for would be needed to
-// overlap the two better.  7263 nodes whose columns hold 50.8 M edges, 22.0 M kept, 64-bit ids
-// and weights: 184 us for the marks and 71-84 us for the copy (new row numbers in 4 bytes and nothing
-// streamed: 225 + 70), where a filter and a table in the
+// What bounds the bitmap form: nothing alone.  450 MB are 94 us at the rate of a copy, the vector ALUs are busy for
+// 50 us and the LDS for 35 (46 before the bitmap's rows were turned, `slot`), and the four waves a SIMD that the
+// set leaves room for overlap them in part: six and eight waves, fewer instructions and ids out of an L2 each change
+// 130 us by less than 15.  7263 nodes whose columns hold 50.8 M edges, 22.0 M kept, 64-bit ids
+// and weights: 130 us for the marks and 114 us for the copy (517 MB, 4.5 TB/s), where a filter and a table in the
 // L2s, parent positions carried along and a gather of the data behind took 546 + 226 + 104.
 #include "gs_common.hpp"
 
@@ -49,6 +51,7 @@ constexpr int kStagedIds = 8192;          // ids up to which the ids themselves 
 constexpr uint32_t kFree = ~0u;
 constexpr size_t kLdsBytes = 160 * 1024;  // of a compute unit
 constexpr int kUnits = 256;               // compute units
+constexpr int64_t kMostBits = 8 * static_cast<int64_t>(kLdsBytes);
 
 struct InducedMarks {
   unsigned long long* mask;  // one bit per position
@@ -56,54 +59,89 @@ struct InducedMarks {
   int64_t* tile_counts;
   int64_t* tile_base;        // exclusive scan of tile_counts
   uint16_t* packed;          // new row numbers (places, 14 bits) of the kept edges, at the front of the tile's range
-  float* packed_data;        // their data (null: none)
+  int64_t* word_at;          // with data (null: none): where a word's edges are in the parent (WordAt)
   int* outside;              // set when an id lies beyond the bitmap: the call has to be repeated
   int64_t n;
   int64_t tiles;
 };
 
-// A bit per node number below `bound`.
+// Where the edges of 64 consecutive positions are in the parent: the place of the first when they are one
+// column's, else the columns of the first and of the last.
+struct WordAt {
+  __device__ static __forceinline__ int64_t columns(int64_t first, int64_t last) {
+    return INT64_MIN | (last - first) << 32 | first;
+  }
+  __device__ static __forceinline__ bool one(int64_t at) { return at >= 0; }
+  __device__ static __forceinline__ int64_t first(int64_t at) { return at & 0xFFFFFFFF; }
+  __device__ static __forceinline__ int64_t more(int64_t at) { return at >> 32 & 0x7FFFFFFF; }
+};
+
+// use(j, id) for this thread's share of the ids, eight of them asked for together: one trip to memory
+// for eight is what building the set waits for.
+template <int BLOCK, typename IdT, typename Use>
+__device__ __forceinline__ void each_set_id(const IdT* __restrict__ ids, int n, Use use) {
+  constexpr int kTogether = 8;
+  for (int j0 = threadIdx.x; j0 < n; j0 += BLOCK * kTogether) {
+    IdT id[kTogether];
+#pragma unroll
+    for (int u = 0; u < kTogether; ++u) id[u] = ids[j0 + u * BLOCK < n ? j0 + u * BLOCK : n - 1];
+#pragma unroll
+    for (int u = 0; u < kTogether; ++u)
+      if (j0 + u * BLOCK < n) use(j0 + u * BLOCK, id[u]);
+  }
+}
+
+// A bit per node number below `bound`, and a clear one for all others.
 template <typename IdT>
 struct BitmapSet {
   uint32_t* bits;
   uint16_t* before;  // set bits before each word
-  uint32_t* place;   // two to a word: place of the id of every set bit
+  uint32_t* place;   // two to a word: nothing, then the place of the id of every set bit
   uint32_t bound;
 
+  // Words of the bitmap, in rows of 64.  A power-of-two-skewed graph (R-MAT's low ids are its hubs) has most of
+  // its ids in words whose numbers share the lower bits, which are the LDS bank: of the cycles that look-ups kept
+  // the LDS busy, three in four were conflicts.  Every row is turned by its own number.
+  __host__ __device__ static __forceinline__ uint32_t slots(uint32_t bound) { return (bound / 32 + 64) & ~63u; }
+  __device__ static __forceinline__ uint32_t slot(uint32_t id) {
+    const uint32_t word = id >> 5;
+    return (word & ~63u) | ((word + (word >> 6) * 37u) & 63u);
+  }
   static size_t lds_bytes(int64_t bound, int64_t n_ids) {
-    const size_t words = static_cast<size_t>(bound + 31) / 32;
+    if (bound > kMostBits) return SIZE_MAX / 4;
+    const size_t words = slots(static_cast<uint32_t>(bound));
     return (words * 4 + 15) / 16 * 16 + (words * 2 + 15) / 16 * 16 +
-           (static_cast<size_t>(n_ids) * 2 + 15) / 16 * 16;
+           (static_cast<size_t>(n_ids + 1) * 2 + 15) / 16 * 16;
   }
   __device__ __forceinline__ char* carve(char* lds, int64_t bound_, int n_ids) {
-    const size_t words = static_cast<size_t>(bound_ + 31) / 32;
+    const size_t words = slots(static_cast<uint32_t>(bound_));
     bound = static_cast<uint32_t>(bound_);
     bits = reinterpret_cast<uint32_t*>(lds);
     lds += (words * 4 + 15) / 16 * 16;
     before = reinterpret_cast<uint16_t*>(lds);
     lds += (words * 2 + 15) / 16 * 16;
     place = reinterpret_cast<uint32_t*>(lds);
-    return lds + (static_cast<size_t>(n_ids) * 2 + 15) / 16 * 16;
+    return lds + (static_cast<size_t>(n_ids + 1) * 2 + 15) / 16 * 16;
   }
   __device__ __forceinline__ uint32_t rank(uint32_t id) const {
-    return before[id >> 5] + __popc(bits[id >> 5] & ((1u << (id & 31)) - 1u));
+    return before[slot(id)] + __popc(bits[slot(id)] & ((1u << (id & 31)) - 1u));
   }
   // every lane of the workgroup; s_scan: BLOCK / 64 + 1 words
   template <int BLOCK>
   __device__ __forceinline__ void build(const IdT* __restrict__ ids, int n_ids, int64_t* s_scan,
                                         int* outside) {
-    const int words = static_cast<int>((bound + 31) / 32);
+    const int words = static_cast<int>(slots(bound));
     for (int j = threadIdx.x; j < words; j += BLOCK) bits[j] = 0;
-    for (int j = threadIdx.x; j < (n_ids + 1) / 2; j += BLOCK) place[j] = 0;
+    for (int j = threadIdx.x; j < n_ids / 2 + 1; j += BLOCK) place[j] = 0;
     if (blockIdx.x == 0 && threadIdx.x == 0) *outside = 0;
     __syncthreads();
-    for (int j = threadIdx.x; j < n_ids; j += BLOCK) {
-      const uint64_t id = static_cast<uint64_t>(static_cast<int64_t>(ids[j]));
+    each_set_id<BLOCK>(ids, n_ids, [&](int, IdT i) {
+      const uint64_t id = static_cast<uint64_t>(static_cast<int64_t>(i));
       if (id < bound)
-        atomicOr(&bits[id >> 5], 1u << (id & 31));
+        atomicOr(&bits[slot(static_cast<uint32_t>(id))], 1u << (id & 31));
       else if (blockIdx.x == 0)
         *outside = 1;
-    }
+    });
     __syncthreads();
     const int each = (words + BLOCK - 1) / BLOCK;
     const int first = threadIdx.x * each;
@@ -116,10 +154,10 @@ struct BitmapSet {
       run += __popc(bits[j]);
     }
     __syncthreads();
-    for (int j = threadIdx.x; j < n_ids; j += BLOCK) {
-      const uint64_t id = static_cast<uint64_t>(static_cast<int64_t>(ids[j]));
-      if (id >= bound) continue;
-      const uint32_t r = rank(static_cast<uint32_t>(id));
+    each_set_id<BLOCK>(ids, n_ids, [&](int j, IdT i) {
+      const uint64_t id = static_cast<uint64_t>(static_cast<int64_t>(i));
+      if (id >= bound) return;
+      const uint32_t r = rank(static_cast<uint32_t>(id)) + 1;
       const int shift = (r & 1) * 16;
       uint32_t was = place[r >> 1];
       // the same id twice: its last place counts
@@ -129,30 +167,42 @@ struct BitmapSet {
         if (seen == was) break;
         was = seen;
       }
-    }
+    });
     __syncthreads();
   }
-  // val[k] = place of id[k], -1 when it is not in the set
-  __device__ __forceinline__ void lookup(const IdT (&id)[kPer], int (&val)[kPer]) const {
-    uint32_t at[kPer], w[kPer];
+  // in[k]: id[k] is in the set; val[k] its place then (something otherwise).  The bit moved to the
+  // top is the sign, and what is below it are the set bits before it: nine vector instructions an edge.
+  __device__ __forceinline__ void lookup(const IdT (&id)[kPer], int (&val)[kPer], bool (&in)[kPer]) const {
+    uint32_t at[kPer], w[kPer], r[kPer];
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-      const uint64_t v = static_cast<uint64_t>(static_cast<int64_t>(id[k]));
-      at[k] = v < bound ? static_cast<uint32_t>(v) : 0u;
-      w[k] = bits[at[k] >> 5];
-      if (v >= bound) w[k] = 0;
+      const uint32_t low = static_cast<uint32_t>(id[k]);
+      at[k] = low < bound ? low : bound;
     }
-    uint32_t r[kPer];
+    if (sizeof(IdT) == 8) {
+      uint32_t high = 0;
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) high |= static_cast<uint32_t>(static_cast<uint64_t>(id[k]) >> 32);
+      if (__ballot(high != 0)) {
+#pragma unroll
+        for (int k = 0; k < kPer; ++k)
+          if (static_cast<uint64_t>(id[k]) >> 32) at[k] = bound;
+      }
+    }
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-      const uint32_t bit = 1u << (at[k] & 31);
-      r[k] = before[at[k] >> 5] + __popc(w[k] & (bit - 1u));
-      val[k] = w[k] & bit ? 0 : -1;
-      if (val[k]) r[k] = 0;
+      w[k] = bits[slot(at[k])];
+      r[k] = before[slot(at[k])];
+    }
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const uint32_t top = w[k] << (~at[k] & 31);
+      in[k] = static_cast<int>(top) < 0;
+      r[k] += __popc(top);
     }
     const uint16_t* half = reinterpret_cast<const uint16_t*>(place);
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) val[k] |= half[r[k]];
+    for (int k = 0; k < kPer; ++k) val[k] = half[r[k]];
   }
 };
 
@@ -192,8 +242,7 @@ struct BucketSet {
     if (blockIdx.x == 0 && threadIdx.x == 0) *outside = 0;
     for (int j = threadIdx.x; j < kBuckets; j += BLOCK)
       bucket[j] = make_uint4(kFree, kFree, kFree, kFree);
-    if (STAGED)
-      for (int j = threadIdx.x; j < n_ids; j += BLOCK) s_ids[j] = list[j];
+    if (STAGED) each_set_id<BLOCK>(list, n_ids, [&](int j, IdT id) { s_ids[j] = id; });
     __syncthreads();
     uint32_t* slot = reinterpret_cast<uint32_t*>(bucket);
     for (int j = threadIdx.x; j < n_ids; j += BLOCK) {
@@ -213,7 +262,7 @@ struct BucketSet {
     }
     __syncthreads();
   }
-  __device__ __forceinline__ void lookup(const IdT (&id)[kPer], int (&val)[kPer]) const {
+  __device__ __forceinline__ void lookup(const IdT (&id)[kPer], int (&val)[kPer], bool (&in)[kPer]) const {
 #pragma unroll
     for (int half = 0; half < kPer; half += 4) {
       uint4 b[4];
@@ -254,6 +303,7 @@ struct BucketSet {
           b[k] = bucket[at];
         }
         val[half + k] = found;
+        in[half + k] = found >= 0;
       }
     }
   }
@@ -268,16 +318,15 @@ __device__ __forceinline__ int row_of(const int64_t* off, int lo, int hi, int64_
   return lo;
 }
 
-// What a wave's edges bring along: nothing, data[position], or data[e_ids[position]].
+// What a kept edge brings along: nothing, data[position], or data[e_ids[position]].
 enum Data { kNoData, kByPosition, kByEdgeId };
 
-template <typename IdT, typename Set, int BLOCK, Data DATA, bool STREAM>
-__global__ void __launch_bounds__(BLOCK, 4)  // (16 waves a compute unit: what the set leaves room for)
+template <typename IdT, typename Set, int BLOCK, int WAVES, bool PLACES, bool STREAM>
+__global__ void __launch_bounds__(BLOCK, WAVES)  // (waves a SIMD)
 induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
                     const IdT* __restrict__ indices, const IdT* __restrict__ cols, int64_t S,
                     const int64_t* __restrict__ sub_indptr, int64_t D, const IdT* __restrict__ ids,
-                    int n_ids, int64_t bound, const float* __restrict__ data,
-                    const int64_t* __restrict__ e_ids, int64_t tiles_each, InducedMarks m) {
+                    int n_ids, int64_t bound, InducedMarks m) {
   __shared__ int64_t s_offsets[BLOCK / kWave][kWindow + 1];
   __shared__ int64_t s_starts[BLOCK / kWave][kWindow];  // start of the column minus its offset
   __shared__ int64_t s_scan[BLOCK / kWave + 1];
@@ -286,11 +335,11 @@ induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
   set.carve(lds, bound, n_ids);
   set.template build<BLOCK>(ids, n_ids, s_scan, m.outside);
 
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // (a scalar, and so is all that follows from it)
   constexpr int kStep = BLOCK / kWave;  // the waves of a workgroup take turns along its run
-  const int64_t run = static_cast<int64_t>(blockIdx.x) * kStep * tiles_each;
-  const int64_t tile0 = run + wave;
-  const int64_t tile1 = run + kStep * tiles_each < m.tiles ? run + kStep * tiles_each : m.tiles;
+  const int64_t tile0 = m.tiles * blockIdx.x / gridDim.x + wave;
+  const int64_t tile1 = m.tiles * (blockIdx.x + 1) / gridDim.x;
   if (tile0 >= tile1) return;  // (no barrier from here on)
 
   int64_t* off = s_offsets[wave];
@@ -320,11 +369,20 @@ induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
     __builtin_amdgcn_wave_barrier();
   };
 
-  // where the 64 positions from q on lie in the parent (q never decreases)
-  auto locate = [&](int64_t q) -> int64_t {
+  // the column of position q, where a tile begins: its place in the window from one look at all offsets
+  auto settle = [&](int64_t q) {
+    if (off[kWindow] <= q) stage(wave_upper_bound(sub_indptr, S + 1, q) - 1);
+    row = __popcll(__ballot(off[lane + 1] <= q));
+    row_end = uniform(off[row + 1]);
+    row_start = uniform(start[row]);
+  };
+
+  // where the 64 positions from q on lie in the parent (q never decreases); word_at: the same as a WordAt
+  auto locate = [&](int64_t q, int64_t& word_at) -> int64_t {
     const int64_t last = (q + kWave < D ? q + kWave : D) - 1;
     int64_t p = q + lane;
     p = p < last ? p : last;
+    word_at = row_start + q;
     if (last < row_end) return row_start + p;
     if (off[kWindow] <= last) {
       // the window ends among them: the next one starts at the column of the first
@@ -342,66 +400,64 @@ induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
         const int64_t mid = (lo + hi) >> 1;
         if (sub_indptr[mid + 1] > p) hi = mid; else lo = mid + 1;
       }
+      if (PLACES) word_at = WordAt::columns(__shfl(lo, 0, kWave), __shfl(lo, kWave - 1, kWave));
       return indptr[static_cast<int64_t>(cols[lo])] + p - sub_indptr[lo];
     }
     if (off[row + 1] <= q) row = row_of(off, row + 1, kWindow - 1, q);
     row_end = uniform(off[row + 1]);
     row_start = uniform(start[row]);
+    word_at = row_start + q;
     if (last < row_end) return row_start + p;
     const int r = row_of(off, row, kWindow - 1, p);
+    if (PLACES) word_at = WordAt::columns(window + row, window + __builtin_amdgcn_readlane(r, kWave - 1));
     return start[r] + p;
   };
 
-  struct Held {
-    IdT id[kPer];
-    float w[DATA == kByPosition ? kPer : 1];
-    int64_t e[DATA == kByEdgeId ? kPer : 1];
-  };
   // (STREAM: beyond the caches' size what a call reads is gone from them before anyone reads it again)
   auto once = [](const auto* p) { return STREAM ? __builtin_nontemporal_load(p) : *p; };
-  auto fetch = [&](int64_t t, Held& h) {
+  IdT id[kPer];
+  int64_t next_at = 0, my_at = 0;  // lane k: of word k of the tile asked for and of this one
+  auto fetch = [&](int64_t t) {
+    const int64_t q0 = t * kTile;
+    if (q0 >= row_end) settle(q0);
+    if (q0 + kTile <= row_end) {  // inside one column: one address
+      const IdT* from = indices + row_start + q0 + lane;
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) id[k] = once(from + k * kWave);
+      if (PLACES) next_at = row_start + q0 + lane * kWave;
+      return;
+    }
     int64_t at[kPer];
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-      const int64_t q = t * kTile + k * kWave;
-      at[k] = locate(q < D ? q : D - 1);
+      const int64_t q = q0 + k * kWave;
+      int64_t word_at;
+      at[k] = locate(q < D ? q : D - 1, word_at);
+      if (PLACES && lane == k) next_at = word_at;
     }
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) h.id[k] = once(indices + at[k]);
-    // (the data of all: 64 neighbours share their lines with the kept ones among them)
-    if constexpr (DATA == kByPosition) {
-#pragma unroll
-      for (int k = 0; k < kPer; ++k) h.w[k] = once(data + at[k]);
-    }
-    if constexpr (DATA == kByEdgeId) {
-#pragma unroll
-      for (int k = 0; k < kPer; ++k) h.e[k] = once(e_ids + at[k]);
-    }
+    for (int k = 0; k < kPer; ++k) id[k] = once(indices + at[k]);
   };
 
-  Held now, next;
   stage(wave_upper_bound(sub_indptr, S + 1, tile0 * kTile) - 1);
-  fetch(tile0, now);
+  fetch(tile0);
   for (int64_t t = tile0; t < tile1; t += kStep) {
-    if (t + kStep < tile1) fetch(t + kStep, next);
     const int64_t p0 = t * kTile;
     int val[kPer];
-    set.lookup(now.id, val);
+    bool in[kPer];
+    set.lookup(id, val, in);
+    my_at = next_at;
+    if (t + kStep < tile1) fetch(t + kStep);
     if (p0 + kTile > D) {
 #pragma unroll
       for (int k = 0; k < kPer; ++k)
-        if (p0 + k * kWave + lane >= D) val[k] = -1;
-    }
-    float w[DATA == kNoData ? 1 : kPer];
-    if constexpr (DATA == kByEdgeId) {
-#pragma unroll
-      for (int k = 0; k < kPer; ++k) w[k] = val[k] >= 0 ? data[now.e[k]] : 0.0f;
+        if (p0 + k * kWave + lane >= D) in[k] = false;
     }
     int before = 0, my_before = 0;
     unsigned long long my_word = 0;
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-      const unsigned long long kept = __ballot(val[k] >= 0);
+      const unsigned long long kept = __ballot(in[k]);
       if (lane == k) {
         my_word = kept;
         my_before = before;
@@ -410,18 +466,14 @@ induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
                                                           __builtin_amdgcn_mbcnt_lo(
                                                               static_cast<uint32_t>(kept), 0));
       before += __popcll(kept);
-      if (val[k] >= 0) {
-        m.packed[p0 + rank] = static_cast<uint16_t>(val[k]);
-        if constexpr (DATA == kByPosition) m.packed_data[p0 + rank] = now.w[k];
-        if constexpr (DATA == kByEdgeId) m.packed_data[p0 + rank] = w[k];
-      }
+      if (in[k]) m.packed[p0 + rank] = static_cast<uint16_t>(val[k]);
     }
     if (lane < kPer && p0 + lane * kWave < D) {
       m.mask[(p0 >> 6) + lane] = my_word;
       m.word_rank[(p0 >> 6) + lane] = my_before;
+      if (PLACES) m.word_at[(p0 >> 6) + lane] = my_at;
     }
     if (lane == 0) m.tile_counts[t] = before;
-    now = next;
   }
 }
 
@@ -446,42 +498,99 @@ induced_indptr_kernel(const int64_t* __restrict__ sub_indptr, int64_t S, Induced
 }
 
 // Every tile's kept edges from the front of its range to their place in the result, a wave at a
-// time: eight times 64, all reads before the stores.
+// time: eight times 64, all reads before the stores.  The data come from the parent, word by word.
 constexpr int kCopyTiles = 4;  // of a workgroup, one for every wave
 
-template <typename IdT, bool STREAM>
+template <typename IdT, Data DATA, bool STREAM>
 __global__ void __launch_bounds__(256)
-induced_compact_kernel(InducedMarks m, IdT* __restrict__ out_indices, float* __restrict__ out_data) {
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const IdT* __restrict__ cols,
+                       const int64_t* __restrict__ sub_indptr, const float* __restrict__ data,
+                       const int64_t* __restrict__ e_ids, IdT* __restrict__ out_indices,
+                       float* __restrict__ out_data) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // (a scalar, and so are all addresses' bases)
   const int64_t t = static_cast<int64_t>(blockIdx.x) * kCopyTiles + wave;
   if (t >= m.tiles) return;
   const int64_t base = m.tile_base[t];
   const int count = static_cast<int>(m.tile_base[t + 1] - base);
+  unsigned long long my_word = 0;  // lane k: word k of the tile
+  int my_rank = 0;
+  int64_t my_at = 0;
+  if (DATA != kNoData && lane < kPer && t * kTile + lane * kWave < m.n) {
+    my_word = m.mask[t * kPer + lane];
+    my_rank = m.word_rank[t * kPer + lane];
+    my_at = m.word_at[t * kPer + lane];
+  }
   if (count == 0) return;
+  auto once = [](const auto* p) { return STREAM ? __builtin_nontemporal_load(p) : *p; };
   uint16_t v[kPer];
-  float x[kPer];
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     const int r = k * kWave + lane;
     v[k] = m.packed[t * kTile + (r < count ? r : count - 1)];
   }
-  if (out_data) {
+  bool kept[DATA == kNoData ? 1 : kPer];
+  int rank[DATA == kNoData ? 1 : kPer];
+  float x[DATA == kNoData ? 1 : kPer];
+  if constexpr (DATA != kNoData) {
+    auto of = [](uint64_t u, int k) {  // lane k's
+      return static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u >> 32), k))) << 32 |
+             static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u), k));
+    };
+    int64_t at[kPer];
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-      const int r = k * kWave + lane;
-      x[k] = m.packed_data[t * kTile + (r < count ? r : count - 1)];
+      const uint64_t word = of(my_word, k);
+      const int64_t where = static_cast<int64_t>(of(static_cast<uint64_t>(my_at), k));
+      kept[k] = word >> lane & 1u;
+      rank[k] = __builtin_amdgcn_readlane(my_rank, k) +
+                __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(word >> 32),
+                                          __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(word), 0));
+      // (lanes whose edge is left out read with the word's first kept one, a word without any the first datum:
+      // data may end before edges that are not kept)
+      const int place = kept[k] ? lane : (word ? __builtin_ctzll(word) : 0);
+      if (!word) {
+        at[k] = 0;
+      } else if (WordAt::one(where)) {
+        at[k] = where + place;
+      } else {
+        const int64_t p = t * kTile + k * kWave + place;
+        int64_t lo = WordAt::first(where), hi = lo + WordAt::more(where);
+        while (lo < hi) {
+          const int64_t mid = (lo + hi) >> 1;
+          if (sub_indptr[mid + 1] > p) hi = mid; else lo = mid + 1;
+        }
+        at[k] = indptr[static_cast<int64_t>(cols[lo])] + p - sub_indptr[lo];
+      }
     }
+    if constexpr (DATA == kByEdgeId) {
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) {
+        const int64_t e = once(e_ids + at[k]);
+        at[k] = of(my_word, k) ? e : 0;  // (data may end before edges that are not kept)
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) x[k] = once(data + at[k]);
   }
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     const int r = k * kWave + lane;
     if (r < count) {
-      if (STREAM) {
+      if (STREAM)
         __builtin_nontemporal_store(static_cast<IdT>(v[k]), out_indices + base + r);
-        if (out_data) __builtin_nontemporal_store(x[k], out_data + base + r);
-      } else {
+      else
         out_indices[base + r] = static_cast<IdT>(v[k]);
-        if (out_data) out_data[base + r] = x[k];
+    }
+  }
+  if constexpr (DATA != kNoData) {
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      if (kept[k]) {
+        if (STREAM)
+          __builtin_nontemporal_store(x[k], out_data + base + rank[k]);
+        else
+          out_data[base + rank[k]] = x[k];
       }
     }
   }
@@ -501,7 +610,7 @@ bool carve_induced(void* workspace, size_t bytes, int64_t D, bool with_data, Ind
   *scan_tiles = ws.take<int64_t>(static_cast<size_t>(scan_num_tiles(m->tiles) + 1));
   m->outside = ws.take<int>(1);
   m->packed = ws.take<uint16_t>(static_cast<size_t>(D));
-  m->packed_data = with_data ? ws.take<float>(static_cast<size_t>(D)) : nullptr;
+  m->word_at = with_data ? ws.take<int64_t>(words) : nullptr;
   return ws.ok;
 }
 
@@ -514,23 +623,24 @@ struct MarkCall {
   int64_t D;
   const void* ids;
   int64_t n_ids, bound;
-  const float* data;
-  const int64_t* e_ids;
+  bool with_data;
 };
 
 // Whether the ids and data of D positions are more than the 256 MB that the memory-side cache holds.
-// The whole call (walk, unique nodes and subgraph), plain / streamed: 50.8 M positions with 64-bit ids and data (610 MB)
-// 398-412 / 383-394 us (marks 216 / 185, copy 67 / 84: who stores past the cache leaves it to the other);
+// The whole call (walk, unique nodes and subgraph), plain / streamed, with the data read by the marks: 50.8 M positions
+// with 64-bit ids and data (610 MB) 398-412 / 383-394 us;
 // graphs of 100 M edges, 1.5 M nodes and of 50 M, 0.2 M, a few hundred seeds, 32-bit ids 217 / 216, 157 / 159.
 inline bool streams(int64_t D, size_t id_bytes, bool with_data) {
   return D * static_cast<int64_t>(id_bytes + (with_data ? 4 : 0)) >= int64_t(1) << 28;
 }
 
-template <typename IdT, typename Set, int BLOCK, Data DATA>
+template <typename IdT, typename Set, int BLOCK, int WAVES>
 int launch_mark(const MarkCall& c, int per_unit, const InducedMarks& m, hipStream_t st) {
-  auto* kernel = streams(c.D, sizeof(IdT), DATA != kNoData)
-                     ? induced_mark_kernel<IdT, Set, BLOCK, DATA, true>
-                     : induced_mark_kernel<IdT, Set, BLOCK, DATA, false>;
+  const bool past = streams(c.D, sizeof(IdT), c.with_data);
+  auto* kernel = c.with_data ? (past ? induced_mark_kernel<IdT, Set, BLOCK, WAVES, true, true>
+                                     : induced_mark_kernel<IdT, Set, BLOCK, WAVES, true, false>)
+                             : (past ? induced_mark_kernel<IdT, Set, BLOCK, WAVES, false, true>
+                                     : induced_mark_kernel<IdT, Set, BLOCK, WAVES, false, false>);
   const size_t bytes = Set::lds_bytes(c.bound, c.n_ids);
   // (per call: the attribute belongs to the device the call runs on)
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -539,21 +649,12 @@ int launch_mark(const MarkCall& c, int per_unit, const InducedMarks& m, hipStrea
     set_error_text("gs_induced_slice_mark: %s", hipGetErrorString(hipGetLastError()));
     return GS_ERR_LAUNCH;
   }
-  const int64_t waves = static_cast<int64_t>(kUnits) * per_unit * (BLOCK / kWave);
-  const int64_t each = (m.tiles + waves - 1) / waves;
-  hipLaunchKernelGGL(kernel, dim3(blocks_for(m.tiles, static_cast<int>(each * (BLOCK / kWave)))),
+  const int64_t runs = (m.tiles + BLOCK / kWave - 1) / (BLOCK / kWave), most = int64_t(kUnits) * per_unit;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(runs < most ? runs : most)),
                      dim3(BLOCK), bytes, st, c.indptr, c.num_cols, static_cast<const IdT*>(c.indices),
                      static_cast<const IdT*>(c.cols), c.S, c.sub_indptr, c.D,
-                     static_cast<const IdT*>(c.ids), static_cast<int>(c.n_ids), c.bound, c.data,
-                     c.e_ids, each, m);
+                     static_cast<const IdT*>(c.ids), static_cast<int>(c.n_ids), c.bound, m);
   return check_launch("induced_slice_mark");
-}
-
-template <typename IdT, typename Set, int BLOCK>
-int launch_mark(const MarkCall& c, int per_unit, const InducedMarks& m, hipStream_t st) {
-  if (!c.data) return launch_mark<IdT, Set, BLOCK, kNoData>(c, per_unit, m, st);
-  if (!c.e_ids) return launch_mark<IdT, Set, BLOCK, kByPosition>(c, per_unit, m, st);
-  return launch_mark<IdT, Set, BLOCK, kByEdgeId>(c, per_unit, m, st);
 }
 
 // LDS that the kernel declares itself
@@ -567,12 +668,26 @@ template <typename IdT>
 int pick_mark(const MarkCall& c, const InducedMarks& m, hipStream_t st) {
   const size_t bitmap = BitmapSet<IdT>::lds_bytes(c.bound, c.n_ids);
   if (2 * (bitmap + fixed_lds(512)) <= kLdsBytes)
-    return launch_mark<IdT, BitmapSet<IdT>, 512>(c, 2, m, st);
+    return launch_mark<IdT, BitmapSet<IdT>, 512, 4>(c, 2, m, st);
   if (bitmap + fixed_lds(1024) <= kLdsBytes)
-    return launch_mark<IdT, BitmapSet<IdT>, 1024>(c, 1, m, st);
+    return launch_mark<IdT, BitmapSet<IdT>, 1024, 4>(c, 1, m, st);
   static_assert(size_t(1 << 13) * 16 + fixed_lds(1024) <= kLdsBytes, "buckets");
-  if (c.n_ids <= kStagedIds) return launch_mark<IdT, BucketSet<IdT, true>, 1024>(c, 1, m, st);
-  return launch_mark<IdT, BucketSet<IdT, false>, 1024>(c, 1, m, st);
+  if (c.n_ids <= kStagedIds) return launch_mark<IdT, BucketSet<IdT, true>, 1024, 4>(c, 1, m, st);
+  return launch_mark<IdT, BucketSet<IdT, false>, 1024, 4>(c, 1, m, st);
+}
+
+template <typename IdT>
+void launch_compact(int64_t D, const InducedMarks& m, const int64_t* indptr, const void* cols,
+                    const int64_t* sub_indptr, const float* data, const int64_t* e_ids, IdT* out_indices,
+                    float* out_data, hipStream_t st) {
+  const bool past = streams(D, sizeof(IdT), data != nullptr);
+  auto* kernel = !data    ? (past ? induced_compact_kernel<IdT, kNoData, true> : induced_compact_kernel<IdT, kNoData, false>)
+                 : !e_ids ? (past ? induced_compact_kernel<IdT, kByPosition, true>
+                                  : induced_compact_kernel<IdT, kByPosition, false>)
+                          : (past ? induced_compact_kernel<IdT, kByEdgeId, true>
+                                  : induced_compact_kernel<IdT, kByEdgeId, false>);
+  hipLaunchKernelGGL(kernel, dim3(blocks_for(m.tiles, kCopyTiles)), dim3(256), 0, st, m, indptr,
+                     static_cast<const IdT*>(cols), sub_indptr, data, e_ids, out_indices, out_data);
 }
 
 }  // namespace
@@ -591,7 +706,7 @@ extern "C" {
 //   positions / columns 4, 8, 12, 16, 32    94/89 94/94 97/96 98/92 93/91    93/93 89/88 88/85 87/89 87/82
 // so the lines lie where nothing is lost with either form.  nnz does not matter.
 int gs_induced_slice_applies(int64_t num_row_ids, int64_t S, int64_t D, int64_t) {
-  return num_row_ids > 0 && num_row_ids <= kMaxIds && S > 0 && D >= (int64_t(1) << 20) && D >= 16 * S;
+  return num_row_ids > 0 && num_row_ids <= kMaxIds && S > 0 && S < (int64_t(1) << 31) && D >= (int64_t(1) << 20) && D >= 16 * S;
 }
 
 size_t gs_induced_slice_workspace_bytes(int64_t D, int with_data) {
@@ -600,7 +715,7 @@ size_t gs_induced_slice_workspace_bytes(int64_t D, int with_data) {
   const int64_t tiles = ((D - 1) >> kTileShift) + 1;
   return padded(words * 8) + padded(words * 4) + padded(static_cast<size_t>(tiles + 1) * 8) +
          padded(static_cast<size_t>(tiles + 2) * 8) + scan_workspace_bytes(tiles) + 256 +
-         padded(n * 2) + (with_data ? padded(n * 4) : 0);
+         padded(n * 2) + (with_data ? padded(words * 8) : 0);
 }
 
 int gs_induced_slice_mark(const int64_t* indptr, int64_t num_cols, const void* indices, int64_t nnz,
@@ -625,7 +740,7 @@ int gs_induced_slice_mark(const int64_t* indptr, int64_t num_cols, const void* i
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t bound = num_rows > 0 ? num_rows : int64_t(1) << 40;  // (no bound given: no bitmap)
   const MarkCall c{indptr, num_cols, indices, column_ids, S, sub_indptr, D, row_ids, num_row_ids,
-                   bound, edge_data, edge_ids};
+                   bound, edge_data != nullptr};
   GS_RETURN_IF_ERROR(id_bytes == 8 ? pick_mark<int64_t>(c, m, st) : pick_mark<int32_t>(c, m, st));
   TileCount f{m.tile_counts};
   GS_RETURN_IF_ERROR(exclusive_scan(f, m.tiles, m.tile_base, scan_tiles, st));
@@ -634,9 +749,12 @@ int gs_induced_slice_mark(const int64_t* indptr, int64_t num_cols, const void* i
   return check_launch("induced_slice_mark");
 }
 
-int gs_induced_slice_compact(int64_t D, int id_bytes, void* out_indices, float* out_data,
+int gs_induced_slice_compact(const int64_t* indptr, int id_bytes, const void* column_ids,
+                             const int64_t* sub_indptr, int64_t D, const float* edge_data,
+                             const int64_t* edge_ids, void* out_indices, float* out_data,
                              void* workspace, size_t workspace_bytes, void* stream) {
-  GS_REQUIRE(D > 0 && out_indices, "gs_induced_slice_compact: bad argument");
+  GS_REQUIRE(D > 0 && out_indices && indptr && column_ids && sub_indptr, "gs_induced_slice_compact: bad argument");
+  GS_REQUIRE(!edge_data == !out_data, "gs_induced_slice_compact: data without a place for them, or the other way round");
   GS_REQUIRE(valid_id_bytes(id_bytes), "gs_induced_slice_compact: id_bytes must be 4 or 8, got %d",
              id_bytes);
   InducedMarks m;
@@ -646,17 +764,12 @@ int gs_induced_slice_compact(int64_t D, int id_bytes, void* out_indices, float* 
     return GS_ERR_WORKSPACE;
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const dim3 grid(blocks_for(m.tiles, kCopyTiles));
-  const bool stream_out = streams(D, static_cast<size_t>(id_bytes), out_data != nullptr);
-  auto go = [&](auto* kernel, auto* indices) {
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, m, indices, out_data);
-  };
   if (id_bytes == 8)
-    go(stream_out ? induced_compact_kernel<int64_t, true> : induced_compact_kernel<int64_t, false>,
-       static_cast<int64_t*>(out_indices));
+    launch_compact(D, m, indptr, column_ids, sub_indptr, edge_data, edge_ids,
+                   static_cast<int64_t*>(out_indices), out_data, st);
   else
-    go(stream_out ? induced_compact_kernel<int32_t, true> : induced_compact_kernel<int32_t, false>,
-       static_cast<int32_t*>(out_indices));
+    launch_compact(D, m, indptr, column_ids, sub_indptr, edge_data, edge_ids,
+                   static_cast<int32_t*>(out_indices), out_data, st);
   return check_launch("induced_slice_compact");
 }
 

@@ -1453,7 +1453,9 @@ std::tuple<torch::Tensor, torch::Tensor> InducedSlicing(const torch::Tensor& ind
   auto out_indices = torch::empty({kept}, indices.options());
   if (edge) *data_out = torch::empty({kept}, edge->data.options());
   if (kept > 0)
-    Check(gs_induced_slice_compact(D, idb, out_indices.data_ptr(),
+    Check(gs_induced_slice_compact(indptr.data_ptr<int64_t>(), idb, column_ids.data_ptr(),
+                                   sub_indptr.data_ptr<int64_t>(), D, edge ? edge->data.data_ptr<float>() : nullptr,
+                                   edge ? OptI64(edge->e_ids, "e_ids") : nullptr, out_indices.data_ptr(),
                                    edge ? data_out->data_ptr<float>() : nullptr, ws.data_ptr(),
                                    ws.numel(), st),
           "gs_induced_slice_compact");

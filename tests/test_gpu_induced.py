@@ -181,6 +181,40 @@ def test_short_columns(dev, hubs, hub_degree, small, n, columns, weights):
         assert np.array_equal(sub._CAPI_GetData("default").cpu().numpy(), w[want[3]])
 
 
+@pytest.mark.parametrize("n", [31, 32, 2016, 2047, 2048, 70_001])
+@pytest.mark.parametrize("map", [False, True])
+def test_bitmap_rows_and_data_from_the_parent(dev, n, map):
+    """Bounds at the ends of the bitmap's words and of its rows of 64 words, every id at the bound's edge; data found
+    word by word in words of one column, of several and of more columns than are staged, by position and by a
+    map."""
+    rng = np.random.default_rng(n)
+    degree = np.concatenate([[700_001, 0, 511, 1, 64, 63, 65], np.zeros(130, int), [448_000, 3, 2, 1, 1]])
+    degree = np.resize(degree, n) if n < degree.size else np.concatenate([degree, np.ones(n - degree.size, int)])
+    degree[0] += max(0, (1 << 20) - degree.sum())
+    indptr = np.concatenate([[0], np.cumsum(degree)]).astype(np.int64)
+    E = int(indptr[-1])
+    indices = rng.integers(0, n, E).astype(np.int64)
+    rows = np.concatenate([[n - 1, 0], rng.permutation(n)[: min(n, 3000)]]).astype(np.int64)  # (two ids twice)
+    order = np.arange(E)
+    g = gs.Graph(False)
+    if map:
+        shuffle = rng.permutation(E)
+        col, row = np.repeat(np.arange(n), degree)[shuffle], indices[shuffle]
+        order = np.argsort(col, kind="stable")
+        indices = row[order]
+        g._CAPI_LoadCOO(to_dev(row, dev), to_dev(col, dev))
+    else:
+        g._CAPI_LoadCSC(to_dev(indptr, dev), to_dev(indices, dev))
+    w = rng.random(E).astype(np.float32)
+    g._CAPI_SetData(to_dev(w, dev))
+    cols = np.arange(n).astype(np.int64)
+    sub = g._CAPI_FusionSlicing(to_dev(cols, dev), to_dev(rows, dev))
+    want = O.col_row_slice(indptr, indices, cols, rows)
+    assert np.array_equal(sub._CAPI_GetCSC()[0].cpu().numpy(), want[0])
+    assert np.array_equal(sub._CAPI_GetCSC()[1].cpu().numpy(), want[1])
+    assert np.array_equal(sub._CAPI_GetData("default").cpu().numpy(), w[order][want[3]])
+
+
 # more bytes of ids and data than are read through the caches; both forms of the set
 @pytest.mark.parametrize("idt", [torch.int32, torch.int64])
 @pytest.mark.parametrize("n", [60_000, 2_000_000])
