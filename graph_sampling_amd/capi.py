@@ -637,8 +637,9 @@ class _Span(ctypes.Structure):
 NARROW_IDS = 0x100  # GS_NARROW_IDS: 64-bit ids that fit 32 bits, on one-word table slots
 
 
-def unique_relabel(mapping, queries, mailbox=None, last_span_len=None, narrow=False):
-    """gs_unique_relabel[_notify].  mapping / queries: lists of 1-D id tensors (one dtype).
+def unique_relabel(mapping, queries, mailbox=None, last_span_len=None, narrow=False, places=None):
+    """gs_unique_relabel[_notify, _places].  mapping / queries: lists of 1-D id tensors (one dtype);
+    places[q] >= 0: query q holds places in that mapping tensor.
 
     Returns (frontier_buf, num_unique_dev, [relabelled query tensors]); frontier_buf has
     capacity sum(len(mapping)) and num_unique_dev is a 1-element int64 device tensor.  With a
@@ -669,6 +670,14 @@ def unique_relabel(mapping, queries, mailbox=None, last_span_len=None, narrow=Fa
                                               _i64(ticket), _stream(dev)),
                "gs_unique_relabel_notify")
         return frontier, num_unique, outs, ticket
+    if places is not None:
+        spans = (ctypes.c_int * max(len(queries), 1))(*places)
+        _check(lib().gs_unique_relabel_places(m_arr, len(mapping), q_arr, spans, o_arr, len(queries), idb,
+                                              _ptr(frontier), _ptr(num_unique), _ptr(ws),
+                                              ctypes.c_size_t(ws.numel()), ctypes.c_void_p(0),
+                                              ctypes.c_void_p(0), _i64(0), _stream(dev)),
+               "gs_unique_relabel_places")
+        return frontier, num_unique, outs
     _check(lib().gs_unique_relabel(m_arr, len(mapping), q_arr, o_arr, len(queries), idb,
                                    _ptr(frontier), _ptr(num_unique), _ptr(ws),
                                    ctypes.c_size_t(ws.numel()), _stream(dev)), "gs_unique_relabel")

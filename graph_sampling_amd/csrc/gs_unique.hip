@@ -176,6 +176,10 @@ struct Query {
   void* out[GS_MAX_SPANS];
   int64_t end[GS_MAX_SPANS];    // exclusive end offset in the concatenation of queries
   int64_t alias[GS_MAX_SPANS];  // >= 0: the query is the mapping span starting there
+  // >= 0: the query holds places in the mapping span that starts there, of via_n items: the rank of the id at such a
+  // place is asked for, which the compaction has set aside (a gather of the ids in a launch in front and a search
+  // for each in the table took longer: 5000 columns sampled by weight, 86 k edges, sampled and relabelled 120 -> 112 us)
+  int64_t via[GS_MAX_SPANS], via_n[GS_MAX_SPANS];
   int n;
 };
 
@@ -298,6 +302,9 @@ lookup_kernel(T t, const uint32_t* __restrict__ first_of, const int64_t* __restr
   if (qs.alias[s] >= 0) {
     // a query that is one of the mapping spans: the compaction has set its first indices aside
     first = first_of[qs.alias[s] + local];
+  } else if (qs.via[s] >= 0) {
+    const int64_t place = static_cast<int64_t>(static_cast<const IdT*>(qs.in[s])[local]);
+    first = place >= 0 && place < qs.via_n[s] ? static_cast<int64_t>(first_of[qs.via[s] + place]) : -1;
   } else {
     const IdT key = static_cast<const IdT*>(qs.in[s])[local];
     const bool fits = sizeof(IdT) == 4 || !std::is_same<T, PackedTable>::value ||
@@ -467,6 +474,7 @@ unique_one_kernel(Spans<IdT> x, int M, int slots, Query qs, int Q, IdT* __restri
   for (int j0 = threadIdx.x; j0 < Q; j0 += kBatch * kOneThreads) {
     IdT key[kBatch];
     IdT* to[kBatch];
+    unsigned int none = 0u;  // places outside their span
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       const int j = j0 + u * kOneThreads < Q ? j0 + u * kOneThreads : Q - 1;
@@ -481,12 +489,18 @@ unique_one_kernel(Spans<IdT> x, int M, int slots, Query qs, int Q, IdT* __restri
       }
       key[u] = static_cast<const IdT*>(qs.in[s])[j - begin];
       to[u] = static_cast<IdT*>(qs.out[s]) + (j - begin);
+      if (qs.via[s] >= 0) {
+        const int64_t place = static_cast<int64_t>(key[u]);
+        const bool there = place >= 0 && place < qs.via_n[s];
+        key[u] = x.get(qs.via[s] + (there ? place : 0));
+        none |= there ? 0u : 1u << u;
+      }
     }
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       if (j0 + u * kOneThreads < Q) {
         const int64_t rank =
-            fits_slot(key[u]) ? t.find(static_cast<long long>(static_cast<uint32_t>(key[u]))) : -1;
+            fits_slot(key[u]) && !(none >> u & 1u) ? t.find(static_cast<long long>(static_cast<uint32_t>(key[u]))) : -1;
         *to[u] = static_cast<IdT>(rank);
       }
     }
@@ -520,9 +534,10 @@ int unique_one(const Spans<IdT>& x, int64_t M, const Query& qs, int64_t Q, IdT* 
 
 template <typename IdT, typename T>
 int unique_relabel_impl(const gs_span* mapping, int n_mapping, const gs_span* query,
-                        void* const* query_out, int n_query, void* frontier, int64_t* num_unique,
-                        void* workspace, size_t workspace_bytes, const int64_t* last_span_len,
-                        gs_mailbox* box, int64_t box_ticket, hipStream_t stream) {
+                        const int* query_span, void* const* query_out, int n_query, void* frontier,
+                        int64_t* num_unique, void* workspace, size_t workspace_bytes,
+                        const int64_t* last_span_len, gs_mailbox* box, int64_t box_ticket,
+                        hipStream_t stream) {
   Spans<IdT> x;
   int64_t M = 0;
   for (int s = 0; s < GS_MAX_SPANS; ++s) {
@@ -560,6 +575,8 @@ int unique_relabel_impl(const gs_span* mapping, int n_mapping, const gs_span* qu
     qs.out[q] = nullptr;
     qs.end[q] = 0;
     qs.alias[q] = -1;
+    qs.via[q] = -1;
+    qs.via_n[q] = 0;
   }
   for (int q = 0; q < n_query; ++q) {
     qs.in[q] = query[q].ptr;
@@ -568,7 +585,14 @@ int unique_relabel_impl(const gs_span* mapping, int n_mapping, const gs_span* qu
     qs.end[q] = Q;
     int64_t off = 0;
     for (int s = 0; s < n_mapping; ++s) {
-      if (mapping[s].ptr == query[q].ptr && mapping[s].n == query[q].n) qs.alias[q] = off;
+      if (query_span && query_span[q] >= 0) {
+        if (query_span[q] == s) {
+          qs.via[q] = off;
+          qs.via_n[q] = mapping[s].n;
+        }
+      } else if (mapping[s].ptr == query[q].ptr && mapping[s].n == query[q].n) {
+        qs.alias[q] = off;
+      }
       off += mapping[s].n;
     }
   }
@@ -1308,10 +1332,10 @@ size_t gs_unique_workspace_bytes(int64_t M) {
   return a > b ? a : b;
 }
 
-int gs_unique_relabel_notify(const gs_span* mapping, int n_mapping, const gs_span* query,
-                             void* const* query_out, int n_query, int id_bytes, void* frontier,
-                             int64_t* num_unique, void* workspace, size_t workspace_bytes,
-                             const int64_t* last_span_len, gs_mailbox* mailbox,
+int gs_unique_relabel_places(const gs_span* mapping, int n_mapping, const gs_span* query,
+                             const int* query_span, void* const* query_out, int n_query, int id_bytes,
+                             void* frontier, int64_t* num_unique, void* workspace,
+                             size_t workspace_bytes, const int64_t* last_span_len, gs_mailbox* mailbox,
                              int64_t mailbox_ticket, void* stream) {
   GS_REQUIRE(mapping && n_mapping >= 1 && n_mapping <= GS_MAX_SPANS,
              "gs_unique_relabel: 1..%d mapping spans required, got %d", GS_MAX_SPANS, n_mapping);
@@ -1331,6 +1355,10 @@ int gs_unique_relabel_notify(const gs_span* mapping, int n_mapping, const gs_spa
   for (int q = 0; q < n_query; ++q)
     GS_REQUIRE(query[q].n >= 0 && (query[q].n == 0 || (query[q].ptr && query_out[q])),
                "gs_unique_relabel: query span %d is null or negative", q);
+  if (query_span)
+    for (int q = 0; q < n_query; ++q)
+      GS_REQUIRE(query_span[q] >= -1 && query_span[q] < n_mapping && (query_span[q] < 0 || query[q].n == 0 || M > 0),
+                 "gs_unique_relabel_places: query %d holds places in mapping span %d of %d", q, query_span[q], n_mapping);
   GS_REQUIRE(M == 0 || frontier, "gs_unique_relabel: frontier is null");
   if (M >= (int64_t(1) << 30)) {
     set_error_text("gs_unique_relabel: %lld mapping items exceed the supported 2^30",
@@ -1339,24 +1367,30 @@ int gs_unique_relabel_notify(const gs_span* mapping, int n_mapping, const gs_spa
   }
   if (last_span_len) {
     const gs_span& last = mapping[n_mapping - 1];
+    GS_REQUIRE(!query_span, "gs_unique_relabel_places: no places with a device-side length");
     GS_REQUIRE(n_query == 0 || (n_query == 1 && query[0].ptr == last.ptr && query[0].n == last.n),
                "gs_unique_relabel_notify: with a device-side length the only query allowed is "
                "the last mapping span itself");
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (id_bytes == 4)
-    return unique_relabel_impl<int32_t, PackedTable>(mapping, n_mapping, query, query_out, n_query,
-                                                     frontier, num_unique, workspace,
+    return unique_relabel_impl<int32_t, PackedTable>(mapping, n_mapping, query, query_span, query_out,
+                                                     n_query, frontier, num_unique, workspace,
                                                      workspace_bytes, last_span_len, mailbox,
                                                      mailbox_ticket, st);
-  return narrow ? unique_relabel_impl<int64_t, PackedTable>(mapping, n_mapping, query, query_out,
-                                                            n_query, frontier, num_unique, workspace,
-                                                            workspace_bytes, last_span_len, mailbox,
-                                                            mailbox_ticket, st)
-                : unique_relabel_impl<int64_t, WideTable>(mapping, n_mapping, query, query_out,
-                                                          n_query, frontier, num_unique, workspace,
-                                                          workspace_bytes, last_span_len, mailbox,
-                                                          mailbox_ticket, st);
+  const auto impl = narrow ? unique_relabel_impl<int64_t, PackedTable> : unique_relabel_impl<int64_t, WideTable>;
+  return impl(mapping, n_mapping, query, query_span, query_out, n_query, frontier, num_unique, workspace,
+              workspace_bytes, last_span_len, mailbox, mailbox_ticket, st);
+}
+
+int gs_unique_relabel_notify(const gs_span* mapping, int n_mapping, const gs_span* query,
+                             void* const* query_out, int n_query, int id_bytes, void* frontier,
+                             int64_t* num_unique, void* workspace, size_t workspace_bytes,
+                             const int64_t* last_span_len, gs_mailbox* mailbox,
+                             int64_t mailbox_ticket, void* stream) {
+  return gs_unique_relabel_places(mapping, n_mapping, query, nullptr, query_out, n_query, id_bytes, frontier,
+                                  num_unique, workspace, workspace_bytes, last_span_len, mailbox,
+                                  mailbox_ticket, stream);
 }
 
 int gs_unique_relabel(const gs_span* mapping, int n_mapping, const gs_span* query,

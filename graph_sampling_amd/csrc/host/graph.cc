@@ -475,7 +475,7 @@ c10::intrusive_ptr<Graph> Graph::SampleImpl(int64_t axis, const torch::Tensor* e
   }
   if (with_coo) {
     ret->SetCOO(on_csc ? std::make_shared<COO>(COO{tmp->coo_in_indices, tmp->coo_in_indptr,
-                                                   torch::nullopt, false, true})
+                                                   torch::nullopt, false, true, tmp->indptr.numel() - 1})
                        : std::make_shared<COO>(COO{tmp->coo_in_indptr, tmp->coo_in_indices,
                                                    torch::nullopt, true, false}));
   }
@@ -1086,9 +1086,14 @@ Graph::Relabel() {
   }
   TORCH_CHECK(csr_ || coo_, "Error in Relabel!");
   CreateSparseFormat(_COO);
-  torch::Tensor coo_col = col_ids.index({coo_->col});
   torch::Tensor coo_row = Pick(row_ids_, coo_->row);
-  std::tie(frontier, renamed) = BatchTensorRelabel({col_ids, coo_row}, {coo_col, coo_row});
+  // an edge's column is a place among the column ids; a sampler's own columns need no check
+  const bool places = coo_->columns >= 0 && coo_->columns <= col_ids.numel() &&
+                      coo_->col.scalar_type() == col_ids.scalar_type();
+  if (places)
+    std::tie(frontier, renamed) = hip::Relabel({col_ids, coo_row}, {coo_->col, coo_row}, {0, -1});
+  else
+    std::tie(frontier, renamed) = BatchTensorRelabel({col_ids, coo_row}, {col_ids.index({coo_->col}), coo_row});
   return {frontier, frontier.numel(), col_ids.numel(), renamed[1], renamed[0], coo_->e_ids, "coo"};
 }
 

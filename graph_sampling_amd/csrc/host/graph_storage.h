@@ -21,6 +21,7 @@ struct COO {
   torch::optional<torch::Tensor> e_ids;
   bool row_sorted = false;
   bool col_sorted = false;
+  int64_t columns = -1;  // every entry of col lies below this (-1: not known)
 };
 
 // Result of a slice / sample before it is wrapped into a format:

@@ -648,7 +648,9 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> SampleOneKeepDim(
 }
 
 std::tuple<torch::Tensor, std::vector<torch::Tensor>> Relabel(
-    const std::vector<torch::Tensor>& mapping, const std::vector<torch::Tensor>& queries) {
+    const std::vector<torch::Tensor>& mapping, const std::vector<torch::Tensor>& queries,
+    const std::vector<int>& places) {
+  TORCH_CHECK(places.empty() || places.size() == queries.size(), "relabel: one span a query expected");
   TORCH_CHECK(!mapping.empty() && mapping.size() <= GS_MAX_SPANS && queries.size() <= GS_MAX_SPANS,
               "relabel takes 1..", GS_MAX_SPANS, " mapping tensors and at most ", GS_MAX_SPANS,
               " tensors to relabel");
@@ -676,7 +678,8 @@ std::tuple<torch::Tensor, std::vector<torch::Tensor>> Relabel(
   int64_t U = kTooWide;
   for (int attempt = 0; attempt < 2 && U == kTooWide; ++attempt) {
     const int64_t ticket = boxes.next++;
-    Check(gs_unique_relabel_notify(m, static_cast<int>(mapping.size()), q, out_ptr,
+    Check(gs_unique_relabel_places(m, static_cast<int>(mapping.size()), q,
+                                   places.empty() ? nullptr : places.data(), out_ptr,
                                    static_cast<int>(queries.size()), TableIds(idb),
                                    frontier.data_ptr(), num.data_ptr<int64_t>(), ws.data_ptr(),
                                    ws.numel(), nullptr, boxes.slot(ticket), ticket, st),

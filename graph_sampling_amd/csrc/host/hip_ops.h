@@ -192,8 +192,10 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> SampleOneKeepDim(
     const torch::Tensor& indptr, const torch::Tensor& indices, const torch::Tensor& column_ids);
 
 torch::Tensor Unique(const torch::Tensor& ids);
+// places[q] >= 0: query q holds places in that mapping tensor, not ids
 std::tuple<torch::Tensor, std::vector<torch::Tensor>> Relabel(
-    const std::vector<torch::Tensor>& mapping, const std::vector<torch::Tensor>& queries);
+    const std::vector<torch::Tensor>& mapping, const std::vector<torch::Tensor>& queries,
+    const std::vector<int>& places = {});
 
 // {unique (batch frontiers back to back), unique_ptr, relabelled ids}: one relabel per batch
 std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> BatchCsrRelabel(

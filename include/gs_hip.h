@@ -445,6 +445,15 @@ int gs_unique_relabel_notify(const gs_span* mapping, int n_mapping, const gs_spa
                              const int64_t* last_span_len, gs_mailbox* mailbox,
                              int64_t mailbox_ticket, void* stream);
 
+/* The same where a query may hold places instead of ids: query_span[q] >= 0 (host array of n_query,
+ * NULL: none) says that query q's values are places in that mapping span, whose ids' ranks are asked
+ * for; -1 where a place lies outside the span.  Not together with last_span_len. */
+int gs_unique_relabel_places(const gs_span* mapping, int n_mapping, const gs_span* query,
+                             const int* query_span, void* const* query_out, int n_query, int id_bytes,
+                             void* frontier, int64_t* num_unique, void* workspace,
+                             size_t workspace_bytes, const int64_t* last_span_len, gs_mailbox* mailbox,
+                             int64_t mailbox_ticket, void* stream);
+
 /* The relabel that follows a sampler, on a hash table that outlives the calls (no
  * counterpart in the reference, which allocates and fills a fresh table per call,
  * src/cuda/unique_reindex.cu:86-88).  Same result as gs_unique_relabel_notify with the

@@ -408,3 +408,28 @@ def test_short_list_with_an_id_beyond_32_bits(dev):
     frontier, num, (out,) = capi.unique_relabel([ids[:3].contiguous()], [ids], narrow=True)
     assert int(num.item()) == 2 and out.tolist() == [0, 1, 0, -1]
     assert capi.unique_relabel([ids], [ids])[2][0].tolist() == [0, 1, 0, 2]
+
+
+@pytest.mark.parametrize("idt", [torch.int64, torch.int32])
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("S,n,queries", [(1, 1, 1), (300, 5000, 700), (4000, 4192, 10_240), (4000, 4193, 20), (4000, 4192, 10_241),
+                                         (5000, 86_000, 86_000)])
+def test_queries_that_hold_places(dev, idt, wide, S, n, queries):
+    """The rank of mapping[span][place], by one workgroup and past it, as by a gather in front of a relabel by
+    ids; repeated ids, places in the second span, and -1 for a place outside its span."""
+    rng = np.random.default_rng(S + n + queries)
+    seeds, ids = rng.integers(0, 3 * S, S), rng.integers(0, 2 * n, n)
+    if wide and idt == torch.int64:
+        seeds[S // 2] += 1 << 40
+    at, second = rng.integers(0, S, queries), rng.integers(0, n, 5)
+    off = at.copy()
+    off[:: 7] = np.where(off[:: 7] % 2, -1 - off[:: 7], S + off[:: 7])
+    m = [to_dev(seeds, dev, idt), to_dev(ids, dev, idt)]
+    frontier, num, outs = capi.unique_relabel(m, [to_dev(off, dev, idt), m[1], to_dev(second, dev, idt), to_dev(seeds[at[:9]], dev, idt)],
+                                              places=[0, -1, 1, -1], narrow=idt == torch.int64 and not wide)
+    w_frontier, w_outs = O.relabel([seeds, ids], [seeds[at], ids, ids[second], seeds[at[:9]]])
+    w_outs[0] = np.where(off == at, w_outs[0], -1)
+    U = int(num.item())
+    assert np.array_equal(frontier[:U].cpu().numpy().astype(np.int64), w_frontier)
+    for got, want in zip(outs, w_outs):
+        assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
