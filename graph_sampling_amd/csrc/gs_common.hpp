@@ -693,4 +693,53 @@ int batch_relabel_binned(const void* seeds, const int64_t* seeds_ptr, const void
                          int64_t* num_unique, void* workspace, size_t workspace_bytes,
                          gs_mailbox* box, int64_t box_ticket, hipStream_t stream);
 
+// Exclusive scan of f over [0, n) in one launch, where the caller has a look-back state: the tiles hand their sums
+// along instead of leaving them to a second launch.  What bounds it are two trips to memory for f and one for the
+// look-back.  out[n] and the mailbox get the total, -1 when a tile gave up or *outside is set.
+template <typename F, int ITEMS>
+__global__ void __launch_bounds__(kScanThreads)
+scan_chain_kernel(F f, int64_t n, int64_t* __restrict__ out, LookbackState lb, const int* __restrict__ outside,
+                  gs_mailbox* box, int64_t ticket) {
+  __shared__ int64_t lds[kScanThreads / kWave + 1];
+  __shared__ int64_t s_prefix;
+  const int64_t base = (static_cast<int64_t>(blockIdx.x) * kScanThreads + threadIdx.x) * ITEMS;
+  auto at = [&](int k) { return base + k; };
+  int64_t v[ITEMS];
+  scan_load(f, n, at, v);
+  int64_t mine = 0;
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) mine += v[k];
+  int64_t total;
+  const int64_t local = block_exclusive_scan<kScanThreads>(mine, &total, lds);
+  if (threadIdx.x == 0) lookback_publish_sum(lb, blockIdx.x, total);
+  if (threadIdx.x < kWave) {
+    const int64_t before = lookback_exclusive_prefix(lb, blockIdx.x, total);
+    if (threadIdx.x == 0) s_prefix = before;
+  }
+  __syncthreads();
+  int64_t run = s_prefix + local;
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    if (at(k) < n) out[at(k)] = run;
+    run += v[k];
+  }
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+    int64_t all = s_prefix + total;
+    if (__hip_atomic_load(lb.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) || (outside && *outside)) all = -1;
+    out[n] = all;
+    post_mailbox(box, all, ticket);
+  }
+}
+
+// n > 0; tiles as exclusive_scan's
+template <typename F>
+inline int chained_scan(F f, int64_t n, int64_t* out, const LookbackState& lb, hipStream_t stream,
+                        gs_mailbox* box = nullptr, int64_t ticket = 0, const int* outside = nullptr) {
+  const dim3 grid(static_cast<unsigned>(scan_num_tiles(n)));
+  auto* kernel = scan_num_tiles(n) > 1 && n <= kScanFew ? scan_chain_kernel<F, kScanFewItems>
+                                                       : scan_chain_kernel<F, kScanItems>;
+  hipLaunchKernelGGL(kernel, grid, dim3(kScanThreads), 0, stream, f, n, out, lb, outside, box, ticket);
+  return check_launch("scan_chain");
+}
+
 }  // namespace gs

@@ -1295,6 +1295,17 @@ struct StaticState {
 StaticState g_static_state[kMaxDevices];
 std::mutex g_static_mu;
 
+inline int chained_state(void* state, size_t bytes, uint32_t epoch, int64_t S, LookbackState* lb) {
+  GS_REQUIRE(epoch >= 1 && epoch <= kLbMaxEpoch, "chained count: epoch %u is not in 1..%u", epoch, kLbMaxEpoch);
+  Carver ws(state, bytes);
+  *lb = carve_lookback(ws, scan_num_tiles(S), epoch);
+  if (!ws.ok) {
+    set_error_text("chained count: state needs %zu bytes, 256-byte aligned", lookback_state_bytes(scan_num_tiles(S)));
+    return GS_ERR_WORKSPACE;
+  }
+  return GS_OK;
+}
+
 static __global__ void __launch_bounds__(256) zero_words_kernel(unsigned long long* p, size_t n) {
   const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0ull;
@@ -1328,6 +1339,41 @@ int gs_slice_count_notify(const int64_t* indptr, int64_t num_cols, const void* c
                                          mailbox, ticket, st)
              : slice_count_impl<int32_t>(indptr, num_cols, column_ids, S, sub_indptr, tiles,
                                          mailbox, ticket, st);
+}
+
+size_t gs_chained_count_state_bytes(int64_t S) { return lookback_state_bytes(scan_num_tiles(S)); }
+
+int gs_slice_count_chained(const int64_t* indptr, int64_t num_cols, const void* column_ids, int id_bytes,
+                           int64_t S, int64_t* sub_indptr, gs_mailbox* mailbox, int64_t ticket, void* state,
+                           size_t state_bytes, uint32_t epoch, void* stream) {
+  GS_REQUIRE(indptr && sub_indptr && S > 0 && num_cols >= 0 && column_ids,
+             "gs_slice_count_chained: null pointer, no columns or a negative size");
+  GS_REQUIRE(valid_id_bytes(id_bytes), "gs_slice_count: id_bytes must be 4 or 8, got %d", id_bytes);
+  LookbackState lb;
+  GS_RETURN_IF_ERROR(chained_state(state, state_bytes, epoch, S, &lb));
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (id_bytes == 8)
+    return chained_scan(ColDegree<int64_t>{indptr, static_cast<const int64_t*>(column_ids), num_cols}, S, sub_indptr,
+                        lb, st, mailbox, ticket);
+  return chained_scan(ColDegree<int32_t>{indptr, static_cast<const int32_t*>(column_ids), num_cols}, S, sub_indptr,
+                      lb, st, mailbox, ticket);
+}
+
+int gs_sample_count_chained(const int64_t* indptr, int64_t num_cols, const void* column_ids, int id_bytes,
+                            int64_t S, int64_t fanout, int replace, int64_t* sub_indptr, gs_mailbox* mailbox,
+                            int64_t ticket, void* state, size_t state_bytes, uint32_t epoch, void* stream) {
+  GS_REQUIRE(indptr && sub_indptr && S > 0 && fanout >= 0 && num_cols >= 0,
+             "gs_sample_count_chained: null pointer, no columns or a negative size");
+  GS_REQUIRE(column_ids || S <= num_cols, "gs_sample_count: S exceeds num_cols without column_ids");
+  GS_REQUIRE(valid_id_bytes(id_bytes), "gs_sample_count: id_bytes must be 4 or 8, got %d", id_bytes);
+  LookbackState lb;
+  GS_RETURN_IF_ERROR(chained_state(state, state_bytes, epoch, S, &lb));
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (id_bytes == 8)
+    return chained_scan(ColCount<int64_t>{indptr, static_cast<const int64_t*>(column_ids), num_cols, fanout, replace},
+                        S, sub_indptr, lb, st, mailbox, ticket);
+  return chained_scan(ColCount<int32_t>{indptr, static_cast<const int32_t*>(column_ids), num_cols, fanout, replace},
+                      S, sub_indptr, lb, st, mailbox, ticket);
 }
 
 int gs_slice_count(const int64_t* indptr, int64_t num_cols, const void* column_ids, int id_bytes,

@@ -279,22 +279,39 @@ int64_t ReadTotal(const torch::Tensor& values, int64_t at, void* stream, const c
 struct TotalBox {
   explicit TotalBox(const torch::Tensor& like) : boxes(Boxes(like.get_device())), ticket(boxes.next++) {}
   gs_mailbox* slot() const { return boxes.slot(ticket); }
-  int64_t Wait(const torch::Tensor& values, int64_t at, void* stream, const char* what) const {
-    const int64_t total = WaitBox(slot(), ticket, stream, what);
-    return total == kLost ? values[at].item<int64_t>() : total;
+  // state: of the launch, when it was one of tiles that wait for one another
+  int64_t Wait(const torch::Tensor& values, int64_t at, void* stream, const char* what,
+               const torch::Tensor* state = nullptr) const {
+    int64_t total = WaitBox(slot(), ticket, stream, what);
+    if (total == kLost) total = values[at].item<int64_t>();
+    if (state && total < 0) GaveUp(*state, stream, what);
+    return total;
   }
   HostBoxes& boxes;
   const int64_t ticket;
 };
+
+// Whether the counts of S columns are scanned in one launch of tiles that wait for one another: one workgroup does up to
+// 2048, and from 2^17 on the tiles' wait costs what the second launch did.  A slice of short columns, two launches / one,
+// us: 2049 columns 25.8/23.3, 5000 26.3/24.5, 15 873 28.8/26.8, 65 536 33.7/31.0, 200 k 37.4/37.1, 1 M 77.7/79.3.
+bool CountsInOneLaunch(int64_t S) { return S > 2048 && S <= (int64_t(1) << 17); }
 
 // offsets of the column slice, its total on the host
 int64_t SliceCount(const torch::Tensor& indptr, const torch::Tensor& column_ids, int idb,
                    torch::Tensor& sub_indptr) {
   const int64_t S = column_ids.numel();
   sub_indptr = torch::empty({S + 1}, I64(indptr));
-  auto ws = Scratch(gs_slice_workspace_bytes(S), indptr);
   void* st = Stream(indptr);
   const TotalBox total(indptr);
+  if (CountsInOneLaunch(S)) {
+    FusedStateBuf& state = FusedState(gs_chained_count_state_bytes(S), indptr, st);
+    Check(gs_slice_count_chained(indptr.data_ptr<int64_t>(), indptr.numel() - 1, column_ids.data_ptr(), idb, S,
+                                 sub_indptr.data_ptr<int64_t>(), total.slot(), total.ticket, state.buf.data_ptr(),
+                                 state.buf.numel(), state.epoch, st),
+          "gs_slice_count");
+    return total.Wait(sub_indptr, S, st, "gs_slice_count", &state.buf);
+  }
+  auto ws = Scratch(gs_slice_workspace_bytes(S), indptr);
   Check(gs_slice_count_notify(indptr.data_ptr<int64_t>(), indptr.numel() - 1, column_ids.data_ptr(),
                               idb, S, sub_indptr.data_ptr<int64_t>(), total.slot(), total.ticket,
                               ws.data_ptr(), ws.numel(), st),
@@ -398,13 +415,23 @@ SliceResult SampleInto(const torch::Tensor& indptr, const torch::Tensor& indices
   void* st = Stream(indptr);
   const void* cols = fused ? column_ids.data_ptr() : nullptr;
   const TotalBox total(indptr);
-  Check(gs_sample_count_notify(indptr.data_ptr<int64_t>(), indptr.numel() - 1, cols, idb, S, fanout,
-                               replace ? 1 : 0, sub_indptr.data_ptr<int64_t>(), total.slot(),
-                               total.ticket, ws.data_ptr(), ws.numel(), st),
-        "gs_sample_count");
+  torch::Tensor state;
+  if (CountsInOneLaunch(S)) {
+    FusedStateBuf& s = FusedState(gs_chained_count_state_bytes(S), indptr, st);
+    state = s.buf;
+    Check(gs_sample_count_chained(indptr.data_ptr<int64_t>(), indptr.numel() - 1, cols, idb, S, fanout,
+                                  replace ? 1 : 0, sub_indptr.data_ptr<int64_t>(), total.slot(), total.ticket,
+                                  state.data_ptr(), state.numel(), s.epoch, st),
+          "gs_sample_count");
+  } else {
+    Check(gs_sample_count_notify(indptr.data_ptr<int64_t>(), indptr.numel() - 1, cols, idb, S, fanout,
+                                 replace ? 1 : 0, sub_indptr.data_ptr<int64_t>(), total.slot(),
+                                 total.ticket, ws.data_ptr(), ws.numel(), st),
+          "gs_sample_count");
+  }
   fill(cols, idb, S, sub_indptr, sub_indices, select_index, coo_col, ws, st);
   // the only host read of the call: the total is there before the fill has run
-  const int64_t nnz = total.Wait(sub_indptr, S, st, "gs_sample_count");
+  const int64_t nnz = total.Wait(sub_indptr, S, st, "gs_sample_count", state.defined() ? &state : nullptr);
   if (with_coo) coo_col = coo_col.narrow(0, 0, nnz);
   return {sub_indptr, coo_col, sub_indices.narrow(0, 0, nnz), select_index.narrow(0, 0, nnz)};
 }

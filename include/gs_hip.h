@@ -128,6 +128,17 @@ int gs_slice_count(const int64_t* indptr, int64_t num_cols, const void* column_i
 int gs_slice_count_notify(const int64_t* indptr, int64_t num_cols, const void* column_ids,
                           int id_bytes, int64_t S, int64_t* sub_indptr, gs_mailbox* mailbox,
                           int64_t ticket, void* workspace, size_t workspace_bytes, void* stream);
+/* The same count (and gs_sample_count_notify's) in one launch where the caller keeps a look-back state: state and
+ * epoch as for gs_sample_uniform_fused, gs_chained_count_state_bytes(S) bytes; S > 0.  sub_indptr[S] and the mailbox
+ * read -1 when a tile gave up waiting. */
+size_t gs_chained_count_state_bytes(int64_t S);
+int gs_slice_count_chained(const int64_t* indptr, int64_t num_cols, const void* column_ids, int id_bytes,
+                           int64_t S, int64_t* sub_indptr, gs_mailbox* mailbox, int64_t ticket, void* state,
+                           size_t state_bytes, uint32_t epoch, void* stream);
+int gs_sample_count_chained(const int64_t* indptr, int64_t num_cols, const void* column_ids, int id_bytes,
+                            int64_t S, int64_t fanout, int replace, int64_t* sub_indptr, gs_mailbox* mailbox,
+                            int64_t ticket, void* state, size_t state_bytes, uint32_t epoch, void* stream);
+
 
 /* Posts *value (a device int64, e.g. sub_indptr + S after gs_slice_count) to a mailbox from a
  * one-thread kernel queued on the stream: the host then spins on the mailbox instead of

@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 import torch
 
+import graph_sampling_amd as gs
 from oracle import oracle as O
 from graph_sampling_amd import capi
 from tests.util import graph_20x5, rmat_csc_np, to_dev, u32_draws
@@ -241,3 +242,38 @@ def test_out_of_range_column_ids_are_empty_columns(dev, idt):
     for g, w in zip(got, want):
         assert np.array_equal(g.cpu().numpy().astype(np.int64), w)
     assert (want[1][::7] == -1).all()
+
+
+@pytest.mark.parametrize("idt", [torch.int32, torch.int64])
+@pytest.mark.parametrize("S", [2048, 2049, 15_872, 15_873, 1 << 17, (1 << 17) + 1])
+def test_counts_in_one_launch_and_past_it(dev, idt, S):
+    """Offsets of slices and of weighted samples on both sides of the lines between one workgroup, tiles that wait for
+    one another and two launches, again and again on one look-back state; an error that sticks to it is reported once."""
+    n = 1 << 15
+    rng = np.random.default_rng(S)
+    degree = rng.integers(0, 4, n)
+    degree[:3] = [5000, 0, 300]
+    indptr = np.concatenate([[0], np.cumsum(degree)]).astype(np.int64)
+    t_ptr = to_dev(indptr, dev)
+    g = gs.Graph(False)
+    g._CAPI_LoadCSC(t_ptr, to_dev(rng.integers(0, n, indptr[-1]), dev, idt))
+
+    def cut(cols):
+        return g._CAPI_Slicing(to_dev(cols, dev, idt), 0, gs._CSC, gs._CSC, False)
+
+    def offsets(counts):
+        return np.concatenate([[0], np.cumsum(counts)])
+
+    for _ in range(3):
+        cols = rng.integers(-1, n + 1, S)  # (ids outside: empty columns)
+        want = np.where((cols >= 0) & (cols < n), degree[np.clip(cols, 0, n - 1)], 0)
+        sub = cut(cols)
+        assert np.array_equal(sub._CAPI_GetCSC()[0].cpu().numpy(), offsets(want))
+        probs = torch.rand(int(want.sum()), device=dev) + 0.1
+        picked = sub._CAPI_SamplingWithProbs(0, probs, 2, False, gs._CSC, gs._CSC)
+        assert np.array_equal(picked._CAPI_GetCSC()[0].cpu().numpy(), offsets(np.minimum(want, 2)))
+    if 2048 < S <= 1 << 17:
+        torch.ops.gs_ops._CAPI_DebugRaiseLookbackError(t_ptr)
+        with pytest.raises(RuntimeError, match="gave up"):
+            cut(cols)
+        assert np.array_equal(cut(cols)._CAPI_GetCSC()[0].cpu().numpy(), offsets(want))
