@@ -61,6 +61,8 @@ struct InducedMarks {
   uint16_t* packed;          // new row numbers (places, 14 bits) of the kept edges, at the front of the tile's range
   int64_t* word_at;          // with data (null: none): where a word's edges are in the parent (WordAt)
   int* outside;              // set when an id lies beyond the bitmap: the call has to be repeated
+  LookbackState lb;          // of the scan of the tile counts; the marks clear it
+  int64_t lb_tiles;
   int64_t n;
   int64_t tiles;
 };
@@ -340,6 +342,10 @@ induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
   constexpr int kStep = BLOCK / kWave;  // the waves of a workgroup take turns along its run
   const int64_t tile0 = m.tiles * blockIdx.x / gridDim.x + wave;
   const int64_t tile1 = m.tiles * (blockIdx.x + 1) / gridDim.x;
+  if (blockIdx.x == 0) {  // (the launch behind this one uses it, under epoch 1)
+    if (threadIdx.x == 0) *m.lb.error = 0u;
+    for (int64_t j = threadIdx.x; j < m.lb_tiles; j += BLOCK) m.lb.status[j] = 0ull;
+  }
   if (tile0 >= tile1) return;  // (no barrier from here on)
 
   int64_t* off = s_offsets[wave];
@@ -489,7 +495,7 @@ induced_indptr_kernel(const int64_t* __restrict__ sub_indptr, int64_t S, Induced
   if (r > S) return;
   const int64_t i = sub_indptr[r];
   if (i >= m.n) {
-    out_indptr[r] = r == S && *m.outside ? int64_t(-1) : m.tile_base[m.tiles];
+    out_indptr[r] = m.tile_base[m.tiles];  // (-1 when an id lay outside or a tile of the scan gave up)
     return;
   }
   const int64_t w = i >> 6;
@@ -596,8 +602,7 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
   }
 }
 
-bool carve_induced(void* workspace, size_t bytes, int64_t D, bool with_data, InducedMarks* m,
-                   int64_t** scan_tiles) {
+bool carve_induced(void* workspace, size_t bytes, int64_t D, bool with_data, InducedMarks* m) {
   Carver ws(workspace, bytes);
   const size_t words = static_cast<size_t>(D / kWave + 1);
   const size_t most = static_cast<size_t>(((D - 1) >> kTileShift) + 1);
@@ -607,7 +612,8 @@ bool carve_induced(void* workspace, size_t bytes, int64_t D, bool with_data, Ind
   m->word_rank = ws.take<int32_t>(words);
   m->tile_counts = ws.take<int64_t>(most + 1);
   m->tile_base = ws.take<int64_t>(most + 2);
-  *scan_tiles = ws.take<int64_t>(static_cast<size_t>(scan_num_tiles(m->tiles) + 1));
+  m->lb_tiles = scan_num_tiles(m->tiles);
+  m->lb = carve_lookback(ws, m->lb_tiles, 1u);
   m->outside = ws.take<int>(1);
   m->packed = ws.take<uint16_t>(static_cast<size_t>(D));
   m->word_at = with_data ? ws.take<int64_t>(words) : nullptr;
@@ -714,7 +720,7 @@ size_t gs_induced_slice_workspace_bytes(int64_t D, int with_data) {
   const size_t words = static_cast<size_t>(D / kWave + 1), n = static_cast<size_t>(D);
   const int64_t tiles = ((D - 1) >> kTileShift) + 1;
   return padded(words * 8) + padded(words * 4) + padded(static_cast<size_t>(tiles + 1) * 8) +
-         padded(static_cast<size_t>(tiles + 2) * 8) + scan_workspace_bytes(tiles) + 256 +
+         padded(static_cast<size_t>(tiles + 2) * 8) + lookback_state_bytes(scan_num_tiles(tiles)) + 256 +
          padded(n * 2) + (with_data ? padded(words * 8) : 0);
 }
 
@@ -722,8 +728,8 @@ int gs_induced_slice_mark(const int64_t* indptr, int64_t num_cols, const void* i
                           int64_t num_rows, int id_bytes, const void* column_ids, int64_t S,
                           const int64_t* sub_indptr, int64_t D, const void* row_ids,
                           int64_t num_row_ids, const float* edge_data, const int64_t* edge_ids,
-                          int64_t* out_indptr, void* workspace, size_t workspace_bytes,
-                          void* stream) {
+                          int64_t* out_indptr, gs_mailbox* mailbox, int64_t ticket, void* workspace,
+                          size_t workspace_bytes, void* stream) {
   GS_REQUIRE(gs_induced_slice_applies(num_row_ids, S, D, nnz) && num_rows >= 0,
              "gs_induced_slice_mark: sizes beyond gs_induced_slice_applies");
   GS_REQUIRE(indptr && indices && column_ids && sub_indptr && row_ids && out_indptr,
@@ -731,8 +737,7 @@ int gs_induced_slice_mark(const int64_t* indptr, int64_t num_cols, const void* i
   GS_REQUIRE(valid_id_bytes(id_bytes), "gs_induced_slice_mark: id_bytes must be 4 or 8, got %d",
              id_bytes);
   InducedMarks m;
-  int64_t* scan_tiles;
-  if (!carve_induced(workspace, workspace_bytes, D, edge_data != nullptr, &m, &scan_tiles)) {
+  if (!carve_induced(workspace, workspace_bytes, D, edge_data != nullptr, &m)) {
     set_error_text("gs_induced_slice_mark: workspace needs %zu bytes, 256-byte aligned",
                    gs_induced_slice_workspace_bytes(D, edge_data != nullptr));
     return GS_ERR_WORKSPACE;
@@ -743,7 +748,7 @@ int gs_induced_slice_mark(const int64_t* indptr, int64_t num_cols, const void* i
                    bound, edge_data != nullptr};
   GS_RETURN_IF_ERROR(id_bytes == 8 ? pick_mark<int64_t>(c, m, st) : pick_mark<int32_t>(c, m, st));
   TileCount f{m.tile_counts};
-  GS_RETURN_IF_ERROR(exclusive_scan(f, m.tiles, m.tile_base, scan_tiles, st));
+  GS_RETURN_IF_ERROR(chained_scan(f, m.tiles, m.tile_base, m.lb, st, mailbox, ticket, m.outside));
   hipLaunchKernelGGL(induced_indptr_kernel, dim3(blocks_for(S + 1, 256)), dim3(256), 0, st,
                      sub_indptr, S, m, out_indptr);
   return check_launch("induced_slice_mark");
@@ -758,8 +763,7 @@ int gs_induced_slice_compact(const int64_t* indptr, int id_bytes, const void* co
   GS_REQUIRE(valid_id_bytes(id_bytes), "gs_induced_slice_compact: id_bytes must be 4 or 8, got %d",
              id_bytes);
   InducedMarks m;
-  int64_t* scan_tiles;
-  if (!carve_induced(workspace, workspace_bytes, D, out_data != nullptr, &m, &scan_tiles)) {
+  if (!carve_induced(workspace, workspace_bytes, D, out_data != nullptr, &m)) {
     set_error_text("gs_induced_slice_compact: pass the workspace given to gs_induced_slice_mark");
     return GS_ERR_WORKSPACE;
   }

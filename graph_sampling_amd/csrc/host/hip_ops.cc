@@ -1470,16 +1470,19 @@ std::tuple<torch::Tensor, torch::Tensor> InducedSlicing(const torch::Tensor& ind
   auto ws = Scratch(gs_induced_slice_workspace_bytes(D, edge != nullptr), indptr);
   int64_t kept = -1;
   for (int64_t bound : {num_rows, int64_t(0)}) {  // (again without a bound when an id reaches it)
+    const TotalBox total(indptr);
     Check(gs_induced_slice_mark(indptr.data_ptr<int64_t>(), indptr.numel() - 1, indices.data_ptr(),
                                 nnz, bound, idb, column_ids.data_ptr(), S,
                                 sub_indptr.data_ptr<int64_t>(), D, row_ids.data_ptr(), nr,
                                 edge ? edge->data.data_ptr<float>() : nullptr,
                                 edge ? OptI64(edge->e_ids, "e_ids") : nullptr,
-                                out_indptr.data_ptr<int64_t>(), ws.data_ptr(), ws.numel(), st),
+                                out_indptr.data_ptr<int64_t>(), total.slot(), total.ticket, ws.data_ptr(),
+                                ws.numel(), st),
           "gs_induced_slice_mark");
-    kept = ReadTotal(out_indptr, S, st, "total");
+    kept = total.Wait(out_indptr, S, st, "gs_induced_slice_mark");
     if (kept >= 0) break;
   }
+  TORCH_CHECK(kept >= 0, "gs_induced_slice_mark: a tile gave up waiting for its predecessors; the call can be repeated");
   auto out_indices = torch::empty({kept}, indices.options());
   if (edge) *data_out = torch::empty({kept}, edge->data.options());
   if (kept > 0)
