@@ -719,8 +719,11 @@ inline Source source_of(const int64_t* emap, const float* data, bool streams) {
 inline int64_t num_tiles(int64_t nnz) { return nnz <= 0 ? 1 : (nnz + kTile - 1) / kTile; }
 
 // The marks cost 12 bytes per edge; walking the offsets costs a workgroup a round of 256 per
-// 256 segments of its tile, and from eight rounds a tile on that is the longer way.
-inline bool use_marks(int64_t num_seg, int64_t nnz) { return 2 * num_seg > nnz; }
+// 256 segments of its tile, and from eight rounds a tile on that is the longer way.  Of few segments no wave has
+// more than one round, and clearing and setting marks are two launches: 1 k columns of 1 k edges normalised, 14 us of
+// kernels, 6.5 so.
+constexpr int64_t kMarkSegments = 4096;
+inline bool use_marks(int64_t num_seg, int64_t nnz) { return num_seg > kMarkSegments && 2 * num_seg > nnz; }
 constexpr int64_t kSearchTiles = 512;  // up to here a normalise's workgroups look for their first segment
 
 bool carve_tiles(void* workspace, size_t bytes, int64_t num_seg, int64_t nnz, Tiles* tl) {

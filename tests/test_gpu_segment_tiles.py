@@ -194,3 +194,24 @@ def test_all_empty_behind_a_first_offset(dev):
     out = torch.full((9000,), -1.0, device=dev)
     capi.segment_normalize(ptr, None, data, out)
     assert torch.equal(out, torch.full((9000,), -1.0, device=dev))
+
+
+@pytest.mark.parametrize("nseg", [1, 64, 4095, 4096, 4097])
+@pytest.mark.parametrize("lens", [[0, 1], [0, 0, 0, 2, 1], [1], [0, 0, 0, 17]])
+def test_few_edges_of_few_segments(dev, nseg, lens):
+    """Fewer edges than twice the segments, on both sides of the number of segments up to which offsets are walked
+    and none are marked: bits of sequential sums, zeros of empty segments, and quotients of one rounding."""
+    lens = np.resize(lens, nseg)
+    lens[-1] = 3
+    indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    nnz = int(indptr[-1])
+    data = (np.random.default_rng(nseg).random(nnz) + 0.25).astype(np.float32)
+    out = torch.full((nseg,), -1.0, device=dev)
+    capi.segment_sum(to_dev(indptr, dev), None, None, to_dev(data, dev), 1, out)
+    want = np.bincount(np.repeat(np.arange(nseg), lens), weights=data.astype(np.float64), minlength=nseg)
+    got = out.cpu().numpy()
+    np.testing.assert_allclose(got, want, rtol=RTOL)
+    assert (got[lens == 0] == 0).all()
+    out = torch.full((nnz,), -1.0, device=dev)
+    capi.segment_normalize(to_dev(indptr, dev), None, to_dev(data, dev), out)
+    np.testing.assert_allclose(out.cpu().numpy(), data / np.repeat(want, lens), rtol=RTOL)
