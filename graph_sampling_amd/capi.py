@@ -1090,19 +1090,21 @@ def coo_sum(target, e_ids, data, powk, out):
                             _i64(powk), _ptr(out), _stream(target.device)), "gs_coo_sum")
 
 
-def coo_sum_binned(target, e_ids, data, powk, out):
+def coo_sum_binned(target, e_ids, data, powk, out, fresh=False):
     """`coo_sum` through the entry point that knows the number of targets (`out.numel()`) and
-    brings a workspace: large inputs are binned by target and added up without atomics."""
+    brings a workspace: large inputs are binned by target and added up without atomics.  fresh:
+    `out` holds nothing yet, every entry is written."""
     idb = _ids(target, "target")
     _need(data, torch.float32, "data")
     _need(out, torch.float32, "out")
     L = lib()
     ws = workspace(L.gs_coo_sum_workspace_bytes(_i64(target.numel()), _i64(out.numel())),
                    target.device)
-    _check(L.gs_coo_sum_binned(_ptr(target), idb, _ptr(e_ids), _ptr(data), _i64(target.numel()),
-                               _i64(powk), _i64(out.numel()), _ptr(out), _ptr(ws),
-                               ctypes.c_size_t(ws.numel()), _stream(target.device)),
-           "gs_coo_sum_binned")
+    call = L.gs_coo_sum_fresh if fresh else L.gs_coo_sum_binned
+    _check(call(_ptr(target), idb, _ptr(e_ids), _ptr(data), _i64(target.numel()),
+                _i64(powk), _i64(out.numel()), _ptr(out), _ptr(ws),
+                ctypes.c_size_t(ws.numel()), _stream(target.device)),
+           "gs_coo_sum_fresh" if fresh else "gs_coo_sum_binned")
 
 
 def segment_normalize(indptr, e_ids, data, out):

@@ -940,7 +940,7 @@ torch::Tensor Graph::Sum(int64_t axis, int64_t powk, int64_t on_format) {
   const auto segments = [&](const std::shared_ptr<CSC>& form, const torch::optional<torch::Tensor>& ids) {
     return form && !ids.has_value() && form->indptr.numel() - 1 == size;
   };
-  const bool all_written = (axis == 0 && IsCscLike(on_format) && segments(csc_, val_col_ids_)) ||
+  const bool all_written = on_format == _COO || (axis == 0 && IsCscLike(on_format) && segments(csc_, val_col_ids_)) ||
                            (axis == 1 && IsCsrLike(on_format) && segments(csr_, val_row_ids_));
   torch::Tensor out = all_written ? torch::empty({size}, data.options()) : torch::zeros({size}, data.options());
   if (on_format == _COO)

@@ -742,6 +742,10 @@ int gs_coo_sum(const void* target, int id_bytes, const int64_t* e_ids, const flo
  * the additions is not fixed in either (impl::COOSumCUDA, src/cuda/graph_ops.cu:45-64, adds
  * with atomics too). */
 size_t gs_coo_sum_workspace_bytes(int64_t E, int64_t num_targets);
+/* The same into an `out` that holds nothing yet: every entry is written. */
+int gs_coo_sum_fresh(const void* target, int id_bytes, const int64_t* e_ids, const float* data, int64_t E,
+                     int64_t powk, int64_t num_targets, float* out, void* workspace, size_t workspace_bytes,
+                     void* stream);
 int gs_coo_sum_binned(const void* target, int id_bytes, const int64_t* e_ids, const float* data,
                       int64_t E, int64_t powk, int64_t num_targets, float* out, void* workspace,
                       size_t workspace_bytes, void* stream);

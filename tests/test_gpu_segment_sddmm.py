@@ -491,3 +491,19 @@ def test_graph_sums_write_every_segment(dev, cols, degree, axis):
     got = g._CAPI_Sum(axis, 2, _CSC if axis == 0 else _CSR).cpu().numpy()
     want = np.add.reduceat(np.append(data, 0.0).astype(np.float64) ** 2, indptr[:-1]) * (lens > 0)
     assert np.array_equal(got, want.astype(np.float32))
+
+
+# edges that go the plain way and by bins; sums that a tile's workgroup clears along with its edges, 2^14, and one more
+@pytest.mark.parametrize("edges,targets", [(0, 5), (1000, 1), (1000, 3_000_001), ((1 << 17) - 1, 70_000), (1 << 17, 65),
+                                           (1 << 17, 16 << 14), (1 << 17, (16 << 14) + 1), (300_001, 2_450_000)])
+@pytest.mark.parametrize("idt", [torch.int32, torch.int64])
+def test_coo_sum_into_what_holds_nothing(dev, idt, edges, targets):
+    rng = np.random.default_rng(edges + targets)
+    t = (rng.random(edges) ** 3 * targets).astype(np.int64)
+    if edges > 100_000:
+        t[: edges // 3] = targets // 2  # a hub: shared by workgroups, which add
+    data = (rng.random(edges) + 0.25).astype(np.float32)
+    out = torch.full((targets,), float("nan"), device=dev)
+    capi.coo_sum_binned(to_dev(t, dev, idt), None, to_dev(data, dev), 2, out, fresh=True)
+    want = np.bincount(t, weights=data.astype(np.float64) ** 2, minlength=targets)
+    np.testing.assert_allclose(out.cpu().numpy(), want, rtol=2e-5)
