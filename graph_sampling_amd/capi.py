@@ -229,6 +229,16 @@ def selftest_lookback(state, epoch, tiles, missing_tile, spin_limit):
     return total
 
 
+def selftest_chained_scan(values, state, epoch, spin_limit):
+    """gs_selftest_chained_scan on the caller's state buffer; returns the n + 1 exclusive sums."""
+    out = torch.full((values.numel() + 1,), -7, dtype=torch.int64, device=values.device)
+    _check(lib().gs_selftest_chained_scan(_ptr(values), _i64(values.numel()), _ptr(out), _ptr(state),
+                                          ctypes.c_size_t(state.numel()), ctypes.c_uint32(epoch),
+                                          int(spin_limit), _stream(state.device)),
+           "gs_selftest_chained_scan")
+    return out
+
+
 class Mailbox:
     """gs_mailbox in pinned host memory plus the host side of the protocol."""
 

@@ -627,11 +627,16 @@ __device__ __forceinline__ int64_t lookback_wait_inclusive(const LookbackState& 
 
 // Call with all 64 lanes of wave 0, after lookback_publish_sum.  Returns the sum
 // of all earlier tiles and (unless publish is false) publishes the tile's inclusive prefix.
+// gave_up, when given, is set where a wait ran out, for all lanes: no error is raised then and nothing
+// published, the caller finds the sum another way and closes the tile itself.
 __device__ __forceinline__ int64_t lookback_exclusive_prefix(const LookbackState& st,
                                                              unsigned int tile, int64_t total,
-                                                             bool publish = true) {
+                                                             bool publish = true,
+                                                             bool* gave_up = nullptr) {
   const int lane = threadIdx.x & (kWave - 1);
+  if (gave_up) *gave_up = false;
   if (tile == 0) return 0;
+  bool late = false;
   const unsigned long long before_first = lb_word(2u, st.epoch, 0);  // "tile -1": inclusive 0
   int64_t running = 0;
   int64_t newest = static_cast<int64_t>(tile) - 1;  // lane l reads tile newest - l (- 64 per window)
@@ -651,7 +656,10 @@ __device__ __forceinline__ int64_t lookback_exclusive_prefix(const LookbackState
         int polls = 0;
         while (lb_flag(s[w], st.epoch) == 0) {
           if (++polls > st.spin_limit) {
-            lookback_raise(st);
+            if (gave_up)
+              late = true;
+            else
+              lookback_raise(st);
             s[w] = before_first;
             break;
           }
@@ -669,6 +677,10 @@ __device__ __forceinline__ int64_t lookback_exclusive_prefix(const LookbackState
       }
     }
     newest -= kLookbackBurst * kWave;
+  }
+  if (gave_up && __any(late)) {
+    *gave_up = true;
+    return 0;
   }
   // (an error raised above was stored with device scope before this point)
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -695,13 +707,16 @@ int batch_relabel_binned(const void* seeds, const int64_t* seeds_ptr, const void
 
 // Exclusive scan of f over [0, n) in one launch, where the caller has a look-back state: the tiles hand their sums
 // along instead of leaving them to a second launch.  What bounds it are two trips to memory for f and one for the
-// look-back.  out[n] and the mailbox get the total, -1 when a tile gave up or *outside is set.
+// look-back.  A tile whose wait runs out adds up what lies in front of it itself, so the offsets are right whatever
+// happens (who reads them does so in launches that are queued already and cannot be told).  out[n] and the mailbox get
+// the total, -1 when *outside is set.
 template <typename F, int ITEMS>
 __global__ void __launch_bounds__(kScanThreads)
 scan_chain_kernel(F f, int64_t n, int64_t* __restrict__ out, LookbackState lb, const int* __restrict__ outside,
                   gs_mailbox* box, int64_t ticket) {
   __shared__ int64_t lds[kScanThreads / kWave + 1];
   __shared__ int64_t s_prefix;
+  __shared__ bool s_late;
   const int64_t base = (static_cast<int64_t>(blockIdx.x) * kScanThreads + threadIdx.x) * ITEMS;
   auto at = [&](int k) { return base + k; };
   int64_t v[ITEMS];
@@ -713,10 +728,25 @@ scan_chain_kernel(F f, int64_t n, int64_t* __restrict__ out, LookbackState lb, c
   const int64_t local = block_exclusive_scan<kScanThreads>(mine, &total, lds);
   if (threadIdx.x == 0) lookback_publish_sum(lb, blockIdx.x, total);
   if (threadIdx.x < kWave) {
-    const int64_t before = lookback_exclusive_prefix(lb, blockIdx.x, total);
-    if (threadIdx.x == 0) s_prefix = before;
+    bool late;
+    const int64_t before = lookback_exclusive_prefix(lb, blockIdx.x, total, true, &late);
+    if (threadIdx.x == 0) {
+      s_prefix = before;
+      s_late = late;
+    }
   }
   __syncthreads();
+  if (s_late) {
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * kScanThreads * ITEMS;
+    int64_t part = 0, before;
+    for (int64_t i = threadIdx.x; i < first; i += kScanThreads) part += f(i);
+    block_exclusive_scan<kScanThreads>(part, &before, lds);
+    if (threadIdx.x == 0) {
+      s_prefix = before;
+      lookback_publish_inclusive(lb, blockIdx.x, before + total);
+    }
+    __syncthreads();
+  }
   int64_t run = s_prefix + local;
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {
@@ -725,7 +755,7 @@ scan_chain_kernel(F f, int64_t n, int64_t* __restrict__ out, LookbackState lb, c
   }
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
     int64_t all = s_prefix + total;
-    if (__hip_atomic_load(lb.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) || (outside && *outside)) all = -1;
+    if (outside && *outside) all = -1;
     out[n] = all;
     post_mailbox(box, all, ticket);
   }

@@ -495,7 +495,7 @@ induced_indptr_kernel(const int64_t* __restrict__ sub_indptr, int64_t S, Induced
   if (r > S) return;
   const int64_t i = sub_indptr[r];
   if (i >= m.n) {
-    out_indptr[r] = m.tile_base[m.tiles];  // (-1 when an id lay outside or a tile of the scan gave up)
+    out_indptr[r] = m.tile_base[m.tiles];  // (-1 when an id lay outside)
     return;
   }
   const int64_t w = i >> 6;

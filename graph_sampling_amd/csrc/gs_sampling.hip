@@ -1836,8 +1836,24 @@ __global__ void __launch_bounds__(kWave) lookback_selftest_kernel(LookbackState 
     *total = t;
   }
 }
+struct PlainValue {
+  const int64_t* p;
+  __device__ __forceinline__ int64_t operator()(int64_t i) const { return p[i]; }
+};
 }  // namespace
 }  // namespace gs
+
+extern "C" int gs_selftest_chained_scan(const int64_t* values, int64_t n, int64_t* out, void* state,
+                                        size_t state_bytes, uint32_t epoch, int spin_limit, void* stream) {
+  using namespace gs;
+  GS_REQUIRE(values && out && n > 0, "gs_selftest_chained_scan: null pointer or no values");
+  GS_REQUIRE(spin_limit >= 0 && spin_limit <= kLookbackSpinLimit,
+             "gs_selftest_chained_scan: spin_limit must be in 0..%d", kLookbackSpinLimit);
+  LookbackState lb;
+  GS_RETURN_IF_ERROR(chained_state(state, state_bytes, epoch, n, &lb));
+  lb.spin_limit = spin_limit;
+  return chained_scan(PlainValue{values}, n, out, lb, static_cast<hipStream_t>(stream));
+}
 
 extern "C" int gs_selftest_lookback(void* state, size_t state_bytes, uint32_t epoch, int64_t tiles,
                                     int64_t missing_tile, int spin_limit, int64_t* total,

@@ -129,8 +129,8 @@ int gs_slice_count_notify(const int64_t* indptr, int64_t num_cols, const void* c
                           int id_bytes, int64_t S, int64_t* sub_indptr, gs_mailbox* mailbox,
                           int64_t ticket, void* workspace, size_t workspace_bytes, void* stream);
 /* The same count (and gs_sample_count_notify's) in one launch where the caller keeps a look-back state: state and
- * epoch as for gs_sample_uniform_fused, gs_chained_count_state_bytes(S) bytes; S > 0.  sub_indptr[S] and the mailbox
- * read -1 when a tile gave up waiting. */
+ * epoch as for gs_sample_uniform_fused, gs_chained_count_state_bytes(S) bytes; S > 0.  The error word in the state is
+ * neither read nor raised: a tile that gives up waiting adds up what lies in front of it. */
 size_t gs_chained_count_state_bytes(int64_t S);
 int gs_slice_count_chained(const int64_t* indptr, int64_t num_cols, const void* column_ids, int id_bytes,
                            int64_t S, int64_t* sub_indptr, gs_mailbox* mailbox, int64_t ticket, void* state,
@@ -319,6 +319,10 @@ int gs_sample_uniform_fused_static(const int64_t* indptr, int64_t num_cols, cons
  * reports -1) until the caller zero-fills it. */
 int gs_selftest_lookback(void* state, size_t state_bytes, uint32_t epoch, int64_t tiles,
                          int64_t missing_tile, int spin_limit, int64_t* total, void* stream);
+/* Self-test of gs_slice_count_chained's scan (no counterpart in the reference): out[0..n] = exclusive sums of
+ * values[0..n), a tile giving up after `spin_limit` >= 0 polls of a predecessor's status word. */
+int gs_selftest_chained_scan(const int64_t* values, int64_t n, int64_t* out, void* state, size_t state_bytes,
+                             uint32_t epoch, int spin_limit, void* stream);
 
 /* fanout == 1 with replacement through the fused entry: exactly one slot per
  * column, -1 in both outputs for an empty column; sub_indptr = 0..S.  Replaces

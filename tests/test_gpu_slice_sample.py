@@ -248,7 +248,8 @@ def test_out_of_range_column_ids_are_empty_columns(dev, idt):
 @pytest.mark.parametrize("S", [2048, 2049, 15_872, 15_873, 1 << 17, (1 << 17) + 1])
 def test_counts_in_one_launch_and_past_it(dev, idt, S):
     """Offsets of slices and of weighted samples on both sides of the lines between one workgroup, tiles that wait for
-    one another and two launches, again and again on one look-back state; an error that sticks to it is reported once."""
+    one another and two launches, again and again on one look-back state; an error that a sampler left in it is not theirs:
+    slices and samples are as they were, and the next one-launch sampler reports it, once."""
     n = 1 << 15
     rng = np.random.default_rng(S)
     degree = rng.integers(0, 4, n)
@@ -274,6 +275,25 @@ def test_counts_in_one_launch_and_past_it(dev, idt, S):
         assert np.array_equal(picked._CAPI_GetCSC()[0].cpu().numpy(), offsets(np.minimum(want, 2)))
     if 2048 < S <= 1 << 17:
         torch.ops.gs_ops._CAPI_DebugRaiseLookbackError(t_ptr)
+        sub = cut(cols)
+        assert np.array_equal(sub._CAPI_GetCSC()[0].cpu().numpy(), offsets(want))
+        for replace in (False, True):
+            picked = sub._CAPI_SamplingWithProbs(0, probs, 2, replace, gs._CSC, gs._CSC)
+            counts = np.where(want > 0, 2, 0) if replace else np.minimum(want, 2)
+            assert np.array_equal(picked._CAPI_GetCSC()[0].cpu().numpy(), offsets(counts))
         with pytest.raises(RuntimeError, match="gave up"):
-            cut(cols)
-        assert np.array_equal(cut(cols)._CAPI_GetCSC()[0].cpu().numpy(), offsets(want))
+            g._CAPI_FusedColumnwiseSlicingSampling(to_dev(cols, dev, idt), 2, False)._CAPI_GetCSC()
+        picked = g._CAPI_FusedColumnwiseSlicingSampling(to_dev(cols, dev, idt), 2, False)
+        assert np.array_equal(picked._CAPI_GetCSC()[0].cpu().numpy(), offsets(np.minimum(want, 2)))
+
+
+@pytest.mark.parametrize("n", [1, 2048, 2049, 15_872, 15_873, 1 << 17, 3_000_001])
+@pytest.mark.parametrize("spin_limit", [0, 1, 1 << 20])
+def test_offsets_where_tiles_give_up_waiting(dev, n, spin_limit):
+    """A tile that does not wait for its predecessors adds up what lies in front of it: same offsets, no error left."""
+    values = torch.randint(0, 1 << 20, (n,), generator=torch.Generator().manual_seed(n)).to(dev)
+    state = torch.zeros(1 << 16, dtype=torch.uint8, device=dev)
+    want = torch.cat([torch.zeros(1, dtype=torch.int64), torch.cumsum(values.cpu(), 0)])
+    for epoch in (1, 2, 3):
+        assert torch.equal(capi.selftest_chained_scan(values, state, epoch, spin_limit).cpu(), want)
+    assert not state[:4].any()
