@@ -39,7 +39,8 @@ def lib():
                      "gs_layer_sample_state_bytes", "gs_layer_relabel_state_bytes",
                      "gs_coo_sum_workspace_bytes", "gs_coo_pick_rows_workspace_bytes",
                      "gs_coo_block_values_workspace_bytes", "gs_random_walk_workspace_bytes",
-                     "gs_metapath_walk_workspace_bytes"):
+                     "gs_metapath_walk_workspace_bytes",
+                     "gs_induced_slice_workspace_bytes"):
             if hasattr(_lib, name):
                 getattr(_lib, name).restype = ctypes.c_size_t
         _lib.gs_sorted_union_max.restype = ctypes.c_int64
@@ -1226,6 +1227,38 @@ def col_row_slice(indptr, indices, column_ids, row_ids, col_ptr=None, row_ptr=No
                                               ctypes.c_size_t(ws.numel()), st),
                "gs_col_row_slice_compact")
     return out_indptr, out_indices, select_index, parent_index
+
+
+def induced_slice(indptr, indices, column_ids, row_ids, num_rows, data=None, e_ids=None):
+    """gs_slice_count + gs_induced_slice_{mark,compact}, the data gone before the second call; returns
+    (out_indptr, out_indices, out_data), out_indptr alone when a row id reached num_rows."""
+    _need(indptr, torch.int64, "indptr")
+    idb = _ids(indices, "indices")
+    _ids(column_ids, "column_ids", like=indices)
+    _ids(row_ids, "row_ids", like=indices)
+    dev = indptr.device
+    S, nr = column_ids.numel(), row_ids.numel()
+    sub_indptr = slice_count(indptr, column_ids)
+    D = _total(sub_indptr, S)
+    out_indptr = torch.empty(S + 1, dtype=torch.int64, device=dev)
+    ws = workspace(lib().gs_induced_slice_workspace_bytes(_i64(D), int(data is not None)), dev)
+    st = _stream(dev)
+    edge_data = None if data is None else data.clone()
+    _check(lib().gs_induced_slice_mark(_ptr(indptr), _i64(indptr.numel() - 1), _ptr(indices), _i64(indices.numel()),
+                                       _i64(num_rows), idb, _ptr(column_ids), _i64(S), _ptr(sub_indptr), _i64(D),
+                                       _ptr(row_ids), _i64(nr), _ptr(edge_data), _ptr(e_ids), _ptr(out_indptr),
+                                       _ptr(ws), ctypes.c_size_t(ws.numel()), st), "gs_induced_slice_mark")
+    kept = _total(out_indptr, S)
+    if kept < 0:
+        return out_indptr
+    if data is not None:
+        edge_data.fill_(float("nan"))
+    out_indices = torch.empty(kept, dtype=indices.dtype, device=dev)
+    out_data = None if data is None else torch.empty(kept, dtype=torch.float32, device=dev)
+    if kept > 0:
+        _check(lib().gs_induced_slice_compact(_i64(D), idb, _ptr(out_indices), _ptr(out_data), _ptr(ws),
+                                              ctypes.c_size_t(ws.numel()), st), "gs_induced_slice_compact")
+    return out_indptr, out_indices, out_data
 
 
 # ------------------------------------------------------- format transform ----

@@ -60,6 +60,7 @@ struct InducedMarks {
   int64_t* tile_base;        // exclusive scan of tile_counts
   uint16_t* packed;          // new row numbers (places, 14 bits) of the kept edges, at the front of the tile's range
   int64_t* word_at;          // with data (null: none): where a word's edges are in the parent (WordAt)
+  float* packed_data;        // the kept edges' data, beside packed, for callers of gs_induced_slice_compact (null: none)
   int* outside;              // set when an id lies beyond the bitmap: the call has to be repeated
   LookbackState lb;          // of the scan of the tile counts; the marks clear it
   int64_t lb_tiles;
@@ -320,8 +321,8 @@ __device__ __forceinline__ int row_of(const int64_t* off, int lo, int hi, int64_
   return lo;
 }
 
-// What a kept edge brings along: nothing, data[position], or data[e_ids[position]].
-enum Data { kNoData, kByPosition, kByEdgeId };
+// What a kept edge brings along: nothing, data[position], data[e_ids[position]], or what lies packed beside its row number.
+enum Data { kNoData, kByPosition, kByEdgeId, kPacked };
 
 template <typename IdT, typename Set, int BLOCK, int WAVES, bool PLACES, bool STREAM>
 __global__ void __launch_bounds__(BLOCK, WAVES)  // (waves a SIMD)
@@ -505,6 +506,7 @@ induced_indptr_kernel(const int64_t* __restrict__ sub_indptr, int64_t S, Induced
 
 // Every tile's kept edges from the front of its range to their place in the result, a wave at a
 // time: eight times 64, all reads before the stores.  The data come from the parent, word by word.
+// (out_indices null: the data only, to the front of the tile's range of out_data.)
 constexpr int kCopyTiles = 4;  // of a workgroup, one for every wave
 
 template <typename IdT, Data DATA, bool STREAM>
@@ -517,17 +519,18 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // (a scalar, and so are all addresses' bases)
   const int64_t t = static_cast<int64_t>(blockIdx.x) * kCopyTiles + wave;
   if (t >= m.tiles) return;
-  const int64_t base = m.tile_base[t];
-  const int count = static_cast<int>(m.tile_base[t + 1] - base);
+  constexpr bool kParent = DATA == kByPosition || DATA == kByEdgeId;
+  const int64_t first = m.tile_base[t], base = out_indices ? first : t * kTile;
+  const int count = static_cast<int>(m.tile_base[t + 1] - first);
   unsigned long long my_word = 0;  // lane k: word k of the tile
   int my_rank = 0;
   int64_t my_at = 0;
-  if (DATA != kNoData && lane < kPer && t * kTile + lane * kWave < m.n) {
+  if (kParent && lane < kPer && t * kTile + lane * kWave < m.n) {
     my_word = m.mask[t * kPer + lane];
     my_rank = m.word_rank[t * kPer + lane];
     my_at = m.word_at[t * kPer + lane];
   }
-  if (count == 0) return;
+  if (count <= 0) return;  // (below: the last tile, where an id lay outside and the total is -1)
   auto once = [](const auto* p) { return STREAM ? __builtin_nontemporal_load(p) : *p; };
   uint16_t v[kPer];
 #pragma unroll
@@ -535,10 +538,17 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
     const int r = k * kWave + lane;
     v[k] = m.packed[t * kTile + (r < count ? r : count - 1)];
   }
-  bool kept[DATA == kNoData ? 1 : kPer];
-  int rank[DATA == kNoData ? 1 : kPer];
+  bool kept[kParent ? kPer : 1];
+  int rank[kParent ? kPer : 1];
   float x[DATA == kNoData ? 1 : kPer];
-  if constexpr (DATA != kNoData) {
+  if constexpr (DATA == kPacked) {
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int r = k * kWave + lane;
+      x[k] = m.packed_data[t * kTile + (r < count ? r : count - 1)];
+    }
+  }
+  if constexpr (kParent) {
     auto of = [](uint64_t u, int k) {  // lane k's
       return static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u >> 32), k))) << 32 |
              static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u), k));
@@ -582,14 +592,20 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     const int r = k * kWave + lane;
-    if (r < count) {
+    if (out_indices && r < count) {
       if (STREAM)
         __builtin_nontemporal_store(static_cast<IdT>(v[k]), out_indices + base + r);
       else
         out_indices[base + r] = static_cast<IdT>(v[k]);
+      if constexpr (DATA == kPacked) {
+        if (STREAM)
+          __builtin_nontemporal_store(x[k], out_data + base + r);
+        else
+          out_data[base + r] = x[k];
+      }
     }
   }
-  if constexpr (DATA != kNoData) {
+  if constexpr (kParent) {
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
       if (kept[k]) {
@@ -602,7 +618,8 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
   }
 }
 
-bool carve_induced(void* workspace, size_t bytes, int64_t D, bool with_data, InducedMarks* m) {
+// pack: the data are to be packed by the marks' call
+bool carve_induced(void* workspace, size_t bytes, int64_t D, bool with_data, bool pack, InducedMarks* m) {
   Carver ws(workspace, bytes);
   const size_t words = static_cast<size_t>(D / kWave + 1);
   const size_t most = static_cast<size_t>(((D - 1) >> kTileShift) + 1);
@@ -617,6 +634,7 @@ bool carve_induced(void* workspace, size_t bytes, int64_t D, bool with_data, Ind
   m->outside = ws.take<int>(1);
   m->packed = ws.take<uint16_t>(static_cast<size_t>(D));
   m->word_at = with_data ? ws.take<int64_t>(words) : nullptr;
+  m->packed_data = with_data && pack ? ws.take<float>(static_cast<size_t>(D)) : nullptr;
   return ws.ok;
 }
 
@@ -686,8 +704,10 @@ template <typename IdT>
 void launch_compact(int64_t D, const InducedMarks& m, const int64_t* indptr, const void* cols,
                     const int64_t* sub_indptr, const float* data, const int64_t* e_ids, IdT* out_indices,
                     float* out_data, hipStream_t st) {
-  const bool past = streams(D, sizeof(IdT), data != nullptr);
-  auto* kernel = !data    ? (past ? induced_compact_kernel<IdT, kNoData, true> : induced_compact_kernel<IdT, kNoData, false>)
+  const bool packed = !data && out_data;
+  const bool past = streams(D, sizeof(IdT), data || packed);
+  auto* kernel = packed   ? (past ? induced_compact_kernel<IdT, kPacked, true> : induced_compact_kernel<IdT, kPacked, false>)
+                 : !data  ? (past ? induced_compact_kernel<IdT, kNoData, true> : induced_compact_kernel<IdT, kNoData, false>)
                  : !e_ids ? (past ? induced_compact_kernel<IdT, kByPosition, true>
                                   : induced_compact_kernel<IdT, kByPosition, false>)
                           : (past ? induced_compact_kernel<IdT, kByEdgeId, true>
@@ -715,7 +735,7 @@ int gs_induced_slice_applies(int64_t num_row_ids, int64_t S, int64_t D, int64_t)
   return num_row_ids > 0 && num_row_ids <= kMaxIds && S > 0 && S < (int64_t(1) << 31) && D >= (int64_t(1) << 20) && D >= 16 * S;
 }
 
-size_t gs_induced_slice_workspace_bytes(int64_t D, int with_data) {
+size_t gs_induced_slice_notify_workspace_bytes(int64_t D, int with_data) {
   if (D < 1) D = 1;
   const size_t words = static_cast<size_t>(D / kWave + 1), n = static_cast<size_t>(D);
   const int64_t tiles = ((D - 1) >> kTileShift) + 1;
@@ -724,12 +744,17 @@ size_t gs_induced_slice_workspace_bytes(int64_t D, int with_data) {
          padded(n * 2) + (with_data ? padded(words * 8) : 0);
 }
 
-int gs_induced_slice_mark(const int64_t* indptr, int64_t num_cols, const void* indices, int64_t nnz,
-                          int64_t num_rows, int id_bytes, const void* column_ids, int64_t S,
-                          const int64_t* sub_indptr, int64_t D, const void* row_ids,
-                          int64_t num_row_ids, const float* edge_data, const int64_t* edge_ids,
-                          int64_t* out_indptr, gs_mailbox* mailbox, int64_t ticket, void* workspace,
-                          size_t workspace_bytes, void* stream) {
+size_t gs_induced_slice_workspace_bytes(int64_t D, int with_data) {
+  return gs_induced_slice_notify_workspace_bytes(D, with_data) +
+         (with_data ? padded(static_cast<size_t>(D < 1 ? 1 : D) * 4) : 0);
+}
+
+int gs_induced_slice_mark_notify(const int64_t* indptr, int64_t num_cols, const void* indices, int64_t nnz,
+                                 int64_t num_rows, int id_bytes, const void* column_ids, int64_t S,
+                                 const int64_t* sub_indptr, int64_t D, const void* row_ids,
+                                 int64_t num_row_ids, int with_data, int64_t* out_indptr,
+                                 gs_mailbox* mailbox, int64_t ticket, void* workspace,
+                                 size_t workspace_bytes, void* stream) {
   GS_REQUIRE(gs_induced_slice_applies(num_row_ids, S, D, nnz) && num_rows >= 0,
              "gs_induced_slice_mark: sizes beyond gs_induced_slice_applies");
   GS_REQUIRE(indptr && indices && column_ids && sub_indptr && row_ids && out_indptr,
@@ -737,15 +762,15 @@ int gs_induced_slice_mark(const int64_t* indptr, int64_t num_cols, const void* i
   GS_REQUIRE(valid_id_bytes(id_bytes), "gs_induced_slice_mark: id_bytes must be 4 or 8, got %d",
              id_bytes);
   InducedMarks m;
-  if (!carve_induced(workspace, workspace_bytes, D, edge_data != nullptr, &m)) {
+  if (!carve_induced(workspace, workspace_bytes, D, with_data != 0, false, &m)) {
     set_error_text("gs_induced_slice_mark: workspace needs %zu bytes, 256-byte aligned",
-                   gs_induced_slice_workspace_bytes(D, edge_data != nullptr));
+                   gs_induced_slice_notify_workspace_bytes(D, with_data));
     return GS_ERR_WORKSPACE;
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t bound = num_rows > 0 ? num_rows : int64_t(1) << 40;  // (no bound given: no bitmap)
   const MarkCall c{indptr, num_cols, indices, column_ids, S, sub_indptr, D, row_ids, num_row_ids,
-                   bound, edge_data != nullptr};
+                   bound, with_data != 0};
   GS_RETURN_IF_ERROR(id_bytes == 8 ? pick_mark<int64_t>(c, m, st) : pick_mark<int32_t>(c, m, st));
   TileCount f{m.tile_counts};
   GS_RETURN_IF_ERROR(chained_scan(f, m.tiles, m.tile_base, m.lb, st, mailbox, ticket, m.outside));
@@ -754,16 +779,16 @@ int gs_induced_slice_mark(const int64_t* indptr, int64_t num_cols, const void* i
   return check_launch("induced_slice_mark");
 }
 
-int gs_induced_slice_compact(const int64_t* indptr, int id_bytes, const void* column_ids,
-                             const int64_t* sub_indptr, int64_t D, const float* edge_data,
-                             const int64_t* edge_ids, void* out_indices, float* out_data,
-                             void* workspace, size_t workspace_bytes, void* stream) {
+int gs_induced_slice_compact_parent(const int64_t* indptr, int id_bytes, const void* column_ids,
+                                    const int64_t* sub_indptr, int64_t D, const float* edge_data,
+                                    const int64_t* edge_ids, void* out_indices, float* out_data,
+                                    void* workspace, size_t workspace_bytes, void* stream) {
   GS_REQUIRE(D > 0 && out_indices && indptr && column_ids && sub_indptr, "gs_induced_slice_compact: bad argument");
   GS_REQUIRE(!edge_data == !out_data, "gs_induced_slice_compact: data without a place for them, or the other way round");
   GS_REQUIRE(valid_id_bytes(id_bytes), "gs_induced_slice_compact: id_bytes must be 4 or 8, got %d",
              id_bytes);
   InducedMarks m;
-  if (!carve_induced(workspace, workspace_bytes, D, out_data != nullptr, &m)) {
+  if (!carve_induced(workspace, workspace_bytes, D, out_data != nullptr, false, &m)) {
     set_error_text("gs_induced_slice_compact: pass the workspace given to gs_induced_slice_mark");
     return GS_ERR_WORKSPACE;
   }
@@ -774,6 +799,49 @@ int gs_induced_slice_compact(const int64_t* indptr, int id_bytes, const void* co
   else
     launch_compact(D, m, indptr, column_ids, sub_indptr, edge_data, edge_ids,
                    static_cast<int32_t*>(out_indices), out_data, st);
+  return check_launch("induced_slice_compact");
+}
+
+int gs_induced_slice_mark(const int64_t* indptr, int64_t num_cols, const void* indices, int64_t nnz,
+                          int64_t num_rows, int id_bytes, const void* column_ids, int64_t S,
+                          const int64_t* sub_indptr, int64_t D, const void* row_ids,
+                          int64_t num_row_ids, const float* edge_data, const int64_t* edge_ids,
+                          int64_t* out_indptr, void* workspace, size_t workspace_bytes,
+                          void* stream) {
+  InducedMarks m;
+  if (D > 0 && !carve_induced(workspace, workspace_bytes, D, edge_data != nullptr, true, &m)) {
+    set_error_text("gs_induced_slice_mark: workspace needs %zu bytes, 256-byte aligned",
+                   gs_induced_slice_workspace_bytes(D, edge_data != nullptr));
+    return GS_ERR_WORKSPACE;
+  }
+  GS_RETURN_IF_ERROR(gs_induced_slice_mark_notify(indptr, num_cols, indices, nnz, num_rows, id_bytes, column_ids, S,
+                                                  sub_indptr, D, row_ids, num_row_ids, edge_data != nullptr, out_indptr,
+                                                  nullptr, 0, workspace, workspace_bytes, stream));
+  if (!edge_data) return GS_OK;
+  // (the other call of the pair knows no data: they wait for it where the row numbers do)
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (id_bytes == 8)
+    launch_compact<int64_t>(D, m, indptr, column_ids, sub_indptr, edge_data, edge_ids, nullptr, m.packed_data, st);
+  else
+    launch_compact<int32_t>(D, m, indptr, column_ids, sub_indptr, edge_data, edge_ids, nullptr, m.packed_data, st);
+  return check_launch("induced_slice_mark");
+}
+
+int gs_induced_slice_compact(int64_t D, int id_bytes, void* out_indices, float* out_data,
+                             void* workspace, size_t workspace_bytes, void* stream) {
+  GS_REQUIRE(D > 0 && out_indices, "gs_induced_slice_compact: bad argument");
+  GS_REQUIRE(valid_id_bytes(id_bytes), "gs_induced_slice_compact: id_bytes must be 4 or 8, got %d",
+             id_bytes);
+  InducedMarks m;
+  if (!carve_induced(workspace, workspace_bytes, D, out_data != nullptr, true, &m)) {
+    set_error_text("gs_induced_slice_compact: pass the workspace given to gs_induced_slice_mark");
+    return GS_ERR_WORKSPACE;
+  }
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (id_bytes == 8)
+    launch_compact(D, m, nullptr, nullptr, nullptr, nullptr, nullptr, static_cast<int64_t*>(out_indices), out_data, st);
+  else
+    launch_compact(D, m, nullptr, nullptr, nullptr, nullptr, nullptr, static_cast<int32_t*>(out_indices), out_data, st);
   return check_launch("induced_slice_compact");
 }
 

@@ -824,20 +824,30 @@ int gs_col_row_slice_compact(int64_t D, int id_bytes, void* out_indices, int64_t
  * sizes; nnz = edges of the parent, any number).  edge_data / edge_ids as for gs_slice_fill_data, NULL:
  * none.  num_rows: a bound on the row ids (0: none known); when a row id reaches it,
  * out_indptr[S] is -1 and the call has to be repeated with num_rows 0.  mark, then (total in
- * out_indptr[S] and, before the offsets are written, in the mailbox, NULL: none) compact with the same arrays and the same workspace; out_data NULL exactly when
- * edge_data is. */
+ * out_indptr[S]) compact with the same workspace; out_data NULL exactly when edge_data was. */
 int gs_induced_slice_applies(int64_t num_row_ids, int64_t S, int64_t D, int64_t nnz);
 size_t gs_induced_slice_workspace_bytes(int64_t D, int with_data);
 int gs_induced_slice_mark(const int64_t* indptr, int64_t num_cols, const void* indices, int64_t nnz,
                           int64_t num_rows, int id_bytes, const void* column_ids, int64_t S,
                           const int64_t* sub_indptr, int64_t D, const void* row_ids,
                           int64_t num_row_ids, const float* edge_data, const int64_t* edge_ids,
-                          int64_t* out_indptr, gs_mailbox* mailbox, int64_t ticket, void* workspace,
-                          size_t workspace_bytes, void* stream);
-int gs_induced_slice_compact(const int64_t* indptr, int id_bytes, const void* column_ids,
-                             const int64_t* sub_indptr, int64_t D, const float* edge_data,
-                             const int64_t* edge_ids, void* out_indices, float* out_data,
+                          int64_t* out_indptr, void* workspace, size_t workspace_bytes,
+                          void* stream);
+int gs_induced_slice_compact(int64_t D, int id_bytes, void* out_indices, float* out_data,
                              void* workspace, size_t workspace_bytes, void* stream);
+/* The same for a caller that keeps the arrays until both calls have run: the data are read by the compact, from the
+ * parent and of kept edges only, and the total is in the mailbox (NULL: none) before the offsets are written. */
+size_t gs_induced_slice_notify_workspace_bytes(int64_t D, int with_data);
+int gs_induced_slice_mark_notify(const int64_t* indptr, int64_t num_cols, const void* indices, int64_t nnz,
+                                 int64_t num_rows, int id_bytes, const void* column_ids, int64_t S,
+                                 const int64_t* sub_indptr, int64_t D, const void* row_ids,
+                                 int64_t num_row_ids, int with_data, int64_t* out_indptr,
+                                 gs_mailbox* mailbox, int64_t ticket, void* workspace,
+                                 size_t workspace_bytes, void* stream);
+int gs_induced_slice_compact_parent(const int64_t* indptr, int id_bytes, const void* column_ids,
+                                    const int64_t* sub_indptr, int64_t D, const float* edge_data,
+                                    const int64_t* edge_ids, void* out_indices, float* out_data,
+                                    void* workspace, size_t workspace_bytes, void* stream);
 
 /* Membership filter of a COO that keeps global ids: replaces
  * impl::COORowSlicingGlobalIdCUDA, BatchCOOSlicingCUDA (src/cuda/batch_slicing.cu:325,232)

@@ -6,6 +6,7 @@ import torch
 
 import graph_sampling_amd as gs
 from oracle import oracle as O
+from graph_sampling_amd import capi
 from util import to_dev
 
 pytestmark = pytest.mark.gpu
@@ -248,3 +249,26 @@ def test_streamed_positions(dev, data, n, idt):
     assert torch.equal(ptr[1:], torch.cumsum((want >= 0).view(S, degree).sum(1), 0))
     if data != "none":
         assert torch.equal(sub._CAPI_GetData("default"), order[want >= 0])
+
+
+@pytest.mark.parametrize("idt", [torch.int32, torch.int64])
+@pytest.mark.parametrize("data", ["none", "by position", "by map"])
+@pytest.mark.parametrize("n", [60_000, 2_000_000])  # both forms of the set
+def test_the_pair_whose_second_call_knows_no_data(dev, n, data, idt):
+    """gs_induced_slice_mark and _compact as they were before the forms that keep the arrays: no mailbox, and the data are
+    read by the first call; a row id at the bound on them is reported as a total of -1."""
+    indptr, indices, rng = _graph(n, 30, 50_001, 40, n)
+    cols, rows = rng.integers(0, n, 30_000).astype(np.int64), rng.integers(0, n, 5000).astype(np.int64)
+    cols[::100] = np.flatnonzero(np.diff(indptr) == 50_001)[0]
+    order = rng.permutation(indices.size)
+    w = rng.random(indices.size).astype(np.float32)
+    args = [to_dev(indptr, dev), to_dev(indices, dev, idt), to_dev(cols, dev, idt), to_dev(rows, dev, idt)]
+    e_ids = to_dev(order, dev) if data == "by map" else None
+    t_w = None if data == "none" else to_dev(w, dev)
+    ptr, idx, got = capi.induced_slice(*args, n, t_w, e_ids)
+    want = O.col_row_slice(indptr, indices, cols, rows)
+    assert np.array_equal(ptr.cpu().numpy(), want[0]) and np.array_equal(idx.cpu().numpy(), want[1])
+    if data != "none":
+        assert np.array_equal(got.cpu().numpy(), (w[order] if data == "by map" else w)[want[3]])
+    if n == 60_000:
+        assert int(capi.induced_slice(*args, int(rows.max()), t_w, e_ids)[-1]) == -1
