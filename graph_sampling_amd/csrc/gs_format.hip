@@ -449,7 +449,7 @@ radix_hist_kernel(Src src, int64_t E, int shift, Count* __restrict__ counts,
   }
   for (int j = threadIdx.x; j < kHistCopies * (kRadix + 1); j += T::kThreadsPerTile)
     (&s_hist[0][0])[j] = 0;
-  if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;
+  if (clear && blockIdx.x == 0 && threadIdx.x < 2) clear[threadIdx.x] = 0;
   lds_barrier();  // (the words stay on their way)
 #pragma unroll
   for (int k = 0; k < T::kPerThread; ++k) {
@@ -547,10 +547,11 @@ struct SortOutputs {
   int64_t* perm;
   uint32_t* key;
   int idx_bits;
-  int* wide;  // raised when a 64-bit value does not fit 32 bits (null: 32-bit values)
+  int* wide;  // [0]: raised when a 64-bit value does not fit 32 bits, [1]: gaps left (null: 32-bit values)
   bool stream;  // packed_pass_kernel: results as streams (kStreamResults)
   int64_t* indptr;  // packed_pass_kernel: the columns' offsets, from the tiles themselves (null: not here)
   int64_t num_keys;
+  uint4* gaps;  // runs of columns of one offset that the last pass leaves to gap_fill_kernel: first, how many, offset
 };
 
 // One pass of the sort over one tile, stable.  A wave owns its share of the tile, in index
@@ -772,6 +773,14 @@ radix_pass_kernel(Src src, const ValT* __restrict__ val_in, int64_t E, int shift
 // moves: that pass 84 -> 85 us, the launch behind it, 19, gone; the list loaded and sorted 392 -> 379.
 constexpr int kPackedPasses = 3;
 constexpr uint32_t kWideTile = 16;  // offsets a thread beyond which a tile has long gaps
+// There a tile goes by its items: one item's columns, those from the item before on, have one offset.  Up to kGapLane of
+// them its lane stores, up to kGapHere its wave together, and more are left to a launch behind the sort in pieces of
+// kGapPiece: the columns above the last lower digit in use are all one tile's, 2.4 M of them where the lower 16 bits of
+// 2.45 M ids stay below 100.  Sorts of such lists and of ids whose lower bits are 30000 to 30004, us, by written keys / by
+// one workgroup with a search a column / so: 14 M edges 340/534/293 and 328/1080/288, 5 M 183/673/162 and 170/1440/155.
+constexpr int64_t kThreeDigitItems = 1'300'000;  // edges from which small tiles' last pass of three leaves the offsets
+constexpr int kGapBlocks = 512;
+constexpr uint32_t kGapLane = 4, kGapHere = 128, kGapPiece = 2048;
 constexpr int64_t kStreamResults = int64_t(1) << 27;  // bytes
 constexpr int rest_at(int passes) { return 64 - kRadixBits * (passes - 1); }  // of the key's digits in a word
 
@@ -1036,20 +1045,46 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
         const uint32_t d = i / lows;
         leave(d, from + i % lows, s_start[d], run_end(d));
       }
-    } else {  // long gaps: a wave or more a digit, and no search behind the digit's last edge
-      const uint32_t parts = digits < T::kWaves ? T::kWaves / digits : 1u;
-      for (uint32_t u = wave; u < digits * parts; u += T::kWaves) {
-        const uint32_t d = u % digits, hi = run_end(d);
-        const uint32_t lo = s_start[d];
-        const uint32_t top = lo < hi ? static_cast<uint32_t>(s_word[hi - 1] >> kRestAt) + 1 : from;
-        uint32_t low = from + u / digits * kWave + lane;
-        for (; low < top; low += parts * kWave) leave(d, low, lo, hi);
-        const int64_t first = static_cast<int64_t>(d) << kLowBits, end = s_base[d] + hi;
-        const int64_t most_low = last.num_keys - first;
-        for (; low < from + lows && low <= most_low; low += parts * kWave) last.indptr[first + low] = end;
+    } else {  // long gaps: by items, and what lies behind a digit's last one
+      for (uint32_t u0 = wave * kWave; u0 < n + digits; u0 += kThreadsHere) {
+        const uint32_t u = u0 + lane;
+        uint32_t first = 0, count = 0, offset = 0;
+        if (u < n + digits) {
+          const uint32_t d = u < n ? s_dig[u] : u - n;
+          const uint32_t j = u < n ? u : run_end(d);
+          const uint32_t begin = j > static_cast<uint32_t>(s_start[d]) ? static_cast<uint32_t>(s_word[j - 1] >> kRestAt) + 1 : from;
+          const uint32_t end = u < n ? static_cast<uint32_t>(s_word[u] >> kRestAt) + 1 : from + lows;
+          first = (d << kLowBits) + begin;
+          const uint32_t most_here = static_cast<uint32_t>(last.num_keys) + 1;
+          if (first < most_here) count = (end < most_here - first + begin ? end : most_here - first + begin) - begin;
+          offset = static_cast<uint32_t>(s_base[d] + j);
+        }
+        if (count <= kGapLane) {
+          for (uint32_t k = 0; k < count; ++k) last.indptr[first + k] = offset;
+        } else if (count > kGapHere) {
+          uint32_t at = atomicAdd(last.wide + 1, (count + kGapPiece - 1) / kGapPiece);
+          for (uint32_t k = 0; k < count; k += kGapPiece, ++at)
+            last.gaps[at] = make_uint4(first + k, count - k < kGapPiece ? count - k : kGapPiece, offset, 0u);
+        }
+        for (unsigned long long some = __ballot(count > kGapLane && count <= kGapHere); some; some &= some - 1) {
+          const int from_lane = __builtin_ctzll(some);
+          const uint32_t f = __builtin_amdgcn_readlane(first, from_lane), c = __builtin_amdgcn_readlane(count, from_lane);
+          const uint32_t o = __builtin_amdgcn_readlane(offset, from_lane);
+          for (uint32_t k = lane; k < c; k += kWave) last.indptr[f + k] = o;
+        }
       }
     }
     if (threadIdx.x == 0 && base + n == E && last.num_keys >> kLowBits == kRadix) last.indptr[last.num_keys] = E;
+  }
+}
+
+// The long gaps of the columns' offsets, a wave a piece.
+__global__ void __launch_bounds__(kThreads)
+gap_fill_kernel(const uint4* __restrict__ gaps, const int* __restrict__ num_gaps, int64_t* __restrict__ indptr) {
+  const int n = *num_gaps, lane = threadIdx.x & (kWave - 1);
+  for (int g = blockIdx.x * (kThreads / kWave) + threadIdx.x / kWave; g < n; g += gridDim.x * (kThreads / kWave)) {
+    const uint4 gap = gaps[g];
+    for (uint32_t k = lane; k < gap.y; k += kWave) indptr[gap.x + k] = gap.z;
   }
 }
 
@@ -1130,7 +1165,7 @@ struct SortSpace {
   uint32_t* value[2];
   int64_t *counts, *offsets, *totals, *totals_before;
   uint32_t* keys;
-  int* wide;
+  int* wide;  // [2]
 };
 // (tables sized for the smaller tile, which has the larger ones)
 inline size_t sort_space_bytes(int64_t E) {
@@ -1149,7 +1184,7 @@ inline bool carve_sort(Carver& ws, int64_t E, SortSpace* s) {
   s->offsets = ws.take<int64_t>(static_cast<size_t>(table));
   s->totals = ws.take<int64_t>(kRadix);
   s->totals_before = ws.take<int64_t>(kRadix);
-  s->wide = ws.take<int>(1);
+  s->wide = ws.take<int>(2);
   return ws.ok;
 }
 
@@ -1254,15 +1289,19 @@ int coo2csc_impl(const IdT* key, const IdT* value, int64_t E, int64_t num_keys, 
       packed_value_bits(E, num_values, passes, blocks_for(E, large ? LargeTile::kSize : SmallTile::kSize));
   const bool may_be_wide = sizeof(IdT) == 8 || value_bits > 0;
   const bool short_keys = passes * kRadixBits <= 32;
-  // (offsets by the last pass's tiles; written keys and a launch of their own / so, us: 14 M edges, 2.45 M columns 301/281,
-  // 20 k 178/165, one of 2.45 M has all 628/557; 5 M, 5 M 151/143; small tiles: 1 M edges, 200 k columns 63/62, 60 k
-  // 46/42, 300 k, 20 k 40/37, but 1 M, 1 M 66/73 and 300 k, 300 k 58/67, a few tiles' searches)
-  const bool by_tiles = indptr && value_bits > 0 && (large ? num_keys : 4 * num_keys) <= E;
+  // (offsets by the last pass's tiles; written keys and a launch of their own / so, us: 14 M edges, 2.45 M columns 301/270,
+  // 20 k 178/157, the first of 2.45 M has all 626/302; 5 M, 5 M 150/139; small tiles: 300 k edges, 60 k columns 39/37, 1 M,
+  // 20 k 45/41, 1.5 M, 375 k 74/71, 3 M, 750 k 91/84, but 1 M, 1 M 66/73 and 300 k, 300 k 58/67, a few tiles' searches, and
+  // with three digits 300 k, 75 k 56/57, 1 M, 250 k 64/66, 32-bit ids, 1.25 M, 312 k 72/70 and 73/73, too few tiles)
+  const bool by_tiles = indptr && value_bits > 0 &&
+                        (large ? num_keys <= E : 4 * num_keys <= E && (passes == 2 || E >= kThreeDigitItems));
   const bool by_keys = indptr && short_keys && !by_tiles;
   const SortOutputs<IdT> outs{out_value, perm, by_keys ? s.keys : nullptr, idx_bits,
                               may_be_wide ? s.wide : nullptr,
                               E * static_cast<int64_t>(sizeof(int64_t) + sizeof(IdT) + sizeof(uint32_t)) >= kStreamResults,
-                              by_tiles ? indptr : nullptr, num_keys};
+                              by_tiles ? indptr : nullptr, num_keys, reinterpret_cast<uint4*>(s.keys)};
+  // (a gap is of more than kGapHere columns, of which there are no more than edges)
+  static_assert(kGapPiece >= kGapHere && 2 * sizeof(uint4) <= kGapHere * sizeof(uint32_t), "gaps fit in place of the keys");
   if (value_bits > 0) {
     const auto sort = large ? packed_passes<LargeTile, IdT> : packed_passes<SmallTile, IdT>;
     GS_RETURN_IF_ERROR(sort(key, value, E, passes, value_bits, s, outs, st));
@@ -1275,7 +1314,9 @@ int coo2csc_impl(const IdT* key, const IdT* value, int64_t E, int64_t num_keys, 
                        dim3(kThreads), 0, st, value, perm, E, s.wide, out_value);
   if (by_keys)  // (null: the caller wants the sorted order only)
     launch_indptr(static_cast<const uint32_t*>(s.keys), E, num_keys, indptr, st);
-  else if (indptr && !by_tiles)
+  else if (by_tiles)
+    hipLaunchKernelGGL(gap_fill_kernel, dim3(kGapBlocks), dim3(kThreads), 0, st, outs.gaps, s.wide + 1, indptr);
+  else if (indptr)
     hipLaunchKernelGGL((indptr_from_sorted_kernel<PermutedKeys<IdT>>),
                        dim3(blocks_for(num_keys + 1, kPtrCols)), dim3(kThreads), 0, st,
                        PermutedKeys<IdT>{key, perm}, E, num_keys, indptr);

@@ -111,17 +111,42 @@ def test_sort_with_the_values_in_its_words(dev, num_keys, skew, E, idt):
 
 @pytest.mark.parametrize("idt", ID_DTYPES)
 @pytest.mark.parametrize("E,num_keys", [(64 * 4096 + 1, 257), (64 * 4096 + 1, 64 * 4096 + 1), (64 * 4096 + 1, 64 * 4096 + 2),
+                                        (1_300_000, 325_000), (1_300_000, 325_001), (1_299_999, 324_999),
+                                        ((1 << 22) + 5, (1 << 22) + 5), ((1 << 22) + 5, (1 << 22) + 6),
                                         (1_000_003, 65_536), ((1 << 22) + 5, 65_537), (1 << 24, 1 << 24)])
 @pytest.mark.parametrize("keys", ["first", "last", "ends", "one low digit", "few"])
 def test_offsets_from_the_last_pass(dev, keys, E, num_keys, idt):
-    """Two digits and three, as many columns as edges and one more, and as many as three digits hold; keys
-    that leave long runs of columns without edges in front, in between and behind, which single tiles write."""
+    """Two digits and three, both sides of the lines up to which the last pass writes the offsets (as many columns as
+    edges; a quarter as many in small tiles, of three digits from 1.3 M edges on), and as many as three digits hold; keys
+    that leave long runs of columns without edges in front, in between and behind, which single tiles find."""
     gen = torch.Generator(device=dev)
     gen.manual_seed(E)
     choice = {"first": [0], "last": [num_keys - 1], "ends": [0, num_keys - 1],
               "one low digit": list(range(5, num_keys, 256)), "few": [1, 3, 255, 256, num_keys // 2 + 1]}[keys]
     choice = torch.tensor([k for k in choice if k < num_keys], device=dev)
     key = choice[torch.randint(0, choice.numel(), (E,), generator=gen, device=dev)].to(idt)
+    ip, val, perm = capi.coo2csc(key, key, num_keys, False)
+    assert torch.equal(val, torch.sort(key).values) and torch.equal(key[perm], val)
+    ends = torch.cumsum(torch.bincount(key.long(), minlength=num_keys), 0)
+    assert int(ip[0]) == 0 and torch.equal(ip[1:], ends)
+
+
+@pytest.mark.parametrize("idt", ID_DTYPES)
+@pytest.mark.parametrize("E,num_keys", [(300_007, 65_536), (1_300_003, 300_000), ((1 << 22) + 5, 1 << 22), ((1 << 22) + 5, 3_000_001),
+                                        ((1 << 24) - 7, (1 << 24) - 7)])
+def test_offsets_of_one_tile_with_gaps_of_every_length(dev, E, num_keys, idt):
+    """Nearly all edges share two lower halves, so one tile finds the columns of all others: gaps on both sides of the
+    lengths that a lane stores, a wave, and a launch behind the sort piece by piece, and those behind the last edges."""
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(E)
+    heavy = torch.arange(0, num_keys, 1 << 16, device=dev)
+    heavy = torch.cat([heavy, heavy + 60_000])
+    chain = torch.cumsum(torch.tensor([1, 4, 5, 6, 63, 64, 65, 127, 128, 129, 130, 2047, 2048, 2049, 4096, 4097, 30_000], device=dev), 0)
+    rare = torch.cat([chain, chain + ((num_keys >> 16) - 1 << 16), torch.randint(0, num_keys, (3000,), generator=gen, device=dev)])
+    rare = rare[(rare >= 0) & (rare & 0xFFFF < 60_000)]
+    heavy = heavy[heavy < num_keys]
+    key = torch.cat([rare, heavy[torch.randint(0, heavy.numel(), (E - rare.numel(),), generator=gen, device=dev)]])
+    key = key[torch.randperm(E, generator=gen, device=dev)].to(idt)
     ip, val, perm = capi.coo2csc(key, key, num_keys, False)
     assert torch.equal(val, torch.sort(key).values) and torch.equal(key[perm], val)
     ends = torch.cumsum(torch.bincount(key.long(), minlength=num_keys), 0)
