@@ -515,11 +515,13 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
                        const int64_t* __restrict__ sub_indptr, const float* __restrict__ data,
                        const int64_t* __restrict__ e_ids, IdT* __restrict__ out_indices,
                        float* __restrict__ out_data) {
+  constexpr bool kParent = DATA == kByPosition || DATA == kByEdgeId;
+  // kept positions of a tile's words of several columns, and above them the places of their data in the tile
+  __shared__ uint32_t s_kept[kParent ? kCopyTiles : 1][kTile];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // (a scalar, and so are all addresses' bases)
   const int64_t t = static_cast<int64_t>(blockIdx.x) * kCopyTiles + wave;
   if (t >= m.tiles) return;
-  constexpr bool kParent = DATA == kByPosition || DATA == kByEdgeId;
   const int64_t first = m.tile_base[t], base = out_indices ? first : t * kTile;
   const int count = static_cast<int>(m.tile_base[t + 1] - first);
   unsigned long long my_word = 0;  // lane k: word k of the tile
@@ -538,6 +540,115 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
     const int r = k * kWave + lane;
     v[k] = m.packed[t * kTile + (r < count ? r : count - 1)];
   }
+  auto put_indices = [&] {
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int r = k * kWave + lane;
+      if (out_indices && r < count) {
+        if (STREAM)
+          __builtin_nontemporal_store(static_cast<IdT>(v[k]), out_indices + base + r);
+        else
+          out_indices[base + r] = static_cast<IdT>(v[k]);
+      }
+    }
+  };
+  auto put_datum = [&](float datum, int r) {
+    if (STREAM)
+      __builtin_nontemporal_store(datum, out_data + base + r);
+    else
+      out_data[base + r] = datum;
+  };
+  auto of = [](uint64_t u, int k) {  // lane k's
+    return static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u >> 32), k))) << 32 |
+           static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u), k));
+  };
+  auto set_before = [](uint64_t word) {
+    return static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(word >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(word), 0)));
+  };
+  if constexpr (kParent) {
+    const bool of_several = my_word && !WordAt::one(my_at);
+    const uint64_t several_words = __ballot(of_several);
+    if (several_words) {
+      // Kept edge by kept edge, so that a column is looked for where an edge is kept, and three of a lane's together, so
+      // that they are the same few trips.  (Position by position, one word behind the other, the whole call took 135 us
+      // where it takes 116, 8 M positions in columns of 16, 4 % kept; all words' positions together 130.)
+      int most = of_several ? static_cast<int>(WordAt::more(my_at)) : 0;
+#pragma unroll
+      for (int d = 1; d < kPer; d <<= 1) {
+        const int other = __shfl_xor(most, d, kWave);
+        most = most > other ? most : other;
+      }
+      most = __builtin_amdgcn_readfirstlane(most);
+      uint32_t* kept_at = s_kept[wave];
+      int listed = 0;
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) {
+        if (!(several_words >> k & 1u)) continue;
+        const uint64_t word = of(my_word, k);
+        const int before = set_before(word);
+        if (word >> lane & 1u)
+          kept_at[listed + before] =
+              static_cast<uint32_t>(__builtin_amdgcn_readlane(my_rank, k) + before) << 16 | (k * kWave + lane);
+        listed += __popcll(word);
+      }
+      __builtin_amdgcn_wave_barrier();
+      auto some = [&](int r0, auto how_many) {
+        constexpr int N = decltype(how_many)::value;
+        int64_t at[N], end[N], start[N];
+        int lo[N], hi[N], r[N];
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+          const int j = r0 + u * kWave + lane;
+          const uint32_t kept_one = kept_at[j < listed ? j : listed - 1];
+          const int p = static_cast<int>(kept_one & 0xFFFFu);
+          const int64_t where = __shfl(my_at, p / kWave, kWave);
+          r[u] = static_cast<int>(kept_one >> 16);
+          at[u] = t * kTile + p;
+          lo[u] = static_cast<int>(WordAt::first(where));
+          hi[u] = lo[u] + static_cast<int>(WordAt::more(where));
+        }
+        for (int left = most; left; left >>= 1) {
+#pragma unroll
+          for (int u = 0; u < N; ++u) end[u] = sub_indptr[lo[u] + ((hi[u] - lo[u]) >> 1) + 1];
+#pragma unroll
+          for (int u = 0; u < N; ++u) {
+            const int mid = lo[u] + ((hi[u] - lo[u]) >> 1);
+            if (lo[u] < hi[u]) {
+              if (end[u] > at[u]) hi[u] = mid; else lo[u] = mid + 1;
+            }
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+          start[u] = static_cast<int64_t>(cols[lo[u]]);
+          end[u] = sub_indptr[lo[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < N; ++u) at[u] += indptr[start[u]] - end[u];
+        if constexpr (DATA == kByEdgeId) {
+#pragma unroll
+          for (int u = 0; u < N; ++u) at[u] = once(e_ids + at[u]);
+        }
+        float datum[N];
+#pragma unroll
+        for (int u = 0; u < N; ++u) datum[u] = once(data + at[u]);
+#pragma unroll
+        for (int u = 0; u < N; ++u)
+          if (r0 + u * kWave + lane < listed) put_datum(datum[u], r[u]);
+      };
+      if (listed <= kWave) {
+        some(0, std::integral_constant<int, 1>());
+      } else {
+        for (int r0 = 0; r0 < listed; r0 += 3 * kWave) some(r0, std::integral_constant<int, 3>());
+      }
+      if (listed == count) {
+        put_indices();
+        return;
+      }
+      if (of_several) my_word = 0;  // (the others' edges below)
+    }
+  }
   bool kept[kParent ? kPer : 1];
   int rank[kParent ? kPer : 1];
   float x[DATA == kNoData ? 1 : kPer];
@@ -549,35 +660,17 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
     }
   }
   if constexpr (kParent) {
-    auto of = [](uint64_t u, int k) {  // lane k's
-      return static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u >> 32), k))) << 32 |
-             static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u), k));
-    };
     int64_t at[kPer];
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
       const uint64_t word = of(my_word, k);
       const int64_t where = static_cast<int64_t>(of(static_cast<uint64_t>(my_at), k));
       kept[k] = word >> lane & 1u;
-      rank[k] = __builtin_amdgcn_readlane(my_rank, k) +
-                __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(word >> 32),
-                                          __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(word), 0));
+      rank[k] = __builtin_amdgcn_readlane(my_rank, k) + set_before(word);
       // (lanes whose edge is left out read with the word's first kept one, a word without any the first datum:
       // data may end before edges that are not kept)
       const int place = kept[k] ? lane : (word ? __builtin_ctzll(word) : 0);
-      if (!word) {
-        at[k] = 0;
-      } else if (WordAt::one(where)) {
-        at[k] = where + place;
-      } else {
-        const int64_t p = t * kTile + k * kWave + place;
-        int64_t lo = WordAt::first(where), hi = lo + WordAt::more(where);
-        while (lo < hi) {
-          const int64_t mid = (lo + hi) >> 1;
-          if (sub_indptr[mid + 1] > p) hi = mid; else lo = mid + 1;
-        }
-        at[k] = indptr[static_cast<int64_t>(cols[lo])] + p - sub_indptr[lo];
-      }
+      at[k] = word ? where + place : 0;
     }
     if constexpr (DATA == kByEdgeId) {
 #pragma unroll
@@ -589,32 +682,16 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
 #pragma unroll
     for (int k = 0; k < kPer; ++k) x[k] = once(data + at[k]);
   }
+  put_indices();
+  if constexpr (DATA == kPacked) {
 #pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    const int r = k * kWave + lane;
-    if (out_indices && r < count) {
-      if (STREAM)
-        __builtin_nontemporal_store(static_cast<IdT>(v[k]), out_indices + base + r);
-      else
-        out_indices[base + r] = static_cast<IdT>(v[k]);
-      if constexpr (DATA == kPacked) {
-        if (STREAM)
-          __builtin_nontemporal_store(x[k], out_data + base + r);
-        else
-          out_data[base + r] = x[k];
-      }
-    }
+    for (int k = 0; k < kPer; ++k)
+      if (k * kWave + lane < count) put_datum(x[k], k * kWave + lane);
   }
   if constexpr (kParent) {
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-      if (kept[k]) {
-        if (STREAM)
-          __builtin_nontemporal_store(x[k], out_data + base + rank[k]);
-        else
-          out_data[base + rank[k]] = x[k];
-      }
-    }
+    for (int k = 0; k < kPer; ++k)
+      if (kept[k]) put_datum(x[k], rank[k]);
   }
 }
 
@@ -726,11 +803,13 @@ extern "C" {
 // An id set that fits one compute unit's LDS; enough positions for every compute unit to earn the
 // building of its copy of the set back; columns that are not all short (the positions of a tile are
 // resolved among a handful of staged offsets).  The whole call in us, general slice / this one, 64-bit
-// ids, of graphs of 200 k nodes (a bit per node) and 1 M (buckets), with the edges' data:
-//   8000 ids, 0.5 M / 1 M / 2 M positions   78/68 80/69 86/75    78/85 81/79 87/83
-//   1000 ids, 0.25 M / 1 M positions        67/49 70/50          75/52 68/51
-//   positions / columns 4, 8, 12, 16, 32    94/89 94/94 97/96 98/92 93/91    93/93 89/88 88/85 87/89 87/82
-// so the lines lie where nothing is lost with either form.  nnz does not matter.
+// ids, 8000 of them, of graphs of 200 k nodes (a bit per node) and 1 M (buckets), with the edges' data:
+//   positions / columns      16       32       64       256           16       32       64       256
+//   1 M positions         74/58    77/56    69/52    65/45         76/72    72/72    71/65    66/57
+//   2 M                   82/63    79/62    76/58    72/49         82/76    81/71    78/68    75/64
+//   8 M                  159/116  157/112  154/93   151/70        163/150  158/152  154/131  145/101
+// and of 1000 ids, 1 M and 8 M, 72/52 159/109, 68/51 154/105, 71/46 151/86, 63/40 147/62; 72/54 160/116, 69/53 149/107,
+// 68/48 145/88, 67/40 124/66: nothing is lost with either form on this side of the lines.  nnz does not matter.
 int gs_induced_slice_applies(int64_t num_row_ids, int64_t S, int64_t D, int64_t) {
   return num_row_ids > 0 && num_row_ids <= kMaxIds && S > 0 && S < (int64_t(1) << 31) && D >= (int64_t(1) << 20) && D >= 16 * S;
 }

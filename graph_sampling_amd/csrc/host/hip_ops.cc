@@ -1446,9 +1446,8 @@ std::tuple<torch::Tensor, torch::Tensor> InducedSlicing(const torch::Tensor& ind
   int64_t D;
   std::tie(sub_indptr, D) = SliceOffsets(indptr, column_ids, idb);
   // Without data to fetch the general slice has less to do, and the other needs longer columns, or
-  // more positions where the set is one of buckets.  General slice / set in LDS, us, 64-bit ids:
-  // 2 M positions in columns of 16, 32, 262 edges 87/95 86/90 81/73 (200 k nodes); 1 M and
-  // 2 M positions of 1 M nodes, 32-bit ids 74/78 83/78.
+  // more positions where the set is one of buckets.  General slice / set in LDS, us, 64-bit ids, 8000 in the set:
+  // 1 M, 2 M, 8 M positions in columns of 64 edges 63/51 70/57 143/89 (200 k nodes), 2 M and 8 M 74/68 146/140 (1 M nodes).
   const bool pays = edge || (D >= 64 * S && (num_rows <= 600'000 || D >= (int64_t(1) << 21)));
   if (!pays || !gs_induced_slice_applies(nr, S, D, nnz)) {
     auto r = ColRowSliceOf(indptr, indices, column_ids, row_ids, sub_indptr, D, torch::nullopt,

@@ -272,3 +272,43 @@ def test_the_pair_whose_second_call_knows_no_data(dev, n, data, idt):
         assert np.array_equal(got.cpu().numpy(), (w[order] if data == "by map" else w)[want[3]])
     if n == 60_000:
         assert int(capi.induced_slice(*args, int(rows.max()), t_w, e_ids)[-1]) == -1
+
+
+@pytest.mark.parametrize("data", ["by position", "by map"])
+@pytest.mark.parametrize("idt", [torch.int32, torch.int64])
+@pytest.mark.parametrize("lens", [[17], [40, 1, 0, 60, 0], [300, 20, 9, 700], [511, 1], [64, 64, 65, 63]])
+def test_data_of_tiles_of_several_columns(dev, lens, idt, data):
+    """Tiles whose words are all of several columns, and some of them; as many of their edges kept as a lane takes at once
+    (64, 192) and one more and less, none and all; a column id that is none stands first."""
+    rng = np.random.default_rng(len(lens))
+    degree = np.resize(lens, (1_100_000 // sum(lens) + 1) * len(lens))
+    cols = rng.permutation(degree.size)
+    parent = np.zeros_like(degree)
+    parent[cols] = degree
+    indptr = np.concatenate([[0], np.cumsum(parent)]).astype(np.int64)
+    D, n = int(indptr[-1]), 70_000
+    kept = np.zeros((D + 511) // 512 * 512, bool)
+    for t, k in zip(range(0, D, 512), np.resize([0, 1, 63, 64, 65, 191, 192, 193, 384, 385, 511, 512], D // 512 + 1)):
+        kept[t + rng.permutation(512)[:k]] = True
+    start = np.repeat(indptr[cols], degree)
+    offset = np.concatenate([[0], np.cumsum(degree)])
+    at = start + np.arange(D) - np.repeat(offset[:-1], degree)  # where the slice's positions are in the parent
+    ids = np.where(kept[:D], rng.integers(0, 3000, D) * 2, rng.integers(0, 3000, D) * 2 + 1)
+    indices = np.empty(D, np.int64)
+    indices[at] = ids
+    cols = np.concatenate([[-1], cols]).astype(np.int64)
+    rows = rng.permutation(3000).astype(np.int64) * 2
+    g = gs.Graph(False)
+    w, order = rng.random(D).astype(np.float32), np.arange(D)
+    if data == "by map":
+        order = rng.permutation(D)
+        ptr, idx, got = capi.induced_slice(to_dev(indptr, dev), to_dev(indices, dev, idt), to_dev(cols, dev, idt),
+                                           to_dev(rows, dev, idt), n, to_dev(w, dev), to_dev(order, dev))
+    else:
+        g._CAPI_LoadCSC(to_dev(indptr, dev), to_dev(indices, dev, idt))
+        g._CAPI_SetData(to_dev(w, dev))
+        sub = g._CAPI_FusionSlicing(to_dev(cols, dev, idt), to_dev(rows, dev, idt))
+        (ptr, idx, _), got = sub._CAPI_GetCSC(), sub._CAPI_GetData("default")
+    want = O.col_row_slice(indptr, indices, cols, rows)
+    assert np.array_equal(ptr.cpu().numpy(), want[0]) and np.array_equal(idx.cpu().numpy(), want[1])
+    assert np.array_equal(got.cpu().numpy(), w[order][want[3]])
