@@ -944,7 +944,7 @@ torch::Tensor Graph::Sum(int64_t axis, int64_t powk, int64_t on_format) {
                            (axis == 1 && IsCsrLike(on_format) && segments(csr_, val_row_ids_));
   torch::Tensor out = all_written ? torch::empty({size}, data.options()) : torch::zeros({size}, data.options());
   if (on_format == _COO)
-    COOGraphSum(coo_, data, out, powk, 1 - axis);
+    hip::CooSum(axis == 1 ? coo_->row : coo_->col, coo_->e_ids, data, out, powk, true);
   else if (axis == 0 && IsCscLike(on_format))
     CSCGraphSum(csc_, val_col_ids_, data, out, powk);
   else if (axis == 1 && IsCsrLike(on_format))

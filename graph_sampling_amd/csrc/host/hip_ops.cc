@@ -1267,15 +1267,15 @@ void SegmentSum(const torch::Tensor& indptr, const torch::optional<torch::Tensor
 }
 
 void CooSum(const torch::Tensor& target, const torch::optional<torch::Tensor>& e_ids,
-            const torch::Tensor& data, torch::Tensor out, int64_t powk) {
+            const torch::Tensor& data, torch::Tensor out, int64_t powk, bool fresh) {
   const int idb = IdBytes(target, "coo target");
   NeedF32(data, "data");
   NeedF32(out, "out");
   auto ws = Scratch(gs_coo_sum_workspace_bytes(target.numel(), out.numel()), target);
-  Check(gs_coo_sum_fresh(target.data_ptr(), idb, OptI64(e_ids, "e_ids"), data.data_ptr<float>(),
-                          target.numel(), powk, out.numel(), out.data_ptr<float>(), ws.data_ptr(),
-                          ws.numel(), Stream(target)),
-        "gs_coo_sum_fresh");
+  const auto sum = fresh ? gs_coo_sum_fresh : gs_coo_sum_binned;
+  Check(sum(target.data_ptr(), idb, OptI64(e_ids, "e_ids"), data.data_ptr<float>(), target.numel(), powk,
+            out.numel(), out.data_ptr<float>(), ws.data_ptr(), ws.numel(), Stream(target)),
+        fresh ? "gs_coo_sum_fresh" : "gs_coo_sum_binned");
 }
 
 void SegmentNormalize(const torch::Tensor& indptr, const torch::optional<torch::Tensor>& e_ids,

@@ -241,8 +241,9 @@ void SddmmCsc(const std::string& op, const Bcast& b, const torch::Tensor& indptr
 void SegmentSum(const torch::Tensor& indptr, const torch::optional<torch::Tensor>& e_ids,
                 const torch::optional<torch::Tensor>& n_ids, const torch::Tensor& data,
                 torch::Tensor out, int64_t powk);
+// added to what `out` holds; fresh: out holds nothing yet, every entry is written
 void CooSum(const torch::Tensor& target, const torch::optional<torch::Tensor>& e_ids,
-            const torch::Tensor& data, torch::Tensor out, int64_t powk);
+            const torch::Tensor& data, torch::Tensor out, int64_t powk, bool fresh = false);
 void SegmentNormalize(const torch::Tensor& indptr, const torch::optional<torch::Tensor>& e_ids,
                       const torch::Tensor& data, torch::Tensor out);
 void EDivUSum(const torch::Tensor& row, const torch::Tensor& col, const torch::Tensor& data,

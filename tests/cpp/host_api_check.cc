@@ -173,6 +173,14 @@ static void EdgeData() {
   CHECK_THAT(torch::allclose(g->Sum(0, 2, _CSC), torch::tensor({5.f, 0.f, 50.f, 36.f}).to(torch::kCUDA)));
   CHECK_THAT(torch::allclose(g->Sum(1, 1, _CSR), torch::tensor({7.f, 9.f, 5.f, 0.f}).to(torch::kCUDA)));
   CHECK_THAT(torch::allclose(g->Sum(1, 1, _COO), torch::tensor({7.f, 9.f, 5.f, 0.f}).to(torch::kCUDA)));
+  // the format-level sum over a COO adds to what its output holds: few edges, and enough for bins
+  for (int64_t edges : {int64_t(3000), int64_t(300000)}) {
+    auto coo = std::make_shared<gs::COO>(gs::COO{torch::arange(0, edges, I64()) % 1000, torch::arange(0, edges, I64()) % 7,
+                                                 torch::nullopt});
+    Tensor held = torch::full({1000}, 5.f, F32());
+    gs::COOGraphSum(coo, torch::ones({edges}, F32()), held, 1, 0);
+    CHECK_THAT(held.equal(torch::full({1000}, 5.f + edges / 1000, F32())));
+  }
   auto n = g->Normalize(0, _CSC);
   CHECK_THAT(torch::allclose(n->GetData().value(),
                              torch::tensor({1 / 3.f, 2 / 3.f, 3 / 12.f, 4 / 12.f, 5 / 12.f, 1.f}).to(torch::kCUDA)));
