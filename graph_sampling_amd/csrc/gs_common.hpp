@@ -709,7 +709,7 @@ int batch_relabel_binned(const void* seeds, const int64_t* seeds_ptr, const void
 // along instead of leaving them to a second launch.  What bounds it are two trips to memory for f and one for the
 // look-back.  A tile whose wait runs out adds up what lies in front of it itself, so the offsets are right whatever
 // happens (who reads them does so in launches that are queued already and cannot be told).  out[n] and the mailbox get
-// the total, -1 when *outside is set.
+// the total, -1 when *outside is set; the mailbox alone -1 too where a launch before this one gave up on the same state.
 template <typename F, int ITEMS>
 __global__ void __launch_bounds__(kScanThreads)
 scan_chain_kernel(F f, int64_t n, int64_t* __restrict__ out, LookbackState lb, const int* __restrict__ outside,
@@ -757,7 +757,9 @@ scan_chain_kernel(F f, int64_t n, int64_t* __restrict__ out, LookbackState lb, c
     int64_t all = s_prefix + total;
     if (outside && *outside) all = -1;
     out[n] = all;
-    post_mailbox(box, all, ticket);
+    // (2: an id was too wide for an earlier launch's table, which is that launch's to report)
+    const unsigned int left = __hip_atomic_load(lb.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    post_mailbox(box, left == 1u ? -1 : all, ticket);
   }
 }
 

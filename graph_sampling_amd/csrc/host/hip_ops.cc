@@ -279,9 +279,13 @@ int64_t ReadTotal(const torch::Tensor& values, int64_t at, void* stream, const c
 struct TotalBox {
   explicit TotalBox(const torch::Tensor& like) : boxes(Boxes(like.get_device())), ticket(boxes.next++) {}
   gs_mailbox* slot() const { return boxes.slot(ticket); }
-  int64_t Wait(const torch::Tensor& values, int64_t at, void* stream, const char* what) const {
+  // state: the launch's look-back state, if it has one that other launches have used
+  int64_t Wait(const torch::Tensor& values, int64_t at, void* stream, const char* what,
+               const torch::Tensor& state = {}) const {
     const int64_t total = WaitBox(slot(), ticket, stream, what);
-    return total == kLost ? values[at].item<int64_t>() : total;
+    if (total == kLost) return values[at].item<int64_t>();
+    if (state.defined() && total < 0) GaveUp(state, stream, what);
+    return total;
   }
   HostBoxes& boxes;
   const int64_t ticket;
@@ -305,7 +309,7 @@ int64_t SliceCount(const torch::Tensor& indptr, const torch::Tensor& column_ids,
                                  sub_indptr.data_ptr<int64_t>(), total.slot(), total.ticket, state.buf.data_ptr(),
                                  state.buf.numel(), state.epoch, st),
           "gs_slice_count");
-    return total.Wait(sub_indptr, S, st, "gs_slice_count");
+    return total.Wait(sub_indptr, S, st, "gs_slice_count", state.buf);
   }
   auto ws = Scratch(gs_slice_workspace_bytes(S), indptr);
   Check(gs_slice_count_notify(indptr.data_ptr<int64_t>(), indptr.numel() - 1, column_ids.data_ptr(),
@@ -411,11 +415,13 @@ SliceResult SampleInto(const torch::Tensor& indptr, const torch::Tensor& indices
   void* st = Stream(indptr);
   const void* cols = fused ? column_ids.data_ptr() : nullptr;
   const TotalBox total(indptr);
+  torch::Tensor state;
   if (CountsInOneLaunch(S)) {
-    FusedStateBuf& state = FusedState(gs_chained_count_state_bytes(S), indptr, st);
+    FusedStateBuf& s = FusedState(gs_chained_count_state_bytes(S), indptr, st);
+    state = s.buf;
     Check(gs_sample_count_chained(indptr.data_ptr<int64_t>(), indptr.numel() - 1, cols, idb, S, fanout,
                                   replace ? 1 : 0, sub_indptr.data_ptr<int64_t>(), total.slot(), total.ticket,
-                                  state.buf.data_ptr(), state.buf.numel(), state.epoch, st),
+                                  state.data_ptr(), state.numel(), s.epoch, st),
           "gs_sample_count");
   } else {
     Check(gs_sample_count_notify(indptr.data_ptr<int64_t>(), indptr.numel() - 1, cols, idb, S, fanout,
@@ -425,7 +431,7 @@ SliceResult SampleInto(const torch::Tensor& indptr, const torch::Tensor& indices
   }
   fill(cols, idb, S, sub_indptr, sub_indices, select_index, coo_col, ws, st);
   // the only host read of the call: the total is there before the fill has run
-  const int64_t nnz = total.Wait(sub_indptr, S, st, "gs_sample_count");
+  const int64_t nnz = total.Wait(sub_indptr, S, st, "gs_sample_count", state);
   if (with_coo) coo_col = coo_col.narrow(0, 0, nnz);
   return {sub_indptr, coo_col, sub_indices.narrow(0, 0, nnz), select_index.narrow(0, 0, nnz)};
 }

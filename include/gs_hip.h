@@ -129,8 +129,9 @@ int gs_slice_count_notify(const int64_t* indptr, int64_t num_cols, const void* c
                           int id_bytes, int64_t S, int64_t* sub_indptr, gs_mailbox* mailbox,
                           int64_t ticket, void* workspace, size_t workspace_bytes, void* stream);
 /* The same count (and gs_sample_count_notify's) in one launch where the caller keeps a look-back state: state and
- * epoch as for gs_sample_uniform_fused, gs_chained_count_state_bytes(S) bytes; S > 0.  The error word in the state is
- * neither read nor raised: a tile that gives up waiting adds up what lies in front of it. */
+ * epoch as for gs_sample_uniform_fused, gs_chained_count_state_bytes(S) bytes; S > 0.  A tile that gives up waiting
+ * adds up what lies in front of it and raises no error; where an earlier launch on the state gave up (its error word is
+ * 1), the mailbox reads -1, and the offsets are right all the same. */
 size_t gs_chained_count_state_bytes(int64_t S);
 int gs_slice_count_chained(const int64_t* indptr, int64_t num_cols, const void* column_ids, int id_bytes,
                            int64_t S, int64_t* sub_indptr, gs_mailbox* mailbox, int64_t ticket, void* state,

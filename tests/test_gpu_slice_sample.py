@@ -1,4 +1,6 @@
 """GPU parity: column slicing and uniform sampling through the C ABI vs the CPU oracle."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -248,8 +250,7 @@ def test_out_of_range_column_ids_are_empty_columns(dev, idt):
 @pytest.mark.parametrize("S", [2048, 2049, 15_872, 15_873, 1 << 17, (1 << 17) + 1])
 def test_counts_in_one_launch_and_past_it(dev, idt, S):
     """Offsets of slices and of weighted samples on both sides of the lines between one workgroup, tiles that wait for
-    one another and two launches, again and again on one look-back state; an error that a sampler left in it is not theirs:
-    slices and samples are as they were, and the next one-launch sampler reports it, once."""
+    one another and two launches, again and again on one look-back state; an error that sticks to it is reported once."""
     n = 1 << 15
     rng = np.random.default_rng(S)
     degree = rng.integers(0, 4, n)
@@ -275,16 +276,89 @@ def test_counts_in_one_launch_and_past_it(dev, idt, S):
         assert np.array_equal(picked._CAPI_GetCSC()[0].cpu().numpy(), offsets(np.minimum(want, 2)))
     if 2048 < S <= 1 << 17:
         torch.ops.gs_ops._CAPI_DebugRaiseLookbackError(t_ptr)
-        sub = cut(cols)
-        assert np.array_equal(sub._CAPI_GetCSC()[0].cpu().numpy(), offsets(want))
-        for replace in (False, True):
-            picked = sub._CAPI_SamplingWithProbs(0, probs, 2, replace, gs._CSC, gs._CSC)
-            counts = np.where(want > 0, 2, 0) if replace else np.minimum(want, 2)
-            assert np.array_equal(picked._CAPI_GetCSC()[0].cpu().numpy(), offsets(counts))
         with pytest.raises(RuntimeError, match="gave up"):
-            g._CAPI_FusedColumnwiseSlicingSampling(to_dev(cols, dev, idt), 2, False)._CAPI_GetCSC()
-        picked = g._CAPI_FusedColumnwiseSlicingSampling(to_dev(cols, dev, idt), 2, False)
-        assert np.array_equal(picked._CAPI_GetCSC()[0].cpu().numpy(), offsets(np.minimum(want, 2)))
+            cut(cols)
+        assert np.array_equal(cut(cols)._CAPI_GetCSC()[0].cpu().numpy(), offsets(want))
+
+
+def _slice_between(dev, idt, S, seed):
+    """(cut, pick, check, degrees) of S columns, some out of range, of a graph of 2^15 nodes with 0 to 3 edges and a hub."""
+    n = 1 << 15
+    rng = np.random.default_rng(seed)
+    degree = rng.integers(0, 4, n)
+    degree[:2] = [5000, 0]
+    indptr = np.concatenate([[0], np.cumsum(degree)]).astype(np.int64)
+    g = gs.Graph(False)
+    g._CAPI_LoadCSC(to_dev(indptr, dev), to_dev(rng.integers(0, n, indptr[-1]), dev, idt))
+    cols = rng.integers(-1, n + 1, S)
+    want = np.where((cols >= 0) & (cols < n), degree[np.clip(cols, 0, n - 1)], 0)
+    t_cols = to_dev(cols, dev, idt)
+
+    def cut():
+        return g._CAPI_Slicing(t_cols, 0, gs._CSC, gs._CSC, False)
+
+    def pick(sub, replace):
+        probs = torch.rand(int(want.sum()), device=dev) + 0.1
+        return sub._CAPI_SamplingWithProbs(0, probs, 2, replace, gs._CSC, gs._CSC)
+
+    def check(graph, counts):
+        assert np.array_equal(graph._CAPI_GetCSC()[0].cpu().numpy(), np.concatenate([[0], np.cumsum(counts)]))
+
+    return cut, pick, check, want
+
+
+@pytest.mark.parametrize("idt", [torch.int32, torch.int64])
+@pytest.mark.parametrize("S", [2049, 15_873, 1 << 17])
+def test_a_state_that_gave_up_is_reported_once_by_weighted_samples(dev, idt, S):
+    """The same error word met by a weighted sample, whose fill is queued before the total is read: reported, once."""
+    cut, pick, check, want = _slice_between(dev, idt, S, S)
+    sub = cut()
+    check(sub, want)
+    for replace in (False, True):
+        torch.ops.gs_ops._CAPI_DebugRaiseLookbackError(sub._CAPI_GetCSC()[0])
+        with pytest.raises(RuntimeError, match="gave up"):
+            pick(sub, replace)
+        check(pick(sub, replace), np.where(want > 0, 2, 0) if replace else np.minimum(want, 2))
+        check(cut(), want)
+
+
+@pytest.mark.parametrize("S", [2048, 2049, 1 << 17])
+def test_slices_between_a_queued_minibatch_and_its_collection(dev, S):
+    """A queued minibatch that met an id beyond 32 bits has left that in the look-back state until it is collected: slices
+    and weighted samples in between are as they were, and so is the minibatch.  (In a thread of its own: it is sampled
+    layer by layer from then on, and the state is the thread's.)"""
+    failure = []
+
+    def body():
+        try:
+            torch.cuda.set_device(dev)
+            cut, pick, check, want = _slice_between(dev, torch.int64, S, S)
+            sub = cut()
+            check(sub, want)
+            nodes = 4000
+            ptr = torch.arange(0, 2 * nodes + 1, 2, device=dev)
+            ids = torch.arange(2 * nodes, device=dev) % nodes
+            ids[77] = (1 << 33) + 5
+            g = gs.Graph(False)
+            g._CAPI_LoadCSC(ptr, ids)
+            seeds = torch.arange(3000, device=dev)
+            handle = g._CAPI_QueueSampleLayers(seeds, [2], False)
+            check(cut(), want)
+            for replace in (False, True):
+                check(pick(sub, replace), np.where(want > 0, 2, 0) if replace else np.minimum(want, 2))
+            frontier, offsets, renamed = handle.collect()
+            assert torch.equal(offsets, ptr[:3001])
+            got = frontier[renamed].view(-1, 2).sort(1).values
+            assert torch.equal(got, ids[:6000].view(-1, 2).sort(1).values)
+            check(cut(), want)
+        except BaseException as e:  # noqa: BLE001
+            failure.append(e)
+
+    t = threading.Thread(target=body)
+    t.start()
+    t.join()
+    if failure:
+        raise failure[0]
 
 
 @pytest.mark.parametrize("n", [1, 2048, 2049, 15_872, 15_873, 1 << 17, 3_000_001])
