@@ -111,14 +111,11 @@ def test_sort_with_the_values_in_its_words(dev, num_keys, skew, E, idt):
 
 @pytest.mark.parametrize("idt", ID_DTYPES)
 @pytest.mark.parametrize("E,num_keys", [(64 * 4096 + 1, 257), (64 * 4096 + 1, 64 * 4096 + 1), (64 * 4096 + 1, 64 * 4096 + 2),
-                                        (1_300_000, 325_000), (1_300_000, 325_001), (1_299_999, 324_999),
-                                        ((1 << 22) + 5, (1 << 22) + 5), ((1 << 22) + 5, (1 << 22) + 6),
                                         (1_000_003, 65_536), ((1 << 22) + 5, 65_537), (1 << 24, 1 << 24)])
 @pytest.mark.parametrize("keys", ["first", "last", "ends", "one low digit", "few"])
 def test_offsets_from_the_last_pass(dev, keys, E, num_keys, idt):
-    """Two digits and three, both sides of the lines up to which the last pass writes the offsets (as many columns as
-    edges; a quarter as many in small tiles, of three digits from 1.3 M edges on), and as many as three digits hold; keys
-    that leave long runs of columns without edges in front, in between and behind, which single tiles find."""
+    """Two digits and three, as many columns as edges and one more, and as many as three digits hold; keys
+    that leave long runs of columns without edges in front, in between and behind, which single tiles write."""
     gen = torch.Generator(device=dev)
     gen.manual_seed(E)
     choice = {"first": [0], "last": [num_keys - 1], "ends": [0, num_keys - 1],
@@ -129,6 +126,17 @@ def test_offsets_from_the_last_pass(dev, keys, E, num_keys, idt):
     assert torch.equal(val, torch.sort(key).values) and torch.equal(key[perm], val)
     ends = torch.cumsum(torch.bincount(key.long(), minlength=num_keys), 0)
     assert int(ip[0]) == 0 and torch.equal(ip[1:], ends)
+
+
+@pytest.mark.parametrize("idt", ID_DTYPES)
+@pytest.mark.parametrize("E,num_keys", [(64 * 4096 + 4, 65_536), (64 * 4096 + 4, 65_537),
+                                        (1_300_000, 325_000), (1_300_000, 325_001), (1_299_999, 324_999),
+                                        ((1 << 22) + 5, (1 << 22) + 5), ((1 << 22) + 5, (1 << 22) + 6)])
+@pytest.mark.parametrize("keys", ["first", "last", "ends", "one low digit", "few"])
+def test_offsets_on_both_sides_of_the_last_pass_s_lines(dev, keys, E, num_keys, idt):
+    """Up to as many columns as edges the last pass writes the offsets; in small tiles a quarter as many, and of three
+    digits only from 1.3 M edges on."""
+    test_offsets_from_the_last_pass(dev, keys, E, num_keys, idt)
 
 
 @pytest.mark.parametrize("idt", ID_DTYPES)
