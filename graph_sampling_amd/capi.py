@@ -40,7 +40,7 @@ def lib():
                      "gs_coo_sum_workspace_bytes", "gs_coo_pick_rows_workspace_bytes",
                      "gs_coo_block_values_workspace_bytes", "gs_random_walk_workspace_bytes",
                      "gs_metapath_walk_workspace_bytes",
-                     "gs_induced_slice_workspace_bytes"):
+                     "gs_induced_slice_workspace_bytes", "gs_induced_slice_notify_workspace_bytes"):
             if hasattr(_lib, name):
                 getattr(_lib, name).restype = ctypes.c_size_t
         _lib.gs_sorted_union_max.restype = ctypes.c_int64
@@ -1229,9 +1229,10 @@ def col_row_slice(indptr, indices, column_ids, row_ids, col_ptr=None, row_ptr=No
     return out_indptr, out_indices, select_index, parent_index
 
 
-def induced_slice(indptr, indices, column_ids, row_ids, num_rows, data=None, e_ids=None):
-    """gs_slice_count + gs_induced_slice_{mark,compact}, the data gone before the second call; returns
-    (out_indptr, out_indices, out_data), out_indptr alone when a row id reached num_rows."""
+def induced_slice(indptr, indices, column_ids, row_ids, num_rows, data=None, e_ids=None, kept=False):
+    """gs_slice_count + gs_induced_slice_{mark,compact}, the data gone before the second call, or, kept, the
+    pair that may read them in either; returns (out_indptr, out_indices, out_data), out_indptr alone when a row id
+    reached num_rows."""
     _need(indptr, torch.int64, "indptr")
     idb = _ids(indices, "indices")
     _ids(column_ids, "column_ids", like=indices)
@@ -1241,23 +1242,31 @@ def induced_slice(indptr, indices, column_ids, row_ids, num_rows, data=None, e_i
     sub_indptr = slice_count(indptr, column_ids)
     D = _total(sub_indptr, S)
     out_indptr = torch.empty(S + 1, dtype=torch.int64, device=dev)
-    ws = workspace(lib().gs_induced_slice_workspace_bytes(_i64(D), int(data is not None)), dev)
+    L = lib()
+    ws = workspace(L.gs_induced_slice_notify_workspace_bytes(_i64(S), _i64(D), int(data is not None)) if kept else
+                   L.gs_induced_slice_workspace_bytes(_i64(D), int(data is not None)), dev)
     st = _stream(dev)
     edge_data = None if data is None else data.clone()
-    _check(lib().gs_induced_slice_mark(_ptr(indptr), _i64(indptr.numel() - 1), _ptr(indices), _i64(indices.numel()),
-                                       _i64(num_rows), idb, _ptr(column_ids), _i64(S), _ptr(sub_indptr), _i64(D),
-                                       _ptr(row_ids), _i64(nr), _ptr(edge_data), _ptr(e_ids), _ptr(out_indptr),
-                                       _ptr(ws), ctypes.c_size_t(ws.numel()), st), "gs_induced_slice_mark")
-    kept = _total(out_indptr, S)
-    if kept < 0:
+    args = (_ptr(indptr), _i64(indptr.numel() - 1), _ptr(indices), _i64(indices.numel()), _i64(num_rows), idb,
+            _ptr(column_ids), _i64(S), _ptr(sub_indptr), _i64(D), _ptr(row_ids), _i64(nr), _ptr(edge_data),
+            _ptr(e_ids), _ptr(out_indptr))
+    room = (_ptr(ws), ctypes.c_size_t(ws.numel()), st)
+    _check(L.gs_induced_slice_mark_notify(*args, ctypes.c_void_p(0), _i64(0), *room) if kept else
+           L.gs_induced_slice_mark(*args, *room), "gs_induced_slice_mark")
+    total = _total(out_indptr, S)
+    if total < 0:
         return out_indptr
-    if data is not None:
-        edge_data.fill_(float("nan"))
-    out_indices = torch.empty(kept, dtype=indices.dtype, device=dev)
-    out_data = None if data is None else torch.empty(kept, dtype=torch.float32, device=dev)
-    if kept > 0:
-        _check(lib().gs_induced_slice_compact(_i64(D), idb, _ptr(out_indices), _ptr(out_data), _ptr(ws),
-                                              ctypes.c_size_t(ws.numel()), st), "gs_induced_slice_compact")
+    out_indices = torch.empty(total, dtype=indices.dtype, device=dev)
+    out_data = None if data is None else torch.empty(total, dtype=torch.float32, device=dev)
+    if total > 0 and kept:
+        _check(L.gs_induced_slice_compact_parent(_ptr(indptr), idb, _ptr(column_ids), _i64(S), _ptr(sub_indptr), _i64(D),
+                                                 _ptr(edge_data), _ptr(e_ids), _ptr(out_indices), _ptr(out_data), *room),
+               "gs_induced_slice_compact_parent")
+    elif total > 0:
+        if data is not None:
+            edge_data.fill_(float("nan"))
+        _check(L.gs_induced_slice_compact(_i64(D), idb, _ptr(out_indices), _ptr(out_data), *room),
+               "gs_induced_slice_compact")
     return out_indptr, out_indices, out_data
 
 

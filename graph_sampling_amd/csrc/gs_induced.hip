@@ -15,11 +15,10 @@
 //   * the ids of the NEXT tile are asked for before this tile's marks leave, since the few waves
 //     beside the set have little else to hide that latency behind;
 //   * kept edges leave one bit each and, packed to the front of the tile's range of a scratch
-//     array, their new row number in 2 bytes; every 64 positions leave where they are in the parent.
-// A scan of the tile counts and one copy kernel put the pieces together; the copy reads the kept
-// edges' data from the parent.  (The marks reading them too and packing them beside the row numbers took
-// 185 us and the copy 85 in the case below, 1142 MB together; 967 MB so, 130 and 114.)  (With the tiles shared
-// by the waves of a workgroup, offsets and counts through LDS and two barriers a tile, the marks
+//     array, their new row number in 2 bytes, and beside it their datum or, with long columns, every
+//     64 positions where they are in the parent (marks_read_data).
+// A scan of the tile counts and one copy kernel put the pieces together; of long columns the copy reads
+// the kept edges' data from the parent.  (With the tiles shared by the waves of a workgroup, offsets and counts through LDS and two barriers a tile, the marks
 // took 293 us where a wave's own tiles took 225, before they were streamed.)
 //
 // Two forms of the set.  BitmapSet, for graphs whose numbers of nodes fit (about 600 k): a bit
@@ -51,6 +50,7 @@ constexpr int kStagedIds = 8192;          // ids up to which the ids themselves 
 constexpr uint32_t kFree = ~0u;
 constexpr size_t kLdsBytes = 160 * 1024;  // of a compute unit
 constexpr int kUnits = 256;               // compute units
+constexpr int64_t kLongColumns = 512;     // positions a column from which the copy reads the data (marks_read_data)
 constexpr int64_t kMostBits = 8 * static_cast<int64_t>(kLdsBytes);
 
 struct InducedMarks {
@@ -59,8 +59,8 @@ struct InducedMarks {
   int64_t* tile_counts;
   int64_t* tile_base;        // exclusive scan of tile_counts
   uint16_t* packed;          // new row numbers (places, 14 bits) of the kept edges, at the front of the tile's range
-  int64_t* word_at;          // with data (null: none): where a word's edges are in the parent (WordAt)
-  float* packed_data;        // the kept edges' data, beside packed, for callers of gs_induced_slice_compact (null: none)
+  int64_t* word_at;          // with data that the copy reads: where a word's edges are in the parent (WordAt)
+  float* packed_data;        // with data that the marks read: the kept edges', beside packed
   int* outside;              // set when an id lies beyond the bitmap: the call has to be repeated
   LookbackState lb;          // of the scan of the tile counts; the marks clear it
   int64_t lb_tiles;
@@ -321,15 +321,20 @@ __device__ __forceinline__ int row_of(const int64_t* off, int lo, int hi, int64_
   return lo;
 }
 
-// What a kept edge brings along: nothing, data[position], data[e_ids[position]], or what lies packed beside its row number.
-enum Data { kNoData, kByPosition, kByEdgeId, kPacked };
+// What a kept edge brings along: nothing, data[position], data[e_ids[position]]; for the copy, what lies packed beside
+// its row number; for the marks, nothing but where its data are.
+enum Data { kNoData, kByPosition, kByEdgeId, kPacked, kPlaces };
 
-template <typename IdT, typename Set, int BLOCK, int WAVES, bool PLACES, bool STREAM>
-__global__ void __launch_bounds__(BLOCK, WAVES)  // (waves a SIMD)
+constexpr int kWavesPerSimd = 4;  // what the set leaves room for
+
+template <typename IdT, typename Set, int BLOCK, Data DATA, bool STREAM>
+__global__ void __launch_bounds__(BLOCK, kWavesPerSimd)
 induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
                     const IdT* __restrict__ indices, const IdT* __restrict__ cols, int64_t S,
                     const int64_t* __restrict__ sub_indptr, int64_t D, const IdT* __restrict__ ids,
-                    int n_ids, int64_t bound, InducedMarks m) {
+                    int n_ids, int64_t bound, const float* __restrict__ data,
+                    const int64_t* __restrict__ e_ids, InducedMarks m) {
+  constexpr bool PLACES = DATA == kPlaces;
   __shared__ int64_t s_offsets[BLOCK / kWave][kWindow + 1];
   __shared__ int64_t s_starts[BLOCK / kWave][kWindow];  // start of the column minus its offset
   __shared__ int64_t s_scan[BLOCK / kWave + 1];
@@ -424,6 +429,9 @@ induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
   auto once = [](const auto* p) { return STREAM ? __builtin_nontemporal_load(p) : *p; };
   IdT id[kPer];
   int64_t next_at = 0, my_at = 0;  // lane k: of word k of the tile asked for and of this one
+  // (the data of all: 64 neighbours share their lines with the kept ones among them)
+  float next_w[DATA == kByPosition ? kPer : 1], w[DATA == kByPosition || DATA == kByEdgeId ? kPer : 1];
+  int64_t e[DATA == kByEdgeId ? kPer : 1];
   auto fetch = [&](int64_t t) {
     const int64_t q0 = t * kTile;
     if (q0 >= row_end) settle(q0);
@@ -431,6 +439,14 @@ induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
       const IdT* from = indices + row_start + q0 + lane;
 #pragma unroll
       for (int k = 0; k < kPer; ++k) id[k] = once(from + k * kWave);
+      if constexpr (DATA == kByPosition) {
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) next_w[k] = once(data + row_start + q0 + lane + k * kWave);
+      }
+      if constexpr (DATA == kByEdgeId) {
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) e[k] = once(e_ids + row_start + q0 + lane + k * kWave);
+      }
       if (PLACES) next_at = row_start + q0 + lane * kWave;
       return;
     }
@@ -444,6 +460,14 @@ induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
     }
 #pragma unroll
     for (int k = 0; k < kPer; ++k) id[k] = once(indices + at[k]);
+    if constexpr (DATA == kByPosition) {
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) next_w[k] = once(data + at[k]);
+    }
+    if constexpr (DATA == kByEdgeId) {
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) e[k] = once(e_ids + at[k]);
+    }
   };
 
   stage(wave_upper_bound(sub_indptr, S + 1, tile0 * kTile) - 1);
@@ -454,12 +478,20 @@ induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
     bool in[kPer];
     set.lookup(id, val, in);
     my_at = next_at;
-    if (t + kStep < tile1) fetch(t + kStep);
     if (p0 + kTile > D) {
 #pragma unroll
       for (int k = 0; k < kPer; ++k)
         if (p0 + k * kWave + lane >= D) in[k] = false;
     }
+    if constexpr (DATA == kByPosition) {
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) w[k] = next_w[k];
+    }
+    if constexpr (DATA == kByEdgeId) {
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) w[k] = in[k] ? data[e[k]] : 0.0f;
+    }
+    if (t + kStep < tile1) fetch(t + kStep);
     int before = 0, my_before = 0;
     unsigned long long my_word = 0;
 #pragma unroll
@@ -473,7 +505,10 @@ induced_mark_kernel(const int64_t* __restrict__ indptr, int64_t num_cols,
                                                           __builtin_amdgcn_mbcnt_lo(
                                                               static_cast<uint32_t>(kept), 0));
       before += __popcll(kept);
-      if (in[k]) m.packed[p0 + rank] = static_cast<uint16_t>(val[k]);
+      if (in[k]) {
+        m.packed[p0 + rank] = static_cast<uint16_t>(val[k]);
+        if constexpr (DATA == kByPosition || DATA == kByEdgeId) m.packed_data[p0 + rank] = w[k];
+      }
     }
     if (lane < kPer && p0 + lane * kWave < D) {
       m.mask[(p0 >> 6) + lane] = my_word;
@@ -506,8 +541,10 @@ induced_indptr_kernel(const int64_t* __restrict__ sub_indptr, int64_t S, Induced
 
 // Every tile's kept edges from the front of its range to their place in the result, a wave at a
 // time: eight times 64, all reads before the stores.  The data come from the parent, word by word.
-// (out_indices null: the data only, to the front of the tile's range of out_data.)
 constexpr int kCopyTiles = 4;  // of a workgroup, one for every wave
+// Up to so many kept edges of a tile are a lane each, whatever their words: 40 M positions in columns of 600, 32-bit ids,
+// 4 and 8 % kept, word by word 202 and 219 us, so 191 and 204 (192, three of a lane: the same).
+constexpr int kFewKept = kWave;
 
 template <typename IdT, Data DATA, bool STREAM>
 __global__ void __launch_bounds__(256)
@@ -516,14 +553,14 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
                        const int64_t* __restrict__ e_ids, IdT* __restrict__ out_indices,
                        float* __restrict__ out_data) {
   constexpr bool kParent = DATA == kByPosition || DATA == kByEdgeId;
-  // kept positions of a tile's words of several columns, and above them the places of their data in the tile
+  // kept positions of a tile's words of several columns (or of all), and above them the places of their data in the tile
   __shared__ uint32_t s_kept[kParent ? kCopyTiles : 1][kTile];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // (a scalar, and so are all addresses' bases)
   const int64_t t = static_cast<int64_t>(blockIdx.x) * kCopyTiles + wave;
   if (t >= m.tiles) return;
-  const int64_t first = m.tile_base[t], base = out_indices ? first : t * kTile;
-  const int count = static_cast<int>(m.tile_base[t + 1] - first);
+  const int64_t base = m.tile_base[t];
+  const int count = static_cast<int>(m.tile_base[t + 1] - base);
   unsigned long long my_word = 0;  // lane k: word k of the tile
   int my_rank = 0;
   int64_t my_at = 0;
@@ -532,7 +569,7 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
     my_rank = m.word_rank[t * kPer + lane];
     my_at = m.word_at[t * kPer + lane];
   }
-  if (count <= 0) return;  // (below: the last tile, where an id lay outside and the total is -1)
+  if (count == 0) return;
   auto once = [](const auto* p) { return STREAM ? __builtin_nontemporal_load(p) : *p; };
   uint16_t v[kPer];
 #pragma unroll
@@ -544,7 +581,7 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
       const int r = k * kWave + lane;
-      if (out_indices && r < count) {
+      if (r < count) {
         if (STREAM)
           __builtin_nontemporal_store(static_cast<IdT>(v[k]), out_indices + base + r);
         else
@@ -569,10 +606,10 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
   if constexpr (kParent) {
     const bool of_several = my_word && !WordAt::one(my_at);
     const uint64_t several_words = __ballot(of_several);
-    if (several_words) {
+    const bool few = count <= kFewKept;
+    if (several_words || few) {
       // Kept edge by kept edge, so that a column is looked for where an edge is kept, and three of a lane's together, so
-      // that they are the same few trips.  (Position by position, one word behind the other, the whole call took 135 us
-      // where it takes 116, 8 M positions in columns of 16, 4 % kept; all words' positions together 130.)
+      // that they are the same few trips.
       int most = of_several ? static_cast<int>(WordAt::more(my_at)) : 0;
 #pragma unroll
       for (int d = 1; d < kPer; d <<= 1) {
@@ -584,7 +621,7 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
       int listed = 0;
 #pragma unroll
       for (int k = 0; k < kPer; ++k) {
-        if (!(several_words >> k & 1u)) continue;
+        if (!few && !(several_words >> k & 1u)) continue;
         const uint64_t word = of(my_word, k);
         const int before = set_before(word);
         if (word >> lane & 1u)
@@ -597,6 +634,7 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
         constexpr int N = decltype(how_many)::value;
         int64_t at[N], end[N], start[N];
         int lo[N], hi[N], r[N];
+        bool one[N];
 #pragma unroll
         for (int u = 0; u < N; ++u) {
           const int j = r0 + u * kWave + lane;
@@ -605,27 +643,37 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
           const int64_t where = __shfl(my_at, p / kWave, kWave);
           r[u] = static_cast<int>(kept_one >> 16);
           at[u] = t * kTile + p;
+          one[u] = WordAt::one(where);
           lo[u] = static_cast<int>(WordAt::first(where));
           hi[u] = lo[u] + static_cast<int>(WordAt::more(where));
-        }
-        for (int left = most; left; left >>= 1) {
-#pragma unroll
-          for (int u = 0; u < N; ++u) end[u] = sub_indptr[lo[u] + ((hi[u] - lo[u]) >> 1) + 1];
-#pragma unroll
-          for (int u = 0; u < N; ++u) {
-            const int mid = lo[u] + ((hi[u] - lo[u]) >> 1);
-            if (lo[u] < hi[u]) {
-              if (end[u] > at[u]) hi[u] = mid; else lo[u] = mid + 1;
-            }
+          if (one[u]) {
+            at[u] = where + (p & (kWave - 1));
+            lo[u] = hi[u] = 0;
           }
         }
+        if (several_words) {
+          for (int left = most; left; left >>= 1) {
 #pragma unroll
-        for (int u = 0; u < N; ++u) {
-          start[u] = static_cast<int64_t>(cols[lo[u]]);
-          end[u] = sub_indptr[lo[u]];
+            for (int u = 0; u < N; ++u) end[u] = sub_indptr[lo[u] + ((hi[u] - lo[u]) >> 1) + 1];
+#pragma unroll
+            for (int u = 0; u < N; ++u) {
+              const int mid = lo[u] + ((hi[u] - lo[u]) >> 1);
+              if (lo[u] < hi[u]) {
+                if (end[u] > at[u]) hi[u] = mid; else lo[u] = mid + 1;
+              }
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < N; ++u) {
+            start[u] = static_cast<int64_t>(cols[lo[u]]);
+            end[u] = sub_indptr[lo[u]];
+          }
+#pragma unroll
+          for (int u = 0; u < N; ++u) start[u] = indptr[one[u] ? 0 : start[u]];
+#pragma unroll
+          for (int u = 0; u < N; ++u)
+            if (!one[u]) at[u] += start[u] - end[u];
         }
-#pragma unroll
-        for (int u = 0; u < N; ++u) at[u] += indptr[start[u]] - end[u];
         if constexpr (DATA == kByEdgeId) {
 #pragma unroll
           for (int u = 0; u < N; ++u) at[u] = once(e_ids + at[u]);
@@ -695,8 +743,27 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
   }
 }
 
-// pack: the data are to be packed by the marks' call
-bool carve_induced(void* workspace, size_t bytes, int64_t D, bool with_data, bool pack, InducedMarks* m) {
+// Whether the marks read the data and pack them beside the row numbers, or the copy reads the kept edges' from the
+// parent.  The first is 8 bytes more of every kept edge, the second a wave's trips to memory one behind the other, and to
+// the offsets too where columns are short.  The whole call, the marks / the copy, us, 40 M positions, 32-bit ids, 8000 of
+// 1 M nodes in the set, 4 % kept by chance, and 64-bit ids of 0.4 M, 10, 50 and 90 % kept:
+//   positions / columns  64 431/455, 360/401, 415/500, 487/573    130 357/380, 267/297, 329/375, 403/436
+//                       300 328/351, 221/235, 279/299, 355/345    600 284/304, 200/210, 264/267, 336/313
+//                      4000 238/252, 177/178, 239/241, 312/287    and 500 of 0.2 M nodes, 139/122
+// and 7263 nodes with columns of 7000, 50.8 M, 43 % kept: 185 + 85 / 130 + 114 us (1142 / 967 MB).
+inline bool marks_read_data(int64_t S, int64_t D) { return D < kLongColumns * S; }
+
+// in_marks: with data, who reads them
+size_t induced_bytes(int64_t D, bool with_data, bool in_marks) {
+  if (D < 1) D = 1;
+  const size_t words = static_cast<size_t>(D / kWave + 1), n = static_cast<size_t>(D);
+  const int64_t tiles = ((D - 1) >> kTileShift) + 1;
+  return padded(words * 8) + padded(words * 4) + padded(static_cast<size_t>(tiles + 1) * 8) +
+         padded(static_cast<size_t>(tiles + 2) * 8) + lookback_state_bytes(scan_num_tiles(tiles)) + 256 +
+         padded(n * 2) + (with_data ? (in_marks ? padded(n * 4) : padded(words * 8)) : 0);
+}
+
+bool carve_induced(void* workspace, size_t bytes, int64_t D, bool with_data, bool in_marks, InducedMarks* m) {
   Carver ws(workspace, bytes);
   const size_t words = static_cast<size_t>(D / kWave + 1);
   const size_t most = static_cast<size_t>(((D - 1) >> kTileShift) + 1);
@@ -710,8 +777,8 @@ bool carve_induced(void* workspace, size_t bytes, int64_t D, bool with_data, boo
   m->lb = carve_lookback(ws, m->lb_tiles, 1u);
   m->outside = ws.take<int>(1);
   m->packed = ws.take<uint16_t>(static_cast<size_t>(D));
-  m->word_at = with_data ? ws.take<int64_t>(words) : nullptr;
-  m->packed_data = with_data && pack ? ws.take<float>(static_cast<size_t>(D)) : nullptr;
+  m->word_at = with_data && !in_marks ? ws.take<int64_t>(words) : nullptr;
+  m->packed_data = with_data && in_marks ? ws.take<float>(static_cast<size_t>(D)) : nullptr;
   return ws.ok;
 }
 
@@ -724,7 +791,9 @@ struct MarkCall {
   int64_t D;
   const void* ids;
   int64_t n_ids, bound;
-  bool with_data;
+  const float* data;
+  const int64_t* e_ids;
+  bool in_marks;
 };
 
 // Whether the ids and data of D positions are more than the 256 MB that the memory-side cache holds.
@@ -735,13 +804,10 @@ inline bool streams(int64_t D, size_t id_bytes, bool with_data) {
   return D * static_cast<int64_t>(id_bytes + (with_data ? 4 : 0)) >= int64_t(1) << 28;
 }
 
-template <typename IdT, typename Set, int BLOCK, int WAVES>
+template <typename IdT, typename Set, int BLOCK, Data DATA>
 int launch_mark(const MarkCall& c, int per_unit, const InducedMarks& m, hipStream_t st) {
-  const bool past = streams(c.D, sizeof(IdT), c.with_data);
-  auto* kernel = c.with_data ? (past ? induced_mark_kernel<IdT, Set, BLOCK, WAVES, true, true>
-                                     : induced_mark_kernel<IdT, Set, BLOCK, WAVES, true, false>)
-                             : (past ? induced_mark_kernel<IdT, Set, BLOCK, WAVES, false, true>
-                                     : induced_mark_kernel<IdT, Set, BLOCK, WAVES, false, false>);
+  auto* kernel = streams(c.D, sizeof(IdT), DATA != kNoData) ? induced_mark_kernel<IdT, Set, BLOCK, DATA, true>
+                                                            : induced_mark_kernel<IdT, Set, BLOCK, DATA, false>;
   const size_t bytes = Set::lds_bytes(c.bound, c.n_ids);
   // (per call: the attribute belongs to the device the call runs on)
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -754,8 +820,17 @@ int launch_mark(const MarkCall& c, int per_unit, const InducedMarks& m, hipStrea
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(runs < most ? runs : most)),
                      dim3(BLOCK), bytes, st, c.indptr, c.num_cols, static_cast<const IdT*>(c.indices),
                      static_cast<const IdT*>(c.cols), c.S, c.sub_indptr, c.D,
-                     static_cast<const IdT*>(c.ids), static_cast<int>(c.n_ids), c.bound, m);
+                     static_cast<const IdT*>(c.ids), static_cast<int>(c.n_ids), c.bound, c.data,
+                     c.e_ids, m);
   return check_launch("induced_slice_mark");
+}
+
+template <typename IdT, typename Set, int BLOCK>
+int launch_mark(const MarkCall& c, int per_unit, const InducedMarks& m, hipStream_t st) {
+  if (!c.data) return launch_mark<IdT, Set, BLOCK, kNoData>(c, per_unit, m, st);
+  if (!c.in_marks) return launch_mark<IdT, Set, BLOCK, kPlaces>(c, per_unit, m, st);
+  if (!c.e_ids) return launch_mark<IdT, Set, BLOCK, kByPosition>(c, per_unit, m, st);
+  return launch_mark<IdT, Set, BLOCK, kByEdgeId>(c, per_unit, m, st);
 }
 
 // LDS that the kernel declares itself
@@ -769,12 +844,12 @@ template <typename IdT>
 int pick_mark(const MarkCall& c, const InducedMarks& m, hipStream_t st) {
   const size_t bitmap = BitmapSet<IdT>::lds_bytes(c.bound, c.n_ids);
   if (2 * (bitmap + fixed_lds(512)) <= kLdsBytes)
-    return launch_mark<IdT, BitmapSet<IdT>, 512, 4>(c, 2, m, st);
+    return launch_mark<IdT, BitmapSet<IdT>, 512>(c, 2, m, st);
   if (bitmap + fixed_lds(1024) <= kLdsBytes)
-    return launch_mark<IdT, BitmapSet<IdT>, 1024, 4>(c, 1, m, st);
+    return launch_mark<IdT, BitmapSet<IdT>, 1024>(c, 1, m, st);
   static_assert(size_t(1 << 13) * 16 + fixed_lds(1024) <= kLdsBytes, "buckets");
-  if (c.n_ids <= kStagedIds) return launch_mark<IdT, BucketSet<IdT, true>, 1024, 4>(c, 1, m, st);
-  return launch_mark<IdT, BucketSet<IdT, false>, 1024, 4>(c, 1, m, st);
+  if (c.n_ids <= kStagedIds) return launch_mark<IdT, BucketSet<IdT, true>, 1024>(c, 1, m, st);
+  return launch_mark<IdT, BucketSet<IdT, false>, 1024>(c, 1, m, st);
 }
 
 template <typename IdT>
@@ -814,26 +889,17 @@ int gs_induced_slice_applies(int64_t num_row_ids, int64_t S, int64_t D, int64_t)
   return num_row_ids > 0 && num_row_ids <= kMaxIds && S > 0 && S < (int64_t(1) << 31) && D >= (int64_t(1) << 20) && D >= 16 * S;
 }
 
-size_t gs_induced_slice_notify_workspace_bytes(int64_t D, int with_data) {
-  if (D < 1) D = 1;
-  const size_t words = static_cast<size_t>(D / kWave + 1), n = static_cast<size_t>(D);
-  const int64_t tiles = ((D - 1) >> kTileShift) + 1;
-  return padded(words * 8) + padded(words * 4) + padded(static_cast<size_t>(tiles + 1) * 8) +
-         padded(static_cast<size_t>(tiles + 2) * 8) + lookback_state_bytes(scan_num_tiles(tiles)) + 256 +
-         padded(n * 2) + (with_data ? padded(words * 8) : 0);
+size_t gs_induced_slice_notify_workspace_bytes(int64_t S, int64_t D, int with_data) {
+  return induced_bytes(D, with_data != 0, marks_read_data(S, D));
 }
 
-size_t gs_induced_slice_workspace_bytes(int64_t D, int with_data) {
-  return gs_induced_slice_notify_workspace_bytes(D, with_data) +
-         (with_data ? padded(static_cast<size_t>(D < 1 ? 1 : D) * 4) : 0);
-}
+size_t gs_induced_slice_workspace_bytes(int64_t D, int with_data) { return induced_bytes(D, with_data != 0, true); }
 
-int gs_induced_slice_mark_notify(const int64_t* indptr, int64_t num_cols, const void* indices, int64_t nnz,
-                                 int64_t num_rows, int id_bytes, const void* column_ids, int64_t S,
-                                 const int64_t* sub_indptr, int64_t D, const void* row_ids,
-                                 int64_t num_row_ids, int with_data, int64_t* out_indptr,
-                                 gs_mailbox* mailbox, int64_t ticket, void* workspace,
-                                 size_t workspace_bytes, void* stream) {
+static int induced_mark(const int64_t* indptr, int64_t num_cols, const void* indices, int64_t nnz, int64_t num_rows,
+                        int id_bytes, const void* column_ids, int64_t S, const int64_t* sub_indptr, int64_t D,
+                        const void* row_ids, int64_t num_row_ids, const float* edge_data, const int64_t* edge_ids,
+                        bool in_marks, int64_t* out_indptr, gs_mailbox* mailbox, int64_t ticket, void* workspace,
+                        size_t workspace_bytes, void* stream) {
   GS_REQUIRE(gs_induced_slice_applies(num_row_ids, S, D, nnz) && num_rows >= 0,
              "gs_induced_slice_mark: sizes beyond gs_induced_slice_applies");
   GS_REQUIRE(indptr && indices && column_ids && sub_indptr && row_ids && out_indptr,
@@ -841,15 +907,15 @@ int gs_induced_slice_mark_notify(const int64_t* indptr, int64_t num_cols, const 
   GS_REQUIRE(valid_id_bytes(id_bytes), "gs_induced_slice_mark: id_bytes must be 4 or 8, got %d",
              id_bytes);
   InducedMarks m;
-  if (!carve_induced(workspace, workspace_bytes, D, with_data != 0, false, &m)) {
+  if (!carve_induced(workspace, workspace_bytes, D, edge_data != nullptr, in_marks, &m)) {
     set_error_text("gs_induced_slice_mark: workspace needs %zu bytes, 256-byte aligned",
-                   gs_induced_slice_notify_workspace_bytes(D, with_data));
+                   induced_bytes(D, edge_data != nullptr, in_marks));
     return GS_ERR_WORKSPACE;
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t bound = num_rows > 0 ? num_rows : int64_t(1) << 40;  // (no bound given: no bitmap)
   const MarkCall c{indptr, num_cols, indices, column_ids, S, sub_indptr, D, row_ids, num_row_ids,
-                   bound, with_data != 0};
+                   bound, edge_data, edge_ids, in_marks};
   GS_RETURN_IF_ERROR(id_bytes == 8 ? pick_mark<int64_t>(c, m, st) : pick_mark<int32_t>(c, m, st));
   TileCount f{m.tile_counts};
   GS_RETURN_IF_ERROR(chained_scan(f, m.tiles, m.tile_base, m.lb, st, mailbox, ticket, m.outside));
@@ -858,19 +924,38 @@ int gs_induced_slice_mark_notify(const int64_t* indptr, int64_t num_cols, const 
   return check_launch("induced_slice_mark");
 }
 
-int gs_induced_slice_compact_parent(const int64_t* indptr, int id_bytes, const void* column_ids,
-                                    const int64_t* sub_indptr, int64_t D, const float* edge_data,
-                                    const int64_t* edge_ids, void* out_indices, float* out_data,
-                                    void* workspace, size_t workspace_bytes, void* stream) {
-  GS_REQUIRE(D > 0 && out_indices && indptr && column_ids && sub_indptr, "gs_induced_slice_compact: bad argument");
-  GS_REQUIRE(!edge_data == !out_data, "gs_induced_slice_compact: data without a place for them, or the other way round");
+int gs_induced_slice_mark(const int64_t* indptr, int64_t num_cols, const void* indices, int64_t nnz,
+                          int64_t num_rows, int id_bytes, const void* column_ids, int64_t S,
+                          const int64_t* sub_indptr, int64_t D, const void* row_ids,
+                          int64_t num_row_ids, const float* edge_data, const int64_t* edge_ids,
+                          int64_t* out_indptr, void* workspace, size_t workspace_bytes,
+                          void* stream) {
+  return induced_mark(indptr, num_cols, indices, nnz, num_rows, id_bytes, column_ids, S, sub_indptr, D, row_ids,
+                      num_row_ids, edge_data, edge_ids, true, out_indptr, nullptr, 0, workspace, workspace_bytes, stream);
+}
+
+int gs_induced_slice_mark_notify(const int64_t* indptr, int64_t num_cols, const void* indices, int64_t nnz,
+                                 int64_t num_rows, int id_bytes, const void* column_ids, int64_t S,
+                                 const int64_t* sub_indptr, int64_t D, const void* row_ids,
+                                 int64_t num_row_ids, const float* edge_data, const int64_t* edge_ids,
+                                 int64_t* out_indptr, gs_mailbox* mailbox, int64_t ticket, void* workspace,
+                                 size_t workspace_bytes, void* stream) {
+  return induced_mark(indptr, num_cols, indices, nnz, num_rows, id_bytes, column_ids, S, sub_indptr, D, row_ids,
+                      num_row_ids, edge_data, edge_ids, marks_read_data(S, D), out_indptr, mailbox, ticket, workspace,
+                      workspace_bytes, stream);
+}
+
+static int induced_compact(const int64_t* indptr, int id_bytes, const void* column_ids, const int64_t* sub_indptr,
+                           int64_t D, const float* edge_data, const int64_t* edge_ids, bool in_marks, void* out_indices,
+                           float* out_data, void* workspace, size_t workspace_bytes, void* stream) {
   GS_REQUIRE(valid_id_bytes(id_bytes), "gs_induced_slice_compact: id_bytes must be 4 or 8, got %d",
              id_bytes);
   InducedMarks m;
-  if (!carve_induced(workspace, workspace_bytes, D, out_data != nullptr, false, &m)) {
+  if (!carve_induced(workspace, workspace_bytes, D, out_data != nullptr, in_marks, &m)) {
     set_error_text("gs_induced_slice_compact: pass the workspace given to gs_induced_slice_mark");
     return GS_ERR_WORKSPACE;
   }
+  if (in_marks) edge_data = nullptr;  // (they lie packed)
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (id_bytes == 8)
     launch_compact(D, m, indptr, column_ids, sub_indptr, edge_data, edge_ids,
@@ -881,47 +966,21 @@ int gs_induced_slice_compact_parent(const int64_t* indptr, int id_bytes, const v
   return check_launch("induced_slice_compact");
 }
 
-int gs_induced_slice_mark(const int64_t* indptr, int64_t num_cols, const void* indices, int64_t nnz,
-                          int64_t num_rows, int id_bytes, const void* column_ids, int64_t S,
-                          const int64_t* sub_indptr, int64_t D, const void* row_ids,
-                          int64_t num_row_ids, const float* edge_data, const int64_t* edge_ids,
-                          int64_t* out_indptr, void* workspace, size_t workspace_bytes,
-                          void* stream) {
-  InducedMarks m;
-  if (D > 0 && !carve_induced(workspace, workspace_bytes, D, edge_data != nullptr, true, &m)) {
-    set_error_text("gs_induced_slice_mark: workspace needs %zu bytes, 256-byte aligned",
-                   gs_induced_slice_workspace_bytes(D, edge_data != nullptr));
-    return GS_ERR_WORKSPACE;
-  }
-  GS_RETURN_IF_ERROR(gs_induced_slice_mark_notify(indptr, num_cols, indices, nnz, num_rows, id_bytes, column_ids, S,
-                                                  sub_indptr, D, row_ids, num_row_ids, edge_data != nullptr, out_indptr,
-                                                  nullptr, 0, workspace, workspace_bytes, stream));
-  if (!edge_data) return GS_OK;
-  // (the other call of the pair knows no data: they wait for it where the row numbers do)
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  if (id_bytes == 8)
-    launch_compact<int64_t>(D, m, indptr, column_ids, sub_indptr, edge_data, edge_ids, nullptr, m.packed_data, st);
-  else
-    launch_compact<int32_t>(D, m, indptr, column_ids, sub_indptr, edge_data, edge_ids, nullptr, m.packed_data, st);
-  return check_launch("induced_slice_mark");
-}
-
 int gs_induced_slice_compact(int64_t D, int id_bytes, void* out_indices, float* out_data,
                              void* workspace, size_t workspace_bytes, void* stream) {
   GS_REQUIRE(D > 0 && out_indices, "gs_induced_slice_compact: bad argument");
-  GS_REQUIRE(valid_id_bytes(id_bytes), "gs_induced_slice_compact: id_bytes must be 4 or 8, got %d",
-             id_bytes);
-  InducedMarks m;
-  if (!carve_induced(workspace, workspace_bytes, D, out_data != nullptr, true, &m)) {
-    set_error_text("gs_induced_slice_compact: pass the workspace given to gs_induced_slice_mark");
-    return GS_ERR_WORKSPACE;
-  }
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  if (id_bytes == 8)
-    launch_compact(D, m, nullptr, nullptr, nullptr, nullptr, nullptr, static_cast<int64_t*>(out_indices), out_data, st);
-  else
-    launch_compact(D, m, nullptr, nullptr, nullptr, nullptr, nullptr, static_cast<int32_t*>(out_indices), out_data, st);
-  return check_launch("induced_slice_compact");
+  return induced_compact(nullptr, id_bytes, nullptr, nullptr, D, nullptr, nullptr, true, out_indices, out_data,
+                         workspace, workspace_bytes, stream);
+}
+
+int gs_induced_slice_compact_parent(const int64_t* indptr, int id_bytes, const void* column_ids, int64_t S,
+                                    const int64_t* sub_indptr, int64_t D, const float* edge_data,
+                                    const int64_t* edge_ids, void* out_indices, float* out_data,
+                                    void* workspace, size_t workspace_bytes, void* stream) {
+  GS_REQUIRE(D > 0 && out_indices && indptr && column_ids && sub_indptr, "gs_induced_slice_compact: bad argument");
+  GS_REQUIRE(!edge_data == !out_data, "gs_induced_slice_compact: data without a place for them, or the other way round");
+  return induced_compact(indptr, id_bytes, column_ids, sub_indptr, D, edge_data, edge_ids, marks_read_data(S, D),
+                         out_indices, out_data, workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"

@@ -1465,14 +1465,16 @@ std::tuple<torch::Tensor, torch::Tensor> InducedSlicing(const torch::Tensor& ind
     return {std::get<0>(r), std::get<1>(r)};
   }
   void* st = Stream(indptr);
+  const float* edge_data = edge ? edge->data.data_ptr<float>() : nullptr;
+  const int64_t* edge_ids = edge ? OptI64(edge->e_ids, "e_ids") : nullptr;
   auto out_indptr = torch::empty({S + 1}, I64(indptr));
-  auto ws = Scratch(gs_induced_slice_notify_workspace_bytes(D, edge != nullptr), indptr);
+  auto ws = Scratch(gs_induced_slice_notify_workspace_bytes(S, D, edge != nullptr), indptr);
   int64_t kept = -1;
   for (int64_t bound : {num_rows, int64_t(0)}) {  // (again without a bound when an id reaches it)
     const TotalBox total(indptr);
     Check(gs_induced_slice_mark_notify(indptr.data_ptr<int64_t>(), indptr.numel() - 1, indices.data_ptr(),
                                        nnz, bound, idb, column_ids.data_ptr(), S,
-                                       sub_indptr.data_ptr<int64_t>(), D, row_ids.data_ptr(), nr, edge != nullptr,
+                                       sub_indptr.data_ptr<int64_t>(), D, row_ids.data_ptr(), nr, edge_data, edge_ids,
                                        out_indptr.data_ptr<int64_t>(), total.slot(), total.ticket, ws.data_ptr(),
                                        ws.numel(), st),
           "gs_induced_slice_mark");
@@ -1482,10 +1484,8 @@ std::tuple<torch::Tensor, torch::Tensor> InducedSlicing(const torch::Tensor& ind
   auto out_indices = torch::empty({kept}, indices.options());
   if (edge) *data_out = torch::empty({kept}, edge->data.options());
   if (kept > 0)
-    Check(gs_induced_slice_compact_parent(indptr.data_ptr<int64_t>(), idb, column_ids.data_ptr(),
-                                          sub_indptr.data_ptr<int64_t>(), D,
-                                          edge ? edge->data.data_ptr<float>() : nullptr,
-                                          edge ? OptI64(edge->e_ids, "e_ids") : nullptr, out_indices.data_ptr(),
+    Check(gs_induced_slice_compact_parent(indptr.data_ptr<int64_t>(), idb, column_ids.data_ptr(), S,
+                                          sub_indptr.data_ptr<int64_t>(), D, edge_data, edge_ids, out_indices.data_ptr(),
                                           edge ? data_out->data_ptr<float>() : nullptr, ws.data_ptr(), ws.numel(), st),
           "gs_induced_slice_compact");
   return {out_indptr, out_indices};

@@ -836,16 +836,16 @@ int gs_induced_slice_mark(const int64_t* indptr, int64_t num_cols, const void* i
                           void* stream);
 int gs_induced_slice_compact(int64_t D, int id_bytes, void* out_indices, float* out_data,
                              void* workspace, size_t workspace_bytes, void* stream);
-/* The same for a caller that keeps the arrays until both calls have run: the data are read by the compact, from the
- * parent and of kept edges only, and the total is in the mailbox (NULL: none) before the offsets are written. */
-size_t gs_induced_slice_notify_workspace_bytes(int64_t D, int with_data);
+/* The same for a caller that keeps the arrays until both calls have run: either call may read the data, and the total is
+ * in the mailbox (NULL: none) before the offsets are written. */
+size_t gs_induced_slice_notify_workspace_bytes(int64_t S, int64_t D, int with_data);
 int gs_induced_slice_mark_notify(const int64_t* indptr, int64_t num_cols, const void* indices, int64_t nnz,
                                  int64_t num_rows, int id_bytes, const void* column_ids, int64_t S,
                                  const int64_t* sub_indptr, int64_t D, const void* row_ids,
-                                 int64_t num_row_ids, int with_data, int64_t* out_indptr,
-                                 gs_mailbox* mailbox, int64_t ticket, void* workspace,
+                                 int64_t num_row_ids, const float* edge_data, const int64_t* edge_ids,
+                                 int64_t* out_indptr, gs_mailbox* mailbox, int64_t ticket, void* workspace,
                                  size_t workspace_bytes, void* stream);
-int gs_induced_slice_compact_parent(const int64_t* indptr, int id_bytes, const void* column_ids,
+int gs_induced_slice_compact_parent(const int64_t* indptr, int id_bytes, const void* column_ids, int64_t S,
                                     const int64_t* sub_indptr, int64_t D, const float* edge_data,
                                     const int64_t* edge_ids, void* out_indices, float* out_data,
                                     void* workspace, size_t workspace_bytes, void* stream);

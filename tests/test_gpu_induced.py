@@ -312,3 +312,40 @@ def test_data_of_tiles_of_several_columns(dev, lens, idt, data):
     want = O.col_row_slice(indptr, indices, cols, rows)
     assert np.array_equal(ptr.cpu().numpy(), want[0]) and np.array_equal(idx.cpu().numpy(), want[1])
     assert np.array_equal(got.cpu().numpy(), w[order][want[3]])
+
+
+@pytest.mark.parametrize("n", [70_000, 2_000_000])  # both forms of the set
+@pytest.mark.parametrize("data", ["by position", "by map"])
+@pytest.mark.parametrize("idt", [torch.int32, torch.int64])
+@pytest.mark.parametrize("more", [0, 1])
+def test_data_on_both_sides_of_long_columns(dev, more, idt, data, n):
+    """512 positions a column, where the copy reads the data from the parent, and one less, where the marks do: one
+    column has most of them, between tiles whose words are of several; few, some and all edges of a tile kept."""
+    rng = np.random.default_rng(n + more)
+    short = np.concatenate([np.resize(np.array(lens), 800) for lens in ([17], [40, 1, 0, 60, 0], [300, 20, 9, 90], [511, 1])])
+    S = short.size + 1
+    degree = np.concatenate([short[:S // 2], [0], short[S // 2:]])
+    degree[S // 2] = 512 * S - short.sum() - more
+    cols = rng.permutation(S)
+    parent = np.zeros_like(degree)
+    parent[cols] = degree
+    indptr = np.concatenate([[0], np.cumsum(parent)]).astype(np.int64)
+    D = int(indptr[-1])
+    assert D == 512 * S - more and D >= 1 << 20
+    kept = np.zeros((D + 511) // 512 * 512, bool)
+    for t, k in zip(range(0, D, 512), np.resize([0, 1, 5, 63, 64, 65, 192, 193, 511, 512], D // 512 + 1)):
+        kept[t + rng.permutation(512)[:k]] = True
+    offset = np.concatenate([[0], np.cumsum(degree)])
+    at = np.repeat(indptr[cols], degree) + np.arange(D) - np.repeat(offset[:-1], degree)
+    indices = np.empty(D, np.int64)
+    indices[at] = np.where(kept[:D], rng.integers(0, 3000, D) * 2, rng.integers(0, 3000, D) * 2 + 1)
+    rows = rng.permutation(3000).astype(np.int64) * 2
+    w = rng.random(D).astype(np.float32)
+    order = rng.permutation(D) if data == "by map" else np.arange(D)
+    want = O.col_row_slice(indptr, indices, cols, rows)
+    args = [to_dev(indptr, dev), to_dev(indices, dev, idt), to_dev(cols, dev, idt), to_dev(rows, dev, idt), n,
+            to_dev(w, dev), to_dev(order, dev) if data == "by map" else None]
+    for stays in (False, True):
+        ptr, idx, got = capi.induced_slice(*args, kept=stays)
+        assert np.array_equal(ptr.cpu().numpy(), want[0]) and np.array_equal(idx.cpu().numpy(), want[1])
+        assert np.array_equal(got.cpu().numpy(), w[order][want[3]])
