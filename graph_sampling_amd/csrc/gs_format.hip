@@ -778,6 +778,7 @@ constexpr uint32_t kWideTile = 16;  // offsets a thread beyond which a tile has 
 // kGapPiece: the columns above the last lower digit in use are all one tile's, 2.4 M of them where the lower 16 bits of
 // 2.45 M ids stay below 100.  Sorts of such lists and of ids whose lower bits are 30000 to 30004, us, by written keys / by
 // one workgroup with a search a column / so: 14 M edges 340/534/293 and 328/1080/288, 5 M 183/673/162 and 170/1440/155.
+// With two digits no item has more than 256 columns, and a launch that finds nothing would be 2 us of 25 to 40.
 constexpr int64_t kThreeDigitItems = 1'300'000;  // edges from which small tiles' last pass of three leaves the offsets
 constexpr int kGapBlocks = 512;
 constexpr uint32_t kGapLane = 4, kGapHere = 128, kGapPiece = 2048;
@@ -1046,6 +1047,7 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
         leave(d, from + i % lows, s_start[d], run_end(d));
       }
     } else {  // long gaps: by items, and what lies behind a digit's last one
+      constexpr uint32_t kHere = kLowBits == kRadixBits ? uint32_t(kRadix) : kGapHere;  // (with two digits none is longer)
       for (uint32_t u0 = wave * kWave; u0 < n + digits; u0 += kThreadsHere) {
         const uint32_t u = u0 + lane;
         uint32_t first = 0, count = 0, offset = 0;
@@ -1061,12 +1063,12 @@ packed_pass_kernel(const IdT* __restrict__ key, const IdT* __restrict__ value,
         }
         if (count <= kGapLane) {
           for (uint32_t k = 0; k < count; ++k) last.indptr[first + k] = offset;
-        } else if (count > kGapHere) {
+        } else if (count > kHere) {
           uint32_t at = atomicAdd(last.wide + 1, (count + kGapPiece - 1) / kGapPiece);
           for (uint32_t k = 0; k < count; k += kGapPiece, ++at)
             last.gaps[at] = make_uint4(first + k, count - k < kGapPiece ? count - k : kGapPiece, offset, 0u);
         }
-        for (unsigned long long some = __ballot(count > kGapLane && count <= kGapHere); some; some &= some - 1) {
+        for (unsigned long long some = __ballot(count > kGapLane && count <= kHere); some; some &= some - 1) {
           const int from_lane = __builtin_ctzll(some);
           const uint32_t f = __builtin_amdgcn_readlane(first, from_lane), c = __builtin_amdgcn_readlane(count, from_lane);
           const uint32_t o = __builtin_amdgcn_readlane(offset, from_lane);
@@ -1314,9 +1316,9 @@ int coo2csc_impl(const IdT* key, const IdT* value, int64_t E, int64_t num_keys, 
                        dim3(kThreads), 0, st, value, perm, E, s.wide, out_value);
   if (by_keys)  // (null: the caller wants the sorted order only)
     launch_indptr(static_cast<const uint32_t*>(s.keys), E, num_keys, indptr, st);
-  else if (by_tiles)
+  else if (by_tiles && passes > 2)
     hipLaunchKernelGGL(gap_fill_kernel, dim3(kGapBlocks), dim3(kThreads), 0, st, outs.gaps, s.wide + 1, indptr);
-  else if (indptr)
+  else if (indptr && !by_tiles)
     hipLaunchKernelGGL((indptr_from_sorted_kernel<PermutedKeys<IdT>>),
                        dim3(blocks_for(num_keys + 1, kPtrCols)), dim3(kThreads), 0, st,
                        PermutedKeys<IdT>{key, perm}, E, num_keys, indptr);
