@@ -715,17 +715,14 @@ induced_compact_kernel(InducedMarks m, const int64_t* __restrict__ indptr, const
       const int64_t where = static_cast<int64_t>(of(static_cast<uint64_t>(my_at), k));
       kept[k] = word >> lane & 1u;
       rank[k] = __builtin_amdgcn_readlane(my_rank, k) + set_before(word);
-      // (lanes whose edge is left out read with the word's first kept one, a word without any the first datum:
-      // data may end before edges that are not kept)
+      // (lanes whose edge is left out read with the word's first kept one, a word without any the first datum: behind
+      // the last position there is no edge)
       const int place = kept[k] ? lane : (word ? __builtin_ctzll(word) : 0);
       at[k] = word ? where + place : 0;
     }
     if constexpr (DATA == kByEdgeId) {
 #pragma unroll
-      for (int k = 0; k < kPer; ++k) {
-        const int64_t e = once(e_ids + at[k]);
-        at[k] = of(my_word, k) ? e : 0;  // (data may end before edges that are not kept)
-      }
+      for (int k = 0; k < kPer; ++k) at[k] = once(e_ids + at[k]);
     }
 #pragma unroll
     for (int k = 0; k < kPer; ++k) x[k] = once(data + at[k]);

@@ -778,7 +778,7 @@ c10::intrusive_ptr<Graph> Graph::FusedBidirSlicing(torch::Tensor column_seeds,
   auto ret = Child(Pick(col_ids_, column_seeds), Pick(row_ids_, row_seeds), column_seeds.numel(),
                    row_seeds.numel());
   auto sliced = std::make_shared<CSC>();
-  // (that form reads the data of every edge of the columns, dropped ones too: all have to be there)
+  // (that form reads the data of every edge of short columns, dropped ones too: all have to be there)
   if (!data_.has_value() || (hip::EdgeData::Fits(data_.value(), csc_->e_ids) &&
                              !hip::EdgeData::Followed(data_.value()) &&
                              data_.value().numel() >= csc_->indices.numel())) {

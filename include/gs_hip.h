@@ -747,13 +747,13 @@ int gs_coo_sum(const void* target, int id_bytes, const int64_t* e_ids, const flo
  * the additions is not fixed in either (impl::COOSumCUDA, src/cuda/graph_ops.cu:45-64, adds
  * with atomics too). */
 size_t gs_coo_sum_workspace_bytes(int64_t E, int64_t num_targets);
-/* The same into an `out` that holds nothing yet: every entry is written. */
-int gs_coo_sum_fresh(const void* target, int id_bytes, const int64_t* e_ids, const float* data, int64_t E,
-                     int64_t powk, int64_t num_targets, float* out, void* workspace, size_t workspace_bytes,
-                     void* stream);
 int gs_coo_sum_binned(const void* target, int id_bytes, const int64_t* e_ids, const float* data,
                       int64_t E, int64_t powk, int64_t num_targets, float* out, void* workspace,
                       size_t workspace_bytes, void* stream);
+/* gs_coo_sum_binned into an `out` that holds nothing yet: every entry is written. */
+int gs_coo_sum_fresh(const void* target, int id_bytes, const int64_t* e_ids, const float* data, int64_t E,
+                     int64_t powk, int64_t num_targets, float* out, void* workspace, size_t workspace_bytes,
+                     void* stream);
 
 /* out[d] = data[d] / sum of its segment, d = e_ids ? e_ids[e] : e; edges outside the offsets are
  * left alone.  nnz as in gs_segment_sum. */
